@@ -8,6 +8,7 @@ import os
 
 _PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_PKG_DIR, "lib", "libbitlinear_hip.so")
+HOST_CALLS_PATH = os.path.join(_PKG_DIR, "lib", "_host_calls.so")
 
 _c_int = ctypes.c_int
 _c_ptr = ctypes.c_void_p
@@ -121,6 +122,7 @@ class Problem(ctypes.Structure):
     ]
 
 _lib = None
+_host = None
 
 
 class BitLinearLibraryError(RuntimeError):
@@ -152,6 +154,31 @@ def load_library(path: str = None) -> ctypes.CDLL:
     if path is None:
         _lib = lib
     return lib
+
+
+def host_calls():
+    """The CPython module built from csrc/host_calls.cpp (torch tensors -> C ABI in native code), bound to the library
+    load_library() opens.  Like the library it has no fallback: a missing build raises."""
+    global _host
+    if _host is None:
+        import importlib.util
+
+        import torch  # noqa: F401  (the module links to torch's libraries)
+
+        if not os.path.exists(HOST_CALLS_PATH):
+            raise BitLinearLibraryError(f"{HOST_CALLS_PATH} not found: build it with `python -m bitnet_amd.build`")
+        spec = importlib.util.spec_from_file_location("_host_calls", HOST_CALLS_PATH)
+        try:
+            mod = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(mod)
+        except ImportError as e:  # another torch or Python than it was built against
+            raise BitLinearLibraryError(f"cannot load {HOST_CALLS_PATH}: {e}") from e
+        lib = load_library()
+        mod.bind(BitLinearLibraryError, *(ctypes.cast(getattr(lib, name), _c_ptr).value for name in (
+            "bitlinear_int8xint2", "bitlinear_last_status", "bitlinear_status_string", "bitlinear_ws_num",
+            "bitlinear_quant_absmax", "bitlinear_forward_bf16", "bitlinear_forward_bf16_seg")))
+        _host = mod
+    return _host
 
 
 def plan_name(entry: int, M: int, N: int, K: int) -> str:

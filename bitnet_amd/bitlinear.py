@@ -6,7 +6,9 @@ Same names, argument meaning and tensor layouts as the reference:
 packed int8 ``weight`` of shape (out_features, in_features // 4) and a 4-slot
 bf16 ``weight_scale``, and the fake-quant ``BitLinear``.  torch is used for
 device memory and the current stream only; all arithmetic of the int8 path
-runs in the HIP library.
+runs in the HIP library.  The three calls of a serving loop (forward, the
+drop-in product, the quantizer) check their arguments, allocate and launch in
+native code (csrc/host_calls.cpp): at one token the host is what they cost.
 """
 import ctypes
 
@@ -50,32 +52,7 @@ def bitnet_int8xint2_linear(input0, input1, s, ws, out=None):
     ``ws`` the bf16 weight scales.  The output is allocated here with
     torch.empty unless ``out`` is given (the library writes every element, so
     the reference's zero fill is not needed)."""
-    _check_device(input0, input1, s, ws)
-    if input0.dtype != torch.int8 or input1.dtype != torch.int8:
-        raise TypeError("input0 and input1 must be int8")
-    if s.dtype != torch.bfloat16 or ws.dtype != torch.bfloat16:
-        raise TypeError("s and ws must be bfloat16")
-    out_shape = list(input0.shape)
-    out_shape[-1] = input1.shape[0]
-    M = _flat_rows(input0)
-    N = input1.shape[0]
-    K = input1.shape[1] * 4
-    if input0.shape[-1] != K:
-        raise ValueError(f"activation width {input0.shape[-1]} does not match packed weight K={K}")
-    if s.numel() < M:
-        raise ValueError(f"need one activation scale per row: {s.numel()} < {M}")
-    lib = _lib.load_library()
-    if ws.numel() < lib.bitlinear_ws_num(N, K):
-        raise ValueError("weight_scale has fewer slots than this shape uses")
-    if out is None:
-        out = torch.empty(*out_shape, dtype=torch.bfloat16, device=input0.device)
-    elif out.dtype != torch.bfloat16 or out.numel() != M * N or not out.is_contiguous() or not out.is_cuda:
-        raise ValueError("out must be a contiguous bfloat16 GPU tensor of M x N elements")
-    if M == 0:
-        return out  # no token rows: nothing to launch
-    lib.bitlinear_int8xint2(_ptr(input0), _ptr(input1), _ptr(out), _ptr(s), _ptr(ws), M, N, K, _stream_ptr())
-    _lib.check(lib.bitlinear_last_status(), f"bitlinear_int8xint2(M={M}, N={N}, K={K})")
-    return out
+    return (_lib._host or _lib.host_calls()).linear(input0, input1, s, ws, out)
 
 
 def bitnet_int8xint2_acc(input0, input1):
@@ -165,19 +142,7 @@ def bitnet_int8xint2_linear_seg(input0, input1, s, ws, seg_ends, out=None):
 def quant_input(input, mode: int = QUANT_COMPILED):
     """Per-token absmax quantizer (gpu/model.py:68-71): bf16 [..., K] ->
     (int8 [..., K], bf16 scales [..., 1]).  One fused HIP kernel."""
-    _check_device(input)
-    if input.dtype != torch.bfloat16:
-        raise TypeError("quant_input expects bfloat16")
-    M = _flat_rows(input)
-    K = input.shape[-1]
-    q = torch.empty(input.shape, dtype=torch.int8, device=input.device)
-    s = torch.empty(*input.shape[:-1], 1, dtype=torch.bfloat16, device=input.device)
-    if M == 0:
-        return q, s
-    lib = _lib.load_library()
-    st = lib.bitlinear_quant_absmax(_ptr(input), _ptr(q), _ptr(s), M, K, mode, _stream_ptr())
-    _lib.check(st, f"bitlinear_quant_absmax(M={M}, K={K})")
-    return q, s
+    return (_lib._host or _lib.host_calls()).quant(input, mode)
 
 
 class BitLinearKernel(nn.Module):
@@ -224,34 +189,13 @@ class BitLinearKernel(nn.Module):
         return quant_input(input, self.quant_mode)
 
     def forward(self, input):
-        _check_device(input, self.weight, self.weight_scale)
-        if input.dtype != torch.bfloat16:
-            raise TypeError("BitLinearKernel.forward expects bfloat16 activations")
-        if input.shape[-1] != self.in_features:
-            raise ValueError(f"activation width {input.shape[-1]} does not match in_features={self.in_features}")
-        if self.weight.shape != (self.out_features, self.in_features // 4) or self.weight.dtype != torch.int8:
-            raise ValueError("weight must be int8 [out_features, in_features // 4] (the packed layout)")
-        M = _flat_rows(input)
-        N, K = self.out_features, self.in_features
-        q = torch.empty(input.shape, dtype=torch.int8, device=input.device)
-        s = torch.empty(M, dtype=torch.bfloat16, device=input.device)
-        out = torch.empty(*input.shape[:-1], N, dtype=torch.bfloat16, device=input.device)
-        if M == 0:
-            return out
-        lib = _lib.load_library()
-        if self.seg_ends is not None:
-            st = lib.bitlinear_forward_bf16_seg(
-                _ptr(input), _ptr(self.weight), _ptr(out), _ptr(self.weight_scale), self._seg_c, len(self.seg_ends),
-                _ptr(q), _ptr(s), M, N, K, self.quant_mode, _stream_ptr(),
-            )
-            _lib.check(st, f"bitlinear_forward_bf16_seg(M={M}, N={N}, K={K})")
-            return out
-        st = lib.bitlinear_forward_bf16(
-            _ptr(input), _ptr(self.weight), _ptr(out), _ptr(self.weight_scale), _ptr(q), _ptr(s), M, N, K,
-            self.quant_mode, _stream_ptr(),
-        )
-        _lib.check(st, f"bitlinear_forward_bf16(M={M}, N={N}, K={K})")
-        return out
+        # the parameters as nn.Module stores them; the attribute look-up, which would go through __getattr__, for a module
+        # whose weight was made something else than a parameter
+        p = self._parameters
+        weight, scale = p.get("weight"), p.get("weight_scale")
+        return (_lib._host or _lib.host_calls()).forward(
+            input, self.weight if weight is None else weight, self.weight_scale if scale is None else scale,
+            self.in_features, self.out_features, self.quant_mode, self._seg_c)
 
 
 class BitLinear(nn.Linear):

@@ -1,4 +1,5 @@
-"""Builds libbitlinear_hip.so for gfx950 with hipcc, in-tree.
+"""Builds libbitlinear_hip.so for gfx950 with hipcc, and the CPython module of
+host calls (csrc/host_calls.cpp, plain C++ against torch's headers), in-tree.
 
     python -m bitnet_amd.build
 
@@ -10,6 +11,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 REPO_ROOT = os.path.dirname(PKG_DIR)
@@ -23,6 +25,8 @@ SOURCES = {
 OBJ_DIR = os.path.join(PKG_DIR, "lib", "obj")
 LIB_DIR = os.path.join(PKG_DIR, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libbitlinear_hip.so")
+HOST_SOURCE = os.path.join(PKG_DIR, "csrc", "host_calls.cpp")
+HOST_PATH = os.path.join(LIB_DIR, "_host_calls.so")
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
@@ -50,15 +54,35 @@ def _finish(cmd, res, verbose):
     # the host pass warns that it does not know the packed-fp32 feature: harmless
     err = "\n".join(l for l in res.stderr.splitlines() if "packed-fp32-ops" not in l)
     if res.returncode != 0:
-        raise RuntimeError("hipcc failed: " + " ".join(cmd) + "\n" + res.stdout + err)
+        raise RuntimeError("compiler failed: " + " ".join(cmd) + "\n" + res.stdout + err)
     if verbose and err.strip():
         print(err, file=sys.stderr)
 
 
+def host_command() -> list:
+    """The host module's compile line: it holds no device code, so the host compiler builds it."""
+    import torch
+
+    root = os.path.dirname(torch.__file__)
+    cxx = shutil.which("g++") or shutil.which("c++")
+    if not cxx:
+        raise RuntimeError("no host C++ compiler found; the host call module cannot be built")
+    inc = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
+           os.path.join(os.path.dirname(os.path.dirname(hipcc_path())), "include"), "/opt/rocm/include", sysconfig.get_paths()["include"]]
+    abi = int(torch._C._GLIBCXX_USE_CXX11_ABI)
+    return [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM", f"-D_GLIBCXX_USE_CXX11_ABI={abi}",
+            *(f"-I{d}" for d in inc if os.path.isdir(d)), HOST_SOURCE, "-o", HOST_PATH, "-L" + os.path.join(root, "lib"),
+            "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python"]
+
+
 def build_library(verbose: bool = True) -> str:
-    """One object per source (compiled side by side), then one link."""
+    """One object per source and the host module (compiled side by side), then one link."""
     os.makedirs(OBJ_DIR, exist_ok=True)
     hipcc = hipcc_path()
+    host_cmd = host_command()
+    if verbose:
+        print(" ".join(host_cmd), flush=True)
+    host_proc = subprocess.Popen(host_cmd, stdout=subprocess.PIPE, stderr=subprocess.PIPE, text=True)
     jobs = []
     for src, extra in SOURCES.items():
         obj = os.path.join(OBJ_DIR, os.path.splitext(os.path.basename(src))[0] + ".o")
@@ -75,6 +99,8 @@ def build_library(verbose: bool = True) -> str:
     if verbose:
         print(" ".join(cmd), flush=True)
     _finish(cmd, subprocess.run(cmd, capture_output=True, text=True), verbose)
+    out, err = host_proc.communicate()
+    _finish(host_cmd, subprocess.CompletedProcess(host_cmd, host_proc.returncode, out, err), verbose)
     return LIB_PATH
 
 

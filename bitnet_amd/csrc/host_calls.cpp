@@ -1,0 +1,290 @@
+// CPython entry points of the three calls a program makes per BitLinear -- BitLinearKernel.forward,
+// bitnet_int8xint2_linear and quant_input (gpu/model.py:21-75 of the reference) -- between torch
+// tensors and the C ABI of libbitlinear_hip.so.
+//
+// What bounds a small call is the host: the kernels of a one-token 2560 x 2560 forward take 3.5 us,
+// and issuing them from Python (three torch.empty, torch.cuda.current_stream, the argument checks
+// and the conversion of twelve ctypes arguments) took 15.4 us per call, back to back; from here it
+// takes 5.5 (8 tokens of 6912 -> 2560: 18.1 -> 8.8, two kernels).  The checks read the tensors' C++
+// objects, the workspaces are one caching-allocator block, the output is allocated without the
+// operator dispatcher, and the stream is read from torch's own thread-local state.  The functions
+// of the library are taken by address (bind), so this file links to torch only and serves
+// whichever libbitlinear_hip.so was opened.
+#include <Python.h>
+
+#include <ATen/hip/EmptyTensor.h>
+#include <ATen/hip/impl/HIPCachingAllocatorMasqueradingAsCUDA.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <cstdint>
+
+namespace {
+
+typedef void (*product_fn)(int8_t*, int8_t*, uint16_t*, uint16_t*, uint16_t*, int, int, int, void*);
+typedef int (*status_fn)();
+typedef const char* (*status_string_fn)(int);
+typedef int (*ws_num_fn)(int, int);
+typedef int (*quant_fn)(const void*, void*, void*, int, int, int, void*);
+typedef int (*forward_fn)(const void*, const void*, void*, const void*, void*, void*, int, int, int, int, void*);
+typedef int (*forward_seg_fn)(const void*, const void*, void*, const void*, const int*, int, void*, void*, int, int, int, int,
+                              void*);
+
+struct Bound {
+    product_fn product = nullptr;
+    status_fn last_status = nullptr;
+    status_string_fn status_string = nullptr;
+    ws_num_fn ws_num = nullptr;
+    quant_fn quant = nullptr;
+    forward_fn forward = nullptr;
+    forward_seg_fn forward_seg = nullptr;
+    PyObject* error = nullptr;  // BitLinearLibraryError
+} g_bound;
+
+const at::Tensor* tensor_of(PyObject* o) {
+    if (!THPVariable_Check(o)) {
+        PyErr_Format(PyExc_TypeError, "bitlinear: expected a tensor, got %s", Py_TYPE(o)->tp_name);
+        return nullptr;
+    }
+    return &THPVariable_Unpack(o);
+}
+
+bool check_device(std::initializer_list<const at::Tensor*> tensors) {
+    for (const at::Tensor* t : tensors) {
+        if (!t->is_cuda()) {
+            PyErr_SetString(PyExc_ValueError, "bitlinear: all tensors must live on the GPU (no CPU path exists)");
+            return false;
+        }
+        if (!t->is_contiguous()) {
+            PyErr_SetString(PyExc_ValueError, "bitlinear: tensors must be contiguous");
+            return false;
+        }
+    }
+    return true;
+}
+
+// rows of a [..., width] tensor; -1 with an exception set for a tensor without dimensions
+int64_t flat_rows(const at::Tensor& t) {
+    if (t.dim() < 1) {
+        PyErr_SetString(PyExc_IndexError, "bitlinear: activations need at least one dimension");
+        return -1;
+    }
+    int64_t m = 1;
+    for (int64_t d = 0; d + 1 < t.dim(); ++d) m *= t.size(d);
+    return m;
+}
+
+at::Tensor empty_like_rows(const at::Tensor& rows, int64_t width, at::ScalarType type) {
+    c10::SmallVector<int64_t, 5> sizes(rows.sizes().begin(), rows.sizes().end());
+    sizes.back() = width;
+    return at::Tensor(at::detail::empty_cuda(sizes, type, rows.device(), std::nullopt));
+}
+
+void* current_stream() { return (void*)c10::hip::getCurrentHIPStream().stream(); }
+
+PyObject* library_error(const char* entry, long long m, long long n, long long k, int status) {
+    PyErr_Format(g_bound.error, "%s(M=%lld, N=%lld, K=%lld): status %d (%s)", entry, m, n, k, status,
+                 g_bound.status_string(status));
+    return nullptr;
+}
+
+bool arg_count(Py_ssize_t got, Py_ssize_t want, const char* name) {
+    if (got == want) return true;
+    PyErr_Format(PyExc_TypeError, "%s: expected %zd arguments, got %zd", name, want, got);
+    return false;
+}
+
+// forward(input, weight, weight_scale, in_features, out_features, quant_mode, seg_ends)
+// seg_ends: None, or an int array that supports the buffer protocol
+PyObject* forward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    if (!arg_count(nargs, 7, "forward")) return nullptr;
+    const at::Tensor *x = tensor_of(args[0]), *w = x ? tensor_of(args[1]) : nullptr, *ws = w ? tensor_of(args[2]) : nullptr;
+    if (!ws || !check_device({x, w, ws})) return nullptr;
+    const long long K = PyLong_AsLongLong(args[3]), N = PyLong_AsLongLong(args[4]), mode = PyLong_AsLongLong(args[5]);
+    if (PyErr_Occurred()) return nullptr;
+    if (x->scalar_type() != at::kBFloat16) {
+        PyErr_SetString(PyExc_TypeError, "BitLinearKernel.forward expects bfloat16 activations");
+        return nullptr;
+    }
+    const int64_t M = flat_rows(*x);
+    if (M < 0) return nullptr;
+    if (x->size(-1) != K) {
+        PyErr_Format(PyExc_ValueError, "activation width %lld does not match in_features=%lld", (long long)x->size(-1), K);
+        return nullptr;
+    }
+    if (w->dim() != 2 || w->size(0) != N || w->size(1) != K / 4 || w->scalar_type() != at::kChar) {
+        PyErr_SetString(PyExc_ValueError, "weight must be int8 [out_features, in_features // 4] (the packed layout)");
+        return nullptr;
+    }
+    const c10::DeviceGuard guard(x->device());
+    at::Tensor out = empty_like_rows(*x, N, at::kBFloat16);
+    if (M == 0) return THPVariable_Wrap(std::move(out));
+    Py_buffer seg;
+    seg.buf = nullptr;
+    if (args[6] != Py_None && PyObject_GetBuffer(args[6], &seg, PyBUF_SIMPLE) != 0) return nullptr;
+    // the quantized rows and, behind them, their scales: one block that goes back to the allocator on return, as
+    // tensors do (reused by later work on the same stream)
+    const size_t q_bytes = ((size_t)M * (size_t)K + 255) & ~(size_t)255;
+    int st = 0;
+    {
+        const c10::DataPtr block = c10::hip::HIPCachingAllocatorMasqueradingAsCUDA::get()->allocate(q_bytes + 2 * (size_t)M);
+        char* q = (char*)block.get();
+        void* stream = current_stream();
+        Py_BEGIN_ALLOW_THREADS;
+        st = seg.buf ? g_bound.forward_seg(x->data_ptr(), w->data_ptr(), out.data_ptr(), ws->data_ptr(), (const int*)seg.buf,
+                                           (int)(seg.len / (Py_ssize_t)sizeof(int)), q, q + q_bytes, (int)M, (int)N, (int)K,
+                                           (int)mode, stream)
+                     : g_bound.forward(x->data_ptr(), w->data_ptr(), out.data_ptr(), ws->data_ptr(), q, q + q_bytes, (int)M,
+                                       (int)N, (int)K, (int)mode, stream);
+        Py_END_ALLOW_THREADS;
+    }
+    const bool segmented = seg.buf != nullptr;
+    if (segmented) PyBuffer_Release(&seg);
+    if (st) return library_error(segmented ? "bitlinear_forward_bf16_seg" : "bitlinear_forward_bf16", M, N, K, st);
+    return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
+// linear(input0, input1, s, ws, out)  -- out: a tensor or None
+PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    if (!arg_count(nargs, 5, "linear")) return nullptr;
+    const at::Tensor *a = tensor_of(args[0]), *w = a ? tensor_of(args[1]) : nullptr, *s = w ? tensor_of(args[2]) : nullptr,
+                     *ws = s ? tensor_of(args[3]) : nullptr;
+    if (!ws || !check_device({a, w, s, ws})) return nullptr;
+    if (a->scalar_type() != at::kChar || w->scalar_type() != at::kChar) {
+        PyErr_SetString(PyExc_TypeError, "input0 and input1 must be int8");
+        return nullptr;
+    }
+    if (s->scalar_type() != at::kBFloat16 || ws->scalar_type() != at::kBFloat16) {
+        PyErr_SetString(PyExc_TypeError, "s and ws must be bfloat16");
+        return nullptr;
+    }
+    const int64_t M = flat_rows(*a);
+    if (M < 0) return nullptr;
+    if (w->dim() < 2) {
+        PyErr_SetString(PyExc_IndexError, "bitlinear: the packed weight must be [N, K/4]");
+        return nullptr;
+    }
+    const int64_t N = w->size(0), K = w->size(1) * 4;
+    if (a->size(-1) != K) {
+        PyErr_Format(PyExc_ValueError, "activation width %lld does not match packed weight K=%lld", (long long)a->size(-1),
+                     (long long)K);
+        return nullptr;
+    }
+    if (s->numel() < M) {
+        PyErr_Format(PyExc_ValueError, "need one activation scale per row: %lld < %lld", (long long)s->numel(), (long long)M);
+        return nullptr;
+    }
+    if (ws->numel() < g_bound.ws_num((int)N, (int)K)) {
+        PyErr_SetString(PyExc_ValueError, "weight_scale has fewer slots than this shape uses");
+        return nullptr;
+    }
+    const c10::DeviceGuard guard(a->device());
+    at::Tensor out;
+    if (args[4] == Py_None) {
+        out = empty_like_rows(*a, N, at::kBFloat16);
+    } else {
+        const at::Tensor* o = tensor_of(args[4]);
+        if (!o) return nullptr;
+        if (o->scalar_type() != at::kBFloat16 || o->numel() != M * N || !o->is_contiguous() || !o->is_cuda()) {
+            PyErr_SetString(PyExc_ValueError, "out must be a contiguous bfloat16 GPU tensor of M x N elements");
+            return nullptr;
+        }
+        out = *o;
+    }
+    if (M > 0) {  // no token rows: nothing to launch
+        void* stream = current_stream();
+        int st = 0;
+        Py_BEGIN_ALLOW_THREADS;
+        g_bound.product((int8_t*)a->data_ptr(), (int8_t*)w->data_ptr(), (uint16_t*)out.data_ptr(), (uint16_t*)s->data_ptr(),
+                        (uint16_t*)ws->data_ptr(), (int)M, (int)N, (int)K, stream);
+        st = g_bound.last_status();
+        Py_END_ALLOW_THREADS;
+        if (st) return library_error("bitlinear_int8xint2", M, N, K, st);
+    }
+    if (args[4] != Py_None) {
+        Py_INCREF(args[4]);
+        return args[4];
+    }
+    return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
+// quant(input, mode) -> (q, s)
+PyObject* quant(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    if (!arg_count(nargs, 2, "quant")) return nullptr;
+    const at::Tensor* x = tensor_of(args[0]);
+    if (!x || !check_device({x})) return nullptr;
+    const long long mode = PyLong_AsLongLong(args[1]);
+    if (PyErr_Occurred()) return nullptr;
+    if (x->scalar_type() != at::kBFloat16) {
+        PyErr_SetString(PyExc_TypeError, "quant_input expects bfloat16");
+        return nullptr;
+    }
+    const int64_t M = flat_rows(*x);
+    if (M < 0) return nullptr;
+    const int64_t K = x->size(-1);
+    const c10::DeviceGuard guard(x->device());
+    at::Tensor q = empty_like_rows(*x, K, at::kChar), s = empty_like_rows(*x, 1, at::kBFloat16);
+    if (M > 0) {
+        void* stream = current_stream();
+        int st = 0;
+        Py_BEGIN_ALLOW_THREADS;
+        st = g_bound.quant(x->data_ptr(), q.data_ptr(), s.data_ptr(), (int)M, (int)K, (int)mode, stream);
+        Py_END_ALLOW_THREADS;
+        if (st) {
+            PyErr_Format(g_bound.error, "bitlinear_quant_absmax(M=%lld, K=%lld): status %d (%s)", (long long)M, (long long)K,
+                         st, g_bound.status_string(st));
+            return nullptr;
+        }
+    }
+    PyObject* pq = THPVariable_Wrap(std::move(q));
+    PyObject* ps = pq ? THPVariable_Wrap(std::move(s)) : nullptr;
+    PyObject* pair = ps ? PyTuple_Pack(2, pq, ps) : nullptr;
+    Py_XDECREF(pq);
+    Py_XDECREF(ps);
+    return pair;
+    END_HANDLE_TH_ERRORS
+}
+
+// bind(error_class, product, last_status, status_string, ws_num, quant, forward, forward_seg): the library's functions by
+// address
+PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    if (!arg_count(nargs, 8, "bind")) return nullptr;
+    void* fn[7];
+    for (int i = 0; i < 7; ++i) {
+        fn[i] = PyLong_AsVoidPtr(args[i + 1]);
+        if (!fn[i]) {
+            if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "bind: null function address");
+            return nullptr;
+        }
+    }
+    g_bound.product = (product_fn)fn[0];
+    g_bound.last_status = (status_fn)fn[1];
+    g_bound.status_string = (status_string_fn)fn[2];
+    g_bound.ws_num = (ws_num_fn)fn[3];
+    g_bound.quant = (quant_fn)fn[4];
+    g_bound.forward = (forward_fn)fn[5];
+    g_bound.forward_seg = (forward_seg_fn)fn[6];
+    Py_INCREF(args[0]);
+    Py_XSETREF(g_bound.error, args[0]);
+    Py_RETURN_NONE;
+}
+
+PyMethodDef methods[] = {
+    {"bind", (PyCFunction)(void*)bind, METH_FASTCALL, nullptr},
+    {"forward", (PyCFunction)(void*)forward, METH_FASTCALL, nullptr},
+    {"linear", (PyCFunction)(void*)linear, METH_FASTCALL, nullptr},
+    {"quant", (PyCFunction)(void*)quant, METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr},
+};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host_calls", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__host_calls() { return PyModule_Create(&module); }

@@ -127,3 +127,24 @@ def test_decoder_entry_argument_checks_need_no_gpu():
     assert lib.bitnet_rope_cache_tokens(None, None, None, None, None, None, None, 1, 8, 64, 4, 2, 128, None) == 2
     assert lib.bitnet_decode_step_begin(None, None, None, None, None, None, None, 1, 100, 250, 64, 128, None) == 1  # dim % 8
     assert lib.bitnet_decode_step_begin(None, None, None, None, None, None, None, 1, 100, 256, 64, 128, None) == 2
+
+
+def test_host_calls_refuse_bad_arguments_before_any_launch():
+    """The native call module checks its operands itself: CPU tensors, non-tensors and wrong argument counts raise here,
+    where no GPU exists."""
+    import torch
+
+    from bitnet_amd import bitlinear
+
+    if not os.path.exists(_lib.HOST_CALLS_PATH):
+        pytest.skip("not built")
+    mod = bitlinear.BitLinearKernel(128, 32, seg_ends=(16, 32))
+    x = torch.zeros(1, 128, dtype=torch.bfloat16)
+    q, s = torch.zeros(1, 128, dtype=torch.int8), torch.ones(1, dtype=torch.bfloat16)
+    for call in (lambda: mod(x), lambda: mod.quant_input(x), lambda: bitlinear.quant_input(x),
+                 lambda: bitlinear.bitnet_int8xint2_linear(q, mod.weight, s, mod.weight_scale)):
+        with pytest.raises(ValueError, match="must live on the GPU"):
+            call()
+    for call in (lambda: mod(None), lambda: bitlinear.quant_input([1.0]), lambda: _lib.host_calls().forward(x)):
+        with pytest.raises(TypeError):
+            call()
