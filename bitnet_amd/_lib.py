@@ -36,6 +36,8 @@ SIGNATURES = {
     "bitlinear_quant_absmax_rowsum": (_c_int, [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr]),
     "bitlinear_repacked_size": (ctypes.c_size_t, [_c_int, _c_int]),
     "bitlinear_repack": (_c_int, [_c_ptr, _c_ptr, _c_int, _c_int, _c_ptr]),
+    "bitlinear_pack_int2": (_c_int, [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr]),
+    "bitlinear_unpack_int2": (_c_int, [_c_ptr, _c_ptr, _c_int, _c_int, _c_ptr]),
     "bitlinear_forward_bf16": (
         _c_int,
         [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_ptr],
@@ -176,7 +178,8 @@ def host_calls():
         lib = load_library()
         mod.bind(BitLinearLibraryError, *(ctypes.cast(getattr(lib, name), _c_ptr).value for name in (
             "bitlinear_int8xint2", "bitlinear_last_status", "bitlinear_status_string", "bitlinear_ws_num",
-            "bitlinear_quant_absmax", "bitlinear_forward_bf16", "bitlinear_forward_bf16_seg")))
+            "bitlinear_quant_absmax", "bitlinear_forward_bf16", "bitlinear_forward_bf16_seg",
+            "bitlinear_pack_int2", "bitlinear_unpack_int2")))
         _host = mod
     return _host
 

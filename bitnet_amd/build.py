@@ -19,6 +19,7 @@ REPO_ROOT = os.path.dirname(PKG_DIR)
 SOURCES = {
     os.path.join(PKG_DIR, "csrc", "bitlinear_hip.hip"): [],
     os.path.join(PKG_DIR, "csrc", "decoder_ops.hip"): [],
+    os.path.join(PKG_DIR, "csrc", "pack.hip"): [],
     # keep the attention kernel's accumulators in the vector register file (see the file's header)
     os.path.join(PKG_DIR, "csrc", "attn_prefill.hip"): ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
 }

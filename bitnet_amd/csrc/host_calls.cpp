@@ -1,6 +1,6 @@
 // CPython entry points of the three calls a program makes per BitLinear -- BitLinearKernel.forward,
-// bitnet_int8xint2_linear and quant_input (gpu/model.py:21-75 of the reference) -- between torch
-// tensors and the C ABI of libbitlinear_hip.so.
+// bitnet_int8xint2_linear and quant_input (gpu/model.py:21-75 of the reference) -- and of the weight
+// layout converters (gpu/pack_weight.py), between torch tensors and the C ABI of libbitlinear_hip.so.
 //
 // What bounds a small call is the host: the kernels of a one-token 2560 x 2560 forward take 3.5 us,
 // and issuing them from Python (three torch.empty, torch.cuda.current_stream, the argument checks
@@ -14,12 +14,16 @@
 
 #include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/impl/HIPCachingAllocatorMasqueradingAsCUDA.h>
+#include <ATen/ops/empty.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
+#include <pybind11/gil.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cstdint>
+#include <mutex>
+#include <vector>
 
 namespace {
 
@@ -31,6 +35,8 @@ typedef int (*quant_fn)(const void*, void*, void*, int, int, int, void*);
 typedef int (*forward_fn)(const void*, const void*, void*, const void*, void*, void*, int, int, int, int, void*);
 typedef int (*forward_seg_fn)(const void*, const void*, void*, const void*, const int*, int, void*, void*, int, int, int, int,
                               void*);
+typedef int (*pack_fn)(const void*, void*, void*, int, int, void*);
+typedef int (*unpack_fn)(const void*, void*, int, int, void*);
 
 struct Bound {
     product_fn product = nullptr;
@@ -40,6 +46,8 @@ struct Bound {
     quant_fn quant = nullptr;
     forward_fn forward = nullptr;
     forward_seg_fn forward_seg = nullptr;
+    pack_fn pack = nullptr;
+    unpack_fn unpack = nullptr;
     PyObject* error = nullptr;  // BitLinearLibraryError
 } g_bound;
 
@@ -252,12 +260,103 @@ PyObject* quant(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     END_HANDLE_TH_ERRORS
 }
 
-// bind(error_class, product, last_status, status_string, ws_num, quant, forward, forward_seg): the library's functions by
-// address
+// Pinned words that a kernel can raise a flag in: reading one after the stream has got there costs no copy.  A caller
+// takes a word for the length of its call; the list grows to the largest number of calls that were under way at once.
+class PinnedFlag {
+public:
+    PinnedFlag() {
+        std::lock_guard<std::mutex> hold(mutex());
+        if (words().empty())
+            word_ = at::empty({1}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+        else {
+            word_ = std::move(words().back());
+            words().pop_back();
+        }
+        *value() = 0;
+    }
+    ~PinnedFlag() {
+        std::lock_guard<std::mutex> hold(mutex());
+        words().push_back(std::move(word_));
+    }
+    volatile int32_t* value() const { return (volatile int32_t*)word_.data_ptr(); }
+
+private:
+    static std::mutex& mutex() {
+        static std::mutex m;
+        return m;
+    }
+    static std::vector<at::Tensor>& words() {  // lives until the process ends: torch's allocator may be gone before it
+        static auto* w = new std::vector<at::Tensor>;
+        return *w;
+    }
+    at::Tensor word_;
+};
+
+// pack(weight): ternary int8 [N, K] on the GPU, contiguous, N % 16 == 0 and K % 32 == 0 -> packed int8 [N, K / 4].
+// Waits for the stream, since a weight outside {-1, 0, 1} is the caller's error and is reported here.
+PyObject* pack(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    if (!arg_count(nargs, 1, "pack")) return nullptr;
+    const at::Tensor* w = tensor_of(args[0]);
+    if (!w || !check_device({w})) return nullptr;
+    if (w->dim() != 2 || w->scalar_type() != at::kChar) {
+        PyErr_SetString(PyExc_TypeError, "pack: expected int8 [N, K]");
+        return nullptr;
+    }
+    const int64_t N = w->size(0), K = w->size(1);
+    const c10::DeviceGuard guard(w->device());
+    at::Tensor out = empty_like_rows(*w, K / 4, at::kChar);
+    int st = 0;
+    bool bad = false;
+    {
+        const PinnedFlag flag;
+        const c10::hip::HIPStream stream = c10::hip::getCurrentHIPStream();
+        pybind11::gil_scoped_release no_gil;
+        st = g_bound.pack(w->data_ptr(), out.data_ptr(), (void*)flag.value(), (int)N, (int)K, (void*)stream.stream());
+        if (!st) {
+            stream.synchronize();
+            bad = *flag.value() != 0;
+        }
+    }
+    if (st) return library_error("bitlinear_pack_int2", 1, N, K, st);
+    if (bad) {
+        PyErr_SetString(PyExc_ValueError, "weights must be ternary (-1, 0, +1)");
+        return nullptr;
+    }
+    return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
+// unpack(packed, N, K): the inverse; packed holds N * K / 4 bytes
+PyObject* unpack(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    if (!arg_count(nargs, 3, "unpack")) return nullptr;
+    const at::Tensor* p = tensor_of(args[0]);
+    if (!p || !check_device({p})) return nullptr;
+    const long long N = PyLong_AsLongLong(args[1]), K = PyLong_AsLongLong(args[2]);
+    if (PyErr_Occurred()) return nullptr;
+    if (p->element_size() != 1 || N < 0 || K < 0 || p->numel() * 4 != N * K) {
+        PyErr_SetString(PyExc_ValueError, "unpack: expected N * K / 4 bytes");
+        return nullptr;
+    }
+    const c10::DeviceGuard guard(p->device());
+    at::Tensor out(at::detail::empty_cuda({N, K}, at::kChar, p->device(), std::nullopt));
+    void* stream = current_stream();
+    int st = 0;
+    Py_BEGIN_ALLOW_THREADS;
+    st = g_bound.unpack(p->data_ptr(), out.data_ptr(), (int)N, (int)K, stream);
+    Py_END_ALLOW_THREADS;
+    if (st) return library_error("bitlinear_unpack_int2", 1, N, K, st);
+    return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
+}
+
+// bind(error_class, product, last_status, status_string, ws_num, quant, forward, forward_seg, pack, unpack): the
+// library's functions by address
 PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
-    if (!arg_count(nargs, 8, "bind")) return nullptr;
-    void* fn[7];
-    for (int i = 0; i < 7; ++i) {
+    if (!arg_count(nargs, 10, "bind")) return nullptr;
+    void* fn[9];
+    for (int i = 0; i < 9; ++i) {
         fn[i] = PyLong_AsVoidPtr(args[i + 1]);
         if (!fn[i]) {
             if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "bind: null function address");
@@ -271,6 +370,8 @@ PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     g_bound.quant = (quant_fn)fn[4];
     g_bound.forward = (forward_fn)fn[5];
     g_bound.forward_seg = (forward_seg_fn)fn[6];
+    g_bound.pack = (pack_fn)fn[7];
+    g_bound.unpack = (unpack_fn)fn[8];
     Py_INCREF(args[0]);
     Py_XSETREF(g_bound.error, args[0]);
     Py_RETURN_NONE;
@@ -281,6 +382,8 @@ PyMethodDef methods[] = {
     {"forward", (PyCFunction)(void*)forward, METH_FASTCALL, nullptr},
     {"linear", (PyCFunction)(void*)linear, METH_FASTCALL, nullptr},
     {"quant", (PyCFunction)(void*)quant, METH_FASTCALL, nullptr},
+    {"pack", (PyCFunction)(void*)pack, METH_FASTCALL, nullptr},
+    {"unpack", (PyCFunction)(void*)unpack, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host_calls", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

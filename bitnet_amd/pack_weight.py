@@ -9,15 +9,24 @@ For logical W[n, k] (ternary, stored as code w + 2):
 i.e. byte (e % 4) of the little-endian word, bits 2 * (e // 4).  The flat byte
 buffer is therefore ordered [nb][kb][r // 8][h][r % 8][e % 4], each byte
 holding the four codes e // 4 = 0..3 from its low bits up, and is viewed as
-int8 [N, K // 4].  Both directions are pure reshapes/permutes, so they run on
-whatever device the tensor lives on.
+int8 [N, K // 4].  On the GPU both directions are one HIP kernel
+(csrc/pack.hip); for host tensors, and inputs that are not int8, they are pure
+reshapes/permutes in torch.
 """
 import torch
+
+from . import _lib
 
 
 def _check_shape(N: int, K: int):
     if N % 16 or K % 32:
         raise ValueError(f"need N % 16 == 0 and K % 32 == 0, got {N}x{K}")
+
+
+def _aligned(t: torch.Tensor) -> torch.Tensor:
+    """Contiguous, at an address the kernels' 16-byte accesses take."""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
 def convert_weight_int8_to_int2(weight: torch.Tensor, keep_device: bool = False) -> torch.Tensor:
@@ -28,6 +37,9 @@ def convert_weight_int8_to_int2(weight: torch.Tensor, keep_device: bool = False)
     w = torch.as_tensor(weight)
     N, K = w.shape
     _check_shape(N, K)
+    if w.is_cuda and w.dtype == torch.int8 and w.numel():
+        packed = _lib.host_calls().pack(_aligned(w))
+        return packed if keep_device else packed.cpu()
     if w.numel() and (int(w.min()) < -1 or int(w.max()) > 1):
         raise ValueError("weights must be ternary (-1, 0, +1)")
     q = (w.to(torch.int16) + 2).to(torch.uint8)
@@ -45,6 +57,8 @@ def convert_weight_int2_to_int8(packed: torch.Tensor, N: int = None, K: int = No
     N = N or p.shape[0]
     K = K or p.shape[1] * 4
     _check_shape(N, K)
+    if p.is_cuda and p.element_size() == 1 and p.numel() and p.numel() * 4 == N * K:
+        return _lib.host_calls().unpack(_aligned(p), N, K)
     b = p.view(torch.uint8).reshape(N // 16, K // 32, 2, 2, 8, 4)  # nb, kb, r_hi, h, r_lo, e_lo
     codes = torch.stack([(b >> (2 * i)) & 3 for i in range(4)], dim=-1)  # ..., e_lo, e_hi
     codes = codes.permute(0, 2, 4, 1, 3, 6, 5)  # nb, r_hi, r_lo, kb, h, e_hi, e_lo

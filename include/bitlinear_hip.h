@@ -165,6 +165,20 @@ int bitlinear_repack(const int8_t* packed_ref, void* packed_out, int N, int K,
                      void* stream);
 
 /*
+ * The reference packer (gpu/pack_weight.py:76-98) and its inverse on the
+ * device: ternary int8 [N, K] row-major <-> packed int8 [N, K/4].  N % 16 == 0,
+ * K % 32 == 0, both buffers 16-byte aligned.  A weight outside {-1, 0, 1}
+ * makes bitlinear_pack_int2 store 1 to *bad_flag (any memory the device can
+ * write, for instance pinned host memory); it is not written otherwise, so the
+ * caller clears it before the call and reads it after the stream has got there.
+ * Unpacking gives code - 2, i.e. -2 for the code the packer never writes.
+ */
+int bitlinear_pack_int2(const int8_t* ternary, int8_t* packed, int32_t* bad_flag,
+                        int N, int K, void* stream);
+int bitlinear_unpack_int2(const int8_t* packed, int8_t* ternary, int N, int K,
+                          void* stream);
+
+/*
  * BitLinearKernel.forward (gpu/model.py:73-75) in one call: quantizer (mode
  * as above), product and epilogue.  While the activation block is small
  * (M * K <= 16384 elements) this is ONE kernel: every workgroup (or every wave

@@ -1474,3 +1474,27 @@ def test_flag_round_trip_probe_completes_and_checks_its_arguments():
     assert lib.bitlinear_probe_flag_roundtrip(P(flags), 3, 3, 10, P(gave_up), None) == 4
     assert lib.bitlinear_probe_flag_roundtrip(P(flags), 0, 1, 0, P(gave_up), None) == 4
     assert lib.bitlinear_probe_flag_roundtrip(None, 0, 1, 10, P(gave_up), None) == 2
+
+
+@pytest.mark.parametrize("n,k", [(16, 32), (16, 256), (48, 288), (2560, 2560), (32, 6912), (1040, 3200)])
+def test_layout_converters_on_the_device_equal_the_host_ones(n, k):
+    """Both directions against the torch closed form on the CPU, an input at an odd address, the code the packer never
+    writes, and a weight outside the ternary range at either end of the matrix."""
+    rng = np.random.default_rng(n + k)
+    w = torch.from_numpy(rng.integers(-1, 2, (n, k)).astype(np.int8))
+    want = pack_weight.convert_weight_int8_to_int2(w)
+    odd = torch.empty(n * k + 1, dtype=torch.int8, device="cuda")[1:].view(n, k)
+    odd.copy_(w)
+    for wd in (w.cuda(), odd, w.cuda().t().contiguous().t()):
+        got = pack_weight.convert_weight_int8_to_int2(wd, keep_device=True)
+        assert got.is_cuda and torch.equal(got.cpu(), want)
+        assert torch.equal(pack_weight.convert_weight_int8_to_int2(wd), want)
+    assert torch.equal(pack_weight.convert_weight_int2_to_int8(want.cuda()).cpu(), w)
+    raw = torch.from_numpy(rng.integers(-128, 128, (n, k // 4)).astype(np.int8))
+    assert torch.equal(pack_weight.convert_weight_int2_to_int8(raw.cuda()).cpu(), pack_weight.convert_weight_int2_to_int8(raw))
+    for r, c, v in ((0, 0, 2), (n - 1, k - 1, -2), (n - 1, 0, -128), (0, k - 1, 127)):
+        bad = w.cuda()
+        bad[r, c] = v
+        with pytest.raises(ValueError, match="ternary"):
+            pack_weight.convert_weight_int8_to_int2(bad, keep_device=True)
+    assert torch.equal(pack_weight.convert_weight_int8_to_int2(w.cuda(), keep_device=True).cpu(), want)
