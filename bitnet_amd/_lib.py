@@ -96,6 +96,14 @@ SIGNATURES = {
         [_c_ptr, _c_ptr, ctypes.c_float, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr,
          _c_int, _c_int, _c_int, _c_ptr],
     ),
+    "bitnet_decode_stack_workspace_bytes": (ctypes.c_longlong, [_c_int] * 8),
+    "bitnet_decode_stack_reset": (_c_int, [_c_ptr] + [_c_int] * 8 + [_c_ptr]),
+    "bitnet_decode_stack_error_offset": (_c_int, []),
+    "bitnet_decode_stack": (_c_int, [_c_ptr] * 6 + [_c_int] * 10 + [_c_ptr]),
+    "bitlinear_scale_runs": (
+        _c_int,
+        [_c_int, _c_int, ctypes.POINTER(_c_int), _c_int, ctypes.POINTER(_c_int), ctypes.POINTER(ctypes.c_uint32)],
+    ),
     "bitnet_lm_head_workgroups": (_c_int, [_c_int]),
     "bitnet_lm_head_set_kernel": (_c_int, [_c_int]),
     "bitlinear_set_tuning": (_c_int, [_c_int, _c_int, _c_int, _c_int]),

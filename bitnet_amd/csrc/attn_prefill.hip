@@ -13,30 +13,10 @@
 #include <math.h>
 #include <stdint.h>
 
+#include "attn_device.h"
 #include "bitnet_decoder_ops.h"
 
 namespace {
-
-typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-typedef float v4f __attribute__((ext_vector_type(4)));
-typedef unsigned v4u __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef float f32x2_t __attribute__((ext_vector_type(2)));
-
-constexpr int kHeadDim = 128;
-
-__device__ __forceinline__ float bf16f(uint32_t bits16) { return __uint_as_float(bits16 << 16); }
-// fp32 -> bf16, round to nearest even, NaN kept: the same expression as the decode-step kernel's
-__device__ __forceinline__ uint16_t to_bf16(float f) {
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return 0x7fc0;
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (uint16_t)(u >> 16);
-}
-__device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {  // round to nearest even, one instruction on gfx950
-    const f32x2_t v = {lo, hi};
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
-}
 
 // Rotary embedding and cache write for a block of new tokens (a prompt): one workgroup per
 // token.  Items are (head, pair) of the token's q | k | v row; q heads are rotated into q_out,
@@ -91,17 +71,7 @@ __global__ __launch_bounds__(kRopeThreads) void rope_cache_tokens_kernel(
 //   lane (c, g4) then holds, for token c, dims 32 g4 + 8 j + t: eight contiguous dims per j.
 // Online softmax per 32 positions: the running maximum of a token is agreed between its four lanes
 // (c, c + 16, c + 32, c + 48) with two lane permutes; the sums stay per lane until the end.
-// Workgroup barrier that orders LDS traffic only (__syncthreads() would also wait for the global
-// loads in flight).
-__device__ __forceinline__ void lds_barrier() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
 constexpr int kApRowBytes = kHeadDim * 2 + 16;  // padded LDS row: the 16 rows of a K operand read spread over all banks
-__device__ __forceinline__ float xor_lane_f32(float v, int lane, int mask) {
-    return __int_as_float(__builtin_amdgcn_ds_bpermute((lane ^ mask) << 2, __float_as_int(v)));
-}
 
 template <int G>
 __global__ __launch_bounds__(64 * G) void attn_prefill_kernel(
@@ -204,8 +174,7 @@ __global__ __launch_bounds__(64 * G) void attn_prefill_kernel(
             }
         }
         float mx = fmaxf(fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3])), fmaxf(fmaxf(sc[4], sc[5]), fmaxf(sc[6], sc[7])));
-        mx = fmaxf(mx, xor_lane_f32(mx, lane, 16));
-        mx = fmaxf(mx, xor_lane_f32(mx, lane, 32));
+        mx = over_rows(mx, [](float a, float b) { return fmaxf(a, b); });
         const float m_new = fmaxf(m_run, mx);  // finite from the first step on: position 0 is visible to every token
         const float m2 = m_new * c2;
         float p[8], psum = 0.0f;
@@ -255,8 +224,7 @@ __global__ __launch_bounds__(64 * G) void attn_prefill_kernel(
         lds_barrier();
     }
 
-    float l_tot = l_run + xor_lane_f32(l_run, lane, 16);
-    l_tot += xor_lane_f32(l_tot, lane, 32);
+    const float l_tot = over_rows(l_run, [](float a, float b) { return a + b; });
     const float inv = 1.0f / l_tot;
     if (t0 + c < T) {
         uint16_t* orow = out + ((size_t)b * T + t0 + c) * n_heads * kHeadDim + (size_t)head * kHeadDim + 32 * g4;
@@ -281,12 +249,6 @@ __global__ __launch_bounds__(64 * G) void attn_prefill_kernel(
 // the slice at a time and does scores, softmax and P.V for the G query heads (columns c < G of the
 // 16-column tiles) entirely in registers; the waves' (maximum, sum, outputs) are combined through
 // LDS once.  No score buffer, no barrier between scores, softmax and P.V.
-constexpr int kDfRecUnits = kHeadDim + 2;  // record of one (sequence, kv head, split, head): 128 outputs, maximum, sum,
-                                            // each an 8-byte unit (value, tag of the call that wrote it)
-constexpr int kDfSpinLimit = 1 << 16;       // polls of the merging workgroup before it gives up (see the merge below)
-constexpr int kDfMaxSplits = 16;
-constexpr int kDfMaxWaves = 8;
-
 // ROWS: the rotation's cos / sin values of every sequence's position come as a ready row
 // (rope_rows[b] = cos[64] | sin[64], written once per step by decode_step_begin_kernel) instead of
 // from the tables at an index that has to be loaded first: one memory round trip less in front of
@@ -422,95 +384,12 @@ __global__ __launch_bounds__(kDfMaxWaves * 64) void attn_decode_flash_kernel(
         if (c < G) t = *(const uint4*)(&qb[c][kk * 32 + g4 * 8]);
         qa[kk] = __builtin_bit_cast(v8bf, t);
     }
-    v4f o_acc[8];
-#pragma unroll
-    for (int t = 0; t < 8; ++t) o_acc[t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
-    float m_run = -INFINITY, l_run = 0.0f;
-    const float scale = 0.08838834764831845f;           // 128^-0.5
-    const float c2 = scale * 1.4426950408889634f;        // * log2(e): the softmax runs in base 2
+    DfState st;
     for (int blk = blk0; blk <= pblk; blk += blk_stride) {
         if (blk != blk0) load_rows(blk);
-        // the new token's own row is not in the cache yet for this kernel's loads: it comes from LDS
-        if (blk == pblk) {
-#pragma unroll
-            for (int bi = 0; bi < 2; ++bi)
-                if (blk * 32 + bi * 16 + c == p) {
-#pragma unroll
-                    for (int kk = 0; kk < 4; ++kk) kb[bi][kk] = *(const v4u*)(&knew[kk * 32 + g4 * 8]);
-                }
-            // V rows behind the position are cleared: their probability is zero, but whatever the
-            // cache holds there (it may never have been written) must not reach the product as 0 x NaN
-#pragma unroll
-            for (int jj = 0; jj < 8; ++jj) {
-                const int r = blk * 32 + (jj & 3) + (jj >> 2) * 16 + 4 * g4;
-                if (r == p) vb[jj] = *(const v4u*)(&vnew[c * 8]);
-                if (r > p) vb[jj] = v4u{0u, 0u, 0u, 0u};
-            }
-        }
-        float sc[8];
-#pragma unroll
-        for (int bi = 0; bi < 2; ++bi) {
-            v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int kk = 0; kk < 4; ++kk)
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, kb[bi][kk]), qa[kk], acc, 0, 0, 0);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int pos = blk * 32 + bi * 16 + 4 * g4 + j;
-                sc[bi * 4 + j] = pos <= p ? acc[j] : -INFINITY;
-            }
-        }
-        float mx = fmaxf(fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3])), fmaxf(fmaxf(sc[4], sc[5]), fmaxf(sc[6], sc[7])));
-        mx = fmaxf(mx, xor_lane_f32(mx, lane, 16));
-        mx = fmaxf(mx, xor_lane_f32(mx, lane, 32));
-        const float m_new = fmaxf(m_run, mx);  // finite: the block's first row is visible (32 blk <= p)
-        const float m2 = m_new * c2;
-        float pr[8], psum = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            pr[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[i], c2, -m2));
-            psum += pr[i];
-        }
-        if (__builtin_amdgcn_ballot_w64(m_new != m_run) != 0) {
-            const float alpha = __builtin_amdgcn_exp2f(__builtin_fmaf(m_run, c2, -m2));
-            l_run *= alpha;
-#pragma unroll
-            for (int t = 0; t < 8; ++t)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) o_acc[t][j] *= alpha;
-            m_run = m_new;
-        }
-        l_run += psum;
-        v4u pw;
-        pw.x = pack_bf16x2(pr[0], pr[1]);
-        pw.y = pack_bf16x2(pr[2], pr[3]);
-        pw.z = pack_bf16x2(pr[4], pr[5]);
-        pw.w = pack_bf16x2(pr[6], pr[7]);
-        const v8bf pb = __builtin_bit_cast(v8bf, pw);
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            const uint32_t sel = (t & 1) ? 0x07060302u : 0x05040100u;
-            v4u va;
-            va.x = __builtin_amdgcn_perm(vb[1][t >> 1], vb[0][t >> 1], sel);
-            va.y = __builtin_amdgcn_perm(vb[3][t >> 1], vb[2][t >> 1], sel);
-            va.z = __builtin_amdgcn_perm(vb[5][t >> 1], vb[4][t >> 1], sel);
-            va.w = __builtin_amdgcn_perm(vb[7][t >> 1], vb[6][t >> 1], sel);
-            o_acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, va), pb, o_acc[t], 0, 0, 0);
-        }
+        df_block(kb, vb, qa, knew, vnew, blk, p, lane, st);
     }
-    // the wave's result for head c (lanes c < G): maximum, sum over its positions, 32 outputs per lane
-    float l_tot = l_run + xor_lane_f32(l_run, lane, 16);
-    l_tot += xor_lane_f32(l_tot, lane, 32);
-    if (c < G) {
-        if (g4 == 0) {
-            part_m[wave][c] = m_run;  // -inf, and a sum of 0, for a wave without visible positions
-            part_l[wave][c] = l_tot;
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int t = 0; t < 8; ++t) part_o[wave][c][32 * g4 + 8 * j + t] = o_acc[t][j];
-    }
+    df_wave_result<G>(st, lane, part_o[wave], part_m[wave], part_l[wave]);
     __syncthreads();
 
     uint16_t* orow = out + (size_t)b * n_heads * kHeadDim + (size_t)(kvh * G) * kHeadDim;
@@ -521,35 +400,7 @@ __global__ __launch_bounds__(kDfMaxWaves * 64) void attn_decode_flash_kernel(
     // acknowledged, device-scope counter, loads" this saves one of the three trips across the chip.
     unsigned long long* rec = (unsigned long long*)workspace + ((size_t)(b * n_kv_heads + kvh) * nsplit) * G * kDfRecUnits;
     const unsigned long long tag = (unsigned long long)(unsigned)(epoch + 1) << 32;
-    for (int hh = wave; hh < G; hh += nwaves) {
-        float mx = -INFINITY;
-        for (int k = 0; k < nwaves; ++k) mx = fmaxf(mx, part_m[k][hh]);
-        float o0 = 0.0f, o1 = 0.0f, l = 0.0f;
-        for (int k = 0; k < nwaves; ++k) {
-            const float lk = part_l[k][hh];
-            if (lk > 0.0f) {
-                const float w = __builtin_amdgcn_exp2f((part_m[k][hh] - mx) * c2);
-                l += lk * w;
-                o0 += w * part_o[k][hh][2 * lane];
-                o1 += w * part_o[k][hh][2 * lane + 1];
-            }
-        }
-        if (nact == 1) {
-            const float is = 1.0f / l;
-            *(uint32_t*)(orow + hh * kHeadDim + 2 * lane) = (uint32_t)to_bf16(o0 * is) | ((uint32_t)to_bf16(o1 * is) << 16);
-        } else {
-            unsigned long long* r = rec + ((size_t)sp * G + hh) * kDfRecUnits;
-            __hip_atomic_store(r + 2 * lane, tag | __float_as_uint(o0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(r + 2 * lane + 1, tag | __float_as_uint(o1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (lane == 0) {
-                __hip_atomic_store(r + kHeadDim, tag | __float_as_uint(mx * scale), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // in units of the scaled scores
-                __hip_atomic_store(r + kHeadDim + 1, tag | __float_as_uint(l), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-        }
-    }
-    if (!merger) return;
-
-    // The merge, eight splits at a time: all units of a batch are requested together and requested
+    // The last active split merges, eight splits at a time: all units of a batch are requested together and requested
     // again while one of them still carries an older tag.  Every split polled was dispatched before
     // this workgroup and writes its record without waiting for anything, so the poll is expected to
     // end after a few rounds; that order of dispatch is observed behaviour, not something the
@@ -557,58 +408,19 @@ __global__ __launch_bounds__(kDfMaxWaves * 64) void attn_decode_flash_kernel(
     // poll is therefore bounded, and a poll that runs out is not papered over: the head's output row
     // becomes NaN and the workspace's error word is set (it stays set; the host reads it, see
     // bitnet_attn_decode_error_index).
-    constexpr int kBatch = 8;
     for (int hh = wave; hh < G; hh += nwaves) {
-        float mx = -INFINITY, l = 0.0f, o0 = 0.0f, o1 = 0.0f;
-        bool gave_up = false;
-        for (int k0 = 0; k0 < nact; k0 += kBatch) {
-            unsigned long long um[kBatch], ul[kBatch], u0[kBatch], u1[kBatch];
-#pragma unroll
-            for (int k = 0; k < kBatch; ++k) um[k] = ul[k] = u0[k] = u1[k] = 0ull;
-            bool complete = false;
-            for (int spin = 0; spin < spin_limit; ++spin) {
-                bool ok = true;
-#pragma unroll
-                for (int k = 0; k < kBatch; ++k) {
-                    const unsigned long long* r = rec + ((size_t)((k0 + k) < nact ? (k0 + k) : k0) * G + hh) * kDfRecUnits;
-                    um[k] = __hip_atomic_load(r + kHeadDim, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    ul[k] = __hip_atomic_load(r + kHeadDim + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    u0[k] = __hip_atomic_load(r + 2 * lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    u1[k] = __hip_atomic_load(r + 2 * lane + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                }
-#pragma unroll
-                for (int k = 0; k < kBatch; ++k)
-                    ok = ok && ((um[k] & ul[k] & u0[k] & u1[k]) >> 32) == (tag >> 32) && ((um[k] | ul[k] | u0[k] | u1[k]) >> 32) == (tag >> 32);
-                if (__builtin_amdgcn_ballot_w64(!ok) == 0) {
-                    complete = true;
-                    break;
-                }
-            }
-            gave_up = gave_up || !complete;
-            float bm = mx;
-#pragma unroll
-            for (int k = 0; k < kBatch; ++k)
-                if (k0 + k < nact) bm = fmaxf(bm, __uint_as_float((unsigned)um[k]));
-            const float wold = l > 0.0f ? __expf(mx - bm) : 0.0f;
-            l *= wold;
-            o0 *= wold;
-            o1 *= wold;
-            mx = bm;
-#pragma unroll
-            for (int k = 0; k < kBatch; ++k) {
-                const float lk = __uint_as_float((unsigned)ul[k]);
-                if (k0 + k < nact && lk > 0.0f) {
-                    const float w = __expf(__uint_as_float((unsigned)um[k]) - mx);
-                    l += lk * w;
-                    o0 += w * __uint_as_float((unsigned)u0[k]);
-                    o1 += w * __uint_as_float((unsigned)u1[k]);
-                }
-            }
+        DfPartial h = df_combine<G>(part_o, part_m, part_l, hh, nwaves, lane);
+        if (nact > 1 && !merger) {
+            df_store_record(rec + ((size_t)sp * G + hh) * kDfRecUnits, tag, h, lane);
+            continue;
         }
-        const float is = gave_up ? __builtin_nanf("") : 1.0f / l;
-        *(uint32_t*)(orow + hh * kHeadDim + 2 * lane) = (uint32_t)to_bf16(o0 * is) | ((uint32_t)to_bf16(o1 * is) << 16);
+        bool gave_up = false;
+        if (nact > 1) h = df_merge<G>(rec, nact, hh, tag, h, lane, spin_limit, gave_up);
+        const float is = gave_up ? __builtin_nanf("") : 1.0f / h.l;
+        *(uint32_t*)(orow + hh * kHeadDim + 2 * lane) = (uint32_t)to_bf16(h.o0 * is) | ((uint32_t)to_bf16(h.o1 * is) << 16);
         if (gave_up && lane == 0) __hip_atomic_store(err_word, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+    if (!merger) return;
     __syncthreads();  // every wave has read its records
     if (tid == 0) epochs[b * n_kv_heads + kvh] = epoch + 1;
 }

@@ -1,0 +1,1083 @@
+// The decoder layers of one decode step (gpu/model.py:214-245 of the reference, one new token per
+// sequence, every layer) in ONE kernel.
+//
+// What bounds a decode step as a chain of launches is the boundary between two of them, not bytes: at
+// one sequence of the 2B decoder a layer is 17 MB of weights, 3.4 us at the card's copy rate, and five
+// dependent kernels, 26 us -- each pays for its launch (1.6 us, empty), for the trip of the activations
+// to memory and back (1.2 us) and for the weights' latency that nothing before it could hide.  Here one
+// workgroup per CU stays for the whole step.  A product's weights are in LDS before its activations
+// exist, and outputs go to their readers directly: every value is written through to memory once, and
+// readers poll for the values themselves.  Nobody waits for an acknowledgement, a counter or a launch;
+// such a hand-over measures 1.4 us, readers' barrier included.  30 layers at 512 positions, us:
+//                        one sequence   two
+//   launches                     755    875
+//   this kernel                  516    621
+// With more sequences the redundant part grows, every workgroup of a product normalises and quantizes
+// the rows of all tokens by itself: at three both take the same time, so two is where the range ends.
+//
+// Hand-over buffers.  Every (layer, step) has buffers of its own, in two sets that alternate between
+// launches; a launch fills the other set with a value that no result can have (bf16 0xffff, a NaN that
+// results are kept from having), so "not that value" means "written".  No buffer is reused within a
+// launch, so nothing has to be protected from being overwritten.
+//
+// Tasks.  A layer is a list of tasks in dependency order -- 32 output rows of wqkv, or one (sequence,
+// kv head, split) of the attention, or 32 gated outputs of w13 ... -- and all layers are one long list.
+// A task needs only tasks in front of it.  Workgroups take the next task of the list whenever they
+// finish one ("ticket mode"): every task in front of a taken one is finished or in the hands of a
+// running workgroup, so the kernel ends with any number of workgroups resident, whatever else occupies
+// the GPU.  Taking tickets costs one contended atomic per task; once all workgroups of the grid have
+// been seen to run (each takes its first ticket from the counter, and the one that takes ticket
+// grid - 1 says so), no counter is needed: ticket t + grid follows ticket t ("static mode").  Exactly
+// one of the modes is decided per launch, by compare-and-swap; who waits for the decision longer than
+// some 50 us decides for ticket mode.
+//
+// Waves.  Between the arrival of its inputs and its outputs a task is bound by the instructions that its
+// SIMDs issue and by chains of dependent ones, so there is ONE computing wave per SIMD: a second one
+// repeats every step that is not per element (reductions, scales, addresses), and eight waves of 320
+// values took 1.9 us where four of 640 take 1.3.  A fifth wave takes the tickets, looks up what a task
+// consists of and brings its weights into LDS, in pieces of 1 KB without a register in between, up to
+// two tasks ahead; its waits for memory hold up nobody.  Loads of 4 bytes per lane, the width in which
+// MFMA operands unpack, cost an instruction each and took 2-3 us a task when the computing waves did
+// them.  The waves tell each other what they have done by numbers in LDS: the hardware's barrier would
+// have to include the wave that fetches.
+//
+// The arithmetic is that of the kernels a step consists of otherwise, value for value (the shared
+// definitions are in bitlinear_device.h and attn_device.h): both give the same bits.
+
+#include <hip/hip_runtime.h>
+#include <stddef.h>
+#include <stdint.h>
+
+#include <type_traits>
+
+#include "attn_device.h"
+#include "bitlinear_device.h"
+#include "bitlinear_hip.h"
+#include "bitnet_decoder_ops.h"
+#include "host_util.h"
+
+namespace {
+
+constexpr int kStWaves = 4;
+constexpr int kStLanes = kStWaves * 64;   // of the computing waves
+constexpr int kStThreads = kStLanes + 64;  // and the wave that fetches
+constexpr int kStUpwD = 10;       // 64-wide k-steps per wave of a product over the model width: up to 2560
+constexpr int kStUpwF = 27;       // ... over the feed-forward width: up to 6912
+constexpr int kStMaxTokens = 2;  // (see above)
+constexpr int kStMaxG = 8;        // query heads per kv head
+constexpr int kStSpinLimit = 1 << 19;   // polls (0.7 us each) before a wait gives up
+constexpr int kStModePolls = 64;        // polls before the mode is decided without all workgroups
+constexpr int kSc1 = kPollPolicy;       // device-coherent accesses
+typedef unsigned v2u __attribute__((ext_vector_type(2)));
+typedef int v2i __attribute__((ext_vector_type(2)));
+constexpr int kBeyond = 0x7ffffff0;     // an offset behind every descriptor: reads as zero, no access
+
+// one product of one layer
+struct StackEntry {
+    const uint32_t* w;
+    const uint16_t* norm;  // of the RMSNorm in front
+    const uint16_t* ws;
+    uint16_t* ck;  // entry 0: the layer's cache
+    uint16_t* cv;
+    float eps;
+    int slot_rows;  // weight-scale runs, as bitlinear_scale_runs gives them
+    uint32_t slot_map;
+    int pad[3];
+};
+static_assert(sizeof(StackEntry) == 64, "the host writes eight 8-byte words per entry");
+
+// control words, each on a 128-byte line of its own
+struct StackControl {
+    unsigned counter, pad0[31];  // next ticket; back to zero at the end of a launch
+    unsigned mode, pad1[31];     // (launch + 1) * 2 + (1: ticket mode), once decided
+    unsigned done, pad2[31];     // workgroups that have finished; back to zero at the end
+    unsigned launch, pad3[31];   // launches so far
+    int error, pad4[31];
+};
+
+struct StackArgs {
+    const __attribute__((address_space(4))) StackEntry* entries;  // [layer][4]: wqkv, wo, w13, w2
+    unsigned char* ws;
+    const uint16_t* h_in;
+    uint16_t* h_out;
+    const __attribute__((address_space(4))) int64_t* positions;
+    const float* rope_rows;
+    int n_layers, B, dim, ffn, n_heads, n_kv, group, S, n_splits, attn_waves, spin_limit;  // group: query heads per kv head
+    int ends[5];  // cumulative task counts of a layer's phases
+    int f_layer, f_o, f_ha, f_g, f_hb;  // a set: bytes per layer, offsets in it
+    int set_bytes;
+    long long sets;     // offset of the first set in the workspace
+    long long records;  // offset of the attention records
+    float inv_dim, inv_ffn;  // correctly rounded reciprocals
+};
+typedef const __attribute__((address_space(4))) StackArgs* StackArgsPtr;  // the kernel's argument block
+
+// wqkv (two 16-row blocks a task), attention, wo (one block), w13 (two pairs of blocks, gated), w2 (one block)
+enum Phase { kP1 = 0, kAttn, kP3, kP4, kP5 };
+
+struct Work {
+    int layer, ph, first, idx;  // idx: the task's number in its phase, whose first task is number `first` of the layer
+};
+
+// A wave's share of a row: UPW 64-wide k-steps, 64 lanes x 8 consecutive values per 512, and what is left of the
+// share as T values per lane
+template <int UPW>
+struct Slice {
+    static constexpr int kValues = UPW * 64;
+    static constexpr int kFull = kValues / 512;
+    static constexpr int kRest = kValues % 512;
+    static constexpr int T = kRest == 0 ? 0 : kRest <= 128 ? 2 : kRest <= 256 ? 4 : 8;
+    static constexpr int kVec = kFull + (T ? 1 : 0);
+};
+constexpr int kStMaxVec = Slice<kStUpwF>::kVec;
+static_assert(Slice<kStUpwF>::kVec == 4 && Slice<kStUpwD>::kVec == 2, "registers below");
+
+constexpr int kStWordBytes = 40 * 1024;  // a task's packed words: at most four row blocks of 2560, or one of 6912
+constexpr int kStBuffers = 3;
+
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+struct Waiter {
+    int limit;
+    int* error;
+    bool dead;  // a wait gave up: nothing is waited for any more, so that the grid drains
+    __device__ __forceinline__ bool give_up(int spin) {
+        if (spin + 1 < limit &&
+            ((spin & 1023) != 1023 || uniform(__hip_atomic_load(error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == 0))
+            return false;
+        if ((threadIdx.x & 63) == 0) __hip_atomic_store(error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        dead = true;
+        return true;
+    }
+};
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* p, int bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, bytes, 0x00020000);
+}
+// both halves of a packed bf16 pair, in the upper half-word: the larger tells whether one is 0xffff
+__device__ __forceinline__ unsigned unset_max(unsigned m, unsigned d) { return max(m, max(d, d << 16)); }
+__device__ __forceinline__ bool is_unset(unsigned m) { return m >= 0xffff0000u; }
+__device__ __forceinline__ void publish16(uint16_t* p, uint16_t v) {
+    __hip_atomic_store(p, v < 0xfffeu ? v : (uint16_t)0xfffeu, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ __forceinline__ unsigned lds_address(const void* p) {
+    return (unsigned)(uintptr_t)(__attribute__((address_space(3))) const void*)p;
+}
+// LDS words that one wave writes while another looks: as LDS accesses (a volatile access through a generic pointer
+// stays a flat one, and waits for all of the wave's memory loads as well)
+template <class T>
+__device__ __forceinline__ T lds_look(const T& v) {
+    return *(const volatile __attribute__((address_space(3))) T*)&v;
+}
+template <class T>
+__device__ __forceinline__ void lds_put(T& to, T v) {
+    *(volatile __attribute__((address_space(3))) T*)&to = v;
+}
+// 16 bytes per lane straight into LDS, lane l's at `to` + 16 l.  In assembly, so that the compiler does not hold it
+// against every later LDS access (it would wait for the load in front of the next one): what makes the words
+// visible is that a wave waits for a later load of its own -- they return in order -- and then meets a barrier.
+__device__ __forceinline__ void load_to_lds(v4u rsrc, unsigned to, int voffset, int soffset) {
+    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds"
+                 :
+                 : "s"(to), "v"(voffset), "s"(rsrc), "s"(soffset)
+                 : "memory");  // (m0 is the compiler's scratch: it sets it in front of each use of its own)
+}
+// The correctly rounded results of the IEEE operations they replace, from the hardware's approximations and one
+// correction step each (found equal on every mantissa; the operands are positive)
+__device__ __forceinline__ float divide(float x, float by, float inv) {  // inv: 1 / by, correctly rounded
+    const float q = x * inv;
+    const float r = __builtin_fmaf(__builtin_fmaf(-q, by, x), inv, q);
+    return q < INFINITY ? r : q;
+}
+__device__ __forceinline__ float reciprocal(float x) {
+    const float r = __builtin_amdgcn_rcpf(x);
+    return x < INFINITY ? __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r) : 0.0f;
+}
+__device__ __forceinline__ float reciprocal_sqrt(float x) {  // 1 / sqrt(x), both rounded
+    const float y = __builtin_amdgcn_rsqf(x);
+    const float s0 = x * y;
+    const float s = __builtin_fmaf(__builtin_fmaf(-s0, s0, x), 0.5f * y, s0);
+    return x < INFINITY ? reciprocal(s) : 0.0f;
+}
+// reductions that leave the wave's result in lane 63: rows of 16 by lane permutes, then row 0 into 1 and 2 into 3,
+// then those two
+template <class T, class Op>
+__device__ __forceinline__ T wave_reduce_last(T v, Op op) {
+    auto step = [&](auto ctrl, auto rows) {
+        constexpr int C = decltype(ctrl)::value, R = decltype(rows)::value;
+        if constexpr (sizeof(T) == 8) {
+            const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+            const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)u, C, R, 0xF, R == 0xF);
+            const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(u >> 32), C, R, 0xF, R == 0xF);
+            v = op(v, __builtin_bit_cast(T, (unsigned long long)hi << 32 | lo));
+        } else {
+            v = op(v, __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), C, R, 0xF, R == 0xF)));
+        }
+    };
+    step(std::integral_constant<int, 0xB1>{}, std::integral_constant<int, 0xF>{});
+    step(std::integral_constant<int, 0x4E>{}, std::integral_constant<int, 0xF>{});
+    step(std::integral_constant<int, 0x141>{}, std::integral_constant<int, 0xF>{});
+    step(std::integral_constant<int, 0x140>{}, std::integral_constant<int, 0xF>{});
+    step(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xA>{});  // row_bcast15
+    step(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xC>{});  // row_bcast31
+    return v;
+}
+// a packed pair of bf16 at a time: what sumsq8 and norm8 do for four
+__device__ __forceinline__ double sumsq2(uint32_t d) {
+    const float lo = __uint_as_float(d << 16), hi = __uint_as_float(d & 0xffff0000u);
+    return (double)(lo * lo) + (double)(hi * hi);
+}
+__device__ __forceinline__ uint32_t norm2(uint32_t d, uint32_t w, float rstd) {
+    return f32x2_to_bf16x2(__uint_as_float(d << 16) * rstd * __uint_as_float(w << 16),
+                           __uint_as_float(d & 0xffff0000u) * rstd * __uint_as_float(w & 0xffff0000u));
+}
+__device__ __forceinline__ uint32_t quant2(uint32_t d, float s) {  // two bytes
+    return __builtin_amdgcn_perm(quant_low_byte<0>(d & 0xffff0000u, s), quant_low_byte<0>(d << 16, s), 0x0c0c0400u);
+}
+
+template <int MT>
+struct Shared {
+    // packed words of this task and the next two (an attention task keeps its waves' outputs in its buffer)
+    __attribute__((aligned(16))) uint8_t words[kStBuffers][kStWordBytes];
+    __attribute__((aligned(16))) int8_t q[kStWaves][MT][kStUpwF * 64 + 80];  // a wave's quantized slices (reads go one step past)
+    int red[4][kStWaves][MT][16];                                       // the waves' partial sums: [row block][wave][token][row]
+    float part_m[kDfMaxWaves][kStMaxG], part_l[kDfMaxWaves][kStMaxG];
+    __attribute__((aligned(16))) uint16_t qb[kStMaxG][kHeadDim], knew[kHeadDim], vnew[kHeadDim];
+    // exchanges between the computing waves: values with the number of the exchange
+    __attribute__((aligned(16))) v4i sumsq[MT][kStWaves];
+    __attribute__((aligned(16))) v2i amax[MT][kStWaves];
+    __attribute__((aligned(16))) int met[kStWaves];
+    // between them and the wave that fetches: counts of tasks
+    __attribute__((aligned(16))) int consumed[kStWaves];
+    int claimed, ready;
+    __attribute__((aligned(16))) v4i tasks[4][4];  // what the computing waves have to know about a task (Task)
+    uint16_t scales[4][2][32];                     // weight scales of its output rows
+};
+
+// A task as the fetching wave describes it: the computing waves find everything they would have to look up or work
+// out in LDS (their own way through arguments and tables took a microsecond between two tasks)
+struct Task {
+    int layer, ph, idx;
+    float eps;
+    const uint16_t *src, *res;  // attention: the published q | k | v rows; the cache's k
+    uint16_t *dst, *aux;        // attention: the published outputs; the cache's v.  Products: aux = the norm's weights
+    int K, n_out;               // attention: kv head, sequence
+    float inv_k;                // attention: split
+    int flags;                  // 1: src is published, 2: dst is.  Attention: the position
+};
+
+// a lane's values of one token's slice
+template <int UPW>
+struct Values {
+    uint4 full[Slice<UPW>::kFull];
+    uint32_t rest[Slice<UPW>::T / 2];
+};
+template <int MT>
+struct Got {
+    v4i e[4 * kStUpwD];     // the weights as MFMA operands: [row block][k-step], or the 27 steps of one block
+    Values<kStUpwF> f[MT];  // (the first members serve the shorter slices)
+    uint4 g[kStMaxVec];     // norm weights of this lane's values
+    uint16_t res;
+};
+
+template <int MT>
+struct Stack {
+    StackArgsPtr a;
+    Shared<MT>& sh;
+    Waiter wt;
+    unsigned char* set;  // this launch's hand-over buffers
+    unsigned launch;
+    int tid, lane, wave;
+    int exchange;  // exchanges so far: the same in all computing waves
+
+    // Makes the compiler compute what follows from the thread's place and the arguments anew from here on: kept
+    // over the whole loop of tasks, the addresses of all phases together do not fit the registers.
+    __device__ __forceinline__ void forget() {
+        asm volatile("" : "+v"(tid), "+v"(lane), "+s"(wave), "+s"(a));
+    }
+
+    // --- where things are ------------------------------------------------------------------------
+    __device__ __forceinline__ unsigned char* layer_set(int layer) const { return set + (size_t)layer * a->f_layer; }
+    __device__ __forceinline__ uint16_t* qkv(int layer) const { return (uint16_t*)layer_set(layer); }
+    __device__ __forceinline__ uint16_t* o(int layer) const { return (uint16_t*)(layer_set(layer) + a->f_o); }
+    __device__ __forceinline__ uint16_t* ha(int layer) const { return (uint16_t*)(layer_set(layer) + a->f_ha); }
+    __device__ __forceinline__ uint16_t* gate(int layer) const { return (uint16_t*)(layer_set(layer) + a->f_g); }
+    __device__ __forceinline__ uint16_t* hb(int layer) const { return (uint16_t*)(layer_set(layer) + a->f_hb); }
+    // the residual stream in front of the attention block of `layer`
+    __device__ __forceinline__ const uint16_t* h_before(int layer) const { return layer == 0 ? a->h_in : hb(layer - 1); }
+
+    __device__ __forceinline__ Work locate(int layer, int r) const {
+        Work w;
+        while (r >= a->ends[4]) {
+            r -= a->ends[4];
+            ++layer;
+        }
+        int ph = 0, base = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (r >= a->ends[i]) {
+                ph = i + 1;
+                base = a->ends[i];
+            }
+        w.layer = layer;
+        w.ph = ph;
+        w.first = base;
+        w.idx = r - base;
+        return w;
+    }
+    // product of a phase: 0 wqkv, 1 wo, 2 w13, 3 w2
+    static __device__ __forceinline__ int product_of(int ph) { return ph < kP3 ? 0 : ph - 1; }
+
+    __device__ __forceinline__ int batch() const { return MT == 1 ? 1 : a->B; }
+
+    // output slot of this thread within a task: row of a 16-row block, token, and -- where a task has two rows of
+    // blocks -- which
+    __device__ __forceinline__ int out_row() const { return tid & 15; }
+    template <int RPW>
+    __device__ __forceinline__ int out_tb() const { return RPW == 1 ? 0 : (tid >> 4) & 1; }
+    template <int RPW>
+    __device__ __forceinline__ int out_token() const { return RPW == 1 ? tid >> 4 : tid >> 5; }
+
+    // --- between the waves of a workgroup ------------------------------------------------------------
+    // (LDS operations of a wave are carried out in order, so a number written behind a value vouches for it; the
+    // hardware's barrier would have to include the wave that fetches)
+    __device__ __forceinline__ void arrive() {
+        ++exchange;
+        if (lane == 0) lds_put(sh.met[wave], exchange);
+        asm volatile("" ::: "memory");
+    }
+    __device__ __forceinline__ void await() const {
+        for (;;) {
+            asm volatile("" ::: "memory");
+            const v4i m = lds_look(*(const v4i*)sh.met);
+            if (uniform(min(min(m.x, m.y), min(m.z, m.w)) - exchange) >= 0) break;
+        }
+        asm volatile("" ::: "memory");
+    }
+    __device__ __forceinline__ void meet() {
+        arrive();
+        await();
+    }
+
+    // --- the wave that fetches -----------------------------------------------------------------------
+    // distance in LDS of the two runs of row blocks that a w13 task multiplies with (and in expand())
+    __device__ __forceinline__ int run_stride() const { return (a->dim * 8 + 4095) & ~4095; }
+    __device__ __forceinline__ void describe(const Work& wk, const __attribute__((address_space(4))) StackEntry* e, v4i* to) const {
+        const int l = wk.layer;
+        const bool last = l + 1 >= a->n_layers;
+        uint64_t src, res = 0, dst, aux = (uint64_t)e->norm;
+        int K = a->dim, n_out = a->dim, flags = 3;
+        float inv_k = a->inv_dim;
+        switch (wk.ph) {
+            case kP1:
+                src = (uint64_t)h_before(l), dst = (uint64_t)qkv(l);
+                n_out = (a->n_heads + 2 * a->n_kv) * kHeadDim;
+                if (l == 0) flags = 2;
+                break;
+            case kAttn: {
+                src = (uint64_t)qkv(l), dst = (uint64_t)o(l), res = (uint64_t)e->ck, aux = (uint64_t)e->cv;
+                const int rest = wk.idx / a->n_kv;
+                K = wk.idx % a->n_kv, n_out = rest / a->n_splits, inv_k = __uint_as_float((unsigned)(rest % a->n_splits));
+                const int64_t p = a->positions[n_out];
+                flags = p < 0 ? 0 : (p >= (int64_t)a->S ? a->S - 1 : (int)p);
+                break;
+            }
+            case kP3: src = (uint64_t)o(l), dst = (uint64_t)ha(l), res = (uint64_t)h_before(l); break;
+            case kP4: src = (uint64_t)ha(l), dst = (uint64_t)gate(l), n_out = a->ffn; break;
+            default:
+                src = (uint64_t)gate(l), dst = (uint64_t)(last ? a->h_out : hb(l)), res = (uint64_t)ha(l);
+                K = a->ffn, inv_k = a->inv_ffn;
+                if (last) flags = 1;
+                break;
+        }
+        if (lane == 0) {
+            lds_put(to[0], v4i{l < a->n_layers ? l : -1, wk.ph, wk.idx, (int)__float_as_uint(e->eps)});
+            lds_put(to[1], v4i{(int)src, (int)(src >> 32), (int)res, (int)(res >> 32)});
+            lds_put(to[2], v4i{(int)dst, (int)(dst >> 32), (int)aux, (int)(aux >> 32)});
+            lds_put(to[3], v4i{K, n_out, (int)__float_as_uint(inv_k), flags});
+        }
+    }
+    // the weight scale of output row lane % 32 of a task, of w13's second half in the upper lanes
+    __device__ __forceinline__ uint16_t scale_of(const Work& wk, const __attribute__((address_space(4))) StackEntry* e) const {
+        const int first = wk.ph == kP1 || wk.ph == kP4 ? 2 * wk.idx : wk.idx;
+        const int n = first * 16 + (lane & 31) + (lane >> 5) * a->ffn;
+        int run = 0;
+#pragma unroll
+        for (int j = 1; j < 8; ++j) run += n >= j * e->slot_rows ? 1 : 0;
+        return e->ws[(e->slot_map >> (3 * run)) & 7u];
+    }
+    // the packed words of a task into LDS, in pieces of 1 KB
+    __device__ __forceinline__ void fetch(const Work& wk, const uint32_t* w, int buffer) const {
+        if (wk.ph == kAttn) return;
+        const int K = wk.ph == kP5 ? a->ffn : a->dim;
+        const int half = a->ffn >> 4;  // row blocks of one half of w13
+        const bool pairs = wk.ph == kP1 || wk.ph == kP4;
+        const int first = pairs ? 2 * wk.idx : wk.idx;
+        const int bytes = uniform((!pairs || (wk.ph == kP4 && first + 1 >= half) ? 1 : 2) * K * 4);
+        for (int i = 0; i < (wk.ph == kP4 ? 2 : 1); ++i) {
+            const uintptr_t from = (uintptr_t)w + (size_t)(i * half + first) * K * 4;
+            const v4u r = {(unsigned)uniform((int)from), (unsigned)uniform((int)(from >> 32)) & 0xffffu, (unsigned)bytes, 0x00020000u};
+            const unsigned to = lds_address(&sh.words[buffer][i ? run_stride() : 0]);
+#pragma nounroll
+            for (int at = 0; at < bytes; at += 1024) load_to_lds(r, to + at, lane * 16, at);
+        }
+    }
+
+    // --- a product -----------------------------------------------------------------------------------
+    // the norm's weights for this lane's values
+    template <int UPW>
+    __device__ __forceinline__ void norm_weights(const uint16_t* norm, int K, Got<MT>& got) const {
+        typedef Slice<UPW> S;
+        const __amdgpu_buffer_rsrc_t r = make_rsrc(norm, K * 2);
+        int off[S::kVec];
+        slice_offsets<UPW>(K * 2, off);
+#pragma unroll
+        for (int i = 0; i < S::kFull; ++i) got.g[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, off[i], 0, 0));
+        if (S::T == 2) got.g[S::kFull].x = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r, off[S::kFull], 0, 0);
+        if (S::T == 4) {
+            const v2u t = __builtin_bit_cast(v2u, __builtin_amdgcn_raw_buffer_load_b64(r, off[S::kFull], 0, 0));
+            got.g[S::kFull].x = t.x;
+            got.g[S::kFull].y = t.y;
+        }
+    }
+    // byte offsets of this lane's values in a row of row_bytes, kBeyond past its end
+    template <int UPW>
+    __device__ __forceinline__ void slice_offsets(int row_bytes, int (&off)[Slice<UPW>::kVec]) const {
+        typedef Slice<UPW> S;
+        const int first = wave * S::kValues * 2;
+#pragma unroll
+        for (int i = 0; i < S::kFull; ++i) {
+            const int at = first + i * 1024 + lane * 16;
+            off[i] = at < row_bytes ? at : kBeyond;
+        }
+        if (S::T) {
+            const int at = first + S::kFull * 1024 + lane * (S::T * 2);
+            off[S::kFull] = lane * S::T < S::kRest && at < row_bytes ? at : kBeyond;
+        }
+    }
+    // The packed words of a task, in LDS, -> MFMA operands.  In front of the wait for the activations, where nothing
+    // else is to be done.
+    template <int UPW, int RPW>
+    __device__ __forceinline__ void expand(int K, int buffer, Got<MT>& got) {
+        const int p = lane & 15, g = lane >> 4;
+        const int lane_word = (g >> 1) * 32 + (p >> 3) * 16 + (g & 1) * 8 + (p & 7);
+        const uint8_t* words = &sh.words[buffer][wave * (UPW * 256) + lane_word * 4];
+        const int stride2 = RPW == 4 ? (K * 8 + 4095) & ~4095 : 0;
+#pragma unroll
+        for (int i = 0; i < RPW; ++i)
+#pragma unroll
+            for (int j = 0; j < UPW; ++j) {
+                // (past the end of K: whatever follows, times activations that are zero)
+                const uint32_t w = *(const uint32_t*)(words + (i >> 1) * stride2 + (i & 1) * K * 4 + j * 256);
+                v4i& e = got.e[i * kStUpwD + j];
+                e.x = (int)(w & 0x03030303u);
+                e.y = (int)((w >> 2) & 0x03030303u);
+                e.z = (int)((w >> 4) & 0x03030303u);
+                e.w = (int)((w >> 6) & 0x03030303u);
+            }
+        // now, not where they are used: the compiler would put this work behind the wait, next to the products
+#pragma unroll
+        for (int i = 0; i < RPW; ++i)
+#pragma unroll
+            for (int j = 0; j < UPW; ++j) asm volatile("" : "+v"(got.e[i * kStUpwD + j]));
+    }
+    // the slices of the tokens' rows and, RES, this thread's value of a row that was complete before them
+    template <int UPW, bool RES>
+    __device__ __forceinline__ void gather_slices(const Task& tk, Got<MT>& got) {
+        typedef Slice<UPW> S;
+        const int K = tk.K, B = batch();
+        int off[S::kVec];
+        slice_offsets<UPW>(K * 2, off);
+        const __amdgpu_buffer_rsrc_t rows = make_rsrc(tk.src, B * K * 2);
+        const __amdgpu_buffer_rsrc_t rs = make_rsrc(RES ? tk.res : tk.src, RES ? B * tk.n_out * 2 : 0);
+        const int res_off = RES && out_token<1>() < B ? (out_token<1>() * tk.n_out + tk.idx * 16 + out_row()) * 2 : kBeyond;
+        const bool published = (tk.flags & 1) != 0;
+        for (int spin = 0;; ++spin) {
+            poll_again();
+            if (RES) got.res = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rs, res_off, 0, kSc1);
+            unsigned m = RES ? (unsigned)got.res << 16 : 0u;
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+                Values<kStUpwF>& v = got.f[t];
+                const int at = (t < B ? t : B - 1) * K * 2;  // tokens beyond the batch repeat the last one
+#pragma unroll
+                for (int i = 0; i < S::kFull; ++i) v.full[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rows, off[i], at, kSc1));
+                if (S::T == 2) v.rest[0] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rows, off[S::kFull], at, kSc1);
+                if (S::T == 4) {
+                    const v2u r = __builtin_bit_cast(v2u, __builtin_amdgcn_raw_buffer_load_b64(rows, off[S::kFull], at, kSc1));
+                    v.rest[0] = r.x;
+                    v.rest[1] = r.y;
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < MT; ++t) {
+                const Values<kStUpwF>& v = got.f[t];
+#pragma unroll
+                for (int i = 0; i < S::kFull; ++i) m = unset_max(unset_max(unset_max(unset_max(m, v.full[i].x), v.full[i].y), v.full[i].z), v.full[i].w);
+#pragma unroll
+                for (int i = 0; i < S::T / 2; ++i) m = unset_max(m, v.rest[i]);
+            }
+            if (__builtin_amdgcn_ballot_w64(is_unset(m)) == 0 || !published || wt.dead || wt.give_up(spin)) break;
+        }
+    }
+
+    // norm + quantizer of the wave's slices, products, outputs.  RPW 1, 2: row blocks; 4: two pairs (x1, x3), gated
+    template <int UPW, int RPW, bool RES>
+    __device__ __forceinline__ void product(const Task& tk, int k, Got<MT>& got) {
+        typedef Slice<UPW> S;
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+            const Values<kStUpwF>& v = got.f[t];
+            double sq = 0.0;  // lanes without a value hold zeros
+#pragma unroll
+            for (int i = 0; i < S::kFull; ++i) sq += sumsq8(v.full[i]);
+#pragma unroll
+            for (int i = 0; i < S::T / 2; ++i) sq += sumsq2(v.rest[i]);
+            sq = wave_reduce_last(sq, [](double x, double y) { return x + y; });
+            const v2i bits = __builtin_bit_cast(v2i, sq);
+            if (lane == 63) lds_put(sh.sumsq[t][wave], v4i{bits.x, bits.y, exchange + 1, 0});
+        }
+        ++exchange;
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+            Values<kStUpwF>& v = got.f[t];
+            v4i x[kStWaves];
+            for (;;) {
+                asm volatile("" ::: "memory");
+#pragma unroll
+                for (int k = 0; k < kStWaves; ++k) x[k] = lds_look(sh.sumsq[t][k]);
+                if (uniform(min(min(x[0].z, x[1].z), min(x[2].z, x[3].z)) - exchange) >= 0) break;
+            }
+            double total = 0.0;
+#pragma unroll
+            for (int k = 0; k < kStWaves; ++k) total += __builtin_bit_cast(double, v2i{x[k].x, x[k].y});
+            const float rstd = reciprocal_sqrt(divide((float)total, (float)tk.K, tk.inv_k) + tk.eps);
+            uint32_t am = 0;
+#pragma unroll
+            for (int i = 0; i < S::kFull; ++i) {
+                v.full[i] = norm8(v.full[i], got.g[i], rstd);
+                am = absmax_bits8(v.full[i], am);
+            }
+            if (S::T) {
+                uint4 r = make_uint4(0u, 0u, 0u, 0u);
+                v.rest[0] = r.x = norm2(v.rest[0], got.g[S::kFull].x, rstd);
+                if (S::T == 4) v.rest[1] = r.y = norm2(v.rest[1], got.g[S::kFull].y, rstd);
+                am = absmax_bits8(r, am);
+            }
+            am = wave_reduce_last(am, [](uint32_t x, uint32_t y) { return max(x, y); });
+            if (lane == 63) lds_put(sh.amax[t][wave], v2i{(int)am, exchange + 1});
+        }
+        ++exchange;
+        float s[MT];
+        int q2[MT];  // twice the sum of the slice: the +2 of the stored codes
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+            const Values<kStUpwF>& v = got.f[t];
+            v4i x[2];
+            for (;;) {
+                asm volatile("" ::: "memory");
+                x[0] = lds_look(*(const v4i*)&sh.amax[t][0]);
+                x[1] = lds_look(*(const v4i*)&sh.amax[t][2]);
+                if (uniform(min(min(x[0].y, x[0].w), min(x[1].y, x[1].w)) - exchange) >= 0) break;
+            }
+            const uint32_t am = (uint32_t)max(max(x[0].x, x[0].z), max(x[1].x, x[1].z));
+            // quant_scale<0>
+            s[t] = bf16_to_f32(f32_to_bf16_rne(reciprocal(fmaxf(__uint_as_float(am << 16), 1e-5f)) * 127.0f));
+            int8_t* q = sh.q[wave][t];
+            int part = 0;
+#pragma unroll
+            for (int i = 0; i < S::kFull; ++i) {
+                const uint2 qv = quant_vec8<0>(v.full[i], s[t]);
+                *(uint2*)(q + i * 512 + lane * 8) = qv;
+                part = __builtin_amdgcn_sdot4((int)qv.x, 0x01010101, __builtin_amdgcn_sdot4((int)qv.y, 0x01010101, part, false), false);
+            }
+            if (S::T) {
+                uint32_t r = quant2(v.rest[0], s[t]);
+                if (S::T == 4) r |= quant2(v.rest[1], s[t]) << 16;
+                if (lane * S::T < S::kRest) {
+                    if (S::T == 2) *(uint16_t*)(q + S::kFull * 512 + lane * 2) = (uint16_t)r;
+                    if (S::T == 4) *(uint32_t*)(q + S::kFull * 512 + lane * 4) = r;
+                }
+                part = __builtin_amdgcn_sdot4((int)r, 0x01010101, part, false);
+            }
+            part = wave_reduce_last(part, [](int x, int y) { return x + y; });
+            q2[t] = 2 * __builtin_amdgcn_readlane(part, 63);
+        }
+        // the same wave wrote its slices and reads them: LDS operations of a wave complete in order
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const int p = lane & 15, g = lane >> 4;
+        // The products' columns beyond the tokens carry the same tokens at other k-steps: one read serves SP steps (a
+        // read per step, of which the columns take the same bytes 16 / MT times, bounds this part: 66 cycles a step),
+        // step s is multiplied into accumulator s, and of that the columns of step s count.
+        constexpr int SP = RPW == 4 ? 2 : 4;
+        const int step = (p / MT) % SP;
+        const int8_t* brow = &sh.q[wave][p % MT][step * 64 + g * 16];
+        v4i acc[RPW][SP];
+#pragma unroll
+        for (int i = 0; i < RPW; ++i)
+#pragma unroll
+            for (int c = 0; c < SP; ++c) acc[i][c] = v4i{0, 0, 0, 0};
+#pragma unroll
+        for (int j = 0; j < UPW; j += SP) {
+            const v4i b = *(const v4i*)(brow + j * 64);  // (steps past the slice: not multiplied)
+#pragma unroll
+            for (int c = 0; c < SP; ++c)
+                if (j + c < UPW) {
+#pragma unroll
+                    for (int i = 0; i < RPW; ++i)
+                        acc[i][c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(got.e[i * kStUpwD + j + c], b, acc[i][c], 0, 0, 0);
+                }
+        }
+        // lane (p, g) holds token p, rows 4 g ..
+        int mine = q2[0];
+#pragma unroll
+        for (int t = 1; t < MT; ++t) mine = p == t ? q2[t] : mine;
+#pragma unroll
+        for (int i = 0; i < RPW; ++i) {
+            v4i v = acc[i][0];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+#pragma unroll
+                for (int c = 1; c < SP; ++c) v[r] = step == c ? acc[i][c][r] : v[r];
+                v[r] += __builtin_amdgcn_update_dpp(0, v[r], 0x120 + MT, 0xF, 0xF, true);  // row_ror
+                if (SP == 4) v[r] += __builtin_amdgcn_update_dpp(0, v[r], 0x120 + 2 * MT, 0xF, 0xF, true);
+            }
+            if (p < MT) *(v4i*)&sh.red[i][wave][p][4 * g] = v - mine;
+        }
+        arrive();
+        if (wave * 64 >= (RPW == 1 ? 16 : 32) * MT) return;  // the first waves finish the outputs
+        await();
+        const int m = out_token<RPW>(), tb = out_tb<RPW>(), row = out_row();
+        const int n = ((RPW == 1 ? tk.idx : 2 * tk.idx + tb) * 16) + row;
+        if (m < batch() && m < MT && n < tk.n_out) {
+            const uint16_t* ws = &sh.scales[k & 3][0][RPW == 1 ? tid & 15 : tid & 31];
+            float sm = s[0];
+#pragma unroll
+            for (int t = 1; t < MT; ++t) sm = m == t ? s[t] : sm;
+            const float inv_s = reciprocal(sm);
+            auto value = [&](int i, uint16_t ws) {
+                int sum = 0;
+#pragma unroll
+                for (int k = 0; k < kStWaves; ++k) sum += sh.red[i][k][m][row];
+                const float x = (float)sum, q = x * inv_s;  // the quotient as in the other kernels' epilogues
+                return f32_to_bf16_rne(__builtin_fmaf(__builtin_fmaf(-q, sm, x), inv_s, q) * bf16_to_f32(ws));
+            };
+            uint16_t v = value(tb, ws[0]);
+            if (RPW == 4) {
+                const uint16_t x3 = value(2 + tb, ws[32]);
+                const float r = fmaxf(bf16_to_f32(v), 0.0f);
+                v = f32_to_bf16_rne(bf16_to_f32(f32_to_bf16_rne(r * r)) * bf16_to_f32(x3));
+            }
+            if (RES) v = f32_to_bf16_rne(bf16_to_f32(got.res) + bf16_to_f32(v));
+            uint16_t* to = tk.dst + (size_t)m * tk.n_out + n;
+            if (tk.flags & 2)
+                publish16(to, v);
+            else
+                *to = v;
+        }
+    }
+
+    // --- attention: rope, cache write and one split of one (sequence, kv head) ------------------------
+    // (attn_decode_flash_kernel's work on published rows; the last active split merges)
+    struct Place {
+        int G, kvh, sp, b, p, pblk, nact;
+    };
+    __device__ __forceinline__ Place attention_place(const Task& tk) const {
+        Place w;
+        w.G = a->group;
+        w.kvh = tk.K;
+        w.b = tk.n_out;
+        w.sp = (int)__float_as_uint(tk.inv_k);
+        w.p = tk.flags;
+        w.pblk = w.p >> 5;
+        w.nact = w.pblk + 1 < a->n_splits ? w.pblk + 1 : a->n_splits;
+        return w;
+    }
+    typedef float (*PartO)[kStMaxG][kHeadDim];  // the waves' outputs
+    // up to the waves' results in LDS
+    __device__ __forceinline__ void attend(const Task& wk, PartO part_o) {
+        const Place at = attention_place(wk);
+        if (at.sp >= at.nact) return;  // no visible rows in this split
+        const int G = at.G, nsplit = a->n_splits, kvh = at.kvh, sp = at.sp, b = at.b, p = at.p, pblk = at.pblk;
+        const bool owns_new = pblk % nsplit == sp;
+        const int c = lane & 15, g4 = lane >> 4;
+        const int row_elems = (a->n_heads + 2 * a->n_kv) * kHeadDim;
+        const size_t cache_row = (size_t)a->n_kv * kHeadDim;
+        uint16_t* ck = (uint16_t*)wk.res + ((size_t)b * a->S * a->n_kv + kvh) * kHeadDim;
+        uint16_t* cv = wk.aux + ((size_t)b * a->S * a->n_kv + kvh) * kHeadDim;
+        const int row_bytes = a->n_kv * kHeadDim * 2;
+        const int cache_bytes = (a->S - 1) * row_bytes + kHeadDim * 2;
+        const __amdgpu_buffer_rsrc_t k_rsrc = make_rsrc(ck, cache_bytes), v_rsrc = make_rsrc(cv, cache_bytes);
+        const int blk_stride = nsplit * a->attn_waves;  // the split's blocks are dealt to this many waves: this one is wave, wave + kStWaves, ...
+        v4u kb[2][4], vb[8];
+        auto load_rows = [&](int blk) {
+            const int base = blk * 32 * row_bytes;
+#pragma unroll
+            for (int bi = 0; bi < 2; ++bi) {
+                const int off = base + (bi * 16 + c) * row_bytes + g4 * 16;
+#pragma unroll
+                for (int kk = 0; kk < 4; ++kk) kb[bi][kk] = __builtin_amdgcn_raw_buffer_load_b128(k_rsrc, off + kk * 64, 0, 0);
+            }
+#pragma unroll
+            for (int jj = 0; jj < 8; ++jj)
+                vb[jj] = __builtin_amdgcn_raw_buffer_load_b128(v_rsrc, base + ((jj & 3) + (jj >> 2) * 16 + 4 * g4) * row_bytes + c * 16, 0, 0);
+        };
+        if (sp + nsplit * wave <= pblk) load_rows(sp + nsplit * wave);
+
+        // the token's q heads of this group, k and v: a head per wave and round, a pair of values per lane
+        constexpr int kRounds = (kStMaxG + 2 + kStWaves - 1) / kStWaves;
+        const __amdgpu_buffer_rsrc_t row = make_rsrc(wk.src + (size_t)b * row_elems, row_elems * 2);
+        uint32_t praw[kRounds];
+        const float cs = a->rope_rows[(size_t)b * kHeadDim + lane], sn = a->rope_rows[(size_t)b * kHeadDim + kHeadDim / 2 + lane];
+        for (int spin = 0;; ++spin) {
+            poll_again();
+            unsigned m = 0;
+#pragma unroll
+            for (int u = 0; u < kRounds; ++u) {
+                const int hh = wave + u * kStWaves;
+                const int head = hh < G ? kvh * G + hh : (hh == G ? a->n_heads + kvh : a->n_heads + a->n_kv + kvh);
+                if (hh < G + 2) praw[u] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(row, lane * 4, head * kHeadDim * 2, kSc1);
+            }
+#pragma unroll
+            for (int u = 0; u < kRounds; ++u)
+                if (wave + u * kStWaves < G + 2) m = unset_max(m, praw[u]);
+            if (__builtin_amdgcn_ballot_w64(is_unset(m)) == 0 || wt.dead || wt.give_up(spin)) break;
+        }
+        // rope on adjacent pairs, fp32, rounded to bf16; the split that holds position p writes the cache row
+#pragma unroll
+        for (int u = 0; u < kRounds; ++u) {
+            const int hh = wave + u * kStWaves;
+            if (hh >= G + 2) break;
+            uint32_t v = praw[u];
+            if (hh <= G) {
+                const float x = bf16f(v & 0xffffu), y = bf16f(v >> 16);
+                v = (uint32_t)to_bf16(x * cs - y * sn) | ((uint32_t)to_bf16(x * sn + y * cs) << 16);
+            }
+            if (hh < G) {
+                *(uint32_t*)(&sh.qb[hh][2 * lane]) = v;
+            } else if (owns_new) {
+                *(uint32_t*)(&(hh == G ? sh.knew : sh.vnew)[2 * lane]) = v;
+                *(uint32_t*)((hh == G ? ck : cv) + (size_t)p * cache_row + 2 * lane) = v;
+            }
+        }
+        meet();
+        v8bf qa[4];
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) {
+            uint4 t = make_uint4(0, 0, 0, 0);
+            if (c < G) t = *(const uint4*)(&sh.qb[c][kk * 32 + g4 * 8]);
+            qa[kk] = __builtin_bit_cast(v8bf, t);
+        }
+        for (int w = wave; w < a->attn_waves; w += kStWaves) {
+            const int blk0 = sp + nsplit * w;
+            DfState st;
+            for (int blk = blk0; blk <= pblk; blk += blk_stride) {
+                if (w != wave || blk != blk0) load_rows(blk);
+                df_block(kb, vb, qa, sh.knew, sh.vnew, blk, p, lane, st);
+            }
+            df_wave_result<kStMaxG>(st, lane, part_o[w], sh.part_m[w], sh.part_l[w]);
+        }
+    }
+    // the waves' results over the workgroup, then over the splits
+    __device__ __forceinline__ void attention_outputs(const Task& wk, PartO part_o) {
+        const Place at = attention_place(wk);
+        if (at.sp >= at.nact) return;
+        const int G = at.G, nsplit = a->n_splits, kvh = at.kvh, sp = at.sp, b = at.b, nact = at.nact;
+        meet();
+        unsigned long long* rec =
+            (unsigned long long*)(a->ws + a->records) + ((size_t)(b * a->n_kv + kvh) * nsplit) * kStMaxG * kDfRecUnits;
+        const unsigned long long tag = (unsigned long long)(launch * (unsigned)a->n_layers + (unsigned)wk.layer + 1u) << 32;
+        uint32_t* orow = (uint32_t*)(wk.dst + (size_t)b * a->dim + (size_t)kvh * G * kHeadDim);
+        for (int hh = wave; hh < G; hh += kStWaves) {
+            DfPartial h = df_combine<kStMaxG>(part_o, sh.part_m, sh.part_l, hh, a->attn_waves, lane);
+            if (sp < nact - 1) {
+                df_store_record(rec + ((size_t)sp * kStMaxG + hh) * kDfRecUnits, tag, h, lane);
+                continue;
+            }
+            bool gave_up = false;
+            if (nact > 1) h = df_merge<kStMaxG>(rec, nact, hh, tag, h, lane, wt.dead ? 1 : wt.limit, gave_up);
+            if (uniform(gave_up)) {
+                if (lane == 0) __hip_atomic_store(wt.error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                wt.dead = true;
+            }
+            const float is = gave_up ? __builtin_nanf("") : 1.0f / h.l;
+            __hip_atomic_store(orow + hh * (kHeadDim / 2) + lane, (uint32_t)to_bf16(h.o0 * is) | ((uint32_t)to_bf16(h.o1 * is) << 16),
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // to_bf16 gives no 0xffff
+        }
+    }
+
+    // --- one task --------------------------------------------------------------------------------------
+    template <int UPW, int RPW, bool RES>
+    __device__ __forceinline__ void product_task(const Task& tk, int k) {
+        Got<MT> got;
+        norm_weights<UPW>(tk.aux, tk.K, got);
+        wait_ready(k);
+        expand<UPW, RPW>(tk.K, k % kStBuffers, got);
+        consume(k);
+        gather_slices<UPW, RES>(tk, got);
+        product<UPW, RPW, RES>(tk, k, got);
+    }
+    // task k's words are in its buffer
+    __device__ __forceinline__ void wait_ready(int k) const {
+        while (uniform(lds_look(sh.ready)) <= k) __builtin_amdgcn_s_sleep(1);
+        asm volatile("" ::: "memory");
+    }
+    // task k's buffer is free again
+    __device__ __forceinline__ void consume(int k) {
+        asm volatile("" ::: "memory");
+        if (lane == 0) lds_put(sh.consumed[wave], k + 1);
+        asm volatile("" ::: "memory");
+    }
+    __device__ __forceinline__ void run(const Task& tk, int k) {
+        switch (tk.ph) {
+            case kP1: product_task<kStUpwD, 2, false>(tk, k); break;
+            case kAttn: {
+                const PartO part_o = (PartO)sh.words[k % kStBuffers];
+                wait_ready(k);
+                attend(tk, part_o);
+                attention_outputs(tk, part_o);
+                consume(k);
+                break;
+            }
+            case kP3: product_task<kStUpwD, 1, true>(tk, k); break;
+            case kP4: product_task<kStUpwD, 4, false>(tk, k); break;
+            default: product_task<kStUpwF, 1, true>(tk, k); break;
+        }
+    }
+};
+
+template <int MT>
+__global__ __launch_bounds__(kStThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void decode_stack_kernel(const StackArgs a) {
+    __shared__ Shared<MT> sh;
+    StackControl* ctl = (StackControl*)a.ws;
+    const int tid = threadIdx.x;
+    // changes only when every workgroup of this launch is done; written past the writer's L2, so read past this one
+    const unsigned launch = (unsigned)uniform((int)__hip_atomic_load(&ctl->launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    Stack<MT> st{(StackArgsPtr)__builtin_amdgcn_kernarg_segment_ptr(), sh, Waiter{a.spin_limit, &ctl->error, false},
+                 a.ws + a.sets + (size_t)(launch & 1u) * a.set_bytes, launch, tid, tid & 63, uniform(tid >> 6), 0};
+    if (tid < kStWaves) sh.met[tid] = sh.consumed[tid] = 0;
+    if (tid < MT * kStWaves) {
+        ((v4i*)sh.sumsq)[tid] = v4i{0, 0, 0, 0};
+        ((v2i*)sh.amax)[tid] = v2i{0, 0};
+    }
+    if (tid == 0) sh.claimed = sh.ready = 0;
+    {
+        // the other set, for the next launch
+        const __amdgpu_buffer_rsrc_t other = make_rsrc(a.ws + a.sets + (size_t)((launch & 1u) ^ 1u) * a.set_bytes, a.set_bytes);
+        for (int at = (blockIdx.x * kStThreads + tid) * 16; at < a.set_bytes; at += gridDim.x * kStThreads * 16)
+            __builtin_amdgcn_raw_buffer_store_b128(v4u{~0u, ~0u, ~0u, ~0u}, other, at, 0, kSc1);
+    }
+    __syncthreads();
+    Work cur = st.locate(0, 0);
+    if (st.wave == kStWaves) {
+        // The wave that fetches: takes tickets and brings the tasks' words into LDS, up to two tasks ahead of the
+        // computing waves.  Its waits for memory hold up nobody (loads of one wave return in order).
+        const unsigned grid = gridDim.x, undecided = (launch + 1u) << 1;
+        auto decide = [&](unsigned mode) {
+            unsigned seen = __hip_atomic_load(&ctl->mode, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            while (((seen ^ undecided) >> 1) != 0) {
+                if (__hip_atomic_compare_exchange_strong(&ctl->mode, &seen, undecided | mode, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                                         __HIP_MEMORY_SCOPE_AGENT))
+                    break;
+            }
+        };
+        auto claim = [&] {
+            unsigned t = 0;
+            if (st.lane == 0) t = __hip_atomic_fetch_add(&ctl->counter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return uniform((int)t);
+        };
+        int mode = -1;  // 0 static, 1 tickets
+        int at = 0;     // ticket of cur
+        for (int k = 0;; ++k) {
+            int t;
+            if (k == 0) {
+                t = claim();
+                if (t == (int)grid - 1 && st.lane == 0) decide(0u);
+            } else {
+                if (mode < 0) {
+                    unsigned seen = 0;
+                    for (int spin = 0; spin < kStModePolls; ++spin) {
+                        seen = (unsigned)uniform((int)__hip_atomic_load(&ctl->mode, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+                        if (((seen ^ undecided) >> 1) == 0) break;
+                    }
+                    if (((seen ^ undecided) >> 1) != 0) {
+                        if (st.lane == 0) decide(1u);
+                        seen = (unsigned)uniform((int)__hip_atomic_load(&ctl->mode, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+                    }
+                    mode = (int)(seen & 1u);
+                }
+                t = mode == 0 ? at + (int)grid : claim();
+            }
+            cur = st.locate(cur.layer, cur.first + cur.idx + (t - at));
+            at = t;
+            const bool end = cur.layer >= a.n_layers;
+            const auto* e = a.entries + ((end ? 0 : cur.layer) * 4 + st.product_of(cur.ph));
+            st.describe(cur, e, sh.tasks[k & 3]);
+            if (st.lane == 0) lds_put(sh.claimed, k + 1);
+            asm volatile("" ::: "memory");
+            if (end) break;
+            // task k - kStBuffers has left this buffer
+            for (;;) {
+                asm volatile("" ::: "memory");
+                const v4i c = lds_look(*(const v4i*)sh.consumed);
+                if (uniform(min(min(c.x, c.y), min(c.z, c.w))) >= k + 1 - kStBuffers) break;
+                __builtin_amdgcn_s_sleep(2);
+            }
+            const uint16_t scale = st.scale_of(cur, e);
+            st.fetch(cur, e->w, k % kStBuffers);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            sh.scales[k & 3][st.lane >> 5][st.lane & 31] = scale;
+            asm volatile("" ::: "memory");
+            if (st.lane == 0) lds_put(sh.ready, k + 1);
+            asm volatile("" ::: "memory");
+        }
+        return;
+    }
+    for (int k = 0;; ++k) {
+        st.forget();
+        while (uniform(lds_look(sh.claimed)) <= k) __builtin_amdgcn_s_sleep(1);
+        asm volatile("" ::: "memory");
+        v4i task[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) task[i] = lds_look(sh.tasks[k & 3][i]);
+        auto word = [&](int i) { return uniform(task[i >> 2][i & 3]); };
+        auto address = [&](int i) { return (uint64_t)(unsigned)word(i + 1) << 32 | (unsigned)word(i); };
+        Task tk;
+        tk.layer = word(0), tk.ph = word(1), tk.idx = word(2);
+        if (tk.layer < 0) break;
+        tk.eps = __uint_as_float((unsigned)word(3));
+        tk.src = (const uint16_t*)address(4);
+        tk.res = (const uint16_t*)address(6);
+        tk.dst = (uint16_t*)address(8);
+        tk.aux = (uint16_t*)address(10);
+        tk.K = word(12), tk.n_out = word(13), tk.flags = word(15);
+        tk.inv_k = __uint_as_float((unsigned)word(14));
+        st.run(tk, k);
+    }
+    if (tid == 0) {
+        const unsigned e = __hip_atomic_fetch_add(&ctl->done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
+        if (e == gridDim.x) {  // every workgroup has taken its last ticket
+            __hip_atomic_store(&ctl->done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&ctl->counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&ctl->launch, launch + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+}
+
+// A fresh workspace: zero control words and records, both sets unset
+__global__ __launch_bounds__(256) void decode_stack_reset_kernel(v4u* ws, long long n, long long sets, long long set_units) {
+    for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256) {
+        const unsigned fill = i >= sets && i < sets + 2 * set_units ? ~0u : 0u;
+        ws[i] = v4u{fill, fill, fill, fill};
+    }
+}
+
+long long up256(long long v) { return (v + 255) & ~255ll; }
+
+// Fills in everything that follows from the sizes; false: not a shape these kernels take
+bool stack_plan(StackArgs& a, long long* bytes) {
+    const int nqkv = (a.n_heads + 2 * a.n_kv) * kHeadDim;
+    if (a.B < 1 || a.B > kStMaxTokens || a.n_layers < 1 || a.n_layers > 4096 || a.n_heads < 1 || a.n_kv < 1) return false;
+    if (a.n_heads % a.n_kv || a.n_heads * kHeadDim != a.dim || a.S < 1) return false;
+    const int g = a.n_heads / a.n_kv;
+    if (g != 1 && g != 2 && g != 4 && g != 8) return false;
+    a.group = g;
+    if (a.dim % 64 || a.dim > kStWaves * kStUpwD * 64 || a.ffn < 64 || a.ffn % 64 || a.ffn > kStWaves * kStUpwF * 64) return false;
+    if (a.n_splits < 1 || a.n_splits > kDfMaxSplits) return false;
+    const int counts[5] = {nqkv / 32, a.n_kv * a.n_splits * a.B, a.dim / 16, (a.ffn / 16 + 1) / 2, a.dim / 16};
+    int sum = 0;
+    for (int i = 0; i < 5; ++i) a.ends[i] = sum += counts[i];
+    if ((long long)sum * a.n_layers > (1ll << 30)) return false;
+    long long f = up256((long long)a.B * nqkv * 2);
+    a.f_o = (int)f;
+    f = up256(f + (long long)a.B * a.dim * 2);
+    a.f_ha = (int)f;
+    f = up256(f + (long long)a.B * a.dim * 2);
+    a.f_g = (int)f;
+    f = up256(f + (long long)a.B * a.ffn * 2);
+    a.f_hb = (int)f;
+    f = up256(f + (long long)a.B * a.dim * 2);
+    a.f_layer = (int)f;
+    if (f * a.n_layers > (1ll << 30)) return false;
+    a.set_bytes = (int)(f * a.n_layers);
+    a.sets = up256(sizeof(StackControl));
+    a.records = a.sets + 2ll * a.set_bytes;
+    a.inv_dim = 1.0f / (float)a.dim;
+    a.inv_ffn = 1.0f / (float)a.ffn;
+    *bytes = up256(a.records + (long long)a.B * a.n_kv * a.n_splits * kStMaxG * kDfRecUnits * 8);
+    return true;
+}
+
+}  // namespace
+
+// in decoder_ops.hip: threads the attention kernel of this shape runs with; 0: a shape it does not take
+int bitnet_attn_decode_threads(int B, int S, int n_heads, int n_kv_heads, int n_splits);
+
+extern "C" {
+
+long long bitnet_decode_stack_workspace_bytes(int n_layers, int B, int S, int dim, int ffn, int n_heads, int n_kv_heads,
+                                              int n_splits) {
+    StackArgs a = {};
+    a.n_layers = n_layers, a.B = B, a.S = S, a.dim = dim, a.ffn = ffn, a.n_heads = n_heads, a.n_kv = n_kv_heads, a.n_splits = n_splits;
+    long long bytes = 0;
+    if (!stack_plan(a, &bytes) || !bitnet_attn_decode_threads(B, S, n_heads, n_kv_heads, n_splits)) return -1;
+    return bytes;
+}
+
+int bitnet_decode_stack_reset(void* workspace, int n_layers, int B, int S, int dim, int ffn, int n_heads, int n_kv_heads,
+                              int n_splits, void* stream) {
+    StackArgs a = {};
+    a.n_layers = n_layers, a.B = B, a.S = S, a.dim = dim, a.ffn = ffn, a.n_heads = n_heads, a.n_kv = n_kv_heads, a.n_splits = n_splits;
+    long long bytes = 0;
+    if (!stack_plan(a, &bytes)) return 1;
+    if (!workspace) return 2;
+    if ((uintptr_t)workspace & 255u) return 1;
+    hipLaunchKernelGGL(decode_stack_reset_kernel, dim3(1024), dim3(256), 0, (hipStream_t)stream, (v4u*)workspace, bytes >> 4, a.sets >> 4,
+                       (long long)a.set_bytes >> 4);
+    return hipGetLastError() == hipSuccess ? 0 : 3;
+}
+
+int bitnet_decode_stack_error_offset(void) { return (int)offsetof(StackControl, error); }
+
+int bitnet_decode_stack(const void* entries, void* workspace, const uint16_t* h_in, uint16_t* h_out, const int64_t* positions,
+                        const float* rope_rows, int n_layers, int B, int S, int dim, int ffn, int n_heads, int n_kv_heads,
+                        int n_splits, int workgroups, int spin_limit, void* stream) {
+    StackArgs a = {};
+    a.n_layers = n_layers, a.B = B, a.S = S, a.dim = dim, a.ffn = ffn, a.n_heads = n_heads, a.n_kv = n_kv_heads, a.n_splits = n_splits;
+    long long bytes = 0;
+    if (!stack_plan(a, &bytes)) return 1;
+    const int threads = bitnet_attn_decode_threads(B, S, n_heads, n_kv_heads, n_splits);
+    if (!threads) return 1;
+    if (!entries || !workspace || !h_in || !h_out || !positions || !rope_rows) return 2;
+    if (((uintptr_t)entries & 63u) || ((uintptr_t)workspace & 255u) || ((uintptr_t)h_in & 15u) || ((uintptr_t)h_out & 15u)) return 1;
+    a.entries = (const __attribute__((address_space(4))) StackEntry*)entries;
+    a.ws = (unsigned char*)workspace;
+    a.h_in = h_in;
+    a.h_out = h_out;
+    a.positions = (const __attribute__((address_space(4))) int64_t*)positions;
+    a.rope_rows = rope_rows;
+    a.attn_waves = threads / 64;
+    a.spin_limit = spin_limit > 0 ? spin_limit : kStSpinLimit;
+    int grid = workgroups;
+    if (grid <= 0) {  // one per CU
+        static int cus[bitnet_host::kMaxDevices];
+        int dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= bitnet_host::kMaxDevices) return 3;
+        if (!cus[dev]) {
+            int n = 0;
+            if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) return 3;
+            cus[dev] = n;
+        }
+        grid = cus[dev];
+    }
+#define BITNET_STACK(MT) hipLaunchKernelGGL(decode_stack_kernel<MT>, dim3(grid), dim3(kStThreads), 0, (hipStream_t)stream, a)
+    if (B == 1) BITNET_STACK(1);
+    else BITNET_STACK(2);
+#undef BITNET_STACK
+    return hipGetLastError() == hipSuccess ? 0 : 3;
+}
+
+}  // extern "C"

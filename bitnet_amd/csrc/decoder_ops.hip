@@ -511,6 +511,21 @@ extern "C" int bitnet_attn_decode_error_index(int B, int n_heads, int n_kv_heads
     return n + 2 < (1ll << 31) ? (int)n : -1;
 }
 
+// Threads per workgroup the attention kernel of this shape runs with; 0: a cache it does not take.  (The decode stack
+// kernel deals a split's rows to its waves the same way, so that both give the same bits.)
+int bitnet_attn_decode_threads(int B, int S, int n_heads, int n_kv_heads, int n_splits) {
+    (void)n_heads;
+    // the kernel's 32-bit byte offsets into one sequence's cache (the first blocks requested may lie up to 4096 rows in)
+    if ((size_t)((S > 4096 ? S : 4096) + 512) * n_kv_heads * kHeadDim * 2 >= ((size_t)1 << 31)) return 0;
+    const int span = ((S + n_splits - 1) / n_splits + 15) & ~15;  // a split's share of the cache capacity
+    // The kernel deals blocks of 32 rows to splits and waves: four waves cover a split's share of up to 128
+    // rows of the capacity in one round (measured at 96 rows: 6.85 us with four waves, 7.12 with eight; at 272
+    // rows 8.77 / 8.46).  Eight waves while every workgroup has a CU of its own (up to 256 of them); beyond
+    // that two 512-thread workgroups share a CU badly and 256 threads are the better choice.
+    if (const int forced = g_attn_threads.load()) return forced;
+    return (span > 128 && (long long)n_kv_heads * B * n_splits <= 256) ? 512 : 256;
+}
+
 static int attn_decode_impl(const uint16_t* qkv, uint16_t* cache_k, uint16_t* cache_v, const int64_t* positions,
                             const float* cos_table, const float* sin_table, const float* rope_rows, uint16_t* out,
                             float* workspace, int* counters, int n_splits, int B, int S, int n_heads, int n_kv_heads,
@@ -523,15 +538,8 @@ static int attn_decode_impl(const uint16_t* qkv, uint16_t* cache_k, uint16_t* ca
     if (!qkv || !cache_k || !cache_v || !positions || !cos_table || !sin_table || !out) return 2;
     if (n_splits > 1 && (!workspace || !counters)) return 2;
     if (((uintptr_t)workspace) & 7u) return 1;
-    // the kernel's 32-bit byte offsets into one sequence's cache (the first blocks requested may lie up to 4096 rows in)
-    if ((size_t)((S > 4096 ? S : 4096) + 512) * n_kv_heads * kHeadDim * 2 >= ((size_t)1 << 31)) return 1;
-    const int span = ((S + n_splits - 1) / n_splits + 15) & ~15;  // a split's share of the cache capacity
-    // The kernel deals blocks of 32 rows to splits and waves: four waves cover a split's share of up to 128
-    // rows of the capacity in one round (measured at 96 rows: 6.85 us with four waves, 7.12 with eight; at 272
-    // rows 8.77 / 8.46).  Eight waves while every workgroup has a CU of its own (up to 256 of them); beyond
-    // that two 512-thread workgroups share a CU badly and 256 threads are the better choice.
-    int threads = (span > 128 && (long long)n_kv_heads * B * n_splits <= 256) ? 512 : 256;
-    if (const int forced = g_attn_threads.load()) threads = forced;
+    const int threads = bitnet_attn_decode_threads(B, S, n_heads, n_kv_heads, n_splits);
+    if (!threads) return 1;
     return bitnet_attn_decode_flash_launch(qkv, cache_k, cache_v, positions, cos_table, sin_table, rope_rows, out, workspace,
                                            counters, n_splits, threads, B, S, n_heads, n_kv_heads, g_attn_spin_limit.load(),
                                            (hipStream_t)stream);

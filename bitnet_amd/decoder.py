@@ -12,6 +12,8 @@ plain torch ops are used: RMSNorm and RoPE are closed forms, attention is
 softmax(QK^T/sqrt(d))V in fp32 over the cache.  One decode step is captured in
 a HIP graph and replayed per token, as the reference does with CUDA graphs.
 """
+import ctypes
+import struct
 import time
 from dataclasses import dataclass
 from typing import List, Optional, Tuple
@@ -271,6 +273,90 @@ def norm_bitlinear(x, norm: "RMSNorm", lin: BitLinearKernel, glu: bool = False, 
     return out
 
 
+class DecodeStack:
+    """All layers of a decode step as one launch (bitnet_decode_stack) for one
+    model, cache and batch: the table of what the layers' parameters point to,
+    and the kernel's workspace.  Parameters and cache must stay where they are,
+    as for a captured graph."""
+
+    def __init__(self, model: "Transformer", batch: int, cache, n_splits: int):
+        lib = _lib.load_library()
+        a = model.args
+        dev = cache[0][0].device
+        self.shape = (a.n_layers, batch, cache[0][0].shape[1], a.dim, a.ffn_dim, a.n_heads, a.n_kv_heads, n_splits)
+        words = []
+        for layer, (ck, cv) in zip(model.layers, cache):
+            att, ffn = layer.attention, layer.feed_forward
+            for lin, norm in ((att.wqkv, layer.attention_norm), (att.wo, att.attn_sub_norm), (ffn.w13, layer.ffn_norm),
+                              (ffn.w2, ffn.ffn_sub_norm)):
+                rows, slots = ctypes.c_int(), ctypes.c_uint32()
+                st = lib.bitlinear_scale_runs(lin.out_features, lin.in_features, lin._seg_c,
+                                              len(lin.seg_ends) if lin.seg_ends else 0, ctypes.byref(rows), ctypes.byref(slots))
+                _lib.check(st, "bitlinear_scale_runs")
+                eps = struct.unpack("<I", struct.pack("<f", norm.eps))[0]
+                own = (ck.data_ptr(), cv.data_ptr()) if lin is att.wqkv else (0, 0)
+                words += [lin.weight.data_ptr(), norm.weight.data_ptr(), lin.weight_scale.data_ptr(), *own,
+                          eps | rows.value << 32, slots.value, 0]
+        self.entries = torch.tensor(words, dtype=torch.int64, device=dev)
+        self.workspace = torch.empty(lib.bitnet_decode_stack_workspace_bytes(*self.shape), dtype=torch.uint8, device=dev)
+        at = lib.bitnet_decode_stack_error_offset()
+        self._error = self.workspace[at : at + 4].view(torch.int32)
+        self.reset()
+
+    @staticmethod
+    def applies(model: "Transformer", batch: int, cache, n_splits: int) -> bool:
+        """Whether the kernel takes this model: its sizes, bf16 norms and caches, the quantizer's default mode, weight
+        scales that change at multiples of 16 rows."""
+        a = model.args
+        lib = _lib.load_library()
+        if lib.bitnet_decode_stack_workspace_bytes(a.n_layers, batch, cache[0][0].shape[1], a.dim, a.ffn_dim, a.n_heads,
+                                                   a.n_kv_heads, n_splits) < 0:
+            return False
+        for layer, (ck, cv) in zip(model.layers, cache):
+            att, ffn = layer.attention, layer.feed_forward
+            if ck.dtype != torch.bfloat16 or cv.dtype != torch.bfloat16:
+                return False
+            for lin, norm in ((att.wqkv, layer.attention_norm), (att.wo, att.attn_sub_norm), (ffn.w13, layer.ffn_norm),
+                              (ffn.w2, ffn.ffn_sub_norm)):
+                rows, slots = ctypes.c_int(), ctypes.c_uint32()
+                if (lin.quant_mode != 0 or norm.weight.dtype != torch.bfloat16 or not lin.weight.is_contiguous()
+                        or (lin.weight.data_ptr() | norm.weight.data_ptr()) % 16
+                        or lib.bitlinear_scale_runs(lin.out_features, lin.in_features, lin._seg_c,
+                                                    len(lin.seg_ends) if lin.seg_ends else 0, ctypes.byref(rows),
+                                                    ctypes.byref(slots)) or rows.value % 16):
+                    return False
+        return True
+
+    def reset(self) -> None:
+        """The workspace as before its first use.  Not inside a graph capture."""
+        st = _lib.load_library().bitnet_decode_stack_reset(_ptr(self.workspace), *self.shape, _stream_ptr())
+        if st != 0:
+            raise _lib.BitLinearLibraryError(f"bitnet_decode_stack_reset: status {st}")
+
+    def __call__(self, h, positions, rope_rows, workgroups: int = 0, spin_limit: int = 0):
+        """h bf16 [B, dim], positions int64 [B], rope_rows as decode_step_begin returns them -> the hidden state behind
+        the last layer, bf16 [B, dim]; the caches get the new token's rows."""
+        n_layers, B, S, dim = self.shape[:4]
+        if h.shape != (B, dim) or h.dtype != torch.bfloat16 or positions.numel() != B or rope_rows.shape != (B, 128):
+            raise ValueError("DecodeStack: h, positions or rope_rows do not match the batch it was made for")
+        out = torch.empty_like(h)
+        st = _lib.load_library().bitnet_decode_stack(
+            _ptr(self.entries), _ptr(self.workspace), _ptr(h), _ptr(out), _ptr(positions), _ptr(rope_rows), *self.shape, workgroups,
+            spin_limit, _stream_ptr())
+        if st != 0:
+            raise _lib.BitLinearLibraryError(f"bitnet_decode_stack: status {st}")
+        return out
+
+    def check(self) -> None:
+        """Raises if a wait inside the kernel gave up since the last check, and clears the condition (synchronises)."""
+        if int(self._error.item()):
+            self.reset()
+            raise _lib.BitLinearLibraryError(
+                "decode stack: a wait between workgroups gave up (workspace shared between overlapping calls?); "
+                "the results of the steps since the last check are void"
+            )
+
+
 class Attention(nn.Module):
     def __init__(self, args: ModelArgs):
         super().__init__()
@@ -382,6 +468,14 @@ class Transformer(nn.Module):
             x13 = norm_bitlinear(h, layer.ffn_norm, ffn.w13)
             h = norm_bitlinear(x13, ffn.ffn_sub_norm, ffn.w2, glu=True, residual=h)
         return h
+
+    @torch.no_grad()
+    def decode_hidden_stack(self, tokens, positions, cos, sin, stack: DecodeStack):
+        """decode_hidden_fused with all layers in one launch."""
+        B = tokens.shape[0]
+        pos = positions.reshape(B)
+        h, rows = decode_step_begin(tokens.reshape(B), pos, self.tok_embeddings.weight, cos, sin)
+        return stack(h, pos, rows)
 
     @torch.no_grad()
     def prefill_hidden_fused(self, tokens, cache, cos, sin):
@@ -505,6 +599,7 @@ class Generator:
         self.pos = torch.zeros(batch, 1, dtype=torch.int64, device=dev)
         self.next_tok = torch.zeros(batch, dtype=torch.int64, device=dev)
         self.graph: Optional[torch.cuda.CUDAGraph] = None
+        self.stack: Optional[DecodeStack] = None  # of the captured step, where the model is one it takes
         self.use_graph = use_graph
         # final norm + bf16 LM head + greedy token as two launches of the library
         self.lm_head = (self.fused and fused_head and model.output.weight.dtype == torch.bfloat16 and a.dim % 64 == 0
@@ -519,11 +614,14 @@ class Generator:
         self._pf_graphs: dict = {}
         self._rows = torch.arange(batch, device=dev)
 
-    def _step(self):
+    def _step(self, stack: Optional[DecodeStack] = None):
         """One decode step including its bookkeeping: next token -> history and
         the input of the following step, position + 1."""
         if self.lm_head:
-            h = self.model.decode_hidden_fused(self.tok, self.pos, self.cache, self.cos, self.sin, self.attn_ws)
+            if stack is not None:
+                h = self.model.decode_hidden_stack(self.tok, self.pos, self.cos, self.sin, stack)
+            else:
+                h = self.model.decode_hidden_fused(self.tok, self.pos, self.cache, self.cos, self.sin, self.attn_ws)
             # the step's bookkeeping rides on the last kernel of the LM head
             lm_head_greedy(h, self.model.norm, self.model.output.weight, self.lm_ws, token_out=self.next_tok,
                            next_input=self.tok, positions=self.pos, history=self.history, step_idx=self.step_idx)
@@ -540,15 +638,26 @@ class Generator:
         self.pos.add_(1)
 
     def _capture(self):
+        a = self.model.args
+        if (self.lm_head and self.model.tok_embeddings.weight.dtype == torch.bfloat16 and a.dim % 8 == 0
+                and DecodeStack.applies(self.model, self.batch, self.cache, self.attn_ws.n_splits)):
+            self.stack = DecodeStack(self.model, self.batch, self.cache, self.attn_ws.n_splits)
         s = torch.cuda.Stream()
         s.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(s):
-            self._step()  # warm-up outside the graph
+            self._step(self.stack)  # warm-up outside the graph
         torch.cuda.current_stream().wait_stream(s)
         torch.cuda.synchronize()
         self.graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(self.graph):
-            self._step()
+            self._step(self.stack)
+
+    def _check(self) -> None:
+        """Raises if a wait inside the steps since the last check gave up (one small copy to the host)."""
+        if self.use_graph and self.stack is not None:
+            self.stack.check()
+        elif self.fused:
+            self.attn_ws.check()
 
     kMaxPrefillGraphs = 12  # captured prompt passes kept; the least recently replayed one makes room for a new one
     kPrefillBucket = 32  # prompts are padded to a multiple of this many tokens, so that lengths share captured passes
@@ -664,8 +773,7 @@ class Generator:
             if eos_id is not None and bool((self.next_tok == eos_id).any()):
                 break
         out = self.history[:taken].clone()
-        if self.fused:
-            self.attn_ws.check()  # one small copy to the host per decode() call
+        self._check()
         return out
 
     @torch.no_grad()

@@ -70,6 +70,14 @@ const char* bitlinear_status_string(int status);
 int bitlinear_ws_num(int N, int K);
 
 /*
+ * Which weight scale an output row takes, as runs of *slot_rows rows: row n reads
+ * ws[(*slot_map >> 3 * (n / *slot_rows)) & 7].  seg_ends NULL: the rule of bitlinear_int8xint2,
+ * otherwise that of bitlinear_int8xint2_seg.  BITLINEAR_ERR_ARG for a segment list that is not valid
+ * or needs more than eight runs.  (Host only; what bitnet_decode_stack's table holds.)
+ */
+int bitlinear_scale_runs(int N, int K, const int* seg_ends, int nseg, int* slot_rows, uint32_t* slot_map);
+
+/*
  * Same computation, also storing the raw int32 accumulators
  * (in_thread_C_local after the reduction, bitnet_kernels.h:74-78) to
  * acc_out [M, N].  output0 may be NULL (then s and ws may be NULL too).

@@ -174,6 +174,44 @@ int bitnet_lm_head_workgroups(int V);
  * 2 = same as 0.  Results differ only in the order of fp32 additions.  Returns 0, or 1. */
 int bitnet_lm_head_set_kernel(int which);
 
+/*
+ * All decoder layers of one decode step (gpu/model.py:214-245: norm + wqkv, rope + cache write +
+ * attention, sub-norm + wo + residual, norm + w13, gate + sub-norm + w2 + residual, n_layers times,
+ * one new token per sequence) in one kernel of one workgroup per CU.  Same results, bit for bit, as
+ * bitlinear_norm_forward_bf16[_seg] (mode 0) and bitnet_attn_decode called for every layer.
+ *
+ *   entries    64-byte aligned table of n_layers x 4 records (wqkv, wo, w13, w2) of eight 64-bit
+ *              words: packed weight, weight of the RMSNorm in front (bf16), weight scales (bf16),
+ *              cache_k, cache_v (wqkv's record only), eps as fp32 bits | slot_rows << 32,
+ *              slot_map, 0 -- the last two from bitlinear_scale_runs; slot_rows a multiple of 16.
+ *              Device memory; what it points to must stay in place.
+ *   workspace  bitnet_decode_stack_workspace_bytes() bytes, 256-byte aligned, set up once by
+ *              bitnet_decode_stack_reset().  Calls that share it must not overlap in time.
+ *   h_in       bf16 [B, dim], h_out bf16 [B, dim] (must not be h_in), 16-byte aligned
+ *   positions  int64 [B] (clamped into the cache), rope_rows fp32 [B, 128] as
+ *              bitnet_decode_step_begin writes them
+ *   workgroups 0 = one per CU; otherwise the grid (a test hook: any number works)
+ *   spin_limit 0 = the built-in bound of every wait inside the kernel; otherwise the bound
+ * dim = n_heads * 128, dim % 64 == 0, dim <= 2560; ffn % 64 == 0, ffn <= 6912; n_heads / n_kv_heads
+ * one of 1, 2, 4, 8; B <= 2; n_splits <= 16: workspace_bytes returns -1 for anything else.
+ *
+ * Workgroups wait for each other inside the kernel, but never for one that does not run yet: the
+ * kernel ends whatever else occupies the GPU.  Should a wait ever run out all the same (a workspace
+ * that was not set up, or one shared by overlapping calls), the int at byte
+ * bitnet_decode_stack_error_offset() of the workspace becomes 1, the kernel drains, and its results
+ * are worthless: the host checks the word when it next synchronises and resets the workspace.
+ * Return 0, 1 (shape / alignment), 2 (null), 3 (launch).
+ */
+long long bitnet_decode_stack_workspace_bytes(int n_layers, int B, int S, int dim, int ffn, int n_heads,
+                                              int n_kv_heads, int n_splits);
+int bitnet_decode_stack_reset(void* workspace, int n_layers, int B, int S, int dim, int ffn, int n_heads,
+                              int n_kv_heads, int n_splits, void* stream);
+int bitnet_decode_stack_error_offset(void);
+int bitnet_decode_stack(const void* entries, void* workspace, const uint16_t* h_in, uint16_t* h_out,
+                        const int64_t* positions, const float* rope_rows, int n_layers, int B, int S,
+                        int dim, int ffn, int n_heads, int n_kv_heads, int n_splits, int workgroups,
+                        int spin_limit, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

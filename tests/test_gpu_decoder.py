@@ -532,6 +532,49 @@ def test_host_checks_refuse_mismatched_buffers_before_any_launch():
 # The end-to-end workload at its real size: 30 layers, dim 2560, ffn 6912, 20 / 5 heads, vocabulary
 # 128256 (gpu/model.py:39-49), a 512-token seeded prompt, greedy decode (gpu/generate.py:264-288)
 # ---------------------------------------------------------------------------
+@pytest.mark.parametrize("workgroups", [0, 1, 7, 600])  # 600: more than can be resident, tasks by ticket
+@pytest.mark.parametrize("B,dim,ffn,nh,nkv,S,n_splits", [
+    (1, 128, 64, 1, 1, 33, 1), (2, 128, 64, 1, 1, 40, 16), (1, 1152, 2112, 9, 9, 70, 3), (2, 1024, 1984, 8, 1, 700, 5),
+    (1, 2560, 6912, 20, 5, 545, 8), (2, 2560, 6912, 20, 5, 300, 8),
+])
+def test_decode_stack_kernel_equals_the_kernels_per_layer(B, dim, ffn, nh, nkv, S, n_splits, workgroups):
+    args = decoder.ModelArgs(dim=dim, n_layers=2, n_heads=nh, n_kv_heads=nkv, vocab_size=256, ffn_dim=ffn)
+    model = _build(args, seed=dim + B)
+    caches = [model.make_cache(B, S, "cuda") for _ in range(2)]
+    for (k, v), (k2, v2) in zip(*caches):
+        k2.copy_(k.normal_())
+        v2.copy_(v.normal_())
+    cos, sin = decoder.rope_tables(128, S, args.rope_theta, "cuda")
+    ws = decoder.AttnWorkspace(B, nh, nkv, n_splits, "cuda")
+    assert decoder.DecodeStack.applies(model, B, caches[1], n_splits)
+    stack = decoder.DecodeStack(model, B, caches[1], n_splits)
+
+    def step(i, p):
+        pos = torch.full((B, 1), p, dtype=torch.int64, device="cuda")
+        pos[0, 0] = min(p + 1, S - 1)
+        tok = torch.arange(B, device="cuda").reshape(B, 1) + 5 * i
+        want = model.decode_hidden_fused(tok, pos, caches[0], cos, sin, ws)
+        h, rows = decoder.decode_step_begin(tok.reshape(B), pos.reshape(B), model.tok_embeddings.weight, cos, sin)
+        got = stack(h, pos.reshape(B), rows, workgroups)
+        stack.check()
+        assert np.array_equal(host_bits(got), host_bits(want)), (i, p)
+        for (k, v), (k2, v2) in zip(*caches):
+            assert torch.equal(k, k2) and torch.equal(v, v2), (i, p)
+        return h, pos.reshape(B), rows
+
+    for i, p in enumerate([0, 30, 31, 32, S // 2, S - 1, 3]):
+        operands = step(i, p)
+    # a wait that runs out is reported, and the next check clears it
+    if workgroups == 0:
+        stack(*operands, 0, 1)
+        with pytest.raises(_lib.BitLinearLibraryError, match="gave up"):
+            stack.check()
+        for (k, v), (k2, v2) in zip(*caches):  # that step wrote rows of its own
+            k2.copy_(k)
+            v2.copy_(v)
+        step(9, min(33, S - 1))
+
+
 @pytest.fixture(scope="module")
 def model_2b():
     model = _build(decoder.ModelArgs(), seed=0)
