@@ -96,6 +96,14 @@ SIGNATURES = {
         [_c_ptr, _c_ptr, ctypes.c_float, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr,
          _c_int, _c_int, _c_int, _c_ptr],
     ),
+    "bitnet_lm_head_logits": (
+        _c_int, [_c_ptr, _c_ptr, ctypes.c_float, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr],
+    ),
+    "bitnet_top_p_workspace_bytes": (ctypes.c_longlong, [_c_int, _c_int]),
+    "bitnet_top_p_sample": (
+        _c_int,
+        [_c_ptr, _c_ptr, _c_ptr, ctypes.c_float, ctypes.c_float, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr],
+    ),
     "bitnet_decode_stack_workspace_bytes": (ctypes.c_longlong, [_c_int] * 8),
     "bitnet_decode_stack_reset": (_c_int, [_c_ptr] + [_c_int] * 8 + [_c_ptr]),
     "bitnet_decode_stack_error_offset": (_c_int, []),

@@ -20,6 +20,7 @@ SOURCES = {
     os.path.join(PKG_DIR, "csrc", "bitlinear_hip.hip"): [],
     os.path.join(PKG_DIR, "csrc", "decoder_ops.hip"): [],
     os.path.join(PKG_DIR, "csrc", "pack.hip"): [],
+    os.path.join(PKG_DIR, "csrc", "sample.hip"): [],
     os.path.join(PKG_DIR, "csrc", "decode_stack.hip"): ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     # keep the attention kernels' accumulators in the vector register file (see the file's header)
     os.path.join(PKG_DIR, "csrc", "attn_prefill.hip"): ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],

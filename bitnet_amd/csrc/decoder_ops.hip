@@ -577,11 +577,12 @@ extern "C" int bitnet_lm_head_workgroups(int V) {
     return (V + rows_per_wg - 1) / rows_per_wg;
 }
 
-static int lm_head_greedy_impl(const uint16_t* h, const uint16_t* norm_weight, float eps, const uint16_t* emb,
+// token_out null: no token is chosen
+static int lm_head_impl(const uint16_t* h, const uint16_t* norm_weight, float eps, const uint16_t* emb,
                                uint16_t* y_ws, float* logits, int64_t* token_out, float* part_val, int* part_idx,
                                const LmStepBook& book, int B, int V, int K, void* stream) {
     if (B < 1 || B > kLmMaxTokens || V < 1 || K < 64 || (K % 64) != 0) return 1;
-    if (!h || !norm_weight || !emb || !y_ws || !token_out || !part_val || !part_idx) return 2;
+    if (!h || !norm_weight || !emb || !y_ws || !(token_out || logits) || !part_val || !part_idx) return 2;
     if ((((uintptr_t)h) | ((uintptr_t)norm_weight) | ((uintptr_t)emb) | ((uintptr_t)y_ws) | ((uintptr_t)part_val) |
          ((uintptr_t)part_idx)) & 15u)
         return 1;
@@ -615,14 +616,23 @@ static int lm_head_greedy_impl(const uint16_t* h, const uint16_t* norm_weight, f
         hipLaunchKernelGGL(lm_head_kernel, dim3(nparts), dim3(kLmThreads), lds, (hipStream_t)stream, y_ws, emb, logits, part_val,
                            part_idx, B, V, K);
     }
-    hipLaunchKernelGGL(lm_head_final_kernel, dim3(1), dim3(kLmFinalThreads), 0, (hipStream_t)stream, part_val, part_idx, token_out, nparts, B, book);
+    if (token_out)
+        hipLaunchKernelGGL(lm_head_final_kernel, dim3(1), dim3(kLmFinalThreads), 0, (hipStream_t)stream, part_val, part_idx, token_out, nparts, B, book);
     return hipGetLastError() == hipSuccess ? 0 : 3;
+}
+
+extern "C" int bitnet_lm_head_logits(const uint16_t* h, const uint16_t* norm_weight, float eps, const uint16_t* emb,
+                                     uint16_t* y_ws, float* logits, float* part_val, int* part_idx, int B, int V, int K,
+                                     void* stream) {
+    return lm_head_impl(h, norm_weight, eps, emb, y_ws, logits, nullptr, part_val, part_idx,
+                        LmStepBook{nullptr, nullptr, nullptr, nullptr}, B, V, K, stream);
 }
 
 extern "C" int bitnet_lm_head_greedy(const uint16_t* h, const uint16_t* norm_weight, float eps, const uint16_t* emb,
                                      uint16_t* y_ws, float* logits, int64_t* token_out, float* part_val,
                                      int* part_idx, int B, int V, int K, void* stream) {
-    return lm_head_greedy_impl(h, norm_weight, eps, emb, y_ws, logits, token_out, part_val, part_idx,
+    if (!token_out) return 2;
+    return lm_head_impl(h, norm_weight, eps, emb, y_ws, logits, token_out, part_val, part_idx,
                                LmStepBook{nullptr, nullptr, nullptr, nullptr}, B, V, K, stream);
 }
 
@@ -631,6 +641,7 @@ extern "C" int bitnet_lm_head_greedy_step(const uint16_t* h, const uint16_t* nor
                                           int* part_idx, int64_t* next_input, int64_t* positions, int64_t* history,
                                           int64_t* step_idx, int B, int V, int K, void* stream) {
     if ((history != nullptr) != (step_idx != nullptr)) return 2;
-    return lm_head_greedy_impl(h, norm_weight, eps, emb, y_ws, logits, token_out, part_val, part_idx,
+    if (!token_out) return 2;
+    return lm_head_impl(h, norm_weight, eps, emb, y_ws, logits, token_out, part_val, part_idx,
                                LmStepBook{next_input, positions, history, step_idx}, B, V, K, stream);
 }

@@ -237,6 +237,55 @@ def lm_head_greedy(h, norm: "RMSNorm", emb_weight, workspace: LmHeadWorkspace, t
     return token_out
 
 
+def lm_head_logits(h, norm: "RMSNorm", emb_weight, workspace: LmHeadWorkspace, logits_out):
+    """lm_head_greedy's logits without the choice of a token (bitnet_lm_head_logits)."""
+    B, K = h.shape
+    st = _lib.load_library().bitnet_lm_head_logits(
+        _ptr(h), _ptr(norm.weight), norm.eps, _ptr(emb_weight), _ptr(workspace.y), _ptr(logits_out), _ptr(workspace.part_val),
+        _ptr(workspace.part_idx), B, emb_weight.shape[0], K, _stream_ptr())
+    if st != 0:
+        raise _lib.BitLinearLibraryError(f"bitnet_lm_head_logits: status {st}")
+    return logits_out
+
+
+class TopPSampler:
+    """top_p_sample(softmax(logits / temperature), top_p) for logits of bf16
+    values on the GPU, as three launches (bitnet_top_p_sample) behind torch's
+    noise: the same draws for the same generator state."""
+
+    def __init__(self, batch: int, vocab: int, device):
+        self.shape = (batch, vocab)
+        self.workspace = torch.empty(_lib.load_library().bitnet_top_p_workspace_bytes(batch, vocab), dtype=torch.uint8, device=device)
+        self.noise = torch.empty(batch, vocab, dtype=torch.float32, device=device)
+        self.error = torch.zeros(1, dtype=torch.int32, device="cpu", pin_memory=True)  # written by the kernels
+
+    @staticmethod
+    def applies(batch: int, vocab: int, temperature: float, top_p: float) -> bool:
+        """(Short rows are left to torch: there is little to gain, and torch.sort, which is not stable on rows of up to
+        some hundred values, draws among tokens of equal probability in an order of its own.)"""
+        return (vocab >= 1024 and 1e-30 < temperature < 1e30 and top_p >= 0.0
+                and _lib.load_library().bitnet_top_p_workspace_bytes(batch, vocab) > 0)
+
+    def __call__(self, logits, temperature: float, top_p: float, rng, token_out, next_input=None, positions=None, history_row=None):
+        """token_out int64 [B] (on the device or pinned); next_input = token, positions += 1, history_row = token if given."""
+        if logits.shape != self.shape or logits.dtype != torch.float32 or not logits.is_contiguous():
+            raise ValueError("TopPSampler: logits do not match the shape it was made for")
+        self.noise.exponential_(1.0, generator=rng)
+        opt = lambda t: _ptr(t) if t is not None else None
+        st = _lib.load_library().bitnet_top_p_sample(
+            _ptr(logits), _ptr(self.noise), _ptr(self.workspace), temperature, top_p, _ptr(token_out), opt(next_input), opt(positions),
+            opt(history_row), _ptr(self.error), *self.shape, _stream_ptr())
+        if st != 0:
+            raise _lib.BitLinearLibraryError(f"bitnet_top_p_sample: status {st}")
+        return token_out
+
+    def check(self) -> None:
+        """Behind a synchronisation: raises if some row since the last check had no distribution to draw from."""
+        if int(self.error[0]):
+            self.error.zero_()
+            raise RuntimeError("top-p sampling: a row of logits holds inf or nan")
+
+
 def norm_bitlinear(x, norm: "RMSNorm", lin: BitLinearKernel, glu: bool = False, residual=None):
     """[squared-ReLU gate ->] RMSNorm -> BitLinearKernel.forward [-> + residual]
     through bitlinear_norm_forward_bf16: one kernel for small activation blocks,
@@ -597,14 +646,19 @@ class Generator:
         self.cache = model.make_cache(batch, max_seq, dev)
         self.tok = torch.zeros(batch, 1, dtype=torch.int64, device=dev)
         self.pos = torch.zeros(batch, 1, dtype=torch.int64, device=dev)
-        self.next_tok = torch.zeros(batch, dtype=torch.int64, device=dev)
         self.graph: Optional[torch.cuda.CUDAGraph] = None
-        self.stack: Optional[DecodeStack] = None  # of the captured step, where the model is one it takes
+        self._logits_graph: Optional[torch.cuda.CUDAGraph] = None  # the step up to its logits
+        self.stack: Optional[DecodeStack] = None  # of the captured steps, where the model is one it takes
         self.use_graph = use_graph
         # final norm + bf16 LM head + greedy token as two launches of the library
         self.lm_head = (self.fused and fused_head and model.output.weight.dtype == torch.bfloat16 and a.dim % 64 == 0
                         and model.output.bias is None)
         self.lm_ws = LmHeadWorkspace(batch, a.vocab_size, a.dim, dev) if self.lm_head else None
+        # with the library's LM head, host memory that its last kernel writes: the test for an end token is then a
+        # look at it, where two kernels, a copy and their launches left the GPU idle for some 50 us a step
+        self.next_tok = torch.zeros(batch, dtype=torch.int64, device="cpu" if self.lm_head else dev, pin_memory=self.lm_head)
+        self._logits: Optional[torch.Tensor] = None
+        self._sampler: Optional[TopPSampler] = None
         # generated tokens of a decode() call, written from inside the step so that a graph replay is the whole step
         self.history = torch.zeros(max_seq, batch, dtype=torch.int64, device=dev)
         self.step_idx = torch.zeros(1, dtype=torch.int64, device=dev)
@@ -614,16 +668,17 @@ class Generator:
         self._pf_graphs: dict = {}
         self._rows = torch.arange(batch, device=dev)
 
+    def _hidden(self, stack: Optional[DecodeStack]):
+        if stack is not None:
+            return self.model.decode_hidden_stack(self.tok, self.pos, self.cos, self.sin, stack)
+        return self.model.decode_hidden_fused(self.tok, self.pos, self.cache, self.cos, self.sin, self.attn_ws)
+
     def _step(self, stack: Optional[DecodeStack] = None):
         """One decode step including its bookkeeping: next token -> history and
         the input of the following step, position + 1."""
         if self.lm_head:
-            if stack is not None:
-                h = self.model.decode_hidden_stack(self.tok, self.pos, self.cos, self.sin, stack)
-            else:
-                h = self.model.decode_hidden_fused(self.tok, self.pos, self.cache, self.cos, self.sin, self.attn_ws)
             # the step's bookkeeping rides on the last kernel of the LM head
-            lm_head_greedy(h, self.model.norm, self.model.output.weight, self.lm_ws, token_out=self.next_tok,
+            lm_head_greedy(self._hidden(stack), self.model.norm, self.model.output.weight, self.lm_ws, token_out=self.next_tok,
                            next_input=self.tok, positions=self.pos, history=self.history, step_idx=self.step_idx)
             return
         else:
@@ -637,20 +692,35 @@ class Generator:
         self.tok.copy_(self.next_tok.view(-1, 1))
         self.pos.add_(1)
 
-    def _capture(self):
+    def _logits_step(self, stack: Optional[DecodeStack] = None):
+        """A decode step up to its logits; the token's choice does the bookkeeping."""
+        lm_head_logits(self._hidden(stack), self.model.norm, self.model.output.weight, self.lm_ws, self._logits)
+
+    def _capture(self, step):
+        """step(stack) as a graph.  It runs once on the way: the caller's inputs are in place, and tok and pos change."""
         a = self.model.args
-        if (self.lm_head and self.model.tok_embeddings.weight.dtype == torch.bfloat16 and a.dim % 8 == 0
+        if (self.stack is None and self.lm_head and self.model.tok_embeddings.weight.dtype == torch.bfloat16 and a.dim % 8 == 0
                 and DecodeStack.applies(self.model, self.batch, self.cache, self.attn_ws.n_splits)):
             self.stack = DecodeStack(self.model, self.batch, self.cache, self.attn_ws.n_splits)
+        saved = [(ck.clone(), cv.clone()) for ck, cv in self.cache]
         s = torch.cuda.Stream()
         s.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(s):
-            self._step(self.stack)  # warm-up outside the graph
+            step(self.stack)  # warm-up outside the graph
         torch.cuda.current_stream().wait_stream(s)
         torch.cuda.synchronize()
-        self.graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(self.graph):
-            self._step(self.stack)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            step(self.stack)
+        for (ck, cv), (sk, sv) in zip(self.cache, saved):
+            ck.copy_(sk)
+            cv.copy_(sv)
+        return graph
+
+    def _ended(self, eos_id: int) -> bool:
+        """Whether the step just issued produced eos_id for any sequence (waits for it)."""
+        torch.cuda.current_stream().synchronize()
+        return bool((self.next_tok == eos_id).any())
 
     def _check(self) -> None:
         """Raises if a wait inside the steps since the last check gave up (one small copy to the host)."""
@@ -754,12 +824,7 @@ class Generator:
         self._set_positions(start_pos)
         if self.use_graph and self.graph is None:
             # capture with the real inputs in place; the captured step is re-run below
-            saved_k = [ck.clone() for ck, _ in self.cache]
-            saved_v = [cv.clone() for _, cv in self.cache]
-            self._capture()
-            for (ck, cv), sk, sv in zip(self.cache, saved_k, saved_v):
-                ck.copy_(sk)
-                cv.copy_(sv)
+            self.graph = self._capture(self._step)
             self.tok.copy_(first.view(-1, 1))
             self._set_positions(start_pos)
         self.step_idx.zero_()
@@ -770,7 +835,7 @@ class Generator:
             else:
                 self._step()
             taken = i + 1
-            if eos_id is not None and bool((self.next_tok == eos_id).any()):
+            if eos_id is not None and self._ended(eos_id):
                 break
         out = self.history[:taken].clone()
         self._check()
@@ -812,8 +877,8 @@ class Generator:
         the top_p nucleus (the reference's 0.7 / 0.95), until gen_length tokens
         are out or, with eos_id, until any sequence has produced it.  Every
         answer is cut behind its first eos_id.  Greedy steps replay the captured
-        graph of the whole step; a sampled step runs the same kernels and draws
-        with torch between them (`rng` makes the draws reproducible).  A dict
+        graph of the whole step; a sampled step replays the captured step up to its
+        logits and draws behind it (`rng` makes the draws reproducible).  A dict
         passed as `timings` receives what the reference's Stats phases report
         (gpu/stats.py, gpu/generate.py:243-288): prefill_s, decode_s,
         decode_tokens (steps x sequences) and decode_tokens_per_s; it costs two
@@ -837,7 +902,13 @@ class Generator:
             torch.cuda.synchronize()
             t_start = time.perf_counter()
         first, logits, lens = self._prefill_ragged(prompts, pad_id, use_sampling)
-        if use_sampling:
+        # the library's sampler takes the LM head kernel's logits (bf16 values)
+        native = use_sampling and self.lm_head and TopPSampler.applies(self.batch, vocab, temperature, top_p)
+        if native:
+            if self._sampler is None:
+                self._sampler = TopPSampler(self.batch, vocab, self.tok.device)
+            first = self._sampler(logits, temperature, top_p, rng, torch.empty_like(first))
+        elif use_sampling:
             first = draw(logits)
         if timings is not None:
             torch.cuda.synchronize()
@@ -849,29 +920,40 @@ class Generator:
             if not use_sampling:
                 out.append(self.decode(first, lens, gen_length - 1, eos_id=eos_id))
             else:
-                if logits is None or not self.lm_head:
-                    logits = torch.empty(self.batch, vocab, dtype=torch.float32, device=self.tok.device)
                 self.tok.copy_(first.view(-1, 1))
                 self._set_positions(lens)
+                if self.lm_head and self._logits is None:
+                    self._logits = torch.empty(self.batch, vocab, dtype=torch.float32, device=self.tok.device)
+                if self.lm_head and self.use_graph and self._logits_graph is None:
+                    self._logits_graph = self._capture(self._logits_step)
+                taken = 0
                 for _ in range(gen_length - 1):
                     if self.lm_head:
-                        h = self.model.decode_hidden_fused(self.tok, self.pos, self.cache, self.cos, self.sin, self.attn_ws)
-                        lm_head_greedy(h, self.model.norm, self.model.output.weight, self.lm_ws, logits_out=logits)
-                        step_logits = logits
+                        if self.use_graph:
+                            self._logits_graph.replay()
+                        else:
+                            self._logits_step()
+                        step_logits = self._logits
                     elif self.fused:
                         step_logits = self.model.forward_decode_fused(self.tok, self.pos, self.cache, self.cos, self.sin,
                                                                       self.attn_ws)[:, -1]
                     else:
                         step_logits = self.model.forward_tokens(self.tok, self.pos, self.cache, self.cos, self.sin)[:, -1]
-                    nxt = draw(step_logits)
-                    out.append(nxt.view(1, -1))
-                    self.tok.copy_(nxt.view(-1, 1))
-                    self.pos.add_(1)
-                    if eos_id is not None and bool((nxt == eos_id).any()):
+                    if native:
+                        self._sampler(step_logits, temperature, top_p, rng, self.next_tok, self.tok, self.pos, self.history[taken])
+                    else:
+                        self.next_tok.copy_(draw(step_logits))
+                        self.history[taken].copy_(self.next_tok)
+                        self.tok.copy_(self.next_tok.view(-1, 1))
+                        self.pos.add_(1)
+                    taken += 1
+                    if eos_id is not None and self._ended(eos_id):
                         break
-                if self.fused:
-                    self.attn_ws.check()
+                out.append(self.history[:taken])
+                self._check()
         tokens = torch.cat(out, dim=0).t().tolist()  # [B][steps]
+        if native:
+            self._sampler.check()
         if timings is not None:
             torch.cuda.synchronize()
             t_end = time.perf_counter()

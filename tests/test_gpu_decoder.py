@@ -312,6 +312,53 @@ def test_lm_head_greedy_kernel(B, V, K, which):
     assert torch.equal(tok2, tok)
 
 
+@pytest.mark.parametrize("logits", ["normal", "flat", "peaked", "masked", "tiny", "huge"])
+@pytest.mark.parametrize("B,V", [(1, 128256), (4, 128256), (3, 1024), (16, 4111), (2, 17), (1, 1)])
+def test_top_p_sampler_draws_what_torch_draws(B, V, logits):
+    gen = torch.Generator(device="cuda").manual_seed(V + B)
+    x = torch.randn(B, V, generator=gen, device="cuda")
+    if logits == "flat":
+        x = torch.zeros_like(x)
+    elif logits == "peaked":
+        x = x * 8.0
+    elif logits == "masked":
+        x = torch.where(torch.rand(B, V, generator=gen, device="cuda") < 0.5, float("-inf"), x)
+        x[:, 0] = 0.5
+    elif logits == "tiny":  # values that share a bucket, in which their order counts
+        x = x * 2.0**-21
+    elif logits == "huge":
+        x = x * 2.0**40
+    x = x.to(torch.bfloat16).float()
+    sampler = decoder.TopPSampler(B, V, "cuda")
+    tok = torch.zeros(B, dtype=torch.int64, device="cpu", pin_memory=True)
+    nxt, pos, row = (torch.full((B,), i, dtype=torch.int64, device="cuda") for i in range(3))
+    for draw, (t, p) in enumerate([(0.7, 0.95), (0.7, 0.95), (1.3, 0.5), (1.0, 1.0), (1.0, 0.0), (0.1, 0.9)]):
+        # (float64: where probabilities differ by less than a float32 resolves, torch's own order is one by index)
+        probs = torch.softmax(x.double() / t, dim=-1)
+        if logits == "tiny":  # ranked by the logits: their probabilities differ in the last bits only
+            order = torch.sort(x, dim=-1, descending=True, stable=True)[1]
+        else:
+            order = torch.sort(probs, dim=-1, descending=True, stable=True)[1]
+        ranked = torch.gather(probs, -1, order)
+        kept = torch.where(torch.cumsum(ranked, -1) - ranked > p + 1e-12, 0.0, ranked)
+        q = torch.empty(B, V, device="cuda").exponential_(1.0, generator=torch.Generator(device="cuda").manual_seed(draw))
+        want = torch.gather(order, -1, torch.argmax(kept / q, dim=-1, keepdim=True)).view(-1)
+        sampler(x, t, p, torch.Generator(device="cuda").manual_seed(draw), tok, nxt, pos, row)
+        torch.cuda.synchronize()
+        sampler.check()
+        assert tok.tolist() == want.tolist(), (draw, t, p)
+        assert nxt.tolist() == want.tolist() and row.tolist() == want.tolist() and pos.tolist() == [draw + 2] * B
+        if logits in ("normal", "peaked", "flat") and V >= 1024:
+            ref = decoder.top_p_sample(torch.softmax(x / t, dim=-1), p, torch.Generator(device="cuda").manual_seed(draw))
+            assert tok.tolist() == ref.view(-1).tolist(), (draw, t, p)
+    for bad in (float("nan"), float("inf")):
+        x[B - 1, V - 1] = bad
+        sampler(x, 1.0, 0.9, gen, tok)
+        torch.cuda.synchronize()
+        with pytest.raises(RuntimeError, match="inf or nan"):
+            sampler.check()
+
+
 def test_generator_with_and_without_the_lm_head_kernel_agree():
     args = decoder.ModelArgs(dim=256, n_layers=2, n_heads=2, n_kv_heads=1, vocab_size=512, ffn_dim=512)
     model = _build(args, seed=3)
