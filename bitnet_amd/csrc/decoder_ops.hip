@@ -8,6 +8,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include <atomic>
 
 #include "bitnet_decoder_ops.h"
@@ -252,22 +254,16 @@ __global__ __launch_bounds__(kLmThreads) void lm_head_stream_kernel(const uint16
     const int steps = K >> 9;  // 512 k per step
     const int groups = (V + kLsRows - 1) / kLsRows;
     const int nwaves = gridDim.x * (kLmThreads / 64);
-    int grp = blockIdx.x * (kLmThreads / 64) + wave;  // persistent: groups grp, grp + nwaves, ...
+    int grp = __builtin_amdgcn_readfirstlane((int)blockIdx.x * (kLmThreads / 64) + wave);  // persistent: groups grp, grp + nwaves, ...
 
-    // first 1 KB of each of the first group's rows (a wave without a group re-reads the last row)
-    const v4u* wp[kLsRows];
-    v4u w[kLsRows];
-    auto group_rows = [&](int gidx) {
-#pragma unroll
-        for (int r = 0; r < kLsRows; ++r) {
-            int row = gidx * kLsRows + r;
-            row = row < V ? row : V - 1;
-            wp[r] = (const v4u*)(emb + (size_t)row * K) + lane;
-        }
+    // the 1 KB of row r of a group that step s needs (rows past the end: the last one again)
+    auto piece = [&](int gidx, int r, int s) {
+        const int row = gidx * kLsRows + r;
+        return (const v4u*)(emb + (size_t)(row < V ? row : V - 1) * K + s * 512) + lane;
     };
-    group_rows(grp < groups ? grp : groups - 1);
+    v4u w[kLsRows];
 #pragma unroll
-    for (int r = 0; r < kLsRows; ++r) w[r] = __builtin_nontemporal_load(wp[r]);
+    for (int r = 0; r < kLsRows; ++r) w[r] = __builtin_nontemporal_load(piece(grp < groups ? grp : groups - 1, r, 0));
     {
         const int nvec = (B * K) >> 3;
         for (int i = tid; i < nvec; i += kLmThreads) *(uint4*)(lds_y + (size_t)i * 16) = *(const uint4*)(y + (size_t)i * 8);
@@ -287,6 +283,7 @@ __global__ __launch_bounds__(kLmThreads) void lm_head_stream_kernel(const uint16
         float acc[NV];
 #pragma unroll
         for (int i = 0; i < NV; ++i) acc[i] = 0.0f;
+#pragma unroll 1
         for (int s = 0; s < steps; ++s) {
             v4u xs[TB];
 #pragma unroll
@@ -294,41 +291,48 @@ __global__ __launch_bounds__(kLmThreads) void lm_head_stream_kernel(const uint16
                 const int tok = t < B ? t : B - 1;
                 xs[t] = *(const v4u*)(lds_y + (size_t)tok * 2 * K + (size_t)s * 1024 + lane * 16);
             }
-            // what to request next: this group's next 1 KB per row, or the first 1 KB of the wave's next group
-            int off = (s + 1) * 64;
-            if (s + 1 == steps) {  // uniform
-                const int nxt = grp + nwaves;
-                group_rows(nxt < groups ? nxt : grp);
-                off = 0;
-            }
+            // What to request next: this group's next 1 KB per row, or the first 1 KB of the wave's next group.  Into the
+            // registers just used, behind their use (the barriers for the scheduler keep it there): requested earlier,
+            // into others, the values are moved at the step's end, where the wave then waits for all of them.  The
+            // indices by selection, not by a branch, over which the compiler makes several copies of the loop.
+            const bool last = s + 1 == steps;
+            const int nxt = last && grp + nwaves < groups ? grp + nwaves : grp, ns = last ? 0 : s + 1;
 #pragma unroll
             for (int r = 0; r < kLsRows; ++r) {
-                const v4u wr = w[r];
-                w[r] = __builtin_nontemporal_load(wp[r] + off);
 #pragma unroll
                 for (int t = 0; t < TB; ++t) {
                     float a = acc[r * TB + t];
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) a = bf16_dot2(wr[j], xs[t][j], a);
+                    for (int j = 0; j < 4; ++j) a = bf16_dot2(w[r][j], xs[t][j], a);
                     acc[r * TB + t] = a;
                 }
+                __builtin_amdgcn_sched_barrier(0);
+                w[r] = __builtin_nontemporal_load(piece(nxt, r, ns));
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
         // halving butterfly: after the stage with lane-xor mask m a lane keeps the half of its values
         // chosen by its bit m; after log2(NV) stages lane l holds pair l >> log2(64 / NV), still as a
         // partial over the lanes that differ in the low bits, which a plain xor reduction finishes
-        int m = 32;
-#pragma unroll
-        for (int n = NV; n > 1; n >>= 1) {
+        // (the stages written out: as a loop over n it was not unrolled at 32 pairs, and every access to acc became a
+        // chain of selects, 5800 instructions)
+        auto stage = [&](auto half, int m) {
+            constexpr int H = decltype(half)::value;
             const bool up = (lane & m) != 0;
 #pragma unroll
-            for (int i = 0; i < n / 2; ++i) {
-                const float keep = up ? acc[i + n / 2] : acc[i];
-                const float send = up ? acc[i] : acc[i + n / 2];
+            for (int i = 0; i < H; ++i) {
+                const float keep = up ? acc[i + H] : acc[i];
+                const float send = up ? acc[i] : acc[i + H];
                 acc[i] = keep + __shfl_xor(send, m);
             }
-            m >>= 1;
-        }
+        };
+        int m = 32;
+        if constexpr (NV >= 64) stage(std::integral_constant<int, 32>{}, m), m >>= 1;
+        if constexpr (NV >= 32) stage(std::integral_constant<int, 16>{}, m), m >>= 1;
+        if constexpr (NV >= 16) stage(std::integral_constant<int, 8>{}, m), m >>= 1;
+        stage(std::integral_constant<int, 4>{}, m), m >>= 1;
+        stage(std::integral_constant<int, 2>{}, m), m >>= 1;
+        stage(std::integral_constant<int, 1>{}, m), m >>= 1;
         float total = acc[0];
         for (; m > 0; m >>= 1) total += __shfl_xor(total, m);
         const int vr = grp * kLsRows + pr;
