@@ -9,11 +9,13 @@
 // exist, and outputs go to their readers directly: every value is written through to memory once, and
 // readers poll for the values themselves.  Nobody waits for an acknowledgement, a counter or a launch;
 // such a hand-over measures 1.4 us, readers' barrier included.  30 layers at 512 positions, us:
-//                        one sequence   two
-//   launches                     755    875
-//   this kernel                  516    621
-// With more sequences the redundant part grows, every workgroup of a product normalises and quantizes
-// the rows of all tokens by itself: at three both take the same time, so two is where the range ends.
+//   sequences            1     2     3     4     8
+//   launches           755   875  1000  1070  1060
+//   this kernel        511   626   690   715   816
+// Up to two tokens every workgroup of a product normalises and quantizes the rows by itself, between their
+// arrival and its matrix instructions.  That part grows with the tokens (three: 1120 us).  Beyond two, one
+// task per token does it for all and publishes int8 rows, which are the matrix instructions' operand as they
+// lie in memory: one more hand-over, but a product's own work hardly depends on the tokens.
 //
 // Hand-over buffers.  Every (layer, step) has buffers of its own, in two sets that alternate between
 // launches; a launch fills the other set with a value that no result can have (bf16 0xffff, a NaN that
@@ -63,13 +65,17 @@ constexpr int kStLanes = kStWaves * 64;   // of the computing waves
 constexpr int kStThreads = kStLanes + 64;  // and the wave that fetches
 constexpr int kStUpwD = 10;       // 64-wide k-steps per wave of a product over the model width: up to 2560
 constexpr int kStUpwF = 27;       // ... over the feed-forward width: up to 6912
-constexpr int kStMaxTokens = 2;  // (see above)
+constexpr int kStDirect = 2;      // tokens up to which every product task quantizes its input (see above)
+constexpr int kStMaxTokens = 8;
 constexpr int kStMaxG = 8;        // query heads per kv head
 constexpr int kStSpinLimit = 1 << 19;   // polls (0.7 us each) before a wait gives up
 constexpr int kStModePolls = 64;        // polls before the mode is decided without all workgroups
 constexpr int kSc1 = kPollPolicy;       // device-coherent accesses
 typedef unsigned v2u __attribute__((ext_vector_type(2)));
 typedef int v2i __attribute__((ext_vector_type(2)));
+// Four int8 of quantized rows that mean "not written".  -128 comes from NaNs alone (|x| * scale rounds to 127 at most), and
+// a word of four of them is written as -127, -128, -128, -128 instead.  As an int, below every written word.
+constexpr int kUnsetBytes = (int)0x80808080;
 constexpr int kBeyond = 0x7ffffff0;     // an offset behind every descriptor: reads as zero, no access
 
 // one product of one layer
@@ -103,17 +109,20 @@ struct StackArgs {
     const __attribute__((address_space(4))) int64_t* positions;
     const float* rope_rows;
     int n_layers, B, dim, ffn, n_heads, n_kv, group, S, n_splits, attn_waves, spin_limit;  // group: query heads per kv head
-    int ends[5];  // cumulative task counts of a layer's phases
-    int f_layer, f_o, f_ha, f_g, f_hb;  // a set: bytes per layer, offsets in it
-    int set_bytes;
+    int ends[9];  // cumulative task counts of a layer's phases
+    // a set: bytes per layer and offsets in it; behind the bf16 values of all layers (set_values bytes) the quantized rows
+    int f_layer, f_o, f_ha, f_g, f_hb, f_rec;
+    int f_bytes;  // quantized rows per layer
+    int set_values, set_bytes;
     long long sets;     // offset of the first set in the workspace
     long long records;  // offset of the attention records
     float inv_dim, inv_ffn;  // correctly rounded reciprocals
 };
 typedef const __attribute__((address_space(4))) StackArgs* StackArgsPtr;  // the kernel's argument block
 
-// wqkv (two 16-row blocks a task), attention, wo (one block), w13 (two pairs of blocks, gated), w2 (one block)
-enum Phase { kP1 = 0, kAttn, kP3, kP4, kP5 };
+// wqkv (two 16-row blocks a task), attention, wo (one block), w13 (two pairs of blocks, gated), w2 (one block); in front
+// of each product, beyond kStDirect tokens, its input rows normalised and quantized, one token a task
+enum Phase { kQ1 = 0, kP1, kAttn, kQ3, kP3, kQ4, kP4, kQ5, kP5 };
 
 struct Work {
     int layer, ph, first, idx;  // idx: the task's number in its phase, whose first task is number `first` of the layer
@@ -236,17 +245,27 @@ __device__ __forceinline__ uint32_t quant2(uint32_t d, float s) {  // two bytes
     return __builtin_amdgcn_perm(quant_low_byte<0>(d & 0xffff0000u, s), quant_low_byte<0>(d << 16, s), 0x0c0c0400u);
 }
 
+// A quantized row's scale (bf16 bits) and the sums of its four waves' slices, 31 bits each: a set top bit is "not written"
+struct RowRecord {
+    int sum[4];
+    unsigned scale, pad[3];
+};
+static_assert(sizeof(RowRecord) == 32 && kStWaves == 4, "one 16-byte and one 4-byte load");
+
 template <int MT>
 struct Shared {
+    static constexpr int TQ = MT <= kStDirect ? MT : 1;  // rows that a task normalises
     // packed words of this task and the next two (an attention task keeps its waves' outputs in its buffer)
     __attribute__((aligned(16))) uint8_t words[kStBuffers][kStWordBytes];
-    __attribute__((aligned(16))) int8_t q[kStWaves][MT][kStUpwF * 64 + 80];  // a wave's quantized slices (reads go one step past)
-    int red[4][kStWaves][MT][16];                                       // the waves' partial sums: [row block][wave][token][row]
+    __attribute__((aligned(16))) int8_t q[kStWaves][TQ][MT <= kStDirect ? kStUpwF * 64 + 80 : 16];  // a wave's quantized slices (reads go one step past)
+    // the waves' partial sums: [row block][wave][token][row].  Twice where nothing else keeps a wave from writing the
+    // next task's while another still reads
+    int red[MT <= kStDirect ? 1 : 2][4][kStWaves][MT][16];
     float part_m[kDfMaxWaves][kStMaxG], part_l[kDfMaxWaves][kStMaxG];
     __attribute__((aligned(16))) uint16_t qb[kStMaxG][kHeadDim], knew[kHeadDim], vnew[kHeadDim];
     // exchanges between the computing waves: values with the number of the exchange
-    __attribute__((aligned(16))) v4i sumsq[MT][kStWaves];
-    __attribute__((aligned(16))) v2i amax[MT][kStWaves];
+    __attribute__((aligned(16))) v4i sumsq[TQ][kStWaves];
+    __attribute__((aligned(16))) v2i amax[TQ][kStWaves];
     __attribute__((aligned(16))) int met[kStWaves];
     // between them and the wave that fetches: counts of tasks
     __attribute__((aligned(16))) int consumed[kStWaves];
@@ -260,8 +279,9 @@ struct Shared {
 struct Task {
     int layer, ph, idx;
     float eps;
-    const uint16_t *src, *res;  // attention: the published q | k | v rows; the cache's k
-    uint16_t *dst, *aux;        // attention: the published outputs; the cache's v.  Products: aux = the norm's weights
+    const uint16_t *src, *res;  // attention: the published q | k | v rows; the cache's k.  Quantizers: res = the row's record
+    uint16_t *dst, *aux;        // attention: the published outputs; the cache's v.  Products: aux = the norm's weights, or,
+                                // where src are quantized rows, their records
     int K, n_out;               // attention: kv head, sequence
     float inv_k;                // attention: split
     int flags;                  // 1: src is published, 2: dst is.  Attention: the position
@@ -276,13 +296,15 @@ struct Values {
 template <int MT>
 struct Got {
     v4i e[4 * kStUpwD];     // the weights as MFMA operands: [row block][k-step], or the 27 steps of one block
-    Values<kStUpwF> f[MT];  // (the first members serve the shorter slices)
+    Values<kStUpwF> f[Shared<MT>::TQ];  // (the first members serve the shorter slices)
     uint4 g[kStMaxVec];     // norm weights of this lane's values
     uint16_t res;
 };
 
 template <int MT>
 struct Stack {
+    static constexpr int TQ = Shared<MT>::TQ;
+    static constexpr bool kDirect = MT <= kStDirect;
     StackArgsPtr a;
     Shared<MT>& sh;
     Waiter wt;
@@ -290,6 +312,7 @@ struct Stack {
     unsigned launch;
     int tid, lane, wave;
     int exchange;  // exchanges so far: the same in all computing waves
+    int turn;      // which part of `red`
 
     // Makes the compiler compute what follows from the thread's place and the arguments anew from here on: kept
     // over the whole loop of tasks, the addresses of all phases together do not fit the registers.
@@ -309,13 +332,13 @@ struct Stack {
 
     __device__ __forceinline__ Work locate(int layer, int r) const {
         Work w;
-        while (r >= a->ends[4]) {
-            r -= a->ends[4];
+        while (r >= a->ends[8]) {
+            r -= a->ends[8];
             ++layer;
         }
         int ph = 0, base = 0;
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 8; ++i)
             if (r >= a->ends[i]) {
                 ph = i + 1;
                 base = a->ends[i];
@@ -327,7 +350,7 @@ struct Stack {
         return w;
     }
     // product of a phase: 0 wqkv, 1 wo, 2 w13, 3 w2
-    static __device__ __forceinline__ int product_of(int ph) { return ph < kP3 ? 0 : ph - 1; }
+    static __device__ __forceinline__ int product_of(int ph) { return ph <= kAttn ? 0 : (ph - 1) >> 1; }
 
     __device__ __forceinline__ int batch() const { return MT == 1 ? 1 : a->B; }
 
@@ -369,27 +392,33 @@ struct Stack {
         uint64_t src, res = 0, dst, aux = (uint64_t)e->norm;
         int K = a->dim, n_out = a->dim, flags = 3;
         float inv_k = a->inv_dim;
-        switch (wk.ph) {
-            case kP1:
-                src = (uint64_t)h_before(l), dst = (uint64_t)qkv(l);
-                n_out = (a->n_heads + 2 * a->n_kv) * kHeadDim;
-                if (l == 0) flags = 2;
-                break;
-            case kAttn: {
-                src = (uint64_t)qkv(l), dst = (uint64_t)o(l), res = (uint64_t)e->ck, aux = (uint64_t)e->cv;
-                const int rest = wk.idx / a->n_kv;
-                K = wk.idx % a->n_kv, n_out = rest / a->n_splits, inv_k = __uint_as_float((unsigned)(rest % a->n_splits));
-                const int64_t p = a->positions[n_out];
-                flags = p < 0 ? 0 : (p >= (int64_t)a->S ? a->S - 1 : (int)p);
-                break;
+        // quantized rows of product i of the layer, and their records
+        auto bytes = [&](int i) { return (uint64_t)(set + a->set_values + (size_t)l * a->f_bytes + (size_t)i * a->B * a->dim); };
+        auto record = [&](int i) { return (uint64_t)(layer_set(l) + a->f_rec) + (uint64_t)(i * a->B) * sizeof(RowRecord); };
+        const int i = product_of(wk.ph);
+        if (wk.ph == kAttn) {
+            src = (uint64_t)qkv(l), dst = (uint64_t)o(l), res = (uint64_t)e->ck, aux = (uint64_t)e->cv;
+            const int rest = wk.idx / a->n_kv;
+            K = wk.idx % a->n_kv, n_out = rest / a->n_splits, inv_k = __uint_as_float((unsigned)(rest % a->n_splits));
+            const int64_t p = a->positions[n_out];
+            flags = p < 0 ? 0 : (p >= (int64_t)a->S ? a->S - 1 : (int)p);
+        } else {
+            src = (uint64_t)(i == 0 ? h_before(l) : i == 1 ? o(l) : i == 2 ? ha(l) : gate(l));
+            if (i == 0 && l == 0) flags &= ~1;
+            if (i == 3) K = a->ffn, inv_k = a->inv_ffn;
+            if (wk.ph == kP1 || wk.ph == kP3 || wk.ph == kP4 || wk.ph == kP5) {
+                if (!kDirect) src = bytes(i), aux = record(i);
+                dst = (uint64_t)(i == 0 ? qkv(l) : i == 1 ? ha(l) : i == 2 ? gate(l) : last ? a->h_out : hb(l));
+                if (i == 0) n_out = (a->n_heads + 2 * a->n_kv) * kHeadDim;
+                if (i == 1) res = (uint64_t)h_before(l);
+                if (i == 2) n_out = a->ffn;
+                if (i == 3) res = (uint64_t)ha(l);
+                if (i == 3 && last) flags &= ~2;
+            } else {
+                src += (uint64_t)wk.idx * K * 2;
+                dst = bytes(i) + (uint64_t)wk.idx * K;
+                res = record(i) + (uint64_t)wk.idx * sizeof(RowRecord);
             }
-            case kP3: src = (uint64_t)o(l), dst = (uint64_t)ha(l), res = (uint64_t)h_before(l); break;
-            case kP4: src = (uint64_t)ha(l), dst = (uint64_t)gate(l), n_out = a->ffn; break;
-            default:
-                src = (uint64_t)gate(l), dst = (uint64_t)(last ? a->h_out : hb(l)), res = (uint64_t)ha(l);
-                K = a->ffn, inv_k = a->inv_ffn;
-                if (last) flags = 1;
-                break;
         }
         if (lane == 0) {
             lds_put(to[0], v4i{l < a->n_layers ? l : -1, wk.ph, wk.idx, (int)__float_as_uint(e->eps)});
@@ -409,7 +438,7 @@ struct Stack {
     }
     // the packed words of a task into LDS, in pieces of 1 KB
     __device__ __forceinline__ void fetch(const Work& wk, const uint32_t* w, int buffer) const {
-        if (wk.ph == kAttn) return;
+        if (wk.ph != kP1 && wk.ph != kP3 && wk.ph != kP4 && wk.ph != kP5) return;
         const int K = wk.ph == kP5 ? a->ffn : a->dim;
         const int half = a->ffn >> 4;  // row blocks of one half of w13
         const bool pairs = wk.ph == kP1 || wk.ph == kP4;
@@ -486,7 +515,7 @@ struct Stack {
     template <int UPW, bool RES>
     __device__ __forceinline__ void gather_slices(const Task& tk, Got<MT>& got) {
         typedef Slice<UPW> S;
-        const int K = tk.K, B = batch();
+        const int K = tk.K, B = TQ == 1 ? 1 : a->B;
         int off[S::kVec];
         slice_offsets<UPW>(K * 2, off);
         const __amdgpu_buffer_rsrc_t rows = make_rsrc(tk.src, B * K * 2);
@@ -498,7 +527,7 @@ struct Stack {
             if (RES) got.res = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rs, res_off, 0, kSc1);
             unsigned m = RES ? (unsigned)got.res << 16 : 0u;
 #pragma unroll
-            for (int t = 0; t < MT; ++t) {
+            for (int t = 0; t < TQ; ++t) {
                 Values<kStUpwF>& v = got.f[t];
                 const int at = (t < B ? t : B - 1) * K * 2;  // tokens beyond the batch repeat the last one
 #pragma unroll
@@ -511,7 +540,7 @@ struct Stack {
                 }
             }
 #pragma unroll
-            for (int t = 0; t < MT; ++t) {
+            for (int t = 0; t < TQ; ++t) {
                 const Values<kStUpwF>& v = got.f[t];
 #pragma unroll
                 for (int i = 0; i < S::kFull; ++i) m = unset_max(unset_max(unset_max(unset_max(m, v.full[i].x), v.full[i].y), v.full[i].z), v.full[i].w);
@@ -522,12 +551,13 @@ struct Stack {
         }
     }
 
-    // norm + quantizer of the wave's slices, products, outputs.  RPW 1, 2: row blocks; 4: two pairs (x1, x3), gated
-    template <int UPW, int RPW, bool RES>
-    __device__ __forceinline__ void product(const Task& tk, int k, Got<MT>& got) {
+    // norm and quantizer of the wave's slices: the scales, the slices' sums, the bytes by put8 (8 of them, a 512-value
+    // piece's) and put_rest (S::T of them)
+    template <int UPW, class Put8, class PutRest>
+    __device__ __forceinline__ void quantize(const Task& tk, Got<MT>& got, float (&s)[TQ], int (&sum)[TQ], Put8 put8, PutRest put_rest) {
         typedef Slice<UPW> S;
 #pragma unroll
-        for (int t = 0; t < MT; ++t) {
+        for (int t = 0; t < TQ; ++t) {
             const Values<kStUpwF>& v = got.f[t];
             double sq = 0.0;  // lanes without a value hold zeros
 #pragma unroll
@@ -540,7 +570,7 @@ struct Stack {
         }
         ++exchange;
 #pragma unroll
-        for (int t = 0; t < MT; ++t) {
+        for (int t = 0; t < TQ; ++t) {
             Values<kStUpwF>& v = got.f[t];
             v4i x[kStWaves];
             for (;;) {
@@ -569,10 +599,8 @@ struct Stack {
             if (lane == 63) lds_put(sh.amax[t][wave], v2i{(int)am, exchange + 1});
         }
         ++exchange;
-        float s[MT];
-        int q2[MT];  // twice the sum of the slice: the +2 of the stored codes
 #pragma unroll
-        for (int t = 0; t < MT; ++t) {
+        for (int t = 0; t < TQ; ++t) {
             const Values<kStUpwF>& v = got.f[t];
             v4i x[2];
             for (;;) {
@@ -584,26 +612,40 @@ struct Stack {
             const uint32_t am = (uint32_t)max(max(x[0].x, x[0].z), max(x[1].x, x[1].z));
             // quant_scale<0>
             s[t] = bf16_to_f32(f32_to_bf16_rne(reciprocal(fmaxf(__uint_as_float(am << 16), 1e-5f)) * 127.0f));
-            int8_t* q = sh.q[wave][t];
             int part = 0;
 #pragma unroll
             for (int i = 0; i < S::kFull; ++i) {
                 const uint2 qv = quant_vec8<0>(v.full[i], s[t]);
-                *(uint2*)(q + i * 512 + lane * 8) = qv;
+                put8(t, i, qv);
                 part = __builtin_amdgcn_sdot4((int)qv.x, 0x01010101, __builtin_amdgcn_sdot4((int)qv.y, 0x01010101, part, false), false);
             }
             if (S::T) {
                 uint32_t r = quant2(v.rest[0], s[t]);
                 if (S::T == 4) r |= quant2(v.rest[1], s[t]) << 16;
-                if (lane * S::T < S::kRest) {
-                    if (S::T == 2) *(uint16_t*)(q + S::kFull * 512 + lane * 2) = (uint16_t)r;
-                    if (S::T == 4) *(uint32_t*)(q + S::kFull * 512 + lane * 4) = r;
-                }
+                put_rest(t, r);
                 part = __builtin_amdgcn_sdot4((int)r, 0x01010101, part, false);
             }
             part = wave_reduce_last(part, [](int x, int y) { return x + y; });
-            q2[t] = 2 * __builtin_amdgcn_readlane(part, 63);
+            sum[t] = __builtin_amdgcn_readlane(part, 63);
         }
+    }
+
+    // norm + quantizer of the wave's slices, products, outputs.  RPW 1, 2: row blocks; 4: two pairs (x1, x3), gated
+    template <int UPW, int RPW, bool RES>
+    __device__ __forceinline__ void product(const Task& tk, int k, Got<MT>& got) {
+        typedef Slice<UPW> S;
+        float s[MT];
+        int q2[MT];  // twice the sum of the slice: the +2 of the stored codes
+        quantize<UPW>(
+            tk, got, s, q2, [&](int t, int i, uint2 v) { *(uint2*)(sh.q[wave][t] + i * 512 + lane * 8) = v; },
+            [&](int t, uint32_t r) {
+                if (lane * S::T < S::kRest) {
+                    if (S::T == 2) *(uint16_t*)(sh.q[wave][t] + S::kFull * 512 + lane * 2) = (uint16_t)r;
+                    if (S::T == 4) *(uint32_t*)(sh.q[wave][t] + S::kFull * 512 + lane * 4) = r;
+                }
+            });
+#pragma unroll
+        for (int t = 0; t < MT; ++t) q2[t] *= 2;
         // the same wave wrote its slices and reads them: LDS operations of a wave complete in order
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -645,23 +687,29 @@ struct Stack {
                 v[r] += __builtin_amdgcn_update_dpp(0, v[r], 0x120 + MT, 0xF, 0xF, true);  // row_ror
                 if (SP == 4) v[r] += __builtin_amdgcn_update_dpp(0, v[r], 0x120 + 2 * MT, 0xF, 0xF, true);
             }
-            if (p < MT) *(v4i*)&sh.red[i][wave][p][4 * g] = v - mine;
+            if (p < MT) *(v4i*)&sh.red[turn][i][wave][p][4 * g] = v - mine;
         }
+        float sm = s[0];
+#pragma unroll
+        for (int t = 1; t < MT; ++t) sm = out_token<RPW>() == t ? s[t] : sm;
+        finish<RPW, RES>(tk, k, sm, 0, got.res);
+    }
+    // The outputs, by the first waves, from the waves' sums in LDS: sm is the scale of this thread's token (out_token),
+    // `less` what its sums still hold too much
+    template <int RPW, bool RES>
+    __device__ __forceinline__ void finish(const Task& tk, int k, float sm, int less, uint16_t res) {
         arrive();
-        if (wave * 64 >= (RPW == 1 ? 16 : 32) * MT) return;  // the first waves finish the outputs
+        if (kDirect && wave * 64 >= (RPW == 1 ? 16 : 32) * MT) return;
         await();
         const int m = out_token<RPW>(), tb = out_tb<RPW>(), row = out_row();
         const int n = ((RPW == 1 ? tk.idx : 2 * tk.idx + tb) * 16) + row;
         if (m < batch() && m < MT && n < tk.n_out) {
             const uint16_t* ws = &sh.scales[k & 3][0][RPW == 1 ? tid & 15 : tid & 31];
-            float sm = s[0];
-#pragma unroll
-            for (int t = 1; t < MT; ++t) sm = m == t ? s[t] : sm;
             const float inv_s = reciprocal(sm);
             auto value = [&](int i, uint16_t ws) {
-                int sum = 0;
+                int sum = -less;
 #pragma unroll
-                for (int k = 0; k < kStWaves; ++k) sum += sh.red[i][k][m][row];
+                for (int k = 0; k < kStWaves; ++k) sum += sh.red[turn][i][k][m][row];
                 const float x = (float)sum, q = x * inv_s;  // the quotient as in the other kernels' epilogues
                 return f32_to_bf16_rne(__builtin_fmaf(__builtin_fmaf(-q, sm, x), inv_s, q) * bf16_to_f32(ws));
             };
@@ -671,13 +719,110 @@ struct Stack {
                 const float r = fmaxf(bf16_to_f32(v), 0.0f);
                 v = f32_to_bf16_rne(bf16_to_f32(f32_to_bf16_rne(r * r)) * bf16_to_f32(x3));
             }
-            if (RES) v = f32_to_bf16_rne(bf16_to_f32(got.res) + bf16_to_f32(v));
+            if (RES) v = f32_to_bf16_rne(bf16_to_f32(res) + bf16_to_f32(v));
             uint16_t* to = tk.dst + (size_t)m * tk.n_out + n;
             if (tk.flags & 2)
                 publish16(to, v);
             else
                 *to = v;
         }
+    }
+
+    // --- beyond kStDirect tokens: a token's row quantized, once for all workgroups ----------------------
+    template <int UPW>
+    __device__ __forceinline__ void quantizer_task(const Task& tk, int k) {
+        typedef Slice<UPW> S;
+        Got<MT> got;
+        norm_weights<UPW>(tk.aux, tk.K, got);
+        wait_ready(k);
+        consume(k);
+        gather_slices<UPW, false>(tk, got);
+        float s[TQ];
+        int sum[TQ];
+        const __amdgpu_buffer_rsrc_t to = make_rsrc(tk.dst, tk.K);
+        const int first = wave * S::kValues;
+        auto written = [](unsigned w) { return w == (unsigned)kUnsetBytes ? w + 1u : w; };
+        // (4 bytes at least a store: a word is there or not; values past the end of K are not stored)
+        quantize<UPW>(
+            tk, got, s, sum,
+            [&](int, int i, uint2 v) {
+                const int at = first + i * 512 + lane * 8;
+                __builtin_amdgcn_raw_buffer_store_b64(v2u{written(v.x), written(v.y)}, to, at < tk.K ? at : kBeyond, 0, kSc1);
+            },
+            [&](int, uint32_t r) {
+                int at = first + S::kFull * 512 + lane * S::T;
+                bool mine = lane * S::T < S::kRest && at < tk.K;
+                if (S::T == 2) {  // with the neighbour's
+                    r = (r & 0xffffu) | (unsigned)__builtin_amdgcn_update_dpp(0, (int)r, 0xB1, 0xF, 0xF, true) << 16;
+                    mine = mine && (lane & 1) == 0;
+                }
+                __builtin_amdgcn_raw_buffer_store_b32(written(r), to, mine ? at : kBeyond, 0, kSc1);
+            });
+        RowRecord* rec = (RowRecord*)tk.res;
+        if (lane == 0) {
+            __hip_atomic_store(&rec->sum[wave], sum[0] & 0x7fffffff, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (wave == 0) __hip_atomic_store(&rec->scale, (unsigned)f32_to_bf16_rne(s[0]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+    // a product of quantized rows: they are the MFMAs' column operand as they lie in memory
+    template <int UPW, int RPW, bool RES>
+    __device__ __forceinline__ void bytes_task(const Task& tk, int k) {
+        Got<MT> got;
+        wait_ready(k);
+        expand<UPW, RPW>(tk.K, k % kStBuffers, got);
+        consume(k);
+        const int p = lane & 15, g = lane >> 4, B = batch(), K = tk.K;
+        const int first = wave * (UPW * 64);
+        const int live = K - first < 0 ? 0 : (K - first) >> 6;  // k-steps of the slice in front of the end of K
+        const int m = out_token<RPW>() < B ? out_token<RPW>() : B - 1;
+        const int base = (p < B ? p : B - 1) * K + first + g * 16;
+        const __amdgpu_buffer_rsrc_t rows = make_rsrc(tk.src, B * K), recs = make_rsrc(tk.aux, B * (int)sizeof(RowRecord));
+        const __amdgpu_buffer_rsrc_t rs = make_rsrc(RES ? tk.res : tk.src, RES ? B * tk.n_out * 2 : 0);
+        const int res_off = RES ? (m * tk.n_out + tk.idx * 16 + out_row()) * 2 : kBeyond;
+        v4i b[UPW], sums;
+        auto get = [&](int j) {
+            b[j] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rows, j < live ? base + j * 64 : kBeyond, 0, kSc1));
+        };
+        auto lowest = [](int m, v4i v) { return min(min(min(m, v.x), min(v.y, v.z)), v.w); };
+        // one piece until it is there, then all: all workgroups asking for all rows all the time fill the fabric
+        for (int spin = 0;; ++spin) {
+            poll_again();
+            get(0);
+            if (__builtin_amdgcn_ballot_w64(lowest(0, b[0]) == kUnsetBytes) == 0 || wt.dead || wt.give_up(spin)) break;
+        }
+        unsigned scale = 0;
+        for (int spin = 0;; ++spin) {
+            poll_again();
+            if (RES) got.res = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rs, res_off, 0, kSc1);
+            sums = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(recs, m * (int)sizeof(RowRecord), 0, kSc1));
+            scale = (unsigned)__builtin_amdgcn_raw_buffer_load_b32(recs, m * (int)sizeof(RowRecord) + 16, 0, kSc1);
+#pragma unroll
+            for (int j = 0; j < UPW; ++j) get(j);
+            int low = 0;
+#pragma unroll
+            for (int j = 0; j < UPW; ++j) low = lowest(low, b[j]);
+            const bool missing = low == kUnsetBytes || (int)(sums.x | sums.y | sums.z | sums.w | (int)scale) < 0 ||
+                                 (RES && got.res == 0xffffu);
+            if (__builtin_amdgcn_ballot_w64(missing) == 0 || wt.dead || wt.give_up(spin)) break;
+        }
+        constexpr int C = RPW == 4 ? 1 : 2;  // chains of dependent products per row block
+        v4i acc[RPW][C];
+#pragma unroll
+        for (int i = 0; i < RPW; ++i)
+#pragma unroll
+            for (int c = 0; c < C; ++c) acc[i][c] = v4i{0, 0, 0, 0};
+#pragma unroll
+        for (int j = 0; j < UPW; ++j)
+#pragma unroll
+            for (int i = 0; i < RPW; ++i)
+                acc[i][j % C] = __builtin_amdgcn_mfma_i32_16x16x64_i8(got.e[i * kStUpwD + j], b[j], acc[i][j % C], 0, 0, 0);
+        if (p < MT) {
+#pragma unroll
+            for (int i = 0; i < RPW; ++i) *(v4i*)&sh.red[turn][i][wave][p][4 * g] = C == 2 ? acc[i][0] + acc[i][C - 1] : acc[i][0];
+        }
+        auto sum31 = [](int v) { return (int)((unsigned)v << 1) >> 1; };
+        finish<RPW, RES>(tk, k, bf16_to_f32((uint16_t)scale), 2 * (sum31(sums.x) + sum31(sums.y) + sum31(sums.z) + sum31(sums.w)), got.res);
+        turn ^= 1;
     }
 
     // --- attention: rope, cache write and one split of one (sequence, kv head) ------------------------
@@ -832,19 +977,28 @@ struct Stack {
         asm volatile("" ::: "memory");
     }
     __device__ __forceinline__ void run(const Task& tk, int k) {
-        switch (tk.ph) {
-            case kP1: product_task<kStUpwD, 2, false>(tk, k); break;
-            case kAttn: {
-                const PartO part_o = (PartO)sh.words[k % kStBuffers];
-                wait_ready(k);
-                attend(tk, part_o);
-                attention_outputs(tk, part_o);
-                consume(k);
-                break;
+        if (tk.ph == kAttn) {
+            const PartO part_o = (PartO)sh.words[k % kStBuffers];
+            wait_ready(k);
+            attend(tk, part_o);
+            attention_outputs(tk, part_o);
+            consume(k);
+        } else if constexpr (kDirect) {
+            switch (tk.ph) {
+                case kP1: product_task<kStUpwD, 2, false>(tk, k); break;
+                case kP3: product_task<kStUpwD, 1, true>(tk, k); break;
+                case kP4: product_task<kStUpwD, 4, false>(tk, k); break;
+                default: product_task<kStUpwF, 1, true>(tk, k); break;
             }
-            case kP3: product_task<kStUpwD, 1, true>(tk, k); break;
-            case kP4: product_task<kStUpwD, 4, false>(tk, k); break;
-            default: product_task<kStUpwF, 1, true>(tk, k); break;
+        } else {
+            switch (tk.ph) {
+                case kP1: bytes_task<kStUpwD, 2, false>(tk, k); break;
+                case kP3: bytes_task<kStUpwD, 1, true>(tk, k); break;
+                case kP4: bytes_task<kStUpwD, 4, false>(tk, k); break;
+                case kP5: bytes_task<kStUpwF, 1, true>(tk, k); break;
+                case kQ5: quantizer_task<kStUpwF>(tk, k); break;
+                default: quantizer_task<kStUpwD>(tk, k); break;
+            }
         }
     }
 };
@@ -857,9 +1011,9 @@ __global__ __launch_bounds__(kStThreads) __attribute__((amdgpu_waves_per_eu(2, 2
     // changes only when every workgroup of this launch is done; written past the writer's L2, so read past this one
     const unsigned launch = (unsigned)uniform((int)__hip_atomic_load(&ctl->launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
     Stack<MT> st{(StackArgsPtr)__builtin_amdgcn_kernarg_segment_ptr(), sh, Waiter{a.spin_limit, &ctl->error, false},
-                 a.ws + a.sets + (size_t)(launch & 1u) * a.set_bytes, launch, tid, tid & 63, uniform(tid >> 6), 0};
+                 a.ws + a.sets + (size_t)(launch & 1u) * a.set_bytes, launch, tid, tid & 63, uniform(tid >> 6), 0, 0};
     if (tid < kStWaves) sh.met[tid] = sh.consumed[tid] = 0;
-    if (tid < MT * kStWaves) {
+    if (tid < Shared<MT>::TQ * kStWaves) {
         ((v4i*)sh.sumsq)[tid] = v4i{0, 0, 0, 0};
         ((v2i*)sh.amax)[tid] = v2i{0, 0};
     }
@@ -867,8 +1021,10 @@ __global__ __launch_bounds__(kStThreads) __attribute__((amdgpu_waves_per_eu(2, 2
     {
         // the other set, for the next launch
         const __amdgpu_buffer_rsrc_t other = make_rsrc(a.ws + a.sets + (size_t)((launch & 1u) ^ 1u) * a.set_bytes, a.set_bytes);
-        for (int at = (blockIdx.x * kStThreads + tid) * 16; at < a.set_bytes; at += gridDim.x * kStThreads * 16)
-            __builtin_amdgcn_raw_buffer_store_b128(v4u{~0u, ~0u, ~0u, ~0u}, other, at, 0, kSc1);
+        for (int at = (blockIdx.x * kStThreads + tid) * 16; at < a.set_bytes; at += gridDim.x * kStThreads * 16) {
+            const unsigned u = at < a.set_values ? ~0u : (unsigned)kUnsetBytes;
+            __builtin_amdgcn_raw_buffer_store_b128(v4u{u, u, u, u}, other, at, 0, kSc1);
+        }
     }
     __syncthreads();
     Work cur = st.locate(0, 0);
@@ -968,9 +1124,11 @@ __global__ __launch_bounds__(kStThreads) __attribute__((amdgpu_waves_per_eu(2, 2
 }
 
 // A fresh workspace: zero control words and records, both sets unset
-__global__ __launch_bounds__(256) void decode_stack_reset_kernel(v4u* ws, long long n, long long sets, long long set_units) {
+__global__ __launch_bounds__(256) void decode_stack_reset_kernel(v4u* ws, long long n, long long sets, long long set_units,
+                                                                 long long value_units) {
     for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long long)gridDim.x * 256) {
-        const unsigned fill = i >= sets && i < sets + 2 * set_units ? ~0u : 0u;
+        const bool in = i >= sets && i < sets + 2 * set_units;
+        const unsigned fill = !in ? 0u : (i - sets) % set_units < value_units ? ~0u : (unsigned)kUnsetBytes;
         ws[i] = v4u{fill, fill, fill, fill};
     }
 }
@@ -987,9 +1145,10 @@ bool stack_plan(StackArgs& a, long long* bytes) {
     a.group = g;
     if (a.dim % 64 || a.dim > kStWaves * kStUpwD * 64 || a.ffn < 64 || a.ffn % 64 || a.ffn > kStWaves * kStUpwF * 64) return false;
     if (a.n_splits < 1 || a.n_splits > kDfMaxSplits) return false;
-    const int counts[5] = {nqkv / 32, a.n_kv * a.n_splits * a.B, a.dim / 16, (a.ffn / 16 + 1) / 2, a.dim / 16};
+    const int nq = a.B <= kStDirect ? 0 : a.B;
+    const int counts[9] = {nq, nqkv / 32, a.n_kv * a.n_splits * a.B, nq, a.dim / 16, nq, (a.ffn / 16 + 1) / 2, nq, a.dim / 16};
     int sum = 0;
-    for (int i = 0; i < 5; ++i) a.ends[i] = sum += counts[i];
+    for (int i = 0; i < 9; ++i) a.ends[i] = sum += counts[i];
     if ((long long)sum * a.n_layers > (1ll << 30)) return false;
     long long f = up256((long long)a.B * nqkv * 2);
     a.f_o = (int)f;
@@ -1000,9 +1159,14 @@ bool stack_plan(StackArgs& a, long long* bytes) {
     f = up256(f + (long long)a.B * a.ffn * 2);
     a.f_hb = (int)f;
     f = up256(f + (long long)a.B * a.dim * 2);
+    a.f_rec = (int)f;
+    if (nq) f = up256(f + 4ll * a.B * (long long)sizeof(RowRecord));
     a.f_layer = (int)f;
-    if (f * a.n_layers > (1ll << 30)) return false;
-    a.set_bytes = (int)(f * a.n_layers);
+    const long long rows = nq ? up256((long long)a.B * (3ll * a.dim + a.ffn)) : 0;
+    if ((f + rows) * a.n_layers > (1ll << 30)) return false;
+    a.f_bytes = (int)rows;
+    a.set_values = (int)(f * a.n_layers);
+    a.set_bytes = (int)((f + rows) * a.n_layers);
     a.sets = up256(sizeof(StackControl));
     a.records = a.sets + 2ll * a.set_bytes;
     a.inv_dim = 1.0f / (float)a.dim;
@@ -1036,7 +1200,7 @@ int bitnet_decode_stack_reset(void* workspace, int n_layers, int B, int S, int d
     if (!workspace) return 2;
     if ((uintptr_t)workspace & 255u) return 1;
     hipLaunchKernelGGL(decode_stack_reset_kernel, dim3(1024), dim3(256), 0, (hipStream_t)stream, (v4u*)workspace, bytes >> 4, a.sets >> 4,
-                       (long long)a.set_bytes >> 4);
+                       (long long)a.set_bytes >> 4, (long long)a.set_values >> 4);
     return hipGetLastError() == hipSuccess ? 0 : 3;
 }
 
@@ -1075,7 +1239,8 @@ int bitnet_decode_stack(const void* entries, void* workspace, const uint16_t* h_
     }
 #define BITNET_STACK(MT) hipLaunchKernelGGL(decode_stack_kernel<MT>, dim3(grid), dim3(kStThreads), 0, (hipStream_t)stream, a)
     if (B == 1) BITNET_STACK(1);
-    else BITNET_STACK(2);
+    else if (B == 2) BITNET_STACK(2);
+    else BITNET_STACK(8);
 #undef BITNET_STACK
     return hipGetLastError() == hipSuccess ? 0 : 3;
 }

@@ -219,7 +219,7 @@ int bitnet_top_p_sample(const float* logits, const float* noise, void* workspace
  *   workgroups 0 = one per CU; otherwise the grid (a test hook: any number works)
  *   spin_limit 0 = the built-in bound of every wait inside the kernel; otherwise the bound
  * dim = n_heads * 128, dim % 64 == 0, dim <= 2560; ffn % 64 == 0, ffn <= 6912; n_heads / n_kv_heads
- * one of 1, 2, 4, 8; B <= 2; n_splits <= 16: workspace_bytes returns -1 for anything else.
+ * one of 1, 2, 4, 8; B <= 8; n_splits <= 16: workspace_bytes returns -1 for anything else.
  *
  * Workgroups wait for each other inside the kernel, but never for one that does not run yet: the
  * kernel ends whatever else occupies the GPU.  Should a wait ever run out all the same (a workspace

@@ -583,6 +583,8 @@ def test_host_checks_refuse_mismatched_buffers_before_any_launch():
 @pytest.mark.parametrize("B,dim,ffn,nh,nkv,S,n_splits", [
     (1, 128, 64, 1, 1, 33, 1), (2, 128, 64, 1, 1, 40, 16), (1, 1152, 2112, 9, 9, 70, 3), (2, 1024, 1984, 8, 1, 700, 5),
     (1, 2560, 6912, 20, 5, 545, 8), (2, 2560, 6912, 20, 5, 300, 8),
+    # beyond two tokens the input rows are quantized by tasks of their own
+    (3, 128, 64, 1, 1, 40, 16), (5, 1152, 2112, 9, 9, 70, 3), (8, 1024, 1984, 8, 1, 700, 5), (8, 2560, 6912, 20, 5, 545, 6),
 ])
 def test_decode_stack_kernel_equals_the_kernels_per_layer(B, dim, ffn, nh, nkv, S, n_splits, workgroups):
     args = decoder.ModelArgs(dim=dim, n_layers=2, n_heads=nh, n_kv_heads=nkv, vocab_size=256, ffn_dim=ffn)
