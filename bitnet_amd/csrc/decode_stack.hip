@@ -11,11 +11,14 @@
 // such a hand-over measures 1.4 us, readers' barrier included.  30 layers at 512 positions, us:
 //   sequences            1     2     3     4     8
 //   launches           755   875  1000  1070  1060
-//   this kernel        511   626   690   715   816
+//   this kernel        511   626   680   705   772
 // Up to two tokens every workgroup of a product normalises and quantizes the rows by itself, between their
 // arrival and its matrix instructions.  That part grows with the tokens (three: 1120 us).  Beyond two, one
 // task per token does it for all and publishes int8 rows, which are the matrix instructions' operand as they
-// lie in memory: one more hand-over, but a product's own work hardly depends on the tokens.
+// lie in memory: one more hand-over, but a product's own work hardly depends on the tokens.  The rows stand
+// with 64 values of every token side by side, so that one 16-byte load of a wave covers 16 / tokens k-steps
+// of all of them and its lines are whole, and the first complete read may hit the XCD's L2 (eight sequences:
+// 816 us with a row per token and every read past L2).
 //
 // Hand-over buffers.  Every (layer, step) has buffers of its own, in two sets that alternate between
 // launches; a launch fills the other set with a value that no result can have (bf16 0xffff, a NaN that
@@ -392,7 +395,7 @@ struct Stack {
         uint64_t src, res = 0, dst, aux = (uint64_t)e->norm;
         int K = a->dim, n_out = a->dim, flags = 3;
         float inv_k = a->inv_dim;
-        // quantized rows of product i of the layer, and their records
+        // quantized rows of product i of the layer, 64 values of every token side by side, and their records
         auto bytes = [&](int i) { return (uint64_t)(set + a->set_values + (size_t)l * a->f_bytes + (size_t)i * a->B * a->dim); };
         auto record = [&](int i) { return (uint64_t)(layer_set(l) + a->f_rec) + (uint64_t)(i * a->B) * sizeof(RowRecord); };
         const int i = product_of(wk.ph);
@@ -416,7 +419,7 @@ struct Stack {
                 if (i == 3 && last) flags &= ~2;
             } else {
                 src += (uint64_t)wk.idx * K * 2;
-                dst = bytes(i) + (uint64_t)wk.idx * K;
+                dst = bytes(i) + (uint64_t)wk.idx * 64;
                 res = record(i) + (uint64_t)wk.idx * sizeof(RowRecord);
             }
         }
@@ -739,15 +742,16 @@ struct Stack {
         gather_slices<UPW, false>(tk, got);
         float s[TQ];
         int sum[TQ];
-        const __amdgpu_buffer_rsrc_t to = make_rsrc(tk.dst, tk.K);
-        const int first = wave * S::kValues;
+        const int first = wave * S::kValues, step = batch() * 64;
+        const __amdgpu_buffer_rsrc_t to = make_rsrc(tk.dst, ((tk.K >> 6) - 1) * step + 64);
+        auto place = [&](int at) { return (at >> 6) * step + (at & 63); };
         auto written = [](unsigned w) { return w == (unsigned)kUnsetBytes ? w + 1u : w; };
         // (4 bytes at least a store: a word is there or not; values past the end of K are not stored)
         quantize<UPW>(
             tk, got, s, sum,
             [&](int, int i, uint2 v) {
                 const int at = first + i * 512 + lane * 8;
-                __builtin_amdgcn_raw_buffer_store_b64(v2u{written(v.x), written(v.y)}, to, at < tk.K ? at : kBeyond, 0, kSc1);
+                __builtin_amdgcn_raw_buffer_store_b64(v2u{written(v.x), written(v.y)}, to, at < tk.K ? place(at) : kBeyond, 0, kSc1);
             },
             [&](int, uint32_t r) {
                 int at = first + S::kFull * 512 + lane * S::T;
@@ -756,7 +760,7 @@ struct Stack {
                     r = (r & 0xffffu) | (unsigned)__builtin_amdgcn_update_dpp(0, (int)r, 0xB1, 0xF, 0xF, true) << 16;
                     mine = mine && (lane & 1) == 0;
                 }
-                __builtin_amdgcn_raw_buffer_store_b32(written(r), to, mine ? at : kBeyond, 0, kSc1);
+                __builtin_amdgcn_raw_buffer_store_b32(written(r), to, mine ? place(at) : kBeyond, 0, kSc1);
             });
         RowRecord* rec = (RowRecord*)tk.res;
         if (lane == 0) {
@@ -775,50 +779,66 @@ struct Stack {
         const int first = wave * (UPW * 64);
         const int live = K - first < 0 ? 0 : (K - first) >> 6;  // k-steps of the slice in front of the end of K
         const int m = out_token<RPW>() < B ? out_token<RPW>() : B - 1;
-        const int base = (p < B ? p : B - 1) * K + first + g * 16;
+        // column p is token p % MT at the k-step p / MT of SP that one load covers (as in product())
+        constexpr int SP = 16 / MT, kLoads = (UPW + SP - 1) / SP;
+        const int ps = p / MT, pt = p % MT;
+        const unsigned step = B * 64;
+        const unsigned base = pt < B ? (first + ps * 64) * B + pt * 64 + g * 16 : kBeyond;  // (no such token: zeros, no access)
         const __amdgpu_buffer_rsrc_t rows = make_rsrc(tk.src, B * K), recs = make_rsrc(tk.aux, B * (int)sizeof(RowRecord));
         const __amdgpu_buffer_rsrc_t rs = make_rsrc(RES ? tk.res : tk.src, RES ? B * tk.n_out * 2 : 0);
         const int res_off = RES ? (m * tk.n_out + tk.idx * 16 + out_row()) * 2 : kBeyond;
-        v4i b[UPW], sums;
-        auto get = [&](int j) {
-            b[j] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rows, j < live ? base + j * 64 : kBeyond, 0, kSc1));
-        };
-        auto lowest = [](int m, v4i v) { return min(min(min(m, v.x), min(v.y, v.z)), v.w); };
-        // one piece until it is there, then all: all workgroups asking for all rows all the time fill the fabric
-        for (int spin = 0;; ++spin) {
-            poll_again();
-            get(0);
-            if (__builtin_amdgcn_ballot_w64(lowest(0, b[0]) == kUnsetBytes) == 0 || wt.dead || wt.give_up(spin)) break;
-        }
+        v4i b[kLoads], sums;
         unsigned scale = 0;
-        for (int spin = 0;; ++spin) {
-            poll_again();
-            if (RES) got.res = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rs, res_off, 0, kSc1);
-            sums = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(recs, m * (int)sizeof(RowRecord), 0, kSc1));
-            scale = (unsigned)__builtin_amdgcn_raw_buffer_load_b32(recs, m * (int)sizeof(RowRecord) + 16, 0, kSc1);
-#pragma unroll
-            for (int j = 0; j < UPW; ++j) get(j);
+        auto recorded = [&] { return (int)(sums.x | sums.y | sums.z | sums.w | (int)scale) >= 0; };
+        auto lowest = [](int m, v4i v) { return min(min(min(m, v.x), min(v.y, v.z)), v.w); };
+        auto incomplete = [&] {
             int low = 0;
 #pragma unroll
-            for (int j = 0; j < UPW; ++j) low = lowest(low, b[j]);
-            const bool missing = low == kUnsetBytes || (int)(sums.x | sums.y | sums.z | sums.w | (int)scale) < 0 ||
-                                 (RES && got.res == 0xffffu);
-            if (__builtin_amdgcn_ballot_w64(missing) == 0 || wt.dead || wt.give_up(spin)) break;
+            for (int j = 0; j < kLoads; ++j) low = lowest(low, b[j]);
+            return __builtin_amdgcn_ballot_w64(low == kUnsetBytes || !recorded() || (RES && got.res == 0xffffu)) != 0;
+        };
+        // one piece until it is there, then all: all workgroups asking for all rows all the time fill the fabric, and so
+        // do all asking for the same piece
+        const int turns = live / SP;  // loads of which every column is in front of the end of K
+        const unsigned probe = turns > 0 ? base + (tk.idx % turns) * (SP * step) : ps < live ? base : (unsigned)kBeyond;
+        for (int spin = 0;; ++spin) {
+            poll_again();
+            const v4i v = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rows, probe, 0, kSc1));
+            if (__builtin_amdgcn_ballot_w64(lowest(0, v) == kUnsetBytes) == 0 || wt.dead || wt.give_up(spin)) break;
         }
-        constexpr int C = RPW == 4 ? 1 : 2;  // chains of dependent products per row block
-        v4i acc[RPW][C];
+        auto get = [&](auto policy) {
+            poll_again();
+            if (RES) got.res = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rs, res_off, 0, kSc1);
+            sums = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(recs, m * (int)sizeof(RowRecord), 0, decltype(policy)::value));
+            scale = (unsigned)__builtin_amdgcn_raw_buffer_load_b32(recs, m * (int)sizeof(RowRecord) + 16, 0, decltype(policy)::value);
+#pragma unroll
+            for (int j = 0; j < kLoads; ++j)
+                b[j] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(
+                                                   rows, j * SP + ps < live ? base + j * (SP * step) : (unsigned)kBeyond, 0, decltype(policy)::value));
+        };
+        get(std::integral_constant<int, 0>{});
+        for (int spin = 0; incomplete() && !wt.dead && !wt.give_up(spin); ++spin) get(std::integral_constant<int, kSc1>{});
+        v4i acc[RPW][SP];
 #pragma unroll
         for (int i = 0; i < RPW; ++i)
 #pragma unroll
-            for (int c = 0; c < C; ++c) acc[i][c] = v4i{0, 0, 0, 0};
+            for (int c = 0; c < SP; ++c) acc[i][c] = v4i{0, 0, 0, 0};
 #pragma unroll
         for (int j = 0; j < UPW; ++j)
 #pragma unroll
             for (int i = 0; i < RPW; ++i)
-                acc[i][j % C] = __builtin_amdgcn_mfma_i32_16x16x64_i8(got.e[i * kStUpwD + j], b[j], acc[i][j % C], 0, 0, 0);
-        if (p < MT) {
+                acc[i][j % SP] = __builtin_amdgcn_mfma_i32_16x16x64_i8(got.e[i * kStUpwD + j], b[j / SP], acc[i][j % SP], 0, 0, 0);
 #pragma unroll
-            for (int i = 0; i < RPW; ++i) *(v4i*)&sh.red[turn][i][wave][p][4 * g] = C == 2 ? acc[i][0] + acc[i][C - 1] : acc[i][0];
+        for (int i = 0; i < RPW; ++i) {
+            v4i v = acc[i][0];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+#pragma unroll
+                for (int c = 1; c < SP; ++c) v[r] = ps == c ? acc[i][c][r] : v[r];
+                v[r] += __builtin_amdgcn_update_dpp(0, v[r], 0x120 + MT, 0xF, 0xF, true);  // row_ror
+                if (SP == 4) v[r] += __builtin_amdgcn_update_dpp(0, v[r], 0x120 + 2 * MT, 0xF, 0xF, true);
+            }
+            if (p < MT) *(v4i*)&sh.red[turn][i][wave][p][4 * g] = v;
         }
         auto sum31 = [](int v) { return (int)((unsigned)v << 1) >> 1; };
         finish<RPW, RES>(tk, k, bf16_to_f32((uint16_t)scale), 2 * (sum31(sums.x) + sum31(sums.y) + sum31(sums.z) + sum31(sums.w)), got.res);
@@ -1240,6 +1260,7 @@ int bitnet_decode_stack(const void* entries, void* workspace, const uint16_t* h_
 #define BITNET_STACK(MT) hipLaunchKernelGGL(decode_stack_kernel<MT>, dim3(grid), dim3(kStThreads), 0, (hipStream_t)stream, a)
     if (B == 1) BITNET_STACK(1);
     else if (B == 2) BITNET_STACK(2);
+    else if (B <= 4) BITNET_STACK(4);
     else BITNET_STACK(8);
 #undef BITNET_STACK
     return hipGetLastError() == hipSuccess ? 0 : 3;
