@@ -188,13 +188,16 @@ __device__ __forceinline__ void lds_put(T& to, T v) {
 }
 // 16 bytes per lane straight into LDS, lane l's at `to` + 16 l.  In assembly, so that the compiler does not hold it
 // against every later LDS access (it would wait for the load in front of the next one): what makes the words
-// visible is that a wave waits for a later load of its own -- they return in order -- and then meets a barrier.
+// visible is that the fetching wave waits for its loads before it says in LDS that they are there.  The compiler does
+// not look into the string for hazards, so the wait state between a write of m0 and a load that takes its LDS address
+// from it is in it; a vector instruction's write of the descriptor needs five in front of the first load (settled).
 __device__ __forceinline__ void load_to_lds(v4u rsrc, unsigned to, int voffset, int soffset) {
-    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds"
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds"
                  :
                  : "s"(to), "v"(voffset), "s"(rsrc), "s"(soffset)
                  : "memory");  // (m0 is the compiler's scratch: it sets it in front of each use of its own)
 }
+__device__ __forceinline__ void settled(v4u& rsrc) { asm volatile("s_nop 4" : "+s"(rsrc)); }
 // The correctly rounded results of the IEEE operations they replace, from the hardware's approximations and one
 // correction step each (found equal on every mantissa; the operands are positive)
 __device__ __forceinline__ float divide(float x, float by, float inv) {  // inv: 1 / by, correctly rounded
@@ -449,7 +452,8 @@ struct Stack {
         const int bytes = uniform((!pairs || (wk.ph == kP4 && first + 1 >= half) ? 1 : 2) * K * 4);
         for (int i = 0; i < (wk.ph == kP4 ? 2 : 1); ++i) {
             const uintptr_t from = (uintptr_t)w + (size_t)(i * half + first) * K * 4;
-            const v4u r = {(unsigned)uniform((int)from), (unsigned)uniform((int)(from >> 32)) & 0xffffu, (unsigned)bytes, 0x00020000u};
+            v4u r = {(unsigned)uniform((int)from), (unsigned)uniform((int)(from >> 32)) & 0xffffu, (unsigned)bytes, 0x00020000u};
+            settled(r);
             const unsigned to = lds_address(&sh.words[buffer][i ? run_stride() : 0]);
 #pragma nounroll
             for (int at = 0; at < bytes; at += 1024) load_to_lds(r, to + at, lane * 16, at);
