@@ -17,7 +17,6 @@
 #include <ATen/ops/empty.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
-#include <pybind11/gil.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -90,6 +89,38 @@ at::Tensor empty_like_rows(const at::Tensor& rows, int64_t width, at::ScalarType
     return at::Tensor(at::detail::empty_cuda(sizes, type, rows.device(), std::nullopt));
 }
 
+// Addresses are taken in front of the part that runs without the interpreter lock: data_ptr() throws for a tensor without
+// storage (vmap, tracing), and the checks before it pass for one.
+template <class T = void>
+T* address(const at::Tensor& t) {
+    return static_cast<T*>(t.data_ptr());
+}
+
+// The interpreter lock is free while one of these lives, and held again behind it, an exception included
+class Unlocked {
+public:
+    Unlocked() : state_(PyEval_SaveThread()) {}
+    ~Unlocked() { PyEval_RestoreThread(state_); }
+    Unlocked(const Unlocked&) = delete;
+
+private:
+    PyThreadState* state_;
+};
+
+// An int array that supports the buffer protocol, or None
+class IntArray {
+public:
+    ~IntArray() {
+        if (view_.buf) PyBuffer_Release(&view_);
+    }
+    bool open(PyObject* o) { return o == Py_None || PyObject_GetBuffer(o, &view_, PyBUF_SIMPLE) == 0; }
+    const int* data() const { return static_cast<const int*>(view_.buf); }
+    int size() const { return static_cast<int>(view_.len / static_cast<Py_ssize_t>(sizeof(int))); }
+
+private:
+    Py_buffer view_ = {};
+};
+
 void* current_stream() { return (void*)c10::hip::getCurrentHIPStream().stream(); }
 
 PyObject* library_error(const char* entry, long long m, long long n, long long k, int status) {
@@ -127,12 +158,13 @@ PyObject* forward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         PyErr_SetString(PyExc_ValueError, "weight must be int8 [out_features, in_features // 4] (the packed layout)");
         return nullptr;
     }
+    const void *px = M ? address(*x) : nullptr, *pw = M ? address(*w) : nullptr, *pws = M ? address(*ws) : nullptr;
     const c10::DeviceGuard guard(x->device());
     at::Tensor out = empty_like_rows(*x, N, at::kBFloat16);
     if (M == 0) return THPVariable_Wrap(std::move(out));
-    Py_buffer seg;
-    seg.buf = nullptr;
-    if (args[6] != Py_None && PyObject_GetBuffer(args[6], &seg, PyBUF_SIMPLE) != 0) return nullptr;
+    void* po = address(out);
+    IntArray seg;
+    if (!seg.open(args[6])) return nullptr;
     // the quantized rows and, behind them, their scales: one block that goes back to the allocator on return, as
     // tensors do (reused by later work on the same stream)
     const size_t q_bytes = ((size_t)M * (size_t)K + 255) & ~(size_t)255;
@@ -141,17 +173,12 @@ PyObject* forward(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         const c10::DataPtr block = c10::hip::HIPCachingAllocatorMasqueradingAsCUDA::get()->allocate(q_bytes + 2 * (size_t)M);
         char* q = (char*)block.get();
         void* stream = current_stream();
-        Py_BEGIN_ALLOW_THREADS;
-        st = seg.buf ? g_bound.forward_seg(x->data_ptr(), w->data_ptr(), out.data_ptr(), ws->data_ptr(), (const int*)seg.buf,
-                                           (int)(seg.len / (Py_ssize_t)sizeof(int)), q, q + q_bytes, (int)M, (int)N, (int)K,
-                                           (int)mode, stream)
-                     : g_bound.forward(x->data_ptr(), w->data_ptr(), out.data_ptr(), ws->data_ptr(), q, q + q_bytes, (int)M,
-                                       (int)N, (int)K, (int)mode, stream);
-        Py_END_ALLOW_THREADS;
+        const Unlocked unlocked;
+        st = seg.data() ? g_bound.forward_seg(px, pw, po, pws, seg.data(), seg.size(), q, q + q_bytes, (int)M, (int)N, (int)K,
+                                              (int)mode, stream)
+                        : g_bound.forward(px, pw, po, pws, q, q + q_bytes, (int)M, (int)N, (int)K, (int)mode, stream);
     }
-    const bool segmented = seg.buf != nullptr;
-    if (segmented) PyBuffer_Release(&seg);
-    if (st) return library_error(segmented ? "bitlinear_forward_bf16_seg" : "bitlinear_forward_bf16", M, N, K, st);
+    if (st) return library_error(seg.data() ? "bitlinear_forward_bf16_seg" : "bitlinear_forward_bf16", M, N, K, st);
     return THPVariable_Wrap(std::move(out));
     END_HANDLE_TH_ERRORS
 }
@@ -191,6 +218,9 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         PyErr_SetString(PyExc_ValueError, "weight_scale has fewer slots than this shape uses");
         return nullptr;
     }
+    int8_t *pa = nullptr, *pw = nullptr;
+    uint16_t *ps = nullptr, *pws = nullptr;
+    if (M > 0) pa = address<int8_t>(*a), pw = address<int8_t>(*w), ps = address<uint16_t>(*s), pws = address<uint16_t>(*ws);
     const c10::DeviceGuard guard(a->device());
     at::Tensor out;
     if (args[4] == Py_None) {
@@ -206,12 +236,13 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     }
     if (M > 0) {  // no token rows: nothing to launch
         void* stream = current_stream();
+        uint16_t* po = address<uint16_t>(out);
         int st = 0;
-        Py_BEGIN_ALLOW_THREADS;
-        g_bound.product((int8_t*)a->data_ptr(), (int8_t*)w->data_ptr(), (uint16_t*)out.data_ptr(), (uint16_t*)s->data_ptr(),
-                        (uint16_t*)ws->data_ptr(), (int)M, (int)N, (int)K, stream);
-        st = g_bound.last_status();
-        Py_END_ALLOW_THREADS;
+        {
+            const Unlocked unlocked;
+            g_bound.product(pa, pw, po, ps, pws, (int)M, (int)N, (int)K, stream);
+            st = g_bound.last_status();
+        }
         if (st) return library_error("bitlinear_int8xint2", M, N, K, st);
     }
     if (args[4] != Py_None) {
@@ -237,14 +268,16 @@ PyObject* quant(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     const int64_t M = flat_rows(*x);
     if (M < 0) return nullptr;
     const int64_t K = x->size(-1);
+    const void* px = M ? address(*x) : nullptr;
     const c10::DeviceGuard guard(x->device());
     at::Tensor q = empty_like_rows(*x, K, at::kChar), s = empty_like_rows(*x, 1, at::kBFloat16);
     if (M > 0) {
-        void* stream = current_stream();
+        void *stream = current_stream(), *pq = address(q), *ps = address(s);
         int st = 0;
-        Py_BEGIN_ALLOW_THREADS;
-        st = g_bound.quant(x->data_ptr(), q.data_ptr(), s.data_ptr(), (int)M, (int)K, (int)mode, stream);
-        Py_END_ALLOW_THREADS;
+        {
+            const Unlocked unlocked;
+            st = g_bound.quant(px, pq, ps, (int)M, (int)K, (int)mode, stream);
+        }
         if (st) {
             PyErr_Format(g_bound.error, "bitlinear_quant_absmax(M=%lld, K=%lld): status %d (%s)", (long long)M, (long long)K,
                          st, g_bound.status_string(st));
@@ -304,6 +337,7 @@ PyObject* pack(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         return nullptr;
     }
     const int64_t N = w->size(0), K = w->size(1);
+    const void* pw = address(*w);
     const c10::DeviceGuard guard(w->device());
     at::Tensor out = empty_like_rows(*w, K / 4, at::kChar);
     int st = 0;
@@ -311,8 +345,9 @@ PyObject* pack(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     {
         const PinnedFlag flag;
         const c10::hip::HIPStream stream = c10::hip::getCurrentHIPStream();
-        pybind11::gil_scoped_release no_gil;
-        st = g_bound.pack(w->data_ptr(), out.data_ptr(), (void*)flag.value(), (int)N, (int)K, (void*)stream.stream());
+        void* po = address(out);
+        const Unlocked unlocked;
+        st = g_bound.pack(pw, po, (void*)flag.value(), (int)N, (int)K, (void*)stream.stream());
         if (!st) {
             stream.synchronize();
             bad = *flag.value() != 0;
@@ -339,13 +374,15 @@ PyObject* unpack(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         PyErr_SetString(PyExc_ValueError, "unpack: expected N * K / 4 bytes");
         return nullptr;
     }
+    const void* pp = address(*p);
     const c10::DeviceGuard guard(p->device());
     at::Tensor out(at::detail::empty_cuda({N, K}, at::kChar, p->device(), std::nullopt));
-    void* stream = current_stream();
+    void *stream = current_stream(), *po = address(out);
     int st = 0;
-    Py_BEGIN_ALLOW_THREADS;
-    st = g_bound.unpack(p->data_ptr(), out.data_ptr(), (int)N, (int)K, stream);
-    Py_END_ALLOW_THREADS;
+    {
+        const Unlocked unlocked;
+        st = g_bound.unpack(pp, po, (int)N, (int)K, stream);
+    }
     if (st) return library_error("bitlinear_unpack_int2", 1, N, K, st);
     return THPVariable_Wrap(std::move(out));
     END_HANDLE_TH_ERRORS

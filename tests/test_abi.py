@@ -148,3 +148,37 @@ def test_host_calls_refuse_bad_arguments_before_any_launch():
     for call in (lambda: mod(None), lambda: bitlinear.quant_input([1.0]), lambda: _lib.host_calls().forward(x)):
         with pytest.raises(TypeError):
             call()
+
+
+def _device_tensor(shape, dtype):
+    """A tensor that says that it lives on the GPU, on a machine without one."""
+    import torch
+
+    class Sub(torch.Tensor):
+        @classmethod
+        def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
+            raise AssertionError(f"no operator is called: {func}")
+
+    return torch.Tensor._make_wrapper_subclass(Sub, shape, dtype=dtype, device="cuda")
+
+
+@pytest.mark.parametrize("call", ["forward", "forward_segments", "linear", "quant", "pack", "unpack"])
+def test_host_calls_refuse_tensors_without_storage(call):
+    """What vmap and tracing hand over passes every check of shape, type and device and has no address: an error, in front
+    of any allocation, and with the interpreter lock held."""
+    import torch
+
+    if not os.path.exists(_lib.HOST_CALLS_PATH):
+        pytest.skip("not built")
+    host = _lib.host_calls()
+    w, ws = _device_tensor((32, 32), torch.int8), _device_tensor((4,), torch.bfloat16)
+    shape, dtype, run = {
+        "forward": ((2, 128), torch.bfloat16, lambda t: host.forward(t, w, ws, 128, 32, 0, None)),
+        "forward_segments": ((2, 128), torch.bfloat16, lambda t: host.forward(t, w, ws, 128, 32, 0, (ctypes.c_int * 2)(16, 32))),
+        "linear": ((2, 128), torch.int8, lambda t: host.linear(t, w, _device_tensor((2,), torch.bfloat16), ws, None)),
+        "quant": ((2, 128), torch.bfloat16, lambda t: host.quant(t, 0)),
+        "pack": ((32, 128), torch.int8, lambda t: host.pack(t)),
+        "unpack": ((32, 32), torch.int8, lambda t: host.unpack(t, 32, 128)),
+    }[call]
+    with pytest.raises(RuntimeError, match="data pointer"):
+        torch.vmap(run)(_device_tensor((3, *shape), dtype))
