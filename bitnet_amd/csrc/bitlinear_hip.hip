@@ -1836,7 +1836,7 @@ __global__ __launch_bounds__(kMaxWaves * 64) void bitlinear_solo_kernel(
             for (int k = 0; k < S; ++k) total += wsq[rbl * S + k][m];
             const float mean = (float)total / (float)K;
             const float rstd = 1.0f / __builtin_sqrtf(mean + eps);
-            sv[m] = norm8(sv[m], gvec, rstd);
+            sv[m] = norm8(sv[m], gvec, slice_lane ? rstd : 0.0f);  // (idle lanes keep their zeros where rstd is not finite)
         }
     }
 

@@ -575,6 +575,36 @@ def test_host_checks_refuse_mismatched_buffers_before_any_launch():
         gen.decode(first, 10, 8)                                                 # positions 10..17 in a cache of 16 rows
 
 
+@pytest.mark.parametrize("M", [1, 2, 4, 5, 8, 40])  # every kernel that holds the norm
+@pytest.mark.parametrize("K,N", [(128, 48), (1152, 128), (2560, 256), (6912, 64)])
+def test_norm_bitlinear_of_rows_that_are_not_finite(M, K, N):
+    """A row whose norm gives NaNs: their code is -128, whatever the number of tokens and however K falls into slices."""
+    gen = torch.Generator(device="cuda").manual_seed(M + K)
+    x = torch.randn(M, K, generator=gen, device="cuda").to(torch.bfloat16)
+    x[0, K // 3] = float("nan")                      # every value of the row becomes NaN
+    if M > 1:
+        x[1, 5] = float("inf")                       # this one does, the others become zeros
+        x[1, K - 1] = float("-inf")
+    if M > 2:
+        x[2] = 0.0
+    norm = decoder.RMSNorm(K, 1e-5).cuda().to(torch.bfloat16)
+    norm.weight.data = torch.rand(K, generator=gen, device="cuda").add(0.5).to(torch.bfloat16)
+    lin = BitLinearKernel(K, N).cuda()
+    w = torch.randint(-1, 2, (N, K), generator=gen, device="cuda", dtype=torch.int8)
+    lin.weight.data = pack_weight.convert_weight_int8_to_int2(w, keep_device=True)
+    lin.weight_scale.data = torch.full((4,), 0.0156, device="cuda").to(torch.bfloat16)
+    got = decoder.norm_bitlinear(x, norm, lin)
+    xf = x.float()
+    mean = xf.double().pow(2).sum(-1, keepdim=True).float() / K
+    y = (xf * (1.0 / torch.sqrt(mean + 1e-5)) * norm.weight.float()).to(torch.bfloat16).float()
+    # (the row's maximum is one of bit patterns, so a NaN is the largest; the lower bound takes its place)
+    amax = torch.where(torch.isnan(y).any(-1, keepdim=True), 0.0, y.nan_to_num().abs().amax(-1, keepdim=True)).clamp(min=1e-5)
+    s = ((1.0 / amax) * 127.0).to(torch.bfloat16).float()
+    q = torch.where(torch.isnan(y), -128.0, (y * s).nan_to_num().round().clamp(-128, 127)).double()
+    want = ((q.cpu() @ w.cpu().double().T).float() / s.cpu() * lin.weight_scale[0].float().cpu()).to(torch.bfloat16)
+    assert np.array_equal(host_bits(got), host_bits(want))
+
+
 # ---------------------------------------------------------------------------
 # The end-to-end workload at its real size: 30 layers, dim 2560, ffn 6912, 20 / 5 heads, vocabulary
 # 128256 (gpu/model.py:39-49), a 512-token seeded prompt, greedy decode (gpu/generate.py:264-288)
