@@ -199,7 +199,7 @@ __device__ __forceinline__ void load_to_lds(v4u rsrc, unsigned to, int voffset, 
 }
 __device__ __forceinline__ void settled(v4u& rsrc) { asm volatile("s_nop 4" : "+s"(rsrc)); }
 // The correctly rounded results of the IEEE operations they replace, from the hardware's approximations and one
-// correction step each (found equal on every mantissa; the operands are positive)
+// correction step each (found equal on every mantissa; the operands are positive or NaN, which stays one)
 __device__ __forceinline__ float divide(float x, float by, float inv) {  // inv: 1 / by, correctly rounded
     const float q = x * inv;
     const float r = __builtin_fmaf(__builtin_fmaf(-q, by, x), inv, q);
@@ -207,13 +207,13 @@ __device__ __forceinline__ float divide(float x, float by, float inv) {  // inv:
 }
 __device__ __forceinline__ float reciprocal(float x) {
     const float r = __builtin_amdgcn_rcpf(x);
-    return x < INFINITY ? __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r) : 0.0f;
+    return x == INFINITY ? 0.0f : __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
 }
 __device__ __forceinline__ float reciprocal_sqrt(float x) {  // 1 / sqrt(x), both rounded
     const float y = __builtin_amdgcn_rsqf(x);
     const float s0 = x * y;
     const float s = __builtin_fmaf(__builtin_fmaf(-s0, s0, x), 0.5f * y, s0);
-    return x < INFINITY ? reciprocal(s) : 0.0f;
+    return x == INFINITY ? 0.0f : reciprocal(s);
 }
 // reductions that leave the wave's result in lane 63: rows of 16 by lane permutes, then row 0 into 1 and 2 into 3,
 // then those two
@@ -590,16 +590,18 @@ struct Stack {
 #pragma unroll
             for (int k = 0; k < kStWaves; ++k) total += __builtin_bit_cast(double, v2i{x[k].x, x[k].y});
             const float rstd = reciprocal_sqrt(divide((float)total, (float)tk.K, tk.inv_k) + tk.eps);
+            // (values past the end of K stay zeros, also where rstd is NaN)
+            const float tail = lane * S::T < S::kRest && wave * S::kValues + S::kFull * 512 + lane * S::T < tk.K ? rstd : 0.0f;
             uint32_t am = 0;
 #pragma unroll
             for (int i = 0; i < S::kFull; ++i) {
-                v.full[i] = norm8(v.full[i], got.g[i], rstd);
+                v.full[i] = norm8(v.full[i], got.g[i], wave * S::kValues + i * 512 + lane * 8 < tk.K ? rstd : 0.0f);
                 am = absmax_bits8(v.full[i], am);
             }
             if (S::T) {
                 uint4 r = make_uint4(0u, 0u, 0u, 0u);
-                v.rest[0] = r.x = norm2(v.rest[0], got.g[S::kFull].x, rstd);
-                if (S::T == 4) v.rest[1] = r.y = norm2(v.rest[1], got.g[S::kFull].y, rstd);
+                v.rest[0] = r.x = norm2(v.rest[0], got.g[S::kFull].x, tail);
+                if (S::T == 4) v.rest[1] = r.y = norm2(v.rest[1], got.g[S::kFull].y, tail);
                 am = absmax_bits8(r, am);
             }
             am = wave_reduce_last(am, [](uint32_t x, uint32_t y) { return max(x, y); });

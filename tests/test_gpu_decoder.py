@@ -654,6 +654,49 @@ def test_decode_stack_kernel_equals_the_kernels_per_layer(B, dim, ffn, nh, nkv, 
         step(9, min(33, S - 1))
 
 
+def _equal_or_both_nan(a, b):
+    """(Which of the NaNs is not part of a result.)"""
+    return bool(torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(a.nan_to_num(7.0), b.nan_to_num(7.0)))
+
+
+@pytest.mark.parametrize("where", ["row", "value", "infinity", "large"])
+@pytest.mark.parametrize("B,dim,ffn,nh,nkv", [
+    (1, 128, 64, 1, 1), (2, 1152, 2112, 9, 9), (1, 2560, 6912, 20, 5),
+])
+def test_decode_stack_kernel_carries_values_that_are_not_finite_like_the_kernels_per_layer(B, dim, ffn, nh, nkv, where):
+    S, n_splits = 70, 3
+    args = decoder.ModelArgs(dim=dim, n_layers=3, n_heads=nh, n_kv_heads=nkv, vocab_size=16, ffn_dim=ffn)
+    model = _build(args, seed=dim + B)
+    emb = model.tok_embeddings.weight.data
+    b = B - 1  # the sequence whose embedding row holds them
+    if where == "row":
+        emb[b] = float("nan")
+    elif where == "value":
+        emb[b, dim // 2 + 3] = float("nan")
+    elif where == "infinity":  # the norm makes zeros of the finite values, a NaN of this one
+        emb[b, 5] = float("-inf")
+        emb[b, 64:72] = float("inf")
+    else:  # the sum of squares is infinite, the values are not
+        emb[b] = emb[b] * 2.0**70
+    caches = [model.make_cache(B, S, "cuda") for _ in range(2)]
+    for (k, v), (k2, v2) in zip(*caches):
+        k2.copy_(k.normal_())
+        v2.copy_(v.normal_())
+    cos, sin = decoder.rope_tables(128, S, args.rope_theta, "cuda")
+    ws = decoder.AttnWorkspace(B, nh, nkv, n_splits, "cuda")
+    stack = decoder.DecodeStack(model, B, caches[1], n_splits)
+    tok = torch.arange(B, device="cuda").reshape(B, 1)
+    for p in (0, 40):
+        pos = torch.full((B, 1), p, dtype=torch.int64, device="cuda")
+        want = model.decode_hidden_fused(tok, pos, caches[0], cos, sin, ws)
+        h, rows = decoder.decode_step_begin(tok.reshape(B), pos.reshape(B), model.tok_embeddings.weight, cos, sin)
+        got = stack(h, pos.reshape(B), rows)
+        stack.check()
+        assert _equal_or_both_nan(got, want), p
+        for (k, v), (k2, v2) in zip(*caches):
+            assert _equal_or_both_nan(k, k2) and _equal_or_both_nan(v, v2), p
+
+
 @pytest.fixture(scope="module")
 def model_2b():
     model = _build(decoder.ModelArgs(), seed=0)
