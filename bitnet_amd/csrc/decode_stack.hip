@@ -76,9 +76,11 @@ constexpr int kStModePolls = 64;        // polls before the mode is decided with
 constexpr int kSc1 = kPollPolicy;       // device-coherent accesses
 typedef unsigned v2u __attribute__((ext_vector_type(2)));
 typedef int v2i __attribute__((ext_vector_type(2)));
-// Four int8 of quantized rows that mean "not written".  -128 comes from NaNs alone (|x| * scale rounds to 127 at most), and
-// a word of four of them is written as -127, -128, -128, -128 instead.  As an int, below every written word.
+// Four int8 of quantized rows that mean "not written": -128 comes from NaNs alone (|x| * scale rounds to 127 at most).  As
+// an int, below every other word.  A slice with a written word of that value says so in its record (kComplete).
 constexpr int kUnsetBytes = (int)0x80808080;
+constexpr unsigned kComplete = 1u << 30;
+constexpr int kLookEvery = 32;          // polls between two looks at that, a power of two
 constexpr int kBeyond = 0x7ffffff0;     // an offset behind every descriptor: reads as zero, no access
 
 // one product of one layer
@@ -251,9 +253,10 @@ __device__ __forceinline__ uint32_t quant2(uint32_t d, float s) {  // two bytes
     return __builtin_amdgcn_perm(quant_low_byte<0>(d & 0xffff0000u, s), quant_low_byte<0>(d << 16, s), 0x0c0c0400u);
 }
 
-// A quantized row's scale (bf16 bits) and the sums of its four waves' slices, 31 bits each: a set top bit is "not written"
+// A quantized row's scale (bf16 bits) and the sums of its four waves' slices, 30 bits each: a set top bit is "not
+// written", kComplete "the whole slice is in memory, also where it looks unset"
 struct RowRecord {
-    int sum[4];
+    unsigned sum[4];
     unsigned scale, pad[3];
 };
 static_assert(sizeof(RowRecord) == 32 && kStWaves == 4, "one 16-byte and one 4-byte load");
@@ -559,9 +562,9 @@ struct Stack {
     }
 
     // norm and quantizer of the wave's slices: the scales, the slices' sums, the bytes by put8 (8 of them, a 512-value
-    // piece's) and put_rest (S::T of them)
+    // piece's) and put_rest (S::T of them).  Whether there is a NaN in one of the rows.
     template <int UPW, class Put8, class PutRest>
-    __device__ __forceinline__ void quantize(const Task& tk, Got<MT>& got, float (&s)[TQ], int (&sum)[TQ], Put8 put8, PutRest put_rest) {
+    __device__ __forceinline__ bool quantize(const Task& tk, Got<MT>& got, float (&s)[TQ], int (&sum)[TQ], Put8 put8, PutRest put_rest) {
         typedef Slice<UPW> S;
 #pragma unroll
         for (int t = 0; t < TQ; ++t) {
@@ -590,27 +593,26 @@ struct Stack {
 #pragma unroll
             for (int k = 0; k < kStWaves; ++k) total += __builtin_bit_cast(double, v2i{x[k].x, x[k].y});
             const float rstd = reciprocal_sqrt(divide((float)total, (float)tk.K, tk.inv_k) + tk.eps);
-            // (values past the end of K stay zeros, also where rstd is NaN)
-            const float tail = lane * S::T < S::kRest && wave * S::kValues + S::kFull * 512 + lane * S::T < tk.K ? rstd : 0.0f;
             uint32_t am = 0;
 #pragma unroll
             for (int i = 0; i < S::kFull; ++i) {
-                v.full[i] = norm8(v.full[i], got.g[i], wave * S::kValues + i * 512 + lane * 8 < tk.K ? rstd : 0.0f);
+                v.full[i] = norm8(v.full[i], got.g[i], rstd);
                 am = absmax_bits8(v.full[i], am);
             }
             if (S::T) {
                 uint4 r = make_uint4(0u, 0u, 0u, 0u);
-                v.rest[0] = r.x = norm2(v.rest[0], got.g[S::kFull].x, tail);
-                if (S::T == 4) v.rest[1] = r.y = norm2(v.rest[1], got.g[S::kFull].y, tail);
+                v.rest[0] = r.x = norm2(v.rest[0], got.g[S::kFull].x, rstd);
+                if (S::T == 4) v.rest[1] = r.y = norm2(v.rest[1], got.g[S::kFull].y, rstd);
                 am = absmax_bits8(r, am);
             }
             am = wave_reduce_last(am, [](uint32_t x, uint32_t y) { return max(x, y); });
             if (lane == 63) lds_put(sh.amax[t][wave], v2i{(int)am, exchange + 1});
         }
         ++exchange;
+        bool nans = false;
 #pragma unroll
         for (int t = 0; t < TQ; ++t) {
-            const Values<kStUpwF>& v = got.f[t];
+            Values<kStUpwF>& v = got.f[t];
             v4i x[2];
             for (;;) {
                 asm volatile("" ::: "memory");
@@ -619,6 +621,16 @@ struct Stack {
                 if (uniform(min(min(x[0].y, x[0].w), min(x[1].y, x[1].w)) - exchange) >= 0) break;
             }
             const uint32_t am = (uint32_t)max(max(x[0].x, x[0].z), max(x[1].x, x[1].z));
+            if (uniform((int)am) > 0x7f80) {  // 0 times a NaN: the values past the end of K have to be zeros again
+                nans = true;
+#pragma unroll
+                for (int i = 0; i < S::kFull; ++i)
+                    if (wave * S::kValues + i * 512 + lane * 8 >= tk.K) v.full[i] = make_uint4(0u, 0u, 0u, 0u);
+                if (S::T && (lane * S::T >= S::kRest || wave * S::kValues + S::kFull * 512 + lane * S::T >= tk.K)) {
+                    v.rest[0] = 0u;
+                    if (S::T == 4) v.rest[1] = 0u;
+                }
+            }
             // quant_scale<0>
             s[t] = bf16_to_f32(f32_to_bf16_rne(reciprocal(fmaxf(__uint_as_float(am << 16), 1e-5f)) * 127.0f));
             int part = 0;
@@ -637,6 +649,7 @@ struct Stack {
             part = wave_reduce_last(part, [](int x, int y) { return x + y; });
             sum[t] = __builtin_amdgcn_readlane(part, 63);
         }
+        return nans;
     }
 
     // norm + quantizer of the wave's slices, products, outputs.  RPW 1, 2: row blocks; 4: two pairs (x1, x3), gated
@@ -751,13 +764,12 @@ struct Stack {
         const int first = wave * S::kValues, step = batch() * 64;
         const __amdgpu_buffer_rsrc_t to = make_rsrc(tk.dst, ((tk.K >> 6) - 1) * step + 64);
         auto place = [&](int at) { return (at >> 6) * step + (at & 63); };
-        auto written = [](unsigned w) { return w == (unsigned)kUnsetBytes ? w + 1u : w; };
         // (4 bytes at least a store: a word is there or not; values past the end of K are not stored)
-        quantize<UPW>(
+        const bool nans = quantize<UPW>(
             tk, got, s, sum,
             [&](int, int i, uint2 v) {
                 const int at = first + i * 512 + lane * 8;
-                __builtin_amdgcn_raw_buffer_store_b64(v2u{written(v.x), written(v.y)}, to, at < tk.K ? place(at) : kBeyond, 0, kSc1);
+                __builtin_amdgcn_raw_buffer_store_b64(v2u{v.x, v.y}, to, at < tk.K ? place(at) : kBeyond, 0, kSc1);
             },
             [&](int, uint32_t r) {
                 int at = first + S::kFull * 512 + lane * S::T;
@@ -766,11 +778,16 @@ struct Stack {
                     r = (r & 0xffffu) | (unsigned)__builtin_amdgcn_update_dpp(0, (int)r, 0xB1, 0xF, 0xF, true) << 16;
                     mine = mine && (lane & 1) == 0;
                 }
-                __builtin_amdgcn_raw_buffer_store_b32(written(r), to, mine ? place(at) : kBeyond, 0, kSc1);
+                __builtin_amdgcn_raw_buffer_store_b32(r, to, mine ? place(at) : kBeyond, 0, kSc1);
             });
         RowRecord* rec = (RowRecord*)tk.res;
+        unsigned mine = (unsigned)sum[0] & (kComplete - 1u);
+        if (nans) {  // readers cannot tell from the words that they are there
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+            mine |= kComplete;
+        }
         if (lane == 0) {
-            __hip_atomic_store(&rec->sum[wave], sum[0] & 0x7fffffff, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&rec->sum[wave], mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (wave == 0) __hip_atomic_store(&rec->scale, (unsigned)f32_to_bf16_rne(s[0]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
@@ -797,11 +814,21 @@ struct Stack {
         unsigned scale = 0;
         auto recorded = [&] { return (int)(sums.x | sums.y | sums.z | sums.w | (int)scale) >= 0; };
         auto lowest = [](int m, v4i v) { return min(min(min(m, v.x), min(v.y, v.z)), v.w); };
+        int unset = kUnsetBytes;  // of this lane's values; 1, which none has, once its slice is known to be in memory
         auto incomplete = [&] {
             int low = 0;
 #pragma unroll
             for (int j = 0; j < kLoads; ++j) low = lowest(low, b[j]);
-            return __builtin_amdgcn_ballot_w64(low == kUnsetBytes || !recorded() || (RES && got.res == 0xffffu)) != 0;
+            return __builtin_amdgcn_ballot_w64(low == unset || !recorded() || (RES && got.res == 0xffffu)) != 0;
+        };
+        // Whether this lane's slice is in memory, whatever it looks like: what is read behind this is what was written.
+        // Asked for seldom: with the answer in every poll eight sequences took 4 % more time.
+        auto vouched = [&] {
+            poll_again();
+            unsigned held = (unsigned)__builtin_amdgcn_raw_buffer_load_b32(
+                recs, pt < B ? pt * (int)sizeof(RowRecord) + wave * 4 : kBeyond, 0, kSc1);
+            asm volatile("" : "+v"(held));
+            return (int)held >= 0 && (held & kComplete) != 0;
         };
         // one piece until it is there, then all: all workgroups asking for all rows all the time fill the fabric, and so
         // do all asking for the same piece
@@ -811,6 +838,7 @@ struct Stack {
             poll_again();
             const v4i v = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rows, probe, 0, kSc1));
             if (__builtin_amdgcn_ballot_w64(lowest(0, v) == kUnsetBytes) == 0 || wt.dead || wt.give_up(spin)) break;
+            if ((spin & (kLookEvery - 1)) == kLookEvery - 1 && __builtin_amdgcn_ballot_w64(vouched()) != 0) break;
         }
         auto get = [&](auto policy) {
             poll_again();
@@ -823,7 +851,10 @@ struct Stack {
                                                    rows, j * SP + ps < live ? base + j * (SP * step) : (unsigned)kBeyond, 0, decltype(policy)::value));
         };
         get(std::integral_constant<int, 0>{});
-        for (int spin = 0; incomplete() && !wt.dead && !wt.give_up(spin); ++spin) get(std::integral_constant<int, kSc1>{});
+        for (int spin = 0; incomplete() && !wt.dead && !wt.give_up(spin); ++spin) {
+            if ((spin & (kLookEvery - 1)) == 3) unset = vouched() ? 1 : kUnsetBytes;
+            get(std::integral_constant<int, kSc1>{});
+        }
         v4i acc[RPW][SP];
 #pragma unroll
         for (int i = 0; i < RPW; ++i)
@@ -846,8 +877,8 @@ struct Stack {
             }
             if (p < MT) *(v4i*)&sh.red[turn][i][wave][p][4 * g] = v;
         }
-        auto sum31 = [](int v) { return (int)((unsigned)v << 1) >> 1; };
-        finish<RPW, RES>(tk, k, bf16_to_f32((uint16_t)scale), 2 * (sum31(sums.x) + sum31(sums.y) + sum31(sums.z) + sum31(sums.w)), got.res);
+        auto sum30 = [](int v) { return (int)((unsigned)v << 2) >> 2; };
+        finish<RPW, RES>(tk, k, bf16_to_f32((uint16_t)scale), 2 * (sum30(sums.x) + sum30(sums.y) + sum30(sums.z) + sum30(sums.w)), got.res);
         turn ^= 1;
     }
 

@@ -662,6 +662,8 @@ def _equal_or_both_nan(a, b):
 @pytest.mark.parametrize("where", ["row", "value", "infinity", "large"])
 @pytest.mark.parametrize("B,dim,ffn,nh,nkv", [
     (1, 128, 64, 1, 1), (2, 1152, 2112, 9, 9), (1, 2560, 6912, 20, 5),
+    # quantized rows between the workgroups: whole words of the code of a NaN, which is also what an unwritten word holds
+    (3, 128, 64, 1, 1), (4, 2560, 6912, 20, 5), (5, 1152, 2112, 9, 9), (8, 2560, 6912, 20, 5),
 ])
 def test_decode_stack_kernel_carries_values_that_are_not_finite_like_the_kernels_per_layer(B, dim, ffn, nh, nkv, where):
     S, n_splits = 70, 3
