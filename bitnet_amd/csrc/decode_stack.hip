@@ -293,7 +293,7 @@ struct Task {
                                 // where src are quantized rows, their records
     int K, n_out;               // attention: kv head, sequence
     float inv_k;                // attention: split
-    int flags;                  // 1: src is published, 2: dst is.  Attention: the position
+    int flags;                  // 1: src is published, 2: dst is, 4: res is.  Attention: the position
 };
 
 // a lane's values of one token's slice
@@ -419,9 +419,9 @@ struct Stack {
                 if (!kDirect) src = bytes(i), aux = record(i);
                 dst = (uint64_t)(i == 0 ? qkv(l) : i == 1 ? ha(l) : i == 2 ? gate(l) : last ? a->h_out : hb(l));
                 if (i == 0) n_out = (a->n_heads + 2 * a->n_kv) * kHeadDim;
-                if (i == 1) res = (uint64_t)h_before(l);
+                if (i == 1) res = (uint64_t)h_before(l), flags |= l == 0 ? 0 : 4;  // (the caller's values may be any)
                 if (i == 2) n_out = a->ffn;
-                if (i == 3) res = (uint64_t)ha(l);
+                if (i == 3) res = (uint64_t)ha(l), flags |= 4;
                 if (i == 3 && last) flags &= ~2;
             } else {
                 src += (uint64_t)wk.idx * K * 2;
@@ -535,7 +535,7 @@ struct Stack {
         for (int spin = 0;; ++spin) {
             poll_again();
             if (RES) got.res = (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(rs, res_off, 0, kSc1);
-            unsigned m = RES ? (unsigned)got.res << 16 : 0u;
+            unsigned m = RES && (tk.flags & 4) ? (unsigned)got.res << 16 : 0u;
 #pragma unroll
             for (int t = 0; t < TQ; ++t) {
                 Values<kStUpwF>& v = got.f[t];
@@ -819,7 +819,7 @@ struct Stack {
             int low = 0;
 #pragma unroll
             for (int j = 0; j < kLoads; ++j) low = lowest(low, b[j]);
-            return __builtin_amdgcn_ballot_w64(low == unset || !recorded() || (RES && got.res == 0xffffu)) != 0;
+            return __builtin_amdgcn_ballot_w64(low == unset || !recorded() || (RES && (tk.flags & 4) && got.res == 0xffffu)) != 0;
         };
         // Whether this lane's slice is in memory, whatever it looks like: what is read behind this is what was written.
         // Asked for seldom: with the answer in every poll eight sequences took 4 % more time.
