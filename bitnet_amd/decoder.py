@@ -299,6 +299,8 @@ def norm_bitlinear(x, norm: "RMSNorm", lin: BitLinearKernel, glu: bool = False, 
         raise ValueError(f"norm_bitlinear: x has shape {tuple(x.shape)}, expected [M, {2 * K if glu else K}]")
     if norm.weight.dtype != torch.bfloat16 or norm.weight.numel() != K:
         raise ValueError("norm_bitlinear: the norm weight must be bfloat16 [K]")
+    if lin.weight.numel() * lin.weight.element_size() * 4 != lin.out_features * K:
+        raise ValueError("norm_bitlinear: the packed weight must hold out_features x in_features codes")
     if residual is not None and (residual.dtype != torch.bfloat16 or residual.shape != (M, lin.out_features)
                                  or not residual.is_contiguous()):
         raise ValueError("norm_bitlinear: residual must be contiguous bfloat16 [M, N]")
@@ -329,21 +331,21 @@ class DecodeStack:
     as for a captured graph."""
 
     def __init__(self, model: "Transformer", batch: int, cache, n_splits: int):
+        if not self.applies(model, batch, cache, n_splits):
+            raise ValueError("DecodeStack: the kernel does not take this model, batch or cache")
         lib = _lib.load_library()
         a = model.args
         dev = cache[0][0].device
         self.shape = (a.n_layers, batch, cache[0][0].shape[1], a.dim, a.ffn_dim, a.n_heads, a.n_kv_heads, n_splits)
         words = []
         for layer, (ck, cv) in zip(model.layers, cache):
-            att, ffn = layer.attention, layer.feed_forward
-            for lin, norm in ((att.wqkv, layer.attention_norm), (att.wo, att.attn_sub_norm), (ffn.w13, layer.ffn_norm),
-                              (ffn.w2, ffn.ffn_sub_norm)):
+            for i, (lin, norm, _, _) in enumerate(self._products(layer, a)):
                 rows, slots = ctypes.c_int(), ctypes.c_uint32()
                 st = lib.bitlinear_scale_runs(lin.out_features, lin.in_features, lin._seg_c,
                                               len(lin.seg_ends) if lin.seg_ends else 0, ctypes.byref(rows), ctypes.byref(slots))
                 _lib.check(st, "bitlinear_scale_runs")
                 eps = struct.unpack("<I", struct.pack("<f", norm.eps))[0]
-                own = (ck.data_ptr(), cv.data_ptr()) if lin is att.wqkv else (0, 0)
+                own = (ck.data_ptr(), cv.data_ptr()) if i == 0 else (0, 0)
                 words += [lin.weight.data_ptr(), norm.weight.data_ptr(), lin.weight_scale.data_ptr(), *own,
                           eps | rows.value << 32, slots.value, 0]
         self.entries = torch.tensor(words, dtype=torch.int64, device=dev)
@@ -354,27 +356,41 @@ class DecodeStack:
 
     @staticmethod
     def applies(model: "Transformer", batch: int, cache, n_splits: int) -> bool:
-        """Whether the kernel takes this model: its sizes, bf16 norms and caches, the quantizer's default mode, weight
-        scales that change at multiples of 16 rows."""
+        """Whether the kernel takes this model: its sizes, the quantizer's default mode, weight scales that change at
+        multiples of 16 rows, and parameters and caches that
+        are what their addresses will be read as.  (The calls per layer look at each of them for themselves.)"""
         a = model.args
         lib = _lib.load_library()
-        if lib.bitnet_decode_stack_workspace_bytes(a.n_layers, batch, cache[0][0].shape[1], a.dim, a.ffn_dim, a.n_heads,
-                                                   a.n_kv_heads, n_splits) < 0:
+        dev, S = cache[0][0].device, cache[0][0].shape[1]
+        if len(cache) != a.n_layers or len(model.layers) != a.n_layers:
             return False
-        for layer, (ck, cv) in zip(model.layers, cache):
-            att, ffn = layer.attention, layer.feed_forward
-            if ck.dtype != torch.bfloat16 or cv.dtype != torch.bfloat16:
+        if lib.bitnet_decode_stack_workspace_bytes(a.n_layers, batch, S, a.dim, a.ffn_dim, a.n_heads, a.n_kv_heads, n_splits) < 0:
+            return False
+
+        def tensor_ok(t, dtype, shape=None, align=2):
+            return (t.dtype == dtype and t.device == dev and t.is_contiguous() and (shape is None or t.shape == shape)
+                    and t.data_ptr() % align == 0)
+
+        for layer, caches in zip(model.layers, cache):
+            if not all(tensor_ok(c, torch.bfloat16, (batch, S, a.n_kv_heads, 128), 16) for c in caches):
                 return False
-            for lin, norm in ((att.wqkv, layer.attention_norm), (att.wo, att.attn_sub_norm), (ffn.w13, layer.ffn_norm),
-                              (ffn.w2, ffn.ffn_sub_norm)):
+            for lin, norm, K, N in DecodeStack._products(layer, a):
                 rows, slots = ctypes.c_int(), ctypes.c_uint32()
-                if (lin.quant_mode != 0 or norm.weight.dtype != torch.bfloat16 or not lin.weight.is_contiguous()
-                        or (lin.weight.data_ptr() | norm.weight.data_ptr()) % 16
-                        or lib.bitlinear_scale_runs(lin.out_features, lin.in_features, lin._seg_c,
-                                                    len(lin.seg_ends) if lin.seg_ends else 0, ctypes.byref(rows),
+                if ((lin.in_features, lin.out_features) != (K, N) or lin.quant_mode != 0
+                        or not tensor_ok(lin.weight, torch.int8, (N, K // 4), 16) or not tensor_ok(norm.weight, torch.bfloat16, (K,), 16)
+                        or not tensor_ok(lin.weight_scale, torch.bfloat16)
+                        or lin.weight_scale.numel() < (len(lin.seg_ends) if lin.seg_ends else lib.bitlinear_ws_num(N, K))
+                        or lib.bitlinear_scale_runs(N, K, lin._seg_c, len(lin.seg_ends) if lin.seg_ends else 0, ctypes.byref(rows),
                                                     ctypes.byref(slots)) or rows.value % 16):
                     return False
         return True
+
+    @staticmethod
+    def _products(layer: "TransformerBlock", a: ModelArgs):
+        """The layer's four products in the kernel's order: module, the norm in front, K, N."""
+        att, ffn = layer.attention, layer.feed_forward
+        return ((att.wqkv, layer.attention_norm, a.dim, (a.n_heads + 2 * a.n_kv_heads) * 128), (att.wo, att.attn_sub_norm, a.dim, a.dim),
+                (ffn.w13, layer.ffn_norm, a.dim, 2 * a.ffn_dim), (ffn.w2, ffn.ffn_sub_norm, a.ffn_dim, a.dim))
 
     def reset(self) -> None:
         """The workspace as before its first use.  Not inside a graph capture."""
@@ -386,7 +402,9 @@ class DecodeStack:
         """h bf16 [B, dim], positions int64 [B], rope_rows as decode_step_begin returns them -> the hidden state behind
         the last layer, bf16 [B, dim]; the caches get the new token's rows."""
         n_layers, B, S, dim = self.shape[:4]
-        if h.shape != (B, dim) or h.dtype != torch.bfloat16 or positions.numel() != B or rope_rows.shape != (B, 128):
+        if (h.shape != (B, dim) or h.dtype != torch.bfloat16 or positions.numel() != B or positions.dtype != torch.int64
+                or rope_rows.shape != (B, 128) or rope_rows.dtype != torch.float32
+                or not (h.is_contiguous() and positions.is_contiguous() and rope_rows.is_contiguous())):
             raise ValueError("DecodeStack: h, positions or rope_rows do not match the batch it was made for")
         out = torch.empty_like(h)
         st = _lib.load_library().bitnet_decode_stack(

@@ -182,3 +182,51 @@ def test_host_calls_refuse_tensors_without_storage(call):
     }[call]
     with pytest.raises(RuntimeError, match="data pointer"):
         torch.vmap(run)(_device_tensor((3, *shape), dtype))
+
+
+def test_decode_stack_looks_at_what_its_addresses_point_to():
+    """The persistent decode kernel gets raw addresses: parameters and caches that it would read as something else leave
+    the step to the calls per layer, which refuse them (or take them)."""
+    import torch
+
+    from bitnet_amd import decoder
+
+    if not os.path.exists(_lib.LIB_PATH):
+        pytest.skip("library not built")
+    args = decoder.ModelArgs(dim=256, n_layers=2, n_heads=2, n_kv_heads=1, vocab_size=32, ffn_dim=128, segment_scales=True)
+
+    def made():
+        model = decoder.Transformer(args).to(torch.bfloat16)
+        return model, model.make_cache(2, 40, "cpu")
+
+    model, cache = made()
+    assert decoder.DecodeStack.applies(model, 2, cache, 3)
+
+    def att(m):
+        return m.layers[1].attention
+
+    def norm_of(width):
+        return lambda m, c: setattr(att(m).attn_sub_norm.weight, "data", torch.ones(width, dtype=torch.bfloat16))
+
+    def weight_of(t):
+        return lambda m, c: setattr(att(m).wqkv.weight, "data", t)
+
+    def scale_of(t):
+        return lambda m, c: setattr(att(m).wqkv.weight_scale, "data", t)
+
+    spoiled = {
+        "a short norm": norm_of(128), "a long norm": norm_of(257),
+        "an unpacked weight": weight_of(torch.zeros(512, 256, dtype=torch.int8)),
+        "a weight of few rows": weight_of(torch.zeros(256, 64, dtype=torch.int8)),
+        "a weight of another type": weight_of(torch.zeros(512, 64, dtype=torch.float32)),
+        "few scales": scale_of(torch.ones(2, dtype=torch.bfloat16)),
+        "scales of another type": scale_of(torch.ones(4, dtype=torch.float32)),
+        "a module of another width": lambda m, c: setattr(m.layers[0].feed_forward, "w2", decoder.BitLinearKernel(256, 256)),
+        "a cache of few rows": lambda m, c: c.__setitem__(1, tuple(t[:, :30].contiguous() for t in c[1])),
+        "a cache with gaps": lambda m, c: c.__setitem__(1, tuple(torch.cat((t, t), dim=3)[..., ::2] for t in c[1])),
+        "a cache of few layers": lambda m, c: c.pop(),
+    }
+    for what, spoil in spoiled.items():
+        model, cache = made()
+        spoil(model, cache)
+        assert not decoder.DecodeStack.applies(model, 2, cache, 3), what
