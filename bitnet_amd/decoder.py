@@ -357,7 +357,7 @@ class DecodeStack:
     @staticmethod
     def applies(model: "Transformer", batch: int, cache, n_splits: int) -> bool:
         """Whether the kernel takes this model: its sizes, the quantizer's default mode, weight scales that change at
-        multiples of 16 rows, and parameters and caches that
+        multiples of 16 rows, an eps that keeps 1 / sqrt away from the smallest numbers, and parameters and caches that
         are what their addresses will be read as.  (The calls per layer look at each of them for themselves.)"""
         a = model.args
         lib = _lib.load_library()
@@ -376,7 +376,7 @@ class DecodeStack:
                 return False
             for lin, norm, K, N in DecodeStack._products(layer, a):
                 rows, slots = ctypes.c_int(), ctypes.c_uint32()
-                if ((lin.in_features, lin.out_features) != (K, N) or lin.quant_mode != 0
+                if ((lin.in_features, lin.out_features) != (K, N) or lin.quant_mode != 0 or not norm.eps >= DecodeStack.kMinEps
                         or not tensor_ok(lin.weight, torch.int8, (N, K // 4), 16) or not tensor_ok(norm.weight, torch.bfloat16, (K,), 16)
                         or not tensor_ok(lin.weight_scale, torch.bfloat16)
                         or lin.weight_scale.numel() < (len(lin.seg_ends) if lin.seg_ends else lib.bitlinear_ws_num(N, K))
@@ -384,6 +384,10 @@ class DecodeStack:
                                                     ctypes.byref(slots)) or rows.value % 16):
                     return False
         return True
+
+    # 1 / sqrt(mean + eps) comes from the hardware's approximation and a correction step, which gives the rounded result
+    # for numbers from 2^-102 on; without an eps a row of zeros, whose norm is not a number, would come out as one
+    kMinEps = 2.0**-96
 
     @staticmethod
     def _products(layer: "TransformerBlock", a: ModelArgs):

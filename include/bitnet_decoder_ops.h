@@ -209,7 +209,8 @@ int bitnet_top_p_sample(const float* logits, const float* noise, void* workspace
  *   entries    64-byte aligned table of n_layers x 4 records (wqkv, wo, w13, w2) of eight 64-bit
  *              words: packed weight, weight of the RMSNorm in front (bf16), weight scales (bf16),
  *              cache_k, cache_v (wqkv's record only), eps as fp32 bits | slot_rows << 32,
- *              slot_map, 0 -- the last two from bitlinear_scale_runs; slot_rows a multiple of 16.
+ *              slot_map, 0 -- the last two from bitlinear_scale_runs; slot_rows a multiple of 16,
+ *              eps at least 2^-96.
  *              Device memory; what it points to must stay in place.
  *   workspace  bitnet_decode_stack_workspace_bytes() bytes, 256-byte aligned, set up once by
  *              bitnet_decode_stack_reset().  Calls that share it must not overlap in time.

@@ -222,6 +222,8 @@ def test_decode_stack_looks_at_what_its_addresses_point_to():
         "few scales": scale_of(torch.ones(2, dtype=torch.bfloat16)),
         "scales of another type": scale_of(torch.ones(4, dtype=torch.float32)),
         "a module of another width": lambda m, c: setattr(m.layers[0].feed_forward, "w2", decoder.BitLinearKernel(256, 256)),
+        "no eps": lambda m, c: setattr(m.layers[0].ffn_norm, "eps", 0.0),
+        "an eps that is no number": lambda m, c: setattr(m.layers[0].ffn_norm, "eps", float("nan")),
         "a cache of few rows": lambda m, c: c.__setitem__(1, tuple(t[:, :30].contiguous() for t in c[1])),
         "a cache with gaps": lambda m, c: c.__setitem__(1, tuple(torch.cat((t, t), dim=3)[..., ::2] for t in c[1])),
         "a cache of few layers": lambda m, c: c.pop(),
