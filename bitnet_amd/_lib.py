@@ -121,6 +121,7 @@ SIGNATURES = {
     "bitlinear_probe_empty": (_c_int, [_c_int, _c_int, _c_ptr]),
     "bitlinear_probe_weight_stream": (_c_int, [_c_ptr, _c_int, _c_int, _c_int, _c_ptr, _c_ptr]),
     "bitlinear_probe_mfma_i8": (_c_int, [_c_int, _c_int, _c_ptr, _c_ptr, _c_ptr]),
+    "bitlinear_probe_stack_math": (_c_int, [_c_int, ctypes.c_float, ctypes.c_uint32, ctypes.c_uint32, _c_ptr, _c_ptr]),
     "bitlinear_probe_flag_roundtrip": (_c_int, [_c_ptr, _c_int, _c_int, _c_int, _c_ptr, _c_ptr]),
 }
 

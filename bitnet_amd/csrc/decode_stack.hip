@@ -58,6 +58,7 @@
 #include "attn_device.h"
 #include "bitlinear_device.h"
 #include "bitlinear_hip.h"
+#include "bitlinear_probes.h"
 #include "bitnet_decoder_ops.h"
 #include "host_util.h"
 
@@ -200,12 +201,18 @@ __device__ __forceinline__ void load_to_lds(v4u rsrc, unsigned to, int voffset, 
                  : "memory");  // (m0 is the compiler's scratch: it sets it in front of each use of its own)
 }
 __device__ __forceinline__ void settled(v4u& rsrc) { asm volatile("s_nop 4" : "+s"(rsrc)); }
-// The correctly rounded results of the IEEE operations they replace, from the hardware's approximations and one
-// correction step each (found equal on every mantissa; the operands are positive or NaN, which stays one)
-__device__ __forceinline__ float divide(float x, float by, float inv) {  // inv: 1 / by, correctly rounded
+// The results of the IEEE operations they replace, bit for bit, from the hardware's approximations and one correction step
+// each, at a third of the instructions.  Not on all arguments (compared one by one by decode_stack_math_kernel): 1 / x
+// from 2^-126 to 2^126, which holds every maximum that leaves the scale's reciprocal a normal number; 1 / sqrt(x) from
+// 2^-102 on, below which no caller's eps lies; x / width from 2^-115 on, below which the quotient vanishes next to such an eps;
+// a sum over a scale as long as its first approximation does not overflow, scales of 2^-108 and more.  NaNs stay NaNs.
+__device__ __forceinline__ float quotient(float x, float by, float inv) {  // inv: 1 / by, correctly rounded
     const float q = x * inv;
-    const float r = __builtin_fmaf(__builtin_fmaf(-q, by, x), inv, q);
-    return q < INFINITY ? r : q;
+    return __builtin_fmaf(__builtin_fmaf(-q, by, x), inv, q);
+}
+__device__ __forceinline__ float divide(float x, float by, float inv) {
+    const float q = x * inv;
+    return q < INFINITY ? quotient(x, by, inv) : q;
 }
 __device__ __forceinline__ float reciprocal(float x) {
     const float r = __builtin_amdgcn_rcpf(x);
@@ -732,8 +739,7 @@ struct Stack {
                 int sum = -less;
 #pragma unroll
                 for (int k = 0; k < kStWaves; ++k) sum += sh.red[turn][i][k][m][row];
-                const float x = (float)sum, q = x * inv_s;  // the quotient as in the other kernels' epilogues
-                return f32_to_bf16_rne(__builtin_fmaf(__builtin_fmaf(-q, sm, x), inv_s, q) * bf16_to_f32(ws));
+                return f32_to_bf16_rne(quotient((float)sum, sm, inv_s) * bf16_to_f32(ws));
             };
             uint16_t v = value(tb, ws[0]);
             if (RPW == 4) {
@@ -1190,6 +1196,35 @@ __global__ __launch_bounds__(256) void decode_stack_reset_kernel(v4u* ws, long l
     }
 }
 
+// The short forms above against the IEEE operations in their place: how many of n arguments give other bits, and the
+// lowest and the highest of them (found[0..2])
+__global__ __launch_bounds__(256) void decode_stack_math_kernel(int what, float by, unsigned first, unsigned n, unsigned* found) {
+    unsigned wrong = 0, low = ~0u, high = 0;
+    const float inv = 1.0f / by;
+    for (unsigned long long i = (unsigned long long)blockIdx.x * 256 + threadIdx.x; i < n; i += (unsigned long long)gridDim.x * 256) {
+        const unsigned at = first + (unsigned)i;
+        const float x = what == 3 ? (float)(int)at : __uint_as_float(at);
+        float a, b;
+        switch (what) {
+            case 0: a = reciprocal(x), b = 1.0f / x; break;
+            case 1: a = reciprocal_sqrt(x), b = 1.0f / __builtin_sqrtf(x); break;
+            case 2: a = divide(x, by, inv), b = x / by; break;
+            default: a = quotient(x, by, inv), b = x / by; break;
+        }
+        const bool same = __float_as_uint(a) == __float_as_uint(b) || (a != a && b != b);
+        if (!same) {
+            ++wrong;
+            low = min(low, at);
+            high = max(high, at);
+        }
+    }
+    if (wrong) {
+        atomicAdd(&found[0], wrong);
+        atomicMin(&found[1], low);
+        atomicMax(&found[2], high);
+    }
+}
+
 long long up256(long long v) { return (v + 255) & ~255ll; }
 
 // Fills in everything that follows from the sizes; false: not a shape these kernels take
@@ -1301,6 +1336,13 @@ int bitnet_decode_stack(const void* entries, void* workspace, const uint16_t* h_
     else BITNET_STACK(8);
 #undef BITNET_STACK
     return hipGetLastError() == hipSuccess ? 0 : 3;
+}
+
+int bitlinear_probe_stack_math(int what, float by, uint32_t first, uint32_t n, uint32_t* found, void* stream) {
+    if (what < 0 || what > 3 || !(by > 0.0f) || !n) return BITLINEAR_ERR_ARG;
+    if (!found) return BITLINEAR_ERR_NULL;
+    hipLaunchKernelGGL(decode_stack_math_kernel, dim3(4096), dim3(256), 0, (hipStream_t)stream, what, by, first, n, found);
+    return hipGetLastError() == hipSuccess ? BITLINEAR_OK : BITLINEAR_ERR_LAUNCH;
 }
 
 }  // extern "C"

@@ -4,8 +4,9 @@
  * run and launch style as its headline, what a kernel launch costs on this
  * machine when the kernel does nothing, when it only requests a matrix's bytes,
  * what the matrix pipe sustains on the operand values of this workload, and what handing a flag from one
- * workgroup to another costs.  Same conventions as include/bitlinear_hip.h: device pointers owned by
- * the caller, no allocation, no synchronisation, launches on the given stream.
+ * workgroup to another costs.  One more compares a kernel's arithmetic, for a test.  Same conventions as
+ * include/bitlinear_hip.h: device pointers owned by the caller, no allocation, no synchronisation, launches
+ * on the given stream.
  */
 #ifndef BITLINEAR_PROBES_H
 #define BITLINEAR_PROBES_H
@@ -57,6 +58,18 @@ int bitlinear_probe_mfma_i8(int mode, int iters, uint32_t* sink, long long* ops,
  * zeroed by the caller) becomes 1 if one ran out.  Returns a BITLINEAR_* code.
  */
 int bitlinear_probe_flag_roundtrip(uint32_t* flags, int wg_a, int wg_b, int rounds, int* gave_up, void* stream);
+
+/*
+ * One launch that compares the short forms of division and square root in the
+ * persistent decode kernel with the IEEE operations in their place, for `n`
+ * consecutive arguments from `first` on: bit patterns of floats for
+ *   what 0: 1 / x    1: 1 / sqrt(x)    2: x / by
+ * and signed integers, as sums of products are, for what 3: x / by.  found:
+ * three device words, set by the caller to 0, ~0, 0: how many arguments give
+ * other bits (NaNs count as equal), the lowest and the highest of them.
+ * Returns a BITLINEAR_* code.
+ */
+int bitlinear_probe_stack_math(int what, float by, uint32_t first, uint32_t n, uint32_t* found, void* stream);
 
 #ifdef __cplusplus
 }

@@ -204,7 +204,8 @@ int bitnet_top_p_sample(const float* logits, const float* noise, void* workspace
  * All decoder layers of one decode step (gpu/model.py:214-245: norm + wqkv, rope + cache write +
  * attention, sub-norm + wo + residual, norm + w13, gate + sub-norm + w2 + residual, n_layers times,
  * one new token per sequence) in one kernel of one workgroup per CU.  Same results, bit for bit, as
- * bitlinear_norm_forward_bf16[_seg] (mode 0) and bitnet_attn_decode called for every layer.
+ * bitlinear_norm_forward_bf16[_seg] (mode 0) and bitnet_attn_decode called for every layer, for rows whose
+ * normalised values stay below 2^115; which of the NaNs a NaN is may differ.
  *
  *   entries    64-byte aligned table of n_layers x 4 records (wqkv, wo, w13, w2) of eight 64-bit
  *              words: packed weight, weight of the RMSNorm in front (bf16), weight scales (bf16),

@@ -654,6 +654,38 @@ def test_decode_stack_kernel_equals_the_kernels_per_layer(B, dim, ffn, nh, nkv, 
         step(9, min(33, S - 1))
 
 
+def test_short_divisions_of_the_decode_stack_kernel_equal_the_ieee_operations():
+    """Every argument in the ranges that the kernel's callers leave it (where the bits of a float end: inf and the NaNs)."""
+    lib = _lib.load_library()
+    found = torch.empty(3, dtype=torch.int32, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+
+    def bits(x):
+        return int(np.float32(x).view(np.uint32))
+
+    def compare(what, calls):
+        found.copy_(torch.tensor([0, -1, 0], dtype=torch.int32))
+        for by, first, n in calls:
+            assert lib.bitlinear_probe_stack_math(what, by, first & 0xFFFFFFFF, n, found.data_ptr(), stream) == 0
+        wrong, low, high = (v & 0xFFFFFFFF for v in found.tolist())
+        assert wrong == 0, (what, wrong, hex(low), hex(high))
+
+    def floats(low, end=1 << 31):
+        return 1.0, bits(low), end - bits(low)
+
+    compare(0, [floats(2.0**-126, bits(2.0**126) + 1), floats(float("inf"))])
+    compare(1, [floats(2.0**-102)])
+    compare(2, [(float(k), *floats(2.0**-115)[1:]) for k in range(64, 6912 + 1, 64)])
+    # a sum of products over the scale of a row: bf16 from 127 / 2^115 to 127 / 1e-5
+    largest = 128 * 6912
+    lo, hi = bits(2.0**-108) >> 16, bits(127 / 1e-5) >> 16
+    scales = (np.arange(lo, hi + 2, dtype=np.uint32) << 16).view(np.float32)
+    compare(3, [(float(v), -largest, 2 * largest + 1) for v in scales])
+    # and the comparison finds differences where there are some: reciprocals that are no normal numbers
+    assert lib.bitlinear_probe_stack_math(0, 1.0, bits(2.0**126) + 1, 1000, found.data_ptr(), stream) == 0
+    assert found.tolist() == [1000, bits(2.0**126) + 1, bits(2.0**126) + 1000]
+
+
 def _equal_or_both_nan(a, b):
     """(Which of the NaNs is not part of a result.)"""
     return bool(torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(a.nan_to_num(7.0), b.nan_to_num(7.0)))
