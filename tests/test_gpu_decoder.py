@@ -610,14 +610,19 @@ def test_norm_bitlinear_of_rows_that_are_not_finite(M, K, N):
 # 128256 (gpu/model.py:39-49), a 512-token seeded prompt, greedy decode (gpu/generate.py:264-288)
 # ---------------------------------------------------------------------------
 @pytest.mark.parametrize("workgroups", [0, 1, 7, 600])  # 600: more than can be resident, tasks by ticket
-@pytest.mark.parametrize("B,dim,ffn,nh,nkv,S,n_splits", [
-    (1, 128, 64, 1, 1, 33, 1), (2, 128, 64, 1, 1, 40, 16), (1, 1152, 2112, 9, 9, 70, 3), (2, 1024, 1984, 8, 1, 700, 5),
-    (1, 2560, 6912, 20, 5, 545, 8), (2, 2560, 6912, 20, 5, 300, 8),
+@pytest.mark.parametrize("B,dim,ffn,nh,nkv,S,n_splits,segments", [
+    (1, 128, 64, 1, 1, 33, 1, False), (2, 128, 64, 1, 1, 40, 16, False), (1, 1152, 2112, 9, 9, 70, 3, False),
+    (2, 1024, 1984, 8, 1, 700, 5, False), (1, 2560, 6912, 20, 5, 545, 8, False), (2, 2560, 6912, 20, 5, 300, 8, False),
     # beyond two tokens the input rows are quantized by tasks of their own
-    (3, 128, 64, 1, 1, 40, 16), (5, 1152, 2112, 9, 9, 70, 3), (8, 1024, 1984, 8, 1, 700, 5), (8, 2560, 6912, 20, 5, 545, 6),
+    (3, 128, 64, 1, 1, 40, 16, False), (5, 1152, 2112, 9, 9, 70, 3, False), (8, 1024, 1984, 8, 1, 700, 5, False),
+    (8, 2560, 6912, 20, 5, 545, 6, False),
+    # a weight scale per sub-tensor, as a converted checkpoint has: up to eight runs of rows (here 6 and 3 of wqkv, 2 of
+    # w13, whose halves meet in one task)
+    (1, 2560, 6912, 20, 5, 70, 3, True), (2, 512, 2112, 4, 1, 40, 2, True), (4, 384, 64, 3, 3, 40, 2, True),
+    (8, 2560, 6912, 20, 5, 70, 6, True),
 ])
-def test_decode_stack_kernel_equals_the_kernels_per_layer(B, dim, ffn, nh, nkv, S, n_splits, workgroups):
-    args = decoder.ModelArgs(dim=dim, n_layers=2, n_heads=nh, n_kv_heads=nkv, vocab_size=256, ffn_dim=ffn)
+def test_decode_stack_kernel_equals_the_kernels_per_layer(B, dim, ffn, nh, nkv, S, n_splits, workgroups, segments):
+    args = decoder.ModelArgs(dim=dim, n_layers=2, n_heads=nh, n_kv_heads=nkv, vocab_size=256, ffn_dim=ffn, segment_scales=segments)
     model = _build(args, seed=dim + B)
     caches = [model.make_cache(B, S, "cuda") for _ in range(2)]
     for (k, v), (k2, v2) in zip(*caches):
