@@ -23,46 +23,62 @@ namespace {
 
 constexpr int kSpPieces = 16;
 constexpr int kSpThreads = 1024;
-// Levels of a magnitude: 0 below 2^-20 (zero included), then one per bf16 value, the last one for all from
-// 2^44 on.  Buckets in the order of the ranks: positive values downwards, level 0, negative ones.
-constexpr int kSpLow = (127 - 20) << 7;
+// Levels of a magnitude: 0 for all below the bf16 bits `low` (zero included), then one per bf16 value, the last one for
+// all from 64 powers of two above on.  Buckets in the order of the ranks: positive values downwards, level 0, negative
+// ones.  `low` follows the temperature (sp_low): values below 2^-24 of it have the probability of zero, to half a unit
+// in the last place of a float, and two different ones of 2^40 of it and more are so far apart that the lower one's
+// probability is zero, so of an outermost bucket only the largest value counts (SpPiece).  All buckets of bf16, 65281,
+// are more than the LDS holds.
 constexpr int kSpLevels = 64 << 7;
 constexpr int kSpBuckets = 2 * kSpLevels + 1;
 constexpr int kSpRow = (kSpBuckets + 7) & ~7;
 
 struct SpPiece {
     int first, last;  // its buckets in use (last < first: none)
+    int key, count;   // the largest value (as sp_key) and how often it is there, where `first` is an outermost bucket
 };
 struct SpWinner {
     float v;
     int r, bucket, place;
 };
-static_assert(sizeof(SpWinner) == 16, "one 16-byte store");
+static_assert(sizeof(SpWinner) == 16 && sizeof(SpPiece) == 16, "one 16-byte store");
 
-__device__ __forceinline__ int sp_bucket(float logit) {
+// bf16 bits of the power of two at least 2^-25 and less than 2^-24 of the temperature; 1, above zero alone, for the smallest
+int sp_low(float temperature) {
+    int e;
+    frexpf(temperature, &e);  // 2^(e - 1) <= temperature < 2^e
+    const int low = (127 + e - 1 - 24) << 7;
+    return low < 1 ? 1 : low;
+}
+__device__ __forceinline__ int sp_bucket(float logit, int low) {
     const int b = (int)(__float_as_uint(logit) >> 16), mag = b & 0x7fff;
-    const int level = mag < kSpLow ? 0 : min(mag - kSpLow + 1, kSpLevels);
+    const int level = mag < low ? 0 : min(mag - low + 1, kSpLevels);
     return b & 0x8000 ? kSpLevels + level : kSpLevels - level;
 }
-__device__ __forceinline__ float sp_value(int bucket) {
+// (an outermost bucket's value of least magnitude)
+__device__ __forceinline__ float sp_value(int bucket, int low) {
     const int d = bucket - kSpLevels, level = d < 0 ? -d : d;
-    const float m = level ? __uint_as_float((unsigned)(kSpLow + level - 1) << 16) : 0.0f;
+    const float m = level ? __uint_as_float((unsigned)(low + level - 1) << 16) : 0.0f;
     return d > 0 ? -m : m;
 }
+__device__ __forceinline__ bool sp_outermost(int bucket) { return bucket == 0 || bucket == kSpBuckets - 1; }
 // order of bf16 values within a bucket of several, larger first
 __device__ __forceinline__ int sp_key(float logit) {
     const int b = (int)(__float_as_uint(logit) >> 16), mag = b & 0x7fff;
     return b & 0x8000 ? 0x7fff + mag : 0x7fff - mag;  // both zeros: 0x7fff
 }
+__device__ __forceinline__ float sp_value_of_key(int key) {
+    return key > 0x7fff ? -__uint_as_float((unsigned)(key - 0x7fff) << 16) : __uint_as_float((unsigned)(0x7fff - key) << 16);
+}
 __device__ __forceinline__ int sp_piece_size(int V) { return ((V + kSpPieces - 1) / kSpPieces + 3) & ~3; }
 
 __global__ __launch_bounds__(kSpThreads) void sample_count_kernel(const float* __restrict__ logits, uint16_t* __restrict__ counts,
-                                                                  SpPiece* __restrict__ pieces, int* __restrict__ error, int V) {
+                                                                  SpPiece* __restrict__ pieces, int* __restrict__ error, int low, int V) {
     __shared__ __attribute__((aligned(16))) unsigned hist[kSpRow];
-    __shared__ int first, last;
+    __shared__ int first, last, top_key, top_count;
     const int tid = threadIdx.x, piece = blockIdx.x, row = blockIdx.y;
     for (int i = tid; i < kSpRow / 4; i += kSpThreads) ((v4u*)hist)[i] = v4u{0u, 0u, 0u, 0u};
-    if (tid == 0) first = kSpBuckets, last = -1;
+    if (tid == 0) first = kSpBuckets, last = -1, top_key = 0xffff, top_count = 0;
     __syncthreads();
     const int size = sp_piece_size(V), lo = piece * size, hi = min(V, lo + size);
     const float* x = logits + (size_t)row * V;
@@ -71,7 +87,7 @@ __global__ __launch_bounds__(kSpThreads) void sample_count_kernel(const float* _
     for (int i = lo + tid; i < hi; i += kSpThreads) {
         const float v = x[i];
         bad = bad || !(v < INFINITY);  // a NaN or an infinite logit: no distribution
-        const int b = sp_bucket(v);
+        const int b = sp_bucket(v, low);
         mn = min(mn, b);
         mx = max(mx, b);
         atomicAdd(&hist[b], 1u);
@@ -87,14 +103,22 @@ __global__ __launch_bounds__(kSpThreads) void sample_count_kernel(const float* _
     }
     if (bad) __hip_atomic_store(error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     __syncthreads();
-    if (tid == 0) pieces[row * kSpPieces + piece] = SpPiece{first, last};
+    if (sp_outermost(first)) {  // rare; the same for all threads
+        for (int i = lo + tid; i < hi; i += kSpThreads)
+            if (sp_bucket(x[i], low) == first) atomicMin(&top_key, sp_key(x[i]));
+        __syncthreads();
+        for (int i = lo + tid; i < hi; i += kSpThreads)
+            if (sp_key(x[i]) == top_key) atomicAdd(&top_count, 1);
+        __syncthreads();
+    }
+    if (tid == 0) pieces[row * kSpPieces + piece] = SpPiece{first, last, top_key, top_count};
     uint32_t* to = (uint32_t*)(counts + (size_t)(row * kSpPieces + piece) * kSpRow);
     for (int i = (first >> 1) + tid; 2 * i <= last; i += kSpThreads) to[i] = hist[2 * i] | hist[2 * i + 1] << 16;
 }
 
 __global__ __launch_bounds__(kSpThreads) void sample_race_kernel(const uint16_t* __restrict__ counts, const SpPiece* __restrict__ pieces,
                                                                  const float* __restrict__ noise, SpWinner* __restrict__ winners,
-                                                                 int* __restrict__ error, float inv_t, float top_p, int V) {
+                                                                 int* __restrict__ error, float inv_t, float top_p, int low, int V) {
     __shared__ __attribute__((aligned(16))) unsigned before[kSpRow];  // counts, then ranks in front of a bucket
     __shared__ __attribute__((aligned(16))) float odds[kSpRow];       // exp(its logit - the largest)
     __shared__ double wave_mass[kSpThreads / 64];
@@ -110,7 +134,15 @@ __global__ __launch_bounds__(kSpThreads) void sample_race_kernel(const uint16_t*
         first = min(first, p[k].first);
         last = max(last, p[k].last);
     }
-    const float m = sp_value(first) * inv_t;
+    // of an outermost bucket the largest value's tokens are in the draw, as its first ranks, and no other token is
+    int key = 0xffff, largest_count = 0;
+    if (sp_outermost(first)) {
+#pragma unroll
+        for (int k = 0; k < kSpPieces; ++k) key = min(key, p[k].first == first ? p[k].key : 0xffff);
+#pragma unroll
+        for (int k = 0; k < kSpPieces; ++k) largest_count += p[k].first == first && p[k].key == key ? p[k].count : 0;
+    }
+    const float m = sp_value(first, low) * inv_t;
     const uint32_t* c = (const uint32_t*)(counts + (size_t)row * kSpPieces * kSpRow);
     const int base = first & ~1, n = last + 1 - base;
     for (int i = tid; 2 * i < n; i += kSpThreads) {
@@ -127,14 +159,20 @@ __global__ __launch_bounds__(kSpThreads) void sample_race_kernel(const uint16_t*
         }
         before[2 * i] = lo;
         before[2 * i + 1] = hi;
-        odds[2 * i] = expf(sp_value(at) * inv_t - m);
-        odds[2 * i + 1] = expf(sp_value(at + 1) * inv_t - m);
+        odds[2 * i] = at < first ? 0.0f : expf(sp_value(at, low) * inv_t - m);  // (a value above the largest: infinite)
+        odds[2 * i + 1] = expf(sp_value(at + 1, low) * inv_t - m);
     }
     if (tid == 0) {
-        kept = V;
-        if (first >= kSpBuckets - 1) __hip_atomic_store(error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);  // all -inf
+        kept = largest_count ? largest_count : V;
+        // the largest logit over the temperature is no number: all are -inf, or it overflows
+        const float largest = (largest_count ? sp_value_of_key(key) : sp_value(first, low)) * inv_t;
+        if (!(fabsf(largest) < INFINITY)) __hip_atomic_store(error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
     __syncthreads();
+    if (largest_count) {
+        if (tid == 0) before[first - base] = (unsigned)largest_count;
+        __syncthreads();
+    }
     // every thread a run of buckets
     const int per = (n + kSpThreads - 1) / kSpThreads, at0 = min(n, tid * per), at1 = min(n, at0 + per);
     unsigned count = 0;
@@ -296,7 +334,7 @@ __global__ __launch_bounds__(kSpThreads) void sample_token_kernel(const float* _
                                                                   const SpPiece* __restrict__ pieces, const SpWinner* __restrict__ winners,
                                                                   int64_t* __restrict__ token_out, int64_t* __restrict__ next_input,
                                                                   int64_t* __restrict__ positions, int64_t* __restrict__ history_row,
-                                                                  int* __restrict__ error, int V) {
+                                                                  int* __restrict__ error, int low, int V) {
     __shared__ int wave_count[kSpThreads / 64];
     __shared__ unsigned hist[256];
     __shared__ int found;
@@ -311,7 +349,7 @@ __global__ __launch_bounds__(kSpThreads) void sample_token_kernel(const float* _
     const float* x = logits + (size_t)row * V;
     int place = w.place;
     __syncthreads();
-    if (w.bucket > 0 && w.bucket < kSpBuckets - 1 && w.bucket != kSpLevels) {  // tokens of one value
+    if (w.bucket >= 0 && !sp_outermost(w.bucket) && w.bucket != kSpLevels) {  // tokens of one value
         const int size = sp_piece_size(V);
         unsigned n[kSpPieces];
 #pragma unroll
@@ -327,7 +365,7 @@ __global__ __launch_bounds__(kSpThreads) void sample_token_kernel(const float* _
                 else place -= (int)n[k];
             }
         const int lo = min(V, piece * size);
-        sp_pick(x, lo, min(V, lo + size), place, wave_count, &found, [&](float v) { return sp_bucket(v) == w.bucket; });
+        sp_pick(x, lo, min(V, lo + size), place, wave_count, &found, [&](float v) { return sp_bucket(v, low) == w.bucket; });
     } else if (w.bucket >= 0) {
         // a bucket of several values: the value by its high byte and then its low one, over the whole row (rare)
         int prefix = 0, mask = 0;
@@ -336,7 +374,7 @@ __global__ __launch_bounds__(kSpThreads) void sample_token_kernel(const float* _
             __syncthreads();
             for (int i = tid; i < V; i += kSpThreads) {
                 const int key = sp_key(x[i]);
-                if (sp_bucket(x[i]) == w.bucket && ((key ^ prefix) & mask) == 0) atomicAdd(&hist[(key >> shift) & 255], 1u);
+                if (sp_bucket(x[i], low) == w.bucket && ((key ^ prefix) & mask) == 0) atomicAdd(&hist[(key >> shift) & 255], 1u);
             }
             __syncthreads();
             int digit = 0;
@@ -345,7 +383,7 @@ __global__ __launch_bounds__(kSpThreads) void sample_token_kernel(const float* _
             mask |= 255 << shift;
             __syncthreads();
         }
-        sp_pick(x, 0, V, place, wave_count, &found, [&](float v) { return sp_bucket(v) == w.bucket && sp_key(v) == prefix; });
+        sp_pick(x, 0, V, place, wave_count, &found, [&](float v) { return sp_bucket(v, low) == w.bucket && sp_key(v) == prefix; });
     }
     if (tid == 0) {
         const int64_t token = found >= 0 ? found : 0;
@@ -373,6 +411,7 @@ int bitnet_top_p_sample(const float* logits, const float* noise, void* workspace
                         int64_t* token_out, int64_t* next_input, int64_t* positions, int64_t* history_row, int* error, int B, int V,
                         void* stream) {
     const float inv_t = 1.0f / temperature;
+    const int low = sp_low(temperature);
     if (bitnet_top_p_workspace_bytes(B, V) < 0 || !(inv_t > 0.0f) || !(inv_t < INFINITY) || !(top_p >= 0.0f)) return 1;
     if (!logits || !noise || !workspace || !token_out || !error) return 2;
     if ((uintptr_t)workspace & 15u) return 1;
@@ -382,10 +421,10 @@ int bitnet_top_p_sample(const float* logits, const float* noise, void* workspace
     SpPiece* pieces = (SpPiece*)ws;
     SpWinner* winners = (SpWinner*)(ws + up16((size_t)B * kSpPieces * sizeof(SpPiece)));
     const hipStream_t s = (hipStream_t)stream;
-    hipLaunchKernelGGL(sample_count_kernel, dim3(kSpPieces, B), dim3(kSpThreads), 0, s, logits, counts, pieces, error, V);
-    hipLaunchKernelGGL(sample_race_kernel, dim3(kSpPieces, B), dim3(kSpThreads), 0, s, counts, pieces, noise, winners, error, inv_t, top_p, V);
+    hipLaunchKernelGGL(sample_count_kernel, dim3(kSpPieces, B), dim3(kSpThreads), 0, s, logits, counts, pieces, error, low, V);
+    hipLaunchKernelGGL(sample_race_kernel, dim3(kSpPieces, B), dim3(kSpThreads), 0, s, counts, pieces, noise, winners, error, inv_t, top_p, low, V);
     hipLaunchKernelGGL(sample_token_kernel, dim3(B), dim3(kSpThreads), 0, s, logits, counts, pieces, winners, token_out, next_input,
-                       positions, history_row, error, V);
+                       positions, history_row, error, low, V);
     return hipGetLastError() == hipSuccess ? 0 : 3;
 }
 

@@ -185,14 +185,14 @@ int bitnet_lm_head_logits(const uint16_t* h, const uint16_t* norm_weight, float 
  * One token per row by nucleus sampling (gpu/sample_utils.py:9-33, gpu/generate.py:270-277): softmax of
  * logits / temperature; a token stays while the probability in front of it in the sorted order (ties by
  * index) is at most top_p; of the ranks that stay, the one with the largest probability / noise[rank].
- *   logits     fp32 [B, V] of bf16 values, as the LM head writes them.  (Magnitudes below 2^-20 count as
- *              zero in the probabilities and from 2^44 as 2^44; their order is kept.)
+ *   logits     fp32 [B, V] of bf16 values, as the LM head writes them.  (In the probabilities magnitudes
+ *              below 2^-24 of the temperature count as zero; their order is kept.)
  *   noise      fp32 [B, V], independent draws of an exponential distribution
  *   workspace  bitnet_top_p_workspace_bytes() bytes, 16-byte aligned; contents need not be kept
  *   token_out  int64 [B] (may be pinned host memory)
  *   next_input, positions, history_row  int64 [B] each or NULL: token, += 1, token
- *   error      set to 1 if a row has no distribution (a NaN or infinite logit, or nothing above -2^44);
- *              may be pinned host memory; never cleared here
+ *   error      set to 1 if a row has no distribution (a NaN or infinite logit, or a largest logit that is
+ *              not finite over the temperature); may be pinned host memory; never cleared here
  * temperature > 0, top_p >= 0, V <= 1048496.  Returns 0, 1 (arguments), 2 (null), 3 (launch).
  */
 long long bitnet_top_p_workspace_bytes(int B, int V);

@@ -359,6 +359,45 @@ def test_top_p_sampler_draws_what_torch_draws(B, V, logits):
             sampler.check()
 
 
+@pytest.mark.parametrize("sign", ["any", "negative", "masked"])
+@pytest.mark.parametrize("scale,temperature", [
+    (2.0**-21, 1e-8), (2.0**-21, 2.0**-21), (2.0**-60, 2.0**-61), (2.0**-90, 2e-27),  # small values at small temperatures
+    (2.0**20, 2.0**-22), (2.0**50, 0.7), (2.0**44, 2.0**44), (2.0**60, 1.0),          # large ones: the largest alone, or not
+    (2.0**95, 3e28), (1.0, 9e29), (2.0**-10, 1e6),                                    # large temperatures
+])
+def test_top_p_sampler_tells_values_apart_at_every_temperature(scale, temperature, sign):
+    B, V = 3, 2048
+    gen = torch.Generator(device="cuda").manual_seed(11)
+    x = torch.randn(B, V, generator=gen, device="cuda") * scale
+    if sign != "any":
+        x = -x.abs() - scale
+    if sign == "masked":
+        x[:, ::3] = float("-inf")
+    x = x.to(torch.bfloat16).float()
+    x[1, :700] = x[1, x[1].argmax()]  # (many tokens of the largest value)
+    assert decoder.TopPSampler.applies(B, V, temperature, 0.9)
+    sampler = decoder.TopPSampler(B, V, "cuda")
+    tok = torch.zeros(B, dtype=torch.int64, device="cuda")
+    probs = torch.softmax(x.double() / float(np.float32(temperature)), dim=-1)
+    order = torch.sort(x, dim=-1, descending=True, stable=True)[1]
+    ranked = torch.gather(probs, -1, order)
+    for draw, p in enumerate((0.95, 0.5, 1.0, 0.0)):
+        kept = torch.where(torch.cumsum(ranked, -1) - ranked > p + 1e-12, 0.0, ranked)
+        q = torch.empty(B, V, device="cuda").exponential_(1.0, generator=torch.Generator(device="cuda").manual_seed(draw))
+        want = torch.gather(order, -1, torch.argmax(kept / q, dim=-1, keepdim=True)).view(-1)
+        sampler(x, temperature, p, torch.Generator(device="cuda").manual_seed(draw), tok)
+        torch.cuda.synchronize()
+        sampler.check()
+        assert tok.tolist() == want.tolist(), p
+    # what softmax(logits / temperature) cannot express is refused, as it was by torch
+    for bad in (x.new_full((), 3e38), x.new_full((), float("-inf"))):
+        y = torch.full_like(x, float(bad))
+        sampler(y, min(temperature, 0.5), 0.9, gen, tok)
+        torch.cuda.synchronize()
+        with pytest.raises(RuntimeError, match="inf or nan"):
+            sampler.check()
+
+
 def test_generator_with_and_without_the_lm_head_kernel_agree():
     args = decoder.ModelArgs(dim=256, n_layers=2, n_heads=2, n_kv_heads=1, vocab_size=512, ffn_dim=512)
     model = _build(args, seed=3)
