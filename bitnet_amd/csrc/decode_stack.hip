@@ -11,7 +11,10 @@
 // such a hand-over measures 1.4 us, readers' barrier included.  30 layers at 512 positions, us:
 //   sequences            1     2     3     4     8
 //   launches           755   875  1000  1070  1060
-//   this kernel        511   626   680   705   772
+//   this kernel        513   630   680   705   746
+// What is left of a phase (of a layer's 17 us at one sequence the five take 3.1, 5.0, 2.4, 3.7 and 3.4): 1.5 to 1.9 us from the
+// arrival of a task's inputs to its outputs (the exchange of the sums of squares 0.2, of the maxima 0.4 to 0.5, products
+// 0.5 to 0.9, the epilogue 0.3), the hand-over, and the last workgroup being late; the weights are not waited for.
 // Up to two tokens every workgroup of a product normalises and quantizes the rows by itself, between their
 // arrival and its matrix instructions.  That part grows with the tokens (three: 1120 us).  Beyond two, one
 // task per token does it for all and publishes int8 rows, which are the matrix instructions' operand as they
@@ -67,8 +70,13 @@ namespace {
 constexpr int kStWaves = 4;
 constexpr int kStLanes = kStWaves * 64;   // of the computing waves
 constexpr int kStThreads = kStLanes + 64;  // and the wave that fetches
-constexpr int kStUpwD = 10;       // 64-wide k-steps per wave of a product over the model width: up to 2560
-constexpr int kStUpwF = 27;       // ... over the feed-forward width: up to 6912
+// 64-wide k-steps per wave of a product over the model width (up to 2560) and over the feed-forward width (up to 6912).
+// The registers set them: a w13 task keeps four row blocks of 10 steps as expanded operands, 160 of the 256 that
+// one computing wave per SIMD has next to the wave that fetches, and a w2 task one block of 27 and its slice of the input.
+// Narrower models take the same steps, multiplied with zeros: the exchanges and hand-overs, which are what a phase
+// costs, do not get shorter with them.  Wider ones and more than kStMaxTokens take the kernels per layer.
+constexpr int kStUpwD = 10;
+constexpr int kStUpwF = 27;
 constexpr int kStDirect = 2;      // tokens up to which every product task quantizes its input (see above)
 constexpr int kStMaxTokens = 8;
 constexpr int kStMaxG = 8;        // query heads per kv head

@@ -7,11 +7,11 @@
 // twenty passes over 128256 values (330 us a step at one sequence).  bf16 logits take only a few thousand
 // different values, though, and tokens of one value are sorted by index, so the sorted distribution is
 // known from a histogram alone: rank r belongs to the value whose cumulative counts enclose it, and only
-// the winner's rank is turned into a token.  Three launches, 30 us together, bound by chains of LDS and
+// the winner's rank is turned into a token.  Three launches, 32 us together, bound by chains of LDS and
 // memory latencies (one row of 128256 logits; at four rows the same):
 //   1. histograms of 16 pieces of the vocabulary, 5 us
 //   2. their sum, its masses and the nucleus's end; the race over one piece of the ranks per workgroup, 18 us
-//   3. the winner: value and place among the tokens of that value -> piece -> token, 7 us
+//   3. the winner: value and place among the tokens of that value -> piece -> token, 9 us
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>

@@ -2,7 +2,7 @@
 (via the ctypes host mirror) and is compared with the CPU oracle.
 
 Bars: int32 accumulators bit-exact; bf16 outputs bit-exact against the
-oracle's IEEE fp32 divide + multiply + RNE cast (the north star allows
+oracle's IEEE fp32 divide + multiply + RNE cast (the contract allows
 1 bf16 ulp / rel 1e-3; the tests assert the tighter bound and would report
 the ulp distance if it ever failed); quantizer outputs bit-exact.
 """
