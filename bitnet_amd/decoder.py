@@ -672,7 +672,7 @@ class Generator:
         self._logits_graph: Optional[torch.cuda.CUDAGraph] = None  # the step up to its logits
         self.stack: Optional[DecodeStack] = None  # of the captured steps, where the model is one it takes
         self.use_graph = use_graph
-        # final norm + bf16 LM head + greedy token as two launches of the library
+        # final norm + bf16 LM head + greedy token as three launches of the library
         self.lm_head = (self.fused and fused_head and model.output.weight.dtype == torch.bfloat16 and a.dim % 64 == 0
                         and model.output.bias is None)
         self.lm_ws = LmHeadWorkspace(batch, a.vocab_size, a.dim, dev) if self.lm_head else None
@@ -832,7 +832,7 @@ class Generator:
         sequence: int64 [B], ragged prompts) and generates up to `steps` further
         tokens greedily.  With eos_id the loop ends after the first step in which
         any sequence produced that token, as the reference's loop does
-        (gpu/generate.py:283-284; one device-to-host copy per step).  Returns
+        (gpu/generate.py:283-284; the host waits for every step).  Returns
         [steps taken, B]."""
         if steps > self.history.shape[0]:
             raise ValueError("more steps than the generator was sized for")
