@@ -226,7 +226,7 @@ def cpu_baseline(shapes, M, budget_s=12.0):
             ts.append(time.perf_counter() - t0)
         mean = sum(ts) / len(ts)
         nx1[sh.name] = {"mean_us": round(mean * 1e6, 1), "min_us": round(min(ts) * 1e6, 1), "iterations": len(ts),
-                        "TOPS": round(2.0 * Mp * sh.N * sh.K / mean / 1e12, 3)}
+                        "TOPS": float(f"{2.0 * Mp * sh.N * sh.K / mean / 1e12:.4g}")}
 
     def one_pass(nt):  # one pass over the n_layers sample
         for layer in range(n_layers):
@@ -245,7 +245,7 @@ def cpu_baseline(shapes, M, budget_s=12.0):
                 break
         out[tag] = (layer_bytes * n / el / 1e9, n, el)
     return {
-        "value": round(out["threads"][0], 3),
+        "value": float(f"{out['threads'][0]:.6g}"),  # (digits, not decimals: tiny shapes on a loaded host are not 0)
         "unit": "GB/s",
         "cores": threads,
         "kind": "port",
