@@ -1164,6 +1164,8 @@ void gemm_i2_prefill_mix_kernel(
     }
 }
 
+#include "gemm_ring.h"
+
 // ---------------------------------------------------------------------------
 // Per-token absmax quantizer: one workgroup per token row
 // ---------------------------------------------------------------------------
@@ -2329,6 +2331,19 @@ constexpr int kPrefillRound64 = 768, kPrefillRound128 = 1024;
 // rounds for which the launch with two tile sizes is taken (about 1.4 per CU; figures at launch_prefill)
 constexpr int kPrefillMixCus = 256;
 constexpr int kPrefillMixMaxQuarters = 360;
+// the GEMM kernel with both operands in LDS (gemm_ring.h; its instances at BITLINEAR_RING_A): the smallest of its tiles of
+// which there is at most one per CU, because a tile's time hardly depends on how many there are until then.  Over 110
+// random shapes of 17 to 2048 tokens against the kernels below: 32 x 64 tiles 1.19 times as fast (101 x 3840 x 2560
+// 6.6 -> 5.6 us, 32 x 2560 x 6912 11.0 -> 7.8), 64 x 128 1.18 (512 x 3840 x 2560 9.4 -> 8.4, 512 x 2560 x 6912
+// 17.4 -> 13.1), 64 x 256 1.19 (513 x 4800 x 3200 21.9 -> 14.4), 128 x 256 1.15 (512 x 13824 x 2560 23.2 -> 20.6)
+constexpr int kRingCus = 256;
+// ... of the 64 x 256 tiles two fit a CU: up to a third more of them (384 x 13824 x 2560, 324 tiles, 23.6 -> 19.7 us; as 162
+// tiles of 128 x 256 20.4; 512 x 13824 x 2560, 432 tiles, 24.6 against 22.6)
+constexpr int kRingMost64x256 = 340;
+// ... from this K on, below which requesting the stages behind the end costs more than the ring gains (380 x 976 x 256
+// 3.5 against 4.1 us, 51 x 3728 x 512 3.85 against 4.0); the 64 x 256 tiles later (76 x 17632 x 640 5.5 against 6.2,
+// 247 x 8384 x 1024 level), and not on very long rows, where two k-groups are ahead (705 x 3200 x 10240 32.4 against 33.9)
+constexpr int kRingMinK = 640, kRingMinK64x256 = 1024, kRingMaxK64x256 = 8192;
 }  // namespace dispatch
 using namespace dispatch;
 
@@ -2882,6 +2897,35 @@ int launch_solo_tok(const uint16_t* x, const int8_t* packed, uint16_t* out, int3
     return launch_status();
 }
 
+// The instances of the kernel in gemm_ring.h: 32 x 64 tiles whose K eight waves split, 64 x 128 tiles split by four, 64 x 256
+// (two workgroups per CU) and 128 x 256 tiles
+#define BITLINEAR_RING_A 1, 2, 1, 1, 8, 512, 6, 0
+#define BITLINEAR_RING_B 2, 2, 1, 2, 4, 256, 6, 4
+#define BITLINEAR_RING_C 2, 2, 1, 4, 1, 128, 4, 4
+#define BITLINEAR_RING_D 2, 2, 2, 4, 1, 128, 6, 4
+constexpr int kRingRows[5] = {0, 32, 64, 64, 128}, kRingCols[5] = {0, 64, 128, 256, 256};
+long long ring_tiles(int M, int N, int ring) {
+    return (long long)((M + kRingRows[ring] - 1) / kRingRows[ring]) * ((N + kRingCols[ring] - 1) / kRingCols[ring]);
+}
+// whole chunks of 128 k, and output rows that can be written in 16-byte pieces
+bool ring_aligned(const uint16_t* out, const int32_t* acc_out, const uint16_t* residual, int K) {
+    return K % 128 == 0 && ((((uintptr_t)out) | ((uintptr_t)acc_out) | ((uintptr_t)residual)) & 15u) == 0;
+}
+// which instance a product takes; 0: none
+int ring_choice(int M, int N, int K, const ScaleMap& smap, bool aligned) {
+    if (!aligned) return 0;
+    for (int j = 0; j + 1 < smap.nseg; ++j)
+        if (smap.ends[j] % 8) return 0;  // eight outputs share a weight scale
+    if (t_tune.path == 5) return t_tune.prefill_big >= 9 ? t_tune.prefill_big - 8 : 0;
+    if (t_tune.path != 0) return 0;
+    if (K < kRingMinK) return 0;
+    if (ring_tiles(M, N, 1) <= kRingCus) return 1;
+    if ((long long)((M + 31) / 32) * ((N + 127) / 128) <= kRingCus) return 0;
+    if (ring_tiles(M, N, 2) <= kRingCus) return 2;
+    if (ring_tiles(M, N, 3) <= kRingMost64x256) return K >= kRingMinK64x256 && K <= kRingMaxK64x256 ? 3 : 0;
+    if (ring_tiles(M, N, 4) <= kRingCus) return 4;
+    return 0;
+}
 int launch_prefill(const int8_t* act, const int8_t* packed, uint16_t* out, int32_t* acc_out, const uint16_t* s,
                    const uint16_t* ws, const ScaleMap& smap, int M, int N, int K, hipStream_t stream,
                    const uint16_t* residual = nullptr) {
@@ -2904,6 +2948,15 @@ int launch_prefill(const int8_t* act, const int8_t* packed, uint16_t* out, int32
         if (e == hipSuccess)
             e = hipFuncSetAttribute((const void*)gemm_i2_prefill_kernel<2, 2, 2>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     2 * 2 * 64 * kPfRowBytes);
+#define BITLINEAR_RING_LDS(...)                                                                                                   \
+    if (e == hipSuccess)                                                                                                         \
+        e = hipFuncSetAttribute((const void*)gemm_i2_prefill_kernel<__VA_ARGS__>, hipFuncAttributeMaxDynamicSharedMemorySize, \
+                                Ring<__VA_ARGS__>::LDS)
+        BITLINEAR_RING_LDS(BITLINEAR_RING_A);
+        BITLINEAR_RING_LDS(BITLINEAR_RING_B);
+        BITLINEAR_RING_LDS(BITLINEAR_RING_C);
+        BITLINEAR_RING_LDS(BITLINEAR_RING_D);
+#undef BITLINEAR_RING_LDS
         return e;
     });
     if (lds_err != hipSuccess) return BITLINEAR_ERR_LAUNCH;
@@ -2918,7 +2971,7 @@ int launch_prefill(const int8_t* act, const int8_t* packed, uint16_t* out, int32
     const long long wide_tiles = (long long)((N + 255) / 256) * ((M + 63) / 64);
     // (the kernel that brings the activation chunks straight into LDS needs 128-k chunks that divide K and 16-byte
     // aligned output rows)
-    const bool dma_fits = K % 128 == 0 && ((((uintptr_t)out) | ((uintptr_t)acc_out) | ((uintptr_t)residual)) & 15u) == 0;
+    const bool dma_fits = ring_aligned(out, acc_out, residual, K);
     int tile = ((N >= kPrefillWideN && M >= kPrefillWideMinTokens) || narrow_tiles > kPrefillFewTiles) ? 2 : 4;
     // 64 x 256 tiles run three workgroups per CU (768 at a time), 128 x 256 tiles two (512): with a little more than
     // one full round of the former, one round of the latter finishes earlier (13824 x 2560 at M = 1024: 864 tiles,
@@ -2958,6 +3011,24 @@ int launch_prefill(const int8_t* act, const int8_t* packed, uint16_t* out, int32
                           out ? 1 : 0, small_cols, s, out, acc_out, ws, smap, residual);
             return launch_status();
         }
+    }
+    const int ring = ring_choice(M, N, K, smap, dma_fits);
+    if (ring) {
+        const int row_tiles = (M + kRingRows[ring] - 1) / kRingRows[ring], col_tiles = (N + kRingCols[ring] - 1) / kRingCols[ring];
+        const long long tiles = ring_tiles(M, N, ring);
+        if (tiles >= (1ll << 22)) return BITLINEAR_ERR_SHAPE;
+        const dim3 rgrid(8 * (unsigned)((tiles + 7) / 8), 1, 1);
+#define BITLINEAR_LAUNCH_RING(...)                                                                                             \
+    BL_LAUNCH((gemm_i2_prefill_kernel<__VA_ARGS__>), rgrid, dim3(Ring<__VA_ARGS__>::THREADS), (Ring<__VA_ARGS__>::LDS), stream, act, wq, M, \
+              N, K, (int)tiles, out ? 1 : 0, row_tiles, col_tiles, s, out, acc_out, ws, smap, residual)
+        switch (ring) {
+            case 1: BITLINEAR_LAUNCH_RING(BITLINEAR_RING_A); break;
+            case 2: BITLINEAR_LAUNCH_RING(BITLINEAR_RING_B); break;
+            case 3: BITLINEAR_LAUNCH_RING(BITLINEAR_RING_C); break;
+            default: BITLINEAR_LAUNCH_RING(BITLINEAR_RING_D); break;
+        }
+#undef BITLINEAR_LAUNCH_RING
+        return launch_status();
     }
     bool dma = true;
     int dma_mt = 2;  // row tiles of 32 tokens per workgroup of that kernel: 64 x 256, or 32 x 256 / 128 x 256 when forced
@@ -3161,7 +3232,12 @@ int launch_gemv(const int8_t* act, const int8_t* packed, uint16_t* out, int32_t*
                                        : (tiles <= kPrefillFewTiles
                                               ? 4.4 + 0.45 * (K / 256.0) * (tiles32 > 400.0 ? tiles32 / 400.0 : 1.0)
                                               : 4.0 + 0.64 * (K / 256.0) * (tiles > 256.0 ? tiles / 256.0 : 1.0));
-            gemm = gemm_us <= splitk_us;
+            // the 32 x 64 tiles against the split-K kernel by rows, of which its last group may hold few (17 x 2560 x 2560
+            // 4.8 us against 5.3, 32 x 2560 x 2560 5.95 against 5.45, 17 x 3840 x 2560 5.6 against 5.3)
+            if (ring_choice(M, N, K, smap, ring_aligned(out, acc_out, residual, K)) == 1)
+                gemm = 4.0 + 0.148 * (K / 256.0) <= 3.5 + (M / 16.0) * ((double)N * K / 4.0) / 1.45e6;
+            else
+                gemm = gemm_us <= splitk_us;
         }
         if (gemm) return launch_prefill(act, packed, out, acc_out, s, ws, smap, M, N, K, stream, residual);
         return launch_splitk(act, packed, out, acc_out, s, ws, smap, M, N, K, stream, residual);
@@ -3457,7 +3533,7 @@ int bitlinear_set_tuning(int kernel, int a, int b, int c) {
         return set_status(BITLINEAR_OK);
     }
     if (kernel == 5) {
-        if (a < 0 || a > 8 || b < 0 || b > 64 || (c != 0 && c != 1 && c != 2 && c != 4)) return set_status(BITLINEAR_ERR_ARG);
+        if (a < 0 || a > 12 || b < 0 || b > 64 || (c != 0 && c != 1 && c != 2 && c != 4)) return set_status(BITLINEAR_ERR_ARG);
         g.path = 5;
         g.prefill_big = a;
         g.prefill_band = b;

@@ -1,0 +1,352 @@
+// Prefill GEMM whose operands both travel through LDS (included by bitlinear_hip.hip): int8 activation rows and packed
+// weight words come by direct-to-LDS loads into a ring of S stages of CK k each.
+//
+// For outputs of about one tile per CU.  A tile is then alone on its CU, and what the other kernels leave to the next
+// workgroup to hide is in the open: their loops request a chunk or two ahead and stop at every wait (512 x 3840 x 2560,
+// 240 tiles of 64 x 128: 9.4 us, of which the matrix instructions are 2.2).  Measured here, on a lone tile (cycles of
+// one CU at 2.4 GHz):
+//  * loads bring 54 to 60 bytes a cycle into a CU whatever they are, so a tile's bytes are worth as much attention as its
+//    multiplications (64 x 128: 96 bytes per k, 1.9 us at K = 2560).  Two thirds of LDS is ring, and the loads of S - 1
+//    stages are on their way before the first is waited for.
+//  * a wave that issues a load waits while the path is taken by others, and does not multiply meanwhile.  So LW further
+//    waves do nothing but load (512 x 3840 x 2560: 9.2 -> 8.6 us); the 32 x 64 tile's eight computing waves issue their
+//    few loads between the MFMAs instead (5.6 against 6.2 us).
+//  * an MFMA hides about four vector instructions of its SIMD and every further one takes 2.5 to 4 cycles, two waves or
+//    one, so a wave's tile is 64 x 64 where it can be (expanding a word is eight instructions, here for two MFMAs).
+//  * LDS reads run at 220 bytes a cycle without conflicts (rows swizzled so that 16 rows at one piece fall on 16
+//    different slots of the 256 bytes that the banks span), writes at 76: with KG groups of waves that split the k-steps
+//    of a stage, sums go through LDS once, and with KG = 1 not at all (512 x 13824 x 2560: 21.2 -> 20.2 us).
+// One barrier per stage: behind it the next stage is complete for every wave, so the first operands of a stage are read
+// while the one in front is still being multiplied, and the stage before that is free for the loaders.  Requests behind
+// the end of K fetch nothing and bring zeros, so every wait counts the same number of requests.
+// Codes are expanded to bytes that read 64 w, as in gemm_i2_prefill_dma_kernel, which also defines the interleaved column
+// tiles of a wave.  K % 128 == 0.
+#ifndef BITNET_AMD_GEMM_RING_H
+#define BITNET_AMD_GEMM_RING_H
+
+// A wave's tile is 32 MT x 32 NT; WM x WN waves side by side, KG of them one behind the other in k; LW loading waves (0:
+// the computing ones load)
+template <int MT, int NT, int WM, int WN, int KG, int CK, int S, int LW>
+struct Ring {
+    static constexpr int WAVES = WM * WN * KG;  // that compute
+    static constexpr int LWAVES = LW ? LW : WAVES;  // that load
+    static constexpr int TM = 32 * MT * WM, TN = 32 * NT * WN;
+    static constexpr int KSTEPS = CK / 32;       // 32-k MFMA steps per stage
+    static constexpr int KPW = KSTEPS / KG;      // ... of which a wave takes this many
+    static constexpr int PPR = CK / 16;          // 16-byte pieces per activation row and stage
+    static constexpr int RPI = 64 / PPR;         // activation rows one load instruction of a wave covers
+    static constexpr int SWZ_SHIFT = PPR == 8 ? 1 : 0, SWZ = PPR == 8 ? 7 : 15;
+    static constexpr int A_BYTES = TM * CK, W_BYTES = TN * CK / 4, STAGE = A_BYTES + W_BYTES;
+    static constexpr int AR = A_BYTES / 1024 / LWAVES, WR = W_BYTES / 1024 / LWAVES, LOADS = AR + WR;
+    static constexpr int OUT_ROW = TN * 4 + 16;  // bytes of a row of sums: 16 rows at one column fall on 16 different 16-byte slots
+    static constexpr int RED = KG > 1 ? KG * TM * OUT_ROW : 0;
+    static constexpr int LDS = S * STAGE > RED ? S * STAGE : RED;
+    static constexpr int THREADS = 64 * (WAVES + LW);
+    static constexpr int WGS = 2 * (LDS + TM * 8 + 64) <= 160 * 1024 ? 2 : 1;  // workgroups per CU
+    static constexpr int PIECES = TM * TN / 8 <= 64 * WAVES ? 1 : TM * TN / 8 / (64 * WAVES);  // 8 outputs each, per thread
+    static_assert(AR * LWAVES * 1024 == A_BYTES && WR * LWAVES * 1024 == W_BYTES, "whole load instructions per wave");
+    static_assert(KPW >= 2 && KPW % 2 == 0 && KPW * KG == KSTEPS, "operand registers alternate");
+    static_assert(S >= 4 && (S - 1) * LOADS <= 63, "loads in flight are counted in six bits");
+    static_assert(LDS + TM * 8 + 64 <= 160 * 1024, "LDS of a CU");
+};
+constexpr int kRingBand = 4;
+// n / d for 0 <= n < 2^22, d >= 1, of wave-uniform values
+__device__ __forceinline__ int ring_div(int n, int d) {
+    int q = (int)((float)n * __builtin_amdgcn_rcpf((float)d));
+    q += (n - q * d >= d ? 1 : 0) - (n - q * d < 0 ? 1 : 0);
+    return __builtin_amdgcn_readfirstlane(q);
+}
+constexpr int kRingBeyond = 0x7ffffff0;  // an offset behind every descriptor: nothing is fetched, zeros arrive
+
+template <int MT, int NT, int WM, int WN, int KG, int CK, int S, int LW>
+__global__ __launch_bounds__(64 * (WM * WN * KG + LW)) __attribute__((amdgpu_waves_per_eu((WM * WN * KG + LW) * Ring<MT, NT, WM, WN, KG, CK, S, LW>::WGS / 4)))
+void gemm_i2_prefill_kernel(
+    const int8_t* __restrict__ act, const uint32_t* __restrict__ wq, int M, int N, int K, int ntiles, int flags,
+    int row_tiles, int col_tiles, const uint16_t* __restrict__ s, uint16_t* __restrict__ out, int32_t* __restrict__ acc_out,
+    const uint16_t* __restrict__ ws, ScaleMap smap, const uint16_t* __restrict__ residual) {
+    typedef Ring<MT, NT, WM, WN, KG, CK, S, LW> R;
+    constexpr int QR = 8 / NT;
+    extern __shared__ __attribute__((aligned(1024))) int8_t lds_x[];
+
+    // Workgroup -> tile.  The tiles, band of kRingBand row tiles by band, column by column within a band, are cut into
+    // eight runs of equal length, one per XCD (workgroups are handed to the XCDs round-robin): the workgroups of an XCD
+    // share a few row and a few column tiles in its L2, and no XCD has more than one tile more than another.
+    const int xcd = blockIdx.x & 7;
+    const int i = (int)(((long long)xcd * ntiles) >> 3) + (int)(blockIdx.x >> 3);
+    if (i >= (int)(((long long)(xcd + 1) * ntiles) >> 3)) return;
+    const int band = ring_div(i, kRingBand * col_tiles);
+    const int in_band = i - band * (kRingBand * col_tiles);
+    const int band_rows = row_tiles - band * kRingBand < kRingBand ? row_tiles - band * kRingBand : kRingBand;
+    const int col_tile = ring_div(in_band, band_rows);
+    const int row_tile = band * kRingBand + in_band - col_tile * band_rows;
+    const bool has_out = flags != 0;  // repeats out != nullptr
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int grp = wave / (WM * WN), wm = (wave / WN) % WM, wn = wave % WN;
+    const int nl = lane & 31, kc = lane >> 5;
+    const int m0 = row_tile * R::TM, n_base = col_tile * R::TN;
+    const int nchunks = (K + CK - 1) / CK;
+
+    const int rows_here = (M - m0) < R::TM ? (M - m0) : R::TM;
+    const __amdgpu_buffer_rsrc_t a_rsrc =
+        __builtin_amdgcn_make_buffer_rsrc((void*)(act + (size_t)m0 * K), 0, rows_here * K, 0x00020000);
+    const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)wq, 0, (N >> 2) * K, 0x00020000);
+
+    const int lw = LW ? wave - R::WAVES : wave;  // (negative: a wave that does not load)
+    // activation requests: rows XOR-swizzled in 16-byte pieces (by choice of the piece a lane fetches)
+    int a_voff[R::AR], a_k[R::AR];
+#pragma unroll
+    for (int r = 0; r < R::AR; ++r) {
+        const int row = (r * R::LWAVES + lw) * R::RPI + lane / R::PPR;
+        a_k[r] = ((lane % R::PPR) ^ ((row >> R::SWZ_SHIFT) & R::SWZ)) * 16;
+        a_voff[r] = row * K + a_k[r];
+    }
+    // weight requests: [k-step][row block][128 bytes] in the stage
+    int w_voff[R::WR], w_k[R::WR];
+#pragma unroll
+    for (int r = 0; r < R::WR; ++r) {
+        const int q = (r * R::LWAVES + lw) * 64 + lane;
+        constexpr int per_step = R::TN / 16 * 8;
+        const int ks = q / per_step;
+        int blk = (n_base >> 4) + (q % per_step) / 8;
+        blk = blk < (N >> 4) ? blk : (N >> 4) - 1;
+        w_k[r] = ks * 32;
+        w_voff[r] = blk * K * 4 + ks * 128 + (q & 7) * 16;
+    }
+    // part p of P of a stage's requests
+    auto issue = [&](int c, int st, int p, int P) {
+        const int left = K - c * CK;  // k in front of the end of the rows
+        const int cc = left > 0 ? c : 0;
+        int8_t* to = lds_x + st * R::STAGE;
+#pragma unroll
+        for (int r = 0; r < R::LOADS; ++r) {
+            if (r * P / R::LOADS != p) continue;
+            if (r < R::AR) {
+                load16_to_lds(a_rsrc, to + (r * R::LWAVES + lw) * 1024, a_k[r] < left ? a_voff[r] : kRingBeyond, cc * CK);
+            } else {
+                const int i = r - R::AR;
+                load16_to_lds(w_rsrc, to + R::A_BYTES + (i * R::LWAVES + lw) * 1024, w_k[i] < left ? w_voff[i] : kRingBeyond, cc * (CK * 4));
+            }
+        }
+    };
+    constexpr int kYounger = (S - 3) * R::LOADS;
+    constexpr int kWaitYounger = 0x0f70 | (kYounger & 15) | ((kYounger >> 4) << 14);
+    auto meet = [&] {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    if (lw >= 0) {
+#pragma unroll
+        for (int c = 0; c < S - 1; ++c) issue(c, c, 0, 1);
+    }
+    if (LW && lw >= 0) {
+        __builtin_amdgcn_s_waitcnt(kWaitYounger);
+        meet();
+        int st = S - 1;
+        for (int c = 0; c < nchunks; ++c) {
+            issue(c + S - 1, st, 0, 1);
+            st = st + 1 == S ? 0 : st + 1;
+            __builtin_amdgcn_s_waitcnt(kWaitYounger);
+            meet();
+        }
+        __builtin_amdgcn_s_waitcnt(0x0f70);
+        meet();
+        lds_barrier();
+        return;
+    }
+
+    // the scales, for the epilogue: requested behind the first stages, in LDS before the sums are
+    __shared__ float sval[R::TM], rinv[R::TM], wsv[kMaxSeg];
+    uint16_t s_raw = 0, ws_raw = 0;
+    if (has_out) {
+        const int m = m0 + (int)threadIdx.x;
+        if (threadIdx.x < R::TM) s_raw = s[m < M ? m : M - 1];
+        if (threadIdx.x < kMaxSeg) ws_raw = ws[(int)threadIdx.x < smap.nseg ? threadIdx.x : 0];
+    }
+
+    v16i acc[MT][NT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[mt][nt][r] = 0;
+
+    // where the lane's operands are within a stage
+    typedef typename PfxWords<NT>::type wvec_t;
+    int a_rd[R::KPW];
+#pragma unroll
+    for (int j = 0; j < R::KPW; ++j)
+        a_rd[j] = (wm * MT * 32 + nl) * CK + ((((grp * R::KPW + j) * 2 + kc) ^ ((nl >> R::SWZ_SHIFT) & R::SWZ)) * 16);
+    const int w_rd = R::A_BYTES + grp * R::KPW * (R::TN * 8) + (wn * NT * 2 + nl / (2 * QR)) * 128 +
+                     (((nl % (2 * QR)) / QR) * 16 + kc * 8 + NT * (nl % QR)) * 4;
+    auto expand = [&](uint32_t wd) -> v4i {
+        const uint32_t x = wd ^ 0xAAAAAAAAu;
+        v4i r;
+        r.x = (int)((x << 6) & 0xC0C0C0C0u);
+        r.y = (int)((x << 4) & 0xC0C0C0C0u);
+        r.z = (int)((x << 2) & 0xC0C0C0C0u);
+        r.w = (int)(x & 0xC0C0C0C0u);
+        return r;
+    };
+    auto read_a = [&](const int8_t* stage, int j, v4i(&a)[MT]) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) a[mt] = *(const v4i*)(stage + a_rd[j] + mt * 32 * CK);
+    };
+    auto read_w = [&](const int8_t* stage, int j) -> wvec_t { return *(const wvec_t*)(stage + w_rd + j * (R::TN * 8)); };
+    // stages 0 and 1 are there (every wave waits for its own requests, then all meet)
+    if (!LW) __builtin_amdgcn_s_waitcnt(kWaitYounger);
+    meet();
+
+    v4i aop[2][MT], bop[2][NT];
+    wvec_t wraw[2];
+    read_a(lds_x, 0, aop[0]);
+    wraw[0] = read_w(lds_x, 0);
+    wraw[1] = read_w(lds_x, 1);
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) bop[0][nt] = expand(wraw[0][nt]);
+
+    int st = 0;
+    for (int c = 0; c < nchunks; ++c) {
+        const int8_t* here = lds_x + st * R::STAGE;
+        const int st1 = st + 1 == S ? 0 : st + 1;
+        const int8_t* next = lds_x + st1 * R::STAGE;
+        // the stage in front of this one was read in the chunk before, which every wave has left
+        constexpr int SLOTS = MT * NT;
+#pragma unroll
+        for (int j = 0; j < R::KPW; ++j) {
+            const int cur = j & 1, nxt = cur ^ 1;
+#pragma unroll
+            for (int slot = 0; slot < SLOTS; ++slot) {
+                const int mt = slot / NT, nt = slot % NT;
+                acc[mt][nt] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bop[cur][nt], aop[cur][mt], acc[mt][nt], 0, 0, 0);
+                if (slot == 0) {
+                    if (j + 1 < R::KPW) read_a(here, j + 1, aop[nxt]);
+                    else read_a(next, 0, aop[nxt]);
+                    wraw[cur] = j + 2 < R::KPW ? read_w(here, j + 2) : read_w(next, j + 2 - R::KPW);
+                }
+#pragma unroll
+                for (int i = 0; i < NT; ++i)
+                    if ((i * SLOTS / NT + (SLOTS > NT ? 1 : 0)) % SLOTS == slot) bop[nxt][i] = expand(wraw[nxt][i]);
+                if (!LW && slot == SLOTS - 1) issue(c + S - 1, st == 0 ? S - 1 : st - 1, j, R::KPW);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        // the chunk behind the next one has to be there before the next one ends
+        if (!LW) __builtin_amdgcn_s_waitcnt(kWaitYounger);
+        meet();
+        st = st1;
+    }
+
+    // the groups' accumulators: each finishes the register quads q with q % KG == group
+    constexpr int QUADS = MT * 4;
+    // eight consecutive outputs of one token from their sums: the reference's epilogue (the bits of the IEEE divide by
+    // the token's scale from its reciprocal and one correction step, as in gemm_i2_prefill_kernel)
+    auto store8 = [&](int m, int n, const int(&x)[8], float sv, float ri, float w) {
+        const size_t o = (size_t)m * N + n;
+        if (acc_out) {
+            *(v4i*)(acc_out + o) = v4i{x[0], x[1], x[2], x[3]};
+            *(v4i*)(acc_out + o + 4) = v4i{x[4], x[5], x[6], x[7]};
+        }
+        if (!has_out) return;
+        uint32_t ob[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float h[2];
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const float a = (float)x[2 * i + e];
+                const float q0 = a * ri;
+                h[e] = __builtin_fmaf(__builtin_fmaf(-q0, sv, a), ri, q0) * w;
+            }
+            ob[i] = f32x2_to_bf16x2(h[0], h[1]);
+        }
+        if (residual) {  // out = bf16(residual + bf16(result))
+            const uint4 rv = *(const uint4*)(residual + o);
+            const uint32_t r4[4] = {rv.x, rv.y, rv.z, rv.w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                ob[i] = f32x2_to_bf16x2(__uint_as_float(r4[i] << 16) + __uint_as_float(ob[i] << 16),
+                                        __uint_as_float(r4[i] & 0xffff0000u) + __uint_as_float(ob[i] & 0xffff0000u));
+        }
+        *(uint4*)(out + o) = make_uint4(ob[0], ob[1], ob[2], ob[3]);
+    };
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // the requests behind the end write zeros into the ring
+    meet();
+    if (threadIdx.x < R::TM) {
+        sval[threadIdx.x] = bf16_to_f32(s_raw);
+        rinv[threadIdx.x] = 1.0f / bf16_to_f32(s_raw);
+    }
+    if (threadIdx.x < kMaxSeg) wsv[threadIdx.x] = bf16_to_f32(ws_raw);
+    if constexpr (KG == 1) {
+        // every wave holds its sums whole: 4 NT consecutive columns per register quad, stored straight from the registers
+        lds_barrier();
+        const int nw = n_base + wn * NT * 32;
+        const int n_last = (nw + NT * 32 - 1) < N ? (nw + NT * 32 - 1) : N - 1;
+        const int slot_first = scale_slot(smap, nw < N ? nw : N - 1);
+        const bool one_slot = slot_first == scale_slot(smap, n_last);
+        const float w1 = wsv[slot_first];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            const int row = (wm * MT + mt) * 32 + nl, m = m0 + row;
+            const float sv = sval[row], ri = rinv[row];
+#pragma unroll
+            for (int g4 = 0; g4 < 4; ++g4) {
+                const int ridx = g4 * 8 + kc * 4;
+                const int n = nw + 16 * (ridx / (2 * QR)) + 8 * ((ridx % (2 * QR)) / QR) + NT * (ridx % QR);
+                int x[4 * NT];
+#pragma unroll
+                for (int i = 0; i < 4 * NT; ++i) x[i] = acc[mt][i % NT][g4 * 4 + i / NT] >> 6;
+                if (m < M && n < N) store8(m, n, x, sv, ri, one_slot ? w1 : wsv[scale_slot(smap, n)]);
+            }
+        }
+        return;
+    }
+    // The sums go through LDS, which adds the groups' shares and turns a lane's pieces of 32 rows into whole runs of a
+    // row.  (A lane holds token nl; register quad g4 of its NT column tiles is 4 NT consecutive columns.)
+    {
+        int8_t* to = lds_x + (grp * R::TM + wm * MT * 32 + nl) * R::OUT_ROW + wn * NT * 128;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int g4 = 0; g4 < 4; ++g4) {
+                const int ridx = g4 * 8 + kc * 4;
+                const int n = 16 * (ridx / (2 * QR)) + 8 * ((ridx % (2 * QR)) / QR) + NT * (ridx % QR);
+#pragma unroll
+                for (int v = 0; v < NT; ++v) {
+                    v4i t;
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const int i = 4 * v + j;  // column n + i: register i / NT of the quad, column tile i % NT
+                        t[j] = acc[mt][i % NT][g4 * 4 + i / NT];
+                    }
+                    *(v4i*)(to + mt * 32 * R::OUT_ROW + (n + 4 * v) * 4) = t;
+                }
+            }
+    }
+    static_assert((R::PIECES == 1 || R::PIECES * R::WAVES * 64 * 8 == R::TM * R::TN), "pieces per thread");
+    constexpr int ROWS = R::WAVES * 64 / (R::TN / 8);  // rows of the tile that the threads' piece number p covers
+    const int pr = threadIdx.x / (R::TN / 8), pc = threadIdx.x % (R::TN / 8) * 8, n = n_base + pc;
+    const int slot = scale_slot(smap, n);
+    lds_barrier();
+    const float w = wsv[slot];
+#pragma unroll
+    for (int p = 0; p < R::PIECES; ++p) {
+        const int row = p * ROWS + pr, m = m0 + row;
+        if (row >= R::TM || m >= M || n >= N) continue;  // N % 16 == 0: the eight columns are in or out together
+        const int8_t* from = lds_x + row * R::OUT_ROW + pc * 4;
+        v4i lo = *(const v4i*)from, hi = *(const v4i*)(from + 16);
+#pragma unroll
+        for (int g = 1; g < KG; ++g) {
+            lo += *(const v4i*)(from + g * R::TM * R::OUT_ROW);
+            hi += *(const v4i*)(from + g * R::TM * R::OUT_ROW + 16);
+        }
+        lo >>= 6, hi >>= 6;  // exact: the accumulators are 64 * sum(w * a)
+        const int x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+        store8(m, n, x, sval[row], rinv[row], w);
+    }
+}
+
+#endif

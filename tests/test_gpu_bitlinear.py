@@ -544,6 +544,49 @@ def test_fused_forward_launch_shapes_and_null_workspaces():
         lib.bitlinear_set_tuning(0, 0, 0, 0)
 
 
+@pytest.mark.parametrize("tile", [9, 10, 11, 12])
+@pytest.mark.parametrize("m,n,k", [(17, 16, 128), (31, 48, 256), (32, 80, 384), (33, 272, 512), (64, 256, 640), (65, 528, 896),
+                                   (129, 1040, 1408), (257, 3840, 2560), (40, 2560, 6912)])
+def test_prefill_gemm_with_both_operands_through_lds(m, n, k, tile):
+    """gemm_ring.h's four instances (32 x 64, 64 x 128, 64 x 256, 128 x 256 tiles) forced at their edges: fewer stages
+    than the ring holds, a last stage that K fills in part, ragged M and N down to one row block, more tiles than CUs --
+    accumulators equal to the oracle's, bf16 outputs with the reference's slots, with segments at multiples of 8 (one
+    scale per eight outputs) and with a residual equal bit for bit; other segments go to another kernel."""
+    lib = _lib.load_library()
+    w, a = _rand_case(n, k, m, seed=7 * m + n + k)
+    s_bits = o.f32_to_bf16_bits(np.linspace(3.0, 90.0, m).astype(np.float32))
+    ws_bits = o.f32_to_bf16_bits(np.array([0.0161, 0.0247, 0.0093, 0.0], dtype=np.float32))
+    acc_want, want = o.bitlinear_int8xint2(a, w, s_bits, ws_bits)
+    ends = [n] if n < 64 else [24, n // 16 * 8, n]
+    odd = [n] if n < 64 else [20, n // 2 + 4, n]
+    want_seg, want_odd = (o.bitlinear_int8xint2_seg(a, w, s_bits, ws_bits, e)[1] for e in (ends, odd))
+    xb = o.f32_to_bf16_bits(np.random.default_rng(m).standard_normal((m, k)).astype(np.float32))
+    g_bits = o.f32_to_bf16_bits(np.linspace(0.5, 1.5, k).astype(np.float32))
+    res_bits = o.f32_to_bf16_bits(np.random.default_rng(n).standard_normal((m, n)).astype(np.float32))
+    want_res = o.norm_bitlinear(xb, g_bits, 1e-5, w, ws_bits, residual_bits=res_bits)
+    ad, pk, sd, wsd = dev_i8(a), _packed_dev(w), dev_bf16(s_bits), dev_bf16(ws_bits)
+    x, gd, rd, out_res = dev_bf16(xb), dev_bf16(g_bits), dev_bf16(res_bits), torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
+    q_ws, s_ws = torch.empty(m, k, dtype=torch.int8, device="cuda"), torch.empty(m, dtype=torch.bfloat16, device="cuda")
+    st = torch.cuda.current_stream().cuda_stream
+    try:
+        assert lib.bitlinear_set_tuning(5, tile, 0, 0) == 0
+        assert _lib.plan_name(0, m, n, k).count(",") >= 7 + 2  # eight template arguments, a grid of three
+        acc = bitlinear.bitnet_int8xint2_acc(ad, pk)
+        out = bitlinear.bitnet_int8xint2_linear(ad, pk, sd, wsd)
+        out_seg = bitlinear.bitnet_int8xint2_linear_seg(ad, pk, sd, wsd, ends)
+        out_odd = bitlinear.bitnet_int8xint2_linear_seg(ad, pk, sd, wsd, odd)
+        assert lib.bitlinear_norm_forward_bf16(x.data_ptr(), gd.data_ptr(), 1e-5, 0, pk.data_ptr(), wsd.data_ptr(), rd.data_ptr(),
+                                               out_res.data_ptr(), q_ws.data_ptr(), s_ws.data_ptr(), m, n, k, 0, st) == 0
+        torch.cuda.synchronize()
+    finally:
+        lib.bitlinear_set_tuning(0, 0, 0, 0)
+    assert np.array_equal(acc.cpu().numpy(), acc_want)
+    _assert_bits_equal(host_bits(out), want, "scaled output")
+    _assert_bits_equal(host_bits(out_seg), want_seg, "segments at multiples of 8")
+    _assert_bits_equal(host_bits(out_odd), want_odd, "segments elsewhere")
+    _assert_bits_equal(host_bits(out_res), want_res, "with residual")
+
+
 @pytest.mark.parametrize("m,n,k", [(17, 48, 128), (33, 16, 256), (64, 272, 384), (65, 1040, 640), (100, 2560, 768), (128, 2560, 2560),
                                    (129, 3840, 2560), (300, 1040, 3200), (512, 2560, 6912), (1000, 13824, 2560)])
 def test_prefill_gemm_through_the_direct_to_lds_kernel(m, n, k):
