@@ -11,10 +11,11 @@
 // such a hand-over measures 1.4 us, readers' barrier included.  30 layers at 512 positions, us:
 //   sequences            1     2     3     4     8
 //   launches           755   875  1000  1070  1060
-//   this kernel        513   630   680   705   746
-// What is left of a phase (of a layer's 17 us at one sequence the five take 3.1, 5.0, 2.4, 3.7 and 3.4): 1.5 to 1.9 us from the
-// arrival of a task's inputs to its outputs (the exchange of the sums of squares 0.2, of the maxima 0.4 to 0.5, products
-// 0.5 to 0.9, the epilogue 0.3), the hand-over, and the last workgroup being late; the weights are not waited for.
+//   this kernel        497   597   675   698   740
+// What is left of a phase (of a layer's 16.5 us at one sequence the five take about 3, 5, 2.2, 3.5 and 3.2): 1.3 to 1.7 us from the
+// arrival of a task's inputs to its outputs (one exchange between the waves, products 0.5 to 0.9, the epilogue 0.3), the hand-over,
+// and the last workgroup being late; the weights are not waited for.  Polls are as dense as pays: two in flight cost 7 %, a pause
+// of 0.2 us behind each 1 %; outputs stored as 4 or 16 bytes a lane instead of two 1 %.
 // Up to two tokens every workgroup of a product normalises and quantizes the rows by itself, between their
 // arrival and its matrix instructions.  That part grows with the tokens (three: 1120 us).  Beyond two, one
 // task per token does it for all and publishes int8 rows, which are the matrix instructions' operand as they
@@ -264,14 +265,19 @@ __device__ __forceinline__ uint32_t norm2(uint32_t d, uint32_t w, float rstd) {
     return f32x2_to_bf16x2(__uint_as_float(d << 16) * rstd * __uint_as_float(w << 16),
                            __uint_as_float(d & 0xffff0000u) * rstd * __uint_as_float(w & 0xffff0000u));
 }
+// the larger of `top` and the magnitudes of a pair's products with its weights
+__device__ __forceinline__ float product_max2(uint32_t d, uint32_t w, float top) {
+    return fmaxf(fmaxf(fabsf(__uint_as_float(d << 16) * __uint_as_float(w << 16)),
+                       fabsf(__uint_as_float(d & 0xffff0000u) * __uint_as_float(w & 0xffff0000u))), top);
+}
 __device__ __forceinline__ uint32_t quant2(uint32_t d, float s) {  // two bytes
     return __builtin_amdgcn_perm(quant_low_byte<0>(d & 0xffff0000u, s), quant_low_byte<0>(d << 16, s), 0x0c0c0400u);
 }
 
-// A quantized row's scale (bf16 bits) and the sums of its four waves' slices, 30 bits each: a set top bit is "not
-// written", kComplete "the whole slice is in memory, also where it looks unset"
+// A quantized row's scale (bf16 bits) and a word for each of its four waves' slices: a set top bit is "not written",
+// kComplete "the whole slice is in memory, also where it looks unset"
 struct RowRecord {
-    unsigned sum[4];
+    unsigned slice[4];
     unsigned scale, pad[3];
 };
 static_assert(sizeof(RowRecord) == 32 && kStWaves == 4, "one 16-byte and one 4-byte load");
@@ -288,7 +294,8 @@ struct Shared {
     float part_m[kDfMaxWaves][kStMaxG], part_l[kDfMaxWaves][kStMaxG];
     __attribute__((aligned(16))) uint16_t qb[kStMaxG][kHeadDim], knew[kHeadDim], vnew[kHeadDim];
     // exchanges between the computing waves: values with the number of the exchange
-    __attribute__((aligned(16))) v4i sumsq[TQ][kStWaves];
+    // (the first in two buffers: a wave may be a task ahead of one that has not looked yet, not two)
+    __attribute__((aligned(16))) v4i sumsq[2][TQ][kStWaves];
     __attribute__((aligned(16))) v2i amax[TQ][kStWaves];
     __attribute__((aligned(16))) int met[kStWaves];
     // between them and the wave that fetches: counts of tasks
@@ -322,6 +329,7 @@ struct Got {
     v4i e[4 * kStUpwD];     // the weights as MFMA operands: [row block][k-step], or the 27 steps of one block
     Values<kStUpwF> f[Shared<MT>::TQ];  // (the first members serve the shorter slices)
     uint4 g[kStMaxVec];     // norm weights of this lane's values
+    float wild;             // infinity if one of them is 2^20 or more or not a number, otherwise 0
     uint16_t res;
 };
 
@@ -337,6 +345,7 @@ struct Stack {
     int tid, lane, wave;
     int exchange;  // exchanges so far: the same in all computing waves
     int turn;      // which part of `red`
+    int side;      // ... of `sumsq`
 
     // Makes the compiler compute what follows from the thread's place and the arguments anew from here on: kept
     // over the whole loop of tasks, the addresses of all phases together do not fit the registers.
@@ -495,6 +504,17 @@ struct Stack {
             got.g[S::kFull].y = t.y;
         }
     }
+    // (behind the loads' way to memory, in front of the wait for the activations)
+    template <int UPW>
+    __device__ __forceinline__ void look_at_weights(Got<MT>& got) const {
+        typedef Slice<UPW> S;
+        uint32_t most = 0;
+#pragma unroll
+        for (int i = 0; i < S::kFull; ++i) most = absmax_bits8(got.g[i], most);
+        if (S::T) most = absmax_bits8(make_uint4(got.g[S::kFull].x, S::T == 4 ? got.g[S::kFull].y : 0u, 0u, 0u), most);
+        got.wild = most >= 0x4980u ? INFINITY : 0.0f;  // 2^20
+        asm volatile("" : "+v"(got.wild));
+    }
     // byte offsets of this lane's values in a row of row_bytes, kBeyond past its end
     template <int UPW>
     __device__ __forceinline__ void slice_offsets(int row_bytes, int (&off)[Slice<UPW>::kVec]) const {
@@ -524,11 +544,13 @@ struct Stack {
             for (int j = 0; j < UPW; ++j) {
                 // (past the end of K: whatever follows, times activations that are zero)
                 const uint32_t w = *(const uint32_t*)(words + (i >> 1) * stride2 + (i & 1) * K * 4 + j * 256);
+                // bytes that read 64 times the weight (two-bit fields at the top, less the codes' 2): sums need no correction
                 v4i& e = got.e[i * kStUpwD + j];
-                e.x = (int)(w & 0x03030303u);
-                e.y = (int)((w >> 2) & 0x03030303u);
-                e.z = (int)((w >> 4) & 0x03030303u);
-                e.w = (int)((w >> 6) & 0x03030303u);
+                const uint32_t c = w ^ 0xaaaaaaaau;
+                e.x = (int)(c << 6 & 0xc0c0c0c0u);
+                e.y = (int)(c << 4 & 0xc0c0c0c0u);
+                e.z = (int)(c << 2 & 0xc0c0c0c0u);
+                e.w = (int)(c & 0xc0c0c0c0u);
             }
         // now, not where they are used: the compiler would put this work behind the wait, next to the products
 #pragma unroll
@@ -576,24 +598,42 @@ struct Stack {
         }
     }
 
-    // norm and quantizer of the wave's slices: the scales, the slices' sums, the bytes by put8 (8 of them, a 512-value
-    // piece's) and put_rest (S::T of them).  Whether there is a NaN in one of the rows.
+    // Norm and quantizer of the wave's slices: the scales, and the bytes by put8 (8 of them, a 512-value piece's) and
+    // put_rest (S::T of them).  Whether there is a NaN in one of the rows.
+    // The waves meet once for both of a row's reductions.  The quantizer needs the largest of the normalised values
+    // bf16((h r) g), and r the sum of squares; but each of those is |h g| r within two roundings, so the largest lies
+    // between max |h g| r (1 - 2^-21) and the same with a plus, and where both ends round to the same bf16 that is it
+    // (all but one row in some 4000, and rows of very small, very large or missing numbers, for which the maximum is
+    // exchanged as well).  Products of bf16 are exact in fp32; `wild`: a weight of 2^20 or more, beyond which what
+    // underflows in h r could matter.  30 layers 513 -> 497 us at one sequence, 630 -> 597 at two.
     template <int UPW, class Put8, class PutRest>
-    __device__ __forceinline__ bool quantize(const Task& tk, Got<MT>& got, float (&s)[TQ], int (&sum)[TQ], Put8 put8, PutRest put_rest) {
+    __device__ __forceinline__ bool quantize(const Task& tk, Got<MT>& got, float (&s)[TQ], Put8 put8, PutRest put_rest) {
         typedef Slice<UPW> S;
+        side ^= 1;
 #pragma unroll
         for (int t = 0; t < TQ; ++t) {
             const Values<kStUpwF>& v = got.f[t];
             double sq = 0.0;  // lanes without a value hold zeros
+            float top = got.wild;
 #pragma unroll
-            for (int i = 0; i < S::kFull; ++i) sq += sumsq8(v.full[i]);
+            for (int i = 0; i < S::kFull; ++i) {
+                sq += sumsq8(v.full[i]);
+                top = product_max2(v.full[i].x, got.g[i].x, product_max2(v.full[i].y, got.g[i].y, top));
+                top = product_max2(v.full[i].z, got.g[i].z, product_max2(v.full[i].w, got.g[i].w, top));
+            }
 #pragma unroll
-            for (int i = 0; i < S::T / 2; ++i) sq += sumsq2(v.rest[i]);
+            for (int i = 0; i < S::T / 2; ++i) {
+                sq += sumsq2(v.rest[i]);
+                top = product_max2(v.rest[i], i == 0 ? got.g[S::kFull].x : got.g[S::kFull].y, top);
+            }
             sq = wave_reduce_last(sq, [](double x, double y) { return x + y; });
+            const int high = wave_reduce_last(__float_as_int(top), [](int x, int y) { return max(x, y); });
             const v2i bits = __builtin_bit_cast(v2i, sq);
-            if (lane == 63) lds_put(sh.sumsq[t][wave], v4i{bits.x, bits.y, exchange + 1, 0});
+            if (lane == 63) lds_put(sh.sumsq[side][t][wave], v4i{bits.x, bits.y, exchange + 1, high});
         }
         ++exchange;
+        uint32_t am[TQ];
+        bool known = true;
 #pragma unroll
         for (int t = 0; t < TQ; ++t) {
             Values<kStUpwF>& v = got.f[t];
@@ -601,27 +641,54 @@ struct Stack {
             for (;;) {
                 asm volatile("" ::: "memory");
 #pragma unroll
-                for (int k = 0; k < kStWaves; ++k) x[k] = lds_look(sh.sumsq[t][k]);
+                for (int k = 0; k < kStWaves; ++k) x[k] = lds_look(sh.sumsq[side][t][k]);
                 if (uniform(min(min(x[0].z, x[1].z), min(x[2].z, x[3].z)) - exchange) >= 0) break;
             }
             double total = 0.0;
 #pragma unroll
             for (int k = 0; k < kStWaves; ++k) total += __builtin_bit_cast(double, v2i{x[k].x, x[k].y});
             const float rstd = reciprocal_sqrt(divide((float)total, (float)tk.K, tk.inv_k) + tk.eps);
-            uint32_t am = 0;
+            const float top = __int_as_float(max(max(x[0].w, x[1].w), max(x[2].w, x[3].w))) * rstd;
+            const uint32_t ends = f32x2_to_bf16x2(__builtin_fmaf(top, -0x1p-21f, top), __builtin_fmaf(top, 0x1p-21f, top));
+            am[t] = ends & 0xffffu;
+            known = known && top >= 0x1p-60f && top <= 0x1p60f && am[t] == ends >> 16;
 #pragma unroll
-            for (int i = 0; i < S::kFull; ++i) {
-                v.full[i] = norm8(v.full[i], got.g[i], rstd);
-                am = absmax_bits8(v.full[i], am);
-            }
+            for (int i = 0; i < S::kFull; ++i) v.full[i] = norm8(v.full[i], got.g[i], rstd);
             if (S::T) {
-                uint4 r = make_uint4(0u, 0u, 0u, 0u);
-                v.rest[0] = r.x = norm2(v.rest[0], got.g[S::kFull].x, rstd);
-                if (S::T == 4) v.rest[1] = r.y = norm2(v.rest[1], got.g[S::kFull].y, rstd);
-                am = absmax_bits8(r, am);
+                v.rest[0] = norm2(v.rest[0], got.g[S::kFull].x, rstd);
+                if (S::T == 4) v.rest[1] = norm2(v.rest[1], got.g[S::kFull].y, rstd);
             }
-            am = wave_reduce_last(am, [](uint32_t x, uint32_t y) { return max(x, y); });
-            if (lane == 63) lds_put(sh.amax[t][wave], v2i{(int)am, exchange + 1});
+        }
+        bool nans = false;
+        if (!uniform(known)) nans = exchange_maxima<UPW>(tk, got, am);
+#pragma unroll
+        for (int t = 0; t < TQ; ++t) {
+            const Values<kStUpwF>& v = got.f[t];
+            // quant_scale<0>
+            s[t] = bf16_to_f32(f32_to_bf16_rne(reciprocal(fmaxf(__uint_as_float(am[t] << 16), 1e-5f)) * 127.0f));
+#pragma unroll
+            for (int i = 0; i < S::kFull; ++i) put8(t, i, quant_vec8<0>(v.full[i], s[t]));
+            if (S::T) {
+                uint32_t r = quant2(v.rest[0], s[t]);
+                if (S::T == 4) r |= quant2(v.rest[1], s[t]) << 16;
+                put_rest(t, r);
+            }
+        }
+        return nans;
+    }
+    // The rows' maxima from the normalised values themselves; whether one of them is a NaN
+    template <int UPW>
+    __device__ __forceinline__ bool exchange_maxima(const Task& tk, Got<MT>& got, uint32_t (&am)[TQ]) {
+        typedef Slice<UPW> S;
+#pragma unroll
+        for (int t = 0; t < TQ; ++t) {
+            const Values<kStUpwF>& v = got.f[t];
+            uint32_t m = 0;
+#pragma unroll
+            for (int i = 0; i < S::kFull; ++i) m = absmax_bits8(v.full[i], m);
+            if (S::T) m = absmax_bits8(make_uint4(v.rest[0], S::T == 4 ? v.rest[1] : 0u, 0u, 0u), m);
+            m = wave_reduce_last(m, [](uint32_t x, uint32_t y) { return max(x, y); });
+            if (lane == 63) lds_put(sh.amax[t][wave], v2i{(int)m, exchange + 1});
         }
         ++exchange;
         bool nans = false;
@@ -635,8 +702,8 @@ struct Stack {
                 x[1] = lds_look(*(const v4i*)&sh.amax[t][2]);
                 if (uniform(min(min(x[0].y, x[0].w), min(x[1].y, x[1].w)) - exchange) >= 0) break;
             }
-            const uint32_t am = (uint32_t)max(max(x[0].x, x[0].z), max(x[1].x, x[1].z));
-            if (uniform((int)am) > 0x7f80) {  // 0 times a NaN: the values past the end of K have to be zeros again
+            am[t] = (uint32_t)max(max(x[0].x, x[0].z), max(x[1].x, x[1].z));
+            if (uniform((int)am[t]) > 0x7f80) {  // 0 times a NaN: the values past the end of K have to be zeros again
                 nans = true;
 #pragma unroll
                 for (int i = 0; i < S::kFull; ++i)
@@ -646,23 +713,6 @@ struct Stack {
                     if (S::T == 4) v.rest[1] = 0u;
                 }
             }
-            // quant_scale<0>
-            s[t] = bf16_to_f32(f32_to_bf16_rne(reciprocal(fmaxf(__uint_as_float(am << 16), 1e-5f)) * 127.0f));
-            int part = 0;
-#pragma unroll
-            for (int i = 0; i < S::kFull; ++i) {
-                const uint2 qv = quant_vec8<0>(v.full[i], s[t]);
-                put8(t, i, qv);
-                part = __builtin_amdgcn_sdot4((int)qv.x, 0x01010101, __builtin_amdgcn_sdot4((int)qv.y, 0x01010101, part, false), false);
-            }
-            if (S::T) {
-                uint32_t r = quant2(v.rest[0], s[t]);
-                if (S::T == 4) r |= quant2(v.rest[1], s[t]) << 16;
-                put_rest(t, r);
-                part = __builtin_amdgcn_sdot4((int)r, 0x01010101, part, false);
-            }
-            part = wave_reduce_last(part, [](int x, int y) { return x + y; });
-            sum[t] = __builtin_amdgcn_readlane(part, 63);
         }
         return nans;
     }
@@ -672,17 +722,14 @@ struct Stack {
     __device__ __forceinline__ void product(const Task& tk, int k, Got<MT>& got) {
         typedef Slice<UPW> S;
         float s[MT];
-        int q2[MT];  // twice the sum of the slice: the +2 of the stored codes
         quantize<UPW>(
-            tk, got, s, q2, [&](int t, int i, uint2 v) { *(uint2*)(sh.q[wave][t] + i * 512 + lane * 8) = v; },
+            tk, got, s, [&](int t, int i, uint2 v) { *(uint2*)(sh.q[wave][t] + i * 512 + lane * 8) = v; },
             [&](int t, uint32_t r) {
                 if (lane * S::T < S::kRest) {
                     if (S::T == 2) *(uint16_t*)(sh.q[wave][t] + S::kFull * 512 + lane * 2) = (uint16_t)r;
                     if (S::T == 4) *(uint32_t*)(sh.q[wave][t] + S::kFull * 512 + lane * 4) = r;
                 }
             });
-#pragma unroll
-        for (int t = 0; t < MT; ++t) q2[t] *= 2;
         // the same wave wrote its slices and reads them: LDS operations of a wave complete in order
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -711,9 +758,6 @@ struct Stack {
                 }
         }
         // lane (p, g) holds token p, rows 4 g ..
-        int mine = q2[0];
-#pragma unroll
-        for (int t = 1; t < MT; ++t) mine = p == t ? q2[t] : mine;
 #pragma unroll
         for (int i = 0; i < RPW; ++i) {
             v4i v = acc[i][0];
@@ -724,34 +768,34 @@ struct Stack {
                 v[r] += __builtin_amdgcn_update_dpp(0, v[r], 0x120 + MT, 0xF, 0xF, true);  // row_ror
                 if (SP == 4) v[r] += __builtin_amdgcn_update_dpp(0, v[r], 0x120 + 2 * MT, 0xF, 0xF, true);
             }
-            if (p < MT) *(v4i*)&sh.red[turn][i][wave][p][4 * g] = v - mine;
+            if (p < MT) *(v4i*)&sh.red[turn][i][wave][p][4 * g] = v;
         }
         float sm = s[0];
 #pragma unroll
         for (int t = 1; t < MT; ++t) sm = out_token<RPW>() == t ? s[t] : sm;
-        finish<RPW, RES>(tk, k, sm, 0, got.res);
+        finish<RPW, RES>(tk, k, sm, got.res);
     }
-    // The outputs, by the first waves, from the waves' sums in LDS: sm is the scale of this thread's token (out_token),
-    // `less` what its sums still hold too much
+    // The outputs, by the first waves, from the waves' sums in LDS: sm is the scale of this thread's token (out_token)
     template <int RPW, bool RES>
-    __device__ __forceinline__ void finish(const Task& tk, int k, float sm, int less, uint16_t res) {
+    __device__ __forceinline__ void finish(const Task& tk, int k, float sm, uint16_t res) {
         arrive();
         if (kDirect && wave * 64 >= (RPW == 1 ? 16 : 32) * MT) return;
-        await();
+        // (what does not need the sums, while they come)
         const int m = out_token<RPW>(), tb = out_tb<RPW>(), row = out_row();
         const int n = ((RPW == 1 ? tk.idx : 2 * tk.idx + tb) * 16) + row;
+        const uint16_t* ws = &sh.scales[k & 3][0][RPW == 1 ? tid & 15 : tid & 31];
+        const float inv_s = reciprocal(sm), w1 = bf16_to_f32(ws[0]), w3 = RPW == 4 ? bf16_to_f32(ws[32]) : 0.0f;
+        await();
         if (m < batch() && m < MT && n < tk.n_out) {
-            const uint16_t* ws = &sh.scales[k & 3][0][RPW == 1 ? tid & 15 : tid & 31];
-            const float inv_s = reciprocal(sm);
-            auto value = [&](int i, uint16_t ws) {
-                int sum = -less;
+            auto value = [&](int i, float w) {
+                int sum = 0;
 #pragma unroll
                 for (int k = 0; k < kStWaves; ++k) sum += sh.red[turn][i][k][m][row];
-                return f32_to_bf16_rne(quotient((float)sum, sm, inv_s) * bf16_to_f32(ws));
+                return f32_to_bf16_rne(quotient((float)(sum >> 6), sm, inv_s) * w);  // (64 times the sum)
             };
-            uint16_t v = value(tb, ws[0]);
+            uint16_t v = value(tb, w1);
             if (RPW == 4) {
-                const uint16_t x3 = value(2 + tb, ws[32]);
+                const uint16_t x3 = value(2 + tb, w3);
                 const float r = fmaxf(bf16_to_f32(v), 0.0f);
                 v = f32_to_bf16_rne(bf16_to_f32(f32_to_bf16_rne(r * r)) * bf16_to_f32(x3));
             }
@@ -772,15 +816,15 @@ struct Stack {
         norm_weights<UPW>(tk.aux, tk.K, got);
         wait_ready(k);
         consume(k);
+        look_at_weights<UPW>(got);
         gather_slices<UPW, false>(tk, got);
         float s[TQ];
-        int sum[TQ];
         const int first = wave * S::kValues, step = batch() * 64;
         const __amdgpu_buffer_rsrc_t to = make_rsrc(tk.dst, ((tk.K >> 6) - 1) * step + 64);
         auto place = [&](int at) { return (at >> 6) * step + (at & 63); };
         // (4 bytes at least a store: a word is there or not; values past the end of K are not stored)
         const bool nans = quantize<UPW>(
-            tk, got, s, sum,
+            tk, got, s,
             [&](int, int i, uint2 v) {
                 const int at = first + i * 512 + lane * 8;
                 __builtin_amdgcn_raw_buffer_store_b64(v2u{v.x, v.y}, to, at < tk.K ? place(at) : kBeyond, 0, kSc1);
@@ -795,13 +839,9 @@ struct Stack {
                 __builtin_amdgcn_raw_buffer_store_b32(r, to, mine ? place(at) : kBeyond, 0, kSc1);
             });
         RowRecord* rec = (RowRecord*)tk.res;
-        unsigned mine = (unsigned)sum[0] & (kComplete - 1u);
-        if (nans) {  // readers cannot tell from the words that they are there
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-            mine |= kComplete;
-        }
+        if (nans) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");  // readers cannot tell from the words that they are there
         if (lane == 0) {
-            __hip_atomic_store(&rec->sum[wave], mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&rec->slice[wave], nans ? kComplete : 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (wave == 0) __hip_atomic_store(&rec->scale, (unsigned)f32_to_bf16_rne(s[0]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
@@ -891,8 +931,7 @@ struct Stack {
             }
             if (p < MT) *(v4i*)&sh.red[turn][i][wave][p][4 * g] = v;
         }
-        auto sum30 = [](int v) { return (int)((unsigned)v << 2) >> 2; };
-        finish<RPW, RES>(tk, k, bf16_to_f32((uint16_t)scale), 2 * (sum30(sums.x) + sum30(sums.y) + sum30(sums.z) + sum30(sums.w)), got.res);
+        finish<RPW, RES>(tk, k, bf16_to_f32((uint16_t)scale), got.res);
         turn ^= 1;
     }
 
@@ -1033,6 +1072,7 @@ struct Stack {
         wait_ready(k);
         expand<UPW, RPW>(tk.K, k % kStBuffers, got);
         consume(k);
+        look_at_weights<UPW>(got);
         gather_slices<UPW, RES>(tk, got);
         product<UPW, RPW, RES>(tk, k, got);
     }
@@ -1082,12 +1122,10 @@ __global__ __launch_bounds__(kStThreads) __attribute__((amdgpu_waves_per_eu(2, 2
     // changes only when every workgroup of this launch is done; written past the writer's L2, so read past this one
     const unsigned launch = (unsigned)uniform((int)__hip_atomic_load(&ctl->launch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
     Stack<MT> st{(StackArgsPtr)__builtin_amdgcn_kernarg_segment_ptr(), sh, Waiter{a.spin_limit, &ctl->error, false},
-                 a.ws + a.sets + (size_t)(launch & 1u) * a.set_bytes, launch, tid, tid & 63, uniform(tid >> 6), 0, 0};
+                 a.ws + a.sets + (size_t)(launch & 1u) * a.set_bytes, launch, tid, tid & 63, uniform(tid >> 6), 0, 0, 0};
     if (tid < kStWaves) sh.met[tid] = sh.consumed[tid] = 0;
-    if (tid < Shared<MT>::TQ * kStWaves) {
-        ((v4i*)sh.sumsq)[tid] = v4i{0, 0, 0, 0};
-        ((v2i*)sh.amax)[tid] = v2i{0, 0};
-    }
+    if (tid < 2 * Shared<MT>::TQ * kStWaves) ((v4i*)sh.sumsq)[tid] = v4i{0, 0, 0, 0};
+    if (tid < Shared<MT>::TQ * kStWaves) ((v2i*)sh.amax)[tid] = v2i{0, 0};
     if (tid == 0) sh.claimed = sh.ready = 0;
     {
         // the other set, for the next launch

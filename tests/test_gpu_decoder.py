@@ -777,6 +777,58 @@ def test_decode_stack_kernel_carries_values_that_are_not_finite_like_the_kernels
             assert _equal_or_both_nan(k, k2) and _equal_or_both_nan(v, v2), p
 
 
+def _rows_whose_largest_value_is_near_a_tie(dim, norm_weight, count, eps=1e-5):
+    """Rows h for which max |h g| / rms(h) lies within 2^-21 of the middle between two bf16 numbers."""
+    rng = np.random.default_rng(dim)
+    g = norm_weight.float().cpu().numpy()
+    rows = []
+    while len(rows) < count:
+        h = torch.from_numpy(rng.standard_normal((20000, dim)).astype(np.float32)).to(torch.bfloat16).float().numpy()
+        mean = (h.astype(np.float64) ** 2).sum(-1).astype(np.float32) / np.float32(dim)
+        top = np.abs(h * g).max(-1) * (np.float32(1) / np.sqrt(mean + np.float32(eps)))
+        bits = lambda x: torch.from_numpy(x.astype(np.float32)).to(torch.bfloat16).view(torch.int16).numpy()
+        rows += list(h[bits(top * (1 - 2.0**-21)) != bits(top * (1 + 2.0**-21))])
+    return torch.from_numpy(np.stack(rows[:count])).to(torch.bfloat16)
+
+
+@pytest.mark.parametrize("where", ["tie", "large weight", "small weights", "nan weight", "zero row"])
+@pytest.mark.parametrize("B,dim,ffn,nh,nkv", [(1, 128, 64, 1, 1), (2, 128, 64, 1, 1), (2, 1152, 2112, 9, 9), (3, 128, 64, 1, 1), (8, 1152, 2112, 9, 9)])
+def test_decode_stack_kernel_exchanges_maxima_that_it_cannot_tell_beforehand(B, dim, ffn, nh, nkv, where):
+    """Rows whose largest normalised value does not follow from max |h g| and the sum of squares alone."""
+    S, n_splits = 40, 2
+    args = decoder.ModelArgs(dim=dim, n_layers=2, n_heads=nh, n_kv_heads=nkv, vocab_size=16, ffn_dim=ffn)
+    model = _build(args, seed=dim + B)
+    emb = model.tok_embeddings.weight.data
+    norms = [l.attention_norm.weight.data for l in model.layers] + [l.ffn_norm.weight.data for l in model.layers]
+    if where == "tie":
+        emb[:16] = _rows_whose_largest_value_is_near_a_tie(dim, norms[0], 16).cuda()
+    for w in norms:
+        if where == "large weight":
+            w[dim // 3] = 2.0**20
+            w[dim // 2] = 2.0**90
+        elif where == "small weights":
+            w.mul_(2.0**-75)
+        elif where == "nan weight":
+            w[dim // 2 + 1] = float("nan")
+    if where == "zero row":
+        emb[B - 1] = 0.0
+    caches = [model.make_cache(B, S, "cuda") for _ in range(2)]
+    cos, sin = decoder.rope_tables(128, S, args.rope_theta, "cuda")
+    ws = decoder.AttnWorkspace(B, nh, nkv, n_splits, "cuda")
+    stack = decoder.DecodeStack(model, B, caches[1], n_splits)
+    for p in range(16 // B if where == "tie" else 2):
+        tok = (torch.arange(B, device="cuda") + (p * B if where == "tie" else 0)).reshape(B, 1)
+        pos = torch.full((B, 1), p, dtype=torch.int64, device="cuda")
+        want = model.decode_hidden_fused(tok, pos, caches[0], cos, sin, ws)
+        h, rows = decoder.decode_step_begin(tok.reshape(B), pos.reshape(B), model.tok_embeddings.weight, cos, sin)
+        for workgroups in (0, 3):
+            got = stack(h, pos.reshape(B), rows, workgroups)
+            stack.check()
+            assert _equal_or_both_nan(got, want), (p, workgroups)
+        for (k, v), (k2, v2) in zip(*caches):
+            assert _equal_or_both_nan(k, k2) and _equal_or_both_nan(v, v2), p
+
+
 @pytest.fixture(scope="module")
 def model_2b():
     model = _build(decoder.ModelArgs(), seed=0)
