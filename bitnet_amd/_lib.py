@@ -28,6 +28,15 @@ SIGNATURES = {
         _c_int,
         [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr],
     ),
+    "bitlinear_norm_epilogue_applies": (_c_int, [_c_int, _c_int, _c_int, ctypes.POINTER(_c_int), _c_int]),
+    "bitlinear_norm_gate_forward_bf16": (
+        _c_int,
+        [_c_ptr, _c_ptr, ctypes.c_float, _c_ptr, _c_ptr, ctypes.POINTER(_c_int), _c_int, _c_ptr, _c_ptr, _c_ptr, *[_c_int] * 4, _c_ptr],
+    ),
+    "bitlinear_norm_rope_forward_bf16": (
+        _c_int,
+        [_c_ptr, _c_ptr, ctypes.c_float, _c_ptr, _c_ptr, ctypes.POINTER(_c_int), _c_int, *[_c_ptr] * 8, *[_c_int] * 7, _c_ptr],
+    ),
     "bitlinear_int8xint2_seg": (
         _c_int,
         [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, ctypes.POINTER(_c_int), _c_int, _c_int, _c_int, _c_int, _c_ptr],

@@ -2926,6 +2926,45 @@ int ring_choice(int M, int N, int K, const ScaleMap& smap, bool aligned) {
     if (ring_tiles(M, N, 4) <= kRingCus) return 4;
     return 0;
 }
+template <class Epi>
+int launch_ring(int ring, const int8_t* act, const int8_t* packed, uint16_t* out, int32_t* acc_out, const uint16_t* s,
+                const uint16_t* ws, const ScaleMap& smap, int M, int N, int K, hipStream_t stream, const uint16_t* residual, Epi epi) {
+    const uint32_t* wq = (const uint32_t*)packed;
+    if ((long long)N * K / 4 >= (1ll << 31)) return BITLINEAR_ERR_SHAPE;  // 32-bit offsets into the weights
+    g_last_kernel = "gemm_i2_prefill_kernel";
+    // more LDS than the 64 KiB that a kernel gets without asking (a host-side attribute, set once per device)
+    static OncePerDevice lds_limit_raised;
+    const hipError_t lds_err = t_plan.active ? hipSuccess : lds_limit_raised.run([] {
+        hipError_t e = hipSuccess;
+#define BITLINEAR_RING_LDS(...)                                                                                                     \
+    if (e == hipSuccess)                                                                                                          \
+    e = hipFuncSetAttribute((const void*)gemm_i2_prefill_kernel<__VA_ARGS__, Epi>, hipFuncAttributeMaxDynamicSharedMemorySize, \
+                            Ring<__VA_ARGS__>::LDS)
+        BITLINEAR_RING_LDS(BITLINEAR_RING_A);
+        BITLINEAR_RING_LDS(BITLINEAR_RING_B);
+        BITLINEAR_RING_LDS(BITLINEAR_RING_C);
+        BITLINEAR_RING_LDS(BITLINEAR_RING_D);
+#undef BITLINEAR_RING_LDS
+        return e;
+    });
+    if (lds_err != hipSuccess) return BITLINEAR_ERR_LAUNCH;
+    const int row_tiles = (M + kRingRows[ring] - 1) / kRingRows[ring], col_tiles = (N + kRingCols[ring] - 1) / kRingCols[ring];
+    const long long tiles = ring_tiles(M, N, ring);
+    if (tiles >= (1ll << 22)) return BITLINEAR_ERR_SHAPE;
+    const dim3 grid(8 * (unsigned)((tiles + 7) / 8), 1, 1);
+#define BITLINEAR_LAUNCH_RING(...)                                                                                                 \
+    BL_LAUNCH((gemm_i2_prefill_kernel<__VA_ARGS__, Epi>), grid, dim3(Ring<__VA_ARGS__>::THREADS), (Ring<__VA_ARGS__>::LDS), stream, act, \
+              wq, M, N, K, (int)tiles, out || Epi::kRope ? 1 : 0, row_tiles, col_tiles, s, out, acc_out, ws, smap, residual, epi)
+    switch (ring) {
+        case 1: BITLINEAR_LAUNCH_RING(BITLINEAR_RING_A); break;
+        case 2: BITLINEAR_LAUNCH_RING(BITLINEAR_RING_B); break;
+        case 3: BITLINEAR_LAUNCH_RING(BITLINEAR_RING_C); break;
+        default: BITLINEAR_LAUNCH_RING(BITLINEAR_RING_D); break;
+    }
+#undef BITLINEAR_LAUNCH_RING
+    return launch_status();
+}
+
 int launch_prefill(const int8_t* act, const int8_t* packed, uint16_t* out, int32_t* acc_out, const uint16_t* s,
                    const uint16_t* ws, const ScaleMap& smap, int M, int N, int K, hipStream_t stream,
                    const uint16_t* residual = nullptr) {
@@ -2948,15 +2987,6 @@ int launch_prefill(const int8_t* act, const int8_t* packed, uint16_t* out, int32
         if (e == hipSuccess)
             e = hipFuncSetAttribute((const void*)gemm_i2_prefill_kernel<2, 2, 2>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     2 * 2 * 64 * kPfRowBytes);
-#define BITLINEAR_RING_LDS(...)                                                                                                   \
-    if (e == hipSuccess)                                                                                                         \
-        e = hipFuncSetAttribute((const void*)gemm_i2_prefill_kernel<__VA_ARGS__>, hipFuncAttributeMaxDynamicSharedMemorySize, \
-                                Ring<__VA_ARGS__>::LDS)
-        BITLINEAR_RING_LDS(BITLINEAR_RING_A);
-        BITLINEAR_RING_LDS(BITLINEAR_RING_B);
-        BITLINEAR_RING_LDS(BITLINEAR_RING_C);
-        BITLINEAR_RING_LDS(BITLINEAR_RING_D);
-#undef BITLINEAR_RING_LDS
         return e;
     });
     if (lds_err != hipSuccess) return BITLINEAR_ERR_LAUNCH;
@@ -3014,21 +3044,7 @@ int launch_prefill(const int8_t* act, const int8_t* packed, uint16_t* out, int32
     }
     const int ring = ring_choice(M, N, K, smap, dma_fits);
     if (ring) {
-        const int row_tiles = (M + kRingRows[ring] - 1) / kRingRows[ring], col_tiles = (N + kRingCols[ring] - 1) / kRingCols[ring];
-        const long long tiles = ring_tiles(M, N, ring);
-        if (tiles >= (1ll << 22)) return BITLINEAR_ERR_SHAPE;
-        const dim3 rgrid(8 * (unsigned)((tiles + 7) / 8), 1, 1);
-#define BITLINEAR_LAUNCH_RING(...)                                                                                             \
-    BL_LAUNCH((gemm_i2_prefill_kernel<__VA_ARGS__>), rgrid, dim3(Ring<__VA_ARGS__>::THREADS), (Ring<__VA_ARGS__>::LDS), stream, act, wq, M, \
-              N, K, (int)tiles, out ? 1 : 0, row_tiles, col_tiles, s, out, acc_out, ws, smap, residual)
-        switch (ring) {
-            case 1: BITLINEAR_LAUNCH_RING(BITLINEAR_RING_A); break;
-            case 2: BITLINEAR_LAUNCH_RING(BITLINEAR_RING_B); break;
-            case 3: BITLINEAR_LAUNCH_RING(BITLINEAR_RING_C); break;
-            default: BITLINEAR_LAUNCH_RING(BITLINEAR_RING_D); break;
-        }
-#undef BITLINEAR_LAUNCH_RING
-        return launch_status();
+        return launch_ring(ring, act, packed, out, acc_out, s, ws, smap, M, N, K, stream, residual, RingPlain{});
     }
     bool dma = true;
     int dma_mt = 2;  // row tiles of 32 tokens per workgroup of that kernel: 64 x 256, or 32 x 256 / 128 x 256 when forced
@@ -3842,6 +3858,47 @@ int bitlinear_norm_forward_bf16_seg(const uint16_t* x, const uint16_t* norm_weig
                              seg_ends, nseg);
 }
 
+// gate / norm / quantizer once per token row
+static int launch_norm_quant(const uint16_t* x, const uint16_t* norm_weight, float eps, int glu, int8_t* q_ws, uint16_t* s_ws, int M,
+                             int K, int mode, hipStream_t stream) {
+    // very many rows, no gate, short rows: a wave per row (norm + product at K = 2560: 32.2 -> 30.1 us at 2048 rows,
+    // 53.6 -> 48.7 at 4096; below 1024 rows 0.2-0.9 us behind, with the gate at K = 6912 4-7 us behind: not taken)
+    if (M >= kNormRowsPerWaveMinRows && !glu && K <= 8 * 64 * 8) {
+        const int per_lane = (K / 8 + 63) / 64;
+        const dim3 rgrid((M + 3) / 4, 1, 1), rblock(256, 1, 1);
+#define BITLINEAR_LAUNCH_NR(P, V) \
+    BL_LAUNCH((norm_quant_rows_kernel<P, V>), rgrid, rblock, 0, stream, x, norm_weight, eps, q_ws, s_ws, M, K, mode)
+#define BITLINEAR_LAUNCH_NR_V(V) BITLINEAR_LAUNCH_NR(1, V)
+        if (per_lane <= 2) { BITLINEAR_LAUNCH_NR_V(2); }
+        else if (per_lane <= 5) { BITLINEAR_LAUNCH_NR_V(5); }
+        else { BITLINEAR_LAUNCH_NR_V(8); }
+#undef BITLINEAR_LAUNCH_NR_V
+#undef BITLINEAR_LAUNCH_NR
+        return launch_status();
+    }
+    const dim3 grid(M, 1, 1), block(kPreThreads, 1, 1);
+    const int per_thread = (K / 8 + kPreThreads - 1) / kPreThreads;
+#define BITLINEAR_LAUNCH_PRE(P, V) \
+    BL_LAUNCH((norm_quant_kernel<P, V>), grid, block, 0, stream, x, norm_weight, eps, q_ws, s_ws, K, mode)
+#define BITLINEAR_LAUNCH_PRE_V(V)    \
+    if (glu)                         \
+        BITLINEAR_LAUNCH_PRE(2, V);  \
+    else                             \
+        BITLINEAR_LAUNCH_PRE(1, V)
+    if (per_thread <= 1) {
+        BITLINEAR_LAUNCH_PRE_V(1);
+    } else if (per_thread <= 2) {
+        BITLINEAR_LAUNCH_PRE_V(2);
+    } else if (per_thread <= 4) {
+        BITLINEAR_LAUNCH_PRE_V(4);
+    } else {
+        BITLINEAR_LAUNCH_PRE_V(8);
+    }
+#undef BITLINEAR_LAUNCH_PRE_V
+#undef BITLINEAR_LAUNCH_PRE
+    return launch_status();
+}
+
 static int norm_forward_impl(const uint16_t* x, const uint16_t* norm_weight, float eps, int glu, const int8_t* packed,
                              const uint16_t* ws, const uint16_t* residual, uint16_t* output0, int8_t* q_ws, uint16_t* s_ws,
                              int M, int N, int K, int mode, void* stream, const int* seg_ends, int nseg) {
@@ -3873,44 +3930,68 @@ static int norm_forward_impl(const uint16_t* x, const uint16_t* norm_weight, flo
     // larger blocks: gate / norm / quantizer once per token row, then the product with the residual epilogue
     if (!q_ws || !s_ws) return set_status(pl.ok ? BITLINEAR_ERR_NULL : BITLINEAR_ERR_SHAPE);
     if (K > kPreThreads * kPreVecs * 8) return set_status(BITLINEAR_ERR_SHAPE);
-    // very many rows, no gate, short rows: a wave per row (norm + product at K = 2560: 32.2 -> 30.1 us at 2048 rows,
-    // 53.6 -> 48.7 at 4096; below 1024 rows 0.2-0.9 us behind, with the gate at K = 6912 4-7 us behind: not taken)
-    if (M >= kNormRowsPerWaveMinRows && !glu && K <= 8 * 64 * 8) {
-        const int per_lane = (K / 8 + 63) / 64;
-        const dim3 rgrid((M + 3) / 4, 1, 1), rblock(256, 1, 1);
-#define BITLINEAR_LAUNCH_NR(P, V) \
-    BL_LAUNCH((norm_quant_rows_kernel<P, V>), rgrid, rblock, 0, (hipStream_t)stream, x, norm_weight, eps, q_ws, s_ws, M, K, mode)
-#define BITLINEAR_LAUNCH_NR_V(V) BITLINEAR_LAUNCH_NR(1, V)
-        if (per_lane <= 2) { BITLINEAR_LAUNCH_NR_V(2); }
-        else if (per_lane <= 5) { BITLINEAR_LAUNCH_NR_V(5); }
-        else { BITLINEAR_LAUNCH_NR_V(8); }
-#undef BITLINEAR_LAUNCH_NR_V
-#undef BITLINEAR_LAUNCH_NR
-        if (launch_status() != BITLINEAR_OK) return set_status(BITLINEAR_ERR_LAUNCH);
-        return set_status(launch_gemv(q_ws, packed, output0, nullptr, s_ws, ws, sm, M, N, K, (hipStream_t)stream, residual));
-    }
-    const dim3 grid(M, 1, 1), block(kPreThreads, 1, 1);
-    const int per_thread = (K / 8 + kPreThreads - 1) / kPreThreads;
-#define BITLINEAR_LAUNCH_PRE(P, V) \
-    BL_LAUNCH((norm_quant_kernel<P, V>), grid, block, 0, (hipStream_t)stream, x, norm_weight, eps, q_ws, s_ws, K, mode)
-#define BITLINEAR_LAUNCH_PRE_V(V)    \
-    if (glu)                         \
-        BITLINEAR_LAUNCH_PRE(2, V);  \
-    else                             \
-        BITLINEAR_LAUNCH_PRE(1, V)
-    if (per_thread <= 1) {
-        BITLINEAR_LAUNCH_PRE_V(1);
-    } else if (per_thread <= 2) {
-        BITLINEAR_LAUNCH_PRE_V(2);
-    } else if (per_thread <= 4) {
-        BITLINEAR_LAUNCH_PRE_V(4);
-    } else {
-        BITLINEAR_LAUNCH_PRE_V(8);
-    }
-#undef BITLINEAR_LAUNCH_PRE_V
-#undef BITLINEAR_LAUNCH_PRE
-    if (launch_status() != BITLINEAR_OK) return set_status(BITLINEAR_ERR_LAUNCH);
+    const int st = launch_norm_quant(x, norm_weight, eps, glu, q_ws, s_ws, M, K, mode, (hipStream_t)stream);
+    if (st != BITLINEAR_OK) return set_status(st);
     return set_status(launch_gemv(q_ws, packed, output0, nullptr, s_ws, ws, sm, M, N, K, (hipStream_t)stream, residual));
+}
+
+}  // extern "C"
+
+// Norm + prompt-sized product with what follows the product in its epilogue: common checks, the norm and quantizer, then
+// the GEMM instance that ring_choice names
+template <class Epi>
+static int norm_ring_impl(const uint16_t* x, const uint16_t* norm_weight, float eps, const int8_t* packed, const uint16_t* ws,
+                          const int* seg_ends, int nseg, uint16_t* output0, int8_t* q_ws, uint16_t* s_ws, int M, int N, int K,
+                          int mode, void* stream, Epi epi) {
+    refresh_tuning();
+    if (!shape_ok(M, N, K)) return set_status(BITLINEAR_ERR_SHAPE);
+    if (!x || !norm_weight || !packed || !ws || !q_ws || !s_ws) return set_status(BITLINEAR_ERR_NULL);
+    if (mode != 0 && mode != 1) return set_status(BITLINEAR_ERR_ARG);
+    if ((((uintptr_t)x) | ((uintptr_t)packed) | ((uintptr_t)norm_weight) | ((uintptr_t)q_ws) | ((uintptr_t)output0)) & 15u)
+        return set_status(BITLINEAR_ERR_ARG);
+    ScaleMap sm = equal_slots(N, bitlinear_ws_num(N, K));
+    if (seg_ends) {
+        const int st = segment_map(seg_ends, nseg, N, &sm);
+        if (st != BITLINEAR_OK) return set_status(st);
+    }
+    const int ring = M > kPrefillMinTokens && K <= kPreThreads * kPreVecs * 8 ? ring_choice(M, N, K, sm, K % 128 == 0) : 0;
+    if (!ring || (Epi::kGate && N % 32)) return set_status(BITLINEAR_ERR_SHAPE);
+    const int st = launch_norm_quant(x, norm_weight, eps, 0, q_ws, s_ws, M, K, mode, (hipStream_t)stream);
+    if (st != BITLINEAR_OK) return set_status(st);
+    return set_status(launch_ring(ring, q_ws, packed, output0, nullptr, s_ws, ws, sm, M, N, K, (hipStream_t)stream, nullptr, epi));
+}
+
+extern "C" {
+
+int bitlinear_norm_epilogue_applies(int M, int N, int K, const int* seg_ends, int nseg) {
+    refresh_tuning();
+    if (!shape_ok(M, N, K) || N % 32 || M <= kPrefillMinTokens || K > kPreThreads * kPreVecs * 8) return 0;
+    ScaleMap sm = equal_slots(N, bitlinear_ws_num(N, K));
+    if (seg_ends && segment_map(seg_ends, nseg, N, &sm) != BITLINEAR_OK) return 0;
+    return ring_choice(M, N, K, sm, K % 128 == 0) != 0;
+}
+
+int bitlinear_norm_gate_forward_bf16(const uint16_t* x, const uint16_t* norm_weight, float eps, const int8_t* packed,
+                                     const uint16_t* ws, const int* seg_ends, int nseg, uint16_t* output0, int8_t* q_ws,
+                                     uint16_t* s_ws, int M, int N, int K, int mode, void* stream) {
+    if (!output0) return set_status(BITLINEAR_ERR_NULL);
+    return norm_ring_impl(x, norm_weight, eps, packed, ws, seg_ends, nseg, output0, q_ws, s_ws, M, N, K, mode, stream, RingGate{});
+}
+
+int bitlinear_norm_rope_forward_bf16(const uint16_t* x, const uint16_t* norm_weight, float eps, const int8_t* packed,
+                                     const uint16_t* ws, const int* seg_ends, int nseg, const int64_t* positions,
+                                     const float* cos_table, const float* sin_table, uint16_t* cache_k, uint16_t* cache_v,
+                                     uint16_t* q_out, int8_t* q_ws, uint16_t* s_ws, int B, int T, int S, int n_heads,
+                                     int n_kv_heads, int K, int mode, void* stream) {
+    if (B < 1 || T < 1 || S < 1 || n_heads < 1 || n_kv_heads < 1 || (long long)B * T >= (1ll << 31) ||
+        ((long long)n_heads + 2ll * n_kv_heads) * 128 >= (1ll << 31))
+        return set_status(BITLINEAR_ERR_SHAPE);
+    if (!positions || !cos_table || !sin_table || !cache_k || !cache_v || !q_out) return set_status(BITLINEAR_ERR_NULL);
+    if ((((uintptr_t)cos_table) | ((uintptr_t)sin_table) | ((uintptr_t)cache_k) | ((uintptr_t)cache_v) | ((uintptr_t)q_out)) & 15u)
+        return set_status(BITLINEAR_ERR_ARG);
+    const RingRope epi = {positions, cos_table, sin_table, cache_k, cache_v, q_out, T, S, n_heads, n_kv_heads};
+    return norm_ring_impl(x, norm_weight, eps, packed, ws, seg_ends, nseg, nullptr, q_ws, s_ws, B * T, (n_heads + 2 * n_kv_heads) * 128, K,
+                          mode, stream, epi);
 }
 
 int bitlinear_plan_name(int entry, int M, int N, int K, char* buf, int buflen) {

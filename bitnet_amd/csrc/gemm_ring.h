@@ -43,7 +43,6 @@ struct Ring {
     static constexpr int LDS = S * STAGE > RED ? S * STAGE : RED;
     static constexpr int THREADS = 64 * (WAVES + LW);
     static constexpr int WGS = 2 * (LDS + TM * 8 + 64) <= 160 * 1024 ? 2 : 1;  // workgroups per CU
-    static constexpr int PIECES = TM * TN / 8 <= 64 * WAVES ? 1 : TM * TN / 8 / (64 * WAVES);  // 8 outputs each, per thread
     static_assert(AR * LWAVES * 1024 == A_BYTES && WR * LWAVES * 1024 == W_BYTES, "whole load instructions per wave");
     static_assert(KPW >= 2 && KPW % 2 == 0 && KPW * KG == KSTEPS, "operand registers alternate");
     static_assert(S >= 4 && (S - 1) * LOADS <= 63, "loads in flight are counted in six bits");
@@ -56,16 +55,43 @@ __device__ __forceinline__ int ring_div(int n, int d) {
     q += (n - q * d >= d ? 1 : 0) - (n - q * d < 0 ? 1 : 0);
     return __builtin_amdgcn_readfirstlane(q);
 }
+// What becomes of the outputs: what follows a prompt's product is a launch and a trip of its rows through memory less (in a
+// layer of a 512-token prompt rope and cache write 5.8 us beside the GEMM's 8.4, together 9.5; the gate's output is half of
+// what w13 wrote, 22 -> 20.9, and the norm behind it reads half, 6.0 -> 5.4).  RingPlain: rows of `out`, with the residual added if there is one.
+struct RingPlain {
+    static constexpr bool kGate = false, kRope = false;
+};
+// RingGate: the weight's rows are two halves, x1 and x3, and out = bf16(bf16(relu(x1)^2) * x3), half as wide.  A wave's two
+// column tiles are the same columns of either half.
+struct RingGate {
+    static constexpr bool kGate = true, kRope = false;
+};
+// RingRope: the columns are heads of 128: q heads are rotated into q_out, k heads rotated and v heads copied into the cache
+// rows of the tokens' positions (what rope_cache_tokens_kernel does with the rows, value for value)
+struct RingRope {
+    static constexpr bool kGate = false, kRope = true;
+    const int64_t* positions;
+    const float *cos_t, *sin_t;
+    uint16_t *cache_k, *cache_v, *q_out;
+    int T, S, n_heads, n_kv;
+};
+typedef float v4f_ring __attribute__((ext_vector_type(4)));
+struct RingTurn {
+    int p;
+    v4f_ring cs, sn;
+};
 constexpr int kRingBeyond = 0x7ffffff0;  // an offset behind every descriptor: nothing is fetched, zeros arrive
 
-template <int MT, int NT, int WM, int WN, int KG, int CK, int S, int LW>
+template <int MT, int NT, int WM, int WN, int KG, int CK, int S, int LW, class Epi>
 __global__ __launch_bounds__(64 * (WM * WN * KG + LW)) __attribute__((amdgpu_waves_per_eu((WM * WN * KG + LW) * Ring<MT, NT, WM, WN, KG, CK, S, LW>::WGS / 4)))
 void gemm_i2_prefill_kernel(
     const int8_t* __restrict__ act, const uint32_t* __restrict__ wq, int M, int N, int K, int ntiles, int flags,
     int row_tiles, int col_tiles, const uint16_t* __restrict__ s, uint16_t* __restrict__ out, int32_t* __restrict__ acc_out,
-    const uint16_t* __restrict__ ws, ScaleMap smap, const uint16_t* __restrict__ residual) {
+    const uint16_t* __restrict__ ws, ScaleMap smap, const uint16_t* __restrict__ residual, const Epi epi) {
     typedef Ring<MT, NT, WM, WN, KG, CK, S, LW> R;
     constexpr int QR = 8 / NT;
+    constexpr int COLS = Epi::kGate ? R::TN / 2 : R::TN;  // output columns of a tile
+    static_assert(!Epi::kGate || NT == 2, "a column tile of either half");
     extern __shared__ __attribute__((aligned(1024))) int8_t lds_x[];
 
     // Workgroup -> tile.  The tiles, band of kRingBand row tiles by band, column by column within a band, are cut into
@@ -85,7 +111,8 @@ void gemm_i2_prefill_kernel(
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int grp = wave / (WM * WN), wm = (wave / WN) % WM, wn = wave % WN;
     const int nl = lane & 31, kc = lane >> 5;
-    const int m0 = row_tile * R::TM, n_base = col_tile * R::TN;
+    const int m0 = row_tile * R::TM, n_base = col_tile * COLS;
+    const int n_out = Epi::kGate ? N >> 1 : N;
     const int nchunks = (K + CK - 1) / CK;
 
     const int rows_here = (M - m0) < R::TM ? (M - m0) : R::TM;
@@ -109,8 +136,15 @@ void gemm_i2_prefill_kernel(
         const int q = (r * R::LWAVES + lw) * 64 + lane;
         constexpr int per_step = R::TN / 16 * 8;
         const int ks = q / per_step;
-        int blk = (n_base >> 4) + (q % per_step) / 8;
-        blk = blk < (N >> 4) ? blk : (N >> 4) - 1;
+        int blk = (q % per_step) / 8;
+        if (Epi::kGate) {  // of a wave's four blocks two are x1's, two x3's
+            const int half = (blk >> 1) & 1;
+            blk = (n_base >> 4) + (blk >> 2) * 2 + (blk & 1);
+            blk = (blk < (n_out >> 4) ? blk : (n_out >> 4) - 1) + half * (n_out >> 4);
+        } else {
+            blk += n_base >> 4;
+            blk = blk < (N >> 4) ? blk : (N >> 4) - 1;  // (row blocks behind the last are never stored)
+        }
         w_k[r] = ks * 32;
         w_voff[r] = blk * K * 4 + ks * 128 + (q & 7) * 16;
     }
@@ -157,6 +191,11 @@ void gemm_i2_prefill_kernel(
         return;
     }
 
+    // the outputs that go through LDS: eight of a row per thread
+    constexpr int PER_ROW = COLS / 8;              // threads that share a row
+    constexpr int ROWS = R::WAVES * 64 / PER_ROW;  // rows that the threads cover at a time
+    constexpr int TIMES = (R::TM + ROWS - 1) / ROWS;
+    const int pr = threadIdx.x / PER_ROW, pc = threadIdx.x % PER_ROW * 8, n = n_base + pc;
     // the scales, for the epilogue: requested behind the first stages, in LDS before the sums are
     __shared__ float sval[R::TM], rinv[R::TM], wsv[kMaxSeg];
     uint16_t s_raw = 0, ws_raw = 0;
@@ -164,6 +203,15 @@ void gemm_i2_prefill_kernel(
         const int m = m0 + (int)threadIdx.x;
         if (threadIdx.x < R::TM) s_raw = s[m < M ? m : M - 1];
         if (threadIdx.x < kMaxSeg) ws_raw = ws[(int)threadIdx.x < smap.nseg ? threadIdx.x : 0];
+    }
+    // ... as are the positions of this thread's outputs
+    int64_t at[KG > 1 ? TIMES : MT] = {};
+    if constexpr (Epi::kRope) {
+#pragma unroll
+        for (int i = 0; i < (KG > 1 ? TIMES : MT); ++i) {
+            const int m = m0 + (KG > 1 ? i * ROWS + pr : (wm * MT + i) * 32 + nl);
+            at[i] = epi.positions[m < M ? m : M - 1];
+        }
     }
 
     v16i acc[MT][NT];
@@ -180,8 +228,9 @@ void gemm_i2_prefill_kernel(
 #pragma unroll
     for (int j = 0; j < R::KPW; ++j)
         a_rd[j] = (wm * MT * 32 + nl) * CK + ((((grp * R::KPW + j) * 2 + kc) ^ ((nl >> R::SWZ_SHIFT) & R::SWZ)) * 16);
-    const int w_rd = R::A_BYTES + grp * R::KPW * (R::TN * 8) + (wn * NT * 2 + nl / (2 * QR)) * 128 +
-                     (((nl % (2 * QR)) / QR) * 16 + kc * 8 + NT * (nl % QR)) * 4;
+    const int w_rd = R::A_BYTES + grp * R::KPW * (R::TN * 8) +
+                     (Epi::kGate ? (wn * 4 + (nl >> 4)) * 128 + ((nl >> 3 & 1) * 16 + kc * 8 + (nl & 7)) * 4
+                                 : (wn * NT * 2 + nl / (2 * QR)) * 128 + (((nl % (2 * QR)) / QR) * 16 + kc * 8 + NT * (nl % QR)) * 4);
     auto expand = [&](uint32_t wd) -> v4i {
         const uint32_t x = wd ^ 0xAAAAAAAAu;
         v4i r;
@@ -195,7 +244,13 @@ void gemm_i2_prefill_kernel(
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) a[mt] = *(const v4i*)(stage + a_rd[j] + mt * 32 * CK);
     };
-    auto read_w = [&](const int8_t* stage, int j) -> wvec_t { return *(const wvec_t*)(stage + w_rd + j * (R::TN * 8)); };
+    auto read_w = [&](const int8_t* stage, int j) -> wvec_t {
+        const int8_t* from = stage + w_rd + j * (R::TN * 8);
+        if constexpr (Epi::kGate)
+            return wvec_t{*(const uint32_t*)from, *(const uint32_t*)(from + 256)};
+        else
+            return *(const wvec_t*)from;
+    };
     // stages 0 and 1 are there (every wave waits for its own requests, then all meet)
     if (!LW) __builtin_amdgcn_s_waitcnt(kWaitYounger);
     meet();
@@ -242,36 +297,65 @@ void gemm_i2_prefill_kernel(
 
     // the groups' accumulators: each finishes the register quads q with q % KG == group
     constexpr int QUADS = MT * 4;
-    // eight consecutive outputs of one token from their sums: the reference's epilogue (the bits of the IEEE divide by
-    // the token's scale from its reciprocal and one correction step, as in gemm_i2_prefill_kernel)
-    auto store8 = [&](int m, int n, const int(&x)[8], float sv, float ri, float w) {
+    // the reference's epilogue (the bits of the IEEE divide by the token's scale from its reciprocal and one correction
+    // step, as in gemm_i2_prefill_kernel): two neighbouring sums -> packed bf16
+    auto result2 = [](int x, int y, float sv, float ri, float w) {
+        const float a = (float)x, b = (float)y;
+        const float p0 = a * ri, q0 = b * ri;
+        return f32x2_to_bf16x2(__builtin_fmaf(__builtin_fmaf(-p0, sv, a), ri, p0) * w, __builtin_fmaf(__builtin_fmaf(-q0, sv, b), ri, q0) * w);
+    };
+    auto low = [](uint32_t d) { return __uint_as_float(d << 16); };
+    auto high = [](uint32_t d) { return __uint_as_float(d & 0xffff0000u); };
+    // two gated outputs (glu8's arithmetic)
+    auto gate2 = [&](uint32_t x1, uint32_t x3) {
+        const float r0 = fmaxf(low(x1), 0.0f), r1 = fmaxf(high(x1), 0.0f);
+        const uint32_t sq = f32x2_to_bf16x2(r0 * r0, r1 * r1);
+        return f32x2_to_bf16x2(low(sq) * low(x3), high(sq) * high(x3));
+    };
+    // a token's position and the angles of four pairs
+    auto turn_of = [&](int64_t at, int n) {
+        RingTurn t = {};
+        if constexpr (Epi::kRope) {
+            t.p = at < 0 ? 0 : (at >= (int64_t)epi.S ? epi.S - 1 : (int)at);  // nothing outside the buffers is touched
+            t.cs = *(const v4f_ring*)(epi.cos_t + (size_t)t.p * 64 + (n & 127) / 2);
+            t.sn = *(const v4f_ring*)(epi.sin_t + (size_t)t.p * 64 + (n & 127) / 2);
+        }
+        return t;
+    };
+    // eight consecutive outputs of one token from their sums
+    auto store8 = [&](int m, int n, const int(&x)[8], float sv, float ri, float w, const RingTurn& turn) {
         const size_t o = (size_t)m * N + n;
-        if (acc_out) {
+        if (!Epi::kRope && acc_out) {
             *(v4i*)(acc_out + o) = v4i{x[0], x[1], x[2], x[3]};
             *(v4i*)(acc_out + o + 4) = v4i{x[4], x[5], x[6], x[7]};
         }
         if (!has_out) return;
         uint32_t ob[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            float h[2];
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const float a = (float)x[2 * i + e];
-                const float q0 = a * ri;
-                h[e] = __builtin_fmaf(__builtin_fmaf(-q0, sv, a), ri, q0) * w;
+        for (int i = 0; i < 4; ++i) ob[i] = result2(x[2 * i], x[2 * i + 1], sv, ri, w);
+        if constexpr (Epi::kRope) {
+            const int head = n >> 7, in = n & 127;
+            uint16_t* to = epi.q_out + ((size_t)m * epi.n_heads + head) * 128 + in;
+            if (head >= epi.n_heads) {
+                const int kv = head - epi.n_heads;
+                to = (kv < epi.n_kv ? epi.cache_k : epi.cache_v) +
+                     (((size_t)(m / epi.T) * epi.S + turn.p) * epi.n_kv + (kv < epi.n_kv ? kv : kv - epi.n_kv)) * 128 + in;
             }
-            ob[i] = f32x2_to_bf16x2(h[0], h[1]);
-        }
-        if (residual) {  // out = bf16(residual + bf16(result))
-            const uint4 rv = *(const uint4*)(residual + o);
-            const uint32_t r4[4] = {rv.x, rv.y, rv.z, rv.w};
+            if (head < epi.n_heads + epi.n_kv) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                ob[i] = f32x2_to_bf16x2(__uint_as_float(r4[i] << 16) + __uint_as_float(ob[i] << 16),
-                                        __uint_as_float(r4[i] & 0xffff0000u) + __uint_as_float(ob[i] & 0xffff0000u));
+                for (int i = 0; i < 4; ++i)
+                    ob[i] = f32x2_to_bf16x2(low(ob[i]) * turn.cs[i] - high(ob[i]) * turn.sn[i], low(ob[i]) * turn.sn[i] + high(ob[i]) * turn.cs[i]);
+            }
+            *(uint4*)to = make_uint4(ob[0], ob[1], ob[2], ob[3]);
+        } else {
+            if (residual) {  // out = bf16(residual + bf16(result))
+                const uint4 rv = *(const uint4*)(residual + o);
+                const uint32_t r4[4] = {rv.x, rv.y, rv.z, rv.w};
+#pragma unroll
+                for (int i = 0; i < 4; ++i) ob[i] = f32x2_to_bf16x2(low(r4[i]) + low(ob[i]), high(r4[i]) + high(ob[i]));
+            }
+            *(uint4*)(out + o) = make_uint4(ob[0], ob[1], ob[2], ob[3]);
         }
-        *(uint4*)(out + o) = make_uint4(ob[0], ob[1], ob[2], ob[3]);
     };
     __builtin_amdgcn_s_waitcnt(0x0f70);  // the requests behind the end write zeros into the ring
     meet();
@@ -283,11 +367,13 @@ void gemm_i2_prefill_kernel(
     if constexpr (KG == 1) {
         // every wave holds its sums whole: 4 NT consecutive columns per register quad, stored straight from the registers
         lds_barrier();
-        const int nw = n_base + wn * NT * 32;
-        const int n_last = (nw + NT * 32 - 1) < N ? (nw + NT * 32 - 1) : N - 1;
-        const int slot_first = scale_slot(smap, nw < N ? nw : N - 1);
-        const bool one_slot = slot_first == scale_slot(smap, n_last);
-        const float w1 = wsv[slot_first];
+        const int nw = n_base + wn * (COLS / WN);
+        const int n_last = nw + COLS / WN - 1 < n_out ? nw + COLS / WN - 1 : n_out - 1;
+        const int n_first = nw < n_out ? nw : n_out - 1;
+        const int slot_first = scale_slot(smap, n_first);
+        const int slot3 = Epi::kGate ? scale_slot(smap, n_out + n_first) : 0;
+        const bool one_slot = slot_first == scale_slot(smap, n_last) && (!Epi::kGate || slot3 == scale_slot(smap, n_out + n_last));
+        const float w1 = wsv[slot_first], w3 = wsv[slot3];
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
             const int row = (wm * MT + mt) * 32 + nl, m = m0 + row;
@@ -295,57 +381,90 @@ void gemm_i2_prefill_kernel(
 #pragma unroll
             for (int g4 = 0; g4 < 4; ++g4) {
                 const int ridx = g4 * 8 + kc * 4;
-                const int n = nw + 16 * (ridx / (2 * QR)) + 8 * ((ridx % (2 * QR)) / QR) + NT * (ridx % QR);
                 int x[4 * NT];
+                if constexpr (Epi::kGate) {
+                    const int n = nw + ridx;
+                    if (m >= M || n >= n_out) continue;
+                    const float wa = one_slot ? w1 : wsv[scale_slot(smap, n)], wb = one_slot ? w3 : wsv[scale_slot(smap, n_out + n)];
 #pragma unroll
-                for (int i = 0; i < 4 * NT; ++i) x[i] = acc[mt][i % NT][g4 * 4 + i / NT] >> 6;
-                if (m < M && n < N) store8(m, n, x, sv, ri, one_slot ? w1 : wsv[scale_slot(smap, n)]);
+                    for (int i = 0; i < 8; ++i) x[i] = acc[mt][i >> 2][g4 * 4 + (i & 3)] >> 6;
+                    *(uint2*)(out + (size_t)m * n_out + n) =
+                        make_uint2(gate2(result2(x[0], x[1], sv, ri, wa), result2(x[4], x[5], sv, ri, wb)),
+                                   gate2(result2(x[2], x[3], sv, ri, wa), result2(x[6], x[7], sv, ri, wb)));
+                } else {
+                    const int n = nw + 16 * (ridx / (2 * QR)) + 8 * ((ridx % (2 * QR)) / QR) + NT * (ridx % QR);
+#pragma unroll
+                    for (int i = 0; i < 4 * NT; ++i) x[i] = acc[mt][i % NT][g4 * 4 + i / NT] >> 6;
+                    if (m >= M || n >= N) continue;
+                    RingTurn turn = {};
+                    if constexpr (Epi::kRope) turn = turn_of(at[mt], n);
+                    store8(m, n, x, sv, ri, one_slot ? w1 : wsv[scale_slot(smap, n)], turn);
+                }
             }
         }
         return;
     }
+    RingTurn turn[TIMES] = {};
+    if constexpr (Epi::kRope) {
+#pragma unroll
+        for (int i = 0; i < TIMES; ++i) turn[i] = turn_of(at[i], n);
+    }
     // The sums go through LDS, which adds the groups' shares and turns a lane's pieces of 32 rows into whole runs of a
     // row.  (A lane holds token nl; register quad g4 of its NT column tiles is 4 NT consecutive columns.)
     {
-        int8_t* to = lds_x + (grp * R::TM + wm * MT * 32 + nl) * R::OUT_ROW + wn * NT * 128;
+        int8_t* to = lds_x + (grp * R::TM + wm * MT * 32 + nl) * R::OUT_ROW + wn * (COLS / WN) * 4;
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
             for (int g4 = 0; g4 < 4; ++g4) {
                 const int ridx = g4 * 8 + kc * 4;
-                const int n = 16 * (ridx / (2 * QR)) + 8 * ((ridx % (2 * QR)) / QR) + NT * (ridx % QR);
+                const int n = Epi::kGate ? ridx : 16 * (ridx / (2 * QR)) + 8 * ((ridx % (2 * QR)) / QR) + NT * (ridx % QR);
 #pragma unroll
                 for (int v = 0; v < NT; ++v) {
                     v4i t;
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
-                        const int i = 4 * v + j;  // column n + i: register i / NT of the quad, column tile i % NT
-                        t[j] = acc[mt][i % NT][g4 * 4 + i / NT];
+                        const int i = 4 * v + j;  // column n + i: register i / NT of the quad, column tile i % NT (gate: of half v)
+                        t[j] = Epi::kGate ? acc[mt][v][g4 * 4 + j] : acc[mt][i % NT][g4 * 4 + i / NT];
                     }
-                    *(v4i*)(to + mt * 32 * R::OUT_ROW + (n + 4 * v) * 4) = t;
+                    *(v4i*)(to + mt * 32 * R::OUT_ROW + (n + v * (Epi::kGate ? COLS : 4)) * 4) = t;
                 }
             }
     }
-    static_assert((R::PIECES == 1 || R::PIECES * R::WAVES * 64 * 8 == R::TM * R::TN), "pieces per thread");
-    constexpr int ROWS = R::WAVES * 64 / (R::TN / 8);  // rows of the tile that the threads' piece number p covers
-    const int pr = threadIdx.x / (R::TN / 8), pc = threadIdx.x % (R::TN / 8) * 8, n = n_base + pc;
-    const int slot = scale_slot(smap, n);
+    const int slot = scale_slot(smap, n), slot3 = Epi::kGate ? scale_slot(smap, n_out + n) : 0;
     lds_barrier();
-    const float w = wsv[slot];
-#pragma unroll
-    for (int p = 0; p < R::PIECES; ++p) {
-        const int row = p * ROWS + pr, m = m0 + row;
-        if (row >= R::TM || m >= M || n >= N) continue;  // N % 16 == 0: the eight columns are in or out together
-        const int8_t* from = lds_x + row * R::OUT_ROW + pc * 4;
+    const float w = wsv[slot], w3 = wsv[slot3];
+    // (exact: the accumulators are 64 * sum(w * a))
+    auto sums = [&](const int8_t* from, int(&x)[8]) {
         v4i lo = *(const v4i*)from, hi = *(const v4i*)(from + 16);
 #pragma unroll
         for (int g = 1; g < KG; ++g) {
             lo += *(const v4i*)(from + g * R::TM * R::OUT_ROW);
             hi += *(const v4i*)(from + g * R::TM * R::OUT_ROW + 16);
         }
-        lo >>= 6, hi >>= 6;  // exact: the accumulators are 64 * sum(w * a)
-        const int x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-        store8(m, n, x, sval[row], rinv[row], w);
+        lo >>= 6, hi >>= 6;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] = lo[i], x[4 + i] = hi[i];
+    };
+#pragma unroll
+    for (int p = 0; p < TIMES; ++p) {
+        const int row = p * ROWS + pr, m = m0 + row;
+        if (row >= R::TM || m >= M || n >= n_out) continue;  // N % 16 == 0: the eight columns are in or out together
+        const int8_t* from = lds_x + row * R::OUT_ROW + pc * 4;
+        const float sv = sval[row], ri = rinv[row];
+        int x[8];
+        sums(from, x);
+        if constexpr (Epi::kGate) {
+            int y[8];
+            sums(from + COLS * 4, y);
+            uint32_t ob[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                ob[i] = gate2(result2(x[2 * i], x[2 * i + 1], sv, ri, w), result2(y[2 * i], y[2 * i + 1], sv, ri, w3));
+            *(uint4*)(out + (size_t)m * n_out + n) = make_uint4(ob[0], ob[1], ob[2], ob[3]);
+        } else {
+            store8(m, n, x, sv, ri, w, turn[p]);
+        }
     }
 }
 

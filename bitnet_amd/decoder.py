@@ -324,6 +324,59 @@ def norm_bitlinear(x, norm: "RMSNorm", lin: BitLinearKernel, glu: bool = False, 
     return out
 
 
+def _epilogue_applies(x, norm: "RMSNorm", lin: BitLinearKernel) -> bool:
+    """Whether a prompt's norm + BitLinear can take what follows the product into its epilogue: the shape is one that the
+    GEMM kernel with such an epilogue is chosen for, and the operands are what norm_bitlinear would take."""
+    return (x.dtype == torch.bfloat16 and x.is_cuda and x.is_contiguous() and x.dim() == 2 and x.shape[1] == lin.in_features
+            and norm.weight.dtype == torch.bfloat16 and norm.weight.numel() == lin.in_features
+            and lin.weight.numel() * lin.weight.element_size() * 4 == lin.out_features * lin.in_features
+            and _lib.load_library().bitlinear_norm_epilogue_applies(
+                x.shape[0], lin.out_features, lin.in_features, lin._seg_c, len(lin.seg_ends) if lin.seg_ends else 0) != 0)
+
+
+def norm_gate_bitlinear(x, norm: "RMSNorm", w13: BitLinearKernel):
+    """RMSNorm -> w13 -> squared-ReLU gate in one norm / quantizer kernel and one GEMM (bitlinear_norm_gate_forward_bf16):
+    x bf16 [M, K] -> bf16 [M, ffn], or None where the separate calls have to be made."""
+    if not _epilogue_applies(x, norm, w13):
+        return None
+    M, K, N = x.shape[0], w13.in_features, w13.out_features
+    out = torch.empty(M, N // 2, dtype=torch.bfloat16, device=x.device)
+    q_ws = torch.empty(M, K, dtype=torch.int8, device=x.device)
+    s_ws = torch.empty(M, dtype=torch.bfloat16, device=x.device)
+    st = _lib.load_library().bitlinear_norm_gate_forward_bf16(
+        _ptr(x), _ptr(norm.weight), norm.eps, _ptr(w13.weight), _ptr(w13.weight_scale), w13._seg_c,
+        len(w13.seg_ends) if w13.seg_ends else 0, _ptr(out), _ptr(q_ws), _ptr(s_ws), M, N, K, w13.quant_mode, _stream_ptr())
+    _lib.check(st, f"bitlinear_norm_gate_forward_bf16(M={M}, N={N}, K={K})")
+    return out
+
+
+def norm_rope_bitlinear(x, norm: "RMSNorm", wqkv: BitLinearKernel, cache_k, cache_v, positions, cos, sin, n_heads, n_kv_heads):
+    """RMSNorm -> wqkv -> rope and cache write in one norm / quantizer kernel and one GEMM
+    (bitlinear_norm_rope_forward_bf16): x bf16 [B * T, K], positions int64 [B, T] -> the rotated q, bf16 [B, T, n_heads,
+    128], or None where the separate calls have to be made."""
+    B, T = positions.shape
+    S, hd = cache_k.shape[1], cache_k.shape[-1]
+
+    def fits(t, dtype, shape):
+        return t.dtype == dtype and t.device == x.device and t.is_contiguous() and t.shape == shape and t.data_ptr() % 16 == 0
+
+    if not (hd == 128 and wqkv.out_features == (n_heads + 2 * n_kv_heads) * hd and x.shape[0] == B * T
+            and all(fits(c, torch.bfloat16, (B, S, n_kv_heads, hd)) for c in (cache_k, cache_v))
+            and all(fits(c, torch.float32, (c.shape[0], hd // 2)) and c.shape[0] >= S for c in (cos, sin))
+            and positions.dtype == torch.int64 and positions.is_contiguous() and _epilogue_applies(x, norm, wqkv)):
+        return None
+    M, K = x.shape[0], wqkv.in_features
+    q = torch.empty(B, T, n_heads, hd, dtype=torch.bfloat16, device=x.device)
+    q_ws = torch.empty(M, K, dtype=torch.int8, device=x.device)
+    s_ws = torch.empty(M, dtype=torch.bfloat16, device=x.device)
+    st = _lib.load_library().bitlinear_norm_rope_forward_bf16(
+        _ptr(x), _ptr(norm.weight), norm.eps, _ptr(wqkv.weight), _ptr(wqkv.weight_scale), wqkv._seg_c,
+        len(wqkv.seg_ends) if wqkv.seg_ends else 0, _ptr(positions), _ptr(cos), _ptr(sin), _ptr(cache_k), _ptr(cache_v), _ptr(q),
+        _ptr(q_ws), _ptr(s_ws), B, T, S, n_heads, n_kv_heads, K, wqkv.quant_mode, _stream_ptr())
+    _lib.check(st, f"bitlinear_norm_rope_forward_bf16(B={B}, T={T}, K={K})")
+    return q
+
+
 class DecodeStack:
     """All layers of a decode step as one launch (bitnet_decode_stack) for one
     model, cache and batch: the table of what the layers' parameters point to,
@@ -551,11 +604,11 @@ class Transformer(nn.Module):
     @torch.no_grad()
     def prefill_hidden_fused(self, tokens, cache, cos, sin):
         """A whole prompt on an empty cache, tokens [B, T] at positions 0..T-1:
-        the layer stack of decode_hidden_fused at prompt size (norms, gate and
-        residual adds folded into the BitLinear calls, which run the int8 GEMM),
-        rope + cache write in one kernel, causal attention over the new tokens
-        in another (the reference calls xformers' rope_padded and flash attention
-        here, gpu/model.py:128-155).  Returns the hidden state in front of the
+        the layer stack of decode_hidden_fused at prompt size (norms, gate, residual
+        adds, rope and cache write folded into the BitLinear calls, which run the int8
+        GEMM), causal attention over the new tokens in a kernel of its own (the
+        reference calls xformers' rope_padded and flash attention here,
+        gpu/model.py:128-155).  Returns the hidden state in front of the
         final norm, [B, T, dim]."""
         a = self.args
         B, T = tokens.shape
@@ -563,12 +616,18 @@ class Transformer(nn.Module):
         h = self.tok_embeddings(tokens.reshape(B * T))
         for layer, (ck, cv) in zip(self.layers, cache):
             att, ffn = layer.attention, layer.feed_forward
-            xqkv = norm_bitlinear(h, layer.attention_norm, att.wqkv)
-            q = rope_cache_tokens(xqkv, ck, cv, pos, cos, sin, a.n_heads, a.n_kv_heads)
+            q = norm_rope_bitlinear(h, layer.attention_norm, att.wqkv, ck, cv, pos, cos, sin, a.n_heads, a.n_kv_heads)
+            if q is None:
+                xqkv = norm_bitlinear(h, layer.attention_norm, att.wqkv)
+                q = rope_cache_tokens(xqkv, ck, cv, pos, cos, sin, a.n_heads, a.n_kv_heads)
             o = attn_prefill(q, ck, cv, 0)
             h = norm_bitlinear(o, att.attn_sub_norm, att.wo, residual=h)
-            x13 = norm_bitlinear(h, layer.ffn_norm, ffn.w13)
-            h = norm_bitlinear(x13, ffn.ffn_sub_norm, ffn.w2, glu=True, residual=h)
+            gated = norm_gate_bitlinear(h, layer.ffn_norm, ffn.w13)
+            if gated is None:
+                x13 = norm_bitlinear(h, layer.ffn_norm, ffn.w13)
+                h = norm_bitlinear(x13, ffn.ffn_sub_norm, ffn.w2, glu=True, residual=h)
+            else:
+                h = norm_bitlinear(gated, ffn.ffn_sub_norm, ffn.w2, residual=h)
         return h.view(B, T, a.dim)
 
     @torch.no_grad()

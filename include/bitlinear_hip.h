@@ -293,6 +293,32 @@ int bitlinear_norm_forward_bf16_seg(const uint16_t* x, const uint16_t* norm_weig
                                     int M, int N, int K, int mode, void* stream);
 
 /*
+ * Prompt-sized norm + BitLinear calls with the operation behind the product in the GEMM's epilogue, so that its input
+ * never goes through memory (gpu/model.py:128-157, 191-196 of the reference, where these are separate kernels):
+ *   bitlinear_norm_gate_forward_bf16: weight rows (x1 | x3), N of them; output0 bf16 [M, N / 2] =
+ *     bf16(bf16(relu(x1)^2) * x3) of the bf16 results, what the glu of bitlinear_norm_forward_bf16 makes of [M, N];
+ *   bitlinear_norm_rope_forward_bf16: weight rows (q | k | v), (n_heads + 2 n_kv_heads) * 128 of them, M = B * T; what
+ *     bitnet_rope_cache_tokens makes of the product's rows, same operands.
+ * Values are those of the separate calls, bit for bit (a NaN may be another one).  seg_ends / nseg as in
+ * bitlinear_norm_forward_bf16_seg, NULL: the equal slots.  BITLINEAR_ERR_SHAPE where bitlinear_norm_epilogue_applies
+ * (host only) says 0: M <= 16, K % 128 != 0, N % 32 != 0, scale segments that end elsewhere than at multiples of 8, and
+ * outputs that another GEMM kernel is ahead on (the separate calls choose it).  All pointers 16-byte aligned.
+ */
+int bitlinear_norm_epilogue_applies(int M, int N, int K, const int* seg_ends, int nseg);
+int bitlinear_norm_gate_forward_bf16(const uint16_t* x, const uint16_t* norm_weight, float eps,
+                                     const int8_t* packed, const uint16_t* ws,
+                                     const int* seg_ends, int nseg, uint16_t* output0,
+                                     int8_t* q_ws, uint16_t* s_ws,
+                                     int M, int N, int K, int mode, void* stream);
+int bitlinear_norm_rope_forward_bf16(const uint16_t* x, const uint16_t* norm_weight, float eps,
+                                     const int8_t* packed, const uint16_t* ws,
+                                     const int* seg_ends, int nseg, const int64_t* positions,
+                                     const float* cos_table, const float* sin_table,
+                                     uint16_t* cache_k, uint16_t* cache_v, uint16_t* q_out,
+                                     int8_t* q_ws, uint16_t* s_ws, int B, int T, int S,
+                                     int n_heads, int n_kv_heads, int K, int mode, void* stream);
+
+/*
  * What the library would launch for a call, without launching it (host only:
  * works without a GPU).  Runs the dispatch code of the entry point itself --
  * entry 0: bitlinear_int8xint2, 1: bitlinear_forward_bf16 (mode 0, with

@@ -648,6 +648,67 @@ def test_norm_bitlinear_of_rows_that_are_not_finite(M, K, N):
 # The end-to-end workload at its real size: 30 layers, dim 2560, ffn 6912, 20 / 5 heads, vocabulary
 # 128256 (gpu/model.py:39-49), a 512-token seeded prompt, greedy decode (gpu/generate.py:264-288)
 # ---------------------------------------------------------------------------
+def _norm_and_linear(K, N, gen, segments=None):
+    norm = decoder.RMSNorm(K, 1e-5).cuda().to(torch.bfloat16)
+    norm.weight.data = torch.rand(K, generator=gen, device="cuda").add(0.5).to(torch.bfloat16)
+    lin = BitLinearKernel(K, N, seg_ends=segments).cuda()
+    w = torch.randint(-1, 2, (N, K), generator=gen, device="cuda", dtype=torch.int8)
+    lin.weight.data = pack_weight.convert_weight_int8_to_int2(w, keep_device=True)
+    lin.weight_scale.data = (0.0156 * (1.0 + 0.3 * torch.arange(4, device="cuda"))).to(torch.bfloat16)
+    return norm, lin
+
+
+@pytest.mark.parametrize("tile", [0, 9, 10, 11, 12])  # the instance chosen, and each of them
+@pytest.mark.parametrize("B,T,nh,nkv,K,ffn,S", [(1, 17, 1, 1, 640, 16, 17), (3, 11, 2, 1, 768, 48, 70), (2, 33, 4, 2, 1280, 336, 40),
+                                                (1, 129, 5, 5, 896, 1040, 200), (2, 150, 20, 5, 2560, 6912, 512)])
+def test_prompt_products_with_rope_and_gate_in_the_epilogue_equal_the_separate_calls(B, T, nh, nkv, K, ffn, S, tile):
+    gen = torch.Generator(device="cuda").manual_seed(B * T + ffn)
+    x = torch.randn(B * T, K, generator=gen, device="cuda").to(torch.bfloat16)
+    qkv_rows = [nh * 128, (nh + nkv) * 128, (nh + 2 * nkv) * 128]
+    norm, wqkv = _norm_and_linear(K, qkv_rows[-1], gen, qkv_rows)
+    norm2, w13 = _norm_and_linear(K, 2 * ffn, gen, [ffn, 2 * ffn])
+    cos, sin = decoder.rope_tables(128, S, 500000.0, "cuda")
+    # any order of positions, some of them outside the cache (clamped)
+    pos = torch.stack([torch.randperm(S + 2, generator=gen, device="cuda")[:T] - 1 for _ in range(B)])
+    pos[:, 1:] = torch.where((pos[:, 1:] <= 0) | (pos[:, 1:] >= S - 1), S // 2, pos[:, 1:])  # (two tokens of one row would race)
+    for b in range(B):
+        seen = set()
+        for i, p in enumerate(pos[b].tolist()):
+            while min(max(p, 0), S - 1) in seen:
+                p = (p + 1) % S
+            seen.add(min(max(p, 0), S - 1))
+            pos[b, i] = p
+    caches = [torch.randn(B, S, nkv, 128, generator=gen, device="cuda").to(torch.bfloat16) for _ in range(2)]
+    got_c, want_c = [c.clone() for c in caches], [c.clone() for c in caches]
+    xqkv = decoder.norm_bitlinear(x, norm, wqkv)
+    want_q = decoder.rope_cache_tokens(xqkv, *want_c, pos, cos, sin, nh, nkv)
+    x13 = decoder.norm_bitlinear(x, norm2, w13)
+    want_h = o.squared_relu_glu_bf16(host_bits(x13))
+    lib = _lib.load_library()
+    try:
+        if tile:
+            assert lib.bitlinear_set_tuning(5, tile, 0, 0) == 0
+        got_q = decoder.norm_rope_bitlinear(x, norm, wqkv, *got_c, pos, cos, sin, nh, nkv)
+        got_h = decoder.norm_gate_bitlinear(x, norm2, w13)
+        torch.cuda.synchronize()
+    finally:
+        lib.bitlinear_set_tuning(0, 0, 0, 0)
+    assert (got_q is not None and got_h is not None) or tile == 0
+    if got_q is not None:
+        assert torch.equal(got_q.view(torch.int16), want_q.view(torch.int16))
+        assert all(torch.equal(a.view(torch.int16), b.view(torch.int16)) for a, b in zip(got_c, want_c))
+    if got_h is not None:
+        assert np.array_equal(host_bits(got_h), want_h)
+
+
+def test_prompt_products_that_the_epilogues_do_not_take_are_left_to_the_separate_calls():
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    for M, K, ffn, ends in ((16, 2560, 6912, None), (512, 2496, 6912, None), (512, 2560, 6912, (6900, 13824)), (4096, 2560, 6912, None),
+                            (512, 256, 64, None)):
+        norm, w13 = _norm_and_linear(K, 2 * ffn, gen, ends)
+        assert decoder.norm_gate_bitlinear(torch.zeros(M, K, dtype=torch.bfloat16, device="cuda"), norm, w13) is None, (M, K, ffn, ends)
+
+
 @pytest.mark.parametrize("workgroups", [0, 1, 7, 600])  # 600: more than can be resident, tasks by ticket
 @pytest.mark.parametrize("B,dim,ffn,nh,nkv,S,n_splits,segments", [
     (1, 128, 64, 1, 1, 33, 1, False), (2, 128, 64, 1, 1, 40, 16, False), (1, 1152, 2112, 9, 9, 70, 3, False),
