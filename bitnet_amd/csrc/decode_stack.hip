@@ -86,9 +86,10 @@ constexpr int kStModePolls = 64;        // polls before the mode is decided with
 constexpr int kSc1 = kPollPolicy;       // device-coherent accesses
 typedef unsigned v2u __attribute__((ext_vector_type(2)));
 typedef int v2i __attribute__((ext_vector_type(2)));
-// Four int8 of quantized rows that mean "not written": -128 comes from NaNs alone (|x| * scale rounds to 127 at most).  As
-// an int, below every other word.  A slice with a written word of that value says so in its record (kComplete).
-constexpr int kUnsetBytes = (int)0x80808080;
+// Four int8 of quantized rows that mean "not written": as an int the least there is, so that the minimum of a lane's words
+// shows whether one of them is that.  Its last byte, -128, comes only with NaNs (|x| * scale rounds to 127 at most; where a
+// NaN is the maximum, finite values are clamped): a slice of such a row says in its record that it is written (kComplete).
+constexpr int kUnsetBytes = INT32_MIN;
 constexpr unsigned kComplete = 1u << 30;
 constexpr int kLookEvery = 32;          // polls between two looks at that, a power of two
 constexpr int kBeyond = 0x7ffffff0;     // an offset behind every descriptor: reads as zero, no access
