@@ -59,8 +59,8 @@ __global__ __launch_bounds__(kRopeThreads) void rope_cache_tokens_kernel(
 // written for them: flash-attention style, scores and output on the bf16 matrix pipe (16x16x32).
 // One wave = 16 consecutive tokens of one query head; the G waves of a workgroup are the G heads
 // that share a kv head, so they walk the same cache rows together: the workgroup brings every
-// block of 32 K and V rows into LDS once (double buffered, requested two steps ahead, one
-// LDS-only barrier per step) and each wave takes its operands from there.
+// block of 32 K and V rows into LDS once (a ring of RING steps, one barrier per step) and each wave
+// takes its operands from there.
 //   S^T block = K rows (A operand: 16 positions x 32 dims per step) x q^T (B operand: 16 tokens),
 //   so a result lane (c, g4) holds, for token c, positions 4 g4 + j of the block (j = 0..3).  Two
 //   blocks make the 8 positions that this lane contributes, as its k-slots, to the B operand of
@@ -71,9 +71,16 @@ __global__ __launch_bounds__(kRopeThreads) void rope_cache_tokens_kernel(
 //   lane (c, g4) then holds, for token c, dims 32 g4 + 8 j + t: eight contiguous dims per j.
 // Online softmax per 32 positions: the running maximum of a token is agreed between its four lanes
 // (c, c + 16, c + 32, c + 48) with two lane permutes; the sums stay per lane until the end.
-constexpr int kApRowBytes = kHeadDim * 2 + 16;  // padded LDS row: the 16 rows of a K operand read spread over all banks
+constexpr int kApStepBytes = 2 * 32 * kHeadDim * 2;  // K and V rows of a step
+// 16 bytes per lane from a buffer straight into LDS: lane l's piece lands at `to` + 16 l (wave-uniform)
+__device__ __forceinline__ void ap_load(__amdgpu_buffer_rsrc_t rsrc, uint8_t* to, int offset) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)to, 16, offset, 0, 0, 0);
+}
 
-template <int G>
+// What bounds it: a step is some 200 instructions of the one wave on a SIMD and a chain of LDS reads, four dependent MFMAs,
+// the maximum, the exponentials (0.56 us; 512 tokens are 16 steps).  Rows that came a step ahead through registers had not
+// arrived in time: 512 tokens 12.9 -> 12.0 us, 1000 29.9 -> 26.7, 2048 77.6 -> 53.9 (20 / 5 heads).
+template <int G, int RING>
 __global__ __launch_bounds__(64 * G) void attn_prefill_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ cache_k, const uint16_t* __restrict__ cache_v,
     uint16_t* __restrict__ out, int T, int S, int start, int n_heads, int n_kv_heads) {
@@ -105,37 +112,32 @@ __global__ __launch_bounds__(64 * G) void attn_prefill_kernel(
         (void*)(cache_k + ((size_t)b * S * n_kv_heads + kvh) * kHeadDim), 0, span_bytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(cache_v + ((size_t)b * S * n_kv_heads + kvh) * kHeadDim), 0, span_bytes, 0x00020000);
-    // staging map: piece p = tid + i * NT is the 16-byte piece p % 16 of row p / 16 of a 32-row block
-    constexpr int NT = 64 * G;
-    constexpr int PPT = 512 / NT;
-    __shared__ __attribute__((aligned(16))) uint8_t lds_kv[2][2][32 * kApRowBytes];  // [buffer][K | V]
-    const int tid = threadIdx.x;
-    int g_off[PPT], l_off[PPT];
+    // The rows come straight into LDS, a ring of RING steps: request number r * G + wave of a step fills 1 KB, four
+    // rows of K (the first eight) or V, whose 16-byte pieces are swizzled by the row (by choice of the piece that a lane
+    // fetches), so that 16 rows at one piece and the 16 pieces of a row are both spread over all banks
+    constexpr int kLoads = 16 / G;
+    extern __shared__ __attribute__((aligned(1024))) uint8_t lds_kv[];  // [stage][K | V][32 rows of 256 bytes]
+    int g_off[kLoads];
 #pragma unroll
-    for (int i = 0; i < PPT; ++i) {
-        const int pce = tid + i * NT;
-        g_off[i] = (pce >> 4) * row_bytes + (pce & 15) * 16;
-        l_off[i] = (pce >> 4) * kApRowBytes + (pce & 15) * 16;
+    for (int r = 0; r < kLoads; ++r) {
+        const int row = ((r * G + wave) & 7) * 4 + (lane >> 4);
+        g_off[r] = row * row_bytes + ((lane & 15) ^ (row & 15)) * 16;
     }
-    v4u kst[PPT], vst[PPT];
-    // the whole offset goes into the per-lane operand: that is the one the range check looks at
     auto request = [&](int st) {
-        const int base = st * 32 * row_bytes;
+        uint8_t* to = lds_kv + (st % RING) * kApStepBytes;
+        // (in the per-lane operand: that is the one the range check looks at; unsigned, as it may lie behind 2^31 there)
+        const unsigned base = (unsigned)st * 32u * (unsigned)row_bytes;
 #pragma unroll
-        for (int i = 0; i < PPT; ++i) {
-            kst[i] = __builtin_amdgcn_raw_buffer_load_b128(k_rsrc, base + g_off[i], 0, 0);
-            vst[i] = __builtin_amdgcn_raw_buffer_load_b128(v_rsrc, base + g_off[i], 0, 0);
-        }
+        for (int r = 0; r < kLoads; ++r)
+            ap_load(r < 8 / G ? k_rsrc : v_rsrc, to + (r * G + wave) * 1024, (int)(base + (unsigned)g_off[r]));
     };
-    auto stage = [&](int buf) {
+    // K operand: row c of a 16-row block, piece kk * 4 + g4; V: rows 4 g4 + jj (and 16 + 4 g4 + jj), piece c
+    int k_off[4], v_off[4];
 #pragma unroll
-        for (int i = 0; i < PPT; ++i) {
-            *(v4u*)(&lds_kv[buf][0][l_off[i]]) = kst[i];
-            *(v4u*)(&lds_kv[buf][1][l_off[i]]) = vst[i];
-        }
-    };
-    const int k_lds_off = c * kApRowBytes + g4 * 16;        // K operand: row c of a 16-row block, piece g4 of a 64-byte step
-    const int v_lds_off = 4 * g4 * kApRowBytes + c * 16;    // V: rows 4 g4 + jj (and 16 + 4 g4 + jj), piece c
+    for (int kk = 0; kk < 4; ++kk) {
+        k_off[kk] = c * 256 + (((kk * 4 + g4) ^ c) * 16);
+        v_off[kk] = 32 * 256 + (4 * g4 + kk) * 256 + ((c ^ (4 * g4 + kk)) * 16);
+    }
 
     v4f o_acc[8];
 #pragma unroll
@@ -145,26 +147,30 @@ __global__ __launch_bounds__(64 * G) void attn_prefill_kernel(
     float m_run = -INFINITY, l_run = 0.0f;
     const float c2 = 0.08838834764831845f * 1.4426950408889634f;  // 128^-0.5 * log2(e)
 
-    auto step = [&](int st) {
-        const uint8_t* kl = &lds_kv[st & 1][0][k_lds_off];
-        const uint8_t* vl = &lds_kv[st & 1][1][v_lds_off];
-        v4u kb[2][4], vb[8];
+    // raw scores of a step's 32 positions
+    auto scores = [&](int st, v4f(&acc)[2]) {
+        const uint8_t* kl = lds_kv + (st % RING) * kApStepBytes;
+        v4u kb[2][4];
 #pragma unroll
         for (int bi = 0; bi < 2; ++bi)
 #pragma unroll
-            for (int kk = 0; kk < 4; ++kk) kb[bi][kk] = *(const v4u*)(kl + bi * 16 * kApRowBytes + kk * 64);
+            for (int kk = 0; kk < 4; ++kk) kb[bi][kk] = *(const v4u*)(kl + bi * 16 * 256 + k_off[kk]);
+        acc[0] = acc[1] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int jj = 0; jj < 8; ++jj) vb[jj] = *(const v4u*)(vl + ((jj & 3) + (jj >> 2) * 16) * kApRowBytes);
+        for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+            for (int bi = 0; bi < 2; ++bi)
+                acc[bi] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, kb[bi][kk]), qa[kk], acc[bi], 0, 0, 0);
+    };
+    // softmax and outputs of a step
+    auto step = [&](int st, const v4f(&acc)[2]) {
+        const uint8_t* vl = lds_kv + (st % RING) * kApStepBytes;
+        v4u vb[8];
+#pragma unroll
+        for (int jj = 0; jj < 8; ++jj) vb[jj] = *(const v4u*)(vl + (jj >> 2) * 16 * 256 + v_off[jj & 3]);
         float sc[8];
 #pragma unroll
-        for (int bi = 0; bi < 2; ++bi) {
-            v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int kk = 0; kk < 4; ++kk)
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, kb[bi][kk]), qa[kk], acc, 0, 0, 0);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) sc[bi * 4 + j] = acc[j];
-        }
+        for (int i = 0; i < 8; ++i) sc[i] = acc[i >> 2][i & 3];
         // only the steps that reach beyond the block's first token need the causal mask (uniform test)
         if (st * 32 + 31 > start + t0) {
 #pragma unroll
@@ -213,16 +219,25 @@ __global__ __launch_bounds__(64 * G) void attn_prefill_kernel(
         }
     };
 
-    request(0);
-    stage(0);
-    request(1);
-    lds_barrier();
+    auto meet = [&] {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+#pragma unroll
+    for (int st = 0; st < RING - 1; ++st) request(st);
+    constexpr int kYounger = (RING - 2) * kLoads, kWait = 0x0f70 | (kYounger & 15) | ((kYounger >> 4) << 14);
+    __builtin_amdgcn_s_waitcnt(kWait);
+    meet();
     for (int st = 0; st < steps; ++st) {
-        step(st);
-        stage((st + 1) & 1);  // rows of step st + 1, requested a step ago, into the buffer that step st - 1 used
-        request(st + 2);
-        lds_barrier();
+        request(st + RING - 1);  // (the stage of step st - 1, which every wave has left; behind the rows: zeros)
+        v4f now[2];
+        scores(st, now);
+        step(st, now);
+        __builtin_amdgcn_s_waitcnt(kWait);
+        meet();
     }
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // nothing may arrive in LDS behind the workgroup's end
 
     const float l_tot = over_rows(l_run, [](float a, float b) { return a + b; });
     const float inv = 1.0f / l_tot;
@@ -518,12 +533,23 @@ extern "C" int bitnet_attn_prefill(const uint16_t* q, const uint16_t* cache_k, c
     if (!q || !cache_k || !cache_v || !out) return 2;
     if ((((uintptr_t)q) | ((uintptr_t)cache_k) | ((uintptr_t)cache_v) | ((uintptr_t)out)) & 15u) return 1;
     const dim3 grid((T + 15) / 16, n_kv_heads, B), block(64 * g, 1, 1);
+    // four steps of rows are 64 KB of LDS, so two workgroups to a CU; with more than that to do three steps and three
+    // workgroups (8 sequences of 512 tokens 40.4 -> 36.0 us; 512 tokens alone 12.0 against 12.4)
+    const bool many = (long long)grid.x * n_kv_heads * B > 2 * 256;
+#define BITNET_AP(G)                                                                                                                    \
+    if (many)                                                                                                                           \
+        hipLaunchKernelGGL((attn_prefill_kernel<G, 3>), grid, block, 3 * kApStepBytes, (hipStream_t)stream, q, cache_k, cache_v, out, T, S, \
+                           start, n_heads, n_kv_heads);                                                                                 \
+    else                                                                                                                                \
+        hipLaunchKernelGGL((attn_prefill_kernel<G, 4>), grid, block, 4 * kApStepBytes, (hipStream_t)stream, q, cache_k, cache_v, out, T, S, \
+                           start, n_heads, n_kv_heads)
     switch (g) {
-        case 1: hipLaunchKernelGGL(attn_prefill_kernel<1>, grid, block, 0, (hipStream_t)stream, q, cache_k, cache_v, out, T, S, start, n_heads, n_kv_heads); break;
-        case 2: hipLaunchKernelGGL(attn_prefill_kernel<2>, grid, block, 0, (hipStream_t)stream, q, cache_k, cache_v, out, T, S, start, n_heads, n_kv_heads); break;
-        case 4: hipLaunchKernelGGL(attn_prefill_kernel<4>, grid, block, 0, (hipStream_t)stream, q, cache_k, cache_v, out, T, S, start, n_heads, n_kv_heads); break;
-        default: hipLaunchKernelGGL(attn_prefill_kernel<8>, grid, block, 0, (hipStream_t)stream, q, cache_k, cache_v, out, T, S, start, n_heads, n_kv_heads); break;
+        case 1: BITNET_AP(1); break;
+        case 2: BITNET_AP(2); break;
+        case 4: BITNET_AP(4); break;
+        default: BITNET_AP(8); break;
     }
+#undef BITNET_AP
     return hipGetLastError() == hipSuccess ? 0 : 3;
 }
 

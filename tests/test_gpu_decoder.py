@@ -648,6 +648,23 @@ def test_norm_bitlinear_of_rows_that_are_not_finite(M, K, N):
 # The end-to-end workload at its real size: 30 layers, dim 2560, ffn 6912, 20 / 5 heads, vocabulary
 # 128256 (gpu/model.py:39-49), a 512-token seeded prompt, greedy decode (gpu/generate.py:264-288)
 # ---------------------------------------------------------------------------
+@pytest.mark.parametrize("T", [1, 31, 33, 64, 65, 97, 129, 161])
+@pytest.mark.parametrize("nh,nkv", [(1, 1), (4, 2), (20, 5), (16, 2)])
+def test_prompt_attention_of_many_sequences_equals_each_alone(nh, nkv, T):
+    """Rows of one to six steps through rings of three (more workgroups than twice the CUs) and of four steps; the cache rows
+    behind the prompt, which the ring's requests reach, hold NaNs."""
+    groups = (T + 15) // 16 * nkv
+    B, S = 512 // groups + 2, T + 40
+    gen = torch.Generator(device="cuda").manual_seed(T)
+    q = torch.randn(B, T, nh, 128, generator=gen, device="cuda").to(torch.bfloat16)
+    k, v = (torch.randn(B, S, nkv, 128, generator=gen, device="cuda").to(torch.bfloat16) for _ in range(2))
+    k[:, T:] = v[:, T:] = float("nan")
+    many = decoder.attn_prefill(q, k, v).view(B, T, -1)
+    for b in (0, B // 2, B - 1):
+        alone = decoder.attn_prefill(q[b : b + 1].contiguous(), k[b : b + 1].contiguous(), v[b : b + 1].contiguous())
+        assert not torch.isnan(alone).any() and torch.equal(alone, many[b])
+
+
 def _norm_and_linear(K, N, gen, segments=None):
     norm = decoder.RMSNorm(K, 1e-5).cuda().to(torch.bfloat16)
     norm.weight.data = torch.rand(K, generator=gen, device="cuda").add(0.5).to(torch.bfloat16)
