@@ -69,6 +69,37 @@ __device__ __forceinline__ int scale_slot_uniform(const ScaleMap& smap, int n) {
     return slot;
 }
 
+// The GEMM kernels' order of tiles.
+constexpr int kTileBand = 4;
+constexpr long long kMostTiles = 1ll << 24;  // 2^32 threads in a grid
+// Workgroup -> tile.  The tiles, band of kTileBand row tiles by band, column by column within a band, are cut into eight runs
+// of equal length, one per XCD (workgroups are handed to the XCDs round-robin): the workgroups of an XCD share a few row and
+// a few column tiles in its L2, and no XCD has more than one tile more than another.  (Whole bands per XCD leave XCDs idle
+// where the bands do not divide the row tiles: 600 x 13824 x 2560 37.6 us against 25.6, 1186 x 3200 x 10240 67.0 against
+// 44.3, 3000 x 3840 x 2560 35.5 against 29.3; where they do, level within 2 %.)  False: no tile (at most seven workgroups of
+// 8 * ceil(tiles / 8)).  The divisions stand before a workgroup's first load: one high product by `magic` (tile_magic), and
+// one by the reciprocal of 1 .. 4 (float reciprocals cost 0.07 us more per launch).
+__device__ __forceinline__ bool tile_of_workgroup(int w, int row_tiles, int col_tiles, unsigned magic, int& row_tile, int& col_tile) {
+    const int tiles = row_tiles * col_tiles, xcd = w & 7;
+    const int i = ((xcd * tiles) >> 3) + (w >> 3);
+    if (i >= ((xcd + 1) * tiles) >> 3) return false;
+    const int band_tiles = kTileBand * col_tiles;
+    const int band = magic ? (int)__umulhi((unsigned)i, magic) : i / band_tiles;
+    const int in_band = i - band * band_tiles;
+    const int band_rows = row_tiles - band * kTileBand;
+    col_tile = band_rows >= 4   ? in_band >> 2
+               : band_rows == 3 ? (int)__umulhi((unsigned)in_band, 0x55555556u)
+                                : in_band >> (band_rows - 1);
+    row_tile = band * kTileBand + in_band - col_tile * (band_rows < kTileBand ? band_rows : kTileBand);
+    return true;
+}
+// ceil(2^32 / d) divides n by d through the high product wherever n * d < 2^32; 0: the kernel divides
+unsigned tile_magic(long long row_tiles, long long col_tiles) {
+    const long long d = kTileBand * col_tiles;
+    if (d == 0) return 0;
+    return row_tiles * col_tiles < kMostTiles && row_tiles * col_tiles * d < (1ll << 32) ? (unsigned)(((1ll << 32) + d - 1) / d) : 0;
+}
+
 // Up to this many tokens a product goes through the kernels that keep the token rows in LDS or registers per
 // wave (the staged and the streaming kernel); beyond, through the kernels that split the tokens over MFMA columns
 constexpr int kDecodeMaxTokens = 4;
@@ -450,9 +481,8 @@ __global__ __launch_bounds__(kPfWaves * 64 * KS)
 __attribute__((amdgpu_waves_per_eu(MT == 2 && NT == 2 && KS == 1 ? 3 : (MT * NT == 8 && KS == 1 ? 2 : 1))))
 void gemm_i2_prefill_kernel(
     // parameter order: what the first loads need comes first (kernel-argument preload)
-    // (band and seg_cols repeat gridDim.x / 8 and gridDim.y: the grid's own size is not among the preloaded dwords)
-    const int8_t* __restrict__ act, const uint32_t* __restrict__ wq, int M, int N, int K, int nunits, int cseg_shift,
-    int band, int seg_cols, const uint16_t* __restrict__ s, uint16_t* __restrict__ out, int32_t* __restrict__ acc_out,
+    const int8_t* __restrict__ act, const uint32_t* __restrict__ wq, int M, int N, int K, int flags, int row_tiles, int col_tiles,
+    unsigned magic, const uint16_t* __restrict__ s, uint16_t* __restrict__ out, int32_t* __restrict__ acc_out,
     const uint16_t* __restrict__ ws, ScaleMap smap, const uint16_t* __restrict__ residual) {
     constexpr int TM = MT * 32;
     constexpr int NTHR = kPfWaves * 64;
@@ -471,28 +501,9 @@ void gemm_i2_prefill_kernel(
     const int tid = threadIdx.x % NTHR;
     const int lane = tid & 63;
     const int wave = tid >> 6;
-    // Workgroup -> tile.  Workgroups are handed to the 8 XCDs round-robin by
-    // linear id, and each XCD has its own L2.  The tile grid is cut into bands of
-    // `band` row tiles; a band belongs to one XCD (band b -> XCD b % 8), which
-    // walks it column tile by column tile.  The workgroups running on an XCD at
-    // any time therefore share a few row tiles (kept in that L2 for the whole
-    // band) and a few column tiles, instead of every tile pulling both of its
-    // operands through the memory-side cache on its own.  Unless the number of
-    // bands is a multiple of 8, the column tiles are cut into segments too, so
-    // that every XCD gets the same number of (band, segment) units.
-    // The grid spells the mapping out so that no division stands between the
-    // kernel's entry and its first load: x = XCD + 8 * (row tile within the
-    // band), y = column tile within the segment, z = round of 8 units (the
-    // linear workgroup id, which picks the XCD, is x + 8 * band * (y + ...)).
-    const int row_tiles = (M + TM - 1) / TM;
-    const int col_tiles = (N + kPfWaves * NT * 32 - 1) / (kPfWaves * NT * 32);
-    const int unit = (blockIdx.x & 7) + 8 * blockIdx.z;  // unit = (band, column segment) -> XCD unit % 8
-    if (unit >= nunits) return;
-    const bool has_out = (cseg_shift >> 8) != 0;  // bit 8 repeats out != nullptr (out itself is not among the preloaded dwords)
-    cseg_shift &= 0xff;
-    const int col_tile = (unit & ((1 << cseg_shift) - 1)) * seg_cols + blockIdx.y;
-    const int row_tile = (unit >> cseg_shift) * band + (blockIdx.x >> 3);
-    if (row_tile >= row_tiles || col_tile >= col_tiles) return;  // ragged last band / segment (uniform over the workgroup)
+    int row_tile, col_tile;
+    if (!tile_of_workgroup(blockIdx.x, row_tiles, col_tiles, magic, row_tile, col_tile)) return;  // (uniform over the workgroup)
+    const bool has_out = flags != 0;  // repeats out != nullptr (out itself is not among the preloaded dwords)
     const int m0 = row_tile * TM;
     const int n0 = (col_tile * kPfWaves + wave) * NT * 32;
     const int nl = lane & 31;
@@ -893,6 +904,8 @@ __device__ __forceinline__ void load16_to_lds(__amdgpu_buffer_rsrc_t rsrc, int8_
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)ldsp, 16, voff, soff, 0, 0);
 }
 
+#include "gemm_ring.h"
+
 // One output tile of (32 MT) rows x (WAVES x 32 NT) columns at (row_tile, column n_base) by the WAVES waves of the
 // calling workgroup (further waves of the workgroup must not enter).
 template <int MT, int NT, int CK, int WAVES>
@@ -1112,19 +1125,12 @@ constexpr int kPfxWaves = 4;
 template <int MT, int NT, int CK>
 __global__ __launch_bounds__(kPfxWaves * 64) __attribute__((amdgpu_waves_per_eu(MT * NT <= 4 ? 3 : 2)))
 void gemm_i2_prefill_dma_kernel(
-    const int8_t* __restrict__ act, const uint32_t* __restrict__ wq, int M, int N, int K, int nunits, int cseg_shift,
-    int band, int seg_cols, const uint16_t* __restrict__ s, uint16_t* __restrict__ out, int32_t* __restrict__ acc_out,
+    const int8_t* __restrict__ act, const uint32_t* __restrict__ wq, int M, int N, int K, int flags, int row_tiles, int col_tiles,
+    unsigned magic, const uint16_t* __restrict__ s, uint16_t* __restrict__ out, int32_t* __restrict__ acc_out,
     const uint16_t* __restrict__ ws, ScaleMap smap, const uint16_t* __restrict__ residual) {
-    // workgroup -> tile: as gemm_i2_prefill_kernel (bands of row tiles per XCD, column segments)
-    const int row_tiles = (M + MT * 32 - 1) / (MT * 32);
-    const int col_tiles = (N + kPfxWaves * NT * 32 - 1) / (kPfxWaves * NT * 32);
-    const int unit = (blockIdx.x & 7) + 8 * blockIdx.z;
-    if (unit >= nunits) return;
-    const bool has_out = (cseg_shift >> 8) != 0;
-    cseg_shift &= 0xff;
-    const int col_tile = (unit & ((1 << cseg_shift) - 1)) * seg_cols + blockIdx.y;
-    const int row_tile = (unit >> cseg_shift) * band + (blockIdx.x >> 3);
-    if (row_tile >= row_tiles || col_tile >= col_tiles) return;
+    const bool has_out = flags != 0;
+    int row_tile, col_tile;
+    if (!tile_of_workgroup(blockIdx.x, row_tiles, col_tiles, magic, row_tile, col_tile)) return;
     pfx_tile<MT, NT, CK, kPfxWaves>(act, wq, M, N, K, row_tile, col_tile * (kPfxWaves * NT * 32), has_out, s, out, acc_out, ws, smap,
                                     residual);
 }
@@ -1133,38 +1139,25 @@ void gemm_i2_prefill_dma_kernel(
 // (2048 x 2560: 320 tiles on 256 CUs -- a quarter of the CUs with two tiles, or three half-height tiles on half of them):
 // the first big_cols column tiles of 256 go to workgroups that take a 64 x 256 tile each, the columns behind them to
 // workgroups of which two waves take a 32 x 128 tile (a quarter of the work; the other two waves leave at once), so that
-// a CU holds one tile of each kind.  Workgroup w of a kind -> XCD w % 8 -> a band of row tiles of its own.
+// a CU holds one tile of each kind.  The tiles of a kind are dealt to the XCDs in equal runs (tile_of_workgroup).
 template <int CK>
 __global__ __launch_bounds__(kPfxWaves * 64) __attribute__((amdgpu_waves_per_eu(3)))
 void gemm_i2_prefill_mix_kernel(
     const int8_t* __restrict__ act, const uint32_t* __restrict__ wq, int M, int N, int K, int nbig, int big_cols, int flags,
-    int small_cols, const uint16_t* __restrict__ s, uint16_t* __restrict__ out, int32_t* __restrict__ acc_out,
+    int small_cols, unsigned big_magic, unsigned small_magic, const uint16_t* __restrict__ s, uint16_t* __restrict__ out, int32_t* __restrict__ acc_out,
     const uint16_t* __restrict__ ws, ScaleMap smap, const uint16_t* __restrict__ residual) {
     const bool has_out = (flags & 1) != 0;
     const int w = blockIdx.x;
+    int row_tile, col_tile;
     if (w < nbig) {
-        // 64-row tiles: XCD x takes a band of row tiles x * band .. and walks the columns (nbig = 8 * band * big_cols)
-        const int rt = (M + 63) >> 6;
-        const int band = (rt + 7) >> 3;
-        const int j = w >> 3;
-        const int row_tile = (w & 7) * band + j % band;
-        const int col_tile = j / band;
-        if (row_tile >= rt) return;  // a ragged last band
+        if (!tile_of_workgroup(w, (M + 63) >> 6, big_cols, big_magic, row_tile, col_tile)) return;
         pfx_tile<2, 2, CK, 4>(act, wq, M, N, K, row_tile, col_tile * 256, has_out, s, out, acc_out, ws, smap, residual);
     } else {
         if (threadIdx.x >= 128) return;
-        const int v = w - nbig;
-        const int rt = (M + 31) >> 5;
-        const int band = (rt + 7) >> 3;  // 32-row tiles per XCD
-        const int j = v >> 3;
-        const int row_tile = (v & 7) * band + j % band;
-        const int col_tile = j / band;
-        if (row_tile >= rt || col_tile >= small_cols) return;
+        if (!tile_of_workgroup(w - nbig, (M + 31) >> 5, small_cols, small_magic, row_tile, col_tile)) return;
         pfx_tile<1, 2, CK, 2>(act, wq, M, N, K, row_tile, big_cols * 256 + col_tile * 128, has_out, s, out, acc_out, ws, smap, residual);
     }
 }
-
-#include "gemm_ring.h"
 
 // ---------------------------------------------------------------------------
 // Per-token absmax quantizer: one workgroup per token row
@@ -2227,7 +2220,6 @@ struct Tuning {
     int path = 0;  // 0 = built-in choice, 2 = split-K kernel, 3 = fused shape, 4 = never fuse, 5 = GEMM tile
     int fused[3] = {1, 10, 4};
     int prefill_big = 0;
-    int prefill_band = 0;  // row tiles per band of the prefill GEMM's tile order, 0 = built-in choice
     int prefill_ks = 0;    // groups of waves splitting K in the small prefill tiles, 0 = built-in choice
     int staged = 0;        // product through the LDS-staged kernel: 0 = built-in choice, 1 = whenever it fits, 2 = never
     int stream = 0;        // product through the streaming kernel: 0 = built-in choice, 1 = whenever it applies, 2 = never
@@ -2954,7 +2946,7 @@ int launch_ring(int ring, const int8_t* act, const int8_t* packed, uint16_t* out
     const dim3 grid(8 * (unsigned)((tiles + 7) / 8), 1, 1);
 #define BITLINEAR_LAUNCH_RING(...)                                                                                                 \
     BL_LAUNCH((gemm_i2_prefill_kernel<__VA_ARGS__, Epi>), grid, dim3(Ring<__VA_ARGS__>::THREADS), (Ring<__VA_ARGS__>::LDS), stream, act, \
-              wq, M, N, K, (int)tiles, out || Epi::kRope ? 1 : 0, row_tiles, col_tiles, s, out, acc_out, ws, smap, residual, epi)
+              wq, M, N, K, out || Epi::kRope ? 1 : 0, row_tiles, col_tiles, tile_magic(row_tiles, col_tiles), s, out, acc_out, ws, smap, residual, epi)
     switch (ring) {
         case 1: BITLINEAR_LAUNCH_RING(BITLINEAR_RING_A); break;
         case 2: BITLINEAR_LAUNCH_RING(BITLINEAR_RING_B); break;
@@ -3016,11 +3008,10 @@ int launch_prefill(const int8_t* act, const int8_t* packed, uint16_t* out, int32
     // first columns, the columns behind them as 32 x 128 tiles.  Taken when those quarter tiles are at most about 1.4
     // per CU (measured, 64 x 256 tiles or half-height ones -> this: 2560 x 2560 at M = 2048 19.0 -> 17.3 us, at M = 3584
     // 28.5 -> 25.9, at 5120 39.4 -> 36.1; 2560 x 6912 41.0 -> 36.5 / 62.7 -> 57.3 / 91.4 -> 82.0; 3200 x 3200 at M = 1536
-    // 22.4 -> 20.1, 2560 33.0 -> 28.5, 5120 58.0 -> 49.9; with more of them the even tiles are ahead: 2560 x 2560 at
+    // 22.4 -> 20.1, 2560 33.0 -> 28.5, 5120 58.0 -> 49.9, 20480 x 3200 at M = 617 46.1 -> 43.6; with more of them the even tiles are ahead: 2560 x 2560 at
     // M = 2560 21.3 against 26.5, 3840 x 2560 at M = 2048 22.8 against 28.0)
     if (dma_fits && (t_tune.path == 0 || (t_tune.path == 5 && t_tune.prefill_big == 8))) {
         const int rt64 = (M + 63) / 64, rt32 = (M + 31) / 32;
-        const int band64 = (rt64 + 7) / 8, band32 = (rt32 + 7) / 8;
         const long long wide = (long long)((N + 255) / 256) * rt64;
         const int rounds = wide / kPrefillMixCus > 1 ? (int)(wide / kPrefillMixCus) : 1;
         int big_cols = (int)((long long)kPrefillMixCus * rounds / rt64);
@@ -3028,17 +3019,18 @@ int launch_prefill(const int8_t* act, const int8_t* packed, uint16_t* out, int32
         const int small_cols = (N - big_cols * 256 + 127) / 128;
         const long long quarters = (long long)rt32 * small_cols;
         const bool wanted = t_tune.path == 5 || (wide > kPrefillMixCus && big_cols >= 1 && quarters > 0 && quarters <= kPrefillMixMaxQuarters);
-        const long long groups = 8ll * band64 * big_cols + 8ll * band32 * small_cols;
-        if (wanted && rt64 <= 4096 && groups < (1ll << 30)) {
-            const int nbig = 8 * band64 * big_cols;
+        const long long bigs = (long long)rt64 * big_cols;
+        const long long groups = 8 * ((bigs + 7) / 8) + 8 * ((quarters + 7) / 8);
+        if (wanted && groups < kMostTiles) {
+            const int nbig = 8 * (int)((bigs + 7) / 8);
             const dim3 mgrid((unsigned)groups, 1, 1), mblock(256, 1, 1);
             g_last_kernel = "gemm_i2_prefill_mix_kernel";
             if (K % 256 == 0)
                 BL_LAUNCH((gemm_i2_prefill_mix_kernel<256>), mgrid, mblock, 3 * 64 * 256, stream, act, wq, M, N, K, nbig, big_cols,
-                          out ? 1 : 0, small_cols, s, out, acc_out, ws, smap, residual);
+                          out ? 1 : 0, small_cols, tile_magic(rt64, big_cols), tile_magic(rt32, small_cols), s, out, acc_out, ws, smap, residual);
             else
                 BL_LAUNCH((gemm_i2_prefill_mix_kernel<128>), mgrid, mblock, 3 * 64 * 128, stream, act, wq, M, N, K, nbig, big_cols,
-                          out ? 1 : 0, small_cols, s, out, acc_out, ws, smap, residual);
+                          out ? 1 : 0, small_cols, tile_magic(rt64, big_cols), tile_magic(rt32, small_cols), s, out, acc_out, ws, smap, residual);
             return launch_status();
         }
     }
@@ -3091,37 +3083,20 @@ int launch_prefill(const int8_t* act, const int8_t* packed, uint16_t* out, int32
     if (t_tune.path == 5 && t_tune.prefill_ks > 0) ks = (tile == 4 || ((tile == 0 || tile == 2) && t_tune.prefill_ks == 2)) ? t_tune.prefill_ks : 1;
     if (K <= kPfChunk * (ks - 1)) ks = 1;  // fewer chunks than groups
     const dim3 block(kPfWaves * 64 * ks, 1, 1);
-    // grid of 8 XCDs x bands per XCD x tiles per band (see the kernel); bands of up to 8 row
-    // tiles, fewer when there are not enough row tiles to give every XCD a band
     if (tile == 8 && !dma_fits) tile = 4;
     const int tm = tile == 1 ? 128 : ((tile == 4 || tile == 8) ? 32 : 64);
     const int tn = (tile == 0 || tile == 4) ? 128 : (tile == 3 ? 512 : 256);
     const int row_tiles = (M + tm - 1) / tm, col_tiles = (N + tn - 1) / tn;
-    int band = row_tiles / 8;
-    band = band < 1 ? 1 : (band > 8 ? 8 : band);
-    if (t_tune.path == 5 && t_tune.prefill_band > 0) band = t_tune.prefill_band;
-    const int nbands = (row_tiles + band - 1) / band;
-    // the columns are cut into segments as well, as many as it takes for the number of (band,
-    // segment) units to be a multiple of the 8 XCDs: every XCD then gets the same number of units
-    // (3 bands x 3 segments left one XCD with two units and the others with one: M = 96 took longer
-    // than M = 128)
-    int g8 = nbands & 7;
-    g8 = g8 == 0 ? 8 : (g8 & -g8);  // gcd(nbands, 8)
-    int cseg_shift = g8 == 8 ? 0 : (g8 == 4 ? 1 : (g8 == 2 ? 2 : 3));  // 8 / g8 segments, a power of two
-    while ((1 << cseg_shift) > col_tiles) --cseg_shift;
-    const int cseg = 1 << cseg_shift;
-    const int seg_cols = (col_tiles + cseg - 1) / cseg;
-    const int units = nbands * cseg;
-    // x = XCD + 8 * (row tile within the band), y = column tile within the segment, z = round of 8
-    // units: the same order of workgroups as a linear grid, without divisions in the kernel
-    if (seg_cols > 65535 || (units + 7) / 8 > 65535) return BITLINEAR_ERR_SHAPE;
-    const dim3 grid(8 * band, seg_cols, (units + 7) / 8);
+    const long long tiles = (long long)row_tiles * col_tiles;
+    const unsigned magic = tile_magic(row_tiles, col_tiles);
+    if (tiles * ks >= kMostTiles) return BITLINEAR_ERR_SHAPE;
+    const dim3 grid(8 * (unsigned)((tiles + 7) / 8), 1, 1);  // dealt to the XCDs by tile_of_workgroup
 #define BITLINEAR_LAUNCH_PF(MT_, NT_, KS_)                                                                          \
     BL_LAUNCH((gemm_i2_prefill_kernel<MT_, NT_, KS_>), grid, block, KS_ * 2 * 32 * MT_ * kPfRowBytes, stream, \
-                       act, wq, M, N, K, units, cseg_shift | (out ? 256 : 0), band, seg_cols, s, out, acc_out, ws, smap, residual)
+                       act, wq, M, N, K, out ? 1 : 0, row_tiles, col_tiles, magic, s, out, acc_out, ws, smap, residual)
 #define BITLINEAR_LAUNCH_PFX(MT_, CK_)                                                                                   \
-    BL_LAUNCH((gemm_i2_prefill_dma_kernel<MT_, 2, CK_>), grid, block, 3 * 32 * MT_ * CK_, stream, act, wq, M, N, K, units, \
-              cseg_shift | (out ? 256 : 0), band, seg_cols, s, out, acc_out, ws, smap, residual)
+    BL_LAUNCH((gemm_i2_prefill_dma_kernel<MT_, 2, CK_>), grid, block, 3 * 32 * MT_ * CK_, stream, act, wq, M, N, K, out ? 1 : 0, \
+              row_tiles, col_tiles, magic, s, out, acc_out, ws, smap, residual)
     if (dma && dma_fits && ks == 1 && (tile == 8 || (tile == 1 && dma_mt == 4))) {
         g_last_kernel = "gemm_i2_prefill_dma_kernel";
         if (tile == 8) {
@@ -3552,7 +3527,6 @@ int bitlinear_set_tuning(int kernel, int a, int b, int c) {
         if (a < 0 || a > 12 || b < 0 || b > 64 || (c != 0 && c != 1 && c != 2 && c != 4)) return set_status(BITLINEAR_ERR_ARG);
         g.path = 5;
         g.prefill_big = a;
-        g.prefill_band = b;
         g.prefill_ks = c;
         return set_status(BITLINEAR_OK);
     }

@@ -48,13 +48,6 @@ struct Ring {
     static_assert(S >= 4 && (S - 1) * LOADS <= 63, "loads in flight are counted in six bits");
     static_assert(LDS + TM * 8 + 64 <= 160 * 1024, "LDS of a CU");
 };
-constexpr int kRingBand = 4;
-// n / d for 0 <= n < 2^22, d >= 1, of wave-uniform values
-__device__ __forceinline__ int ring_div(int n, int d) {
-    int q = (int)((float)n * __builtin_amdgcn_rcpf((float)d));
-    q += (n - q * d >= d ? 1 : 0) - (n - q * d < 0 ? 1 : 0);
-    return __builtin_amdgcn_readfirstlane(q);
-}
 // What becomes of the outputs: what follows a prompt's product is a launch and a trip of its rows through memory less (in a
 // layer of a 512-token prompt rope and cache write 5.8 us beside the GEMM's 8.4, together 9.5; the gate's output is half of
 // what w13 wrote, 22 -> 20.9, and the norm behind it reads half, 6.0 -> 5.4).  RingPlain: rows of `out`, with the residual added if there is one.
@@ -85,8 +78,8 @@ constexpr int kRingBeyond = 0x7ffffff0;  // an offset behind every descriptor: n
 template <int MT, int NT, int WM, int WN, int KG, int CK, int S, int LW, class Epi>
 __global__ __launch_bounds__(64 * (WM * WN * KG + LW)) __attribute__((amdgpu_waves_per_eu((WM * WN * KG + LW) * Ring<MT, NT, WM, WN, KG, CK, S, LW>::WGS / 4)))
 void gemm_i2_prefill_kernel(
-    const int8_t* __restrict__ act, const uint32_t* __restrict__ wq, int M, int N, int K, int ntiles, int flags,
-    int row_tiles, int col_tiles, const uint16_t* __restrict__ s, uint16_t* __restrict__ out, int32_t* __restrict__ acc_out,
+    const int8_t* __restrict__ act, const uint32_t* __restrict__ wq, int M, int N, int K, int flags,
+    int row_tiles, int col_tiles, unsigned magic, const uint16_t* __restrict__ s, uint16_t* __restrict__ out, int32_t* __restrict__ acc_out,
     const uint16_t* __restrict__ ws, ScaleMap smap, const uint16_t* __restrict__ residual, const Epi epi) {
     typedef Ring<MT, NT, WM, WN, KG, CK, S, LW> R;
     constexpr int QR = 8 / NT;
@@ -94,17 +87,8 @@ void gemm_i2_prefill_kernel(
     static_assert(!Epi::kGate || NT == 2, "a column tile of either half");
     extern __shared__ __attribute__((aligned(1024))) int8_t lds_x[];
 
-    // Workgroup -> tile.  The tiles, band of kRingBand row tiles by band, column by column within a band, are cut into
-    // eight runs of equal length, one per XCD (workgroups are handed to the XCDs round-robin): the workgroups of an XCD
-    // share a few row and a few column tiles in its L2, and no XCD has more than one tile more than another.
-    const int xcd = blockIdx.x & 7;
-    const int i = (int)(((long long)xcd * ntiles) >> 3) + (int)(blockIdx.x >> 3);
-    if (i >= (int)(((long long)(xcd + 1) * ntiles) >> 3)) return;
-    const int band = ring_div(i, kRingBand * col_tiles);
-    const int in_band = i - band * (kRingBand * col_tiles);
-    const int band_rows = row_tiles - band * kRingBand < kRingBand ? row_tiles - band * kRingBand : kRingBand;
-    const int col_tile = ring_div(in_band, band_rows);
-    const int row_tile = band * kRingBand + in_band - col_tile * band_rows;
+    int row_tile, col_tile;
+    if (!tile_of_workgroup(blockIdx.x, row_tiles, col_tiles, magic, row_tile, col_tile)) return;
     const bool has_out = flags != 0;  // repeats out != nullptr
 
     const int lane = threadIdx.x & 63;

@@ -356,8 +356,8 @@ int bitlinear_plan_name(int entry, int M, int N, int K, char* buf, int buflen);
  *             K % 128 == 0), 9 .. 12 = 32 x 64, 64 x 128, 64 x 256 and 128 x 256 through
  *             the kernel that brings activations and weights through LDS (the built-in
  *             choice while there is about one such tile per CU; needs K % 128 == 0, else
- *             as 5; neither b nor c applies); b = row tiles per band of the tile order (0 = the
- *             library's choice, up to 64); c = groups of four waves that split a
+ *             as 5; c does not apply); b = without effect (0 .. 64; the order of
+ *             tiles is one for all sizes); c = groups of four waves that split a
  *             tile's K between them (0 = the library's choice, 1, 2 (tiles 0 and 4)
  *             or 4 (tile 4))
  *   kernel 6: product of int8 rows (M <= 16) through the kernel that stages

@@ -666,6 +666,22 @@ def test_prefill_gemm_acc_bit_exact(m, n, k, tile):
     assert np.array_equal(acc.cpu().numpy(), o.acc_int32(a, w))
 
 
+@pytest.mark.parametrize("tile", [0, 1, 2, 4, 5, 6, 7, 8, 9, 10, 11, 12])
+@pytest.mark.parametrize("m,n,k", [(17, 16, 128), (1500, 16, 128), (40, 4112, 256), (700, 1296, 256), (1100, 2576, 128)])
+def test_prefill_gemm_deals_out_every_tile(m, n, k, tile):
+    """The order of tiles (eight runs of bands of four row tiles) in each GEMM kernel: one tile, one column or one row of
+    tiles, fewer tiles than XCDs, last bands of one, two and three row tiles, runs of unequal length -- accumulators equal
+    to the oracle's."""
+    lib = _lib.load_library()
+    w, a = _rand_case(n, k, m, seed=m + n + k)
+    try:
+        assert lib.bitlinear_set_tuning(5, tile, 0, 0) == 0
+        acc = bitlinear.bitnet_int8xint2_acc(dev_i8(a), _packed_dev(w))
+    finally:
+        lib.bitlinear_set_tuning(0, 0, 0, 0)
+    assert np.array_equal(acc.cpu().numpy(), o.acc_int32(a, w))
+
+
 @pytest.mark.parametrize("tile,ks", [(4, 2), (4, 4), (0, 2), (2, 2)])
 @pytest.mark.parametrize("m,n,k", [(17, 48, 192), (64, 128, 64), (100, 272, 320), (128, 2560, 2560), (33, 3840, 2560),
                                    (300, 1040, 3200), (512, 2560, 6912), (70, 256, 768), (40, 512, 1024)])
