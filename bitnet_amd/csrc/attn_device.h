@@ -8,6 +8,8 @@
 #include <math.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "bitlinear_device.h"
 
 namespace {
@@ -60,28 +62,68 @@ struct DfState {
     }
 };
 
-// One block of 32 cache rows (positions 32 blk ..): scores, softmax and P.V for the heads in the columns of qa.
-// kb[bi][kk]: dims 32 kk + 8 g4 .. of row 16 bi + c; vb[jj]: dims 8 c .. of row 4 g4 + (jj & 3) + 16 (jj >> 2).  The
-// row of the new token (position p) is not in the cache yet: it comes from LDS (knew, vnew).
-__device__ __forceinline__ void df_block(v4u (&kb)[2][4], v4u (&vb)[8], const v8bf (&qa)[4], const uint16_t* knew,
-                                         const uint16_t* vnew, int blk, int p, int lane, DfState& st) {
-    const int c = lane & 15, g4 = lane >> 4;
-    if (blk == p >> 5) {
+// What follows is bound by the number of instructions of one wave, not by memory: V rows are turned where a caller waits
+// anyway, masks and the new row only in the block that needs them, results stored as the registers hold them, and the
+// caller's own record added behind the others without selects (a step of 12 sequences at 512 positions, where
+// attn_decode_flash_kernel runs 30 times: 1440 -> 1348 us).
+
+// A block of 32 cache rows (positions 32 blk ..) as loaded: kb[bi][kk], dims 32 kk + 8 g4 .. of row 16 bi + c; vb[jj], dims
+// 8 c .. of row 4 g4 + (jj & 3) + 16 (jj >> 2).  df_block wants the V rows turned (df_turn); in the block of the new
+// token's position p the rows behind p are cleared in front of that, and row p, which is not in the cache yet, is put in:
+// k by df_new_key, v (dims 8 c ..) by df_block.
+
+// V rows behind the position: their probability is zero, but whatever the cache holds there (it may never have been
+// written) must not reach the product as 0 x NaN
+__device__ __forceinline__ void df_clear(v4u (&vb)[8], int p, int lane) {
+    const int last = (p & 31) - 4 * (lane >> 4);
 #pragma unroll
-        for (int bi = 0; bi < 2; ++bi)
-            if (blk * 32 + bi * 16 + c == p) {
+    for (int jj = 0; jj < 8; ++jj)
+        if ((jj & 3) + (jj >> 2) * 16 > last) vb[jj] = v4u{0u, 0u, 0u, 0u};
+}
+// vb[t] becomes the operand of output dims 8 j + t of P.V: eight rows of one dim per lane
+__device__ __forceinline__ void df_turn(v4u (&vb)[8]) {
+    v4u va[8];
 #pragma unroll
-                for (int kk = 0; kk < 4; ++kk) kb[bi][kk] = *(const v4u*)(knew + kk * 32 + g4 * 8);
-            }
-        // V rows behind the position are cleared: their probability is zero, but whatever the
-        // cache holds there (it may never have been written) must not reach the product as 0 x NaN
-#pragma unroll
-        for (int jj = 0; jj < 8; ++jj) {
-            const int r = blk * 32 + (jj & 3) + (jj >> 2) * 16 + 4 * g4;
-            if (r == p) vb[jj] = *(const v4u*)(vnew + c * 8);
-            if (r > p) vb[jj] = v4u{0u, 0u, 0u, 0u};
-        }
+    for (int t = 0; t < 8; ++t) {
+        const uint32_t sel = (t & 1) ? 0x07060302u : 0x05040100u;
+        va[t].x = __builtin_amdgcn_perm(vb[1][t >> 1], vb[0][t >> 1], sel);
+        va[t].y = __builtin_amdgcn_perm(vb[3][t >> 1], vb[2][t >> 1], sel);
+        va[t].z = __builtin_amdgcn_perm(vb[5][t >> 1], vb[4][t >> 1], sel);
+        va[t].w = __builtin_amdgcn_perm(vb[7][t >> 1], vb[6][t >> 1], sel);
     }
+#pragma unroll
+    for (int t = 0; t < 8; ++t) vb[t] = va[t];
+}
+
+// Row p of K, from LDS
+__device__ __forceinline__ void df_new_key(v4u (&kb)[2][4], const uint16_t* knew, int p, int lane) {
+    const int c = lane & 15, g4 = lane >> 4;
+#pragma unroll
+    for (int bi = 0; bi < 2; ++bi)
+        if (bi * 16 + c == (p & 31)) {
+#pragma unroll
+            for (int kk = 0; kk < 4; ++kk) kb[bi][kk] = *(const v4u*)(knew + kk * 32 + g4 * 8);
+        }
+}
+// Row p of V: of turned rows it is a half-word of one of four words, in the operands of a quarter of the lanes.  All words
+// are permuted, by selectors that leave the others as they are: branches on the word copy registers.
+__device__ __forceinline__ void df_new_value(v4u (&va)[8], const v4u& vn, int p, int lane) {
+    const int r = p & 31;
+    const bool mine = lane >> 4 == ((r >> 2) & 3);
+    const uint32_t even = r & 1 ? 0x05040100u : 0x03020504u, odd = r & 1 ? 0x07060100u : 0x03020706u, as_it_is = 0x03020100u;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        const bool here = w == ((r & 3) + (r >> 4) * 4) >> 1;
+        const uint32_t sel[2] = {mine ? (here ? even : as_it_is) : as_it_is, mine ? (here ? odd : as_it_is) : as_it_is};
+#pragma unroll
+        for (int t = 0; t < 8; ++t) va[t][w] = __builtin_amdgcn_perm(vn[t >> 1], va[t][w], sel[t & 1]);
+    }
+}
+
+// Scores, softmax and P.V of one block for the heads in the columns of qa
+__device__ __forceinline__ void df_block(const v4u (&kb)[2][4], v4u (&va)[8], const v4u& vn, const v8bf (&qa)[4], int blk, int p, int lane,
+                                         DfState& st) {
+    const int g4 = lane >> 4;
     float sc[8];
 #pragma unroll
     for (int bi = 0; bi < 2; ++bi) {
@@ -90,10 +132,13 @@ __device__ __forceinline__ void df_block(v4u (&kb)[2][4], v4u (&vb)[8], const v8
         for (int kk = 0; kk < 4; ++kk)
             acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, kb[bi][kk]), qa[kk], acc, 0, 0, 0);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int pos = blk * 32 + bi * 16 + 4 * g4 + j;
-            sc[bi * 4 + j] = pos <= p ? acc[j] : -INFINITY;
-        }
+        for (int j = 0; j < 4; ++j) sc[bi * 4 + j] = acc[j];
+    }
+    if (blk == p >> 5) {  // (every other block is in the cache, and visible, as a whole)
+        df_new_value(va, vn, p, lane);  // (while the matrix pipe has the scores)
+        const int last = (p & 31) - 4 * g4;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) sc[i] = (i & 3) + (i >> 2) * 16 <= last ? sc[i] : -INFINITY;
     }
     float mx = fmaxf(fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3])), fmaxf(fmaxf(sc[4], sc[5]), fmaxf(sc[6], sc[7])));
     mx = over_rows(mx, [](float a, float b) { return fmaxf(a, b); });
@@ -123,21 +168,16 @@ __device__ __forceinline__ void df_block(v4u (&kb)[2][4], v4u (&vb)[8], const v8
     pw.w = pack_bf16x2(pr[6], pr[7]);
     const v8bf pb = __builtin_bit_cast(v8bf, pw);
 #pragma unroll
-    for (int t = 0; t < 8; ++t) {
-        const uint32_t sel = (t & 1) ? 0x07060302u : 0x05040100u;
-        v4u va;
-        va.x = __builtin_amdgcn_perm(vb[1][t >> 1], vb[0][t >> 1], sel);
-        va.y = __builtin_amdgcn_perm(vb[3][t >> 1], vb[2][t >> 1], sel);
-        va.z = __builtin_amdgcn_perm(vb[5][t >> 1], vb[4][t >> 1], sel);
-        va.w = __builtin_amdgcn_perm(vb[7][t >> 1], vb[6][t >> 1], sel);
-        st.o_acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, va), pb, st.o_acc[t], 0, 0, 0);
-    }
+    for (int t = 0; t < 8; ++t) st.o_acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, va[t]), pb, st.o_acc[t], 0, 0, 0);
 }
 
+// A head's outputs of one wave in LDS: output 32 g4 + 8 j + t at 32 g4 + 4 t + j, as a lane has them in registers; the rows
+// four banks apart, so that the heads' stores do not meet in one
+constexpr int kDfOutRow = kHeadDim + 4;
 // The wave's result for head c (lanes c < G) -> LDS: maximum (-inf, with a sum of 0, for a wave without visible
-// positions), sum over its positions, 32 outputs per lane.
+// positions), sum over its positions, 32 outputs per lane
 template <int G>
-__device__ __forceinline__ void df_wave_result(const DfState& st, int lane, float (*part_o)[kHeadDim], float* part_m,
+__device__ __forceinline__ void df_wave_result(const DfState& st, int lane, float (*part_o)[kDfOutRow], float* part_m,
                                                float* part_l) {
     const int c = lane & 15, g4 = lane >> 4;
     const float l_tot = over_rows(st.l_run, [](float a, float b) { return a + b; });
@@ -147,9 +187,7 @@ __device__ __forceinline__ void df_wave_result(const DfState& st, int lane, floa
             part_l[c] = l_tot;
         }
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int t = 0; t < 8; ++t) part_o[c][32 * g4 + 8 * j + t] = st.o_acc[t][j];
+        for (int t = 0; t < 8; ++t) *(v4f*)&part_o[c][32 * g4 + 4 * t] = st.o_acc[t];
     }
 }
 
@@ -158,43 +196,44 @@ struct DfPartial {
     float o0, o1, mx, l;
 };
 
-// One head over the workgroup's waves
-template <int G>
-__device__ __forceinline__ DfPartial df_combine(const float (*part_o)[G][kHeadDim], const float (*part_m)[G],
-                                                const float (*part_l)[G], int hh, int nwaves, int lane) {
+// One head over the results of N waves, of which the first n are there (ALL: every one)
+template <int G, int N, bool ALL>
+__device__ __forceinline__ DfPartial df_combine(const float (*part_o)[G][kDfOutRow], const float (*part_m)[G],
+                                                const float (*part_l)[G], int hh, int n, int lane) {
     DfPartial h = {0.0f, 0.0f, -INFINITY, 0.0f};
-    static_assert(kDfMaxWaves == 8, "two batches");
-    float m[8], l[8];
-    f32x2_t o[8];
+    static_assert(N == 4 || N == 8, "one or two batches");
+    const int at0 = 32 * (lane >> 4) + 8 * (lane & 3) + ((lane >> 2) & 3);  // of output 2 lane; 2 lane + 1 four behind
+    float m[N], l[N], o0[N], o1[N];
     // all values are requested together: left to itself the compiler waits for one wave's before the next one's.
     // A wave without visible positions adds nothing (by selects: branches cost more than what they skip).
     auto request = [&](int k0) {
 #pragma unroll
         for (int k = k0; k < k0 + 4; ++k) {
-            const int at = k < nwaves ? k : 0;
+            const int at = ALL || k < n ? k : 0;
             m[k] = part_m[at][hh];
             l[k] = part_l[at][hh];
-            o[k] = *(const f32x2_t*)&part_o[at][hh][2 * lane];
+            o0[k] = part_o[at][hh][at0];
+            o1[k] = part_o[at][hh][at0 + 4];
         }
 #pragma unroll
         for (int k = k0; k < k0 + 4; ++k) {
-            asm volatile("" : "+v"(m[k]), "+v"(l[k]), "+v"(o[k]));
+            asm volatile("" : "+v"(m[k]), "+v"(l[k]), "+v"(o0[k]), "+v"(o1[k]));
             h.mx = fmaxf(h.mx, m[k]);
         }
     };
     auto add = [&](int k0) {
 #pragma unroll
         for (int k = k0; k < k0 + 4; ++k) {
-            const float w = k < nwaves && l[k] > 0.0f ? __builtin_amdgcn_exp2f((m[k] - h.mx) * kDfC2) : 0.0f;
+            const float w = (ALL || k < n) && l[k] > 0.0f ? __builtin_amdgcn_exp2f((m[k] - h.mx) * kDfC2) : 0.0f;
             h.l += l[k] * w;
-            h.o0 += w * o[k].x;
-            h.o1 += w * o[k].y;
+            h.o0 += w * o0[k];
+            h.o1 += w * o1[k];
         }
     };
     request(0);
-    if (nwaves > 4) request(4);
+    if (N > 4) request(4);
     add(0);
-    if (nwaves > 4) add(4);
+    if (N > 4) add(4);
     return h;
 }
 
@@ -243,31 +282,33 @@ __device__ __forceinline__ DfPartial df_merge(const unsigned long long* rec, int
             }
         }
         gave_up = gave_up || !complete;
+        // records here (those behind them repeat the first split's, which does not change a maximum); then, in the
+        // last batch, the caller's
+        const int there = nact - 1 - k0;
+        const float own_mx = own.mx * kDfScale;
+        float bm = there < kBatch ? fmaxf(h.mx, own_mx) : h.mx;
 #pragma unroll
-        for (int k = 0; k < kBatch; ++k)
-            if (k0 + k == nact - 1) {
-                ml[k].x = __float_as_uint(own.mx * kDfScale);
-                ml[k].z = __float_as_uint(own.l);
-                oo[k].x = __float_as_uint(own.o0);
-                oo[k].z = __float_as_uint(own.o1);
-            }
-        float bm = h.mx;
-#pragma unroll
-        for (int k = 0; k < kBatch; ++k)
-            if (k0 + k < nact) bm = fmaxf(bm, __uint_as_float(ml[k].x));
-        const float wold = h.l > 0.0f ? __expf(h.mx - bm) : 0.0f;
-        h.l *= wold;
-        h.o0 *= wold;
-        h.o1 *= wold;
-        h.mx = bm;
-#pragma unroll
-        for (int k = 0; k < kBatch; ++k) {
-            const float lk = __uint_as_float(ml[k].z);
-            const float w = k0 + k < nact && lk > 0.0f ? __expf(__uint_as_float(ml[k].x) - h.mx) : 0.0f;
-            h.l += lk * w;
-            h.o0 += w * __uint_as_float(oo[k].x);
-            h.o1 += w * __uint_as_float(oo[k].z);
+        for (int k = 0; k < kBatch; ++k) bm = fmaxf(bm, __uint_as_float(ml[k].x));
+        if (k0) {
+            const float wold = h.l > 0.0f ? __expf(h.mx - bm) : 0.0f;
+            h.l *= wold;
+            h.o0 *= wold;
+            h.o1 *= wold;
         }
+        h.mx = bm;
+        float w[kBatch + 1];
+#pragma unroll
+        for (int k = 0; k < kBatch; ++k) w[k] = __uint_as_float(ml[k].z) > 0.0f ? __expf(__uint_as_float(ml[k].x) - bm) : 0.0f;
+        w[kBatch] = own.l > 0.0f ? __expf(own_mx - bm) : 0.0f;
+        auto add = [&](float l, float o0, float o1, float w) {
+            h.l += l * w;
+            h.o0 += w * o0;
+            h.o1 += w * o1;
+        };
+#pragma unroll
+        for (int k = 0; k < kBatch; ++k)
+            if (k < there) add(__uint_as_float(ml[k].z), __uint_as_float(oo[k].x), __uint_as_float(oo[k].z), w[k]);
+        if (there < kBatch) add(own.l, own.o0, own.o1, w[kBatch]);
     }
     return h;
 }

@@ -282,7 +282,7 @@ __global__ __launch_bounds__(kDfMaxWaves * 64) void attn_decode_flash_kernel(
     __shared__ __attribute__((aligned(16))) uint16_t qb[G][kHeadDim];  // rotated q as bf16
     __shared__ __attribute__((aligned(16))) uint16_t knew[kHeadDim];   // rotated k of the new token
     __shared__ __attribute__((aligned(16))) uint16_t vnew[kHeadDim];
-    __shared__ __attribute__((aligned(16))) float part_o[kDfMaxWaves][G][kHeadDim];
+    __shared__ __attribute__((aligned(16))) float part_o[kDfMaxWaves][G][kDfOutRow];
     __shared__ float part_m[kDfMaxWaves][G], part_l[kDfMaxWaves][G];
 
     const int tid = threadIdx.x;
@@ -402,7 +402,10 @@ __global__ __launch_bounds__(kDfMaxWaves * 64) void attn_decode_flash_kernel(
     DfState st;
     for (int blk = blk0; blk <= pblk; blk += blk_stride) {
         if (blk != blk0) load_rows(blk);
-        df_block(kb, vb, qa, knew, vnew, blk, p, lane, st);
+        if (blk == pblk) df_clear(vb, p, lane);
+        df_turn(vb);
+        if (blk == pblk) df_new_key(kb, knew, p, lane);
+        df_block(kb, vb, *(const v4u*)(vnew + c * 8), qa, blk, p, lane, st);
     }
     df_wave_result<G>(st, lane, part_o[wave], part_m[wave], part_l[wave]);
     __syncthreads();
@@ -424,7 +427,8 @@ __global__ __launch_bounds__(kDfMaxWaves * 64) void attn_decode_flash_kernel(
     // becomes NaN and the workspace's error word is set (it stays set; the host reads it, see
     // bitnet_attn_decode_error_index).
     for (int hh = wave; hh < G; hh += nwaves) {
-        DfPartial h = df_combine<G>(part_o, part_m, part_l, hh, nwaves, lane);
+        DfPartial h = nwaves <= 4 ? df_combine<G, 4, false>(part_o, part_m, part_l, hh, nwaves, lane)
+                                 : df_combine<G, 8, false>(part_o, part_m, part_l, hh, nwaves, lane);
         if (nact > 1 && !merger) {
             df_store_record(rec + ((size_t)sp * G + hh) * kDfRecUnits, tag, h, lane);
             continue;

@@ -283,6 +283,14 @@ struct RowRecord {
 };
 static_assert(sizeof(RowRecord) == 32 && kStWaves == 4, "one 16-byte and one 4-byte load");
 
+// what the waves of an attention task found, in the task's words buffer
+struct WaveResults {
+    float o[kDfMaxWaves][kStMaxG][kDfOutRow];
+    float m[kDfMaxWaves][kStMaxG], l[kDfMaxWaves][kStMaxG];
+};
+static_assert(sizeof(WaveResults) <= kStWordBytes, "");
+constexpr int kStRow = kHeadDim + 8;  // so that the heads' pieces of 16 bytes do not meet in one bank
+
 template <int MT>
 struct Shared {
     static constexpr int TQ = MT <= kStDirect ? MT : 1;  // rows that a task normalises
@@ -292,8 +300,8 @@ struct Shared {
     // the waves' partial sums: [row block][wave][token][row].  Twice where nothing else keeps a wave from writing the
     // next task's while another still reads
     int red[MT <= kStDirect ? 1 : 2][4][kStWaves][MT][16];
-    float part_m[kDfMaxWaves][kStMaxG], part_l[kDfMaxWaves][kStMaxG];
-    __attribute__((aligned(16))) uint16_t qb[kStMaxG][kHeadDim], knew[kHeadDim], vnew[kHeadDim];
+    // each wave's copy of an attention task's new rows: the q heads of the group, k, v
+    __attribute__((aligned(16))) uint16_t rows[kStWaves][kStMaxG + 2][kStRow];
     // exchanges between the computing waves: values with the number of the exchange
     // (the first in two buffers: a wave may be a task ahead of one that has not looked yet, not two)
     __attribute__((aligned(16))) v4i sumsq[2][TQ][kStWaves];
@@ -939,35 +947,56 @@ struct Stack {
     // --- attention: rope, cache write and one split of one (sequence, kv head) ------------------------
     // (attn_decode_flash_kernel's work on published rows; the last active split merges)
     struct Place {
-        int G, kvh, sp, b, p, pblk, nact;
+        int G, kvh, sp, b, p, pblk, nact, busy, n_heads, n_kv, nsplit, attn_waves;
+        unsigned tag;              // of this task's records
+        unsigned long long *rec, *own;  // of its (sequence, kv head), and of its split
+        uint32_t* out;
     };
     __device__ __forceinline__ Place attention_place(const Task& tk) const {
         Place w;
         w.G = a->group;
+        w.n_heads = a->n_heads;
+        w.n_kv = a->n_kv;
+        w.nsplit = a->n_splits;
+        w.attn_waves = a->attn_waves;
         w.kvh = tk.K;
         w.b = tk.n_out;
         w.sp = (int)__float_as_uint(tk.inv_k);
         w.p = tk.flags;
         w.pblk = w.p >> 5;
-        w.nact = w.pblk + 1 < a->n_splits ? w.pblk + 1 : a->n_splits;
+        w.nact = w.pblk + 1 < w.nsplit ? w.pblk + 1 : w.nsplit;
+        // the split's blocks are dealt to attn_waves waves in turn: this many of them have one
+        const int blocks = uniform((w.pblk - w.sp) / w.nsplit) + 1;
+        w.busy = blocks < w.attn_waves ? blocks : w.attn_waves;
+        w.tag = launch * (unsigned)a->n_layers + (unsigned)tk.layer + 1u;
+        w.rec = (unsigned long long*)(a->ws + a->records) + ((size_t)(w.b * w.n_kv + w.kvh) * w.nsplit) * kStMaxG * kDfRecUnits;
+        w.own = w.rec + (size_t)w.sp * kStMaxG * kDfRecUnits;
+        w.out = (uint32_t*)(tk.dst + (size_t)w.b * a->dim + (size_t)w.kvh * w.G * kHeadDim);
+        // (looked up here, not where they are used: a scalar load behind the task's inputs is waited for)
+        asm volatile("" : "+s"(w.tag), "+s"(w.rec), "+s"(w.own), "+s"(w.out), "+s"(w.G), "+s"(w.busy), "+s"(w.nact), "+s"(w.nsplit));
         return w;
     }
-    typedef float (*PartO)[kStMaxG][kHeadDim];  // the waves' outputs
-    // up to the waves' results in LDS
-    __device__ __forceinline__ void attend(const Task& wk, PartO part_o) {
-        const Place at = attention_place(wk);
-        if (at.sp >= at.nact) return;  // no visible rows in this split
-        const int G = at.G, nsplit = a->n_splits, kvh = at.kvh, sp = at.sp, b = at.b, p = at.p, pblk = at.pblk;
-        const bool owns_new = pblk % nsplit == sp;
+    // Up to the waves' results in LDS.  From the arrival of the token's row on a task is bound by the number of its instructions
+    // (one wave per SIMD), so everything that does not need the row is in registers before: the first block's cache rows, V
+    // turned, the rotation's factors, who has the new row, all of Place.  Every wave rotates the q heads for itself, eight
+    // values a lane, so the waves meet only once, over the results.  From the row to the split's record 2.5 us -> 1.3 (the split
+    // with the new row 2.9 -> 1.6; blocks and products where the compiler put them, and two meetings), one sequence at
+    // 512 positions 613 -> 587 us a step, two 720 -> 690, eight 870 -> 856.
+    // fresh, has_new: the cache's row p, k in lanes 0 .. 15 and v in those behind, for its caller to store.
+    __device__ __forceinline__ void attend(const Task& wk, const Place& at, WaveResults& res, v4u& fresh, bool& has_new) {
+        if (wave >= at.busy) {
+            df_wave_result<kStMaxG>(DfState(), lane, res.o[wave], res.m[wave], res.l[wave]);
+            return;
+        }
+        const int G = at.G, nsplit = at.nsplit, kvh = at.kvh, sp = at.sp, b = at.b, p = at.p, pblk = at.pblk, n_kv = at.n_kv;
         const int c = lane & 15, g4 = lane >> 4;
-        const int row_elems = (a->n_heads + 2 * a->n_kv) * kHeadDim;
-        const size_t cache_row = (size_t)a->n_kv * kHeadDim;
-        uint16_t* ck = (uint16_t*)wk.res + ((size_t)b * a->S * a->n_kv + kvh) * kHeadDim;
-        uint16_t* cv = wk.aux + ((size_t)b * a->S * a->n_kv + kvh) * kHeadDim;
-        const int row_bytes = a->n_kv * kHeadDim * 2;
+        const int row_elems = (at.n_heads + 2 * n_kv) * kHeadDim;
+        uint16_t* ck = (uint16_t*)wk.res + ((size_t)b * a->S * n_kv + kvh) * kHeadDim;
+        uint16_t* cv = wk.aux + ((size_t)b * a->S * n_kv + kvh) * kHeadDim;
+        const int row_bytes = n_kv * kHeadDim * 2;
         const int cache_bytes = (a->S - 1) * row_bytes + kHeadDim * 2;
         const __amdgpu_buffer_rsrc_t k_rsrc = make_rsrc(ck, cache_bytes), v_rsrc = make_rsrc(cv, cache_bytes);
-        const int blk_stride = nsplit * a->attn_waves;  // the split's blocks are dealt to this many waves: this one is wave, wave + kStWaves, ...
+        const int blk_stride = nsplit * at.attn_waves;  // this wave takes the blocks of waves wave, wave + kStWaves, ...
         v4u kb[2][4], vb[8];
         auto load_rows = [&](int blk) {
             const int base = blk * 32 * row_bytes;
@@ -980,87 +1009,108 @@ struct Stack {
 #pragma unroll
             for (int jj = 0; jj < 8; ++jj)
                 vb[jj] = __builtin_amdgcn_raw_buffer_load_b128(v_rsrc, base + ((jj & 3) + (jj >> 2) * 16 + 4 * g4) * row_bytes + c * 16, 0, 0);
+            if (blk == pblk) df_clear(vb, p, lane);
+            df_turn(vb);
         };
-        if (sp + nsplit * wave <= pblk) load_rows(sp + nsplit * wave);
+        load_rows(sp + nsplit * wave);
+        // the factors of pairs 4 c ..
+        const __amdgpu_buffer_rsrc_t factors = make_rsrc(a->rope_rows + (size_t)b * kHeadDim, kHeadDim * 4);
+        v4u cs = __builtin_amdgcn_raw_buffer_load_b128(factors, c * 16, 0, 0);
+        v4u sn = __builtin_amdgcn_raw_buffer_load_b128(factors, kHeadDim * 2 + c * 16, 0, 0);
+        const int turn = uniform(pblk / nsplit);
+        has_new = uniform(pblk - turn * nsplit == sp && (turn % at.attn_waves) % kStWaves == wave);
+        DfState st;
+        // (kept in front of the polls)
+#pragma unroll
+        for (int t = 0; t < 8; ++t) asm volatile("" : "+v"(st.o_acc[t]), "+v"(vb[t]), "+v"(kb[t >> 2][t & 3]));
+        asm volatile("" : "+v"(cs), "+v"(sn));
 
-        // the token's q heads of this group, k and v: a head per wave and round, a pair of values per lane
-        constexpr int kRounds = (kStMaxG + 2 + kStWaves - 1) / kStWaves;
+        // heads 4 u + g4 of the group, dims 8 c .. (lanes beyond the last head repeat it); where it is wanted k by lanes
+        // 0 .. 15 and v by the others
+        constexpr int kRounds = kStMaxG / 4;
         const __amdgpu_buffer_rsrc_t row = make_rsrc(wk.src + (size_t)b * row_elems, row_elems * 2);
-        uint32_t praw[kRounds];
-        const float cs = a->rope_rows[(size_t)b * kHeadDim + lane], sn = a->rope_rows[(size_t)b * kHeadDim + kHeadDim / 2 + lane];
+        v4u raw[kRounds] = {};
+        int head[kRounds];
+#pragma unroll
+        for (int u = 0; u < kRounds; ++u) head[u] = 4 * u + g4 < G ? 4 * u + g4 : G - 1;
+        const int new_head = lane < 16 ? at.n_heads + kvh : at.n_heads + n_kv + kvh;
         for (int spin = 0;; ++spin) {
             poll_again();
             unsigned m = 0;
 #pragma unroll
-            for (int u = 0; u < kRounds; ++u) {
-                const int hh = wave + u * kStWaves;
-                const int head = hh < G ? kvh * G + hh : (hh == G ? a->n_heads + kvh : a->n_heads + a->n_kv + kvh);
-                if (hh < G + 2) praw[u] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(row, lane * 4, head * kHeadDim * 2, kSc1);
-            }
+            for (int u = 0; u < kRounds; ++u)
+                if (4 * u < G) raw[u] = __builtin_amdgcn_raw_buffer_load_b128(row, ((kvh * G + head[u]) * kHeadDim + 8 * c) * 2, 0, kSc1);
+            if (has_new) fresh = __builtin_amdgcn_raw_buffer_load_b128(row, (new_head * kHeadDim + 8 * c) * 2, 0, kSc1);
+            auto look = [&](const v4u& v) { m = unset_max(unset_max(unset_max(unset_max(m, v.x), v.y), v.z), v.w); };
 #pragma unroll
             for (int u = 0; u < kRounds; ++u)
-                if (wave + u * kStWaves < G + 2) m = unset_max(m, praw[u]);
+                if (4 * u < G) look(raw[u]);
+            look(fresh);
             if (__builtin_amdgcn_ballot_w64(is_unset(m)) == 0 || wt.dead || wt.give_up(spin)) break;
         }
-        // rope on adjacent pairs, fp32, rounded to bf16; the split that holds position p writes the cache row
+        // rope on adjacent pairs, fp32, rounded to bf16
+        auto rotated = [&](const v4u& v) {
+            auto pair = [](unsigned d, unsigned cs, unsigned sn) {
+                const float x = bf16f(d), y = __uint_as_float(d & 0xffff0000u), k = __uint_as_float(cs), s = __uint_as_float(sn);
+                return pack_bf16x2(x * k - y * s, x * s + y * k);
+            };
+            return v4u{pair(v.x, cs.x, sn.x), pair(v.y, cs.y, sn.y), pair(v.z, cs.z, sn.z), pair(v.w, cs.w, sn.w)};
+        };
+        uint16_t(*rows)[kStRow] = sh.rows[wave];
 #pragma unroll
-        for (int u = 0; u < kRounds; ++u) {
-            const int hh = wave + u * kStWaves;
-            if (hh >= G + 2) break;
-            uint32_t v = praw[u];
-            if (hh <= G) {
-                const float x = bf16f(v & 0xffffu), y = bf16f(v >> 16);
-                v = (uint32_t)to_bf16(x * cs - y * sn) | ((uint32_t)to_bf16(x * sn + y * cs) << 16);
-            }
-            if (hh < G) {
-                *(uint32_t*)(&sh.qb[hh][2 * lane]) = v;
-            } else if (owns_new) {
-                *(uint32_t*)(&(hh == G ? sh.knew : sh.vnew)[2 * lane]) = v;
-                *(uint32_t*)((hh == G ? ck : cv) + (size_t)p * cache_row + 2 * lane) = v;
-            }
+        for (int u = 0; u < kRounds; ++u)
+            if (4 * u < G) *(v4u*)&rows[head[u]][8 * c] = rotated(raw[u]);
+        if (has_new) {
+            const v4u r = rotated(fresh);
+            fresh = lane < 16 ? r : fresh;
+            *(v4u*)&rows[lane < 16 ? kStMaxG : kStMaxG + 1][8 * c] = fresh;
         }
-        meet();
+        v4u vn = {0u, 0u, 0u, 0u};
+        auto new_row = [&]() {
+            df_new_key(kb, rows[kStMaxG], p, lane);
+            vn = *(const v4u*)&rows[kStMaxG + 1][8 * c];
+        };
+        int blk = sp + nsplit * wave;
+        if (blk == pblk) new_row();
+        // q^T as the B operand: column c = head c (columns beyond the group repeat its heads and are not looked at)
         v8bf qa[4];
 #pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-            uint4 t = make_uint4(0, 0, 0, 0);
-            if (c < G) t = *(const uint4*)(&sh.qb[c][kk * 32 + g4 * 8]);
-            qa[kk] = __builtin_bit_cast(v8bf, t);
-        }
-        for (int w = wave; w < a->attn_waves; w += kStWaves) {
-            const int blk0 = sp + nsplit * w;
-            DfState st;
-            for (int blk = blk0; blk <= pblk; blk += blk_stride) {
-                if (w != wave || blk != blk0) load_rows(blk);
-                df_block(kb, vb, qa, sh.knew, sh.vnew, blk, p, lane, st);
-            }
-            df_wave_result<kStMaxG>(st, lane, part_o[w], sh.part_m[w], sh.part_l[w]);
-        }
+        for (int kk = 0; kk < 4; ++kk) qa[kk] = __builtin_bit_cast(v8bf, *(const v4u*)&rows[c & (G - 1)][kk * 32 + g4 * 8]);
+        auto later_block = [&]() {
+            load_rows(blk);
+            if (blk == pblk) new_row();
+            df_block(kb, vb, vn, qa, blk, p, lane, st);
+        };
+        // (the first block stands by itself: nothing that a loop over the others needs is in its way)
+        df_block(kb, vb, vn, qa, blk, p, lane, st);
+        while ((blk += blk_stride) <= pblk) later_block();
+        df_wave_result<kStMaxG>(st, lane, res.o[wave], res.m[wave], res.l[wave]);
+        if (at.busy <= kStWaves) return;
+        st = DfState();
+        const int w = wave + kStWaves;
+        for (blk = sp + nsplit * w; blk <= pblk && w < at.attn_waves; blk += blk_stride) later_block();
+        df_wave_result<kStMaxG>(st, lane, res.o[w], res.m[w], res.l[w]);
     }
     // the waves' results over the workgroup, then over the splits
-    __device__ __forceinline__ void attention_outputs(const Task& wk, PartO part_o) {
-        const Place at = attention_place(wk);
-        if (at.sp >= at.nact) return;
-        const int G = at.G, nsplit = a->n_splits, kvh = at.kvh, sp = at.sp, b = at.b, nact = at.nact;
+    __device__ __forceinline__ void attention_outputs(const Place& at, const WaveResults& res) {
+        const int G = at.G, sp = at.sp, nact = at.nact;
+        const unsigned long long tag = (unsigned long long)at.tag << 32;
         meet();
-        unsigned long long* rec =
-            (unsigned long long*)(a->ws + a->records) + ((size_t)(b * a->n_kv + kvh) * nsplit) * kStMaxG * kDfRecUnits;
-        const unsigned long long tag = (unsigned long long)(launch * (unsigned)a->n_layers + (unsigned)wk.layer + 1u) << 32;
-        uint32_t* orow = (uint32_t*)(wk.dst + (size_t)b * a->dim + (size_t)kvh * G * kHeadDim);
         for (int hh = wave; hh < G; hh += kStWaves) {
-            DfPartial h = df_combine<kStMaxG>(part_o, sh.part_m, sh.part_l, hh, a->attn_waves, lane);
+            DfPartial h = at.busy <= kStWaves ? df_combine<kStMaxG, 4, true>(res.o, res.m, res.l, hh, 4, lane)
+                                              : df_combine<kStMaxG, 8, true>(res.o, res.m, res.l, hh, 8, lane);
             if (sp < nact - 1) {
-                df_store_record(rec + ((size_t)sp * kStMaxG + hh) * kDfRecUnits, tag, h, lane);
+                df_store_record(at.own + hh * kDfRecUnits, tag, h, lane);
                 continue;
             }
             bool gave_up = false;
-            if (nact > 1) h = df_merge<kStMaxG>(rec, nact, hh, tag, h, lane, wt.dead ? 1 : wt.limit, gave_up);
+            if (nact > 1) h = df_merge<kStMaxG>(at.rec, nact, hh, tag, h, lane, wt.dead ? 1 : wt.limit, gave_up);
             if (uniform(gave_up)) {
                 if (lane == 0) __hip_atomic_store(wt.error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 wt.dead = true;
             }
             const float is = gave_up ? __builtin_nanf("") : 1.0f / h.l;
-            __hip_atomic_store(orow + hh * (kHeadDim / 2) + lane, (uint32_t)to_bf16(h.o0 * is) | ((uint32_t)to_bf16(h.o1 * is) << 16),
+            __hip_atomic_store(at.out + hh * (kHeadDim / 2) + lane, (uint32_t)to_bf16(h.o0 * is) | ((uint32_t)to_bf16(h.o1 * is) << 16),
                                __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // to_bf16 gives no 0xffff
         }
     }
@@ -1090,10 +1140,18 @@ struct Stack {
     }
     __device__ __forceinline__ void run(const Task& tk, int k) {
         if (tk.ph == kAttn) {
-            const PartO part_o = (PartO)sh.words[k % kStBuffers];
+            WaveResults& res = *(WaveResults*)sh.words[k % kStBuffers];
             wait_ready(k);
-            attend(tk, part_o);
-            attention_outputs(tk, part_o);
+            const Place at = attention_place(tk);
+            if (at.sp < at.nact) {  // (else no visible rows in this split)
+                v4u fresh = {0u, 0u, 0u, 0u};
+                bool has_new = false;
+                attend(tk, at, res, fresh, has_new);
+                attention_outputs(at, res);
+                // the cache's row p, k in lanes 0 .. 15 and v in those behind: nothing in this launch reads it
+                if (has_new && lane < 32)
+                    *(v4u*)((lane < 16 ? (uint16_t*)tk.res : tk.aux) + (((size_t)at.b * a->S + at.p) * at.n_kv + at.kvh) * kHeadDim + 8 * (lane & 15)) = fresh;
+            }
             consume(k);
         } else if constexpr (kDirect) {
             switch (tk.ph) {

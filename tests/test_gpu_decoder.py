@@ -225,6 +225,37 @@ def test_attention_decode_long_cache_any_position(p, n_splits):
     assert not bad.any(), f"{int(bad.sum())} of {bad.numel()} outside tolerance"
 
 
+@pytest.mark.parametrize("n_splits", [1, 3])
+@pytest.mark.parametrize("nh,nkv", [(1, 1), (4, 1), (16, 2)])
+def test_attention_decode_takes_the_new_row_at_every_place_of_a_block(nh, nkv, n_splits):
+    """The new token's k and v are put into a block's registers at a place that depends on the position: all 32 of them, with
+    keys along the queries, so that the new row has most of the weight.  Comparison and tolerance as above."""
+    B, S, hd = 32, 70, 128
+    dev = torch.device("cuda")
+    g = torch.Generator(device="cuda").manual_seed(nh)
+    att = decoder.Attention.__new__(decoder.Attention)
+    torch.nn.Module.__init__(att)
+    att.head_dim, att.n_heads, att.n_kv_heads = hd, nh, nkv
+    xqkv = torch.randn(B, nh + 2 * nkv, hd, generator=g, device=dev)
+    xqkv[:, nh : nh + nkv] = xqkv[:, :nh].reshape(B, nkv, nh // nkv, hd).mean(2)
+    xqkv = xqkv.reshape(B, -1).to(torch.bfloat16)
+    ck, cv = (torch.randn(B, S, nkv, hd, generator=g, device=dev).to(torch.bfloat16) for _ in range(2))
+    pos = torch.arange(32, 64, device=dev)
+    cos, sin = decoder.rope_tables(hd, S, 500000.0, dev)
+    q, k, v = att.split_qkv(xqkv[:, None, :])
+    c, s_ = cos[pos][:, None, None, :], sin[pos][:, None, None, :]
+    q, k = decoder.apply_rope(q, c, s_), decoder.apply_rope(k, c, s_)
+    rk, rv = ck.clone(), cv.clone()
+    bidx = torch.arange(B, device=dev)
+    rk[bidx, pos], rv[bidx, pos] = k[:, 0], v[:, 0]
+    want = att.attend(q, rk, rv, torch.arange(S, device=dev)[None, None, :] <= pos[:, None, None])[:, 0]
+    got = decoder.attn_decode(xqkv, ck, cv, pos, cos, sin, nh, nkv, decoder.AttnWorkspace(B, nh, nkv, n_splits, dev) if n_splits > 1 else None)
+    torch.cuda.synchronize()
+    assert torch.equal(ck, rk) and torch.equal(cv, rv)
+    bad = (_ulp(got, want) > 3) & ((got.float() - want.float()).abs() > 4e-3)
+    assert not bad.any(), f"{int(bad.sum())} of {bad.numel()} outside tolerance"
+
+
 @pytest.mark.parametrize("n_splits", [1, 8])
 def test_attention_decode_ignores_rows_behind_the_position(n_splits):
     """Cache rows behind a sequence's position may never have been written:
@@ -774,6 +805,28 @@ def test_decode_stack_kernel_equals_the_kernels_per_layer(B, dim, ffn, nh, nkv, 
             k2.copy_(k)
             v2.copy_(v)
         step(9, min(33, S - 1))
+
+
+@pytest.mark.parametrize("B,dim,ffn,nh,nkv,S,n_splits", [(1, 128, 64, 1, 1, 70, 1), (2, 1024, 1984, 8, 1, 70, 2), (8, 512, 64, 4, 1, 70, 3)])
+def test_decode_stack_kernel_takes_the_new_row_at_every_place_of_a_block(B, dim, ffn, nh, nkv, S, n_splits):
+    """As test_decode_stack_kernel_equals_the_kernels_per_layer, sequence after sequence over the 32 positions of a block."""
+    args = decoder.ModelArgs(dim=dim, n_layers=1, n_heads=nh, n_kv_heads=nkv, vocab_size=256, ffn_dim=ffn)
+    model = _build(args, seed=dim + B)
+    caches = [model.make_cache(B, S, "cuda") for _ in range(2)]
+    for (k, v), (k2, v2) in zip(*caches):
+        k2.copy_(k.normal_())
+        v2.copy_(v.normal_())
+    cos, sin = decoder.rope_tables(128, S, args.rope_theta, "cuda")
+    ws, stack = decoder.AttnWorkspace(B, nh, nkv, n_splits, "cuda"), decoder.DecodeStack(model, B, caches[1], n_splits)
+    for p in range(32, 64):
+        pos = 32 + (torch.arange(B, device="cuda") * 5 + p) % 32
+        tok = torch.arange(B, device="cuda").reshape(B, 1) + 3 * p
+        want = model.decode_hidden_fused(tok, pos.reshape(B, 1), caches[0], cos, sin, ws)
+        h, rows = decoder.decode_step_begin(tok.reshape(B), pos, model.tok_embeddings.weight, cos, sin)
+        got = stack(h, pos, rows, 0)
+        stack.check()
+        assert np.array_equal(host_bits(got), host_bits(want)), p
+        assert all(torch.equal(x, y) for pair in zip(*caches) for x, y in zip(*pair)), p
 
 
 def test_short_divisions_of_the_decode_stack_kernel_equal_the_ieee_operations():
