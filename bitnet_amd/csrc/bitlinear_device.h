@@ -71,16 +71,23 @@ __device__ __forceinline__ uint32_t absmax_bits8(const uint4& v, uint32_t cur) {
 }
 
 // One value to its int8 code, left in the low byte of the result: the product
-// x * s in fp32 (mode 1: rounded to bf16), clamped to [-128, 127], then
-// + 1.5 * 2^23, which rounds to the nearest integer (ties to even, as rint does)
-// and leaves that integer's two's complement in the low mantissa bits.
-// Clamping before rounding equals rounding before clamping: the bounds are integers.
+// x * s in fp32 (mode 1: rounded to bf16) + 1.5 * 2^23, which rounds to the
+// nearest integer (ties to even, as rint does) and leaves that integer's two's
+// complement in the low mantissa bits, clamped to [-128, 127] there (clamping
+// after rounding equals rounding after clamping: the bounds are integers; a NaN
+// becomes -128).  In mode 0 x and s are bf16 values, so their product is exact in
+// fp32 and one fused operation gives the sum's bits (a decode step of one
+// sequence 584 -> 580 us, of two 693 -> 687, of eight 858 -> 855).
 template <int MODE>
 __device__ __forceinline__ uint32_t quant_low_byte(uint32_t x_f32_bits, float s32) {
-    float pr = __uint_as_float(x_f32_bits) * s32;
-    if (MODE == 1) pr = bf16_to_f32(f32_to_bf16_rne(pr));
-    pr = __builtin_amdgcn_fmed3f(pr, -128.0f, 127.0f);
-    return __float_as_uint(pr + 12582912.0f);
+    constexpr float kRound = 12582912.0f;
+    const float x = __uint_as_float(x_f32_bits);
+    float t;
+    if (MODE == 1)
+        t = bf16_to_f32(f32_to_bf16_rne(x * s32)) + kRound;
+    else
+        t = __builtin_fmaf(x, s32, kRound);
+    return __float_as_uint(__builtin_amdgcn_fmed3f(t, kRound - 128.0f, kRound + 127.0f));
 }
 
 template <int MODE>
