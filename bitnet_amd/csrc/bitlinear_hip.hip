@@ -2299,9 +2299,10 @@ constexpr int kSoloMaxK = 8192;
 // 13824 x 2560 5.14 -> 6.07, not taken); with a norm in front only at one token up to this K (3840 x 2560
 // 3.95 -> 3.80, 13824 x 2560 5.44 -> 5.16; 2560 x 6912 with gate and residual 5.87 -> 6.12, not taken)
 constexpr int kSoloLongRowK = 4096;
-// rows from which the norm + quantizer kernel of a prompt runs a wave per row (norm + product at K = 2560:
-// 32.2 -> 30.1 us at 2048 rows, 53.6 -> 48.7 at 4096; below 0.2-0.9 us behind)
-constexpr int kNormRowsPerWaveMinRows = 1024;
+// rows from which the norm + quantizer kernel of a prompt runs a wave per row (K = 2560, a workgroup per row against that:
+// 200 rows 2.95 us against 3.44, 300 3.56 / 3.49, 512 3.75 / 3.56, 600 4.37 / 3.68, 800 4.99 / 3.96; a prompt pass of 600 rows
+// 2954 -> 2904 us, of 1000 4550 -> 4440, of 300 level)
+constexpr int kNormRowsPerWaveMinRows = 512;
 // --- prefill GEMM: tile and k-split by the number of tiles ------------------
 // up to this many 64 x 128 tiles the GEMM uses 32 x 128 tiles (M = 128: 11.4 -> 9.0 us at 3840 x 2560, 21.5 -> 16.4
 // at 2560 x 6912); beyond, 64 x 256 (level or ahead from here on: 2560 x 6912 at M = 1536 31.7 -> 29.2)
@@ -3835,8 +3836,8 @@ int bitlinear_norm_forward_bf16_seg(const uint16_t* x, const uint16_t* norm_weig
 // gate / norm / quantizer once per token row
 static int launch_norm_quant(const uint16_t* x, const uint16_t* norm_weight, float eps, int glu, int8_t* q_ws, uint16_t* s_ws, int M,
                              int K, int mode, hipStream_t stream) {
-    // very many rows, no gate, short rows: a wave per row (norm + product at K = 2560: 32.2 -> 30.1 us at 2048 rows,
-    // 53.6 -> 48.7 at 4096; below 1024 rows 0.2-0.9 us behind, with the gate at K = 6912 4-7 us behind: not taken)
+    // very many rows, no gate, short rows: a wave per row (with the gate at K = 6912 4-7 us behind, without it 512 rows 5.1 us
+    // against 8: not taken)
     if (M >= kNormRowsPerWaveMinRows && !glu && K <= 8 * 64 * 8) {
         const int per_lane = (K / 8 + 63) / 64;
         const dim3 rgrid((M + 3) / 4, 1, 1), rblock(256, 1, 1);

@@ -666,6 +666,29 @@ def test_prefill_gemm_acc_bit_exact(m, n, k, tile):
     assert np.array_equal(acc.cpu().numpy(), o.acc_int32(a, w))
 
 
+@pytest.mark.parametrize("m,k", [(512, 128), (515, 2560), (514, 4096), (513, 4224)])
+def test_norm_and_quantizer_by_a_wave_per_row_equal_a_workgroup_per_row(m, k):
+    """From 512 rows on (up to 4096 values) the prompt's norm and quantizer take a wave per row: rows and scales equal those
+    of calls of fewer rows, of zeros and of infinities too."""
+    n, lib = 32, _lib.load_library()
+    w, _ = _rand_case(n, k, 1, seed=k)
+    g = torch.Generator(device="cuda").manual_seed(m)
+    x = torch.randn(m, k, generator=g, device="cuda").to(torch.bfloat16)
+    x[3], x[5, 7] = 0.0, float("inf")
+    norm_w = (torch.rand(k, generator=g, device="cuda") + 0.5).to(torch.bfloat16)
+    pk, ws = _packed_dev(w), torch.full((4,), 0.02, device="cuda").to(torch.bfloat16)
+    q, s = torch.zeros(2, m, k, dtype=torch.int8, device="cuda"), torch.zeros(2, m, dtype=torch.bfloat16, device="cuda")
+    out = torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
+    st = torch.cuda.current_stream().cuda_stream
+    for i, rows in enumerate((m, 300)):
+        for a in range(0, m, rows):
+            b = min(a + rows, m)
+            assert lib.bitlinear_norm_forward_bf16(x[a:b].data_ptr(), norm_w.data_ptr(), 1e-5, 0, pk.data_ptr(), ws.data_ptr(), None,
+                                                   out.data_ptr(), q[i, a:b].data_ptr(), s[i, a:b].data_ptr(), b - a, n, k, 0, st) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(q[0], q[1]) and torch.equal(s[0].view(torch.int16), s[1].view(torch.int16))
+
+
 @pytest.mark.parametrize("tile", [0, 1, 2, 4, 5, 6, 7, 8, 9, 10, 11, 12])
 @pytest.mark.parametrize("m,n,k", [(17, 16, 128), (1500, 16, 128), (40, 4112, 256), (700, 1296, 256), (1100, 2576, 128)])
 def test_prefill_gemm_deals_out_every_tile(m, n, k, tile):
