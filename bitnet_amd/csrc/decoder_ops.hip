@@ -12,6 +12,7 @@
 
 #include <atomic>
 
+#include "bitlinear_device.h"
 #include "bitnet_decoder_ops.h"
 #include "host_util.h"
 
@@ -239,9 +240,17 @@ __device__ __forceinline__ float bf16_dot2(uint32_t w, uint32_t x, float a) {
     return __builtin_fmaf(__uint_as_float(w & 0xffff0000u), __uint_as_float(x & 0xffff0000u), a);
 }
 
-template <int TB>  // tokens (columns) computed: 1, 2, 4 or 8 >= B
+// NORM: y holds the rows in front of the final norm, and every workgroup normalises them for itself (the first one leaves them
+// in y_out), in the shadow of its first weight requests: a launch and the rows' way to memory and back less (4.9 us), for 1.8
+// more here (a decode step of one sequence 580 -> 577.5 us, of two 683 -> 680.5).  For up to two rows of kLmNormMost values:
+// more would not be in registers before the weights' requests.
+constexpr int kLmNormVecs = 2;                             // vectors of 8 values per thread and row
+constexpr int kLmNormMost = kLmNormVecs * kLmThreads * 8;
+template <int TB, bool NORM>  // TB: tokens (columns) computed: 1, 2, 4 or 8 >= B
 __global__ __launch_bounds__(kLmThreads) void lm_head_stream_kernel(const uint16_t* __restrict__ y,
                                                                     const uint16_t* __restrict__ emb,
+                                                                    const uint16_t* __restrict__ norm_weight, float eps,
+                                                                    uint16_t* __restrict__ y_out,
                                                                     float* __restrict__ logits,
                                                                     float* __restrict__ part_val,
                                                                     int* __restrict__ part_idx, int B, int V, int K) {
@@ -261,10 +270,47 @@ __global__ __launch_bounds__(kLmThreads) void lm_head_stream_kernel(const uint16
         const int row = gidx * kLsRows + r;
         return (const v4u*)(emb + (size_t)(row < V ? row : V - 1) * K + s * 512) + lane;
     };
+    // the rows first: what is waited for behind the weights' requests are then these alone
+    uint4 hv[NORM ? TB : 1][kLmNormVecs], gv[kLmNormVecs];
+    if (NORM) {
+#pragma unroll
+        for (int j = 0; j < kLmNormVecs; ++j) {
+            const int i = tid + j * kLmThreads < K >> 3 ? tid + j * kLmThreads : (K >> 3) - 1;
+            gv[j] = ((const uint4*)norm_weight)[i];
+#pragma unroll
+            for (int t = 0; t < TB; ++t) hv[NORM ? t : 0][j] = ((const uint4*)(y + (size_t)(t < B ? t : B - 1) * K))[i];
+        }
+    }
     v4u w[kLsRows];
 #pragma unroll
     for (int r = 0; r < kLsRows; ++r) w[r] = __builtin_nontemporal_load(piece(grp < groups ? grp : groups - 1, r, 0));
-    {
+    if (NORM) {  // as rmsnorm_rows_kernel
+        __shared__ double wsum[kLmThreads / 64][TB];
+#pragma unroll
+        for (int t = 0; t < TB; ++t) {
+            double sq = 0.0;
+#pragma unroll
+            for (int j = 0; j < kLmNormVecs; ++j)
+                if (tid + j * kLmThreads < K >> 3) sq += sumsq8(hv[NORM ? t : 0][j]);
+            sq = wave_sum_f64(sq);
+            if (lane == 0) wsum[wave][t] = sq;
+        }
+        lds_barrier();
+#pragma unroll
+        for (int t = 0; t < TB; ++t) {
+            double total = 0.0;
+#pragma unroll
+            for (int k = 0; k < kLmThreads / 64; ++k) total += wsum[k][t];
+            const float rstd = 1.0f / __builtin_sqrtf((float)total / (float)K + eps);
+#pragma unroll
+            for (int j = 0; j < kLmNormVecs; ++j)
+                if (t < B && tid + j * kLmThreads < K >> 3) {
+                    const uint4 v = norm8(hv[NORM ? t : 0][j], gv[j], rstd);
+                    *(uint4*)(lds_y + (size_t)t * 2 * K + (size_t)(tid + j * kLmThreads) * 16) = v;
+                    if (blockIdx.x == 0) *(uint4*)(y_out + (size_t)t * K + (size_t)(tid + j * kLmThreads) * 8) = v;
+                }
+        }
+    } else {
         const int nvec = (B * K) >> 3;
         for (int i = tid; i < nvec; i += kLmThreads) *(uint4*)(lds_y + (size_t)i * 16) = *(const uint4*)(y + (size_t)i * 8);
     }
@@ -597,22 +643,27 @@ static int lm_head_impl(const uint16_t* h, const uint16_t* norm_weight, float ep
             return hipFuncSetAttribute((const void*)lm_head_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
         }) != hipSuccess)
         return 3;
-    hipLaunchKernelGGL(rmsnorm_rows_kernel, dim3(B), dim3(kNormThreads), 0, (hipStream_t)stream, h, norm_weight, eps, y_ws, K);
     int nparts = 0;
-    const bool stream_ok = B <= 8 && (K % 512) == 0 && (size_t)B * 2 * K <= 60u * 1024u;
-    if (stream_ok && g_lm_kernel != 1) {
+    const bool streams = B <= 8 && (K % 512) == 0 && (size_t)B * 2 * K <= 60u * 1024u && g_lm_kernel != 1;
+    // (not over the rows themselves: other workgroups read them while the first one writes)
+    const bool norm_inside = streams && B <= 2 && K <= kLmNormMost && (h + (size_t)B * K <= y_ws || y_ws + (size_t)B * K <= h);
+    if (!norm_inside)
+        hipLaunchKernelGGL(rmsnorm_rows_kernel, dim3(B), dim3(kNormThreads), 0, (hipStream_t)stream, h, norm_weight, eps, y_ws, K);
+    if (streams) {
         // persistent waves: at most 4 workgroups per CU of a 256-CU part, each wave walking row groups
         const int full = (V + kLsRows * (kLmThreads / 64) - 1) / (kLsRows * (kLmThreads / 64));
         const dim3 grid(full < 1024 ? full : 1024);
         nparts = (int)grid.x;
         const size_t lds_s = (size_t)B * 2 * K;
-#define BITNET_LM_STREAM(TB)                                                                                          \
-    hipLaunchKernelGGL(lm_head_stream_kernel<TB>, grid, dim3(kLmThreads), lds_s, (hipStream_t)stream, y_ws, emb, logits, \
-                       part_val, part_idx, B, V, K)
-        if (B == 1) BITNET_LM_STREAM(1);
-        else if (B == 2) BITNET_LM_STREAM(2);
-        else if (B <= 4) BITNET_LM_STREAM(4);
-        else BITNET_LM_STREAM(8);
+#define BITNET_LM_STREAM(TB, NORM)                                                                                         \
+    hipLaunchKernelGGL((lm_head_stream_kernel<TB, NORM>), grid, dim3(kLmThreads), lds_s, (hipStream_t)stream, NORM ? h : y_ws, \
+                       emb, norm_weight, eps, y_ws, logits, part_val, part_idx, B, V, K)
+        if (norm_inside && B == 1) BITNET_LM_STREAM(1, true);
+        else if (norm_inside) BITNET_LM_STREAM(2, true);
+        else if (B == 1) BITNET_LM_STREAM(1, false);
+        else if (B == 2) BITNET_LM_STREAM(2, false);
+        else if (B <= 4) BITNET_LM_STREAM(4, false);
+        else BITNET_LM_STREAM(8, false);
 #undef BITNET_LM_STREAM
     } else {
         const int rows_per_wg = 16 * (kLmThreads / 64);

@@ -757,6 +757,24 @@ def test_prompt_products_that_the_epilogues_do_not_take_are_left_to_the_separate
         assert decoder.norm_gate_bitlinear(torch.zeros(M, K, dtype=torch.bfloat16, device="cuda"), norm, w13) is None, (M, K, ffn, ends)
 
 
+@pytest.mark.parametrize("B", [1, 2])
+@pytest.mark.parametrize("V,K", [(70, 512), (1000, 2560), (333, 4096), (333, 4608)])
+def test_lm_head_that_normalises_its_rows_equals_the_norm_by_itself(B, V, K):
+    """One and two rows of up to 4096 values are normalised inside the LM head's kernel: the logits are those of a call of
+    three rows, for which the norm is a kernel of its own."""
+    gen = torch.Generator(device="cuda").manual_seed(V + K)
+    norm = decoder.RMSNorm(K, 1e-5).cuda().to(torch.bfloat16)
+    norm.weight.data = torch.rand(K, generator=gen, device="cuda").add(0.5).to(torch.bfloat16)
+    h = torch.randn(3, K, generator=gen, device="cuda").to(torch.bfloat16)
+    emb = torch.randn(V, K, generator=gen, device="cuda").mul(0.05).to(torch.bfloat16)
+    logits = [torch.empty(n, V, device="cuda") for n in (3, B)]
+    for out in logits:
+        n = out.shape[0]
+        tok = decoder.lm_head_greedy(h[:n], norm, emb, decoder.LmHeadWorkspace(n, V, K, "cuda"), logits_out=out)
+        assert torch.equal(tok, out.argmax(-1))
+    assert torch.equal(logits[0][:B], logits[1])
+
+
 @pytest.mark.parametrize("workgroups", [0, 1, 7, 600])  # 600: more than can be resident, tasks by ticket
 @pytest.mark.parametrize("B,dim,ffn,nh,nkv,S,n_splits,segments", [
     (1, 128, 64, 1, 1, 33, 1, False), (2, 128, 64, 1, 1, 40, 16, False), (1, 1152, 2112, 9, 9, 70, 3, False),
