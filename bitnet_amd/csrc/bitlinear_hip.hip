@@ -2965,24 +2965,6 @@ int launch_prefill(const int8_t* act, const int8_t* packed, uint16_t* out, int32
     // the kernel addresses the packed weights through a buffer descriptor with 32-bit offsets
     if ((long long)N * K / 4 >= (1ll << 31)) return BITLINEAR_ERR_SHAPE;
     g_last_kernel = "gemm_i2_prefill_kernel";
-    // the large tile double-buffers 2 x 128 rows x 272 bytes = 68 KiB of LDS (so do four groups of the
-    // small one): above the 64 KiB a kernel gets without asking (a host-side attribute, set once per process)
-    static OncePerDevice lds_limit_raised;
-    const hipError_t lds_err = t_plan.active ? hipSuccess : lds_limit_raised.run([] {
-        hipError_t e = hipFuncSetAttribute((const void*)gemm_i2_prefill_kernel<4, 2, 1>,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, 2 * 128 * kPfRowBytes);
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute((const void*)gemm_i2_prefill_kernel<1, 1, 4>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    4 * 2 * 32 * kPfRowBytes);
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute((const void*)gemm_i2_prefill_kernel<2, 1, 2>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    2 * 2 * 64 * kPfRowBytes);
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute((const void*)gemm_i2_prefill_kernel<2, 2, 2>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    2 * 2 * 64 * kPfRowBytes);
-        return e;
-    });
-    if (lds_err != hipSuccess) return BITLINEAR_ERR_LAUNCH;
     // tile (rows x columns of the output per workgroup): 0 = 64 x 128, 1 = 128 x 256, 2 = 64 x 256,
     // 3 = 64 x 512, 4 = 32 x 128.  Measured: the wide tile pays once there are many tiles (about four
     // per CU of the narrow kind); with few tiles (up to about 1.3 per CU) half-height tiles put twice as
@@ -3039,6 +3021,24 @@ int launch_prefill(const int8_t* act, const int8_t* packed, uint16_t* out, int32
     if (ring) {
         return launch_ring(ring, act, packed, out, acc_out, s, ws, smap, M, N, K, stream, residual, RingPlain{});
     }
+    // the large tile double-buffers 2 x 128 rows x 272 bytes = 68 KiB of LDS (so do four groups of the
+    // small one): above the 64 KiB a kernel gets without asking (a host-side attribute, set once per process)
+    static OncePerDevice lds_limit_raised;
+    const hipError_t lds_err = t_plan.active ? hipSuccess : lds_limit_raised.run([] {
+        hipError_t e = hipFuncSetAttribute((const void*)gemm_i2_prefill_kernel<4, 2, 1>,
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, 2 * 128 * kPfRowBytes);
+        if (e == hipSuccess)
+            e = hipFuncSetAttribute((const void*)gemm_i2_prefill_kernel<1, 1, 4>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    4 * 2 * 32 * kPfRowBytes);
+        if (e == hipSuccess)
+            e = hipFuncSetAttribute((const void*)gemm_i2_prefill_kernel<2, 1, 2>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    2 * 2 * 64 * kPfRowBytes);
+        if (e == hipSuccess)
+            e = hipFuncSetAttribute((const void*)gemm_i2_prefill_kernel<2, 2, 2>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    2 * 2 * 64 * kPfRowBytes);
+        return e;
+    });
+    if (lds_err != hipSuccess) return BITLINEAR_ERR_LAUNCH;
     bool dma = true;
     int dma_mt = 2;  // row tiles of 32 tokens per workgroup of that kernel: 64 x 256, or 32 x 256 / 128 x 256 when forced
     if (t_tune.path == 5) {

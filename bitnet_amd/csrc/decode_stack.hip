@@ -11,11 +11,12 @@
 // such a hand-over measures 1.4 us, readers' barrier included.  30 layers at 512 positions, us:
 //   sequences            1     2     3     4     8
 //   launches           755   875  1000  1070  1060
-//   this kernel        497   597   675   698   740
-// What is left of a phase (of a layer's 16.5 us at one sequence the five take about 3, 5, 2.2, 3.5 and 3.2): 1.3 to 1.7 us from the
-// arrival of a task's inputs to its outputs (one exchange between the waves, products 0.5 to 0.9, the epilogue 0.3), the hand-over,
-// and the last workgroup being late; the weights are not waited for.  Polls are as dense as pays: two in flight cost 7 %, a pause
-// of 0.2 us behind each 1 %; outputs stored as 4 or 16 bytes a lane instead of two 1 %.
+//   this kernel        462   569   634   662   724
+// (the launches with the attention's earlier instructions.)  What is left of a phase (of a layer's 15 us at one sequence the
+// five take about 2.7, 3.9, 2, 3.5 and 2.9): 1 to 1.3 us from the arrival of a task's inputs to its outputs (the exchange between
+// the waves 0.3, norm and quantizer 0.3 to 0.5, products 0.1 to 0.3, the epilogue 0.3), the hand-over, and the last workgroup
+// being late; the weights are not waited for.  Polls are as dense as pays: two in flight cost 7 %, a pause of 0.2 us behind
+// each 1 %; outputs stored as 4 or 16 bytes a lane instead of two 1 %.
 // Up to two tokens every workgroup of a product normalises and quantizes the rows by itself, between their
 // arrival and its matrix instructions.  That part grows with the tokens (three: 1120 us).  Beyond two, one
 // task per token does it for all and publishes int8 rows, which are the matrix instructions' operand as they
