@@ -241,8 +241,8 @@ __device__ __forceinline__ float bf16_dot2(uint32_t w, uint32_t x, float a) {
 }
 
 // NORM: y holds the rows in front of the final norm, and every workgroup normalises them for itself (the first one leaves them
-// in y_out), in the shadow of its first weight requests: a launch and the rows' way to memory and back less (4.9 us), for 1.8
-// more here (a decode step of one sequence 580 -> 577.5 us, of two 683 -> 680.5).  For up to two rows of kLmNormMost values:
+// in y_out), in the shadow of its first weight requests: a launch and the rows' way to memory and back less (a decode step of one
+// sequence 580 -> 577.5 us, of two 683 -> 680.5).  For up to two rows of kLmNormMost values:
 // more would not be in registers before the weights' requests.
 constexpr int kLmNormVecs = 2;                             // vectors of 8 values per thread and row
 constexpr int kLmNormMost = kLmNormVecs * kLmThreads * 8;
