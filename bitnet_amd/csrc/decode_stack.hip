@@ -88,8 +88,9 @@ constexpr int kSc1 = kPollPolicy;       // device-coherent accesses
 typedef unsigned v2u __attribute__((ext_vector_type(2)));
 typedef int v2i __attribute__((ext_vector_type(2)));
 // Four int8 of quantized rows that mean "not written": as an int the least there is, so that the minimum of a lane's words
-// shows whether one of them is that.  Its last byte, -128, comes only with NaNs (|x| * scale rounds to 127 at most; where a
-// NaN is the maximum, finite values are clamped): a slice of such a row says in its record that it is written (kComplete).
+// shows whether one of them is that.  Its last byte, -128, comes only where the row's maximum is not finite: a finite one leaves
+// |x| * scale below 127.5, an infinite one makes the scale 0, codes of 0 and, of infinity * 0, -128, and beside a NaN
+// finite values are clamped.  A slice of such a row says in its record that it is written (kComplete).
 constexpr int kUnsetBytes = INT32_MIN;
 constexpr unsigned kComplete = 1u << 30;
 constexpr int kLookEvery = 32;          // polls between two looks at that, a power of two
@@ -609,7 +610,7 @@ struct Stack {
     }
 
     // Norm and quantizer of the wave's slices: the scales, and the bytes by put8 (8 of them, a 512-value piece's) and
-    // put_rest (S::T of them).  Whether there is a NaN in one of the rows.
+    // put_rest (S::T of them).  Whether one of the rows has a value that is not finite.
     // The waves meet once for both of a row's reductions.  The quantizer needs the largest of the normalised values
     // bf16((h r) g), and r the sum of squares; but each of those is |h g| r within two roundings, so the largest lies
     // between max |h g| r (1 - 2^-21) and the same with a plus, and where both ends round to the same bf16 that is it
@@ -669,8 +670,8 @@ struct Stack {
                 if (S::T == 4) v.rest[1] = norm2(v.rest[1], got.g[S::kFull].y, rstd);
             }
         }
-        bool nans = false;
-        if (!uniform(known)) nans = exchange_maxima<UPW>(tk, got, am);
+        bool nonfinite = false;
+        if (!uniform(known)) nonfinite = exchange_maxima<UPW>(tk, got, am);
 #pragma unroll
         for (int t = 0; t < TQ; ++t) {
             const Values<kStUpwF>& v = got.f[t];
@@ -684,9 +685,9 @@ struct Stack {
                 put_rest(t, r);
             }
         }
-        return nans;
+        return nonfinite;
     }
-    // The rows' maxima from the normalised values themselves; whether one of them is a NaN
+    // The rows' maxima from the normalised values themselves; whether one of them is infinite or a NaN
     template <int UPW>
     __device__ __forceinline__ bool exchange_maxima(const Task& tk, Got<MT>& got, uint32_t (&am)[TQ]) {
         typedef Slice<UPW> S;
@@ -701,7 +702,7 @@ struct Stack {
             if (lane == 63) lds_put(sh.amax[t][wave], v2i{(int)m, exchange + 1});
         }
         ++exchange;
-        bool nans = false;
+        bool nonfinite = false;
 #pragma unroll
         for (int t = 0; t < TQ; ++t) {
             Values<kStUpwF>& v = got.f[t];
@@ -713,8 +714,8 @@ struct Stack {
                 if (uniform(min(min(x[0].y, x[0].w), min(x[1].y, x[1].w)) - exchange) >= 0) break;
             }
             am[t] = (uint32_t)max(max(x[0].x, x[0].z), max(x[1].x, x[1].z));
-            if (uniform((int)am[t]) > 0x7f80) {  // 0 times a NaN: the values past the end of K have to be zeros again
-                nans = true;
+            if (uniform((int)am[t]) >= 0x7f80) {  // 0 times a NaN: the values past the end of K have to be zeros again
+                nonfinite = true;
 #pragma unroll
                 for (int i = 0; i < S::kFull; ++i)
                     if (wave * S::kValues + i * 512 + lane * 8 >= tk.K) v.full[i] = make_uint4(0u, 0u, 0u, 0u);
@@ -724,7 +725,7 @@ struct Stack {
                 }
             }
         }
-        return nans;
+        return nonfinite;
     }
 
     // norm + quantizer of the wave's slices, products, outputs.  RPW 1, 2: row blocks; 4: two pairs (x1, x3), gated
@@ -833,7 +834,7 @@ struct Stack {
         const __amdgpu_buffer_rsrc_t to = make_rsrc(tk.dst, ((tk.K >> 6) - 1) * step + 64);
         auto place = [&](int at) { return (at >> 6) * step + (at & 63); };
         // (4 bytes at least a store: a word is there or not; values past the end of K are not stored)
-        const bool nans = quantize<UPW>(
+        const bool nonfinite = quantize<UPW>(
             tk, got, s,
             [&](int, int i, uint2 v) {
                 const int at = first + i * 512 + lane * 8;
@@ -849,9 +850,9 @@ struct Stack {
                 __builtin_amdgcn_raw_buffer_store_b32(r, to, mine ? place(at) : kBeyond, 0, kSc1);
             });
         RowRecord* rec = (RowRecord*)tk.res;
-        if (nans) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");  // readers cannot tell from the words that they are there
+        if (nonfinite) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");  // readers cannot tell from the words that they are there
         if (lane == 0) {
-            __hip_atomic_store(&rec->slice[wave], nans ? kComplete : 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&rec->slice[wave], nonfinite ? kComplete : 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (wave == 0) __hip_atomic_store(&rec->scale, (unsigned)f32_to_bf16_rne(s[0]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }

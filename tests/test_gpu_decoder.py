@@ -940,7 +940,7 @@ def _rows_whose_largest_value_is_near_a_tie(dim, norm_weight, count, eps=1e-5):
     return torch.from_numpy(np.stack(rows[:count])).to(torch.bfloat16)
 
 
-@pytest.mark.parametrize("where", ["tie", "large weight", "small weights", "nan weight", "zero row"])
+@pytest.mark.parametrize("where", ["tie", "large weight", "small weights", "nan weight", "zero row", "infinite weight", "overflow"])
 @pytest.mark.parametrize("B,dim,ffn,nh,nkv", [(1, 128, 64, 1, 1), (2, 128, 64, 1, 1), (2, 1152, 2112, 9, 9), (3, 128, 64, 1, 1), (8, 1152, 2112, 9, 9)])
 def test_decode_stack_kernel_exchanges_maxima_that_it_cannot_tell_beforehand(B, dim, ffn, nh, nkv, where):
     """Rows whose largest normalised value does not follow from max |h g| and the sum of squares alone."""
@@ -961,6 +961,12 @@ def test_decode_stack_kernel_exchanges_maxima_that_it_cannot_tell_beforehand(B, 
             w[dim // 2 + 1] = float("nan")
     if where == "zero row":
         emb[B - 1] = 0.0
+    if where in ("infinite weight", "overflow"):
+        # an infinite maximum: scale 0, codes 0 but for the infinity's -128, here the last of four, which beyond two tokens
+        # is the word of a row not yet written.  (In front of the gate, where the quotients by a scale of 0 end as NaNs.)
+        emb[:, dim // 2 + 3] = 16.0
+        for layer in model.layers:
+            layer.ffn_norm.weight.data[dim // 2 + 3] = float("inf") if where == "infinite weight" else 2.0**127
     caches = [model.make_cache(B, S, "cuda") for _ in range(2)]
     cos, sin = decoder.rope_tables(128, S, args.rope_theta, "cuda")
     ws = decoder.AttnWorkspace(B, nh, nkv, n_splits, "cuda")
