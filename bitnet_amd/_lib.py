@@ -29,6 +29,7 @@ SIGNATURES = {
         [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_ptr],
     ),
     "bitlinear_norm_epilogue_applies": (_c_int, [_c_int, _c_int, _c_int, ctypes.POINTER(_c_int), _c_int]),
+    "bitlinear_norm_gate_ahead": (_c_int, [_c_int, _c_int, _c_int, ctypes.POINTER(_c_int), _c_int]),
     "bitlinear_norm_gate_forward_bf16": (
         _c_int,
         [_c_ptr, _c_ptr, ctypes.c_float, _c_ptr, _c_ptr, ctypes.POINTER(_c_int), _c_int, _c_ptr, _c_ptr, _c_ptr, *[_c_int] * 4, _c_ptr],

@@ -2919,6 +2919,60 @@ int ring_choice(int M, int N, int K, const ScaleMap& smap, bool aligned) {
     if (ring_tiles(M, N, 4) <= kRingCus) return 4;
     return 0;
 }
+// the tiles of gemm_i2_prefill_mix_kernel: whole rounds of 64 x 256 over the first columns, 32 x 128 ("quarters") behind them
+struct MixPlan {
+    int rt64, rt32, big_cols, small_cols;
+    long long bigs, quarters, groups;
+    bool wanted;  // the built-in choice (figures at launch_prefill)
+};
+MixPlan plan_mix(int M, int N) {
+    MixPlan p;
+    p.rt64 = (M + 63) / 64, p.rt32 = (M + 31) / 32;
+    const long long wide = (long long)((N + 255) / 256) * p.rt64;
+    const int rounds = wide / kPrefillMixCus > 1 ? (int)(wide / kPrefillMixCus) : 1;
+    p.big_cols = (int)((long long)kPrefillMixCus * rounds / p.rt64);
+    if (p.big_cols > N / 256) p.big_cols = N / 256;
+    p.small_cols = (N - p.big_cols * 256 + 127) / 128;
+    p.bigs = (long long)p.rt64 * p.big_cols;
+    p.quarters = (long long)p.rt32 * p.small_cols;
+    p.groups = 8 * ((p.bigs + 7) / 8) + 8 * ((p.quarters + 7) / 8);
+    p.wanted = wide > kPrefillMixCus && p.big_cols >= 1 && p.quarters > 0 && p.quarters <= kPrefillMixMaxQuarters && p.groups < kMostTiles;
+    return p;
+}
+// Whether a product of more than kPrefillMinTokens tokens goes through the split-K kernel instead of a GEMM.  A few dozen
+// tokens on a narrow matrix leave most CUs without a GEMM tile, and a tile's chain of 256-k chunks is then pure latency
+// (about 0.64 us each).  There the split-K kernel, run once per 16 tokens and re-reading the weights from L2 (about
+// 1.45 TB/s measured), finishes earlier.  Both estimates in microseconds, fitted to measurements at the 2B shapes.
+bool splitk_ahead(int M, int N, int K, int ring) {
+    if (M > kSplitKMaxTokens || t_tune.path != 0) return false;
+    // the 32 x 64 tiles against the split-K kernel by rows, of which its last group may hold few (17 x 2560 x 2560
+    // 4.8 us against 5.3, 32 x 2560 x 2560 5.95 against 5.45, 17 x 3840 x 2560 5.6 against 5.3)
+    if (ring == 1) return 4.0 + 0.148 * (K / 256.0) > 3.5 + (M / 16.0) * ((double)N * K / 4.0) / 1.45e6;
+    const double groups = (M + 15) / 16;
+    const double splitk_us = 3.5 + groups * ((double)N * K / 4.0) / 1.45e6;
+    const double tiles = ((N + 127) / 128) * (double)((M + 63) / 64);
+    const double tiles32 = ((N + 127) / 128) * (double)((M + 31) / 32);
+    const double gemm_us = tiles32 <= kPrefillSplit2Tiles
+                               ? 5.1 + ((tiles32 <= kPrefillSplit4Tiles && K >= kPrefillSplit4MinK) ? 0.267 : 0.29) * (K / 256.0)
+                               : (tiles <= kPrefillFewTiles
+                                      ? 4.4 + 0.45 * (K / 256.0) * (tiles32 > 400.0 ? tiles32 / 400.0 : 1.0)
+                                      : 4.0 + 0.64 * (K / 256.0) * (tiles > 256.0 ? tiles / 256.0 : 1.0));
+    return gemm_us > splitk_us;
+}
+// Whether the gate in the ring kernel's epilogue is ahead of the separate calls, which may take another GEMM kernel: norm, w13,
+// gate, norm and w2 of a block, fused against separate.  Where both take the ring kernel it is (a prompt pass of 512 tokens
+// 2623 us against 2677).  Where the separate product goes through tiles of two sizes the 1 to 2 us that the gate saves are less
+// than that kernel's lead as long as its small tiles are at most one per CU (288 tokens, 13824 x 2560: 54 of them, 38.2 us
+// against 36.7, and a pass of 320 tokens 2279 against 2218; 448, 11264 x 2560: 224, 39.4 against 38.2) and its chunks 256 k
+// (300, 13824 x 3200: 42.6 against 45.6); with more of them it is ahead (352, 13824 x 2560: 264, 39.9 against 41.0).  Where the
+// separate product takes the split-K kernel it is behind (17, 2048 x 2560 14.6 against 13.1; level at the rule's edge, 23,
+// 3072 x 2560 15.5 and 15.5).  Rope in the epilogue saves a launch and is ahead in all of these (1.04 to 1.6 times).
+constexpr int kGateMixQuarters = 256;
+bool gate_ahead(int M, int N, int K, int ring) {
+    if (!ring || t_tune.path != 0) return ring != 0;
+    const MixPlan mp = plan_mix(M, N);
+    return !(mp.wanted && mp.quarters <= kGateMixQuarters && K % 256 == 0) && !splitk_ahead(M, N, K, ring);
+}
 template <class Epi>
 int launch_ring(int ring, const int8_t* act, const int8_t* packed, uint16_t* out, int32_t* acc_out, const uint16_t* s,
                 const uint16_t* ws, const ScaleMap& smap, int M, int N, int K, hipStream_t stream, const uint16_t* residual, Epi epi) {
@@ -2994,26 +3048,18 @@ int launch_prefill(const int8_t* act, const int8_t* packed, uint16_t* out, int32
     // 22.4 -> 20.1, 2560 33.0 -> 28.5, 5120 58.0 -> 49.9, 20480 x 3200 at M = 617 46.1 -> 43.6; with more of them the even tiles are ahead: 2560 x 2560 at
     // M = 2560 21.3 against 26.5, 3840 x 2560 at M = 2048 22.8 against 28.0)
     if (dma_fits && (t_tune.path == 0 || (t_tune.path == 5 && t_tune.prefill_big == 8))) {
-        const int rt64 = (M + 63) / 64, rt32 = (M + 31) / 32;
-        const long long wide = (long long)((N + 255) / 256) * rt64;
-        const int rounds = wide / kPrefillMixCus > 1 ? (int)(wide / kPrefillMixCus) : 1;
-        int big_cols = (int)((long long)kPrefillMixCus * rounds / rt64);
-        if (big_cols > N / 256) big_cols = N / 256;
-        const int small_cols = (N - big_cols * 256 + 127) / 128;
-        const long long quarters = (long long)rt32 * small_cols;
-        const bool wanted = t_tune.path == 5 || (wide > kPrefillMixCus && big_cols >= 1 && quarters > 0 && quarters <= kPrefillMixMaxQuarters);
-        const long long bigs = (long long)rt64 * big_cols;
-        const long long groups = 8 * ((bigs + 7) / 8) + 8 * ((quarters + 7) / 8);
-        if (wanted && groups < kMostTiles) {
-            const int nbig = 8 * (int)((bigs + 7) / 8);
-            const dim3 mgrid((unsigned)groups, 1, 1), mblock(256, 1, 1);
+        const MixPlan mp = plan_mix(M, N);
+        if ((t_tune.path == 5 || mp.wanted) && mp.groups < kMostTiles) {
+            const int nbig = 8 * (int)((mp.bigs + 7) / 8);
+            const dim3 mgrid((unsigned)mp.groups, 1, 1), mblock(256, 1, 1);
+            const unsigned magic = tile_magic(mp.rt64, mp.big_cols), small_magic = tile_magic(mp.rt32, mp.small_cols);
             g_last_kernel = "gemm_i2_prefill_mix_kernel";
             if (K % 256 == 0)
-                BL_LAUNCH((gemm_i2_prefill_mix_kernel<256>), mgrid, mblock, 3 * 64 * 256, stream, act, wq, M, N, K, nbig, big_cols,
-                          out ? 1 : 0, small_cols, tile_magic(rt64, big_cols), tile_magic(rt32, small_cols), s, out, acc_out, ws, smap, residual);
+                BL_LAUNCH((gemm_i2_prefill_mix_kernel<256>), mgrid, mblock, 3 * 64 * 256, stream, act, wq, M, N, K, nbig, mp.big_cols,
+                          out ? 1 : 0, mp.small_cols, magic, small_magic, s, out, acc_out, ws, smap, residual);
             else
-                BL_LAUNCH((gemm_i2_prefill_mix_kernel<128>), mgrid, mblock, 3 * 64 * 128, stream, act, wq, M, N, K, nbig, big_cols,
-                          out ? 1 : 0, small_cols, tile_magic(rt64, big_cols), tile_magic(rt32, small_cols), s, out, acc_out, ws, smap, residual);
+                BL_LAUNCH((gemm_i2_prefill_mix_kernel<128>), mgrid, mblock, 3 * 64 * 128, stream, act, wq, M, N, K, nbig, mp.big_cols,
+                          out ? 1 : 0, mp.small_cols, magic, small_magic, s, out, acc_out, ws, smap, residual);
             return launch_status();
         }
     }
@@ -3209,30 +3255,9 @@ int launch_gemv(const int8_t* act, const int8_t* packed, uint16_t* out, int32_t*
     // vector loads: 16-byte groups of both operands must be 16-byte aligned
     if ((((uintptr_t)act) | ((uintptr_t)packed)) & 15u) return BITLINEAR_ERR_ARG;
     if (M > kPrefillMinTokens && t_tune.path != 2) {
-        // A few dozen tokens on a narrow matrix leave most CUs without a GEMM tile, and a tile's
-        // chain of 256-k chunks is then pure latency (about 0.64 us each).  There the split-K kernel,
-        // run once per 16 tokens and re-reading the weights from L2 (about 1.45 TB/s measured),
-        // finishes earlier.  Both estimates in microseconds, fitted to measurements at the 2B shapes.
-        bool gemm = true;
-        if (M <= kSplitKMaxTokens && t_tune.path == 0) {
-            const double groups = (M + 15) / 16;
-            const double splitk_us = 3.5 + groups * ((double)N * K / 4.0) / 1.45e6;
-            const double tiles = ((N + 127) / 128) * (double)((M + 63) / 64);
-            const double tiles32 = ((N + 127) / 128) * (double)((M + 31) / 32);
-            const double gemm_us = tiles32 <= kPrefillSplit2Tiles
-                                       ? 5.1 + ((tiles32 <= kPrefillSplit4Tiles && K >= kPrefillSplit4MinK) ? 0.267 : 0.29) * (K / 256.0)
-                                       : (tiles <= kPrefillFewTiles
-                                              ? 4.4 + 0.45 * (K / 256.0) * (tiles32 > 400.0 ? tiles32 / 400.0 : 1.0)
-                                              : 4.0 + 0.64 * (K / 256.0) * (tiles > 256.0 ? tiles / 256.0 : 1.0));
-            // the 32 x 64 tiles against the split-K kernel by rows, of which its last group may hold few (17 x 2560 x 2560
-            // 4.8 us against 5.3, 32 x 2560 x 2560 5.95 against 5.45, 17 x 3840 x 2560 5.6 against 5.3)
-            if (ring_choice(M, N, K, smap, ring_aligned(out, acc_out, residual, K)) == 1)
-                gemm = 4.0 + 0.148 * (K / 256.0) <= 3.5 + (M / 16.0) * ((double)N * K / 4.0) / 1.45e6;
-            else
-                gemm = gemm_us <= splitk_us;
-        }
-        if (gemm) return launch_prefill(act, packed, out, acc_out, s, ws, smap, M, N, K, stream, residual);
-        return launch_splitk(act, packed, out, acc_out, s, ws, smap, M, N, K, stream, residual);
+        if (M <= kSplitKMaxTokens && splitk_ahead(M, N, K, ring_choice(M, N, K, smap, ring_aligned(out, acc_out, residual, K))))
+            return launch_splitk(act, packed, out, acc_out, s, ws, smap, M, N, K, stream, residual);
+        return launch_prefill(act, packed, out, acc_out, s, ws, smap, M, N, K, stream, residual);
     }
     // The kernel that stages the int8 rows in LDS once per workgroup and shares
     // them between several row blocks: fewer activation bytes through L2 than
@@ -3944,6 +3969,13 @@ int bitlinear_norm_epilogue_applies(int M, int N, int K, const int* seg_ends, in
     ScaleMap sm = equal_slots(N, bitlinear_ws_num(N, K));
     if (seg_ends && segment_map(seg_ends, nseg, N, &sm) != BITLINEAR_OK) return 0;
     return ring_choice(M, N, K, sm, K % 128 == 0) != 0;
+}
+
+int bitlinear_norm_gate_ahead(int M, int N, int K, const int* seg_ends, int nseg) {
+    if (!bitlinear_norm_epilogue_applies(M, N, K, seg_ends, nseg)) return 0;
+    ScaleMap sm = equal_slots(N, bitlinear_ws_num(N, K));
+    if (seg_ends) segment_map(seg_ends, nseg, N, &sm);
+    return gate_ahead(M, N, K, ring_choice(M, N, K, sm, true));
 }
 
 int bitlinear_norm_gate_forward_bf16(const uint16_t* x, const uint16_t* norm_weight, float eps, const int8_t* packed,

@@ -334,6 +334,13 @@ def _epilogue_applies(x, norm: "RMSNorm", lin: BitLinearKernel) -> bool:
                 x.shape[0], lin.out_features, lin.in_features, lin._seg_c, len(lin.seg_ends) if lin.seg_ends else 0) != 0)
 
 
+def gate_epilogue_ahead(rows: int, w13: BitLinearKernel) -> bool:
+    """Whether norm_gate_bitlinear is ahead of the separate calls for that many rows: not everywhere that it applies, since
+    those may take another GEMM kernel."""
+    return _lib.load_library().bitlinear_norm_gate_ahead(
+        rows, w13.out_features, w13.in_features, w13._seg_c, len(w13.seg_ends) if w13.seg_ends else 0) != 0
+
+
 def norm_gate_bitlinear(x, norm: "RMSNorm", w13: BitLinearKernel):
     """RMSNorm -> w13 -> squared-ReLU gate in one norm / quantizer kernel and one GEMM (bitlinear_norm_gate_forward_bf16):
     x bf16 [M, K] -> bf16 [M, ffn], or None where the separate calls have to be made."""
@@ -622,7 +629,7 @@ class Transformer(nn.Module):
                 q = rope_cache_tokens(xqkv, ck, cv, pos, cos, sin, a.n_heads, a.n_kv_heads)
             o = attn_prefill(q, ck, cv, 0)
             h = norm_bitlinear(o, att.attn_sub_norm, att.wo, residual=h)
-            gated = norm_gate_bitlinear(h, layer.ffn_norm, ffn.w13)
+            gated = norm_gate_bitlinear(h, layer.ffn_norm, ffn.w13) if gate_epilogue_ahead(B * T, ffn.w13) else None
             if gated is None:
                 x13 = norm_bitlinear(h, layer.ffn_norm, ffn.w13)
                 h = norm_bitlinear(x13, ffn.ffn_sub_norm, ffn.w2, glu=True, residual=h)

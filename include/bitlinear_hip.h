@@ -301,10 +301,14 @@ int bitlinear_norm_forward_bf16_seg(const uint16_t* x, const uint16_t* norm_weig
  *     bitnet_rope_cache_tokens makes of the product's rows, same operands.
  * Values are those of the separate calls, bit for bit (a NaN may be another one).  seg_ends / nseg as in
  * bitlinear_norm_forward_bf16_seg, NULL: the equal slots.  BITLINEAR_ERR_SHAPE where bitlinear_norm_epilogue_applies
- * (host only) says 0: M <= 16, K % 128 != 0, N % 32 != 0, scale segments that end elsewhere than at multiples of 8, and
- * outputs that another GEMM kernel is ahead on (the separate calls choose it).  All pointers 16-byte aligned.
+ * (host only) says 0: M <= 16, K % 128 != 0, K < 640 or more than the norm's kernel holds, N % 32 != 0, scale segments that
+ * end elsewhere than at multiples of 8, and outputs of which the GEMM kernel with these epilogues has no tile that gives
+ * about one per CU, or only one that it is not used with.  For some of the outputs that it does take, the separate calls
+ * choose another GEMM kernel.  With rope the one call is ahead there all the same; with the gate it is not always, and
+ * bitlinear_norm_gate_ahead (host only) says 1 where the call applies and is ahead.  All pointers 16-byte aligned.
  */
 int bitlinear_norm_epilogue_applies(int M, int N, int K, const int* seg_ends, int nseg);
+int bitlinear_norm_gate_ahead(int M, int N, int K, const int* seg_ends, int nseg);
 int bitlinear_norm_gate_forward_bf16(const uint16_t* x, const uint16_t* norm_weight, float eps,
                                      const int8_t* packed, const uint16_t* ws,
                                      const int* seg_ends, int nseg, uint16_t* output0,

@@ -41,6 +41,33 @@ def test_plan_rows_say_what_the_design_says():
     assert p(0, 1, 20480, 3200).startswith("bitlinear_fused_kernel<")
 
 
+def test_the_gate_is_in_the_epilogue_only_where_that_is_ahead():
+    """Against what the separate product would take: the launch with two tile sizes (ahead with 256-k chunks and at most one small
+    tile per CU), the split-K kernel (ahead), the kernel with the epilogues (behind)."""
+    lib = _lib.load_library()
+    seen = set()
+    for k in (640, 1152, 2560, 3200, 4096):
+        for n in (1024, 2048, 4096, 5120, 8192, 10240, 11264, 13824, 20480):
+            for m in (16, 17, 24, 33, 64, 129, 200, 256, 257, 300, 321, 352, 384, 400, 448, 512, 640, 800, 1088, 1300, 2048):
+                applies, ahead = lib.bitlinear_norm_epilogue_applies(m, n, k, None, 0), lib.bitlinear_norm_gate_ahead(m, n, k, None, 0)
+                product = _lib.plan_name(2, m, n, k).split(" + ")[-1]
+                if "gemm_i2_prefill_mix_kernel" in product:
+                    groups = int(product.split("grid=(")[1].split(",")[0])
+                    rt = -(-m // 64)
+                    bigs = min(256 * max(1, -(-n // 256) * rt // 256) // rt, n // 256) * rt
+                    # (both kinds are rounded up to eight in the grid)
+                    behind = k % 256 == 0 and groups - -(-bigs // 8) * 8 <= 256
+                else:
+                    behind = "gemv" in product
+                want = int(applies and not behind)
+                assert ahead == want, (m, n, k, product)
+                seen.add((applies, ahead, product.split("<")[0]))
+    assert {(1, 0, "gemm_i2_prefill_mix_kernel"), (1, 1, "gemm_i2_prefill_mix_kernel"), (1, 0, "gemv_i2_mfma_kernel"),
+            (1, 1, "gemm_i2_prefill_kernel"), (0, 0, "gemm_i2_prefill_mix_kernel")} <= seen, seen
+    # the 2B decoder's w13
+    assert [lib.bitlinear_norm_gate_ahead(m, 13824, 2560, None, 0) for m in (32, 257, 320, 321, 512, 513)] == [1, 0, 0, 1, 1, 0]
+
+
 def test_plan_name_argument_checks():
     import ctypes
 
