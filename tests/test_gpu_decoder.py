@@ -884,10 +884,10 @@ def _equal_or_both_nan(a, b):
     return bool(torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(a.nan_to_num(7.0), b.nan_to_num(7.0)))
 
 
-@pytest.mark.parametrize("where", ["row", "value", "infinity", "large", "all bits set"])
+@pytest.mark.parametrize("where", ["row", "value", "infinity", "last of four", "large", "all bits set"])
 @pytest.mark.parametrize("B,dim,ffn,nh,nkv", [
     (1, 128, 64, 1, 1), (2, 1152, 2112, 9, 9), (1, 2560, 6912, 20, 5),
-    # quantized rows between the workgroups: whole words of the code of a NaN, which is also what an unwritten word holds
+    # quantized rows between the workgroups; "last of four": the codes 0, 0, 0 and a NaN's, the word that one not yet written holds
     (3, 128, 64, 1, 1), (4, 2560, 6912, 20, 5), (5, 1152, 2112, 9, 9), (8, 2560, 6912, 20, 5),
 ])
 def test_decode_stack_kernel_carries_values_that_are_not_finite_like_the_kernels_per_layer(B, dim, ffn, nh, nkv, where):
@@ -903,6 +903,8 @@ def test_decode_stack_kernel_carries_values_that_are_not_finite_like_the_kernels
     elif where == "infinity":  # the norm makes zeros of the finite values, a NaN of this one
         emb[b, 5] = float("-inf")
         emb[b, 64:72] = float("inf")
+    elif where == "last of four":
+        emb[b, dim // 2 + 11] = float("inf")
     elif where == "all bits set":  # the NaN that a value of the hand-over buffers holds before it is written
         emb.view(torch.int16)[b, dim // 2 : dim // 2 + 2] = -1
     else:  # the sum of squares is infinite, the values are not
