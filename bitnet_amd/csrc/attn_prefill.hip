@@ -79,7 +79,9 @@ __device__ __forceinline__ void ap_load(__amdgpu_buffer_rsrc_t rsrc, uint8_t* to
 
 // What bounds it: a step is some 200 instructions of the one wave on a SIMD and a chain of LDS reads, four dependent MFMAs,
 // the maximum, the exponentials (0.56 us; 512 tokens are 16 steps).  Rows that came a step ahead through registers had not
-// arrived in time: 512 tokens 12.9 -> 12.0 us, 1000 29.9 -> 26.7, 2048 77.6 -> 53.9 (20 / 5 heads).
+// arrived in time: 512 tokens 12.9 -> 12.0 us, 1000 29.9 -> 26.5, 2048 77.6 -> 66.7 (20 / 5 heads).  The ring is RING - 1 steps
+// ahead from step 0 on, not in front of it: q, first in the source, is loaded by the generated code behind the ring's first
+// requests and the first barrier, and its wait for all loads drains the ring once per tile.
 template <int G, int RING>
 __global__ __launch_bounds__(64 * G) void attn_prefill_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ cache_k, const uint16_t* __restrict__ cache_v,

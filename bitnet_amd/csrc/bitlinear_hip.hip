@@ -2300,8 +2300,9 @@ constexpr int kSoloMaxK = 8192;
 // 3.95 -> 3.80, 13824 x 2560 5.44 -> 5.16; 2560 x 6912 with gate and residual 5.87 -> 6.12, not taken)
 constexpr int kSoloLongRowK = 4096;
 // rows from which the norm + quantizer kernel of a prompt runs a wave per row (K = 2560, a workgroup per row against that:
-// 200 rows 2.95 us against 3.44, 300 3.56 / 3.49, 512 3.75 / 3.56, 600 4.37 / 3.68, 800 4.99 / 3.96; a prompt pass of 600 rows
-// 2954 -> 2904 us, of 1000 4550 -> 4440, of 300 level)
+// 200 rows 2.95 us against 3.44, 300 3.56 / 3.49, 512 3.75 / 3.56, 600 4.37 / 3.68, 800 4.99 / 3.96).  From 300 to 511 rows it is
+// ahead by 0.04 to 0.2 us of a launch, which a prompt pass does not show: 300 rows 2236 .. 2246 us against 2246, 384 2420 .. 2431
+// against 2414 .. 2418, 448 2519 .. 2527 against 2518; from 512 on it does: 2630 .. 2641 against 2622, 600 3141 against 3082
 constexpr int kNormRowsPerWaveMinRows = 512;
 // --- prefill GEMM: tile and k-split by the number of tiles ------------------
 // up to this many 64 x 128 tiles the GEMM uses 32 x 128 tiles (M = 128: 11.4 -> 9.0 us at 3840 x 2560, 21.5 -> 16.4
@@ -2325,7 +2326,13 @@ constexpr int kPrefillRound64 = 768, kPrefillRound128 = 1024;
 constexpr int kPrefillMixCus = 256;
 constexpr int kPrefillMixMaxQuarters = 360;
 // the GEMM kernel with both operands in LDS (gemm_ring.h; its instances at BITLINEAR_RING_A): the smallest of its tiles of
-// which there is at most one per CU, because a tile's time hardly depends on how many there are until then.  Over 110
+// which there is at most one per CU, because a tile's time hardly depends on how many there are until then -- but not where
+// there are more 32 x 64 tiles than that and at most as many of 32 x 128: those, with k-groups in registers, are ahead (160 x
+// 3840 x 2560 6.6 us against 7.7 in 64 x 128 tiles of this kernel and 9.5 in 32 x 64, 256 7.0 against 8.0, 48 x 13824 x 2560
+// 7.4 / 8.3, 300 x 2560 x 2560 6.8 / 7.9, 300 x 2560 x 6912 11.7 / 13.3, 384 13.0 / 13.7).  The products with rope or gate in the
+// epilogue follow the same line (bitlinear_norm_epilogue_applies), though with rope 64 x 128 tiles would be ahead below it: prompt
+// passes of the 2B decoder of 144, 192 and 256 tokens 1771, 1852 and 2055 us, with wqkv so 1658, 1720 and 1933; with
+// the gate not (48 tokens 1363 against 1387).  Over 110
 // random shapes of 17 to 2048 tokens against the kernels below: 32 x 64 tiles 1.19 times as fast (101 x 3840 x 2560
 // 6.6 -> 5.6 us, 32 x 2560 x 6912 11.0 -> 7.8), 64 x 128 1.18 (512 x 3840 x 2560 9.4 -> 8.4, 512 x 2560 x 6912
 // 17.4 -> 13.1), 64 x 256 1.19 (513 x 4800 x 3200 21.9 -> 14.4), 128 x 256 1.15 (512 x 13824 x 2560 23.2 -> 20.6)

@@ -7,7 +7,9 @@
 // one CU at 2.4 GHz):
 //  * loads bring 54 to 60 bytes a cycle into a CU whatever they are, so a tile's bytes are worth as much attention as its
 //    multiplications (64 x 128: 96 bytes per k, 1.9 us at K = 2560).  Two thirds of LDS is ring, and the loads of S - 1
-//    stages are on their way before the first is waited for.
+//    stages are on their way before the first is waited for.  In the generated code the waves that multiply also
+//    wait, in front of the first barrier, for all of their own loads, because of the weight scales among them.  Loader waves
+//    have none of those; in the instance without them (32 x 64) wave 0 waits so for all S - 1 stages, at K = 2560 for all of K.
 //  * a wave that issues a load waits while the path is taken by others, and does not multiply meanwhile.  So LW further
 //    waves do nothing but load (512 x 3840 x 2560: 9.2 -> 8.6 us); the 32 x 64 tile's eight computing waves issue their
 //    few loads between the MFMAs instead (5.6 against 6.2 us).
@@ -18,7 +20,8 @@
 //    of a stage, sums go through LDS once, and with KG = 1 not at all (512 x 13824 x 2560: 21.2 -> 20.2 us).
 // One barrier per stage: behind it the next stage is complete for every wave, so the first operands of a stage are read
 // while the one in front is still being multiplied, and the stage before that is free for the loaders.  Requests behind
-// the end of K fetch nothing and bring zeros, so every wait counts the same number of requests.
+// the end of K fetch nothing and bring zeros, so every wait counts the same number of requests: S - 1 stages of them, whose
+// zeros are written into LDS and waited for at the end (a good part of the work of short rows: kRingMinK).
 // Codes are expanded to bytes that read 64 w, as in gemm_i2_prefill_dma_kernel, which also defines the interleaved column
 // tiles of a wave.  K % 128 == 0.
 #ifndef BITNET_AMD_GEMM_RING_H
@@ -180,7 +183,8 @@ void gemm_i2_prefill_kernel(
     constexpr int ROWS = R::WAVES * 64 / PER_ROW;  // rows that the threads cover at a time
     constexpr int TIMES = (R::TM + ROWS - 1) / ROWS;
     const int pr = threadIdx.x / PER_ROW, pc = threadIdx.x % PER_ROW * 8, n = n_base + pc;
-    // the scales, for the epilogue: requested behind the first stages, in LDS before the sums are
+    // the scales, for the epilogue: requested behind the first stages, in LDS before the sums are.  (The weight scales are waited
+    // for where they are requested, see the top.)
     __shared__ float sval[R::TM], rinv[R::TM], wsv[kMaxSeg];
     uint16_t s_raw = 0, ws_raw = 0;
     if (has_out) {
