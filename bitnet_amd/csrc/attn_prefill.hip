@@ -15,6 +15,7 @@
 
 #include "attn_device.h"
 #include "bitnet_decoder_ops.h"
+#include "host_util.h"
 
 namespace {
 
@@ -71,7 +72,8 @@ __global__ __launch_bounds__(kRopeThreads) void rope_cache_tokens_kernel(
 //   lane (c, g4) then holds, for token c, dims 32 g4 + 8 j + t: eight contiguous dims per j.
 // Online softmax per 32 positions: the running maximum of a token is agreed between its four lanes
 // (c, c + 16, c + 32, c + 48) with two lane permutes; the sums stay per lane until the end.
-constexpr int kApStepBytes = 2 * 32 * kHeadDim * 2;  // K and V rows of a step
+constexpr int kApRowsBytes = 32 * kHeadDim * 2;  // K or V rows of a step
+constexpr int kApStepBytes = 2 * kApRowsBytes;   // both
 // 16 bytes per lane from a buffer straight into LDS: lane l's piece lands at `to` + 16 l (wave-uniform)
 __device__ __forceinline__ void ap_load(__amdgpu_buffer_rsrc_t rsrc, uint8_t* to, int offset) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)to, 16, offset, 0, 0, 0);
@@ -82,15 +84,20 @@ __device__ __forceinline__ void ap_load(__amdgpu_buffer_rsrc_t rsrc, uint8_t* to
 // arrived in time: 512 tokens 12.9 -> 12.0 us, 1000 29.9 -> 26.5, 2048 77.6 -> 66.7 (20 / 5 heads).  The ring is RING - 1 steps
 // ahead from step 0 on, not in front of it: q, first in the source, is loaded by the generated code behind the ring's first
 // requests and the first barrier, and its wait for all loads drains the ring once per tile.
+// Workgroups start in the order of their index, so the heads and sequences are its fast part and the blocks of tokens its
+// slow one, those with the most positions first: with the blocks as the fast part the longest of the last heads started last
+// and stood alone at the end (2048 tokens 66.6 -> 44.8 us, 8 sequences of 512 35.5 -> 25.9, 4 of 1024 53.8 -> 40.7).
+// Taken where there are more than two workgroups per CU, which hide one another's waits (attn_prefill_split_kernel below:
+// 8 sequences of 512 31.5 us).
 template <int G, int RING>
 __global__ __launch_bounds__(64 * G) void attn_prefill_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ cache_k, const uint16_t* __restrict__ cache_v,
-    uint16_t* __restrict__ out, int T, int S, int start, int n_heads, int n_kv_heads) {
+    uint16_t* __restrict__ out, int T, int S, int start, int n_heads, int n_kv_heads, int last_block) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int c = lane & 15, g4 = lane >> 4;
-    const int qb = gridDim.x - 1 - blockIdx.x;  // the blocks with the most positions start first
-    const int kvh = blockIdx.y, b = blockIdx.z;
+    const int qb = last_block - blockIdx.z;  // the blocks with the most positions start first
+    const int kvh = blockIdx.x, b = blockIdx.y;
     const int head = kvh * G + wave;
     const int t0 = qb * 16;
     const int tq = (t0 + c) < T ? (t0 + c) : (T - 1);
@@ -243,6 +250,241 @@ __global__ __launch_bounds__(64 * G) void attn_prefill_kernel(
 
     const float l_tot = over_rows(l_run, [](float a, float b) { return a + b; });
     const float inv = 1.0f / l_tot;
+    if (t0 + c < T) {
+        uint16_t* orow = out + ((size_t)b * T + t0 + c) * n_heads * kHeadDim + (size_t)head * kHeadDim + 32 * g4;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            v4u w;
+            w.x = pack_bf16x2(o_acc[0][j] * inv, o_acc[1][j] * inv);
+            w.y = pack_bf16x2(o_acc[2][j] * inv, o_acc[3][j] * inv);
+            w.z = pack_bf16x2(o_acc[4][j] * inv, o_acc[5][j] * inv);
+            w.w = pack_bf16x2(o_acc[6][j] * inv, o_acc[7][j] * inv);
+            *(v4u*)(orow + 8 * j) = w;
+        }
+    }
+}
+
+
+// The same attention with two waves per head: one makes the scores and probabilities of a step, the other multiplies the
+// probabilities of the step before with V; they pass through LDS with the factor that the outputs so far are scaled with.  One
+// more wave does nothing but request rows.  One barrier per step; the results are those of attn_prefill_kernel bit for bit.
+//
+// What bounds it: the chain of steps (512 tokens: 16) and in it the wave of the scores, whose maximum, exponentials and LDS
+// reads follow one another.  In the kernel above a step is some 200 instructions of the one wave on a SIMD, 0.53 us, of which
+// the requests are 0.1 (sixteen of them hold the load path for 256 cycles, and a wave that issues one waits).  Here, with
+// the next step's scores among this step's exponentials, it is 0.37.  20 / 5 heads, kernel above -> here: 64 tokens 4.2 -> 4.2
+// us, 512 11.9 -> 9.4, 900 19.0 -> 14.0, 1024 21.8 -> 15.9, 3 x 224 7.2 -> 6.4, 2 x 512 12.9 -> 9.8.  Behind were: the
+// exponentials in the wave of the outputs (13.2 at 512), waves that take two heads and half of V's dims, for half of its
+// LDS reads (10.9), requests by the computing waves (9.7), rows three steps ahead (10.0: a ring of five slots takes a
+// division).  Without any one part it takes 8.7 .. 9.4: none is the bound alone.
+//
+// Rows come AHEAD steps in front of their use: the rings hold what is read (K by the wave of the scores a step early, V a
+// step late), what is on its way, and for K the slot that the first scores are still read from when the requests of step 0 go out
+constexpr int kApAhead = 2;
+template <int G, int AHEAD>
+struct ApRing {
+    static constexpr int KR = AHEAD + 2, VR = AHEAD + 2;
+    static constexpr int P_BYTES = 64 * 16, A_BYTES = 16 * 4;  // of a head and step: the lanes' probabilities; the tokens' factors
+    static constexpr int LDS = (KR + VR) * kApRowsBytes + 2 * G * (P_BYTES + A_BYTES);
+    static constexpr int THREADS = 64 * (2 * G + 1);
+    static_assert((AHEAD - 1) * 16 <= 63, "loads in flight are counted in six bits");
+    static_assert(LDS <= 160 * 1024, "LDS of a CU");
+};
+template <int G, int AHEAD>
+__global__ __launch_bounds__((ApRing<G, AHEAD>::THREADS)) void attn_prefill_split_kernel(
+    const uint16_t* __restrict__ q, const uint16_t* __restrict__ cache_k, const uint16_t* __restrict__ cache_v,
+    uint16_t* __restrict__ out, int T, int S, int start, int n_heads, int n_kv_heads, int heads_per_kv, int last_block) {
+    typedef ApRing<G, AHEAD> R;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c = lane & 15, g4 = lane >> 4;
+    const int qb = last_block - blockIdx.z;  // the blocks with the most positions start first
+    const int kvh = blockIdx.x * G / heads_per_kv, b = blockIdx.y;
+    const int part = wave % G;  // of the workgroup's heads (both waves of a head; the requesting wave has none)
+    const int head = blockIdx.x * G + part;
+    const int t0 = qb * 16;
+    const int n_pos = start + ((t0 + 16) < T ? (t0 + 16) : T);  // rows [0, n_pos) matter to this block
+    const int steps = (n_pos + 31) >> 5;
+
+    extern __shared__ __attribute__((aligned(1024))) uint8_t lds_kv[];  // K ring [KR][32 rows of 256 bytes], V ring [VR]
+    uint8_t* const lds_v = lds_kv + R::KR * kApRowsBytes;
+    uint8_t* const lds_p = lds_v + R::VR * kApRowsBytes;         // [2][G]: probabilities of this step and the one before
+    float* const lds_a = (float*)(lds_p + 2 * G * R::P_BYTES);   // [2][G]: what the outputs so far are scaled with
+    // what this wave has read and written in LDS is read and written, then all waves meet
+    auto meet = [&] {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0xc07f);
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+
+    if (wave == 2 * G) {
+        // Cache rows through descriptors that end behind row n_pos - 1: requests beyond read as zero
+        // at no cost, so neither the last step nor the prefetch past it needs a clamped index, and no
+        // stale row behind the prompt can put a NaN into the products.  A request fills 1 KB, four rows, whose 16-byte
+        // pieces are swizzled by the row (by choice of the piece that a lane fetches), so that 16 rows at one piece and
+        // the 16 pieces of a row are both spread over all banks.
+        const int row_bytes = n_kv_heads * kHeadDim * 2;
+        const int span_bytes = (n_pos - 1) * row_bytes + kHeadDim * 2;
+        const __amdgpu_buffer_rsrc_t k_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            (void*)(cache_k + ((size_t)b * S * n_kv_heads + kvh) * kHeadDim), 0, span_bytes, 0x00020000);
+        const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            (void*)(cache_v + ((size_t)b * S * n_kv_heads + kvh) * kHeadDim), 0, span_bytes, 0x00020000);
+        int off[8];
+#pragma unroll
+        for (int r = 0; r < 8; ++r) off[r] = (r * 4 + g4) * row_bytes + (c ^ ((r * 4 + g4) & 15)) * 16;
+        auto request = [&](__amdgpu_buffer_rsrc_t rsrc, uint8_t* to, int st) {
+            // (in the per-lane operand: that is the one the range check looks at; unsigned, as it may lie behind 2^31 there)
+            const unsigned base = (unsigned)st * 32u * (unsigned)row_bytes;
+#pragma unroll
+            for (int r = 0; r < 8; ++r) ap_load(rsrc, to + r * 1024, (int)(base + (unsigned)off[r]));
+        };
+        // the K rows of a step together with the V rows of the step in front of it, in the order of their use
+        auto request_pair = [&](int st) {
+            request(k_rsrc, lds_kv + (st + 1) % R::KR * kApRowsBytes, st + 1);
+            request(v_rsrc, lds_v + st % R::VR * kApRowsBytes, st);
+        };
+        constexpr int kYounger = (AHEAD - 1) * 16, kWait = 0x0f70 | (kYounger & 15) | ((kYounger >> 4) << 14);
+        request(k_rsrc, lds_kv, 0);
+#pragma unroll
+        for (int st = 0; st < AHEAD; ++st) request_pair(st);
+        __builtin_amdgcn_s_waitcnt(kWait);
+        meet();
+        for (int st = 0; st < steps; ++st) {
+            // (into the slots of K rows st - 1 and V rows st - 2, which were last read in the step before)
+            request_pair(st + AHEAD);
+            __builtin_amdgcn_s_waitcnt(kWait);
+            meet();
+        }
+        __builtin_amdgcn_s_waitcnt(0x0f70);  // nothing may arrive in LDS behind the workgroup's end
+        meet();
+        return;
+    }
+
+    if (wave < G) {
+        const int tq = (t0 + c) < T ? (t0 + c) : (T - 1);
+        const int pq = start + t0 + c;  // position of this lane's token: cache rows 0..pq are visible to it
+        // q^T as the B operand of the four 32-dim steps
+        v8bf qa[4];
+        const uint16_t* qrow = q + (((size_t)b * T + tq) * n_heads + head) * kHeadDim;
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) qa[kk] = __builtin_bit_cast(v8bf, *(const uint4*)(qrow + kk * 32 + g4 * 8));
+        int k_off[4];  // row c of a 16-row block, piece kk * 4 + g4
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) k_off[kk] = c * 256 + (((kk * 4 + g4) ^ c) * 16);
+        auto read_k = [&](int st, v4u(&kb)[8]) {
+            const uint8_t* kl = lds_kv + st % R::KR * kApRowsBytes;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) kb[i] = *(const v4u*)(kl + (i & 1) * 16 * 256 + k_off[i >> 1]);
+        };
+        // raw scores of 32 positions: the i-th of eight products (two blocks of 16, four pieces of the dims)
+        auto product = [&](int i, const v4u(&kb)[8], v4f(&acc)[2]) {
+            acc[i & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, kb[i]), qa[i >> 1], acc[i & 1], 0, 0, 0);
+        };
+        // softmax in base 2: exp(x * scale - m) = exp2(x * c2 - m2) with c2 = scale * log2(e); the running
+        // maximum m_run is kept in raw score units (the scale is positive, so maxima commute with it)
+        float m_run = -INFINITY, l_run = 0.0f;
+        const float c2 = 0.08838834764831845f * 1.4426950408889634f;  // 128^-0.5 * log2(e)
+        // probabilities of a step from its scores, and the scores of the step behind it
+        auto step = [&](int st, const v4f(&acc)[2], v4f(&next)[2]) {
+            v4u kb[8];
+            read_k(st + 1, kb);
+            __builtin_amdgcn_sched_barrier(0);
+            float sc[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) sc[i] = acc[i >> 2][i & 3];
+            // only the steps that reach beyond the block's first token need the causal mask (uniform test)
+            if (st * 32 + 31 > start + t0) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const int pos = st * 32 + (i >> 2) * 16 + 4 * g4 + (i & 3);
+                    sc[i] = pos <= pq ? sc[i] : -INFINITY;
+                }
+            }
+            float mx = fmaxf(fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3])), fmaxf(fmaxf(sc[4], sc[5]), fmaxf(sc[6], sc[7])));
+            mx = over_rows(mx, [](float a, float b) { return fmaxf(a, b); });
+            const float m_new = fmaxf(m_run, mx);  // finite from the first step on: position 0 is visible to every token
+            const float m2 = m_new * c2;
+            float p[8], psum = 0.0f;
+            next[0] = next[1] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                p[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(sc[i], c2, -m2));
+                product(i, kb, next);
+                psum += p[i];
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            // sum and outputs so far are rescaled only when some token's maximum has moved (uniform test): after the
+            // first few steps it rarely does
+            float alpha = 1.0f;
+            if (__builtin_amdgcn_ballot_w64(m_new != m_run) != 0) {
+                alpha = __builtin_amdgcn_exp2f(__builtin_fmaf(m_run, c2, -m2));
+                l_run *= alpha;
+                m_run = m_new;
+            }
+            l_run += psum;
+            const int slot = (st & 1) * G + part;
+            *(v4u*)(lds_p + slot * R::P_BYTES + lane * 16) =
+                v4u{pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3]), pack_bf16x2(p[4], p[5]), pack_bf16x2(p[6], p[7])};
+            if (g4 == 0) lds_a[slot * 16 + c] = alpha;
+            meet();
+        };
+        meet();
+        v4f scores[2][2];
+        {
+            v4u kb[8];
+            read_k(0, kb);
+            scores[0][0] = scores[0][1] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int i = 0; i < 8; ++i) product(i, kb, scores[0]);
+        }
+        for (int st = 0; st < steps; st += 2) {
+            step(st, scores[0], scores[1]);
+            if (st + 1 < steps) step(st + 1, scores[1], scores[0]);
+        }
+        const float l_tot = over_rows(l_run, [](float a, float b) { return a + b; });
+        if (g4 == 0) lds_a[((steps & 1) * G + part) * 16 + c] = 1.0f / l_tot;
+        meet();
+        return;
+    }
+
+    int v_off[4];  // rows 4 g4 + jj (and 16 + 4 g4 + jj), piece c
+#pragma unroll
+    for (int jj = 0; jj < 4; ++jj) v_off[jj] = (4 * g4 + jj) * 256 + ((c ^ (4 * g4 + jj)) * 16);
+    v4f o_acc[8];
+#pragma unroll
+    for (int t = 0; t < 8; ++t) o_acc[t] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    meet();
+    meet();  // the probabilities of step 0
+    for (int st = 0; st < steps; ++st) {
+        const uint8_t* vl = lds_v + st % R::VR * kApRowsBytes;
+        const int slot = (st & 1) * G + part;
+        const v8bf pb = __builtin_bit_cast(v8bf, *(const v4u*)(lds_p + slot * R::P_BYTES + lane * 16));
+        const float alpha = lds_a[slot * 16 + c];
+        v4u vb[8];
+#pragma unroll
+        for (int jj = 0; jj < 8; ++jj) vb[jj] = *(const v4u*)(vl + (jj >> 2) * 16 * 256 + v_off[jj & 3]);
+        __builtin_amdgcn_sched_barrier(0);
+        if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
+#pragma unroll
+            for (int t = 0; t < 8; ++t)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) o_acc[t][j] *= alpha;
+        }
+#pragma unroll
+        for (int t = 0; t < 8; ++t) {
+            const uint32_t sel = (t & 1) ? 0x07060302u : 0x05040100u;  // both high halves / both low halves
+            v4u va;
+            va.x = __builtin_amdgcn_perm(vb[1][t >> 1], vb[0][t >> 1], sel);
+            va.y = __builtin_amdgcn_perm(vb[3][t >> 1], vb[2][t >> 1], sel);
+            va.z = __builtin_amdgcn_perm(vb[5][t >> 1], vb[4][t >> 1], sel);
+            va.w = __builtin_amdgcn_perm(vb[7][t >> 1], vb[6][t >> 1], sel);
+            o_acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, va), pb, o_acc[t], 0, 0, 0);
+        }
+        meet();
+    }
+    const float inv = lds_a[((steps & 1) * G + part) * 16 + c];
     if (t0 + c < T) {
         uint16_t* orow = out + ((size_t)b * T + t0 + c) * n_heads * kHeadDim + (size_t)head * kHeadDim + 32 * g4;
 #pragma unroll
@@ -538,23 +780,42 @@ extern "C" int bitnet_attn_prefill(const uint16_t* q, const uint16_t* cache_k, c
     if (B > 65535 || n_kv_heads > 65535) return 1;
     if (!q || !cache_k || !cache_v || !out) return 2;
     if ((((uintptr_t)q) | ((uintptr_t)cache_k) | ((uintptr_t)cache_v) | ((uintptr_t)out)) & 15u) return 1;
-    const dim3 grid((T + 15) / 16, n_kv_heads, B), block(64 * g, 1, 1);
-    // four steps of rows are 64 KB of LDS, so two workgroups to a CU; with more than that to do three steps and three
-    // workgroups (8 sequences of 512 tokens 40.4 -> 36.0 us; 512 tokens alone 12.0 against 12.4)
-    const bool many = (long long)grid.x * n_kv_heads * B > 2 * 256;
-#define BITNET_AP(G)                                                                                                                    \
-    if (many)                                                                                                                           \
-        hipLaunchKernelGGL((attn_prefill_kernel<G, 3>), grid, block, 3 * kApStepBytes, (hipStream_t)stream, q, cache_k, cache_v, out, T, S, \
-                           start, n_heads, n_kv_heads);                                                                                 \
-    else                                                                                                                                \
-        hipLaunchKernelGGL((attn_prefill_kernel<G, 4>), grid, block, 4 * kApStepBytes, (hipStream_t)stream, q, cache_k, cache_v, out, T, S, \
-                           start, n_heads, n_kv_heads)
-    switch (g) {
-        case 1: BITNET_AP(1); break;
-        case 2: BITNET_AP(2); break;
-        case 4: BITNET_AP(4); break;
-        default: BITNET_AP(8); break;
+    // A workgroup of attn_prefill_split_kernel takes up to four heads, of attn_prefill_kernel all of a kv head's.  The former is
+    // ahead while its workgroups are at most two per CU, which is what fits: 20 / 5 heads, the former against the latter, 1500
+    // tokens (470) 23.9 against 30.8 us, 2 x 700 (440) 14.4 against 17.0, 4 x 300 (380) 9.5 against 9.7; 2048 tokens (640) 42.8 against
+    // 44.8, but 2 x 1024 (640) 26.2 against 25.4, 8 x 256 (640) 13.6 against 11.1, 4 x 1024 (1280) 46.7 against 40.7.
+    const int gs = g < 4 ? g : 4;
+    const int blocks = (T + 15) / 16;
+    const bool split = (long long)blocks * (n_heads / gs) * B <= 2 * 256;
+    if (split) {
+        // more LDS than the 64 KiB that a kernel gets without asking (a host-side attribute, set once per device)
+        static bitnet_host::OncePerDevice raised;
+        const hipError_t e = raised.run([] {
+            return hipFuncSetAttribute((const void*)attn_prefill_split_kernel<4, kApAhead>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       ApRing<4, kApAhead>::LDS);
+        });
+        if (e != hipSuccess) return 3;
     }
+#define BITNET_AP_SPLIT(G)                                                                                                        \
+    hipLaunchKernelGGL((attn_prefill_split_kernel<G, kApAhead>), dim3(n_heads / gs, B, here), dim3(ApRing<G, kApAhead>::THREADS),  \
+                       (ApRing<G, kApAhead>::LDS), (hipStream_t)stream, q, cache_k, cache_v, out, T, S, start, n_heads, n_kv_heads, g, \
+                       last)
+#define BITNET_AP(G)                                                                                                                \
+    hipLaunchKernelGGL((attn_prefill_kernel<G, 3>), dim3(n_kv_heads, B, here), dim3(64 * G), 3 * kApStepBytes, (hipStream_t)stream, q,  \
+                       cache_k, cache_v, out, T, S, start, n_heads, n_kv_heads, last)
+    for (int last = blocks - 1; last >= 0; last -= 65535) {  // (what a grid's third dimension holds)
+        const int here = last + 1 < 65535 ? last + 1 : 65535;
+        switch (split ? gs : g + 8) {
+            case 1: BITNET_AP_SPLIT(1); break;
+            case 2: BITNET_AP_SPLIT(2); break;
+            case 4: BITNET_AP_SPLIT(4); break;
+            case 9: BITNET_AP(1); break;
+            case 10: BITNET_AP(2); break;
+            case 12: BITNET_AP(4); break;
+            default: BITNET_AP(8); break;
+        }
+    }
+#undef BITNET_AP_SPLIT
 #undef BITNET_AP
     return hipGetLastError() == hipSuccess ? 0 : 3;
 }

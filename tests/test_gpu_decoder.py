@@ -696,6 +696,25 @@ def test_prompt_attention_of_many_sequences_equals_each_alone(nh, nkv, T):
         assert not torch.isnan(alone).any() and torch.equal(alone, many[b])
 
 
+@pytest.mark.parametrize("nh,nkv,start", [(64, 16, 0), (64, 16, 21), (32, 32, 3), (64, 8, 16)])
+def test_prompt_attention_at_the_edge_between_its_two_kernels(nh, nkv, start):
+    """The longest prompt with two workgroups per CU and one of a block more, which goes through the other kernel: the rows that
+    both have are the same bits, also where a key's infinities make scores infinite and NaN for the tokens that see it."""
+    heads = min(nh // nkv, 4)
+    blocks = 512 // (nh // heads)
+    T, S = 16 * blocks, start + 16 * blocks + 40
+    gen = torch.Generator(device="cuda").manual_seed(nh + start)
+    q = torch.randn(1, T + 16, nh, 128, generator=gen, device="cuda").to(torch.bfloat16)
+    k, v = (torch.randn(1, S, nkv, 128, generator=gen, device="cuda").to(torch.bfloat16) for _ in range(2))
+    k[0, start + T - 70, 0, :5] = float("inf")
+    k[0, start + T - 40, nkv - 1, 7] = float("-inf")
+    longer = decoder.attn_prefill(q, k, v, start).view(T + 16, nh, 128)[:T]
+    edge = decoder.attn_prefill(q[:, :T].contiguous(), k, v, start).view(T, nh, 128)
+    assert torch.isnan(edge).any() and not torch.isnan(edge[: T - 70]).any()
+    assert torch.equal(torch.isnan(edge), torch.isnan(longer))
+    assert torch.equal(edge.nan_to_num(), longer.nan_to_num())
+
+
 def _norm_and_linear(K, N, gen, segments=None):
     norm = decoder.RMSNorm(K, 1e-5).cuda().to(torch.bfloat16)
     norm.weight.data = torch.rand(K, generator=gen, device="cuda").add(0.5).to(torch.bfloat16)
