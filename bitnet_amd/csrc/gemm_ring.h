@@ -6,10 +6,16 @@
 // 240 tiles of 64 x 128: 9.4 us, of which the matrix instructions are 2.2).  Measured here, on a lone tile (cycles of
 // one CU at 2.4 GHz):
 //  * loads bring 54 to 60 bytes a cycle into a CU whatever they are, so a tile's bytes are worth as much attention as its
-//    multiplications (64 x 128: 96 bytes per k, 1.9 us at K = 2560).  Two thirds of LDS is ring, and the loads of S - 1
-//    stages are on their way before the first is waited for.  In the generated code the waves that multiply also
-//    wait, in front of the first barrier, for all of their own loads, because of the weight scales among them.  Loader waves
-//    have none of those; in the instance without them (32 x 64) wave 0 waits so for all S - 1 stages, at K = 2560 for all of K.
+//    multiplications (64 x 128: 96 bytes per k, 1.9 us at K = 2560).  Two thirds of LDS is ring.
+//  * the first stages are there some 2000 cycles behind the start, of which half is the trip to memory.  So three stages are
+//    requested, two waited for, and the ring is filled up beside the first two chunks: with S - 1 stages in front of
+//    the first wait it ended after 3050 cycles (512 x 2560 x 2560 7.95 -> 7.6 us).  The instance without loader waves
+//    requests S - 1 stages at once, and waits for the first two alone: a weight scale that is converted where it is
+//    loaded makes the wave wait for all its requests there, at K = 2560 for all of K.
+//  * a request behind the end of K costs what any other does (its zeros are written into LDS), so there are none: the last
+//    S - 1 chunks wait for fewer and fewer stages.  Both together: 101 x 3840 x 2560 5.35 -> 4.9 us, 60 x 2560 x 640 4.3 -> 3.8.
+//  * what the epilogue reads from memory (residual, scales, angles) is requested in front of the exchange of the sums
+//    (norm, wo and residual of 512 tokens 12.9 -> 12.5 us, norm, w2 and residual 20.9 -> 20.0).
 //  * a wave that issues a load waits while the path is taken by others, and does not multiply meanwhile.  So LW further
 //    waves do nothing but load (512 x 3840 x 2560: 9.2 -> 8.6 us); the 32 x 64 tile's eight computing waves issue their
 //    few loads between the MFMAs instead (5.6 against 6.2 us).
@@ -19,9 +25,11 @@
 //    different slots of the 256 bytes that the banks span), writes at 76: with KG groups of waves that split the k-steps
 //    of a stage, sums go through LDS once, and with KG = 1 not at all (512 x 13824 x 2560: 21.2 -> 20.2 us).
 // One barrier per stage: behind it the next stage is complete for every wave, so the first operands of a stage are read
-// while the one in front is still being multiplied, and the stage before that is free for the loaders.  Requests behind
-// the end of K fetch nothing and bring zeros, so every wait counts the same number of requests: S - 1 stages of them, whose
-// zeros are written into LDS and waited for at the end (a good part of the work of short rows: kRingMinK).
+// while the one in front is still being multiplied, and the stage before that is free for the loaders.  (Behind the last
+// chunk operands are read from a stage that was not requested; nothing multiplies them.)
+// Beyond a tile's start and end it is the matrix instructions: 512 x 13824 x 2560 in 128 x 256 tiles is 13.3 us per 2560 k and
+// 7.4 us besides, 11.0 on zeros (what the pipe's clock makes of the operands), and the same with half the expansions and two
+// thirds of the LDS reads (a wave's tile 128 x 64), with seven instructions a word instead of eight, and with two k-groups.
 // Codes are expanded to bytes that read 64 w, as in gemm_i2_prefill_dma_kernel, which also defines the interleaved column
 // tiles of a wave.  K % 128 == 0.
 #ifndef BITNET_AMD_GEMM_RING_H
@@ -71,10 +79,17 @@ struct RingRope {
     uint16_t *cache_k, *cache_v, *q_out;
     int T, S, n_heads, n_kv;
 };
-typedef float v4f_ring __attribute__((ext_vector_type(4)));
+// N words, two or four, in one piece
+template <int N>
+struct RingWords {
+    typedef uint32_t type __attribute__((ext_vector_type(N)));
+};
+// a token's position, and the angles of N neighbouring pairs there
+template <int N>
 struct RingTurn {
+    typedef float angles __attribute__((ext_vector_type(N)));
     int p;
-    v4f_ring cs, sn;
+    angles cs, sn;
 };
 constexpr int kRingBeyond = 0x7ffffff0;  // an offset behind every descriptor: nothing is fetched, zeros arrive
 
@@ -138,60 +153,110 @@ void gemm_i2_prefill_kernel(
     // part p of P of a stage's requests
     auto issue = [&](int c, int st, int p, int P) {
         const int left = K - c * CK;  // k in front of the end of the rows
-        const int cc = left > 0 ? c : 0;
         int8_t* to = lds_x + st * R::STAGE;
 #pragma unroll
         for (int r = 0; r < R::LOADS; ++r) {
             if (r * P / R::LOADS != p) continue;
             if (r < R::AR) {
-                load16_to_lds(a_rsrc, to + (r * R::LWAVES + lw) * 1024, a_k[r] < left ? a_voff[r] : kRingBeyond, cc * CK);
+                load16_to_lds(a_rsrc, to + (r * R::LWAVES + lw) * 1024, a_k[r] < left ? a_voff[r] : kRingBeyond, c * CK);
             } else {
                 const int i = r - R::AR;
-                load16_to_lds(w_rsrc, to + R::A_BYTES + (i * R::LWAVES + lw) * 1024, w_k[i] < left ? w_voff[i] : kRingBeyond, cc * (CK * 4));
+                load16_to_lds(w_rsrc, to + R::A_BYTES + (i * R::LWAVES + lw) * 1024, w_k[i] < left ? w_voff[i] : kRingBeyond, c * (CK * 4));
             }
         }
     };
-    constexpr int kYounger = (S - 3) * R::LOADS;
-    constexpr int kWaitYounger = 0x0f70 | (kYounger & 15) | ((kYounger >> 4) << 14);
+    // all of a wave's requests have arrived but those of its last `stages` stages
+    auto wait_all_but = [](auto stages) {
+        constexpr int n = decltype(stages)::value * R::LOADS;
+        __builtin_amdgcn_s_waitcnt(0x0f70 | (n & 15) | (n >> 4 << 14));
+    };
+    constexpr std::integral_constant<int, 0> none{};
+    constexpr std::integral_constant<int, 1> one_stage{};
+    constexpr std::integral_constant<int, 2> two_stages{};
+    constexpr std::integral_constant<int, S - 3> full{};  // the ring's stages behind the two that are in use
     auto meet = [&] {
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
     };
+    constexpr int kFirst = LW ? 3 : S - 1;  // stages requested in front of the first wait
     if (lw >= 0) {
 #pragma unroll
-        for (int c = 0; c < S - 1; ++c) issue(c, c, 0, 1);
+        for (int c = 0; c < kFirst; ++c)
+            if (c < nchunks) issue(c, c, 0, 1);
     }
     if (LW && lw >= 0) {
-        __builtin_amdgcn_s_waitcnt(kWaitYounger);
-        meet();
-        int st = S - 1;
-        for (int c = 0; c < nchunks; ++c) {
-            issue(c + S - 1, st, 0, 1);
-            st = st + 1 == S ? 0 : st + 1;
-            __builtin_amdgcn_s_waitcnt(kWaitYounger);
+        // at the end of chunk c stage c + 2 has to be there
+        if (nchunks <= S) {  // all of K fits the ring
+            wait_all_but(none);
             meet();
+            for (int c = kFirst; c < nchunks; ++c) issue(c, c, 0, 1);
+            wait_all_but(none);
+            for (int c = 0; c < nchunks; ++c) meet();
+        } else {
+            wait_all_but(one_stage);
+            meet();
+            int c = 0, st = kFirst % S;
+            auto next_stage = [&](int i) {
+                issue(i, st, 0, 1);
+                st = st + 1 == S ? 0 : st + 1;
+            };
+            if constexpr (S > 4) {  // two stages at a time until S - 1 are on their way
+                static_assert(S == 6, "two chunks of two stages");
+                next_stage(3);
+                next_stage(4);
+                wait_all_but(two_stages);
+                meet();
+                next_stage(5);
+                next_stage(6);
+                wait_all_but(full);
+                meet();
+                c = 2;
+            }
+            for (; c + S - 1 < nchunks; ++c) {
+                next_stage(c + S - 1);
+                wait_all_but(full);
+                meet();
+            }
+            if constexpr (S > 4) {
+                wait_all_but(two_stages);
+                meet();
+                wait_all_but(one_stage);
+                meet();
+            }
+            wait_all_but(none);
+            for (int i = 0; i < 3; ++i) meet();
         }
-        __builtin_amdgcn_s_waitcnt(0x0f70);
         meet();
         lds_barrier();
         return;
     }
 
-    // the outputs that go through LDS: eight of a row per thread
-    constexpr int PER_ROW = COLS / 8;              // threads that share a row
+    // the outputs that go through LDS: eight of a row per thread, four where there are fewer
+    constexpr int CPT = KG > 1 && R::TM * COLS < R::WAVES * 64 * 8 ? 4 : 8;
+    constexpr int PER_ROW = COLS / CPT;            // threads that share a row
     constexpr int ROWS = R::WAVES * 64 / PER_ROW;  // rows that the threads cover at a time
     constexpr int TIMES = (R::TM + ROWS - 1) / ROWS;
-    const int pr = threadIdx.x / PER_ROW, pc = threadIdx.x % PER_ROW * 8, n = n_base + pc;
-    // the scales, for the epilogue: requested behind the first stages, in LDS before the sums are.  (The weight scales are waited
-    // for where they are requested, see the top.)
+    const int pr = threadIdx.x / PER_ROW, pc = threadIdx.x % PER_ROW * CPT, n = n_base + pc;
+    // the scales, for the epilogue
     __shared__ float sval[R::TM], rinv[R::TM], wsv[kMaxSeg];
-    uint16_t s_raw = 0, ws_raw = 0;
+    uint32_t s_raw = 0, ws_raw = 0;
     if (has_out) {
         const int m = m0 + (int)threadIdx.x;
         if (threadIdx.x < R::TM) s_raw = s[m < M ? m : M - 1];
         if (threadIdx.x < kMaxSeg) ws_raw = ws[(int)threadIdx.x < smap.nseg ? threadIdx.x : 0];
     }
+    auto put_scales = [&] {
+        asm volatile("" : "+v"(s_raw), "+v"(ws_raw));  // (converted here and not where they are loaded, see the top)
+        if (threadIdx.x < R::TM) {
+            const float sv = bf16_to_f32((uint16_t)s_raw);
+            sval[threadIdx.x] = sv;
+            rinv[threadIdx.x] = 1.0f / sv;
+        }
+        if (threadIdx.x < kMaxSeg) wsv[threadIdx.x] = bf16_to_f32((uint16_t)ws_raw);
+    };
+    // with loader waves while the first stages are on their way (in the instances without k-groups behind the loop measures 0.3 us less)
+    if (LW && KG > 1) put_scales();
     // ... as are the positions of this thread's outputs
     int64_t at[KG > 1 ? TIMES : MT] = {};
     if constexpr (Epi::kRope) {
@@ -240,7 +305,10 @@ void gemm_i2_prefill_kernel(
             return *(const wvec_t*)from;
     };
     // stages 0 and 1 are there (every wave waits for its own requests, then all meet)
-    if (!LW) __builtin_amdgcn_s_waitcnt(kWaitYounger);
+    if (!LW) {
+        if (nchunks < S - 1) wait_all_but(none);
+        else wait_all_but(full);
+    }
     meet();
 
     v4i aop[2][MT], bop[2][NT];
@@ -252,11 +320,12 @@ void gemm_i2_prefill_kernel(
     for (int nt = 0; nt < NT; ++nt) bop[0][nt] = expand(wraw[0][nt]);
 
     int st = 0;
-    for (int c = 0; c < nchunks; ++c) {
+    // chunk c; `load`: and part by part the requests of stage c + S - 1, into the stage in front of this one, which was read in
+    // the chunk before and every wave has left
+    auto chunk = [&](int c, auto load) {
         const int8_t* here = lds_x + st * R::STAGE;
         const int st1 = st + 1 == S ? 0 : st + 1;
         const int8_t* next = lds_x + st1 * R::STAGE;
-        // the stage in front of this one was read in the chunk before, which every wave has left
         constexpr int SLOTS = MT * NT;
 #pragma unroll
         for (int j = 0; j < R::KPW; ++j) {
@@ -273,18 +342,38 @@ void gemm_i2_prefill_kernel(
 #pragma unroll
                 for (int i = 0; i < NT; ++i)
                     if ((i * SLOTS / NT + (SLOTS > NT ? 1 : 0)) % SLOTS == slot) bop[nxt][i] = expand(wraw[nxt][i]);
-                if (!LW && slot == SLOTS - 1) issue(c + S - 1, st == 0 ? S - 1 : st - 1, j, R::KPW);
+                if (load.value && slot == SLOTS - 1) issue(c + S - 1, st == 0 ? S - 1 : st - 1, j, R::KPW);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
-        // the chunk behind the next one has to be there before the next one ends
-        if (!LW) __builtin_amdgcn_s_waitcnt(kWaitYounger);
-        meet();
         st = st1;
+    };
+    if constexpr (LW > 0) {
+        for (int c = 0; c < nchunks; ++c) {
+            chunk(c, std::false_type{});
+            meet();
+        }
+    } else {
+        for (int c = 0; c + S - 1 < nchunks; ++c) {
+            chunk(c, std::true_type{});
+            wait_all_but(full);  // the chunk behind the next one has to be there before the next one ends
+            meet();
+        }
+        auto last = [&](auto behind) {  // ... that has `behind` chunks behind it
+            constexpr int n = decltype(behind)::value;
+            if (nchunks <= n) return;
+            chunk(0, std::false_type{});
+            wait_all_but(std::integral_constant<int, (n > 2 ? n - 2 : 0)>{});
+            meet();
+        };
+        static_assert(S == 6, "S - 1 chunks without requests");
+        last(std::integral_constant<int, 4>{});
+        last(std::integral_constant<int, 3>{});
+        last(std::integral_constant<int, 2>{});
+        last(std::integral_constant<int, 1>{});
+        last(std::integral_constant<int, 0>{});
     }
 
-    // the groups' accumulators: each finishes the register quads q with q % KG == group
-    constexpr int QUADS = MT * 4;
     // the reference's epilogue (the bits of the IEEE divide by the token's scale from its reciprocal and one correction
     // step, as in gemm_i2_prefill_kernel): two neighbouring sums -> packed bf16
     auto result2 = [](int x, int y, float sv, float ri, float w) {
@@ -300,27 +389,29 @@ void gemm_i2_prefill_kernel(
         const uint32_t sq = f32x2_to_bf16x2(r0 * r0, r1 * r1);
         return f32x2_to_bf16x2(low(sq) * low(x3), high(sq) * high(x3));
     };
-    // a token's position and the angles of four pairs
+    constexpr int PAIRS = CPT / 2;  // of neighbouring outputs, a word each
+    typedef typename RingWords<PAIRS>::type words_t;
+    typedef RingTurn<PAIRS> turn_t;
     auto turn_of = [&](int64_t at, int n) {
-        RingTurn t = {};
+        turn_t t = {};
         if constexpr (Epi::kRope) {
             t.p = at < 0 ? 0 : (at >= (int64_t)epi.S ? epi.S - 1 : (int)at);  // nothing outside the buffers is touched
-            t.cs = *(const v4f_ring*)(epi.cos_t + (size_t)t.p * 64 + (n & 127) / 2);
-            t.sn = *(const v4f_ring*)(epi.sin_t + (size_t)t.p * 64 + (n & 127) / 2);
+            t.cs = *(const typename turn_t::angles*)(epi.cos_t + (size_t)t.p * 64 + (n & 127) / 2);
+            t.sn = *(const typename turn_t::angles*)(epi.sin_t + (size_t)t.p * 64 + (n & 127) / 2);
         }
         return t;
     };
-    // eight consecutive outputs of one token from their sums
-    auto store8 = [&](int m, int n, const int(&x)[8], float sv, float ri, float w, const RingTurn& turn) {
+    // CPT consecutive outputs of one token from their sums
+    auto store = [&](int m, int n, const int(&x)[CPT], float sv, float ri, float w, const turn_t& turn, auto residual_here) {
         const size_t o = (size_t)m * N + n;
         if (!Epi::kRope && acc_out) {
-            *(v4i*)(acc_out + o) = v4i{x[0], x[1], x[2], x[3]};
-            *(v4i*)(acc_out + o + 4) = v4i{x[4], x[5], x[6], x[7]};
+#pragma unroll
+            for (int i = 0; i < CPT; i += 4) *(v4i*)(acc_out + o + i) = v4i{x[i], x[i + 1], x[i + 2], x[i + 3]};
         }
         if (!has_out) return;
-        uint32_t ob[4];
+        words_t ob;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) ob[i] = result2(x[2 * i], x[2 * i + 1], sv, ri, w);
+        for (int i = 0; i < PAIRS; ++i) ob[i] = result2(x[2 * i], x[2 * i + 1], sv, ri, w);
         if constexpr (Epi::kRope) {
             const int head = n >> 7, in = n & 127;
             uint16_t* to = epi.q_out + ((size_t)m * epi.n_heads + head) * 128 + in;
@@ -331,27 +422,21 @@ void gemm_i2_prefill_kernel(
             }
             if (head < epi.n_heads + epi.n_kv) {
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
+                for (int i = 0; i < PAIRS; ++i)
                     ob[i] = f32x2_to_bf16x2(low(ob[i]) * turn.cs[i] - high(ob[i]) * turn.sn[i], low(ob[i]) * turn.sn[i] + high(ob[i]) * turn.cs[i]);
             }
-            *(uint4*)to = make_uint4(ob[0], ob[1], ob[2], ob[3]);
+            *(words_t*)to = ob;
         } else {
             if (residual) {  // out = bf16(residual + bf16(result))
-                const uint4 rv = *(const uint4*)(residual + o);
-                const uint32_t r4[4] = {rv.x, rv.y, rv.z, rv.w};
+                const words_t res = residual_here(o);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) ob[i] = f32x2_to_bf16x2(low(r4[i]) + low(ob[i]), high(r4[i]) + high(ob[i]));
+                for (int i = 0; i < PAIRS; ++i) ob[i] = f32x2_to_bf16x2(low(res[i]) + low(ob[i]), high(res[i]) + high(ob[i]));
             }
-            *(uint4*)(out + o) = make_uint4(ob[0], ob[1], ob[2], ob[3]);
+            *(words_t*)(out + o) = ob;
         }
     };
-    __builtin_amdgcn_s_waitcnt(0x0f70);  // the requests behind the end write zeros into the ring
     meet();
-    if (threadIdx.x < R::TM) {
-        sval[threadIdx.x] = bf16_to_f32(s_raw);
-        rinv[threadIdx.x] = 1.0f / bf16_to_f32(s_raw);
-    }
-    if (threadIdx.x < kMaxSeg) wsv[threadIdx.x] = bf16_to_f32(ws_raw);
+    if (!LW || KG == 1) put_scales();
     if constexpr (KG == 1) {
         // every wave holds its sums whole: 4 NT consecutive columns per register quad, stored straight from the registers
         lds_barrier();
@@ -366,13 +451,16 @@ void gemm_i2_prefill_kernel(
         for (int mt = 0; mt < MT; ++mt) {
             const int row = (wm * MT + mt) * 32 + nl, m = m0 + row;
             const float sv = sval[row], ri = rinv[row];
+            auto column = [&](int g4) {  // the first of a register quad's columns
+                const int ridx = g4 * 8 + kc * 4;
+                return Epi::kGate ? nw + ridx : nw + 16 * (ridx / (2 * QR)) + 8 * ((ridx % (2 * QR)) / QR) + NT * (ridx % QR);
+            };
 #pragma unroll
             for (int g4 = 0; g4 < 4; ++g4) {
-                const int ridx = g4 * 8 + kc * 4;
+                const int n = column(g4);
+                if (m >= M || n >= n_out) continue;
                 int x[4 * NT];
                 if constexpr (Epi::kGate) {
-                    const int n = nw + ridx;
-                    if (m >= M || n >= n_out) continue;
                     const float wa = one_slot ? w1 : wsv[scale_slot(smap, n)], wb = one_slot ? w3 : wsv[scale_slot(smap, n_out + n)];
 #pragma unroll
                     for (int i = 0; i < 8; ++i) x[i] = acc[mt][i >> 2][g4 * 4 + (i & 3)] >> 6;
@@ -380,22 +468,29 @@ void gemm_i2_prefill_kernel(
                         make_uint2(gate2(result2(x[0], x[1], sv, ri, wa), result2(x[4], x[5], sv, ri, wb)),
                                    gate2(result2(x[2], x[3], sv, ri, wa), result2(x[6], x[7], sv, ri, wb)));
                 } else {
-                    const int n = nw + 16 * (ridx / (2 * QR)) + 8 * ((ridx % (2 * QR)) / QR) + NT * (ridx % QR);
 #pragma unroll
                     for (int i = 0; i < 4 * NT; ++i) x[i] = acc[mt][i % NT][g4 * 4 + i / NT] >> 6;
-                    if (m >= M || n >= N) continue;
-                    RingTurn turn = {};
+                    turn_t turn = {};
                     if constexpr (Epi::kRope) turn = turn_of(at[mt], n);
-                    store8(m, n, x, sv, ri, one_slot ? w1 : wsv[scale_slot(smap, n)], turn);
+                    store(m, n, x, sv, ri, one_slot ? w1 : wsv[scale_slot(smap, n)], turn, [&](size_t o) { return *(const words_t*)(residual + o); });
                 }
             }
         }
         return;
     }
-    RingTurn turn[TIMES] = {};
-    if constexpr (Epi::kRope) {
+    // requested in front of the exchange
+    turn_t turn[TIMES] = {};
+    words_t res[TIMES] = {};
 #pragma unroll
-        for (int i = 0; i < TIMES; ++i) turn[i] = turn_of(at[i], n);
+    for (int i = 0; i < TIMES; ++i) {
+        if constexpr (Epi::kRope) turn[i] = turn_of(at[i], n);
+    }
+    if (!Epi::kGate && !Epi::kRope && residual) {
+#pragma unroll
+        for (int i = 0; i < TIMES; ++i) {
+            const int row = i * ROWS + pr, m = m0 + row;
+            if (row < R::TM && m < M && n < N) res[i] = *(const words_t*)(residual + (size_t)m * N + n);
+        }
     }
     // The sums go through LDS, which adds the groups' shares and turns a lane's pieces of 32 rows into whole runs of a
     // row.  (A lane holds token nl; register quad g4 of its NT column tiles is 4 NT consecutive columns.)
@@ -423,35 +518,34 @@ void gemm_i2_prefill_kernel(
     lds_barrier();
     const float w = wsv[slot], w3 = wsv[slot3];
     // (exact: the accumulators are 64 * sum(w * a))
-    auto sums = [&](const int8_t* from, int(&x)[8]) {
-        v4i lo = *(const v4i*)from, hi = *(const v4i*)(from + 16);
+    auto sums = [&](const int8_t* from, int(&x)[CPT]) {
 #pragma unroll
-        for (int g = 1; g < KG; ++g) {
-            lo += *(const v4i*)(from + g * R::TM * R::OUT_ROW);
-            hi += *(const v4i*)(from + g * R::TM * R::OUT_ROW + 16);
+        for (int i = 0; i < CPT; i += 4) {
+            v4i t = *(const v4i*)(from + i * 4);
+#pragma unroll
+            for (int g = 1; g < KG; ++g) t += *(const v4i*)(from + g * R::TM * R::OUT_ROW + i * 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[i + e] = t[e] >> 6;
         }
-        lo >>= 6, hi >>= 6;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) x[i] = lo[i], x[4 + i] = hi[i];
     };
 #pragma unroll
     for (int p = 0; p < TIMES; ++p) {
         const int row = p * ROWS + pr, m = m0 + row;
-        if (row >= R::TM || m >= M || n >= n_out) continue;  // N % 16 == 0: the eight columns are in or out together
+        if (row >= R::TM || m >= M || n >= n_out) continue;  // N % 16 == 0: the columns are in or out together
         const int8_t* from = lds_x + row * R::OUT_ROW + pc * 4;
         const float sv = sval[row], ri = rinv[row];
-        int x[8];
+        int x[CPT];
         sums(from, x);
         if constexpr (Epi::kGate) {
-            int y[8];
+            int y[CPT];
             sums(from + COLS * 4, y);
-            uint32_t ob[4];
+            words_t ob;
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+            for (int i = 0; i < PAIRS; ++i)
                 ob[i] = gate2(result2(x[2 * i], x[2 * i + 1], sv, ri, w), result2(y[2 * i], y[2 * i + 1], sv, ri, w3));
-            *(uint4*)(out + (size_t)m * n_out + n) = make_uint4(ob[0], ob[1], ob[2], ob[3]);
+            *(words_t*)(out + (size_t)m * n_out + n) = ob;
         } else {
-            store8(m, n, x, sv, ri, w, turn[p]);
+            store(m, n, x, sv, ri, w, turn[p], [&](size_t) { return res[p]; });
         }
     }
 }
