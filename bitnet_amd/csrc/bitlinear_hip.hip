@@ -1065,7 +1065,30 @@ __device__ __forceinline__ void pfx_tile(
     const int n_last = (n0 + NT * 32 - 1) < N ? (n0 + NT * 32 - 1) : N - 1;
     const int slot_first = scale_slot(smap, n_first);
     const bool one_slot = slot_first == scale_slot(smap, n_last);
-    const float w1 = out ? bf16_to_f32(ws[slot_first]) : 1.0f;
+    // The weight scales of the lane's register quads.  Where the wave's columns share a slot that is one load; where the slots
+    // end at multiples of a quad's columns, one per quad, all in front of the outputs (loaded column by column where they are
+    // used 1024 x 4800 x 3200, whose slots of 800 end within a wave's 64 columns, took 28.2 us, now 20.4).
+    auto quad_column = [&](int g4) {
+        const int ridx = g4 * 8 + kc * 4;
+        return n0 + 16 * (ridx / (2 * QR)) + 8 * ((ridx % (2 * QR)) / QR) + NT * (ridx % QR);
+    };
+    bool quad_slots = true;
+    for (int j = 0; j + 1 < smap.nseg; ++j) quad_slots = quad_slots && smap.ends[j] % (4 * NT) == 0;
+    float wq4[4] = {1.0f, 1.0f, 1.0f, 1.0f};
+    if (out) {
+        if (one_slot) {
+            const float w1 = bf16_to_f32(ws[slot_first]);
+#pragma unroll
+            for (int g4 = 0; g4 < 4; ++g4) wq4[g4] = w1;
+        } else if (quad_slots) {
+#pragma unroll
+            for (int g4 = 0; g4 < 4; ++g4) {
+                const int n = quad_column(g4);
+                wq4[g4] = bf16_to_f32(ws[scale_slot(smap, n < N ? n : N - 1)]);
+            }
+        }
+    }
+    const bool by_quad = one_slot || quad_slots;
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
         const int m = m0 + mt * 32 + nl;
@@ -1074,8 +1097,7 @@ __device__ __forceinline__ void pfx_tile(
         if (m >= M) continue;
 #pragma unroll
         for (int g4 = 0; g4 < 4; ++g4) {
-            const int ridx = g4 * 8 + kc * 4;
-            const int n = n0 + 16 * (ridx / (2 * QR)) + 8 * ((ridx % (2 * QR)) / QR) + NT * (ridx % QR);
+            const int n = quad_column(g4);
             if (n >= N) continue;  // N % 16 == 0 and n % (4 * NT) == 0: the columns of a quad are in or out together
             const size_t o = (size_t)m * N + n;
             int sum[4 * NT];
@@ -1098,7 +1120,7 @@ __device__ __forceinline__ void pfx_tile(
                     const float a = (float)sum[col];
                     const float q0 = a * ri;
                     const float q = __builtin_fmaf(__builtin_fmaf(-q0, sv, a), ri, q0);
-                    h[col] = q * (one_slot ? w1 : bf16_to_f32(ws[scale_slot(smap, n + col)]));
+                    h[col] = q * (by_quad ? wq4[g4] : bf16_to_f32(ws[scale_slot(smap, n + col)]));
                 }
 #pragma unroll
                 for (int v = 0; v < NT / 2; ++v) {
@@ -2326,13 +2348,11 @@ constexpr int kPrefillRound64 = 768, kPrefillRound128 = 1024;
 constexpr int kPrefillMixCus = 256;
 constexpr int kPrefillMixMaxQuarters = 360;
 // the GEMM kernel with both operands in LDS (gemm_ring.h; its instances at BITLINEAR_RING_A): the smallest of its tiles of
-// which there is at most one per CU, because a tile's time hardly depends on how many there are until then -- but not where
-// there are more 32 x 64 tiles than that and at most as many of 32 x 128: those, with k-groups in registers, are ahead (160 x
-// 3840 x 2560 6.6 us against 7.7 in 64 x 128 tiles of this kernel and 9.5 in 32 x 64, 256 7.0 against 8.0, 48 x 13824 x 2560
-// 7.4 / 8.3, 300 x 2560 x 2560 6.8 / 7.9, 300 x 2560 x 6912 11.7 / 13.3, 384 13.0 / 13.7).  The products with rope or gate in the
-// epilogue follow the same line (bitlinear_norm_epilogue_applies), though with rope 64 x 128 tiles would be ahead below it: prompt
-// passes of the 2B decoder of 144, 192 and 256 tokens 1771, 1852 and 2055 us, with wqkv so 1658, 1720 and 1933; with
-// the gate not (48 tokens 1363 against 1387).  Over 110
+// which there is at most one per CU, because a tile's time hardly depends on how many there are until then.  64 x 64 tiles
+// against what was taken between 32 x 64 and 64 x 128 (32 x 128 tiles with k-groups in registers): 129 x 3840 x 2560 6.7 -> 5.8
+// us, 256 6.85 -> 6.05, 384 x 2560 x 2560 6.85 -> 6.05, 193 x 2560 x 6912 10.9 -> 9.4, 384 12.35 -> 9.95, 64 x 13824 x 2560
+// 6.85 -> 6.1, 100 x 4800 x 3200 7.8 -> 6.6; and where there are at most 256 of those 32 x 128 but more of 64 x 64 (65 to 96
+// rows) 64 x 128 ones, 96 x 9600 x 2560 9.0 -> 7.85, 90 x 10240 x 3200 10.75 -> 8.7.  Over 110
 // random shapes of 17 to 2048 tokens against the kernels below: 32 x 64 tiles 1.19 times as fast (101 x 3840 x 2560
 // 6.6 -> 5.6 us, 32 x 2560 x 6912 11.0 -> 7.8), 64 x 128 1.18 (512 x 3840 x 2560 9.4 -> 8.4, 512 x 2560 x 6912
 // 17.4 -> 13.1), 64 x 256 1.19 (513 x 4800 x 3200 21.9 -> 14.4), 128 x 256 1.15 (512 x 13824 x 2560 23.2 -> 20.6)
@@ -2340,10 +2360,11 @@ constexpr int kRingCus = 256;
 // ... of the 64 x 256 tiles two fit a CU: up to a third more of them (384 x 13824 x 2560, 324 tiles, 23.6 -> 19.7 us; as 162
 // tiles of 128 x 256 20.4; 512 x 13824 x 2560, 432 tiles, 24.6 against 22.6)
 constexpr int kRingMost64x256 = 340;
-// ... from this K on, below which requesting the stages behind the end costs more than the ring gains (380 x 976 x 256
-// 3.5 against 4.1 us, 51 x 3728 x 512 3.85 against 4.0); the 64 x 256 tiles later (76 x 17632 x 640 5.5 against 6.2,
-// 247 x 8384 x 1024 level), and not on very long rows, where two k-groups are ahead (705 x 3200 x 10240 32.4 against 33.9)
-constexpr int kRingMinK = 640, kRingMinK64x256 = 1024, kRingMaxK64x256 = 8192;
+// ... from this K on (128 x 2560 x 384 3.6 against 4.1 us, 512 x 2560 x 384 5.1 against 5.5; at K = 256 512 rows level, 300
+// 4.0 against 3.8); the 64 x 256 tiles later (76 x 17632 x 640 6.2 against 5.55, 247 x 8384 x 1024 7.4 against 7.5)
+constexpr int kRingMinK = 384, kRingMinK64x256 = 1024;
+// ... and with rope or gate in the epilogue from the K on that their entry points state
+constexpr int kRingEpilogueMinK = 640;
 }  // namespace dispatch
 using namespace dispatch;
 
@@ -2898,12 +2919,13 @@ int launch_solo_tok(const uint16_t* x, const int8_t* packed, uint16_t* out, int3
 }
 
 // The instances of the kernel in gemm_ring.h: 32 x 64 tiles whose K eight waves split, 64 x 128 tiles split by four, 64 x 256
-// (two workgroups per CU) and 128 x 256 tiles
+// (two workgroups per CU) and 128 x 256 tiles, 64 x 64 tiles split by four
 #define BITLINEAR_RING_A 1, 2, 1, 1, 8, 512, 6, 0
 #define BITLINEAR_RING_B 2, 2, 1, 2, 4, 256, 6, 4
 #define BITLINEAR_RING_C 2, 2, 1, 4, 1, 128, 4, 4
 #define BITLINEAR_RING_D 2, 2, 2, 4, 1, 128, 6, 4
-constexpr int kRingRows[5] = {0, 32, 64, 64, 128}, kRingCols[5] = {0, 64, 128, 256, 256};
+#define BITLINEAR_RING_E 2, 2, 1, 1, 4, 256, 6, 4
+constexpr int kRingRows[6] = {0, 32, 64, 64, 128, 64}, kRingCols[6] = {0, 64, 128, 256, 256, 64};
 long long ring_tiles(int M, int N, int ring) {
     return (long long)((M + kRingRows[ring] - 1) / kRingRows[ring]) * ((N + kRingCols[ring] - 1) / kRingCols[ring]);
 }
@@ -2920,9 +2942,9 @@ int ring_choice(int M, int N, int K, const ScaleMap& smap, bool aligned) {
     if (t_tune.path != 0) return 0;
     if (K < kRingMinK) return 0;
     if (ring_tiles(M, N, 1) <= kRingCus) return 1;
-    if ((long long)((M + 31) / 32) * ((N + 127) / 128) <= kRingCus) return 0;
+    if (ring_tiles(M, N, 5) <= kRingCus) return 5;
     if (ring_tiles(M, N, 2) <= kRingCus) return 2;
-    if (ring_tiles(M, N, 3) <= kRingMost64x256) return K >= kRingMinK64x256 && K <= kRingMaxK64x256 ? 3 : 0;
+    if (ring_tiles(M, N, 3) <= kRingMost64x256) return K >= kRingMinK64x256 ? 3 : 0;
     if (ring_tiles(M, N, 4) <= kRingCus) return 4;
     return 0;
 }
@@ -2952,9 +2974,17 @@ MixPlan plan_mix(int M, int N) {
 // 1.45 TB/s measured), finishes earlier.  Both estimates in microseconds, fitted to measurements at the 2B shapes.
 bool splitk_ahead(int M, int N, int K, int ring) {
     if (M > kSplitKMaxTokens || t_tune.path != 0) return false;
-    // the 32 x 64 tiles against the split-K kernel by rows, of which its last group may hold few (17 x 2560 x 2560
-    // 4.8 us against 5.3, 32 x 2560 x 2560 5.95 against 5.45, 17 x 3840 x 2560 5.6 against 5.3)
-    if (ring == 1) return 4.0 + 0.148 * (K / 256.0) > 3.5 + (M / 16.0) * ((double)N * K / 4.0) / 1.45e6;
+    // The ring kernel's tiles against the split-K kernel, whose time follows the rows (its last group may hold few).  Graph
+    // replays against these lines, 32 x 64 tiles / split-K: 17 x 2560 x 2560 4.7 / 4.9 us, 24 x 2560 x 2560 4.75 / 5.15, 17 x 3840 x 2560
+    // 4.75 / 5.65, 17 x 2560 x 6912 7.45 / 7.75, 17 x 2560 x 512 3.3 / 3.15, 51 x 2560 x 384 3.45 / 3.3, 51 x 1024 x 512 3.4 / 2.85, 51 x
+    // 3728 x 512 3.55 / 3.95, 128 x 2560 x 384 3.6 / 4.15, 200 x 1024 x 512 3.5 / 3.85; 64 x 64 4.1 at 200 x 2560 x 384, 5.75 at 193 x 2560 x
+    // 2560, 9.4 at 193 x 2560 x 6912; 64 x 128 4.7 at 100 x 10240 x 384, 7.3, 12.4
+    if (ring == 1 || ring == 2 || ring == 5) {
+        const double splitk_us = 2.6 + 1.09 * (M / 16.0) * ((double)N * K / 4.0) / 1.45e6 + 0.0004 * K;
+        const double chunks = K / 256.0;
+        const double ring_us = ring == 1 ? 3.2 + 0.148 * chunks + 0.002 * ring_tiles(M, N, 1) : (ring == 5 ? 3.7 + 0.21 * chunks : 4.2 + 0.29 * chunks);
+        return ring_us > splitk_us;
+    }
     const double groups = (M + 15) / 16;
     const double splitk_us = 3.5 + groups * ((double)N * K / 4.0) / 1.45e6;
     const double tiles = ((N + 127) / 128) * (double)((M + 63) / 64);
@@ -2980,6 +3010,10 @@ bool gate_ahead(int M, int N, int K, int ring) {
     const MixPlan mp = plan_mix(M, N);
     return !(mp.wanted && mp.quarters <= kGateMixQuarters && K % 256 == 0) && !splitk_ahead(M, N, K, ring);
 }
+// which instance a product with rope or gate in its epilogue takes; 0: none
+int epilogue_ring(int M, int N, int K, const ScaleMap& smap) {
+    return K < kRingEpilogueMinK && t_tune.path == 0 ? 0 : ring_choice(M, N, K, smap, K % 128 == 0);
+}
 template <class Epi>
 int launch_ring(int ring, const int8_t* act, const int8_t* packed, uint16_t* out, int32_t* acc_out, const uint16_t* s,
                 const uint16_t* ws, const ScaleMap& smap, int M, int N, int K, hipStream_t stream, const uint16_t* residual, Epi epi) {
@@ -2998,6 +3032,7 @@ int launch_ring(int ring, const int8_t* act, const int8_t* packed, uint16_t* out
         BITLINEAR_RING_LDS(BITLINEAR_RING_B);
         BITLINEAR_RING_LDS(BITLINEAR_RING_C);
         BITLINEAR_RING_LDS(BITLINEAR_RING_D);
+        BITLINEAR_RING_LDS(BITLINEAR_RING_E);
 #undef BITLINEAR_RING_LDS
         return e;
     });
@@ -3013,6 +3048,7 @@ int launch_ring(int ring, const int8_t* act, const int8_t* packed, uint16_t* out
         case 1: BITLINEAR_LAUNCH_RING(BITLINEAR_RING_A); break;
         case 2: BITLINEAR_LAUNCH_RING(BITLINEAR_RING_B); break;
         case 3: BITLINEAR_LAUNCH_RING(BITLINEAR_RING_C); break;
+        case 5: BITLINEAR_LAUNCH_RING(BITLINEAR_RING_E); break;
         default: BITLINEAR_LAUNCH_RING(BITLINEAR_RING_D); break;
     }
 #undef BITLINEAR_LAUNCH_RING
@@ -3054,9 +3090,13 @@ int launch_prefill(const int8_t* act, const int8_t* packed, uint16_t* out, int32
     // 28.5 -> 25.9, at 5120 39.4 -> 36.1; 2560 x 6912 41.0 -> 36.5 / 62.7 -> 57.3 / 91.4 -> 82.0; 3200 x 3200 at M = 1536
     // 22.4 -> 20.1, 2560 33.0 -> 28.5, 5120 58.0 -> 49.9, 20480 x 3200 at M = 617 46.1 -> 43.6; with more of them the even tiles are ahead: 2560 x 2560 at
     // M = 2560 21.3 against 26.5, 3840 x 2560 at M = 2048 22.8 against 28.0)
+    const int ring = ring_choice(M, N, K, smap, dma_fits);
     if (dma_fits && (t_tune.path == 0 || (t_tune.path == 5 && t_tune.prefill_big == 8))) {
         const MixPlan mp = plan_mix(M, N);
-        if ((t_tune.path == 5 || mp.wanted) && mp.groups < kMostTiles) {
+        // (with more than one small tile per CU the ring kernel's 64 x 256 tiles are ahead of it where they are few enough: 352 x
+        // 13824 x 2560 18.9 us against 19.3, 384 x 13824 x 3200 22.0 against 23.4, 640 x 8192 x 3200 22.0 against 23.6; with fewer not, 300 x
+        // 13824 x 2560 18.3 against 16.2, 1500 x 3200 x 3200, 235 of them, 21.8 against 19.8)
+        if ((t_tune.path == 5 || (mp.wanted && !(ring == 3 && mp.quarters > kPrefillMixCus))) && mp.groups < kMostTiles) {
             const int nbig = 8 * (int)((mp.bigs + 7) / 8);
             const dim3 mgrid((unsigned)mp.groups, 1, 1), mblock(256, 1, 1);
             const unsigned magic = tile_magic(mp.rt64, mp.big_cols), small_magic = tile_magic(mp.rt32, mp.small_cols);
@@ -3070,7 +3110,6 @@ int launch_prefill(const int8_t* act, const int8_t* packed, uint16_t* out, int32
             return launch_status();
         }
     }
-    const int ring = ring_choice(M, N, K, smap, dma_fits);
     if (ring) {
         return launch_ring(ring, act, packed, out, acc_out, s, ws, smap, M, N, K, stream, residual, RingPlain{});
     }
@@ -3557,7 +3596,7 @@ int bitlinear_set_tuning(int kernel, int a, int b, int c) {
         return set_status(BITLINEAR_OK);
     }
     if (kernel == 5) {
-        if (a < 0 || a > 12 || b < 0 || b > 64 || (c != 0 && c != 1 && c != 2 && c != 4)) return set_status(BITLINEAR_ERR_ARG);
+        if (a < 0 || a > 13 || b < 0 || b > 64 || (c != 0 && c != 1 && c != 2 && c != 4)) return set_status(BITLINEAR_ERR_ARG);
         g.path = 5;
         g.prefill_big = a;
         g.prefill_ks = c;
@@ -3961,7 +4000,7 @@ static int norm_ring_impl(const uint16_t* x, const uint16_t* norm_weight, float 
         const int st = segment_map(seg_ends, nseg, N, &sm);
         if (st != BITLINEAR_OK) return set_status(st);
     }
-    const int ring = M > kPrefillMinTokens && K <= kPreThreads * kPreVecs * 8 ? ring_choice(M, N, K, sm, K % 128 == 0) : 0;
+    const int ring = M > kPrefillMinTokens && K <= kPreThreads * kPreVecs * 8 ? epilogue_ring(M, N, K, sm) : 0;
     if (!ring || (Epi::kGate && N % 32)) return set_status(BITLINEAR_ERR_SHAPE);
     const int st = launch_norm_quant(x, norm_weight, eps, 0, q_ws, s_ws, M, K, mode, (hipStream_t)stream);
     if (st != BITLINEAR_OK) return set_status(st);
@@ -3975,7 +4014,7 @@ int bitlinear_norm_epilogue_applies(int M, int N, int K, const int* seg_ends, in
     if (!shape_ok(M, N, K) || N % 32 || M <= kPrefillMinTokens || K > kPreThreads * kPreVecs * 8) return 0;
     ScaleMap sm = equal_slots(N, bitlinear_ws_num(N, K));
     if (seg_ends && segment_map(seg_ends, nseg, N, &sm) != BITLINEAR_OK) return 0;
-    return ring_choice(M, N, K, sm, K % 128 == 0) != 0;
+    return epilogue_ring(M, N, K, sm) != 0;
 }
 
 int bitlinear_norm_gate_ahead(int M, int N, int K, const int* seg_ends, int nseg) {

@@ -587,6 +587,38 @@ def test_prefill_gemm_with_both_operands_through_lds(m, n, k, tile):
     _assert_bits_equal(host_bits(out_res), want_res, "with residual")
 
 
+@pytest.mark.parametrize("m,n,k", [(17, 16, 128), (33, 80, 384), (64, 64, 512), (65, 528, 896), (129, 1040, 1408), (257, 3840, 2560)])
+def test_prefill_gemm_in_64_x_64_tiles(m, n, k):
+    test_prefill_gemm_with_both_operands_through_lds(m, n, k, 13)
+
+
+@pytest.mark.parametrize("tile", [9, 10, 11, 12, 13])
+@pytest.mark.parametrize("k", [128, 512, 640, 768, 1024, 1152, 1536, 1792, 2048, 2432, 3072, 3584, 4096])
+def test_prefill_gemm_through_lds_from_the_first_stage_to_the_last(k, tile):
+    """Chunk counts (K over 512, 256 or 128) below, at and above the stages of each instance's ring, which is filled up
+    beside the first chunks and emptied beside the last."""
+    test_prefill_gemm_with_both_operands_through_lds(49, 96, k, tile)
+
+
+@pytest.mark.parametrize("m,n,k", [(600, 4800, 640), (1100, 4800, 1152), (300, 5120, 640)])
+@pytest.mark.parametrize("tile", [5, 6, 7, 8])
+def test_prefill_gemm_with_slots_that_end_within_a_waves_columns(m, n, k, tile):
+    """Weight scales by register quad: slots that end at multiples of a quad's eight columns, at others, and at the last row block."""
+    w, a = _rand_case(n, k, m, seed=m + n + k)
+    s_bits = o.f32_to_bf16_bits(np.linspace(3.0, 90.0, m).astype(np.float32))
+    ws_bits = o.f32_to_bf16_bits(np.array([0.0161, 0.0247, 0.0093, 0.031, 0.0112, 0.0204], dtype=np.float32))
+    lib = _lib.load_library()
+    for ends in ([800, 1608, 2400, 3208, n - 16, n], [804, 1600, 2412, n]):
+        want = o.bitlinear_int8xint2_seg(a, w, s_bits, ws_bits, ends)[1]
+        try:
+            assert lib.bitlinear_set_tuning(5, tile, 0, 0) == 0
+            out = bitlinear.bitnet_int8xint2_linear_seg(dev_i8(a), _packed_dev(w), dev_bf16(s_bits), dev_bf16(ws_bits), ends)
+            torch.cuda.synchronize()
+        finally:
+            lib.bitlinear_set_tuning(0, 0, 0, 0)
+        _assert_bits_equal(host_bits(out), want, f"tile {tile} segments {ends}")
+
+
 @pytest.mark.parametrize("m,n,k", [(17, 48, 128), (33, 16, 256), (64, 272, 384), (65, 1040, 640), (100, 2560, 768), (128, 2560, 2560),
                                    (129, 3840, 2560), (300, 1040, 3200), (512, 2560, 6912), (1000, 13824, 2560)])
 def test_prefill_gemm_through_the_direct_to_lds_kernel(m, n, k):

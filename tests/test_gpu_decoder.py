@@ -768,6 +768,11 @@ def test_prompt_products_with_rope_and_gate_in_the_epilogue_equal_the_separate_c
         assert np.array_equal(host_bits(got_h), want_h)
 
 
+@pytest.mark.parametrize("B,T,nh,nkv,K,ffn,S", [(1, 17, 1, 1, 640, 16, 17), (1, 33, 20, 5, 2560, 6912, 40), (3, 65, 20, 5, 1280, 1040, 200)])
+def test_prompt_products_with_epilogues_in_64_x_64_tiles_equal_the_separate_calls(B, T, nh, nkv, K, ffn, S):
+    test_prompt_products_with_rope_and_gate_in_the_epilogue_equal_the_separate_calls(B, T, nh, nkv, K, ffn, S, 13)
+
+
 def test_prompt_products_that_the_epilogues_do_not_take_are_left_to_the_separate_calls():
     gen = torch.Generator(device="cuda").manual_seed(3)
     for M, K, ffn, ends in ((16, 2560, 6912, None), (512, 2496, 6912, None), (512, 2560, 6912, (6900, 13824)), (4096, 2560, 6912, None),
