@@ -1951,6 +1951,96 @@ __global__ __launch_bounds__(kMaxWaves * 64) void bitlinear_solo_kernel(
 }
 
 // ---------------------------------------------------------------------------
+// The quantizer in the product's launch: the first workgroups quantize a row each and hand it on
+// ---------------------------------------------------------------------------
+// Of a call that is not part of a graph the second launch costs the host more than the GPU needs for the quantizer (9 x 3840 x 2560:
+// the host issues the two launches in 7.5 us, their kernels take 5.7 in a chain).  So workgroup r quantizes row r before its share of
+// the product, with all its waves, and publishes it: the int8 values by write-through stores, and when those are acknowledged a
+// flag word that holds the row's scale and the launch's tag.  Every workgroup's first wave polls the flags of its rows past the
+// caches; the rows themselves are then ordinary loads, which the XCD's L2 serves from the second workgroup on: nobody has read
+// their lines in this launch before they were published.  Weights are requested behind the publishing (in front of it
+// the acknowledgement waits for them too: 8 x 2560 x 6912 7.6 us instead of 7.0).
+//
+// The flag words lie in the library's image, one set per launch in turn, and a set's tag is another each time (the
+// number of the turn), so they are never cleared and a stale word is never taken for one of this launch.  That does not hold
+// for a launch that is recorded once and replayed: under a capture the two launches are made.  Two launches that overlap
+// on the same set after a full turn overwrite each other's words; a workgroup that waits in vain, for this or for any other
+// reason (its producer has not been started), stops after a bounded number of polls and quantizes what it misses itself,
+// to the same bytes: no wait depends on the order in which workgroups start.
+constexpr int kHandSets = 256, kHandRows = 16;
+static __device__ unsigned long long hand_flags[kHandSets][kHandRows];
+constexpr int kHandPolls = 512;  // some hundreds of microseconds; a wait is one or two
+
+struct HandedRows {
+    static constexpr bool kGiven = false;
+    const uint16_t* x;
+    int8_t* q;
+    uint16_t* s;
+    int set, polls;
+    unsigned tag;
+
+    __device__ __forceinline__ void put(int8_t* row, int vec, uint2 v) const {
+        __hip_atomic_store((unsigned long long*)row + vec, (unsigned long long)v.y << 32 | v.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    // the workgroup's rows, of M of K values, with all of its threads, a vector of 8 values each
+    __device__ __forceinline__ void produce(int M, int K) const {
+        __shared__ uint32_t wmax[kMaxWaves];
+        const int lane = threadIdx.x & 63, waves = blockDim.x >> 6;
+        const bool has = (int)threadIdx.x < K / 8;
+        for (int row = blockIdx.x; row < M; row += gridDim.x) {
+            const uint4 mine = has ? ((const uint4*)(x + (size_t)row * K))[threadIdx.x] : make_uint4(0, 0, 0, 0);
+            const uint32_t am = wave_max_u32(absmax_bits8(mine, 0));
+            if (lane == 0) wmax[threadIdx.x >> 6] = am;
+            lds_barrier();
+            const float s32 = quant_scale<0>(wave_max_u32(lane < waves ? wmax[lane] : 0));
+            if (has) put(q + (size_t)row * K, threadIdx.x, quant_vec8<0>(mine, s32));
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the stores are acknowledged
+            lds_barrier();
+            if (threadIdx.x == 0) {
+                const uint32_t bits = f32_to_bf16_rne(s32);
+                s[row] = (uint16_t)bits;
+                __hip_atomic_store(&hand_flags[set][row], (unsigned long long)tag << 32 | bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        }
+    }
+    // by one wave: waits for all rows; returns the scale (bf16 bits) of row lane % 16
+    __device__ __forceinline__ uint32_t wait(int M, int K) const {
+        const int lane = threadIdx.x & 63, row = lane & 15;
+        unsigned long long f = 0;
+        bool here = false;
+        for (int i = 0; i < polls; ++i) {
+            f = __hip_atomic_load(&hand_flags[set][row], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            here = row >= M || (unsigned)(f >> 32) == tag;
+            if (__builtin_amdgcn_ballot_w64(!here) == 0) break;
+        }
+        uint32_t bits = (uint32_t)f;
+        // the way out of a wait that does not end: a row by this wave, through memory twice
+        for (unsigned missing = (unsigned)__builtin_amdgcn_ballot_w64(row < M && !here) & 0xffffu; missing; missing &= missing - 1) {
+            const int r = __builtin_ctz(missing);
+            const uint4* from = (const uint4*)(x + (size_t)r * K);
+            uint32_t am = 0;
+            for (int vec = lane; vec < K / 8; vec += 64) am = absmax_bits8(from[vec], am);
+            const float s32 = quant_scale<0>(wave_max_u32(am));
+            for (int vec = lane; vec < K / 8; vec += 64) put(q + (size_t)r * K, vec, quant_vec8<0>(from[vec], s32));
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            if (row == r) bits = f32_to_bf16_rne(s32);
+        }
+        asm volatile("" ::: "memory");
+        return bits;
+    }
+    // by the workgroup: all rows are there; returns the scale, bf16 bits, of token threadIdx.x % 16
+    __device__ __forceinline__ uint16_t meet(int M, int K) const {
+        __shared__ uint32_t scales[16];
+        if (threadIdx.x < 64) {
+            const uint32_t bits = wait(M, K);
+            if (threadIdx.x < 16) scales[threadIdx.x] = bits;
+        }
+        lds_barrier();
+        return (uint16_t)scales[threadIdx.x & 15];
+    }
+};
+
+// ---------------------------------------------------------------------------
 // The drop-in product (int8 rows in, up to 16 tokens) in the same decomposition: no staging at all
 // ---------------------------------------------------------------------------
 // A workgroup owns RB x RPW 16-row blocks, S waves split K, every wave multiplies exactly UPW k-steps
@@ -1960,11 +2050,11 @@ __global__ __launch_bounds__(kMaxWaves * 64) void bitlinear_solo_kernel(
 // products and no wave waits for another.  The +2 of the stored codes leaves with a second product
 // per k-step whose row operand is all ones (sum_k a[p, k] in every row of the tile), shared by the
 // wave's row blocks.  One barrier, behind the products, as in bitlinear_solo_kernel.
-template <int UPW, int RPW, bool RES>
-__global__ __launch_bounds__(kMaxWaves * 64) void gemv_i2_solo_kernel(
-    const int8_t* __restrict__ act, const uint32_t* __restrict__ wq, int M, int N, int K, int rb_map, int S, int slot_rows,
-    const uint16_t* __restrict__ s, const uint16_t* __restrict__ ws, uint16_t* __restrict__ out,
-    const uint16_t* __restrict__ residual, int32_t* __restrict__ acc_out) {
+template <int UPW, int RPW, bool RES, class Rows>
+__device__ __forceinline__ void solo_product(const int8_t* act, const uint32_t* __restrict__ wq, int M, int N, int K, int rb_map, int S,
+                                             int slot_rows, const uint16_t* __restrict__ s, const uint16_t* __restrict__ ws,
+                                             uint16_t* __restrict__ out, const uint16_t* __restrict__ residual,
+                                             int32_t* __restrict__ acc_out, const Rows& rows) {
     __shared__ __attribute__((aligned(16))) int red[kSoloRedSlots][256];  // partial 16 x 16 tiles, [row block * S + k slice]
     const int RB = rb_map & 0xff;                      // row blocks per workgroup
     const uint32_t slot_map = (uint32_t)rb_map >> 8;   // run j of slot_rows output rows reads ws[(slot_map >> 3 j) & 7]
@@ -1982,11 +2072,15 @@ __global__ __launch_bounds__(kMaxWaves * 64) void gemv_i2_solo_kernel(
     const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc((void*)act, 0, M * K, 0x00020000);
     const int slice_k0 = ks * (UPW * 64);
     v4i b[UPW];
+    auto load_rows = [&] {
 #pragma unroll
-    for (int j = 0; j < UPW; ++j) {
-        const bool live = p < M && slice_k0 + j * 64 < K;  // K % 64 == 0: a k-step is inside K or outside
-        b[j] = __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, live ? p * K + slice_k0 + j * 64 + g * 16 : 0x7ffffff0, 0, 0);
-    }
+        for (int j = 0; j < UPW; ++j) {
+            const bool live = p < M && slice_k0 + j * 64 < K;  // K % 64 == 0: a k-step is inside K or outside
+            b[j] = __builtin_amdgcn_raw_buffer_load_b128(a_rsrc, live ? p * K + slice_k0 + j * 64 + g * 16 : 0x7ffffff0, 0, 0);
+        }
+    };
+    if constexpr (Rows::kGiven) load_rows();
+    else rows.produce(M, K);
     const int lane_word = (g >> 1) * 32 + (p >> 3) * 16 + (g & 1) * 8 + (p & 7);
     const int w_voff = lane_word * 4 + ks * (UPW * 256);
     uint32_t w[RPW][UPW];
@@ -2008,7 +2102,8 @@ __global__ __launch_bounds__(kMaxWaves * 64) void gemv_i2_solo_kernel(
         slot_last += n_last >= j * slot_rows ? 1 : 0;
     }
     const uint16_t wsb_first = ws[(slot_map >> (3 * slot_first)) & 7u];
-    const uint16_t e_sb = s[(tid & 15) < M ? (tid & 15) : M - 1];  // every output slot of a thread belongs to token tid % 16
+    uint16_t e_sb = 0;  // every output slot of a thread belongs to token tid % 16
+    if constexpr (Rows::kGiven) e_sb = s[(tid & 15) < M ? (tid & 15) : M - 1];
     const int nthreads = 64 * RB * S;
     uint16_t e_res[kFusedMaxRB];
     if (RES) {
@@ -2023,6 +2118,10 @@ __global__ __launch_bounds__(kMaxWaves * 64) void gemv_i2_solo_kernel(
         }
     }
     __builtin_amdgcn_sched_barrier(0);  // every request above is on its way before anything below is looked at
+    if constexpr (!Rows::kGiven) {
+        e_sb = rows.meet(M, K);
+        load_rows();
+    }
 
     // sum_k a[p, k] over the slice, in the accumulator layout (every row of the tile holds it)
     const int ones_w = 0x01010101;
@@ -2073,6 +2172,25 @@ __global__ __launch_bounds__(kMaxWaves * 64) void gemv_i2_solo_kernel(
             if (out) out[(size_t)m * N + n] = o;
         }
     }
+}
+
+struct GivenRows {
+    static constexpr bool kGiven = true;
+};
+template <int UPW, int RPW, bool RES>
+__global__ __launch_bounds__(kMaxWaves * 64) void gemv_i2_solo_kernel(
+    const int8_t* __restrict__ act, const uint32_t* __restrict__ wq, int M, int N, int K, int rb_map, int S, int slot_rows,
+    const uint16_t* __restrict__ s, const uint16_t* __restrict__ ws, uint16_t* __restrict__ out,
+    const uint16_t* __restrict__ residual, int32_t* __restrict__ acc_out) {
+    solo_product<UPW, RPW, RES>(act, wq, M, N, K, rb_map, S, slot_rows, s, ws, out, residual, acc_out, GivenRows{});
+}
+
+// BitLinearKernel.forward for up to sixteen tokens in one launch, its rows handed on by the first workgroups (HandedRows)
+template <int UPW, int RPW>
+__global__ __launch_bounds__(kMaxWaves * 64) void bitlinear_handed_kernel(
+    const uint32_t* __restrict__ wq, int M, int N, int K, int rb_map, int S, int slot_rows, const uint16_t* __restrict__ ws,
+    uint16_t* __restrict__ out, const HandedRows rows, int32_t* __restrict__ acc_out) {
+    solo_product<UPW, RPW, false>(rows.q, wq, M, N, K, rb_map, S, slot_rows, nullptr, ws, out, nullptr, acc_out, rows);
 }
 
 // ---------------------------------------------------------------------------
@@ -2241,6 +2359,8 @@ struct Tuning {
     int upw = 0;
     int path = 0;  // 0 = built-in choice, 2 = split-K kernel, 3 = fused shape, 4 = never fuse, 5 = GEMM tile
     int fused[3] = {1, 10, 4};
+    int hand = 0;          // forward with the quantizer in the product's launch: 0 built-in choice, 1 wherever it applies, 2 never
+    int hand_polls = -1;   // its polls before a workgroup quantizes by itself, -1 = built-in
     int prefill_big = 0;
     int prefill_ks = 0;    // groups of waves splitting K in the small prefill tiles, 0 = built-in choice
     int staged = 0;        // product through the LDS-staged kernel: 0 = built-in choice, 1 = whenever it fits, 2 = never
@@ -2365,6 +2485,13 @@ constexpr int kRingMost64x256 = 340;
 constexpr int kRingMinK = 384, kRingMinK64x256 = 1024;
 // ... and with rope or gate in the epilogue from the K on that their entry points state
 constexpr int kRingEpilogueMinK = 640;
+// the forward call's quantizer in the product's launch (HandedRows) while the rows, which every workgroup reads behind the hand-over,
+// are few, and up to this many row blocks.  Issued one by one, two launches -> one: 9 x 3840 x 2560 7.3 -> 5.8 us, 16 x 3840 x 2560 7.3
+// -> 6.6, 5 x 2560 x 6912 7.5 -> 6.2, 8 x 2560 x 6912 7.5 .. 8.9 -> 7.1; 16 x 2560 x 6912 8.5 -> 8.4, 16 x 13824 x 2560 7.6 -> 7.6, 16 x 20480 x
+// 3200 11.2 -> 12.5.  Behind a full queue, where the host's part does not count, 5.6 -> 5.8, 6.1 -> 6.6, 6.85 -> 6.3, 7.5 -> 7.1.  The
+// same in front of the ring kernel's 32 x 64 tiles was built and left out: 101 x 3840 x 2560 7.8 -> 8.3, 64 x 2560 x 6912 10.65 -> 10.4.
+constexpr long long kHandMaxElems = 57344;
+constexpr int kHandMostBlocks = 432;
 }  // namespace dispatch
 using namespace dispatch;
 
@@ -2886,6 +3013,47 @@ int launch_prod_solo(const int8_t* act, const int8_t* packed, uint16_t* out, int
 #undef BITLINEAR_LAUNCH_PS_U
 #undef BITLINEAR_LAUNCH_PS_W
 #undef BITLINEAR_LAUNCH_PS
+    return launch_status();
+}
+
+// Whether a launch on this stream runs (and is not recorded)
+bool stream_runs(hipStream_t stream) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &status) == hipSuccess) return status == hipStreamCaptureStatusNone;
+    (void)hipGetLastError();
+    return false;
+}
+// the next launch's set of flag words and its tag
+HandedRows handed_rows(const uint16_t* x, int8_t* q, uint16_t* s) {
+    static std::atomic<unsigned long long> launches{0};
+    const unsigned long long launch = launches.fetch_add(1, std::memory_order_relaxed);
+    return HandedRows{x, q, s, (int)(launch % kHandSets), t_tune.hand_polls >= 0 ? t_tune.hand_polls : kHandPolls,
+                      (unsigned)(launch / kHandSets) + 1u};
+}
+
+int launch_handed(const uint16_t* x, const int8_t* packed, uint16_t* out, int32_t* acc_out, const uint16_t* ws, const ScaleMap& smap,
+                  int8_t* q_out, uint16_t* s_out, int M, int N, int K, const ProdPlan& pl, hipStream_t stream) {
+    const dim3 grid((N / 16 + pl.rpw - 1) / pl.rpw, 1, 1), block(64 * pl.s, 1, 1);
+    const uint32_t* wq = (const uint32_t*)packed;
+    const SlotRule rule = slot_rule(smap, N);
+    if (!rule.ok || M > 16 || K > 512 * pl.s) return BITLINEAR_ERR_ARG;
+    const int slot_rows = rule.slot_rows, rb_map = 1 | (int)(rule.map << 8);
+    const HandedRows rows = handed_rows(x, q_out, s_out);
+    g_last_kernel = "bitlinear_handed_kernel";
+#define BITLINEAR_LAUNCH_HAND(U, W)                                                                                          \
+    BL_LAUNCH((bitlinear_handed_kernel<U, W>), grid, block, 0, stream, wq, M, N, K, rb_map, pl.s, slot_rows, ws, out, rows, acc_out)
+#define BITLINEAR_LAUNCH_HAND_U(U)                     \
+    if (pl.rpw == 1) BITLINEAR_LAUNCH_HAND(U, 1);      \
+    else if (pl.rpw == 2) BITLINEAR_LAUNCH_HAND(U, 2); \
+    else BITLINEAR_LAUNCH_HAND(U, 4)
+    switch (pl.upw) {
+        case 4: BITLINEAR_LAUNCH_HAND_U(4); break;
+        case 5: BITLINEAR_LAUNCH_HAND_U(5); break;
+        case 7: BITLINEAR_LAUNCH_HAND_U(7); break;
+        default: BITLINEAR_LAUNCH_HAND_U(8); break;
+    }
+#undef BITLINEAR_LAUNCH_HAND_U
+#undef BITLINEAR_LAUNCH_HAND
     return launch_status();
 }
 
@@ -3518,7 +3686,8 @@ int bitlinear_set_tuning(int kernel, int a, int b, int c) {
     std::lock_guard<std::mutex> lock(g_tuning_mutex);
     Tuning& g = g_tuning_shared;
     if (kernel == 0) {
-        g.path = g.waves = g.upw = g.staged = g.stream = g.stream_depth = g.stream_waves = g.solo = g.solo_coop = g.solo_rpw = g.prod_solo = g.tok = 0;
+        g.path = g.waves = g.upw = g.staged = g.stream = g.stream_depth = g.stream_waves = g.solo = g.solo_coop = g.solo_rpw = g.prod_solo = g.tok = g.hand = 0;
+        g.hand_polls = -1;
         return set_status(BITLINEAR_OK);
     }
     if (kernel == 6) {
@@ -3538,6 +3707,12 @@ int bitlinear_set_tuning(int kernel, int a, int b, int c) {
         if (a < 0 || a > 2 || b < 0 || b > 4) return set_status(BITLINEAR_ERR_ARG);
         g.solo_coop = a;
         g.solo_rpw = b;
+        return set_status(BITLINEAR_OK);
+    }
+    if (kernel == 13) {
+        if (a < 0 || a > 2 || b < 0 || b > kHandPolls) return set_status(BITLINEAR_ERR_ARG);
+        g.hand = a;
+        g.hand_polls = b - 1;
         return set_status(BITLINEAR_OK);
     }
     if (kernel == 11) {
@@ -3811,8 +3986,14 @@ static int forward_impl(const uint16_t* x, const int8_t* packed, uint16_t* outpu
         return set_status(launch_fused(x, packed, output0, ws, sm, q_ws, s_ws,
                                        FusedExtras{nullptr, nullptr, 0.0f, 0, nullptr, acc_out}, M, N, K, mode, pl,
                                        (hipStream_t)stream));
-    // larger blocks: the quantizer once, in a kernel of its own, then the product
+    // larger blocks: the quantizer once, in the product's launch or in a kernel of its own, then the product
     if (!q_ws || !s_ws) return set_status(BITLINEAR_ERR_NULL);
+    if (mode == 0 && t_tune.path == 0 && t_tune.hand != 2 && !t_plan.active && M <= kHandRows && (long long)M * K <= kHandMaxElems &&
+        (t_tune.hand == 1 || N / 16 < kHandMostBlocks) && slot_rule(sm, N).ok) {
+        const ProdPlan hp = plan_prod_solo(M, N, K);
+        if (hp.ok && K <= 512 * hp.s && stream_runs((hipStream_t)stream))
+            return set_status(launch_handed(x, packed, output0, acc_out, ws, sm, q_ws, s_ws, M, N, K, hp, (hipStream_t)stream));
+    }
     const int st = bitlinear_quant_absmax(x, q_ws, s_ws, M, K, mode, stream);
     if (st != BITLINEAR_OK) return st;
     return set_status(launch_gemv(q_ws, packed, output0, acc_out, s_ws, ws, sm, M, N, K, (hipStream_t)stream));

@@ -331,7 +331,9 @@ int bitlinear_norm_rope_forward_bf16(const uint16_t* x, const uint16_t* norm_wei
  * of the call in launch order and joined by " + ", the kernel with its template
  * arguments, the grid, the workgroup size and the dynamic LDS bytes, e.g.
  * "bitlinear_solo_kernel<5, 1, 1, true, 0, false, 1> grid=(160,1,1) block=512
- * lds=0".  Returns the status the call itself would return for the shape.
+ * lds=0".  Entry 1 stands for a call that is recorded in a graph: of one that
+ * is not, the quantizer may be part of the product's launch (kernel 13 below).
+ * Returns the status the call itself would return for the shape.
  * The current bitlinear_set_tuning overrides apply.  No counterpart in the
  * reference, whose dispatch is a table of ten shapes (bitnet_kernels.cu:4-33).
  */
@@ -404,6 +406,13 @@ int bitlinear_plan_name(int entry, int M, int N, int K, char* buf, int buflen);
  *             row blocks per wave; the kernel 8 setting a = 5
  *             keeps the one-to-four-token kernel out of the way), 2 never.
  *             Applies with kernel 0 only; kernel 0 resets it.
+ *   kernel 13: bitlinear_forward_bf16 (mode 0, M <= 16, with workspaces, on a
+ *             stream that is not being captured) in one launch whose first
+ *             workgroups quantize the rows and hand them on: a = 0 built-in
+ *             choice (where the quantizer would be a launch of its own, M * K <=
+ *             57344, N < 6912), 1 for any N, 2 never; b = 0 the built-in bound of
+ *             a workgroup's polls before it quantizes the rows itself, else b - 1
+ *             polls (b <= 512).  Applies with kernel 0 only; kernel 0 resets it.
  */
 int bitlinear_set_tuning(int kernel, int a, int b, int c);
 

@@ -1372,6 +1372,74 @@ def test_solo_kernel_with_several_row_blocks_per_wave(n, k, s_, upw, rpw, coop, 
     _assert_bits_equal(host_bits(out), want, f"rpw={rpw}")
 
 
+@pytest.mark.parametrize("polls", [0, 1, 2])  # the built-in bound; none, every workgroup quantizes all rows; one
+@pytest.mark.parametrize("m,n,k", [(9, 16, 2560), (16, 48, 3520), (11, 2560, 2560), (16, 3840, 2560), (8, 2560, 6912), (5, 1040, 8192),
+                                   (7, 6896, 7168), (12, 13824, 2560), (16, 816, 2112)])
+def test_forward_with_rows_handed_on_inside_the_launch(m, n, k, polls):
+    """Fewer workgroups than rows, waves with and without values of a row, one to four row blocks a wave, an infinity, a NaN and a
+    row of zeros: rows, scales, accumulators and outputs are those of the two launches, for other rows in the same buffers too."""
+    lib = _lib.load_library()
+    rng = np.random.default_rng(m + n + k)
+    pk = _packed_dev(rng.integers(-1, 2, size=(n, k), dtype=np.int8))
+    wsd = dev_bf16(o.f32_to_bf16_bits(np.array([0.0161, 0.0247, 0.0093, 0.0], dtype=np.float32)))
+    x = torch.empty(m, k, dtype=torch.bfloat16, device="cuda")
+    q = [torch.zeros(m, k, dtype=torch.int8, device="cuda") for _ in range(2)]
+    s = [torch.zeros(m, dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+    acc = [torch.zeros(m, n, dtype=torch.int32, device="cuda") for _ in range(2)]
+    out = [torch.zeros(m, n, dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+    st = torch.cuda.current_stream().cuda_stream
+    try:
+        for turn in range(3):
+            x.copy_(torch.randn(m, k, device="cuda") * 10.0**turn)
+            x[turn, 5], x[turn + 1, k - 1], x[turn + 2] = float("inf"), float("nan"), 0.0
+            for i, args in enumerate(((2, 0), (1, polls))):
+                assert lib.bitlinear_set_tuning(13, *args, 0) == 0
+                assert lib.bitlinear_forward_bf16_acc_i32(x.data_ptr(), pk.data_ptr(), acc[i].data_ptr(), out[i].data_ptr(), wsd.data_ptr(),
+                                                          q[i].data_ptr(), s[i].data_ptr(), m, n, k, 0, st) == 0
+                assert (bitlinear.last_kernel() == "bitlinear_handed_kernel") == (i == 1)
+            torch.cuda.synchronize()
+            for a, b in (q, s, acc, out):
+                assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+    finally:
+        lib.bitlinear_set_tuning(0, 0, 0, 0)
+
+
+def test_forward_with_handed_rows_on_two_streams_and_in_a_graph():
+    """Launches of two streams overlap, more of them than there are sets of flag words; a captured call is replayed with
+    other rows."""
+    m, n, k, calls = 9, 2560, 2560, 300
+    mod = bitlinear.BitLinearKernel(k, n).cuda()
+    mod.weight.data = _packed_dev(np.random.default_rng(1).integers(-1, 2, size=(n, k), dtype=np.int8))
+    mod.weight_scale.data = torch.full((4,), 0.0161, device="cuda").to(torch.bfloat16)
+    xs = [torch.randn(m, k, device="cuda").to(torch.bfloat16) * (i + 1) for i in range(5)]
+    lib = _lib.load_library()
+    try:
+        assert lib.bitlinear_set_tuning(13, 2, 0, 0) == 0
+        want = [mod(x) for x in xs]
+    finally:
+        lib.bitlinear_set_tuning(0, 0, 0, 0)
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    outs = []
+    for i in range(calls):
+        for st in streams:
+            with torch.cuda.stream(st):
+                outs.append((i % 5, mod(xs[i % 5])))
+    assert bitlinear.last_kernel() == "bitlinear_handed_kernel"
+    torch.cuda.synchronize()
+    assert all(torch.equal(out, want[i]) for i, out in outs)
+    x = xs[0].clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = mod(x)
+    assert bitlinear.last_kernel() != "bitlinear_handed_kernel"
+    for i in (1, 2, 3, 1):
+        x.copy_(xs[i])
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want[i])
+
+
 @pytest.mark.parametrize("res", [0, 1])
 @pytest.mark.parametrize("m", [1, 3, 4, 8, 13, 16])
 @pytest.mark.parametrize("n,k,s_,upw,rpw", [(2560, 2560, 8, 5, 1), (3840, 2560, 5, 8, 1), (13824, 2560, 8, 5, 2),
