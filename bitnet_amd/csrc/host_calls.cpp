@@ -20,6 +20,8 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <atomic>
+#include <chrono>
 #include <cstdint>
 #include <mutex>
 #include <vector>
@@ -388,6 +390,38 @@ PyObject* unpack(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     END_HANDLE_TH_ERRORS
 }
 
+// await_words(tensor, unset, microseconds): a contiguous int64 tensor in host memory that a kernel writes; whether all of its words
+// have become another value than `unset` within that time.  Looks at the words themselves: waiting for the stream takes some 15 us more
+// (a marker behind the kernel, and its signal).
+PyObject* await_words(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+    HANDLE_TH_ERRORS
+    if (!arg_count(nargs, 3, "await_words")) return nullptr;
+    const at::Tensor* t = tensor_of(args[0]);
+    if (!t) return nullptr;
+    const long long unset = PyLong_AsLongLong(args[1]), limit = PyLong_AsLongLong(args[2]);
+    if (PyErr_Occurred()) return nullptr;
+    if (!t->device().is_cpu() || t->scalar_type() != at::kLong || !t->is_contiguous()) {
+        PyErr_SetString(PyExc_TypeError, "await_words: expected contiguous int64 words in host memory");
+        return nullptr;
+    }
+    const volatile int64_t* word = (const volatile int64_t*)t->data_ptr();
+    const int64_t count = t->numel();
+    bool all = true;
+    {
+        const Unlocked unlocked;
+        const auto end = std::chrono::steady_clock::now() + std::chrono::microseconds(limit);
+        for (int64_t i = 0; all && i < count; ++i)
+            for (int n = 1; word[i] == unset; ++n)
+                if (n % 256 == 0 && std::chrono::steady_clock::now() > end) {
+                    all = false;
+                    break;
+                }
+        std::atomic_thread_fence(std::memory_order_acquire);
+    }
+    return PyBool_FromLong(all);
+    END_HANDLE_TH_ERRORS
+}
+
 // bind(error_class, product, last_status, status_string, ws_num, quant, forward, forward_seg, pack, unpack): the
 // library's functions by address
 PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
@@ -421,6 +455,7 @@ PyMethodDef methods[] = {
     {"quant", (PyCFunction)(void*)quant, METH_FASTCALL, nullptr},
     {"pack", (PyCFunction)(void*)pack, METH_FASTCALL, nullptr},
     {"unpack", (PyCFunction)(void*)unpack, METH_FASTCALL, nullptr},
+    {"await_words", (PyCFunction)(void*)await_words, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host_calls", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

@@ -745,6 +745,7 @@ class Generator:
         # with the library's LM head, host memory that its last kernel writes: the test for an end token is then a
         # look at it, where two kernels, a copy and their launches left the GPU idle for some 50 us a step
         self.next_tok = torch.zeros(batch, dtype=torch.int64, device="cpu" if self.lm_head else dev, pin_memory=self.lm_head)
+        self._await = self.lm_head  # whether the host may wait for the tokens themselves
         self._logits: Optional[torch.Tensor] = None
         self._sampler: Optional[TopPSampler] = None
         # generated tokens of a decode() call, written from inside the step so that a graph replay is the whole step
@@ -805,9 +806,23 @@ class Generator:
             cv.copy_(sv)
         return graph
 
-    def _ended(self, eos_id: int) -> bool:
-        """Whether the step just issued produced eos_id for any sequence (waits for it)."""
-        torch.cuda.current_stream().synchronize()
+    kUnset = -(1 << 63)  # no token
+    kAwaitUs = 20000  # longer than a step takes; behind it the stream is waited for
+
+    def _expect(self) -> bool:
+        """Marks the host's tokens as not written, in front of a step whose tokens the host looks at.  Every earlier step must
+        have been waited for: one that is still under way would write them again."""
+        if self._await:
+            self.next_tok.fill_(self.kUnset)
+        return self._await
+
+    def _ended(self, eos_id: int, expected: bool) -> bool:
+        """Whether the step just issued produced eos_id for any sequence (waits for it).  expected: _expect() was called in
+        front of it, so that its tokens themselves can be waited for; the stream otherwise."""
+        if not expected or not _lib.host_calls().await_words(self.next_tok, self.kUnset, self.kAwaitUs):
+            torch.cuda.current_stream().synchronize()
+            if expected:
+                self._await = False  # (steps that take longer, or writes to host memory that only a wait makes visible)
         return bool((self.next_tok == eos_id).any())
 
     def _check(self) -> None:
@@ -918,12 +933,13 @@ class Generator:
         self.step_idx.zero_()
         taken = 0
         for i in range(steps):
+            expected = eos_id is not None and i > 0 and self._expect()  # (behind the first step nothing older is under way)
             if self.use_graph:
                 self.graph.replay()
             else:
                 self._step()
             taken = i + 1
-            if eos_id is not None and self._ended(eos_id):
+            if eos_id is not None and self._ended(eos_id, expected):
                 break
         out = self.history[:taken].clone()
         self._check()
@@ -1016,6 +1032,7 @@ class Generator:
                     self._logits_graph = self._capture(self._logits_step)
                 taken = 0
                 for _ in range(gen_length - 1):
+                    expected = eos_id is not None and taken > 0 and self._expect()
                     if self.lm_head:
                         if self.use_graph:
                             self._logits_graph.replay()
@@ -1035,7 +1052,7 @@ class Generator:
                         self.tok.copy_(self.next_tok.view(-1, 1))
                         self.pos.add_(1)
                     taken += 1
-                    if eos_id is not None and self._ended(eos_id):
+                    if eos_id is not None and self._ended(eos_id, expected):
                         break
                 out.append(self.history[:taken])
                 self._check()

@@ -1255,6 +1255,34 @@ def test_generate_all_stops_at_the_end_token_and_trims_the_answers():
     assert cut0[1] == want1 and len(cut0[1]) > 1
 
 
+@pytest.mark.parametrize("use_graph", [True, False])
+@pytest.mark.parametrize("sample", [False, True])
+def test_steps_awaited_by_their_tokens_end_where_steps_awaited_by_the_stream_do(sample, use_graph):
+    """With an end token the host waits for a step's tokens in host memory: directly behind steps that nobody waited for,
+    with waits that run out at once (from then on the stream is waited for), and for end tokens of the first, a middle and no step."""
+    model = _build(BIG_HEADS, seed=16)
+    gen = decoder.Generator(model, batch=2, max_seq=64, use_graph=use_graph)
+    prompts = [[5, 9, 2, 44, 7], [3, 1, 8]]
+    first, lens = torch.tensor([4, 9], device="cuda"), torch.tensor([5, 3], device="cuda")
+
+    def answers(**kw):
+        gen.decode(first, lens, 20)  # still under way when the next call starts
+        return gen.generate_all(prompts, 20, use_sampling=sample, rng=torch.Generator(device="cuda").manual_seed(3), **kw)
+
+    full = answers()
+    for eos in (full[0][1], full[1][9], 10**6):
+        gen._await = True
+        got = answers(eos_id=eos)
+        assert gen._await
+        gen.kAwaitUs = 0  # a wait that is not over at once gives up
+        assert answers(eos_id=eos) == got
+        del gen.kAwaitUs
+        gen._await = False
+        assert answers(eos_id=eos) == got
+        steps = next((t for t in range(1, 20) if any(f[t] == eos for f in full)), 19)
+        assert max(len(a) for a in got) <= steps + 1
+
+
 def test_generate_all_sampling_is_reproducible_and_greedy_for_a_tiny_nucleus():
     model = _build(BIG_HEADS, seed=7)
     g = torch.Generator().manual_seed(5)
