@@ -1000,7 +1000,7 @@ struct Stack {
         const __amdgpu_buffer_rsrc_t k_rsrc = make_rsrc(ck, cache_bytes), v_rsrc = make_rsrc(cv, cache_bytes);
         const int blk_stride = nsplit * at.attn_waves;  // this wave takes the blocks of waves wave, wave + kStWaves, ...
         v4u kb[2][4], vb[8];
-        auto load_rows = [&](int blk) {
+        auto request_rows = [&](int blk) {
             const int base = blk * 32 * row_bytes;
 #pragma unroll
             for (int bi = 0; bi < 2; ++bi) {
@@ -1011,21 +1011,18 @@ struct Stack {
 #pragma unroll
             for (int jj = 0; jj < 8; ++jj)
                 vb[jj] = __builtin_amdgcn_raw_buffer_load_b128(v_rsrc, base + ((jj & 3) + (jj >> 2) * 16 + 4 * g4) * row_bytes + c * 16, 0, 0);
+        };
+        auto turn_rows = [&](int blk) {
             if (blk == pblk) df_clear(vb, p, lane);
             df_turn(vb);
         };
-        load_rows(sp + nsplit * wave);
+        request_rows(sp + nsplit * wave);
         // the factors of pairs 4 c ..
         const __amdgpu_buffer_rsrc_t factors = make_rsrc(a->rope_rows + (size_t)b * kHeadDim, kHeadDim * 4);
         v4u cs = __builtin_amdgcn_raw_buffer_load_b128(factors, c * 16, 0, 0);
         v4u sn = __builtin_amdgcn_raw_buffer_load_b128(factors, kHeadDim * 2 + c * 16, 0, 0);
         const int turn = uniform(pblk / nsplit);
         has_new = uniform(pblk - turn * nsplit == sp && (turn % at.attn_waves) % kStWaves == wave);
-        DfState st;
-        // (kept in front of the polls)
-#pragma unroll
-        for (int t = 0; t < 8; ++t) asm volatile("" : "+v"(st.o_acc[t]), "+v"(vb[t]), "+v"(kb[t >> 2][t & 3]));
-        asm volatile("" : "+v"(cs), "+v"(sn));
 
         // heads 4 u + g4 of the group, dims 8 c .. (lanes beyond the last head repeat it); where it is wanted k by lanes
         // 0 .. 15 and v by the others
@@ -1036,13 +1033,29 @@ struct Stack {
 #pragma unroll
         for (int u = 0; u < kRounds; ++u) head[u] = 4 * u + g4 < G ? 4 * u + g4 : G - 1;
         const int new_head = lane < 16 ? at.n_heads + kvh : at.n_heads + n_kv + kvh;
-        for (int spin = 0;; ++spin) {
+        auto request_token = [&]() {
             poll_again();
-            unsigned m = 0;
 #pragma unroll
             for (int u = 0; u < kRounds; ++u)
                 if (4 * u < G) raw[u] = __builtin_amdgcn_raw_buffer_load_b128(row, ((kvh * G + head[u]) * kHeadDim + 8 * c) * 2, 0, kSc1);
             if (has_new) fresh = __builtin_amdgcn_raw_buffer_load_b128(row, (new_head * kHeadDim + 8 * c) * 2, 0, kSc1);
+        };
+        // Where wqkv's and the attention's tasks together are more than the workgroups (288 of 256 at four sequences, 368 at
+        // eight), some come here from a wqkv task: the token's row is there by the time that the cache rows are, 1.5 us later,
+        // and a poll behind those is another 0.4.  So the row is requested along with them and looked at once they are turned: four
+        // sequences 784 -> 775 us a step at 512 positions, five 798 -> 783, eight 853 -> 845.  (With the cache rows brought into
+        // the L2 by the wave that fetches it is there 0.5 us earlier, and wo's phase takes 0.8 longer.)  Up to two sequences
+        // everybody waits for the row, and an early look costs 0.5 %.
+        if constexpr (!kDirect) request_token();
+        turn_rows(sp + nsplit * wave);
+        DfState st;
+        // (kept in front of the polls)
+#pragma unroll
+        for (int t = 0; t < 8; ++t) asm volatile("" : "+v"(st.o_acc[t]), "+v"(vb[t]), "+v"(kb[t >> 2][t & 3]));
+        asm volatile("" : "+v"(cs), "+v"(sn));
+        for (int spin = 0;; ++spin) {
+            if (kDirect || spin > 0) request_token();
+            unsigned m = 0;
             auto look = [&](const v4u& v) { m = unset_max(unset_max(unset_max(unset_max(m, v.x), v.y), v.z), v.w); };
 #pragma unroll
             for (int u = 0; u < kRounds; ++u)
@@ -1079,7 +1092,8 @@ struct Stack {
 #pragma unroll
         for (int kk = 0; kk < 4; ++kk) qa[kk] = __builtin_bit_cast(v8bf, *(const v4u*)&rows[c & (G - 1)][kk * 32 + g4 * 8]);
         auto later_block = [&]() {
-            load_rows(blk);
+            request_rows(blk);
+            turn_rows(blk);
             if (blk == pblk) new_row();
             df_block(kb, vb, vn, qa, blk, p, lane, st);
         };
