@@ -118,6 +118,7 @@ SIGNATURES = {
     "bitnet_decode_stack_reset": (_c_int, [_c_ptr] + [_c_int] * 8 + [_c_ptr]),
     "bitnet_decode_stack_error_offset": (_c_int, []),
     "bitnet_decode_stack": (_c_int, [_c_ptr] * 6 + [_c_int] * 10 + [_c_ptr]),
+    "bitnet_decode_stack_step": (_c_int, [_c_ptr] * 8 + [_c_int] * 11 + [_c_ptr]),
     "bitlinear_scale_runs": (
         _c_int,
         [_c_int, _c_int, ctypes.POINTER(_c_int), _c_int, ctypes.POINTER(_c_int), ctypes.POINTER(ctypes.c_uint32)],

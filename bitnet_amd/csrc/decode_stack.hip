@@ -122,10 +122,16 @@ struct StackControl {
 struct StackArgs {
     const __attribute__((address_space(4))) StackEntry* entries;  // [layer][4]: wqkv, wo, w13, w2
     unsigned char* ws;
+    // The first layer's input: sequence m's row of h_in is m, or, with tokens, its token's; the rotation's factors likewise: in
+    // row m or the position's of cos and sin, whose rows are `factors` apart.  Against a kernel that collects them in front of
+    // this one (4.6 us, most of them launch) a step of one sequence takes 578 us instead of 583 at 512 positions, of eight 843
+    // instead of 848: the lookups and a row from memory stay.
     const uint16_t* h_in;
     uint16_t* h_out;
     const __attribute__((address_space(4))) int64_t* positions;
-    const float* rope_rows;
+    const __attribute__((address_space(4))) int64_t* tokens;
+    const float *cos, *sin;
+    int in_rows, factors;
     int n_layers, B, dim, ffn, n_heads, n_kv, group, S, n_splits, attn_waves, spin_limit;  // group: query heads per kv head
     int ends[9];  // cumulative task counts of a layer's phases
     // a set: bytes per layer and offsets in it; behind the bf16 values of all layers (set_values bytes) the quantized rows
@@ -326,7 +332,8 @@ struct Task {
                                 // where src are quantized rows, their records
     int K, n_out;               // attention: kv head, sequence
     float inv_k;                // attention: split
-    int flags;                  // 1: src is published, 2: dst is, 4: res is.  Attention: the position
+    int flags;                  // 1: src is published, 2: dst is, 4: res is, 8: the rows of src or res are input_row()'s.
+                                // Attention: the position
 };
 
 // a lane's values of one token's slice
@@ -372,7 +379,16 @@ struct Stack {
     __device__ __forceinline__ uint16_t* gate(int layer) const { return (uint16_t*)(layer_set(layer) + a->f_g); }
     __device__ __forceinline__ uint16_t* hb(int layer) const { return (uint16_t*)(layer_set(layer) + a->f_hb); }
     // the residual stream in front of the attention block of `layer`
-    __device__ __forceinline__ const uint16_t* h_before(int layer) const { return layer == 0 ? a->h_in : hb(layer - 1); }
+    // (of one sequence its row, of more the first row of what the first layer reads by input_row())
+    __device__ __forceinline__ const uint16_t* h_before(int layer) const {
+        return layer == 0 ? a->h_in + (MT == 1 ? (size_t)input_row(0) * a->dim : 0) : hb(layer - 1);
+    }
+    __device__ __forceinline__ int input_row(int m) const {
+        if (!a->tokens) return m;
+        const int64_t t = a->tokens[m];
+        return t < 0 ? 0 : t >= (int64_t)a->in_rows ? a->in_rows - 1 : (int)t;  // nothing outside the table is read
+    }
+    __device__ __forceinline__ int input_bytes() const { return a->in_rows * a->dim * 2; }
 
     __device__ __forceinline__ Work locate(int layer, int r) const {
         Work w;
@@ -448,18 +464,18 @@ struct Stack {
             flags = p < 0 ? 0 : (p >= (int64_t)a->S ? a->S - 1 : (int)p);
         } else {
             src = (uint64_t)(i == 0 ? h_before(l) : i == 1 ? o(l) : i == 2 ? ha(l) : gate(l));
-            if (i == 0 && l == 0) flags &= ~1;
+            if (i == 0 && l == 0) flags = (flags & ~1) | (MT == 2 ? 8 : 0);
             if (i == 3) K = a->ffn, inv_k = a->inv_ffn;
             if (wk.ph == kP1 || wk.ph == kP3 || wk.ph == kP4 || wk.ph == kP5) {
                 if (!kDirect) src = bytes(i), aux = record(i);
                 dst = (uint64_t)(i == 0 ? qkv(l) : i == 1 ? ha(l) : i == 2 ? gate(l) : last ? a->h_out : hb(l));
                 if (i == 0) n_out = (a->n_heads + 2 * a->n_kv) * kHeadDim;
-                if (i == 1) res = (uint64_t)h_before(l), flags |= l == 0 ? 0 : 4;  // (the caller's values may be any)
+                if (i == 1) res = (uint64_t)h_before(l), flags |= l == 0 ? (MT == 1 ? 0 : 8) : 4;  // (the caller's values may be any)
                 if (i == 2) n_out = a->ffn;
                 if (i == 3) res = (uint64_t)ha(l), flags |= 4;
                 if (i == 3 && last) flags &= ~2;
             } else {
-                src += (uint64_t)wk.idx * K * 2;
+                src += (uint64_t)(i == 0 && l == 0 ? input_row(wk.idx) : wk.idx) * K * 2;
                 dst = bytes(i) + (uint64_t)wk.idx * 64;
                 res = record(i) + (uint64_t)wk.idx * sizeof(RowRecord);
             }
@@ -576,9 +592,21 @@ struct Stack {
         const int K = tk.K, B = TQ == 1 ? 1 : a->B;
         int off[S::kVec];
         slice_offsets<UPW>(K * 2, off);
-        const __amdgpu_buffer_rsrc_t rows = make_rsrc(tk.src, B * K * 2);
-        const __amdgpu_buffer_rsrc_t rs = make_rsrc(RES ? tk.res : tk.src, RES ? B * tk.n_out * 2 : 0);
-        const int res_off = RES && out_token<1>() < B ? (out_token<1>() * tk.n_out + tk.idx * 16 + out_row()) * 2 : kBeyond;
+        const bool by_token = MT > 1 && kDirect && (tk.flags & 8) != 0;
+        const __amdgpu_buffer_rsrc_t rows = make_rsrc(tk.src, by_token && !RES ? input_bytes() : B * K * 2);
+        const __amdgpu_buffer_rsrc_t rs = make_rsrc(RES ? tk.res : tk.src, RES ? (by_token ? input_bytes() : B * tk.n_out * 2) : 0);
+        int row_at[TQ], res_row = out_token<1>();
+#pragma unroll
+        for (int t = 0; t < TQ; ++t) row_at[t] = (t < B ? t : B - 1) * K * 2;  // tokens beyond the batch repeat the last one
+        if (by_token) {
+            if (RES) {
+                res_row = input_row(res_row < B ? res_row : 0);
+            } else {
+#pragma unroll
+                for (int t = 0; t < TQ; ++t) row_at[t] = input_row(t < B ? t : B - 1) * K * 2;
+            }
+        }
+        const int res_off = RES && out_token<1>() < B ? (res_row * tk.n_out + tk.idx * 16 + out_row()) * 2 : kBeyond;
         const bool published = (tk.flags & 1) != 0;
         for (int spin = 0;; ++spin) {
             poll_again();
@@ -587,7 +615,7 @@ struct Stack {
 #pragma unroll
             for (int t = 0; t < TQ; ++t) {
                 Values<kStUpwF>& v = got.f[t];
-                const int at = (t < B ? t : B - 1) * K * 2;  // tokens beyond the batch repeat the last one
+                const int at = row_at[t];
 #pragma unroll
                 for (int i = 0; i < S::kFull; ++i) v.full[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rows, off[i], at, kSc1));
                 if (S::T == 2) v.rest[0] = (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rows, off[S::kFull], at, kSc1);
@@ -873,8 +901,9 @@ struct Stack {
         const unsigned step = B * 64;
         const unsigned base = pt < B ? (first + ps * 64) * B + pt * 64 + g * 16 : kBeyond;  // (no such token: zeros, no access)
         const __amdgpu_buffer_rsrc_t rows = make_rsrc(tk.src, B * K), recs = make_rsrc(tk.aux, B * (int)sizeof(RowRecord));
-        const __amdgpu_buffer_rsrc_t rs = make_rsrc(RES ? tk.res : tk.src, RES ? B * tk.n_out * 2 : 0);
-        const int res_off = RES ? (m * tk.n_out + tk.idx * 16 + out_row()) * 2 : kBeyond;
+        const bool by_token = RES && (tk.flags & 8) != 0;
+        const __amdgpu_buffer_rsrc_t rs = make_rsrc(RES ? tk.res : tk.src, RES ? (by_token ? input_bytes() : B * tk.n_out * 2) : 0);
+        const int res_off = RES ? ((by_token ? input_row(m) : m) * tk.n_out + tk.idx * 16 + out_row()) * 2 : kBeyond;
         v4i b[kLoads], sums;
         unsigned scale = 0;
         auto recorded = [&] { return (int)(sums.x | sums.y | sums.z | sums.w | (int)scale) >= 0; };
@@ -1018,9 +1047,9 @@ struct Stack {
         };
         request_rows(sp + nsplit * wave);
         // the factors of pairs 4 c ..
-        const __amdgpu_buffer_rsrc_t factors = make_rsrc(a->rope_rows + (size_t)b * kHeadDim, kHeadDim * 4);
-        v4u cs = __builtin_amdgcn_raw_buffer_load_b128(factors, c * 16, 0, 0);
-        v4u sn = __builtin_amdgcn_raw_buffer_load_b128(factors, kHeadDim * 2 + c * 16, 0, 0);
+        const size_t factors = (size_t)(a->tokens ? p : b) * a->factors;
+        v4u cs = __builtin_amdgcn_raw_buffer_load_b128(make_rsrc(a->cos + factors, kHeadDim * 2), c * 16, 0, 0);
+        v4u sn = __builtin_amdgcn_raw_buffer_load_b128(make_rsrc(a->sin + factors, kHeadDim * 2), c * 16, 0, 0);
         const int turn = uniform(pblk / nsplit);
         has_new = uniform(pblk - turn * nsplit == sp && (turn % at.attn_waves) % kStWaves == wave);
 
@@ -1393,6 +1422,42 @@ bool stack_plan(StackArgs& a, long long* bytes) {
 // in decoder_ops.hip: threads the attention kernel of this shape runs with; 0: a shape it does not take
 int bitnet_attn_decode_threads(int B, int S, int n_heads, int n_kv_heads, int n_splits);
 
+static int stack_launch(StackArgs a, const void* entries, void* workspace, uint16_t* h_out, const int64_t* positions, int n_layers, int B, int S, int dim, int ffn,
+                        int n_heads, int n_kv_heads, int n_splits, int workgroups, int spin_limit, void* stream) {
+    a.n_layers = n_layers, a.B = B, a.S = S, a.dim = dim, a.ffn = ffn, a.n_heads = n_heads, a.n_kv = n_kv_heads, a.n_splits = n_splits;
+    long long bytes = 0;
+    if (!stack_plan(a, &bytes)) return 1;
+    const int threads = bitnet_attn_decode_threads(B, S, n_heads, n_kv_heads, n_splits);
+    if (!threads) return 1;
+    if (!entries || !workspace || !a.h_in || !h_out || !positions || !a.cos || !a.sin) return 2;
+    if (((uintptr_t)entries & 63u) || ((uintptr_t)workspace & 255u) || ((uintptr_t)a.h_in & 15u) || ((uintptr_t)h_out & 15u)) return 1;
+    a.entries = (const __attribute__((address_space(4))) StackEntry*)entries;
+    a.ws = (unsigned char*)workspace;
+    a.h_out = h_out;
+    a.positions = (const __attribute__((address_space(4))) int64_t*)positions;
+    a.attn_waves = threads / 64;
+    a.spin_limit = spin_limit > 0 ? spin_limit : kStSpinLimit;
+    int grid = workgroups;
+    if (grid <= 0) {  // one per CU
+        static int cus[bitnet_host::kMaxDevices];
+        int dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= bitnet_host::kMaxDevices) return 3;
+        if (!cus[dev]) {
+            int n = 0;
+            if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) return 3;
+            cus[dev] = n;
+        }
+        grid = cus[dev];
+    }
+#define BITNET_STACK(MT) hipLaunchKernelGGL(decode_stack_kernel<MT>, dim3(grid), dim3(kStThreads), 0, (hipStream_t)stream, a)
+    if (B == 1) BITNET_STACK(1);
+    else if (B == 2) BITNET_STACK(2);
+    else if (B <= 4) BITNET_STACK(4);
+    else BITNET_STACK(8);
+#undef BITNET_STACK
+    return hipGetLastError() == hipSuccess ? 0 : 3;
+}
+
 extern "C" {
 
 long long bitnet_decode_stack_workspace_bytes(int n_layers, int B, int S, int dim, int ffn, int n_heads, int n_kv_heads,
@@ -1423,40 +1488,24 @@ int bitnet_decode_stack(const void* entries, void* workspace, const uint16_t* h_
                         const float* rope_rows, int n_layers, int B, int S, int dim, int ffn, int n_heads, int n_kv_heads,
                         int n_splits, int workgroups, int spin_limit, void* stream) {
     StackArgs a = {};
-    a.n_layers = n_layers, a.B = B, a.S = S, a.dim = dim, a.ffn = ffn, a.n_heads = n_heads, a.n_kv = n_kv_heads, a.n_splits = n_splits;
-    long long bytes = 0;
-    if (!stack_plan(a, &bytes)) return 1;
-    const int threads = bitnet_attn_decode_threads(B, S, n_heads, n_kv_heads, n_splits);
-    if (!threads) return 1;
-    if (!entries || !workspace || !h_in || !h_out || !positions || !rope_rows) return 2;
-    if (((uintptr_t)entries & 63u) || ((uintptr_t)workspace & 255u) || ((uintptr_t)h_in & 15u) || ((uintptr_t)h_out & 15u)) return 1;
-    a.entries = (const __attribute__((address_space(4))) StackEntry*)entries;
-    a.ws = (unsigned char*)workspace;
-    a.h_in = h_in;
-    a.h_out = h_out;
-    a.positions = (const __attribute__((address_space(4))) int64_t*)positions;
-    a.rope_rows = rope_rows;
-    a.attn_waves = threads / 64;
-    a.spin_limit = spin_limit > 0 ? spin_limit : kStSpinLimit;
-    int grid = workgroups;
-    if (grid <= 0) {  // one per CU
-        static int cus[bitnet_host::kMaxDevices];
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= bitnet_host::kMaxDevices) return 3;
-        if (!cus[dev]) {
-            int n = 0;
-            if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) return 3;
-            cus[dev] = n;
-        }
-        grid = cus[dev];
-    }
-#define BITNET_STACK(MT) hipLaunchKernelGGL(decode_stack_kernel<MT>, dim3(grid), dim3(kStThreads), 0, (hipStream_t)stream, a)
-    if (B == 1) BITNET_STACK(1);
-    else if (B == 2) BITNET_STACK(2);
-    else if (B <= 4) BITNET_STACK(4);
-    else BITNET_STACK(8);
-#undef BITNET_STACK
-    return hipGetLastError() == hipSuccess ? 0 : 3;
+    a.h_in = h_in, a.in_rows = B;
+    a.cos = rope_rows, a.sin = rope_rows ? rope_rows + kHeadDim / 2 : nullptr, a.factors = kHeadDim;
+    return stack_launch(a, entries, workspace, h_out, positions, n_layers, B, S, dim, ffn, n_heads, n_kv_heads, n_splits, workgroups,
+                        spin_limit, stream);
+}
+
+int bitnet_decode_stack_step(const void* entries, void* workspace, const int64_t* tokens, const uint16_t* emb, const float* cos_table,
+                             const float* sin_table, uint16_t* h_out, const int64_t* positions, int V, int n_layers, int B, int S,
+                             int dim, int ffn, int n_heads, int n_kv_heads, int n_splits, int workgroups, int spin_limit,
+                             void* stream) {
+    if (V < 1 || dim < 1 || (long long)V * dim * 2 > kBeyond) return 1;  // 32-bit byte offsets into the embedding
+    if (!tokens) return 2;
+    StackArgs a = {};
+    a.h_in = emb, a.in_rows = V;
+    a.tokens = (const __attribute__((address_space(4))) int64_t*)tokens;
+    a.cos = cos_table, a.sin = sin_table, a.factors = kHeadDim / 2;
+    return stack_launch(a, entries, workspace, h_out, positions, n_layers, B, S, dim, ffn, n_heads, n_kv_heads, n_splits, workgroups,
+                        spin_limit, stream);
 }
 
 int bitlinear_probe_stack_math(int what, float by, uint32_t first, uint32_t n, uint32_t* found, void* stream) {

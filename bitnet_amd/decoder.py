@@ -478,6 +478,30 @@ class DecodeStack:
             raise _lib.BitLinearLibraryError(f"bitnet_decode_stack: status {st}")
         return out
 
+    def step(self, tokens, positions, emb_weight, cos, sin, workgroups: int = 0):
+        """decode_step_begin and the call above in one launch, the first layer reading the tokens' rows of the embedding
+        itself; as two where the tables are not what that reads (rows of cos and sin for each of the cache's, an embedding
+        of less than 2 GiB)."""
+        B, S, dim = self.shape[1:4]
+        dev = self.workspace.device
+
+        def table_ok(t, dtype, shape):
+            return t.dtype == dtype and t.device == dev and t.is_contiguous() and t.shape == shape and t.data_ptr() % 16 == 0
+
+        if not (emb_weight.dim() == 2 and table_ok(emb_weight, torch.bfloat16, (emb_weight.shape[0], dim))
+                and 0 < emb_weight.numel() * 2 < 2**31 - 16 and all(table_ok(t, torch.float32, (S, 64)) for t in (cos, sin))):
+            h, rows = decode_step_begin(tokens, positions, emb_weight, cos, sin)
+            return self(h, positions, rows, workgroups)
+        if any(t.shape != (B,) or t.dtype != torch.int64 or t.device != dev or not t.is_contiguous() for t in (tokens, positions)):
+            raise ValueError("DecodeStack: tokens or positions do not match the batch it was made for")
+        out = torch.empty(B, dim, dtype=torch.bfloat16, device=dev)
+        st = _lib.load_library().bitnet_decode_stack_step(
+            _ptr(self.entries), _ptr(self.workspace), _ptr(tokens), _ptr(emb_weight), _ptr(cos), _ptr(sin), _ptr(out),
+            _ptr(positions), emb_weight.shape[0], *self.shape, workgroups, 0, _stream_ptr())
+        if st != 0:
+            raise _lib.BitLinearLibraryError(f"bitnet_decode_stack_step: status {st}")
+        return out
+
     def check(self) -> None:
         """Raises if a wait inside the kernel gave up since the last check, and clears the condition (synchronises)."""
         if int(self._error.item()):
@@ -605,8 +629,7 @@ class Transformer(nn.Module):
         """decode_hidden_fused with all layers in one launch."""
         B = tokens.shape[0]
         pos = positions.reshape(B)
-        h, rows = decode_step_begin(tokens.reshape(B), pos, self.tok_embeddings.weight, cos, sin)
-        return stack(h, pos, rows)
+        return stack.step(tokens.reshape(B), pos, self.tok_embeddings.weight, cos, sin)
 
     @torch.no_grad()
     def prefill_hidden_fused(self, tokens, cache, cos, sin):

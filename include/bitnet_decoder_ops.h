@@ -239,6 +239,17 @@ int bitnet_decode_stack(const void* entries, void* workspace, const uint16_t* h_
                         const int64_t* positions, const float* rope_rows, int n_layers, int B, int S,
                         int dim, int ffn, int n_heads, int n_kv_heads, int n_splits, int workgroups,
                         int spin_limit, void* stream);
+/*
+ * bitnet_decode_step_begin and bitnet_decode_stack in one: the first layer reads the tokens' rows of the embedding, the
+ * attention the positions' rows of the tables.  Same results.
+ *   tokens     int64 [B] (clamped into the embedding), emb bf16 [V, dim], 16-byte aligned, V * dim * 2 below 2^31 - 16
+ *   cos_table, sin_table  fp32 [S, 64], a row for each of the cache's
+ */
+int bitnet_decode_stack_step(const void* entries, void* workspace, const int64_t* tokens, const uint16_t* emb,
+                             const float* cos_table, const float* sin_table, uint16_t* h_out,
+                             const int64_t* positions, int V, int n_layers, int B, int S, int dim, int ffn,
+                             int n_heads, int n_kv_heads, int n_splits, int workgroups, int spin_limit,
+                             void* stream);
 
 #ifdef __cplusplus
 }

@@ -849,6 +849,38 @@ def test_decode_stack_kernel_equals_the_kernels_per_layer(B, dim, ffn, nh, nkv, 
         step(9, min(33, S - 1))
 
 
+@pytest.mark.parametrize("workgroups", [0, 7])
+@pytest.mark.parametrize("B,dim,ffn,nh,nkv,S,V", [(1, 128, 64, 1, 1, 33, 3), (2, 1152, 2112, 9, 9, 40, 70), (3, 128, 64, 1, 1, 40, 1),
+                                                  (8, 2560, 6912, 20, 5, 70, 256)])
+def test_decode_stack_kernel_looks_tokens_and_positions_up_as_the_kernel_in_front_of_it(B, dim, ffn, nh, nkv, S, V, workgroups):
+    """Tokens that repeat and that lie outside the embedding, positions outside the cache, a 0xffff in the embedding (which a
+    published row cannot hold); tables longer than the cache take the two launches."""
+    args = decoder.ModelArgs(dim=dim, n_layers=2, n_heads=nh, n_kv_heads=nkv, vocab_size=256, ffn_dim=ffn)
+    model = _build(args, seed=dim + B)
+    caches = [model.make_cache(B, S, "cuda") for _ in range(2)]
+    for (k, v), (k2, v2) in zip(*caches):
+        k2.copy_(k.normal_())
+        v2.copy_(v.normal_())
+    emb = torch.randn(V, dim, device="cuda").to(torch.bfloat16)
+    emb.view(torch.int16)[V - 1, dim - 1] = -1
+    stacks = [decoder.DecodeStack(model, B, c, 3) for c in caches]
+    for rows in (S, S + 5):
+        cos, sin = decoder.rope_tables(128, rows, args.rope_theta, "cuda")
+        for tok, pos in (([0] * B, range(B)), (range(V - B, V), [S - 1] * B), (range(-1, B - 1), range(S - 2, S - 2 + B)),
+                         ([V // 2, V, 0, V - 1, 1, V + 9, -(1 << 40), 1 << 40][:B], [-3, 31, 32, S + 4, 0, 1, 1 << 40, 5][:B])):
+            tok, pos = (torch.tensor(list(t), dtype=torch.int64, device="cuda") for t in (tok, pos))
+            h, factors = decoder.decode_step_begin(tok, pos, emb, cos, sin)
+            want = stacks[0](h, pos, factors, workgroups)
+            got = stacks[1].step(tok, pos, emb, cos, sin, workgroups)
+            for stack in stacks:
+                stack.check()
+            assert torch.equal(torch.isnan(got), torch.isnan(want))
+            same = (got.view(torch.int16) == want.view(torch.int16)) | torch.isnan(want)
+            assert bool(same.all())
+            for (k, v), (k2, v2) in zip(*caches):
+                assert torch.equal(k.view(torch.int16), k2.view(torch.int16)) and torch.equal(v.view(torch.int16), v2.view(torch.int16))
+
+
 @pytest.mark.parametrize("B,dim,ffn,nh,nkv,S,n_splits", [(1, 128, 64, 1, 1, 70, 1), (2, 1024, 1984, 8, 1, 70, 2), (8, 512, 64, 4, 1, 70, 3)])
 def test_decode_stack_kernel_takes_the_new_row_at_every_place_of_a_block(B, dim, ffn, nh, nkv, S, n_splits):
     """As test_decode_stack_kernel_equals_the_kernels_per_layer, sequence after sequence over the 32 positions of a block."""
