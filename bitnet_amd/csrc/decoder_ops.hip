@@ -221,8 +221,10 @@ __global__ __launch_bounds__(kLmThreads) void lm_head_kernel(const uint16_t* __r
                 v = wv[k][tid];
                 i = wi[k][tid];
             }
-        part_val[(size_t)blockIdx.x * kLmMaxTokens + tid] = v;
-        part_idx[(size_t)blockIdx.x * kLmMaxTokens + tid] = i;
+        if (tid < B) {
+            part_val[(size_t)tid * gridDim.x + blockIdx.x] = v;
+            part_idx[(size_t)tid * gridDim.x + blockIdx.x] = i;
+        }
     }
 }
 
@@ -409,12 +411,14 @@ __global__ __launch_bounds__(kLmThreads) void lm_head_stream_kernel(const uint16
                         i = ci[k][tid][r];
                     }
         }
-        part_val[(size_t)blockIdx.x * kLmMaxTokens + tid] = v;
-        part_idx[(size_t)blockIdx.x * kLmMaxTokens + tid] = i;
+        if (tid < B) {
+            part_val[(size_t)tid * gridDim.x + blockIdx.x] = v;
+            part_idx[(size_t)tid * gridDim.x + blockIdx.x] = i;
+        }
     }
 }
 
-// Best (value, row) per token over the workgroups' partial results: one workgroup, all loads of a
+// Best (value, row) per token over the workgroups' partial results, [token][workgroup]: one workgroup, all loads of a
 // thread independent and in flight together (a dependent chain of single loads would cost a
 // memory round trip each).  A kernel of its own: the kernel boundary orders the partial results for
 // free, where a device-wide arrival counter would serialise thousands of atomics on one address.
@@ -433,87 +437,71 @@ __global__ __launch_bounds__(kLmFinalThreads) void lm_head_final_kernel(const fl
                                                                         const int* __restrict__ part_idx,
                                                                         int64_t* __restrict__ token_out, int nparts, int B,
                                                                         LmStepBook book) {
-    // The candidates are [nparts][16 token slots]; a thread reads whole 16-byte pieces (four token
-    // slots of one workgroup's candidates), consecutive threads consecutive pieces.  One workgroup's
-    // loads all go through one CU's address path, which handles one 64-byte segment per cycle: with
-    // a lane per candidate and a wave per token every load instruction touched 64 segments and the
-    // kernel took 16 us; now a load instruction touches 16.
-    __shared__ float sv[kLmFinalThreads / 64][kLmMaxTokens];
-    __shared__ int si[kLmFinalThreads / 64][kLmMaxTokens];
+    // The waves are dealt to the tokens (their number rounded up to a power of two) in turn.  With [workgroup][16 tokens], all
+    // read whatever the batch, one CU's address path had 128 KB to fetch, and what the bookkeeping reads was requested behind the
+    // reduction: 5.4 us at one token, 4.0 now; 5.7 and 4.0 at eight (under the profiler)
+    __shared__ float sv[kLmFinalThreads / 64];
+    __shared__ int si[kLmFinalThreads / 64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int q = tid & 3;  // this thread's token slots are 4 q .. 4 q + 3
-    float v[4];
-    int i[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        v[e] = -INFINITY;
-        i[e] = 0x7fffffff;
-    }
-    const int nvec = nparts * 4;
-    constexpr int U = 4;
-    for (int base = tid; base < nvec; base += kLmFinalThreads * U) {
-        v4f ov[U];
-        v4i oi[U];
+    const int slots = B <= 1 ? 1 : B <= 2 ? 2 : B <= 4 ? 4 : B <= 8 ? 8 : 16;
+    const int mine = wave & (slots - 1), stride = kLmFinalThreads / slots;
+    const size_t row = (size_t)(mine < B ? mine : B - 1) * nparts;
+    const int64_t step = book.step_idx ? book.step_idx[0] : 0;
+    const int64_t position = book.positions && tid < B ? book.positions[tid] : 0;
+    float v = -INFINITY;
+    int i = 0x7fffffff;
+    constexpr int U = 8;
+    for (int base = wave / slots * 64 + lane; base < nparts; base += stride * U) {
+        float ov[U];
+        int oi[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int k = base + kLmFinalThreads * u;
-            const int at = k < nvec ? k : nvec - 4 + q;  // a piece of the same token slots
-            ov[u] = ((const v4f*)part_val)[at];
-            oi[u] = ((const v4i*)part_idx)[at];
+            const int k = base + stride * u;
+            ov[u] = -INFINITY;
+            oi[u] = 0x7fffffff;
+            if (k < nparts) {
+                ov[u] = part_val[row + k];
+                oi[u] = part_idx[row + k];
+            }
         }
 #pragma unroll
         for (int u = 0; u < U; ++u)
-            if (base + kLmFinalThreads * u < nvec) {
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (lm_better(ov[u][e], oi[u][e], v[e], i[e])) {
-                        v[e] = ov[u][e];
-                        i[e] = oi[u][e];
-                    }
+            if (lm_better(ov[u], oi[u], v, i)) {
+                v = ov[u];
+                i = oi[u];
             }
     }
-    // the 16 lanes of a wave that hold the same token slots
 #pragma unroll
-    for (int off = 4; off < 64; off <<= 1) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const float ov = __shfl_xor(v[e], off);
-            const int oi = __shfl_xor(i[e], off);
-            if (lm_better(ov, oi, v[e], i[e])) {
-                v[e] = ov;
-                i[e] = oi;
-            }
+    for (int off = 1; off < 64; off <<= 1) {
+        const float ov = __shfl_xor(v, off);
+        const int oi = __shfl_xor(i, off);
+        if (lm_better(ov, oi, v, i)) {
+            v = ov;
+            i = oi;
         }
     }
-    if (lane < 4) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            sv[wave][4 * lane + e] = v[e];
-            si[wave][4 * lane + e] = i[e];
-        }
+    if (lane == 0) {
+        sv[wave] = v;
+        si[wave] = i;
     }
     __syncthreads();
     if (tid < kLmMaxTokens) {
-        const int t = tid;
-        float bv = sv[0][t];
-        int bi = si[0][t];
-#pragma unroll
-        for (int w = 1; w < kLmFinalThreads / 64; ++w)
-            if (lm_better(sv[w][t], si[w][t], bv, bi)) {
-                bv = sv[w][t];
-                bi = si[w][t];
+        const int t = tid & (slots - 1);
+        float bv = sv[t];
+        int bi = si[t];
+        for (int w = t + slots; w < kLmFinalThreads / 64; w += slots)
+            if (lm_better(sv[w], si[w], bv, bi)) {
+                bv = sv[w];
+                bi = si[w];
             }
-        if (t < B) {
+        if (tid < B) {
             token_out[t] = (int64_t)bi;
             if (book.next_input) book.next_input[t] = (int64_t)bi;
-            if (book.positions) book.positions[t] += 1;
-            if (book.history && book.step_idx) book.history[book.step_idx[0] * B + t] = (int64_t)bi;
+            if (book.positions) book.positions[t] = position + 1;
+            if (book.history && book.step_idx) book.history[step * B + t] = (int64_t)bi;
         }
     }
-    if (book.step_idx) {
-        __syncthreads();  // every token's history row index has been read
-        if (tid == 0) book.step_idx[0] += 1;
-    }
+    if (book.step_idx && tid == 0) book.step_idx[0] = step + 1;  // (read in front of the barrier by all)
 }
 
 
