@@ -2483,6 +2483,13 @@ constexpr int kRingMost64x256 = 340;
 // ... from this K on (128 x 2560 x 384 3.6 against 4.1 us, 512 x 2560 x 384 5.1 against 5.5; at K = 256 512 rows level, 300
 // 4.0 against 3.8); the 64 x 256 tiles later (76 x 17632 x 640 6.2 against 5.55, 247 x 8384 x 1024 7.4 against 7.5)
 constexpr int kRingMinK = 384, kRingMinK64x256 = 1024;
+// 64 x 96 tiles instead of 64 x 128, and 64 x 192 instead of 64 x 256, where there are at most one per CU of them: what a tile
+// multiplies is a quarter less, what it brings into its CU a twelfth or an eighth, and its time besides the loop 0.1 to 0.2 us
+// more (half the computing waves; sums through LDS, which the 64 x 256 tile does without).  So from these K on: 64 x 128 / 64 x 96 at 512 x 2560 x 2560 7.8 / 7.85 us, 300 x 4800 x 3200 8.7 / 8.65, 501 x 2656 x 5120 10.9 / 10.7, 403 x 2560 x 6912
+// 12.7 / 12.2, 412 x 3200 x 10240 18.7 / 17.6; 64 x 256 / 64 x 192 at 182 x 13520 x 1152 7.65 / 7.85, 937 x 2576 x 1536 8.67 / 8.7, 456 x
+// 4368 x 1664 8.85 / 8.75, 685 x 3840 x 2560 11.4 / 10.95, 70 x 20480 x 3200 12.8 / 11.9, 1032 x 2560 x 6912 23.25 / 21.65, 94 x
+// 19152 x 7552 24.2 / 21.1
+constexpr int kRingMinK64x96 = 4096, kRingMinK64x192 = 1664;
 // ... and with rope or gate in the epilogue from the K on that their entry points state
 constexpr int kRingEpilogueMinK = 640;
 // the forward call's quantizer in the product's launch (HandedRows) while the rows, which every workgroup reads behind the hand-over,
@@ -3087,13 +3094,15 @@ int launch_solo_tok(const uint16_t* x, const int8_t* packed, uint16_t* out, int3
 }
 
 // The instances of the kernel in gemm_ring.h: 32 x 64 tiles whose K eight waves split, 64 x 128 tiles split by four, 64 x 256
-// (two workgroups per CU) and 128 x 256 tiles, 64 x 64 tiles split by four
+// (two workgroups per CU) and 128 x 256 tiles, 64 x 64 and 64 x 96 tiles split by four, 64 x 192 ones by two
 #define BITLINEAR_RING_A 1, 2, 1, 1, 8, 512, 6, 0
 #define BITLINEAR_RING_B 2, 2, 1, 2, 4, 256, 6, 4
 #define BITLINEAR_RING_C 2, 2, 1, 4, 1, 128, 4, 4
 #define BITLINEAR_RING_D 2, 2, 2, 4, 1, 128, 6, 4
 #define BITLINEAR_RING_E 2, 2, 1, 1, 4, 256, 6, 4
-constexpr int kRingRows[6] = {0, 32, 64, 64, 128, 64}, kRingCols[6] = {0, 64, 128, 256, 256, 64};
+#define BITLINEAR_RING_F 2, 3, 1, 1, 4, 256, 6, 4
+#define BITLINEAR_RING_G 2, 3, 1, 2, 2, 128, 6, 4
+constexpr int kRingRows[8] = {0, 32, 64, 64, 128, 64, 64, 64}, kRingCols[8] = {0, 64, 128, 256, 256, 64, 96, 192};
 long long ring_tiles(int M, int N, int ring) {
     return (long long)((M + kRingRows[ring] - 1) / kRingRows[ring]) * ((N + kRingCols[ring] - 1) / kRingCols[ring]);
 }
@@ -3101,17 +3110,19 @@ long long ring_tiles(int M, int N, int ring) {
 bool ring_aligned(const uint16_t* out, const int32_t* acc_out, const uint16_t* residual, int K) {
     return K % 128 == 0 && ((((uintptr_t)out) | ((uintptr_t)acc_out) | ((uintptr_t)residual)) & 15u) == 0;
 }
-// which instance a product takes; 0: none
-int ring_choice(int M, int N, int K, const ScaleMap& smap, bool aligned) {
+// which instance a product takes; 0: none.  gate: of those that have it
+int ring_choice(int M, int N, int K, const ScaleMap& smap, bool aligned, bool gate = false) {
     if (!aligned) return 0;
     for (int j = 0; j + 1 < smap.nseg; ++j)
         if (smap.ends[j] % 8) return 0;  // eight outputs share a weight scale
-    if (t_tune.path == 5) return t_tune.prefill_big >= 9 ? t_tune.prefill_big - 8 : 0;
+    if (t_tune.path == 5) return t_tune.prefill_big >= 9 && !(gate && t_tune.prefill_big >= 14) ? t_tune.prefill_big - 8 : 0;
     if (t_tune.path != 0) return 0;
     if (K < kRingMinK) return 0;
     if (ring_tiles(M, N, 1) <= kRingCus) return 1;
     if (ring_tiles(M, N, 5) <= kRingCus) return 5;
+    if (!gate && K >= kRingMinK64x96 && ring_tiles(M, N, 6) <= kRingCus) return 6;
     if (ring_tiles(M, N, 2) <= kRingCus) return 2;
+    if (!gate && K >= kRingMinK64x192 && ring_tiles(M, N, 7) <= kRingCus) return 7;
     if (ring_tiles(M, N, 3) <= kRingMost64x256) return K >= kRingMinK64x256 ? 3 : 0;
     if (ring_tiles(M, N, 4) <= kRingCus) return 4;
     return 0;
@@ -3147,10 +3158,10 @@ bool splitk_ahead(int M, int N, int K, int ring) {
     // 4.75 / 5.65, 17 x 2560 x 6912 7.45 / 7.75, 17 x 2560 x 512 3.3 / 3.15, 51 x 2560 x 384 3.45 / 3.3, 51 x 1024 x 512 3.4 / 2.85, 51 x
     // 3728 x 512 3.55 / 3.95, 128 x 2560 x 384 3.6 / 4.15, 200 x 1024 x 512 3.5 / 3.85; 64 x 64 4.1 at 200 x 2560 x 384, 5.75 at 193 x 2560 x
     // 2560, 9.4 at 193 x 2560 x 6912; 64 x 128 4.7 at 100 x 10240 x 384, 7.3, 12.4
-    if (ring == 1 || ring == 2 || ring == 5) {
+    if (ring == 1 || ring == 2 || ring == 5 || ring == 6) {
         const double splitk_us = 2.6 + 1.09 * (M / 16.0) * ((double)N * K / 4.0) / 1.45e6 + 0.0004 * K;
         const double chunks = K / 256.0;
-        const double ring_us = ring == 1 ? 3.2 + 0.148 * chunks + 0.002 * ring_tiles(M, N, 1) : (ring == 5 ? 3.7 + 0.21 * chunks : 4.2 + 0.29 * chunks);
+        const double ring_us = ring == 1 ? 3.2 + 0.148 * chunks + 0.002 * ring_tiles(M, N, 1) : (ring == 5 ? 3.7 + 0.21 * chunks : ring == 6 ? 3.9 + 0.25 * chunks : 4.2 + 0.29 * chunks);
         return ring_us > splitk_us;
     }
     const double groups = (M + 15) / 16;
@@ -3179,8 +3190,8 @@ bool gate_ahead(int M, int N, int K, int ring) {
     return !(mp.wanted && mp.quarters <= kGateMixQuarters && K % 256 == 0) && !splitk_ahead(M, N, K, ring);
 }
 // which instance a product with rope or gate in its epilogue takes; 0: none
-int epilogue_ring(int M, int N, int K, const ScaleMap& smap) {
-    return K < kRingEpilogueMinK && t_tune.path == 0 ? 0 : ring_choice(M, N, K, smap, K % 128 == 0);
+int epilogue_ring(int M, int N, int K, const ScaleMap& smap, bool gate) {
+    return K < kRingEpilogueMinK && t_tune.path == 0 ? 0 : ring_choice(M, N, K, smap, K % 128 == 0, gate);
 }
 template <class Epi>
 int launch_ring(int ring, const int8_t* act, const int8_t* packed, uint16_t* out, int32_t* acc_out, const uint16_t* s,
@@ -3201,6 +3212,10 @@ int launch_ring(int ring, const int8_t* act, const int8_t* packed, uint16_t* out
         BITLINEAR_RING_LDS(BITLINEAR_RING_C);
         BITLINEAR_RING_LDS(BITLINEAR_RING_D);
         BITLINEAR_RING_LDS(BITLINEAR_RING_E);
+        if constexpr (!Epi::kGate) {
+            BITLINEAR_RING_LDS(BITLINEAR_RING_F);
+            BITLINEAR_RING_LDS(BITLINEAR_RING_G);
+        }
 #undef BITLINEAR_RING_LDS
         return e;
     });
@@ -3217,6 +3232,12 @@ int launch_ring(int ring, const int8_t* act, const int8_t* packed, uint16_t* out
         case 2: BITLINEAR_LAUNCH_RING(BITLINEAR_RING_B); break;
         case 3: BITLINEAR_LAUNCH_RING(BITLINEAR_RING_C); break;
         case 5: BITLINEAR_LAUNCH_RING(BITLINEAR_RING_E); break;
+        case 6:
+            if constexpr (!Epi::kGate) BITLINEAR_LAUNCH_RING(BITLINEAR_RING_F);
+            break;
+        case 7:
+            if constexpr (!Epi::kGate) BITLINEAR_LAUNCH_RING(BITLINEAR_RING_G);
+            break;
         default: BITLINEAR_LAUNCH_RING(BITLINEAR_RING_D); break;
     }
 #undef BITLINEAR_LAUNCH_RING
@@ -3771,7 +3792,7 @@ int bitlinear_set_tuning(int kernel, int a, int b, int c) {
         return set_status(BITLINEAR_OK);
     }
     if (kernel == 5) {
-        if (a < 0 || a > 13 || b < 0 || b > 64 || (c != 0 && c != 1 && c != 2 && c != 4)) return set_status(BITLINEAR_ERR_ARG);
+        if (a < 0 || a > 15 || b < 0 || b > 64 || (c != 0 && c != 1 && c != 2 && c != 4)) return set_status(BITLINEAR_ERR_ARG);
         g.path = 5;
         g.prefill_big = a;
         g.prefill_ks = c;
@@ -4181,7 +4202,7 @@ static int norm_ring_impl(const uint16_t* x, const uint16_t* norm_weight, float 
         const int st = segment_map(seg_ends, nseg, N, &sm);
         if (st != BITLINEAR_OK) return set_status(st);
     }
-    const int ring = M > kPrefillMinTokens && K <= kPreThreads * kPreVecs * 8 ? epilogue_ring(M, N, K, sm) : 0;
+    const int ring = M > kPrefillMinTokens && K <= kPreThreads * kPreVecs * 8 ? epilogue_ring(M, N, K, sm, Epi::kGate) : 0;
     if (!ring || (Epi::kGate && N % 32)) return set_status(BITLINEAR_ERR_SHAPE);
     const int st = launch_norm_quant(x, norm_weight, eps, 0, q_ws, s_ws, M, K, mode, (hipStream_t)stream);
     if (st != BITLINEAR_OK) return set_status(st);
@@ -4195,14 +4216,14 @@ int bitlinear_norm_epilogue_applies(int M, int N, int K, const int* seg_ends, in
     if (!shape_ok(M, N, K) || N % 32 || M <= kPrefillMinTokens || K > kPreThreads * kPreVecs * 8) return 0;
     ScaleMap sm = equal_slots(N, bitlinear_ws_num(N, K));
     if (seg_ends && segment_map(seg_ends, nseg, N, &sm) != BITLINEAR_OK) return 0;
-    return epilogue_ring(M, N, K, sm) != 0;
+    return epilogue_ring(M, N, K, sm, true) != 0 && epilogue_ring(M, N, K, sm, false) != 0;
 }
 
 int bitlinear_norm_gate_ahead(int M, int N, int K, const int* seg_ends, int nseg) {
     if (!bitlinear_norm_epilogue_applies(M, N, K, seg_ends, nseg)) return 0;
     ScaleMap sm = equal_slots(N, bitlinear_ws_num(N, K));
     if (seg_ends) segment_map(seg_ends, nseg, N, &sm);
-    return gate_ahead(M, N, K, ring_choice(M, N, K, sm, true));
+    return gate_ahead(M, N, K, ring_choice(M, N, K, sm, true, true));
 }
 
 int bitlinear_norm_gate_forward_bf16(const uint16_t* x, const uint16_t* norm_weight, float eps, const int8_t* packed,

@@ -24,6 +24,8 @@
 //  * LDS reads run at 220 bytes a cycle without conflicts (rows swizzled so that 16 rows at one piece fall on 16
 //    different slots of the 256 bytes that the banks span), writes at 76: with KG groups of waves that split the k-steps
 //    of a stage, sums go through LDS once, and with KG = 1 not at all (512 x 13824 x 2560: 21.2 -> 20.2 us).
+//  * two loader waves instead of four: the 64 x 64 tile's loop 2.46 -> 3.06 us per 2560 k.  So where a stage's loads do not divide by
+//    four some of those waves have one load less (64 x 96 tiles 13.6 -> 12.5 us at 512 x 2560 x 6912).
 // One barrier per stage: behind it the next stage is complete for every wave, so the first operands of a stage are read
 // while the one in front is still being multiplied, and the stage before that is free for the loaders.  (Behind the last
 // chunk operands are read from a stage that was not requested; nothing multiplies them.)
@@ -48,13 +50,14 @@ struct Ring {
     static constexpr int RPI = 64 / PPR;         // activation rows one load instruction of a wave covers
     static constexpr int SWZ_SHIFT = PPR == 8 ? 1 : 0, SWZ = PPR == 8 ? 7 : 15;
     static constexpr int A_BYTES = TM * CK, W_BYTES = TN * CK / 4, STAGE = A_BYTES + W_BYTES;
-    static constexpr int AR = A_BYTES / 1024 / LWAVES, WR = W_BYTES / 1024 / LWAVES, LOADS = AR + WR;
+    static constexpr int AR = A_BYTES / 1024 / LWAVES, WR = (W_BYTES / 1024 + LWAVES - 1) / LWAVES, LOADS = AR + WR;
+    static constexpr int WX = W_BYTES / 1024 % LWAVES;  // not zero: that many loading waves have the last load of a stage, the others not
     static constexpr int OUT_ROW = TN * 4 + 16;  // bytes of a row of sums: 16 rows at one column fall on 16 different 16-byte slots
     static constexpr int RED = KG > 1 ? KG * TM * OUT_ROW : 0;
     static constexpr int LDS = S * STAGE > RED ? S * STAGE : RED;
     static constexpr int THREADS = 64 * (WAVES + LW);
     static constexpr int WGS = 2 * (LDS + TM * 8 + 64) <= 160 * 1024 ? 2 : 1;  // workgroups per CU
-    static_assert(AR * LWAVES * 1024 == A_BYTES && WR * LWAVES * 1024 == W_BYTES, "whole load instructions per wave");
+    static_assert(AR * LWAVES * 1024 == A_BYTES && W_BYTES % 1024 == 0 && (LW || WX == 0), "whole load instructions per wave");
     static_assert(KPW >= 2 && KPW % 2 == 0 && KPW * KG == KSTEPS, "operand registers alternate");
     static_assert(S >= 4 && (S - 1) * LOADS <= 63, "loads in flight are counted in six bits");
     static_assert(LDS + TM * 8 + 64 <= 160 * 1024, "LDS of a CU");
@@ -79,7 +82,7 @@ struct RingRope {
     uint16_t *cache_k, *cache_v, *q_out;
     int T, S, n_heads, n_kv;
 };
-// N words, two or four, in one piece
+// N words, two to four
 template <int N>
 struct RingWords {
     typedef uint32_t type __attribute__((ext_vector_type(N)));
@@ -102,6 +105,9 @@ void gemm_i2_prefill_kernel(
     typedef Ring<MT, NT, WM, WN, KG, CK, S, LW> R;
     constexpr int QR = 8 / NT;
     constexpr int COLS = Epi::kGate ? R::TN / 2 : R::TN;  // output columns of a tile
+    // a wave's column tiles lie 32 columns (of the gate: half the rows) apart; otherwise they interleave, and their words are one read
+    constexpr bool kApart = Epi::kGate || NT == 3;
+    static_assert(NT != 3 || KG > 1, "outputs straight from the registers are those of interleaved column tiles");
     static_assert(!Epi::kGate || NT == 2, "a column tile of either half");
     extern __shared__ __attribute__((aligned(1024))) int8_t lds_x[];
 
@@ -150,12 +156,12 @@ void gemm_i2_prefill_kernel(
         w_k[r] = ks * 32;
         w_voff[r] = blk * K * 4 + ks * 128 + (q & 7) * 16;
     }
-    // part p of P of a stage's requests
-    auto issue = [&](int c, int st, int p, int P) {
+    // part p of P of a stage's requests, `loads` a wave
+    auto issue = [&](int c, int st, int p, int P, auto loads) {
         const int left = K - c * CK;  // k in front of the end of the rows
         int8_t* to = lds_x + st * R::STAGE;
 #pragma unroll
-        for (int r = 0; r < R::LOADS; ++r) {
+        for (int r = 0; r < loads.value; ++r) {
             if (r * P / R::LOADS != p) continue;
             if (r < R::AR) {
                 load16_to_lds(a_rsrc, to + (r * R::LWAVES + lw) * 1024, a_k[r] < left ? a_voff[r] : kRingBeyond, c * CK);
@@ -166,8 +172,8 @@ void gemm_i2_prefill_kernel(
         }
     };
     // all of a wave's requests have arrived but those of its last `stages` stages
-    auto wait_all_but = [](auto stages) {
-        constexpr int n = decltype(stages)::value * R::LOADS;
+    auto wait_all_but = [](auto stages, auto loads) {
+        constexpr int n = decltype(stages)::value * decltype(loads)::value;
         __builtin_amdgcn_s_waitcnt(0x0f70 | (n & 15) | (n >> 4 << 14));
     };
     constexpr std::integral_constant<int, 0> none{};
@@ -180,64 +186,76 @@ void gemm_i2_prefill_kernel(
         asm volatile("" ::: "memory");
     };
     constexpr int kFirst = LW ? 3 : S - 1;  // stages requested in front of the first wait
-    if (lw >= 0) {
+    constexpr std::integral_constant<int, R::LOADS> all_loads{};
+    auto first_stages = [&](auto loads) {
 #pragma unroll
         for (int c = 0; c < kFirst; ++c)
-            if (c < nchunks) issue(c, c, 0, 1);
-    }
-    if (LW && lw >= 0) {
-        // at the end of chunk c stage c + 2 has to be there
+            if (c < nchunks) issue(c, c, 0, 1, loads);
+    };
+    // what a loading wave does: at the end of chunk c stage c + 2 has to be there
+    auto load_stages = [&](auto loads) {
+        first_stages(loads);
         if (nchunks <= S) {  // all of K fits the ring
-            wait_all_but(none);
+            wait_all_but(none, loads);
             meet();
-            for (int c = kFirst; c < nchunks; ++c) issue(c, c, 0, 1);
-            wait_all_but(none);
+            for (int c = kFirst; c < nchunks; ++c) issue(c, c, 0, 1, loads);
+            wait_all_but(none, loads);
             for (int c = 0; c < nchunks; ++c) meet();
         } else {
-            wait_all_but(one_stage);
+            wait_all_but(one_stage, loads);
             meet();
             int c = 0, st = kFirst % S;
             auto next_stage = [&](int i) {
-                issue(i, st, 0, 1);
+                issue(i, st, 0, 1, loads);
                 st = st + 1 == S ? 0 : st + 1;
             };
             if constexpr (S > 4) {  // two stages at a time until S - 1 are on their way
                 static_assert(S == 6, "two chunks of two stages");
                 next_stage(3);
                 next_stage(4);
-                wait_all_but(two_stages);
+                wait_all_but(two_stages, loads);
                 meet();
                 next_stage(5);
                 next_stage(6);
-                wait_all_but(full);
+                wait_all_but(full, loads);
                 meet();
                 c = 2;
             }
             for (; c + S - 1 < nchunks; ++c) {
                 next_stage(c + S - 1);
-                wait_all_but(full);
+                wait_all_but(full, loads);
                 meet();
             }
             if constexpr (S > 4) {
-                wait_all_but(two_stages);
+                wait_all_but(two_stages, loads);
                 meet();
-                wait_all_but(one_stage);
+                wait_all_but(one_stage, loads);
                 meet();
             }
-            wait_all_but(none);
+            wait_all_but(none, loads);
             for (int i = 0; i < 3; ++i) meet();
         }
         meet();
         lds_barrier();
+    };
+    if (LW && lw >= 0) {
+        if constexpr (R::WX != 0) {
+            if (lw >= R::WX) {
+                load_stages(std::integral_constant<int, R::LOADS - 1>{});
+                return;
+            }
+        }
+        load_stages(all_loads);
         return;
     }
+    if (!LW) first_stages(all_loads);
 
     // the outputs that go through LDS: eight of a row per thread, four where there are fewer
     constexpr int CPT = KG > 1 && R::TM * COLS < R::WAVES * 64 * 8 ? 4 : 8;
     constexpr int PER_ROW = COLS / CPT;            // threads that share a row
     constexpr int ROWS = R::WAVES * 64 / PER_ROW;  // rows that the threads cover at a time
     constexpr int TIMES = (R::TM + ROWS - 1) / ROWS;
-    const int pr = threadIdx.x / PER_ROW, pc = threadIdx.x % PER_ROW * CPT, n = n_base + pc;
+    const int pr = threadIdx.x / PER_ROW < ROWS ? threadIdx.x / PER_ROW : R::TM, pc = threadIdx.x % PER_ROW * CPT, n = n_base + pc;
     // the scales, for the epilogue
     __shared__ float sval[R::TM], rinv[R::TM], wsv[kMaxSeg];
     uint32_t s_raw = 0, ws_raw = 0;
@@ -276,14 +294,14 @@ void gemm_i2_prefill_kernel(
             for (int r = 0; r < 16; ++r) acc[mt][nt][r] = 0;
 
     // where the lane's operands are within a stage
-    typedef typename PfxWords<NT>::type wvec_t;
+    typedef typename RingWords<NT>::type wvec_t;
     int a_rd[R::KPW];
 #pragma unroll
     for (int j = 0; j < R::KPW; ++j)
         a_rd[j] = (wm * MT * 32 + nl) * CK + ((((grp * R::KPW + j) * 2 + kc) ^ ((nl >> R::SWZ_SHIFT) & R::SWZ)) * 16);
     const int w_rd = R::A_BYTES + grp * R::KPW * (R::TN * 8) +
-                     (Epi::kGate ? (wn * 4 + (nl >> 4)) * 128 + ((nl >> 3 & 1) * 16 + kc * 8 + (nl & 7)) * 4
-                                 : (wn * NT * 2 + nl / (2 * QR)) * 128 + (((nl % (2 * QR)) / QR) * 16 + kc * 8 + NT * (nl % QR)) * 4);
+                     (kApart ? (wn * NT * 2 + (nl >> 4)) * 128 + ((nl >> 3 & 1) * 16 + kc * 8 + (nl & 7)) * 4
+                             : (wn * NT * 2 + nl / (2 * QR)) * 128 + (((nl % (2 * QR)) / QR) * 16 + kc * 8 + NT * (nl % QR)) * 4);
     auto expand = [&](uint32_t wd) -> v4i {
         const uint32_t x = wd ^ 0xAAAAAAAAu;
         v4i r;
@@ -299,15 +317,19 @@ void gemm_i2_prefill_kernel(
     };
     auto read_w = [&](const int8_t* stage, int j) -> wvec_t {
         const int8_t* from = stage + w_rd + j * (R::TN * 8);
-        if constexpr (Epi::kGate)
-            return wvec_t{*(const uint32_t*)from, *(const uint32_t*)(from + 256)};
-        else
+        if constexpr (kApart) {
+            wvec_t w;
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) w[nt] = *(const uint32_t*)(from + nt * 256);
+            return w;
+        } else {
             return *(const wvec_t*)from;
+        }
     };
     // stages 0 and 1 are there (every wave waits for its own requests, then all meet)
     if (!LW) {
-        if (nchunks < S - 1) wait_all_but(none);
-        else wait_all_but(full);
+        if (nchunks < S - 1) wait_all_but(none, all_loads);
+        else wait_all_but(full, all_loads);
     }
     meet();
 
@@ -342,7 +364,7 @@ void gemm_i2_prefill_kernel(
 #pragma unroll
                 for (int i = 0; i < NT; ++i)
                     if ((i * SLOTS / NT + (SLOTS > NT ? 1 : 0)) % SLOTS == slot) bop[nxt][i] = expand(wraw[nxt][i]);
-                if (load.value && slot == SLOTS - 1) issue(c + S - 1, st == 0 ? S - 1 : st - 1, j, R::KPW);
+                if (load.value && slot == SLOTS - 1) issue(c + S - 1, st == 0 ? S - 1 : st - 1, j, R::KPW, all_loads);
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
@@ -356,14 +378,14 @@ void gemm_i2_prefill_kernel(
     } else {
         for (int c = 0; c + S - 1 < nchunks; ++c) {
             chunk(c, std::true_type{});
-            wait_all_but(full);  // the chunk behind the next one has to be there before the next one ends
+            wait_all_but(full, all_loads);  // the chunk behind the next one has to be there before the next one ends
             meet();
         }
         auto last = [&](auto behind) {  // ... that has `behind` chunks behind it
             constexpr int n = decltype(behind)::value;
             if (nchunks <= n) return;
             chunk(0, std::false_type{});
-            wait_all_but(std::integral_constant<int, (n > 2 ? n - 2 : 0)>{});
+            wait_all_but(std::integral_constant<int, (n > 2 ? n - 2 : 0)>{}, all_loads);
             meet();
         };
         static_assert(S == 6, "S - 1 chunks without requests");
@@ -501,16 +523,16 @@ void gemm_i2_prefill_kernel(
 #pragma unroll
             for (int g4 = 0; g4 < 4; ++g4) {
                 const int ridx = g4 * 8 + kc * 4;
-                const int n = Epi::kGate ? ridx : 16 * (ridx / (2 * QR)) + 8 * ((ridx % (2 * QR)) / QR) + NT * (ridx % QR);
+                const int n = kApart ? ridx : 16 * (ridx / (2 * QR)) + 8 * ((ridx % (2 * QR)) / QR) + NT * (ridx % QR);
 #pragma unroll
                 for (int v = 0; v < NT; ++v) {
                     v4i t;
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
-                        const int i = 4 * v + j;  // column n + i: register i / NT of the quad, column tile i % NT (gate: of half v)
-                        t[j] = Epi::kGate ? acc[mt][v][g4 * 4 + j] : acc[mt][i % NT][g4 * 4 + i / NT];
+                        const int i = 4 * v + j;  // column n + i: register i / NT of the quad, column tile i % NT (apart: of tile v)
+                        t[j] = kApart ? acc[mt][v][g4 * 4 + j] : acc[mt][i % NT][g4 * 4 + i / NT];
                     }
-                    *(v4i*)(to + mt * 32 * R::OUT_ROW + (n + v * (Epi::kGate ? COLS : 4)) * 4) = t;
+                    *(v4i*)(to + mt * 32 * R::OUT_ROW + (n + v * (Epi::kGate ? COLS : kApart ? 32 : 4)) * 4) = t;
                 }
             }
     }

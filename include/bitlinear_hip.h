@@ -359,8 +359,8 @@ int bitlinear_plan_name(int entry, int M, int N, int K, char* buf, int buflen);
  *             128 x 256 through the other), 8 = whole rounds of 64 x 256 tiles over
  *             the first columns and 32 x 128 tiles behind them in one launch (the
  *             built-in choice when those are at most about 1.4 per CU; needs
- *             K % 128 == 0), 9 .. 13 = 32 x 64, 64 x 128, 64 x 256, 128 x 256 and 64 x 64 through
- *             the kernel that brings activations and weights through LDS (the built-in
+ *             K % 128 == 0), 9 .. 15 = 32 x 64, 64 x 128, 64 x 256, 128 x 256, 64 x 64, 64 x 96 and
+ *             64 x 192 (the last two not with the gate) through the kernel that brings activations and weights through LDS (the built-in
  *             choice while there is about one such tile per CU; needs K % 128 == 0, else
  *             as 5; c does not apply); b = without effect (0 .. 64; the order of
  *             tiles is one for all sizes); c = groups of four waves that split a

@@ -592,6 +592,18 @@ def test_prefill_gemm_in_64_x_64_tiles(m, n, k):
     test_prefill_gemm_with_both_operands_through_lds(m, n, k, 13)
 
 
+@pytest.mark.parametrize("m,n,k", [(17, 16, 128), (33, 80, 384), (63, 96, 512), (64, 192, 640), (65, 208, 896), (129, 1040, 1408), (257, 3840, 2560)])
+@pytest.mark.parametrize("tile", [14, 15])
+def test_prefill_gemm_in_tiles_of_96_and_192_columns(m, n, k, tile):
+    test_prefill_gemm_with_both_operands_through_lds(m, n, k, tile)
+
+
+@pytest.mark.parametrize("tile", [14, 15])
+@pytest.mark.parametrize("k", [128, 512, 640, 768, 1024, 1280, 1536, 1792, 2048, 2432])
+def test_prefill_gemm_in_tiles_of_96_and_192_columns_from_the_first_stage_to_the_last(k, tile):
+    test_prefill_gemm_with_both_operands_through_lds(49, 112, k, tile)
+
+
 @pytest.mark.parametrize("tile", [9, 10, 11, 12, 13])
 @pytest.mark.parametrize("k", [128, 512, 640, 768, 1024, 1152, 1536, 1792, 2048, 2432, 3072, 3584, 4096])
 def test_prefill_gemm_through_lds_from_the_first_stage_to_the_last(k, tile):

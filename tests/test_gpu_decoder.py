@@ -768,6 +768,13 @@ def test_prompt_products_with_rope_and_gate_in_the_epilogue_equal_the_separate_c
         assert np.array_equal(host_bits(got_h), want_h)
 
 
+@pytest.mark.parametrize("B,T,K", [(3, 224, 2560), (3, 90, 4096)])  # 64 x 192 and 64 x 96 tiles, which have rope and not the gate
+def test_prompt_products_with_rope_in_the_epilogue_of_tiles_of_three_column_tiles_a_wave(B, T, K):
+    name = _lib.plan_name(0, B * T, 3840, K)
+    assert "<2, 3, 1, 2, 2, 128" in name or "<2, 3, 1, 1, 4, 256" in name, name
+    test_prompt_products_with_rope_and_gate_in_the_epilogue_equal_the_separate_calls(B, T, 20, 5, K, 1040, 300, 0)
+
+
 @pytest.mark.parametrize("B,T,nh,nkv,K,ffn,S", [(1, 17, 1, 1, 640, 16, 17), (1, 33, 20, 5, 2560, 6912, 40), (3, 65, 20, 5, 1280, 1040, 200)])
 def test_prompt_products_with_epilogues_in_64_x_64_tiles_equal_the_separate_calls(B, T, nh, nkv, K, ffn, S):
     test_prompt_products_with_rope_and_gate_in_the_epilogue_equal_the_separate_calls(B, T, nh, nkv, K, ffn, S, 13)
