@@ -1330,16 +1330,16 @@ struct FusedExtras {
 // is too large for every workgroup of the fused kernel to redo this work.
 // Same arithmetic, in the same order, as the PRO 1 / 2 prologue below.
 // ---------------------------------------------------------------------------
-constexpr int kPreThreads = 512;
+constexpr int kPreThreads = 512;  // ... or 256
 constexpr int kPreVecs = 8;  // at most this many 16-byte vectors per thread: rows up to 8 * 512 * 8 = 32768 elements
 
-template <int PRO, int VQ>  // VQ: vectors per thread, VQ * 512 * 8 >= K
-__global__ __launch_bounds__(kPreThreads) void norm_quant_kernel(const uint16_t* __restrict__ x,
-                                                                 const uint16_t* __restrict__ norm_weight, float eps,
-                                                                 int8_t* __restrict__ q, uint16_t* __restrict__ s,
-                                                                 int K, int mode) {
-    __shared__ uint32_t wmax[kPreThreads / 64];
-    __shared__ double wsq[kPreThreads / 64];
+template <int PRO, int VQ, int THREADS>  // VQ: vectors per thread, VQ * THREADS * 8 >= K
+__global__ __launch_bounds__(THREADS) void norm_quant_kernel(const uint16_t* __restrict__ x,
+                                                             const uint16_t* __restrict__ norm_weight, float eps,
+                                                             int8_t* __restrict__ q, uint16_t* __restrict__ s,
+                                                             int K, int mode) {
+    __shared__ uint32_t wmax[THREADS / 64];
+    __shared__ double wsq[THREADS / 64];
     const int row = blockIdx.x;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -1351,7 +1351,7 @@ __global__ __launch_bounds__(kPreThreads) void norm_quant_kernel(const uint16_t*
     uint4 xv[VQ], gv[VQ], x3v[PRO == 2 ? VQ : 1];
 #pragma unroll
     for (int r = 0; r < VQ; ++r) {
-        const int idx = (tid + r * kPreThreads) < nvec ? (tid + r * kPreThreads) : (nvec - 1);
+        const int idx = (tid + r * THREADS) < nvec ? (tid + r * THREADS) : (nvec - 1);
         xv[r] = *(const uint4*)(xr + idx * 8);
         if (PRO == 2) x3v[r] = *(const uint4*)(xr + K + idx * 8);
         gv[r] = *(const uint4*)(norm_weight + idx * 8);
@@ -1360,34 +1360,34 @@ __global__ __launch_bounds__(kPreThreads) void norm_quant_kernel(const uint16_t*
 #pragma unroll
     for (int r = 0; r < VQ; ++r) {
         if (PRO == 2) xv[r] = glu8(xv[r], x3v[r]);
-        if (tid + r * kPreThreads < nvec) sq += sumsq8(xv[r]);
+        if (tid + r * THREADS < nvec) sq += sumsq8(xv[r]);
     }
     const double wsum = wave_sum_f64(sq);
     if (lane == 0) wsq[wave] = wsum;
     __syncthreads();
     double total = 0.0;
 #pragma unroll
-    for (int i = 0; i < kPreThreads / 64; ++i) total += wsq[i];
+    for (int i = 0; i < THREADS / 64; ++i) total += wsq[i];
     const float mean = (float)total / (float)K;
     const float rstd = 1.0f / __builtin_sqrtf(mean + eps);
     uint32_t am = 0;
 #pragma unroll
     for (int r = 0; r < VQ; ++r) {
         xv[r] = norm8(xv[r], gv[r], rstd);
-        if (tid + r * kPreThreads < nvec) am = absmax_bits8(xv[r], am);
+        if (tid + r * THREADS < nvec) am = absmax_bits8(xv[r], am);
     }
     am = wave_max_u32(am);
     if (lane == 0) wmax[wave] = am;
     __syncthreads();
     am = wmax[0];
 #pragma unroll
-    for (int i = 1; i < kPreThreads / 64; ++i) am = max(am, wmax[i]);
+    for (int i = 1; i < THREADS / 64; ++i) am = max(am, wmax[i]);
     const float s32 = mode == 0 ? quant_scale<0>(am) : quant_scale<1>(am);
     if (tid == 0) s[row] = f32_to_bf16_rne(s32);
     uint2* qr = (uint2*)(q + (size_t)row * K);
 #pragma unroll
     for (int r = 0; r < VQ; ++r) {
-        const int idx = tid + r * kPreThreads;
+        const int idx = tid + r * THREADS;
         if (idx < nvec) qr[idx] = mode == 0 ? quant_vec8<0>(xv[r], s32) : quant_vec8<1>(xv[r], s32);
     }
 }
@@ -2441,11 +2441,15 @@ constexpr int kSoloMaxK = 8192;
 // 13824 x 2560 5.14 -> 6.07, not taken); with a norm in front only at one token up to this K (3840 x 2560
 // 3.95 -> 3.80, 13824 x 2560 5.44 -> 5.16; 2560 x 6912 with gate and residual 5.87 -> 6.12, not taken)
 constexpr int kSoloLongRowK = 4096;
-// rows from which the norm + quantizer kernel of a prompt runs a wave per row (K = 2560, a workgroup per row against that:
-// 200 rows 2.95 us against 3.44, 300 3.56 / 3.49, 512 3.75 / 3.56, 600 4.37 / 3.68, 800 4.99 / 3.96).  From 300 to 511 rows it is
-// ahead by 0.04 to 0.2 us of a launch, which a prompt pass does not show: 300 rows 2236 .. 2246 us against 2246, 384 2420 .. 2431
-// against 2414 .. 2418, 448 2519 .. 2527 against 2518; from 512 on it does: 2630 .. 2641 against 2622, 600 3141 against 3082
-constexpr int kNormRowsPerWaveMinRows = 512;
+// The norm + quantizer kernel in front of a prompt's product: a workgroup of 512 or 256 threads per row, or a wave per row.  A
+// row's time is two reductions over what holds it, and of smaller workgroups more fit a CU.  With a small product behind, 512 threads
+// / 256 / a wave, us: 320 x 512 6.65 / 6.15 / 5.8, 17 x 1024 5.5 / 5.3 / 5.2, 1024 x 1024 8.65 / 7.6 / 6.65 (always a wave); 320 x 2560 8.4 / 8.1 / 8.45,
+// 512 8.7 / 8.35 / 8.55, 672 9.55 / 8.75 / 8.8, 768 9.7 / 8.9 / 8.9, 1024 10.65 / 9.7 / 9.2, 640 x 2048 9.0 / 8.3 / 8.3 (a wave from 768 rows on); 320 x
+// 3200 9.05 / 8.85 / 9.8, 512 9.45 / 9.1 / 10.1, 2048 15.75 / 13.8 / 13.9, 512 x 4096 9.95 / 9.65 / 10.65.  512 threads / 256: 256 x 6912 10.3 / 10.45,
+// 512 12.95 / 12.85, 1024 16.3 / 15.95, 512 x 5120 11.15 / 11.05, 512 x 10240 16.4 / 16.6; with the gate 512 x 2560 9.05 / 8.7, 2048 15.35 / 13.9,
+// 320 x 6912 13.25 / 13.35, 672 15.85 / 15.9.
+constexpr int kNormRowsPerWaveAlwaysK = 1024, kNormRowsPerWaveMostK = 2560, kNormRowsPerWaveMinRows = 768;
+constexpr int kNormHalfK = 4096, kNormHalfManyRowsK = 8192, kNormHalfMinRows = 512;
 // --- prefill GEMM: tile and k-split by the number of tiles ------------------
 // up to this many 64 x 128 tiles the GEMM uses 32 x 128 tiles (M = 128: 11.4 -> 9.0 us at 3840 x 2560, 21.5 -> 16.4
 // at 2560 x 6912); beyond, 64 x 256 (level or ahead from here on: 2560 x 6912 at M = 1536 31.7 -> 29.2)
@@ -4109,38 +4113,43 @@ int bitlinear_norm_forward_bf16_seg(const uint16_t* x, const uint16_t* norm_weig
 // gate / norm / quantizer once per token row
 static int launch_norm_quant(const uint16_t* x, const uint16_t* norm_weight, float eps, int glu, int8_t* q_ws, uint16_t* s_ws, int M,
                              int K, int mode, hipStream_t stream) {
-    // very many rows, no gate, short rows: a wave per row (with the gate at K = 6912 4-7 us behind, without it 512 rows 5.1 us
-    // against 8: not taken)
-    if (M >= kNormRowsPerWaveMinRows && !glu && K <= 8 * 64 * 8) {
+    if (!glu && (K <= kNormRowsPerWaveAlwaysK || (M >= kNormRowsPerWaveMinRows && K <= kNormRowsPerWaveMostK))) {
         const int per_lane = (K / 8 + 63) / 64;
         const dim3 rgrid((M + 3) / 4, 1, 1), rblock(256, 1, 1);
 #define BITLINEAR_LAUNCH_NR(P, V) \
     BL_LAUNCH((norm_quant_rows_kernel<P, V>), rgrid, rblock, 0, stream, x, norm_weight, eps, q_ws, s_ws, M, K, mode)
 #define BITLINEAR_LAUNCH_NR_V(V) BITLINEAR_LAUNCH_NR(1, V)
         if (per_lane <= 2) { BITLINEAR_LAUNCH_NR_V(2); }
-        else if (per_lane <= 5) { BITLINEAR_LAUNCH_NR_V(5); }
-        else { BITLINEAR_LAUNCH_NR_V(8); }
+        else { BITLINEAR_LAUNCH_NR_V(5); }
 #undef BITLINEAR_LAUNCH_NR_V
 #undef BITLINEAR_LAUNCH_NR
         return launch_status();
     }
-    const dim3 grid(M, 1, 1), block(kPreThreads, 1, 1);
-    const int per_thread = (K / 8 + kPreThreads - 1) / kPreThreads;
-#define BITLINEAR_LAUNCH_PRE(P, V) \
-    BL_LAUNCH((norm_quant_kernel<P, V>), grid, block, 0, stream, x, norm_weight, eps, q_ws, s_ws, K, mode)
-#define BITLINEAR_LAUNCH_PRE_V(V)    \
-    if (glu)                         \
-        BITLINEAR_LAUNCH_PRE(2, V);  \
-    else                             \
-        BITLINEAR_LAUNCH_PRE(1, V)
-    if (per_thread <= 1) {
-        BITLINEAR_LAUNCH_PRE_V(1);
+    const bool half = K <= kNormHalfK || (!glu && K <= kNormHalfManyRowsK && M >= kNormHalfMinRows);
+    const int threads = half ? kPreThreads / 2 : kPreThreads;
+    const dim3 grid(M, 1, 1), block(threads, 1, 1);
+    const int per_thread = (K / 8 + threads - 1) / threads;
+#define BITLINEAR_LAUNCH_PRE(P, V, T) \
+    BL_LAUNCH((norm_quant_kernel<P, V, T>), grid, block, 0, stream, x, norm_weight, eps, q_ws, s_ws, K, mode)
+#define BITLINEAR_LAUNCH_PRE_V(V, T)    \
+    if (glu)                            \
+        BITLINEAR_LAUNCH_PRE(2, V, T);  \
+    else                                \
+        BITLINEAR_LAUNCH_PRE(1, V, T)
+    if (half) {
+        if (per_thread <= 1) {
+            BITLINEAR_LAUNCH_PRE_V(1, kPreThreads / 2);
+        } else if (per_thread <= 2) {
+            BITLINEAR_LAUNCH_PRE_V(2, kPreThreads / 2);
+        } else {
+            BITLINEAR_LAUNCH_PRE(1, 4, kPreThreads / 2);
+        }
     } else if (per_thread <= 2) {
-        BITLINEAR_LAUNCH_PRE_V(2);
+        BITLINEAR_LAUNCH_PRE_V(2, kPreThreads);
     } else if (per_thread <= 4) {
-        BITLINEAR_LAUNCH_PRE_V(4);
+        BITLINEAR_LAUNCH_PRE_V(4, kPreThreads);
     } else {
-        BITLINEAR_LAUNCH_PRE_V(8);
+        BITLINEAR_LAUNCH_PRE_V(8, kPreThreads);
     }
 #undef BITLINEAR_LAUNCH_PRE_V
 #undef BITLINEAR_LAUNCH_PRE

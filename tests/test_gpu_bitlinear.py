@@ -733,6 +733,30 @@ def test_norm_and_quantizer_by_a_wave_per_row_equal_a_workgroup_per_row(m, k):
     assert torch.equal(q[0], q[1]) and torch.equal(s[0].view(torch.int16), s[1].view(torch.int16))
 
 
+# a wave per row (768 rows on, up to 2560 values), 256 threads (up to 4096; from 512 rows on up to 8192) and 512 behind
+@pytest.mark.parametrize("m,k", [(767, 2560), (768, 2560), (769, 1152), (768, 2688), (511, 4224), (512, 8192), (512, 8320)])
+def test_norm_and_quantizer_by_256_threads_per_row_equal_the_others(m, k):
+    test_norm_and_quantizer_by_a_wave_per_row_equal_a_workgroup_per_row(m, k)
+
+
+@pytest.mark.parametrize("k", [1024, 1152, 2048, 2176, 4096, 4224])
+@pytest.mark.parametrize("glu", [0, 1])
+def test_norm_and_quantizer_of_a_prompt_at_the_edges_of_their_workgroups(k, glu):
+    m, n, lib = 40, 32, _lib.load_library()
+    w, _ = _rand_case(n, k, 1, seed=k)
+    rng = np.random.default_rng(k + glu)
+    xb = o.f32_to_bf16_bits(rng.standard_normal((m, k << glu)).astype(np.float32))
+    g_bits = o.f32_to_bf16_bits(np.linspace(0.5, 1.5, k).astype(np.float32))
+    ws_bits = o.f32_to_bf16_bits(np.array([0.0161, 0.0247, 0.0093, 0.0], dtype=np.float32))
+    x, gd, pk, wsd = dev_bf16(xb), dev_bf16(g_bits), _packed_dev(w), dev_bf16(ws_bits)
+    out, s_ws = (torch.empty(*shape, dtype=torch.bfloat16, device="cuda") for shape in ((m, n), (m,)))
+    q_ws = torch.empty(m, k, dtype=torch.int8, device="cuda")
+    assert lib.bitlinear_norm_forward_bf16(x.data_ptr(), gd.data_ptr(), 1e-5, glu, pk.data_ptr(), wsd.data_ptr(), None, out.data_ptr(), q_ws.data_ptr(),
+                                           s_ws.data_ptr(), m, n, k, 0, torch.cuda.current_stream().cuda_stream) == 0
+    want = o.norm_bitlinear(o.squared_relu_glu_bf16(xb) if glu else xb, g_bits, 1e-5, w, ws_bits)
+    _assert_bits_equal(host_bits(out), want, "output")
+
+
 @pytest.mark.parametrize("tile", [0, 1, 2, 4, 5, 6, 7, 8, 9, 10, 11, 12])
 @pytest.mark.parametrize("m,n,k", [(17, 16, 128), (1500, 16, 128), (40, 4112, 256), (700, 1296, 256), (1100, 2576, 128)])
 def test_prefill_gemm_deals_out_every_tile(m, n, k, tile):
