@@ -1187,7 +1187,11 @@ void gemm_i2_prefill_mix_kernel(
 constexpr int kQuantThreads = 256;
 constexpr int kQuantMaxThreads = 1024;
 constexpr int kQuantRegVecs = 4;  // 16-byte vectors (8 bf16) kept in registers per thread
-constexpr int kQuantRowsMin = 2;   // from this many rows on the quantizer runs a wave per row (rows of up to 4096 values)
+// From this many rows on the quantizer runs a wave per row, rows of more than kQuantRowsMostK values (up to 4096) from the latter
+// on: a wave takes eight requests for one, and what that costs is hidden only where all wave slots are taken (a workgroup per row
+// against that, K = 3200: 8 rows 2.42 / 2.38 us, 100 2.54 / 2.65, 333 2.65 / 2.74, 512 2.74 / 2.80, 700 3.01 / 2.94, 1024 3.63 / 3.13; K = 4096: 2 2.21 / 2.45,
+// 333 2.70 / 2.84, 512 2.80 / 2.88, 700 level; K = 2560: 2 2.18 / 2.05, 333 2.59 / 2.45, 1024 3.15 / 2.71)
+constexpr int kQuantRowsMin = 2, kQuantRowsMostK = 2560, kQuantLongRowsMin = 640;
 
 template <int MODE>
 __global__ __launch_bounds__(kQuantMaxThreads) void quant_absmax_kernel(const uint16_t* __restrict__ x,
@@ -3948,10 +3952,9 @@ static int quant_absmax_impl(const uint16_t* x, int8_t* q, uint16_t* s, int32_t*
     if (mode != 0 && mode != 1) return set_status(BITLINEAR_ERR_ARG);
     // 256 threads keep rows of up to 8192 elements in registers between the two passes; longer rows
     // get more threads (a second pass that re-reads the row costs a chain of dependent loads)
-    // two rows or more: a wave per row while a lane holds at most 8 vectors of the row (measured at K = 2560: 2.41 -> 2.18 us
-    // at 8 rows, 2.45 -> 2.26 at 16, 4.49 -> 3.66 at 64, 5.79 -> 5.39 at 2048, 14.7 -> 12.4 at 8192; longer rows keep the
-    // kernel below)
-    if (M >= kQuantRowsMin && K <= 8 * 64 * 8) {
+    // a wave per row while a lane holds at most 5 vectors of the row, 8 where there are many (K = 2560: 2.45 -> 2.26 us at 16 rows,
+    // 4.49 -> 3.66 at 64, 14.7 -> 12.4 at 8192)
+    if (K <= kQuantRowsMostK ? M >= kQuantRowsMin : M >= kQuantLongRowsMin && K <= 8 * 64 * 8) {
         const int per_lane = (K / 8 + 63) / 64;
         const dim3 grid((M + 3) / 4, 1, 1), block(256, 1, 1);
 #define BITLINEAR_LAUNCH_QR(MODE_, V_) \

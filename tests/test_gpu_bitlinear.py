@@ -296,6 +296,11 @@ def test_quantizer_bit_exact(mode, m, k):
     assert np.array_equal(q.cpu().numpy(), wq)
 
 
+@pytest.mark.parametrize("m,k", [(1, 2560), (2, 2560), (2, 2568), (639, 2568), (640, 2568), (640, 4096), (640, 4104)])
+def test_quantizer_at_the_edges_of_a_wave_per_row(m, k):
+    test_quantizer_bit_exact(0, m, k)
+
+
 def test_quantizer_matches_committed_torch_vectors():
     import os
 
