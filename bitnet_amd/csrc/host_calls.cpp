@@ -1,11 +1,12 @@
 // CPython entry points of the three calls a program makes per BitLinear -- BitLinearKernel.forward,
 // bitnet_int8xint2_linear and quant_input (gpu/model.py:21-75 of the reference) -- and of the weight
-// layout converters (gpu/pack_weight.py), between torch tensors and the C ABI of libbitlinear_hip.so.
+// layout converters (gpu/pack_weight.py), between torch tensors and the C ABI of libbitlinear_hip.so; and the wait
+// for a decode step's tokens (await_words).
 //
 // What bounds a small call is the host: the kernels of a one-token 2560 x 2560 forward take 3.5 us,
 // and issuing them from Python (three torch.empty, torch.cuda.current_stream, the argument checks
 // and the conversion of twelve ctypes arguments) took 15.4 us per call, back to back; from here it
-// takes 5.5 (8 tokens of 6912 -> 2560: 18.1 -> 8.8, two kernels).  The checks read the tensors' C++
+// takes 5.5 (8 tokens of 6912 -> 2560: 18.1 -> 8.8 as two kernels, 6.9 as one).  The checks read the tensors' C++
 // objects, the workspaces are one caching-allocator block, the output is allocated without the
 // operator dispatcher, and the stream is read from torch's own thread-local state.  The functions
 // of the library are taken by address (bind), so this file links to torch only and serves
