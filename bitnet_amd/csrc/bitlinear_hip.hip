@@ -1961,8 +1961,10 @@ __global__ __launch_bounds__(kMaxWaves * 64) void bitlinear_solo_kernel(
 // the host issues the two launches in 7.5 us, their kernels take 5.7 in a chain).  So workgroup r quantizes row r before its share of
 // the product, with all its waves, and publishes it: the int8 values by write-through stores, and when those are acknowledged a
 // flag word that holds the row's scale and the launch's tag.  Every workgroup's first wave polls the flags of its rows past the
-// caches; the rows themselves are then ordinary loads, which the XCD's L2 serves from the second workgroup on: nobody has read
-// their lines in this launch before they were published.  Weights are requested behind the publishing (in front of it
+// caches; the rows themselves are then ordinary loads, which the XCD's L2 serves from the second workgroup on.  Nothing drops
+// what an L2 holds behind the poll, so no line of theirs may have been read in this launch before they were published: the
+// launch reads scales, weights and x in front of the poll, so the rows must be whole lines that hold nothing else
+// (hand_rows_alone; other workspaces take the two launches).  Weights are requested behind the publishing (in front of it
 // the acknowledgement waits for them too: 8 x 2560 x 6912 7.6 us instead of 7.0).
 //
 // The flag words lie in the library's image, one set per launch in turn, and a set's tag is another each time (the
@@ -1974,6 +1976,9 @@ __global__ __launch_bounds__(kMaxWaves * 64) void bitlinear_solo_kernel(
 constexpr int kHandSets = 256, kHandRows = 16;
 static __device__ unsigned long long hand_flags[kHandSets][kHandRows];
 constexpr int kHandPolls = 512;  // some hundreds of microseconds; a wait is one or two
+constexpr int kL2Line = 128;     // bytes
+// whether M rows of K int8 values at q share no L2 line with anything else
+bool hand_rows_alone(const int8_t* q, int M, int K) { return (uintptr_t)q % kL2Line == 0 && (long long)M * K % kL2Line == 0; }
 
 struct HandedRows {
     static constexpr bool kGiven = false;
@@ -4017,7 +4022,7 @@ static int forward_impl(const uint16_t* x, const int8_t* packed, uint16_t* outpu
     // larger blocks: the quantizer once, in the product's launch or in a kernel of its own, then the product
     if (!q_ws || !s_ws) return set_status(BITLINEAR_ERR_NULL);
     if (mode == 0 && t_tune.path == 0 && t_tune.hand != 2 && !t_plan.active && M <= kHandRows && (long long)M * K <= kHandMaxElems &&
-        (t_tune.hand == 1 || N / 16 < kHandMostBlocks) && slot_rule(sm, N).ok) {
+        (t_tune.hand == 1 || N / 16 < kHandMostBlocks) && hand_rows_alone(q_ws, M, K) && slot_rule(sm, N).ok) {
         const ProdPlan hp = plan_prod_solo(M, N, K);
         if (hp.ok && K <= 512 * hp.s && stream_runs((hipStream_t)stream))
             return set_status(launch_handed(x, packed, output0, acc_out, ws, sm, q_ws, s_ws, M, N, K, hp, (hipStream_t)stream));

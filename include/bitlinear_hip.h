@@ -410,7 +410,9 @@ int bitlinear_plan_name(int entry, int M, int N, int K, char* buf, int buflen);
  *             stream that is not being captured) in one launch whose first
  *             workgroups quantize the rows and hand them on: a = 0 built-in
  *             choice (where the quantizer would be a launch of its own, M * K <=
- *             57344, N < 6912), 1 for any N, 2 never; b = 0 the built-in bound of
+ *             57344, N < 6912), 1 for any N, 2 never; not where q_ws is not 128-byte
+ *             aligned or M * K no multiple of 128 (the rows would share a cache line
+ *             with what lies beside them); b = 0 the built-in bound of
  *             a workgroup's polls before it quantizes the rows itself, else b - 1
  *             polls (b <= 512).  Applies with kernel 0 only; kernel 0 resets it.
  */

@@ -1445,6 +1445,38 @@ def test_forward_with_rows_handed_on_inside_the_launch(m, n, k, polls):
         lib.bitlinear_set_tuning(0, 0, 0, 0)
 
 
+@pytest.mark.parametrize("m,k,at,handed", [(9, 2560, 128, True), (9, 2560, 16, False), (9, 2560, 64, False), (9, 2112, 128, False),
+                                           (16, 2112, 128, True), (5, 6912, 112, False), (7, 3904, 256, False)])
+def test_rows_are_handed_on_only_where_no_other_operand_shares_their_cache_lines(m, k, at, handed):
+    """Weight scales directly in front of the quantized rows and the activations directly behind them, in one block: a line
+    that holds both is read before the rows are there, so those calls quantize in a launch of their own."""
+    n, lib = 1040, _lib.load_library()
+    pk = _packed_dev(np.random.default_rng(m + k).integers(-1, 2, size=(n, k), dtype=np.int8))
+    block = torch.zeros(at + 3 * m * k + 256, dtype=torch.int8, device="cuda")
+    assert block.data_ptr() % 256 == 0
+    ws = block[at - 8 : at].view(torch.bfloat16)
+    behind = at + (m * k + 15) // 16 * 16
+    q, x = block[at : at + m * k].view(m, k), block[behind : behind + 2 * m * k].view(torch.bfloat16).view(m, k)
+    ws.copy_(torch.tensor([0.0161, 0.0247, 0.0093, 0.0]))
+    s = torch.zeros(m, dtype=torch.bfloat16, device="cuda")
+    out = [torch.zeros(m, n, dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+    st = torch.cuda.current_stream().cuda_stream
+    try:
+        for turn in range(3):
+            x.copy_(torch.randn(m, k, device="cuda") * 10.0**turn)
+            rows = []
+            for i in range(2):
+                assert lib.bitlinear_set_tuning(13, 2 - i, 0, 0) == 0
+                assert lib.bitlinear_forward_bf16(x.data_ptr(), pk.data_ptr(), out[i].data_ptr(), ws.data_ptr(), q.data_ptr(), s.data_ptr(),
+                                                  m, n, k, 0, st) == 0
+                assert (bitlinear.last_kernel() == "bitlinear_handed_kernel") == (handed and i == 1)
+                rows.append((q.clone(), s.clone()))
+            torch.cuda.synchronize()
+            assert all(torch.equal(a, b) for a, b in zip(*rows)) and torch.equal(out[0], out[1])
+    finally:
+        lib.bitlinear_set_tuning(0, 0, 0, 0)
+
+
 def test_forward_with_handed_rows_on_two_streams_and_in_a_graph():
     """Launches of two streams overlap, more of them than there are sets of flag words; a captured call is replayed with
     other rows."""
