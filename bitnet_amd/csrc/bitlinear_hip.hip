@@ -2519,6 +2519,7 @@ using namespace dispatch;
 // the kernel with its template arguments, grid, block and dynamic LDS -- instead of issued.  Nothing touches a device.
 struct PlanLog {
     bool active = false;
+    bool captured = true;  // what is planned is a call that is recorded in a graph
     std::string text;
 };
 thread_local PlanLog t_plan;
@@ -3038,6 +3039,7 @@ int launch_prod_solo(const int8_t* act, const int8_t* packed, uint16_t* out, int
 
 // Whether a launch on this stream runs (and is not recorded)
 bool stream_runs(hipStream_t stream) {
+    if (t_plan.active) return !t_plan.captured;
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &status) == hipSuccess) return status == hipStreamCaptureStatusNone;
     (void)hipGetLastError();
@@ -4021,7 +4023,7 @@ static int forward_impl(const uint16_t* x, const int8_t* packed, uint16_t* outpu
                                        (hipStream_t)stream));
     // larger blocks: the quantizer once, in the product's launch or in a kernel of its own, then the product
     if (!q_ws || !s_ws) return set_status(BITLINEAR_ERR_NULL);
-    if (mode == 0 && t_tune.path == 0 && t_tune.hand != 2 && !t_plan.active && M <= kHandRows && (long long)M * K <= kHandMaxElems &&
+    if (mode == 0 && t_tune.path == 0 && t_tune.hand != 2 && M <= kHandRows && (long long)M * K <= kHandMaxElems &&
         (t_tune.hand == 1 || N / 16 < kHandMostBlocks) && hand_rows_alone(q_ws, M, K) && slot_rule(sm, N).ok) {
         const ProdPlan hp = plan_prod_solo(M, N, K);
         if (hp.ok && K <= 512 * hp.s && stream_runs((hipStream_t)stream))
@@ -4266,14 +4268,18 @@ int bitlinear_norm_rope_forward_bf16(const uint16_t* x, const uint16_t* norm_wei
                           mode, stream, epi);
 }
 
+constexpr int kPlanDirect = 16;  // added to an entry: the call outside of a capture
 int bitlinear_plan_name(int entry, int M, int N, int K, char* buf, int buflen) {
     if (!buf || buflen < 1) return set_status(BITLINEAR_ERR_NULL);
     buf[0] = 0;
+    const bool direct = entry >= kPlanDirect;
+    if (direct) entry -= kPlanDirect;
     if (entry < 0 || entry > 4) return set_status(BITLINEAR_ERR_ARG);
     // operands of a planning call are never dereferenced, on the host or anywhere: any aligned address does
     uint16_t* const h = reinterpret_cast<uint16_t*>((uintptr_t)0x100000);
     int8_t* const b = reinterpret_cast<int8_t*>((uintptr_t)0x100000);
     t_plan.active = true;
+    t_plan.captured = !direct;
     t_plan.text.clear();
     int st = BITLINEAR_OK;
     switch (entry) {

@@ -331,8 +331,9 @@ int bitlinear_norm_rope_forward_bf16(const uint16_t* x, const uint16_t* norm_wei
  * of the call in launch order and joined by " + ", the kernel with its template
  * arguments, the grid, the workgroup size and the dynamic LDS bytes, e.g.
  * "bitlinear_solo_kernel<5, 1, 1, true, 0, false, 1> grid=(160,1,1) block=512
- * lds=0".  Entry 1 stands for a call that is recorded in a graph: of one that
- * is not, the quantizer may be part of the product's launch (kernel 13 below).
+ * lds=0".  Entries 0 .. 4 stand for a call that is recorded in a graph, 16 .. 20
+ * for the same calls made directly: there the quantizer of entry 17 may be part of
+ * the product's launch (kernel 13 below; for workspaces of whole cache lines).
  * Returns the status the call itself would return for the shape.
  * The current bitlinear_set_tuning overrides apply.  No counterpart in the
  * reference, whose dispatch is a table of ten shapes (bitnet_kernels.cu:4-33).

@@ -41,6 +41,21 @@ def test_plan_rows_say_what_the_design_says():
     assert p(0, 1, 20480, 3200).startswith("bitlinear_fused_kernel<")
 
 
+def test_a_direct_forward_call_quantizes_in_the_products_launch_where_a_recorded_one_does_not():
+    """Entries from 16 on stand for calls outside of a capture; only the forward call of 5 to 16 tokens is another one there."""
+    p = _lib.plan_name
+    for m, n, k, shape in ((16, 2560, 2560, "<5, 1> grid=(160,1,1) block=512"), (8, 2560, 6912, "<7, 1> grid=(160,1,1) block=1024")):
+        assert p(17, m, n, k) == f"bitlinear_handed_kernel{shape} lds=0"
+        quantizer, product = p(1, m, n, k).split(" + ")
+        assert quantizer.startswith("quant_absmax") and product == f"gemv_i2_solo_kernel{shape[:5]}, false>{shape[6:]} lds=0"
+    # one token, rows that every workgroup quantizes, many columns, rows that end within a cache line, more than sixteen tokens
+    for m, n, k in ((1, 2560, 2560), (8, 3840, 2560), (16, 55296, 5120), (9, 2560, 2112), (17, 2560, 2560)):
+        assert p(17, m, n, k) == p(1, m, n, k)
+    for entry in (0, 2, 3, 4):
+        for m in (1, 8, 16, 512):
+            assert p(16 + entry, m, 2560, 6912) == p(entry, m, 2560, 6912)
+
+
 def test_the_gate_is_in_the_epilogue_only_where_that_is_ahead():
     """Against what the separate product would take: the launch with two tile sizes (ahead with 256-k chunks and at most one small
     tile per CU), the split-K kernel (ahead), the kernel with the epilogues (behind)."""
@@ -74,5 +89,6 @@ def test_plan_name_argument_checks():
     lib = _lib.load_library()
     buf = ctypes.create_string_buffer(64)
     assert lib.bitlinear_plan_name(5, 1, 2560, 2560, buf, 64) == 4 and lib.bitlinear_plan_name(0, 1, 2560, 2560, None, 64) == 2
+    assert [lib.bitlinear_plan_name(e, 1, 2560, 2560, buf, 64) for e in (-1, 15, 16, 20, 21)] == [4, 4, 0, 0, 4]
     assert lib.bitlinear_plan_name(0, 1, 100, 2560, buf, 64) == 1 and buf.value == b""  # a shape the library refuses
     assert lib.bitlinear_plan_name(0, 1, 2560, 2560, buf, 8) == 0 and len(buf.value) == 7  # truncated, terminated
