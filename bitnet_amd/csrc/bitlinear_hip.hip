@@ -2505,13 +2505,18 @@ constexpr int kRingMinK = 384, kRingMinK64x256 = 1024;
 constexpr int kRingMinK64x96 = 4096, kRingMinK64x192 = 1664;
 // ... and with rope or gate in the epilogue from the K on that their entry points state
 constexpr int kRingEpilogueMinK = 640;
-// the forward call's quantizer in the product's launch (HandedRows) while the rows, which every workgroup reads behind the hand-over,
-// are few, and up to this many row blocks.  Issued one by one, two launches -> one: 9 x 3840 x 2560 7.3 -> 5.8 us, 16 x 3840 x 2560 7.3
-// -> 6.6, 5 x 2560 x 6912 7.5 -> 6.2, 8 x 2560 x 6912 7.5 .. 8.9 -> 7.1; 16 x 2560 x 6912 8.5 -> 8.4, 16 x 13824 x 2560 7.6 -> 7.6, 16 x 20480 x
-// 3200 11.2 -> 12.5.  Behind a full queue, where the host's part does not count, 5.6 -> 5.8, 6.1 -> 6.6, 6.85 -> 6.3, 7.5 -> 7.1.  The
-// same in front of the ring kernel's 32 x 64 tiles was built and left out: 101 x 3840 x 2560 7.8 -> 8.3, 64 x 2560 x 6912 10.65 -> 10.4.
-constexpr long long kHandMaxElems = 57344;
-constexpr int kHandMostBlocks = 432;
+// The forward call's quantizer in the product's launch (HandedRows) up to this many outputs.  Issued one by one a call is bound by its
+// launches (two: 7.3 .. 8.9 us of the host, one: 5.0 .. 6.1), behind a full queue by what the GPU does, and there the hand-over
+// is longer than the kernel boundary that it replaces when the rows are many and short, and shorter when they are few or long.
+// Two launches -> one, us, one by one / behind a full queue: 9 x 2560 x 2560 7.3 -> 5.7 / 5.5 -> 5.7, 16 x 2560 x 2560 7.2 -> 6.3 / 6.0 -> 6.4,
+// 16 x 3840 x 2560 8.1 -> 6.6 / 6.0 -> 6.45, 12 x 4800 x 3200 8.9 -> 7.75 / 7.15 -> 7.55, 16 x 4096 x 4096 8.85 -> 7.4 / 6.95 -> 7.25,
+// 8 x 2560 x 6912 8.85 -> 7.4 / 7.4 -> 7.15, 16 x 2560 x 6912 9.2 -> 8.65 / 8.55 -> 8.7, 16 x 2560 x 8192 9.8 -> 9.1 / 9.1 -> 9.15, 8 x 8192 x 4096
+// 7.55 -> 6.4 / 6.6 -> 6.55, 7 x 6912 x 6912 7.6 -> 6.95 / 7.6 -> 7.15.  Taken while the first gains about twice what the second loses, or more; over 150
+// shapes of 5 to 16 rows that is so up to here but where both are below 0.1 us (12 x 5120 x 6912 10.25 -> 10.25 / 10.4 -> 10.45).  Behind it the
+// gain shrinks and the loss grows: 16 x 4800 x 3200 8.9 -> 8.35 / 7.7 -> 8.25, 16 x 6400 x 2560 8.3 -> 7.75 / 7.0 -> 7.65, 16 x 6832 x 3456
+// 7.95 -> 8.4 / 7.85 -> 8.6, 14 x 4928 x 6208 8.8 -> 8.85 / 8.85 -> 9.05, 12 x 8192 x 8192 8.9 -> 8.9 / 9.05 -> 9.2.
+// The same in front of the ring kernel's 32 x 64 tiles was built and left out: 101 x 3840 x 2560 7.8 -> 8.3, 64 x 2560 x 6912 10.65 -> 10.4.
+constexpr long long kHandMostOutputs = 65536;
 }  // namespace dispatch
 using namespace dispatch;
 
@@ -4023,8 +4028,8 @@ static int forward_impl(const uint16_t* x, const int8_t* packed, uint16_t* outpu
                                        (hipStream_t)stream));
     // larger blocks: the quantizer once, in the product's launch or in a kernel of its own, then the product
     if (!q_ws || !s_ws) return set_status(BITLINEAR_ERR_NULL);
-    if (mode == 0 && t_tune.path == 0 && t_tune.hand != 2 && M <= kHandRows && (long long)M * K <= kHandMaxElems &&
-        (t_tune.hand == 1 || N / 16 < kHandMostBlocks) && hand_rows_alone(q_ws, M, K) && slot_rule(sm, N).ok) {
+    if (mode == 0 && t_tune.path == 0 && t_tune.hand != 2 && M <= kHandRows &&
+        (t_tune.hand == 1 || (long long)M * N <= kHandMostOutputs) && hand_rows_alone(q_ws, M, K) && slot_rule(sm, N).ok) {
         const ProdPlan hp = plan_prod_solo(M, N, K);
         if (hp.ok && K <= 512 * hp.s && stream_runs((hipStream_t)stream))
             return set_status(launch_handed(x, packed, output0, acc_out, ws, sm, q_ws, s_ws, M, N, K, hp, (hipStream_t)stream));

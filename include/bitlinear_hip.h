@@ -410,8 +410,8 @@ int bitlinear_plan_name(int entry, int M, int N, int K, char* buf, int buflen);
  *   kernel 13: bitlinear_forward_bf16 (mode 0, M <= 16, with workspaces, on a
  *             stream that is not being captured) in one launch whose first
  *             workgroups quantize the rows and hand them on: a = 0 built-in
- *             choice (where the quantizer would be a launch of its own, M * K <=
- *             57344, N < 6912), 1 for any N, 2 never; not where q_ws is not 128-byte
+ *             choice (where the quantizer would be a launch of its own and M * N <=
+ *             65536), 1 for any N, 2 never; not where q_ws is not 128-byte
  *             aligned or M * K no multiple of 128 (the rows would share a cache line
  *             with what lies beside them); b = 0 the built-in bound of
  *             a workgroup's polls before it quantizes the rows itself, else b - 1

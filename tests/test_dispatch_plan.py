@@ -51,6 +51,10 @@ def test_a_direct_forward_call_quantizes_in_the_products_launch_where_a_recorded
     # one token, rows that every workgroup quantizes, many columns, rows that end within a cache line, more than sixteen tokens
     for m, n, k in ((1, 2560, 2560), (8, 3840, 2560), (16, 55296, 5120), (9, 2560, 2112), (17, 2560, 2560)):
         assert p(17, m, n, k) == p(1, m, n, k)
+    # the line, 65536 outputs, at one and at several row blocks a wave, and the longest rows
+    for m, n, k in ((16, 4096, 2560), (16, 4096, 8192), (15, 4368, 3200), (8, 8192, 4096), (5, 13104, 3328)):
+        wider = n + 16 * -(-(65537 - m * n) // (16 * m))
+        assert p(17, m, n, k).startswith("bitlinear_handed_kernel<") and p(17, m, wider, k) == p(1, m, wider, k)
     for entry in (0, 2, 3, 4):
         for m in (1, 8, 16, 512):
             assert p(16 + entry, m, 2560, 6912) == p(entry, m, 2560, 6912)

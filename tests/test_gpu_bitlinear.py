@@ -1445,6 +1445,11 @@ def test_forward_with_rows_handed_on_inside_the_launch(m, n, k, polls):
         lib.bitlinear_set_tuning(0, 0, 0, 0)
 
 
+@pytest.mark.parametrize("m,n,k", [(16, 1040, 8192), (16, 4096, 6912), (5, 13104, 3328), (8, 8192, 4096)])
+def test_forward_with_the_longest_and_the_widest_products_rows_handed_on(m, n, k):
+    test_forward_with_rows_handed_on_inside_the_launch(m, n, k, 0)
+
+
 @pytest.mark.parametrize("m,k,at,handed", [(9, 2560, 128, True), (9, 2560, 16, False), (9, 2560, 64, False), (9, 2112, 128, False),
                                            (16, 2112, 128, True), (5, 6912, 112, False), (7, 3904, 256, False)])
 def test_rows_are_handed_on_only_where_no_other_operand_shares_their_cache_lines(m, k, at, handed):
