@@ -790,11 +790,19 @@ extern "C" int bitnet_attn_prefill(const uint16_t* q, const uint16_t* cache_k, c
     if (split) {
         // more LDS than the 64 KiB that a kernel gets without asking (a host-side attribute, set once per device)
         static bitnet_host::OncePerDevice raised;
-        const hipError_t e = raised.run([] {
-            return hipFuncSetAttribute((const void*)attn_prefill_split_kernel<4, kApAhead>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                       ApRing<4, kApAhead>::LDS);
+        const hipError_t err = raised.run([] {
+            hipError_t e = hipSuccess;
+#define BITNET_AP_LDS(G)                                                                                                                \
+    if (e == hipSuccess)                                                                                                                \
+    e = hipFuncSetAttribute((const void*)attn_prefill_split_kernel<G, kApAhead>, hipFuncAttributeMaxDynamicSharedMemorySize, \
+                            ApRing<G, kApAhead>::LDS)
+            BITNET_AP_LDS(1);
+            BITNET_AP_LDS(2);
+            BITNET_AP_LDS(4);
+#undef BITNET_AP_LDS
+            return e;
         });
-        if (e != hipSuccess) return 3;
+        if (err != hipSuccess) return 3;
     }
 #define BITNET_AP_SPLIT(G)                                                                                                        \
     hipLaunchKernelGGL((attn_prefill_split_kernel<G, kApAhead>), dim3(n_heads / gs, B, here), dim3(ApRing<G, kApAhead>::THREADS),  \
