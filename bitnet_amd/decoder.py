@@ -769,6 +769,7 @@ class Generator:
         # look at it, where two kernels, a copy and their launches left the GPU idle for some 50 us a step
         self.next_tok = torch.zeros(batch, dtype=torch.int64, device="cpu" if self.lm_head else dev, pin_memory=self.lm_head)
         self._await = self.lm_head  # whether the host may wait for the tokens themselves
+        self._late = False  # such a wait of the running call has run out
         self._logits: Optional[torch.Tensor] = None
         self._sampler: Optional[TopPSampler] = None
         # generated tokens of a decode() call, written from inside the step so that a graph replay is the whole step
@@ -835,17 +836,20 @@ class Generator:
     def _expect(self) -> bool:
         """Marks the host's tokens as not written, in front of a step whose tokens the host looks at.  Every earlier step must
         have been waited for: one that is still under way would write them again."""
-        if self._await:
+        if self._await and not self._late:
             self.next_tok.fill_(self.kUnset)
-        return self._await
+            return True
+        return False
 
     def _ended(self, eos_id: int, expected: bool) -> bool:
         """Whether the step just issued produced eos_id for any sequence (waits for it).  expected: _expect() was called in
         front of it, so that its tokens themselves can be waited for; the stream otherwise."""
         if not expected or not _lib.host_calls().await_words(self.next_tok, self.kUnset, self.kAwaitUs):
             torch.cuda.current_stream().synchronize()
-            if expected:
-                self._await = False  # (steps that take longer, or writes to host memory that only a wait makes visible)
+            # Steps that take longer, writes to host memory that only a wait makes visible, or one step behind other work: the
+            # rest of the call waits for the stream, the next call tries again (a wait that runs out costs what is
+            # left of it behind the step, once a call)
+            self._late = self._late or expected
         return bool((self.next_tok == eos_id).any())
 
     def _check(self) -> None:
@@ -954,6 +958,7 @@ class Generator:
             self.tok.copy_(first.view(-1, 1))
             self._set_positions(start_pos)
         self.step_idx.zero_()
+        self._late = False
         taken = 0
         for i in range(steps):
             expected = eos_id is not None and i > 0 and self._expect()  # (behind the first step nothing older is under way)
@@ -1053,6 +1058,7 @@ class Generator:
                     self._logits = torch.empty(self.batch, vocab, dtype=torch.float32, device=self.tok.device)
                 if self.lm_head and self.use_graph and self._logits_graph is None:
                     self._logits_graph = self._capture(self._logits_step)
+                self._late = False
                 taken = 0
                 for _ in range(gen_length - 1):
                     expected = eos_id is not None and taken > 0 and self._expect()

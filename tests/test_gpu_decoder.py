@@ -1322,6 +1322,27 @@ def test_steps_awaited_by_their_tokens_end_where_steps_awaited_by_the_stream_do(
         assert max(len(a) for a in got) <= steps + 1
 
 
+@pytest.mark.parametrize("sample", [False, True])
+def test_a_late_step_costs_the_call_it_is_in_its_waits_for_tokens_and_no_later_call(sample, monkeypatch):
+    model = _build(BIG_HEADS, seed=16)
+    gen = decoder.Generator(model, batch=1, max_seq=64)
+    calls, late, host = [], [], _lib.host_calls()
+    real = host.await_words
+    monkeypatch.setattr(host, "await_words", lambda *args: calls.append(1) or (real(*args) and len(calls) not in late))
+
+    def answer():
+        calls.clear()
+        rng = torch.Generator(device="cuda").manual_seed(3)
+        return gen.generate_all([[5, 9, 2]], 10, use_sampling=sample, eos_id=10**6, rng=rng), len(calls)
+
+    want = answer()
+    assert want[1] == 8  # every step of nine but the first
+    late.append(3)
+    assert answer() == (want[0], 3)
+    late.clear()
+    assert answer() == want
+
+
 def test_generate_all_sampling_is_reproducible_and_greedy_for_a_tiny_nucleus():
     model = _build(BIG_HEADS, seed=7)
     g = torch.Generator().manual_seed(5)
