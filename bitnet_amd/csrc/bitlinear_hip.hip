@@ -2456,7 +2456,9 @@ constexpr int kSoloLongRowK = 4096;
 // 512 8.7 / 8.35 / 8.55, 672 9.55 / 8.75 / 8.8, 768 9.7 / 8.9 / 8.9, 1024 10.65 / 9.7 / 9.2, 640 x 2048 9.0 / 8.3 / 8.3 (a wave from 768 rows on); 320 x
 // 3200 9.05 / 8.85 / 9.8, 512 9.45 / 9.1 / 10.1, 2048 15.75 / 13.8 / 13.9, 512 x 4096 9.95 / 9.65 / 10.65.  512 threads / 256: 256 x 6912 10.3 / 10.45,
 // 512 12.95 / 12.85, 1024 16.3 / 15.95, 512 x 5120 11.15 / 11.05, 512 x 10240 16.4 / 16.6; with the gate 512 x 2560 9.05 / 8.7, 2048 15.35 / 13.9,
-// 320 x 6912 13.25 / 13.35, 672 15.85 / 15.9.
+// 320 x 6912 13.25 / 13.35, 672 15.85 / 15.9.  Behind 4096 values, without the gate, the two are within 0.15 us of each other at 300, 340, 384, 448
+// and 512 rows (4224, 5120, 6144, 6912 and 8192 values: no line is to be seen there), at 640 256 threads are ahead by 0.05 to 0.3, at
+// 32 to 256 behind by up to 0.13.
 constexpr int kNormRowsPerWaveAlwaysK = 1024, kNormRowsPerWaveMostK = 2560, kNormRowsPerWaveMinRows = 768;
 constexpr int kNormHalfK = 4096, kNormHalfManyRowsK = 8192, kNormHalfMinRows = 512;
 // --- prefill GEMM: tile and k-split by the number of tiles ------------------

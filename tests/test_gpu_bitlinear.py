@@ -715,33 +715,36 @@ def test_prefill_gemm_acc_bit_exact(m, n, k, tile):
     assert np.array_equal(acc.cpu().numpy(), o.acc_int32(a, w))
 
 
-@pytest.mark.parametrize("m,k", [(512, 128), (515, 2560), (514, 4096), (513, 4224)])
-def test_norm_and_quantizer_by_a_wave_per_row_equal_a_workgroup_per_row(m, k):
-    """From 512 rows on (up to 4096 values) the prompt's norm and quantizer take a wave per row: rows and scales equal those
-    of calls of fewer rows, of zeros and of infinities too."""
+# a wave per row (up to 1024 values always, up to 2560 from 768 rows on), 256 threads (up to 4096 values, up to 8192 from 512
+# rows on) and 512, on both sides of each line; the last workgroup of four rows full, with one and with three
+WAVE, HALF, FULL = "norm_quant_rows_kernel<1, ", "kPreThreads / 2>", "kPreThreads>"
+
+
+@pytest.mark.parametrize("m,k,kernel", [(18, 128, WAVE), (512, 128, WAVE), (515, 1024, WAVE), (17, 1152, HALF), (515, 2560, HALF), (767, 2560, HALF),
+                                        (768, 2560, WAVE), (769, 1152, WAVE), (768, 2688, HALF), (514, 4096, HALF), (511, 4224, FULL),
+                                        (512, 4224, HALF), (513, 8192, HALF), (512, 8320, FULL)])
+def test_norm_and_quantizer_of_a_prompt_at_the_lines_between_its_kernels(m, k, kernel):
+    """Quantized rows and scales are the oracle's, of zeros too; of a row with an infinity, whose norm holds a NaN and zeros,
+    they are the quantizer call's of the oracle's norm."""
     n, lib = 32, _lib.load_library()
+    assert kernel in _lib.plan_name(2, m, n, k).split(" + ")[0]
     w, _ = _rand_case(n, k, 1, seed=k)
-    g = torch.Generator(device="cuda").manual_seed(m)
-    x = torch.randn(m, k, generator=g, device="cuda").to(torch.bfloat16)
-    x[3], x[5, 7] = 0.0, float("inf")
-    norm_w = (torch.rand(k, generator=g, device="cuda") + 0.5).to(torch.bfloat16)
-    pk, ws = _packed_dev(w), torch.full((4,), 0.02, device="cuda").to(torch.bfloat16)
-    q, s = torch.zeros(2, m, k, dtype=torch.int8, device="cuda"), torch.zeros(2, m, dtype=torch.bfloat16, device="cuda")
+    rng = np.random.default_rng(m)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[3], x[5, 7], x[m - 1] = 0.0, np.inf, 30.0 * x[m - 1]
+    xb, gb = o.f32_to_bf16_bits(x), o.f32_to_bf16_bits(rng.uniform(0.5, 1.5, k).astype(np.float32))
+    xd, gd, pk, ws = dev_bf16(xb), dev_bf16(gb), _packed_dev(w), torch.full((4,), 0.02, device="cuda").to(torch.bfloat16)
+    q, s = torch.zeros(m, k, dtype=torch.int8, device="cuda"), torch.zeros(m, dtype=torch.bfloat16, device="cuda")
     out = torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
-    st = torch.cuda.current_stream().cuda_stream
-    for i, rows in enumerate((m, 300)):
-        for a in range(0, m, rows):
-            b = min(a + rows, m)
-            assert lib.bitlinear_norm_forward_bf16(x[a:b].data_ptr(), norm_w.data_ptr(), 1e-5, 0, pk.data_ptr(), ws.data_ptr(), None,
-                                                   out.data_ptr(), q[i, a:b].data_ptr(), s[i, a:b].data_ptr(), b - a, n, k, 0, st) == 0
-    torch.cuda.synchronize()
-    assert torch.equal(q[0], q[1]) and torch.equal(s[0].view(torch.int16), s[1].view(torch.int16))
-
-
-# a wave per row (768 rows on, up to 2560 values), 256 threads (up to 4096; from 512 rows on up to 8192) and 512 behind
-@pytest.mark.parametrize("m,k", [(767, 2560), (768, 2560), (769, 1152), (768, 2688), (511, 4224), (512, 8192), (512, 8320)])
-def test_norm_and_quantizer_by_256_threads_per_row_equal_the_others(m, k):
-    test_norm_and_quantizer_by_a_wave_per_row_equal_a_workgroup_per_row(m, k)
+    assert lib.bitlinear_norm_forward_bf16(xd.data_ptr(), gd.data_ptr(), 1e-5, 0, pk.data_ptr(), ws.data_ptr(), None, out.data_ptr(), q.data_ptr(),
+                                           s.data_ptr(), m, n, k, 0, torch.cuda.current_stream().cuda_stream) == 0
+    finite = np.arange(m) != 5
+    with np.errstate(invalid="ignore"):
+        norm = o.rmsnorm_bf16(xb, gb, 1e-5)
+    want_q, want_s = o.quant_input(norm[finite])
+    assert np.array_equal(q.cpu().numpy()[finite], want_q) and np.array_equal(host_bits(s)[finite], want_s)
+    q5, s5 = bitlinear.quant_input(dev_bf16(norm[5:6]))
+    assert torch.equal(q[5:6], q5) and torch.equal(s[5:6].view(torch.int16), s5.view(-1).view(torch.int16))
 
 
 @pytest.mark.parametrize("k", [1024, 1152, 2048, 2176, 4096, 4224])

@@ -682,8 +682,8 @@ def test_norm_bitlinear_of_rows_that_are_not_finite(M, K, N):
 @pytest.mark.parametrize("T", [1, 31, 33, 64, 65, 97, 129, 161])
 @pytest.mark.parametrize("nh,nkv", [(1, 1), (4, 2), (20, 5), (16, 2)])
 def test_prompt_attention_of_many_sequences_equals_each_alone(nh, nkv, T):
-    """Rows of one to six steps through rings of three (more workgroups than twice the CUs) and of four steps; the cache rows
-    behind the prompt, which the ring's requests reach, hold NaNs."""
+    """Rows of one to six steps through attn_prefill_kernel (many sequences: more workgroups than two per CU) and, alone, through
+    attn_prefill_split_kernel; the cache rows behind the prompt, which the rings' requests reach, hold NaNs."""
     groups = (T + 15) // 16 * nkv
     B, S = 512 // groups + 2, T + 40
     gen = torch.Generator(device="cuda").manual_seed(T)
