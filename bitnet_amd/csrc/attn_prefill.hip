@@ -60,7 +60,7 @@ __global__ __launch_bounds__(kRopeThreads) void rope_cache_tokens_kernel(
 // written for them: flash-attention style, scores and output on the bf16 matrix pipe (16x16x32).
 // One wave = 16 consecutive tokens of one query head; the G waves of a workgroup are the G heads
 // that share a kv head, so they walk the same cache rows together: the workgroup brings every
-// block of 32 K and V rows into LDS once (a ring of RING steps, one barrier per step) and each wave
+// block of 32 K and V rows into LDS once (a ring of steps, one barrier per step) and each wave
 // takes its operands from there.
 //   S^T block = K rows (A operand: 16 positions x 32 dims per step) x q^T (B operand: 16 tokens),
 //   so a result lane (c, g4) holds, for token c, positions 4 g4 + j of the block (j = 0..3).  Two
@@ -74,6 +74,7 @@ __global__ __launch_bounds__(kRopeThreads) void rope_cache_tokens_kernel(
 // (c, c + 16, c + 32, c + 48) with two lane permutes; the sums stay per lane until the end.
 constexpr int kApRowsBytes = 32 * kHeadDim * 2;  // K or V rows of a step
 constexpr int kApStepBytes = 2 * kApRowsBytes;   // both
+constexpr int kApRing = 3;                       // steps of attn_prefill_kernel's ring: 48 KB, so that three workgroups fit a CU
 // 16 bytes per lane from a buffer straight into LDS: lane l's piece lands at `to` + 16 l (wave-uniform)
 __device__ __forceinline__ void ap_load(__amdgpu_buffer_rsrc_t rsrc, uint8_t* to, int offset) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)to, 16, offset, 0, 0, 0);
@@ -81,7 +82,7 @@ __device__ __forceinline__ void ap_load(__amdgpu_buffer_rsrc_t rsrc, uint8_t* to
 
 // What bounds it: a step is some 200 instructions of the one wave on a SIMD and a chain of LDS reads, four dependent MFMAs,
 // the maximum, the exponentials (0.56 us; 512 tokens are 16 steps).  Rows that came a step ahead through registers had not
-// arrived in time: 512 tokens 12.9 -> 12.0 us, 1000 29.9 -> 26.5, 2048 77.6 -> 66.7 (20 / 5 heads).  The ring is RING - 1 steps
+// arrived in time: 512 tokens 12.9 -> 12.0 us, 1000 29.9 -> 26.5, 2048 77.6 -> 66.7 (20 / 5 heads).  The ring is two steps
 // ahead from step 0 on, not in front of it: q, first in the source, is loaded by the generated code behind the ring's first
 // requests and the first barrier, and its wait for all loads drains the ring once per tile.
 // Workgroups start in the order of their index, so the heads and sequences are its fast part and the blocks of tokens its
@@ -89,7 +90,7 @@ __device__ __forceinline__ void ap_load(__amdgpu_buffer_rsrc_t rsrc, uint8_t* to
 // and stood alone at the end (2048 tokens 66.6 -> 44.8 us, 8 sequences of 512 35.5 -> 25.9, 4 of 1024 53.8 -> 40.7).
 // Taken where there are more than two workgroups per CU, which hide one another's waits (attn_prefill_split_kernel below:
 // 8 sequences of 512 31.5 us).
-template <int G, int RING>
+template <int G>
 __global__ __launch_bounds__(64 * G) void attn_prefill_kernel(
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ cache_k, const uint16_t* __restrict__ cache_v,
     uint16_t* __restrict__ out, int T, int S, int start, int n_heads, int n_kv_heads, int last_block) {
@@ -121,7 +122,7 @@ __global__ __launch_bounds__(64 * G) void attn_prefill_kernel(
         (void*)(cache_k + ((size_t)b * S * n_kv_heads + kvh) * kHeadDim), 0, span_bytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(cache_v + ((size_t)b * S * n_kv_heads + kvh) * kHeadDim), 0, span_bytes, 0x00020000);
-    // The rows come straight into LDS, a ring of RING steps: request number r * G + wave of a step fills 1 KB, four
+    // The rows come straight into LDS, a ring of three steps: request number r * G + wave of a step fills 1 KB, four
     // rows of K (the first eight) or V, whose 16-byte pieces are swizzled by the row (by choice of the piece that a lane
     // fetches), so that 16 rows at one piece and the 16 pieces of a row are both spread over all banks
     constexpr int kLoads = 16 / G;
@@ -133,7 +134,7 @@ __global__ __launch_bounds__(64 * G) void attn_prefill_kernel(
         g_off[r] = row * row_bytes + ((lane & 15) ^ (row & 15)) * 16;
     }
     auto request = [&](int st) {
-        uint8_t* to = lds_kv + (st % RING) * kApStepBytes;
+        uint8_t* to = lds_kv + (st % kApRing) * kApStepBytes;
         // (in the per-lane operand: that is the one the range check looks at; unsigned, as it may lie behind 2^31 there)
         const unsigned base = (unsigned)st * 32u * (unsigned)row_bytes;
 #pragma unroll
@@ -158,7 +159,7 @@ __global__ __launch_bounds__(64 * G) void attn_prefill_kernel(
 
     // raw scores of a step's 32 positions
     auto scores = [&](int st, v4f(&acc)[2]) {
-        const uint8_t* kl = lds_kv + (st % RING) * kApStepBytes;
+        const uint8_t* kl = lds_kv + (st % kApRing) * kApStepBytes;
         v4u kb[2][4];
 #pragma unroll
         for (int bi = 0; bi < 2; ++bi)
@@ -173,7 +174,7 @@ __global__ __launch_bounds__(64 * G) void attn_prefill_kernel(
     };
     // softmax and outputs of a step
     auto step = [&](int st, const v4f(&acc)[2]) {
-        const uint8_t* vl = lds_kv + (st % RING) * kApStepBytes;
+        const uint8_t* vl = lds_kv + (st % kApRing) * kApStepBytes;
         v4u vb[8];
 #pragma unroll
         for (int jj = 0; jj < 8; ++jj) vb[jj] = *(const v4u*)(vl + (jj >> 2) * 16 * 256 + v_off[jj & 3]);
@@ -234,12 +235,12 @@ __global__ __launch_bounds__(64 * G) void attn_prefill_kernel(
         asm volatile("" ::: "memory");
     };
 #pragma unroll
-    for (int st = 0; st < RING - 1; ++st) request(st);
-    constexpr int kYounger = (RING - 2) * kLoads, kWait = 0x0f70 | (kYounger & 15) | ((kYounger >> 4) << 14);
+    for (int st = 0; st < kApRing - 1; ++st) request(st);
+    constexpr int kYounger = (kApRing - 2) * kLoads, kWait = 0x0f70 | (kYounger & 15) | ((kYounger >> 4) << 14);
     __builtin_amdgcn_s_waitcnt(kWait);
     meet();
     for (int st = 0; st < steps; ++st) {
-        request(st + RING - 1);  // (the stage of step st - 1, which every wave has left; behind the rows: zeros)
+        request(st + kApRing - 1);  // (the stage of step st - 1, which every wave has left; behind the rows: zeros)
         v4f now[2];
         scores(st, now);
         step(st, now);
@@ -809,7 +810,7 @@ extern "C" int bitnet_attn_prefill(const uint16_t* q, const uint16_t* cache_k, c
                        (ApRing<G, kApAhead>::LDS), (hipStream_t)stream, q, cache_k, cache_v, out, T, S, start, n_heads, n_kv_heads, g, \
                        last)
 #define BITNET_AP(G)                                                                                                                \
-    hipLaunchKernelGGL((attn_prefill_kernel<G, 3>), dim3(n_kv_heads, B, here), dim3(64 * G), 3 * kApStepBytes, (hipStream_t)stream, q,  \
+    hipLaunchKernelGGL((attn_prefill_kernel<G>), dim3(n_kv_heads, B, here), dim3(64 * G), kApRing * kApStepBytes, (hipStream_t)stream, q,  \
                        cache_k, cache_v, out, T, S, start, n_heads, n_kv_heads, last)
     for (int last = blocks - 1; last >= 0; last -= 65535) {  // (what a grid's third dimension holds)
         const int here = last + 1 < 65535 ? last + 1 : 65535;

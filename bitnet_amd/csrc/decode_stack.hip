@@ -1069,7 +1069,7 @@ struct Stack {
                 if (4 * u < G) raw[u] = __builtin_amdgcn_raw_buffer_load_b128(row, ((kvh * G + head[u]) * kHeadDim + 8 * c) * 2, 0, kSc1);
             if (has_new) fresh = __builtin_amdgcn_raw_buffer_load_b128(row, (new_head * kHeadDim + 8 * c) * 2, 0, kSc1);
         };
-        // Where wqkv's and the attention's tasks together are more than the workgroups (288 of 256 at four sequences, 368 at
+        // Where wqkv's and the attention's tasks together are more than the workgroups (280 of 256 at four sequences, 360 at
         // eight), some come here from a wqkv task: the token's row is there by the time that the cache rows are, 1.5 us later,
         // and a poll behind those is another 0.4.  So the row is requested along with them and looked at once they are turned: four
         // sequences 784 -> 775 us a step at 512 positions, five 798 -> 783, eight 853 -> 845.  (With the cache rows brought into
